@@ -179,6 +179,10 @@ struct rbmoe_layer {
     rbmoe_ctx* ctx = nullptr;
     rbmoe_config cfg{};
     int Fs = 0;       // shared expert width
+    // Expert widths as the kernels see them: the matrix-core kernels take whole tiles, so a width between two multiples
+    // of the tile is rounded up and the extra gate and up rows and down columns are zero (their hidden values are
+    // silu(0) * 0 = 0 and add nothing).  Equal to the true widths where nothing is rounded.
+    int Fw = 0, Fsw = 0;
     int max_T = 0;
     int max_S = 0;
     int max_nb = 0;
@@ -277,20 +281,31 @@ struct Plan {
 void choose_kernel_sets(rbmoe_layer* L) {
     const rbmoe_config* cfg = &L->cfg;
     L->use_stream = L->use_f32_mc = L->cast_rows = false;
+    // Expert widths are rounded up to whole tiles (the model width is the caller's row pitch and is not): 64 columns
+    // for the packed bf16 / int8 kernels, 32 for the f32 ones.  The any-shape kernels run at a thirtieth of the bf16
+    // matrix-core rate and a third of the f32 one, so rounding pays while it multiplies the work by less than that:
+    // up to four times (bf16) and twice (f32).  d_ff 352 (the default model's) is 384 columns: 9 % more work.
+    auto rounded = [](int f, int unit, int most) {
+        const int up = (f + unit - 1) / unit * unit;
+        return up <= most * f ? up : f;
+    };
+    const int unit = cfg->weight_dtype == RBMOE_F32 ? 32 : 64, most = cfg->weight_dtype == RBMOE_F32 ? 2 : 4;
+    L->Fw = rounded(cfg->d_ff, unit, most);
+    L->Fsw = rounded(L->Fs, unit, most);
     // bf16 matrix cores: bf16 activations, bf16 or int8 weights, widths that fit the packed layout
     // (f32 rows with bf16 / int8 weights - what a caller with f32 matrices and a quantized or bf16 checkpoint has -
     // take the same kernels over a bf16 copy of the rows)
     const bool mc = !L->force_generic && cfg->weight_dtype != RBMOE_F32;
-    L->use_stream = mc && stream_shape_ok(cfg->d_ff, cfg->d_model) && stream_shape_ok(cfg->d_model, cfg->d_ff) &&
+    L->use_stream = mc && stream_shape_ok(L->Fw, cfg->d_model) && stream_shape_ok(cfg->d_model, L->Fw) &&
                     (!cfg->shared_expert ||
-                     (stream_shape_ok(L->Fs, cfg->d_model) && stream_shape_ok(cfg->d_model, L->Fs)));
+                     (stream_shape_ok(L->Fsw, cfg->d_model) && stream_shape_ok(cfg->d_model, L->Fsw)));
 
     L->use_f32_mc = !L->force_generic && cfg->act_dtype == RBMOE_F32 && cfg->weight_dtype == RBMOE_F32 &&
-                    f32_shape_ok(cfg->d_ff, cfg->d_model) && f32_shape_ok(cfg->d_model, cfg->d_ff) &&
-                    (!cfg->shared_expert || (f32_shape_ok(L->Fs, cfg->d_model) && f32_shape_ok(cfg->d_model, L->Fs)));
+                    f32_shape_ok(L->Fw, cfg->d_model) && f32_shape_ok(cfg->d_model, L->Fw) &&
+                    (!cfg->shared_expert || (f32_shape_ok(L->Fsw, cfg->d_model) && f32_shape_ok(cfg->d_model, L->Fsw)));
     {
         // the streaming kernel addresses activation rows with 32-bit byte offsets
-        const size_t widest = (size_t)std::max(std::max(cfg->d_model, cfg->d_ff), L->Fs);
+        const size_t widest = (size_t)std::max(std::max(cfg->d_model, L->Fw), L->Fsw);
         const size_t rows = (size_t)cfg->max_tokens * (size_t)std::max(1, cfg->experts_per_token);
         if (rows * widest * 2 >= ((size_t)1 << 32)) L->use_stream = false;
     }
@@ -299,12 +314,16 @@ void choose_kernel_sets(rbmoe_layer* L) {
         if (cfg->d_model % 8 == 0) L->cast_rows = true;
         else L->use_stream = false;
     }
+    if (!L->use_stream && !L->use_f32_mc) {  // the any-shape kernels take the widths as they are
+        L->Fw = cfg->d_ff;
+        L->Fsw = L->Fs;
+    }
 }
 
 Plan make_plan(rbmoe_layer* L) {
     const rbmoe_config& c = L->cfg;
-    const size_t E = c.num_experts, d = c.d_model, F = c.d_ff, k = c.experts_per_token;
-    const size_t Fs = L->Fs, T = L->max_T, S = L->max_S, nb = L->max_nb;
+    const size_t E = c.num_experts, d = c.d_model, F = L->Fw, k = c.experts_per_token;
+    const size_t Fs = L->Fsw, T = L->max_T, S = L->max_S, nb = L->max_nb;
     const size_t ws = dtype_size(c.weight_dtype), as = dtype_size(c.act_dtype);
     Plan p;
     p.add(&L->router, E * d * 4);
@@ -609,15 +628,15 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
         case RBMOE_W_UP:
             want_rows = F; want_cols = d;
             if (expert < 0 || expert >= E) return fail(ctx, RBMOE_INVALID_CONFIG, "expert index out of range");
-            elem_off = ((size_t)expert * 2 + (which == RBMOE_W_UP ? 1 : 0)) * F * d;
-            scale_off = ((size_t)expert * 2 + (which == RBMOE_W_UP ? 1 : 0)) * F;
+            elem_off = ((size_t)expert * 2 + (which == RBMOE_W_UP ? 1 : 0)) * L->Fw * d;
+            scale_off = ((size_t)expert * 2 + (which == RBMOE_W_UP ? 1 : 0)) * L->Fw;
             dst = static_cast<char*>(L->wgu.p);
             sdst = static_cast<float*>(L->sgu.p);
             break;
         case RBMOE_W_DOWN:
             want_rows = d; want_cols = F;
             if (expert < 0 || expert >= E) return fail(ctx, RBMOE_INVALID_CONFIG, "expert index out of range");
-            elem_off = (size_t)expert * d * F;
+            elem_off = (size_t)expert * d * L->Fw;
             scale_off = (size_t)expert * d;
             dst = static_cast<char*>(L->wd.p);
             sdst = static_cast<float*>(L->sd.p);
@@ -626,8 +645,8 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
         case RBMOE_W_SHARED_UP:
             if (!c.shared_expert) return fail(ctx, RBMOE_INVALID_CONFIG, "the layer has no shared expert");
             want_rows = Fs; want_cols = d;
-            elem_off = (size_t)(which == RBMOE_W_SHARED_UP ? 1 : 0) * Fs * d;
-            scale_off = (size_t)(which == RBMOE_W_SHARED_UP ? 1 : 0) * Fs;
+            elem_off = (size_t)(which == RBMOE_W_SHARED_UP ? 1 : 0) * L->Fsw * d;
+            scale_off = (size_t)(which == RBMOE_W_SHARED_UP ? 1 : 0) * L->Fsw;
             dst = static_cast<char*>(L->swgu.p);
             sdst = static_cast<float*>(L->ssgu.p);
             break;
@@ -646,7 +665,7 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
                       want_rows, want_cols);
         return fail(ctx, RBMOE_INVALID_INPUT, buf);
     }
-    const size_t n = (size_t)rows * cols;
+    const size_t n_given = (size_t)rows * cols;
     // The router is f32 whatever the experts' dtype - unless it is given as int8 rows with scales, or the layer
     // was told to quantize it like every other Linear (TransformerLm::quantize, src/transformer.rs:899-910, reaches
     // it through MoeLayer::linears_mut, src/moe.rs:491-500): the layer then routes with the quantized product.
@@ -665,16 +684,16 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
             if (!scales) return fail(ctx, RBMOE_NULL_POINTER, "int8 weights need scales");
         }
     } else if (dtype == RBMOE_F32 && target == RBMOE_BF16) {
-        staged.resize(n * 2);
+        staged.resize(n_given * 2);
         const float* f = static_cast<const float*>(data);
         uint16_t* o = reinterpret_cast<uint16_t*>(staged.data());
-        for (size_t i = 0; i < n; ++i) o[i] = host_f32_to_bf16(f[i]);
+        for (size_t i = 0; i < n_given; ++i) o[i] = host_f32_to_bf16(f[i]);
         src = staged.data();
     } else if (dtype == RBMOE_BF16 && target == RBMOE_F32) {
-        staged.resize(n * 4);
+        staged.resize(n_given * 4);
         const uint16_t* h = static_cast<const uint16_t*>(data);
         float* o = reinterpret_cast<float*>(staged.data());
-        for (size_t i = 0; i < n; ++i) o[i] = host_bf16_to_f32(h[i]);
+        for (size_t i = 0; i < n_given; ++i) o[i] = host_bf16_to_f32(h[i]);
         src = staged.data();
     } else if (dtype == RBMOE_F32 && target == RBMOE_I8) {
         // Per row: scale = absmax / 127, then
@@ -684,7 +703,7 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
         //           TransformerLm::quantize applies: q = clamp(round(w * (1 / scale))).
         // `round` is f32::round: halves away from zero.  The two differ where the reciprocal's rounding moves a
         // quotient across a half.
-        staged.resize(n);
+        staged.resize(n_given);
         staged_scales.resize(rows);
         const float* f = static_cast<const float*>(data);
         int8_t* q = reinterpret_cast<int8_t*>(staged.data());
@@ -708,16 +727,35 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
     }
     if (is_router) {
         if (router_to_i8) {
-            HIP_TRY(ctx, hipMemcpy(L->router_q.p, src, n, hipMemcpyHostToDevice));
+            HIP_TRY(ctx, hipMemcpy(L->router_q.p, src, n_given, hipMemcpyHostToDevice));
             HIP_TRY(ctx, hipMemcpy(L->router_s.p, scales, (size_t)rows * 4, hipMemcpyHostToDevice));
         } else {
-            HIP_TRY(ctx, hipMemcpy(L->router.p, src, n * 4, hipMemcpyHostToDevice));
+            HIP_TRY(ctx, hipMemcpy(L->router.p, src, n_given * 4, hipMemcpyHostToDevice));
         }
         L->router_q8 = router_to_i8;
         L->weights_set = true;
         return RBMOE_OK;
     }
     const size_t es = dtype_size(target);
+    const int scale_rows = rows;  // (the scales of rows added below stay zero)
+    std::vector<unsigned char> widened;
+    {
+        const bool shared_w = which >= RBMOE_W_SHARED_GATE;
+        const bool is_down = which == RBMOE_W_DOWN || which == RBMOE_W_SHARED_DOWN;
+        const int wide = shared_w ? L->Fsw : L->Fw;
+        const int to_rows = is_down ? rows : wide, to_cols = is_down ? wide : cols;
+        if (to_rows != rows || to_cols != cols) {  // the width the kernels see: zero rows below, zero columns behind
+            widened.assign((size_t)to_rows * to_cols * es, 0);
+            for (int r = 0; r < rows; ++r)
+                std::memcpy(widened.data() + (size_t)r * to_cols * es,
+                            static_cast<const unsigned char*>(src) + (size_t)r * cols * es, (size_t)cols * es);
+            src = widened.data();
+            rows = to_rows;
+            cols = to_cols;
+        }
+    }
+    const size_t n = (size_t)rows * cols;
+    const void* const plain_src = src;  // row-major, in the weight dtype
     std::vector<unsigned char> packed;
     if (L->use_stream && !is_router) {
         // operand order of the matrix cores, matrix by matrix (same offsets, different inner layout)
@@ -730,7 +768,7 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
     }
     HIP_TRY(ctx, hipMemcpy(dst + elem_off * es, src, n * es, hipMemcpyHostToDevice));
     if (target == RBMOE_I8)
-        HIP_TRY(ctx, hipMemcpy(sdst + scale_off, scales, (size_t)rows * 4, hipMemcpyHostToDevice));
+        HIP_TRY(ctx, hipMemcpy(sdst + scale_off, scales, (size_t)scale_rows * 4, hipMemcpyHostToDevice));
     L->weights_set = true;
     if (L->training && !is_router) {
         // The backward products multiply by the weight itself, not by its transpose (grad_input =
@@ -740,7 +778,7 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
         const bool shared_w = which >= RBMOE_W_SHARED_GATE;
         const bool is_down = which == RBMOE_W_DOWN || which == RBMOE_W_SHARED_DOWN;
         const bool is_up = which == RBMOE_W_UP || which == RBMOE_W_SHARED_UP;
-        const int Fw = shared_w ? Fs : F;
+        const int Fw = shared_w ? L->Fsw : L->Fw;
         if (target == RBMOE_F32) {
             // plain row-major f32, as the f32 product kernel reads its weights
             const float* f = static_cast<const float*>(src);
@@ -773,13 +811,8 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
             }
         } else {
             // packed bf16; column steps of 16 never straddle the two halves of [d, 2F]
-            std::vector<uint16_t> plain(n), tr(n), trp(n);
-            if (dtype == RBMOE_BF16) {
-                std::memcpy(plain.data(), data, n * 2);
-            } else {
-                const float* f = static_cast<const float*>(data);
-                for (size_t i = 0; i < n; ++i) plain[i] = host_f32_to_bf16(f[i]);
-            }
+            const uint16_t* const plain = static_cast<const uint16_t*>(plain_src);
+            std::vector<uint16_t> tr(n), trp(n);
             for (int r = 0; r < rows; ++r)
                 for (int cc = 0; cc < cols; ++cc) tr[(size_t)cc * rows + r] = plain[(size_t)r * cols + cc];
             pack_weight_bf16(tr.data(), cols, rows, trp.data());  // [cols, rows] matrix
@@ -854,7 +887,7 @@ Work work_of_layer(const rbmoe_layer* L) {
 // bytes used.  With base == nullptr only the size is computed.
 size_t carve_decode_work(const rbmoe_layer* L, int T, unsigned char* base, Work* w) {
     const rbmoe_config& c = L->cfg;
-    const size_t E = c.num_experts, d = c.d_model, F = c.d_ff, k = c.experts_per_token, Fs = L->Fs;
+    const size_t E = c.num_experts, d = c.d_model, F = L->Fw, k = c.experts_per_token, Fs = L->Fsw;
     const size_t S = (size_t)T * k, as = L->cast_rows ? 2 : dtype_size(c.act_dtype);
     const size_t tiles = S / kDecodeTileM + E + 1;
     size_t used = 0;
@@ -900,7 +933,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
     rbmoe_ctx* ctx = L->ctx;
     const rbmoe_config& c = L->cfg;
-    const int E = c.num_experts, d = c.d_model, F = c.d_ff, k = c.experts_per_token, Fs = L->Fs;
+    const int E = c.num_experts, d = c.d_model, F = L->Fw, k = c.experts_per_token, Fs = L->Fsw;
     // MoeLayer::forward_train's width check (reference src/moe.rs:248-253)
     if (cols != d) {
         char buf[120];
@@ -1539,7 +1572,7 @@ int rbmoe_layer_enable_training(rbmoe_layer* L) {
                       router_grad_max_tokens(), L->max_T);
         return fail(ctx, RBMOE_UNSUPPORTED, buf);
     }
-    const size_t E = c.num_experts, d = c.d_model, F = c.d_ff, Fs = L->Fs, T = L->max_T, S = L->max_S;
+    const size_t E = c.num_experts, d = c.d_model, F = L->Fw, Fs = L->Fsw, T = L->max_T, S = L->max_S;
     if (bf16_layer) {
         if (!stream_shape_ok((int)d, (int)(2 * F)) || (c.shared_expert && !stream_shape_ok((int)d, (int)(2 * Fs))))
             return fail(ctx, RBMOE_UNSUPPORTED, "expert width not supported by the backward products");
@@ -1694,7 +1727,7 @@ int rbmoe_backward(rbmoe_layer* L, const void* grad_output, int32_t tokens, int3
     if (L->last_T < 0) return fail(ctx, RBMOE_INVALID_INPUT, "no forward pass has run yet");
     if (const int rc = backward_shape_problem(L, tokens, cols)) return rc;
     const rbmoe_config& c = L->cfg;
-    const int E = c.num_experts, d = c.d_model, F = c.d_ff, k = c.experts_per_token, Fs = L->Fs, T = L->last_T;
+    const int E = c.num_experts, d = c.d_model, F = L->Fw, k = c.experts_per_token, Fs = L->Fsw, T = L->last_T;
     if (T == 0) return RBMOE_OK;
     if (!grad_output || !grad_input) return fail(ctx, RBMOE_NULL_POINTER, "grad_output or grad_input is NULL");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
@@ -1912,33 +1945,33 @@ int rbmoe_get_weight_grad(rbmoe_layer* L, int32_t which, int32_t expert, float* 
     if (!L->training) return fail(ctx, RBMOE_INVALID_CONFIG, "training is not enabled on this layer");
     if (!host) return fail(ctx, RBMOE_NULL_POINTER, "host buffer is NULL");
     const rbmoe_config& c = L->cfg;
-    const size_t E = c.num_experts, d = c.d_model, F = c.d_ff, Fs = L->Fs;
+    const size_t E = c.num_experts, d = c.d_model, F = c.d_ff, Fs = L->Fs, Fw = L->Fw, Fsw = L->Fsw;
     const float* src = nullptr;
-    size_t want_rows = 0, want_cols = 0;
+    size_t want_rows = 0, want_cols = 0, pitch = 0;  // pitch: of the rows in `src` where it is not want_cols
     const bool bad_expert = expert < 0 || (size_t)expert >= E;
     switch (which) {
         case RBMOE_W_ROUTER: src = (const float*)L->g_router.p; want_rows = E; want_cols = d; break;
         case RBMOE_W_GATE:
         case RBMOE_W_UP:
             if (bad_expert) return fail(ctx, RBMOE_INVALID_CONFIG, "expert index out of range");
-            src = (const float*)L->g_gu.p + ((size_t)expert * 2 + (which == RBMOE_W_UP ? 1 : 0)) * F * d;
+            src = (const float*)L->g_gu.p + ((size_t)expert * 2 + (which == RBMOE_W_UP ? 1 : 0)) * Fw * d;
             want_rows = F; want_cols = d;
             break;
         case RBMOE_W_DOWN:
             if (bad_expert) return fail(ctx, RBMOE_INVALID_CONFIG, "expert index out of range");
-            src = (const float*)L->g_down.p + (size_t)expert * d * F;
-            want_rows = d; want_cols = F;
+            src = (const float*)L->g_down.p + (size_t)expert * d * Fw;
+            want_rows = d; want_cols = F; pitch = Fw;
             break;
         case RBMOE_W_SHARED_GATE:
         case RBMOE_W_SHARED_UP:
             if (!c.shared_expert) return fail(ctx, RBMOE_INVALID_CONFIG, "the layer has no shared expert");
-            src = (const float*)L->g_sgu.p + (size_t)(which == RBMOE_W_SHARED_UP ? 1 : 0) * Fs * d;
+            src = (const float*)L->g_sgu.p + (size_t)(which == RBMOE_W_SHARED_UP ? 1 : 0) * Fsw * d;
             want_rows = Fs; want_cols = d;
             break;
         case RBMOE_W_SHARED_DOWN:
             if (!c.shared_expert) return fail(ctx, RBMOE_INVALID_CONFIG, "the layer has no shared expert");
             src = (const float*)L->g_sdown.p;
-            want_rows = d; want_cols = Fs;
+            want_rows = d; want_cols = Fs; pitch = Fsw;
             break;
         case RBMOE_W_NORM:
             if (!L->g_norm.p) return fail(ctx, RBMOE_INVALID_CONFIG, "the feed-forward norm has not been set");
@@ -1955,7 +1988,10 @@ int rbmoe_get_weight_grad(rbmoe_layer* L, int32_t which, int32_t expert, float* 
         return RBMOE_OK;
     }
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    HIP_TRY(ctx, hipMemcpy(host, src, want_rows * want_cols * 4, hipMemcpyDeviceToHost));
+    if (pitch == 0 || pitch == want_cols)
+        HIP_TRY(ctx, hipMemcpy(host, src, want_rows * want_cols * 4, hipMemcpyDeviceToHost));
+    else
+        HIP_TRY(ctx, hipMemcpy2D(host, want_cols * 4, src, pitch * 4, want_cols * 4, want_rows, hipMemcpyDeviceToHost));
     return RBMOE_OK;
 }
 
@@ -1996,7 +2032,7 @@ int rbmoe_get_expert_rows(rbmoe_layer* L, float* hidden, float* expert_out) {
     if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
     rbmoe_ctx* ctx = L->ctx;
     if (L->last_T < 0) return fail(ctx, RBMOE_INVALID_INPUT, "no forward pass has run yet");
-    const int E = L->cfg.num_experts, d = L->cfg.d_model, F = L->cfg.d_ff;
+    const int E = L->cfg.num_experts, d = L->cfg.d_model, F = L->cfg.d_ff, Fw = L->Fw;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     int R = 0;
     HIP_TRY(ctx, hipMemcpy(&R, L->last.offsets + E, 4, hipMemcpyDeviceToHost));
@@ -2013,10 +2049,12 @@ int rbmoe_get_expert_rows(rbmoe_layer* L, float* hidden, float* expert_out) {
         return RBMOE_OK;
     };
     int rc = RBMOE_OK;
+    // the hidden rows lie Fw apart; the columns past F are the zeros of the rounded width
+    std::vector<float> wide;
     if (L->last_front && hidden && R > 0) {
         // the hidden rows lie per expert over all the call's rows: pick the routed ones, in permuted order
         const int T = L->last_T;
-        std::vector<float> all((size_t)E * T * F);
+        std::vector<float> all((size_t)E * T * Fw);
         std::vector<int> offs(E + 1), ptok(R);
         rc = fetch(all.data(), L->last.hall, all.size());
         if (rc != RBMOE_OK) return rc;
@@ -2024,7 +2062,12 @@ int rbmoe_get_expert_rows(rbmoe_layer* L, float* hidden, float* expert_out) {
         HIP_TRY(ctx, hipMemcpy(ptok.data(), L->last.perm_token, (size_t)R * 4, hipMemcpyDeviceToHost));
         for (int e = 0; e < E; ++e)
             for (int pos = offs[e]; pos < offs[e + 1]; ++pos)
-                std::memcpy(hidden + (size_t)pos * F, all.data() + ((size_t)e * T + ptok[pos]) * F, (size_t)F * 4);
+                std::memcpy(hidden + (size_t)pos * F, all.data() + ((size_t)e * T + ptok[pos]) * Fw, (size_t)F * 4);
+    } else if (hidden && F != Fw) {
+        wide.resize((size_t)R * Fw);
+        rc = fetch(wide.data(), L->last.h, wide.size());
+        if (rc == RBMOE_OK)
+            for (int r = 0; r < R; ++r) std::memcpy(hidden + (size_t)r * F, wide.data() + (size_t)r * Fw, (size_t)F * 4);
     } else {
         rc = fetch(hidden, L->last.h, (size_t)R * F);
     }

@@ -209,6 +209,18 @@ int rbmoe_forward_host(rbmoe_layer* layer, const void* x, int32_t T, int32_t col
                        const uint8_t* valid, const float* router_bias, const void* residual,
                        void* out);
 
+/* forward_train on HOST matrices together with its MoeCache (src/moe.rs:243-341), in two halves.  _begin copies the
+ * rows in, enqueues the forward (block != 0: the block step of rbmoe_forward_block, `residual` is then ignored) and
+ * returns when `routing` and `losses` ([2]: auxiliary, z; either may be NULL) are filled, which is while the expert
+ * products are still under way; `out` is complete after _finish.  `x_dtype` is the dtype of x, residual and out: the
+ * layer's own, or RBMOE_F32 on a bf16 layer (rows are rounded to nearest even on the way in and widened on the way
+ * out).  x, residual and out belong to the call until _finish.  Between the two calls no other call may
+ * be made on the layer. */
+int rbmoe_forward_train_begin(rbmoe_layer* layer, const void* x, int32_t x_dtype, int32_t T, int32_t cols,
+                              const uint8_t* valid, const float* router_bias, const void* residual, int32_t block,
+                              void* out, rbmoe_routing* routing, float* losses);
+int rbmoe_forward_train_finish(rbmoe_layer* layer);
+
 /* MoeCache::aux_loss / z_loss (src/moe.rs:158-172) of the last forward.
  * Synchronises the stream. */
 int rbmoe_get_losses(rbmoe_layer* layer, float* aux_loss, float* z_loss);
@@ -260,6 +272,10 @@ int rbmoe_backward(rbmoe_layer* layer, const void* grad_output, int32_t tokens, 
 /* Same on HOST pointers; synchronises. */
 int rbmoe_backward_host(rbmoe_layer* layer, const void* grad_output, int32_t tokens, int32_t cols,
                         void* grad_input);
+/* The same (block != 0: rbmoe_backward_block) on host gradients of dtype `dtype`: the layer's own, or RBMOE_F32 on a
+ * bf16 layer.  Synchronises. */
+int rbmoe_backward_train_host(rbmoe_layer* layer, const void* grad_output, int32_t dtype, int32_t tokens, int32_t cols,
+                              int32_t block, void* grad_input);
 /* Param::zero_grad for every weight of the layer. */
 int rbmoe_zero_grads(rbmoe_layer* layer);
 /* One accumulated weight gradient as f32 [rows, cols] into host memory (same ids and shapes as
@@ -328,6 +344,12 @@ const char* rbmoe_expert_kernel_name(const rbmoe_layer* layer);
 /* Device memory helpers for hosts without their own HIP binding. */
 int rbmoe_device_alloc(rbmoe_ctx* ctx, size_t bytes, void** out);
 int rbmoe_device_free(rbmoe_ctx* ctx, void* ptr);
+/* Host memory the GPU writes to and reads from directly (57 GB/s over the link here, against 4 to 30 for a copy to or
+ * from memory that is not pinned): every entry point above that fills or reads a host array recognises these blocks.
+ * They come from a pool of at most 1 GiB that keeps freed blocks for the next caller and is emptied when the last
+ * context goes; RBMOE_OUT_OF_MEMORY when it is exhausted (use ordinary memory then).  Any thread may free. */
+int rbmoe_host_alloc(rbmoe_ctx* ctx, size_t bytes, void** out);
+void rbmoe_host_free(void* ptr);
 int rbmoe_copy_to_device(rbmoe_ctx* ctx, void* dst, const void* src, size_t bytes);
 int rbmoe_copy_to_host(rbmoe_ctx* ctx, void* dst, const void* src, size_t bytes);
 /* Device-to-device copy on the context's stream, then synchronise (also serves as the

@@ -108,6 +108,11 @@ extern "C" {
     pub fn rbmoe_forward_kernel_times(layer: *mut rbmoe_layer, x: *const c_void, tokens: i32, cols: i32, valid: *const u8,
                                router_bias: *const f32, residual: *const c_void, out: *mut c_void,
                                ms: *mut f32) -> c_int;
+    // forward_train with its MoeCache in two halves: tables and losses are filled when _begin returns, `out` after _finish
+    pub fn rbmoe_forward_train_begin(layer: *mut rbmoe_layer, x: *const c_void, x_dtype: i32, tokens: i32, cols: i32,
+                                     valid: *const u8, router_bias: *const f32, residual: *const c_void, block: i32,
+                                     out: *mut c_void, routing: *mut rbmoe_routing, losses: *mut f32) -> c_int;
+    pub fn rbmoe_forward_train_finish(layer: *mut rbmoe_layer) -> c_int;
     pub fn rbmoe_get_losses(layer: *mut rbmoe_layer, aux_loss: *mut f32, z_loss: *mut f32) -> c_int;
     pub fn rbmoe_get_routing(layer: *mut rbmoe_layer, routing: *mut rbmoe_routing) -> c_int;
     pub fn rbmoe_get_expert_rows(layer: *mut rbmoe_layer, hidden: *mut f32, expert_out: *mut f32) -> c_int;
@@ -127,12 +132,16 @@ extern "C" {
                                 grad_input: *mut c_void) -> c_int;
     pub fn rbmoe_backward_block_host(layer: *mut rbmoe_layer, grad_output: *const c_void, tokens: i32, cols: i32,
                                      grad_input: *mut c_void) -> c_int;
+    pub fn rbmoe_backward_train_host(layer: *mut rbmoe_layer, grad_output: *const c_void, dtype: i32, tokens: i32,
+                                     cols: i32, block: i32, grad_input: *mut c_void) -> c_int;
     pub fn rbmoe_zero_grads(layer: *mut rbmoe_layer) -> c_int;
     pub fn rbmoe_get_weight_grad(layer: *mut rbmoe_layer, which: i32, expert: i32, host: *mut f32, rows: i32,
                                  cols: i32) -> c_int;
     pub fn rbmoe_expert_kernel_name(layer: *const rbmoe_layer) -> *const c_char;
     pub fn rbmoe_device_alloc(ctx: *mut rbmoe_ctx, bytes: usize, out: *mut *mut c_void) -> c_int;
     pub fn rbmoe_device_free(ctx: *mut rbmoe_ctx, ptr: *mut c_void) -> c_int;
+    pub fn rbmoe_host_alloc(ctx: *mut rbmoe_ctx, bytes: usize, out: *mut *mut c_void) -> c_int;
+    pub fn rbmoe_host_free(ptr: *mut c_void);
     pub fn rbmoe_copy_to_device(ctx: *mut rbmoe_ctx, dst: *mut c_void, src: *const c_void, bytes: usize) -> c_int;
     pub fn rbmoe_copy_to_host(ctx: *mut rbmoe_ctx, dst: *mut c_void, src: *const c_void, bytes: usize) -> c_int;
     pub fn rbmoe_copy_device(ctx: *mut rbmoe_ctx, dst: *mut c_void, src: *const c_void, bytes: usize) -> c_int;

@@ -66,12 +66,17 @@ SIGNATURES = {
                                      C.c_void_p, C.c_void_p]),
     "rbmoe_forward_timed": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p,
                                       C.c_void_p, C.c_void_p, C.POINTER(C.c_float)]),
+    "rbmoe_forward_train_begin": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p,
+                                            C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p]),
+    "rbmoe_forward_train_finish": (C.c_int, [C.c_void_p]),
     "rbmoe_get_losses": (C.c_int, [C.c_void_p, C.POINTER(C.c_float), C.POINTER(C.c_float)]),
-    "rbmoe_get_routing": (C.c_int, [C.c_void_p, C.POINTER(Routing)]),
+    "rbmoe_get_routing": (C.c_int, [C.c_void_p, C.c_void_p]),  # rbmoe_routing*: the words of a Routing
     "rbmoe_get_expert_rows": (C.c_int, [C.c_void_p, C.POINTER(C.c_float), C.POINTER(C.c_float)]),
     "rbmoe_expert_kernel_name": (C.c_char_p, [C.c_void_p]),
     "rbmoe_device_alloc": (C.c_int, [C.c_void_p, C.c_size_t, C.POINTER(C.c_void_p)]),
     "rbmoe_device_free": (C.c_int, [C.c_void_p, C.c_void_p]),
+    "rbmoe_host_alloc": (C.c_int, [C.c_void_p, C.c_size_t, C.POINTER(C.c_void_p)]),
+    "rbmoe_host_free": (None, [C.c_void_p]),
     "rbmoe_copy_to_device": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]),
     "rbmoe_copy_to_host": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]),
     "rbmoe_copy_device": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]),
@@ -84,6 +89,7 @@ SIGNATURES = {
     "rbmoe_backward_host": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_void_p]),
     "rbmoe_backward_block": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_void_p]),
     "rbmoe_backward_block_host": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_void_p]),
+    "rbmoe_backward_train_host": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_void_p]),
     "rbmoe_zero_grads": (C.c_int, [C.c_void_p]),
     "rbmoe_get_weight_grad": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.POINTER(C.c_float), C.c_int32, C.c_int32]),
     "rbmoe_forward_kernel_times": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p,

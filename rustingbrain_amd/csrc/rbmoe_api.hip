@@ -8,15 +8,18 @@
 // fallback: without a usable GPU every device entry point fails.
 #include "../../include/rbmoe.h"
 
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
 
+#include "host_io.h"
 #include "rbmoe_kernels.h"
 
 using namespace rbmoe;
@@ -52,6 +55,8 @@ hipError_t static_scratch_of(int device, void** out) {
     *out = g_scratch_ptr[device];
     return hipSuccess;
 }
+
+std::atomic<int> g_live_contexts{0};  // the last one to go gives the kept pinned blocks back
 
 thread_local std::string g_global_error;
 
@@ -114,6 +119,9 @@ struct rbmoe_ctx {
     // priority, like the first) forked from and joined to `stream` with two events.  Created on first use.
     hipStream_t side_stream = nullptr;
     hipEvent_t ev_fork = nullptr, ev_fork2 = nullptr, ev_join = nullptr, ev_tables = nullptr;
+    // host calls: the routing of a forward is complete (recorded on `stream`), its tables are in host memory (recorded
+    // on the side stream).  Created with the side stream.
+    hipEvent_t ev_routed = nullptr, ev_fetched = nullptr;
     size_t budget_bytes = 0;
     size_t allocated = 0;
     void* static_scratch = nullptr;  // this device's copy of rbmoe_static_scratch (RBMOE_STATIC_SCRATCH_BYTES)
@@ -175,8 +183,41 @@ struct Work {
     unsigned int* expert_tokens = nullptr;  // [E] the tokens of every expert, one bit a token (decode_front launches), or null
 };
 
+// Host memory of a call that is still under way: a pinned block, or plain memory when the pool is exhausted.
+struct Staging {
+    HostBlock block;
+    std::unique_ptr<unsigned char[]> plain;
+    unsigned char* p = nullptr;
+    bool pinned() const { return block.p != nullptr; }
+    bool take(size_t bytes) {
+        block = HostBlock(bytes);
+        plain.reset();
+        if (!block.p) plain.reset(new (std::nothrow) unsigned char[bytes]);
+        p = block.p ? static_cast<unsigned char*>(block.p) : plain.get();
+        return p != nullptr;
+    }
+    void reset() {
+        block.reset();
+        plain.reset();
+        p = nullptr;
+    }
+};
+
+// The output of a host call between its begin and its finish.
+struct PendingOut {
+    bool any = false;
+    hipStream_t stream = nullptr;
+    Staging in, out;
+    void* user = nullptr;      // where the rows go from out.p once the stream is done (null: they are written in place)
+    size_t elements = 0;
+    bool from_bf16 = false;    // out.p holds bf16 rows and the caller wants f32
+    size_t element_bytes = 0;  // otherwise: a plain copy
+};
+
 struct rbmoe_layer {
     rbmoe_ctx* ctx = nullptr;
+    PendingOut pending;
+    hipEvent_t record_routed = nullptr;  // forward_impl records it once the routing tables are complete
     rbmoe_config cfg{};
     int Fs = 0;       // shared expert width
     // Expert widths as the kernels see them: the matrix-core kernels take whole tiles, so a width between two multiples
@@ -475,6 +516,7 @@ int rbmoe_ctx_create(int32_t device, size_t budget_mib, rbmoe_ctx** out) {
         return hip_fail(nullptr, se, "hipStreamCreateWithFlags");
     }
     ctx->stream = ctx->own_stream;
+    ++g_live_contexts;
     *out = ctx;
     return RBMOE_OK;
 }
@@ -489,11 +531,14 @@ static void ctx_release(rbmoe_ctx* ctx) {
     if (ctx->ev_fork2) (void)hipEventDestroy(ctx->ev_fork2);
     if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
     if (ctx->ev_tables) (void)hipEventDestroy(ctx->ev_tables);
+    if (ctx->ev_routed) (void)hipEventDestroy(ctx->ev_routed);
+    if (ctx->ev_fetched) (void)hipEventDestroy(ctx->ev_fetched);
     if (ctx->own_stream) {
         (void)hipStreamSynchronize(ctx->own_stream);
         (void)hipStreamDestroy(ctx->own_stream);
     }
     delete ctx;
+    if (--g_live_contexts == 0) host_pool_trim();
 }
 
 // Layers keep their context alive: destroying the context while layers exist
@@ -842,11 +887,11 @@ namespace {
 int ensure_side_stream(rbmoe_ctx* ctx) {
     if (ctx->side_stream) return RBMOE_OK;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    // all five or none: a stream without its events would be used as if it were complete
+    // all of them or none: a stream without its events would be used as if it were complete
     hipStream_t st = nullptr;
-    hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+    hipEvent_t ev[6] = {};
     hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
-    for (int i = 0; i < 4 && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
+    for (int i = 0; i < 6 && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
     if (e != hipSuccess) {
         for (hipEvent_t x : ev)
             if (x) (void)hipEventDestroy(x);
@@ -858,6 +903,8 @@ int ensure_side_stream(rbmoe_ctx* ctx) {
     ctx->ev_fork2 = ev[1];
     ctx->ev_join = ev[2];
     ctx->ev_tables = ev[3];
+    ctx->ev_routed = ev[4];
+    ctx->ev_fetched = ev[5];
     return RBMOE_OK;
 }
 
@@ -1077,6 +1124,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
             HIP_TRY(ctx, launch_decode_gemm(d1, wk, s));
             L->replay[RBMOE_STAGE_GATE_UP] = [=](hipStream_t st) { return launch_decode_gemm(d1, wk, st); };
         }
+        if (L->record_routed) HIP_TRY(ctx, hipEventRecord(L->record_routed, s));
         HIP_TRY(ctx, mark(4));
 
         DecodeGemmArgs d2 = d1;
@@ -1226,6 +1274,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     da.perm_slot = (int*)L->perm_slot.p; da.perm_token = (int*)L->perm_token.p; da.inv_pos = (int*)L->inv_pos.p;
     da.xg = gather_in_product ? nullptr : L->xg.p;
     HIP_TRY(ctx, launch_dispatch(da, abf || cast, s));
+    if (L->record_routed) HIP_TRY(ctx, hipEventRecord(L->record_routed, s));
     {
         const bool rows_bf16 = abf || cast;
         L->replay[RBMOE_STAGE_DISPATCH] = [=](hipStream_t st) { return launch_dispatch(da, rows_bf16, st); };
@@ -1357,6 +1406,275 @@ int ensure_block_training_buffers(rbmoe_layer* L) {
     return allocate_plan(L, p, "the norm's backward buffers");
 }
 
+// The backward entry points differentiate the LAST forward, whose shape the reference takes from the cached input
+// (src/moe.rs:349-350).  Here the cache is the layer's own state, so the caller states the shape of its buffers
+// and a mismatch is refused before any of their bytes is read or written.
+int backward_shape_problem(rbmoe_layer* L, int32_t tokens, int32_t cols) {
+    rbmoe_ctx* ctx = L->ctx;
+    char buf[160];
+    if (cols != L->cfg.d_model) {
+        std::snprintf(buf, sizeof buf, "gradient length %d does not match expected length %d", cols, L->cfg.d_model);
+        return fail(ctx, RBMOE_INVALID_INPUT, buf);
+    }
+    if (tokens != L->last_T) {
+        std::snprintf(buf, sizeof buf, "gradient rows %d do not match the %d rows of the last forward pass", tokens,
+                      L->last_T);
+        return fail(ctx, RBMOE_INVALID_INPUT, buf);
+    }
+    return RBMOE_OK;
+}
+
+// ---- host calls -----------------------------------------------------------------------------------------------
+// Rows travel through pinned memory: a copy from pageable memory is cut into pieces that a host thread moves (and
+// rounds, for f32 rows of a bf16 layer) while the DMA engine sends the pieces before; results go to the caller's
+// memory directly when it is one of the library's pinned blocks.
+
+// Bytes of a piece.  Every DMA costs about 8 us beside its bytes and the first piece's host copy is not covered by
+// anything: 4.7 MB from pageable memory take 246 us in pieces of 256 KB, 174 in 512 KB, 148 in 1 MB, 143 in 1.5 MB,
+// 163 in one (the link alone: 90).
+constexpr size_t kCopyPiece = (size_t)1280 << 10;
+
+// `n` elements of the caller's host array to the device; `stage` is room for them in the layer's element type.
+int host_rows_in(rbmoe_ctx* ctx, void* dst, const void* src, size_t n, bool round_to_bf16, size_t es, unsigned char* stage,
+                 bool stage_pinned, hipStream_t s) {
+    if (n == 0) return RBMOE_OK;
+    if (!round_to_bf16 && host_block_holds(src, n * es)) {
+        HIP_TRY(ctx, hipMemcpyAsync(dst, src, n * es, hipMemcpyHostToDevice, s));
+        return RBMOE_OK;
+    }
+    const size_t step = stage_pinned ? kCopyPiece / es : n;
+    for (size_t i = 0; i < n; i += step) {
+        const size_t m = std::min(step, n - i);
+        if (round_to_bf16)
+            host_rows_to_bf16(static_cast<const float*>(src) + i, reinterpret_cast<uint16_t*>(stage) + i, m);
+        else
+            std::memcpy(stage + i * es, static_cast<const unsigned char*>(src) + i * es, m * es);
+        HIP_TRY(ctx, hipMemcpyAsync(static_cast<char*>(dst) + i * es, stage + i * es, m * es, hipMemcpyHostToDevice, s));
+    }
+    return RBMOE_OK;
+}
+
+// Device rows (`es` bytes an element) to the caller's array; what is left to do once the stream has come this far is
+// noted in `po`.
+int host_rows_out(rbmoe_ctx* ctx, const void* src, void* user, size_t n, bool widen_to_f32, size_t es, PendingOut& po,
+                  hipStream_t s) {
+    po.user = nullptr;
+    po.from_bf16 = false;
+    if (n == 0) return RBMOE_OK;
+    const size_t out_bytes = n * (widen_to_f32 ? 4 : es);
+    unsigned char* to = static_cast<unsigned char*>(user);
+    bool pinned = host_block_holds(user, out_bytes);
+    if (!pinned) {
+        if (!po.out.take(out_bytes)) return fail(ctx, RBMOE_OUT_OF_MEMORY, "no host memory for the results");
+        pinned = po.out.pinned();
+        to = po.out.p;
+        po.user = user;
+    }
+    po.elements = n;
+    po.element_bytes = widen_to_f32 ? 4 : es;
+    if (widen_to_f32 && pinned && n % 4 == 0 && reinterpret_cast<uintptr_t>(to) % 16 == 0) {
+        HIP_TRY(ctx, launch_widen_rows(src, reinterpret_cast<float*>(to), n, s));
+        return RBMOE_OK;
+    }
+    if (widen_to_f32) {  // bf16 rows to host memory of their own, widened by the host at the end
+        if (po.user == nullptr) {
+            if (!po.out.take(n * 2)) return fail(ctx, RBMOE_OUT_OF_MEMORY, "no host memory for the results");
+            to = po.out.p;
+            po.user = user;
+        }
+        po.from_bf16 = true;
+    }
+    HIP_TRY(ctx, hipMemcpyAsync(to, src, n * es, hipMemcpyDeviceToHost, s));
+    return RBMOE_OK;
+}
+
+int host_out_finish(rbmoe_ctx* ctx, PendingOut& po) {
+    if (!po.any) return RBMOE_OK;
+    const hipError_t e = hipStreamSynchronize(po.stream);
+    if (e == hipSuccess && po.user != nullptr) {
+        if (po.from_bf16) host_rows_to_f32(reinterpret_cast<const uint16_t*>(po.out.p), static_cast<float*>(po.user), po.elements);
+        else std::memcpy(po.user, po.out.p, po.elements * po.element_bytes);
+    }
+    po.any = false;
+    po.user = nullptr;
+    po.in.reset();
+    po.out.reset();
+    if (e != hipSuccess) return hip_fail(ctx, e, "hipStreamSynchronize");
+    return RBMOE_OK;
+}
+
+int host_forward_finish(rbmoe_layer* L) { return host_out_finish(L->ctx, L->pending); }
+
+// The routing tables of the last forward and its two losses to host memory, by one launch that writes them there
+// (arrays outside the library's pinned blocks through `stage`).  The copies still to be made once the stream has come
+// this far are left in `after`.
+struct TableCopy {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+int fetch_tables(rbmoe_layer* L, const rbmoe_routing* r, float* losses, Staging& stage, std::vector<TableCopy>& after, hipStream_t s) {
+    rbmoe_ctx* ctx = L->ctx;
+    const int T = L->last_T, E = L->cfg.num_experts, k = L->cfg.experts_per_token;
+    const size_t S = (size_t)T * k;
+    const Work& w = L->last;
+    struct Want {
+        void* dst;
+        const void* src;
+        size_t words;
+    } want[9];
+    int nw = 0;
+    auto add = [&](void* dst, const void* src, size_t words) {
+        if (dst && words) want[nw++] = {dst, src, words};
+    };
+    if (r) {
+        add(r->counts, w.counts, (size_t)E);
+        add(r->offsets, w.offsets, (size_t)E + 1);
+        add(r->expert_of, w.expert_of, S);
+        add(r->gate_of, w.gate_of, S);
+        add(r->perm_slot, w.perm_slot, S);
+        add(r->perm_token, w.perm_token, S);
+        add(r->probabilities, w.P, (size_t)T * E);
+        add(r->log_sum_exp, w.lse, (size_t)T);
+    }
+    add(losses, w.losses, 2);
+    size_t staged = 0;
+    bool direct[9];
+    for (int i = 0; i < nw; ++i) {
+        direct[i] = reinterpret_cast<uintptr_t>(want[i].dst) % 4 == 0 && host_block_holds(want[i].dst, want[i].words * 4);
+        if (!direct[i]) staged += want[i].words * 4;
+    }
+    if (staged && !stage.take(staged)) return fail(ctx, RBMOE_OUT_OF_MEMORY, "no host memory for the routing tables");
+    CopySegment seg[kMaxCopySegments];
+    int ns = 0;
+    size_t at = 0;
+    for (int i = 0; i < nw; ++i) {
+        void* to = want[i].dst;
+        if (!direct[i]) {
+            to = stage.p + at;
+            at += want[i].words * 4;
+            after.push_back({want[i].dst, to, want[i].words * 4});
+        }
+        if (direct[i] || stage.pinned()) seg[ns++] = {want[i].src, to, (unsigned int)want[i].words};
+        else HIP_TRY(ctx, hipMemcpyAsync(to, want[i].src, want[i].words * 4, hipMemcpyDeviceToHost, s));
+    }
+    HIP_TRY(ctx, launch_copy_segments(seg, ns, s));
+    return RBMOE_OK;
+}
+
+// forward_train (or the block step) on host rows.  Returns when the routing tables and losses asked for are in place;
+// `out` is complete after host_forward_finish.  `io`: dtype of x, residual and out, the layer's own or f32.
+int host_forward_begin(rbmoe_layer* L, const void* x, int io, int T, int cols, const uint8_t* valid, const float* router_bias,
+                       const void* residual, bool block, void* out, rbmoe_routing* routing, float* losses) {
+    rbmoe_ctx* ctx = L->ctx;
+    const rbmoe_config& c = L->cfg;
+    if (const int rc = host_forward_finish(L)) return rc;  // (a call begun and never finished)
+    if (block && !L->norm_set) return fail(ctx, RBMOE_INVALID_CONFIG, "the feed-forward norm has not been set");
+    if (cols != c.d_model) {
+        char buf[120];
+        std::snprintf(buf, sizeof buf, "input length %d does not match expected length %d", cols, c.d_model);
+        return fail(ctx, RBMOE_INVALID_INPUT, buf);
+    }
+    if (io != c.act_dtype && io != RBMOE_F32) return fail(ctx, RBMOE_INVALID_CONFIG, "rows must be f32 or the layer's own dtype");
+    if (T < 0 || T > L->max_T) return fail(ctx, RBMOE_INVALID_INPUT, "token count outside [0, max_tokens]");
+    if (T > 0 && (!x || !out)) return fail(ctx, RBMOE_NULL_POINTER, "x or out is NULL");
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    const bool convert = io != c.act_dtype;  // f32 host rows of a bf16 layer
+    const size_t as = dtype_size(c.act_dtype), n = (size_t)T * c.d_model, nbytes = n * as;
+    hipStream_t s = ctx->stream;
+    PendingOut& po = L->pending;
+    struct Abandon {  // an error on the way: nothing may still be using the staging memory when it is given back
+        rbmoe_ctx* ctx;
+        PendingOut* po;
+        ~Abandon() {
+            if (!po) return;
+            po->user = nullptr;
+            (void)host_out_finish(ctx, *po);
+        }
+    } abandon{ctx, &po};
+    po.any = true;
+    po.stream = s;
+    const size_t row_room = (nbytes + 255) & ~(size_t)255;
+    const size_t res_at = row_room, valid_at = res_at + (residual ? row_room : 0), bias_at = valid_at + (((size_t)T + 255) & ~(size_t)255);
+    if (!po.in.take(bias_at + (size_t)c.num_experts * 4)) return fail(ctx, RBMOE_OUT_OF_MEMORY, "no host memory for the rows");
+    if (valid && T > 0) {
+        std::memcpy(po.in.p + valid_at, valid, (size_t)T);
+        HIP_TRY(ctx, hipMemcpyAsync(L->st_valid.p, po.in.p + valid_at, (size_t)T, hipMemcpyHostToDevice, s));
+    }
+    if (router_bias) {
+        std::memcpy(po.in.p + bias_at, router_bias, (size_t)c.num_experts * 4);
+        HIP_TRY(ctx, hipMemcpyAsync(L->st_bias.p, po.in.p + bias_at, (size_t)c.num_experts * 4, hipMemcpyHostToDevice, s));
+    }
+    if (const int rc = host_rows_in(ctx, L->st_x.p, x, n, convert, as, po.in.p, po.in.pinned(), s)) return rc;
+    if (residual)
+        if (const int rc = host_rows_in(ctx, L->st_res.p, residual, n, convert, as, po.in.p + res_at, po.in.pinned(), s)) return rc;
+    const uint8_t* const dvalid = valid ? (const uint8_t*)L->st_valid.p : nullptr;
+    const float* const dbias = router_bias ? (const float*)L->st_bias.p : nullptr;
+    // the tables are fetched on the side stream, beside the expert products
+    const bool tables = routing != nullptr || losses != nullptr;
+    if (tables) {
+        if (const int rc = ensure_side_stream(ctx)) return rc;
+        L->record_routed = ctx->ev_routed;
+    }
+    int rc = block ? rbmoe_forward_block(L, L->st_x.p, T, cols, dvalid, dbias, L->st_out.p)
+                   : forward_impl(L, L->st_x.p, T, cols, dvalid, dbias, residual ? L->st_res.p : nullptr, L->st_out.p, 0);
+    L->record_routed = nullptr;
+    if (rc != RBMOE_OK) return rc;
+    Staging stage;
+    std::vector<TableCopy> after;
+    if (tables) {
+        HIP_TRY(ctx, hipStreamWaitEvent(ctx->side_stream, ctx->ev_routed, 0));
+        rc = fetch_tables(L, routing, losses, stage, after, ctx->side_stream);
+        const hipError_t e = hipEventRecord(ctx->ev_fetched, ctx->side_stream);
+        if (rc != RBMOE_OK || e != hipSuccess) {
+            (void)hipStreamSynchronize(ctx->side_stream);
+            return rc != RBMOE_OK ? rc : hip_fail(ctx, e, "hipEventRecord");
+        }
+    }
+    rc = host_rows_out(ctx, L->st_out.p, out, n, convert, as, po, s);
+    if (tables) {
+        const hipError_t e = hipEventSynchronize(ctx->ev_fetched);
+        if (rc == RBMOE_OK && e != hipSuccess) rc = hip_fail(ctx, e, "hipEventSynchronize");
+        for (const TableCopy& t : after) std::memcpy(t.dst, t.src, t.bytes);
+    }
+    if (rc != RBMOE_OK) return rc;
+    abandon.po = nullptr;
+    return RBMOE_OK;
+}
+
+// backward (of the layer, or of the block step) on host gradients; `io` as in host_forward_begin.
+int host_backward(rbmoe_layer* L, const void* grad_output, int io, int tokens, int cols, bool block, void* grad_input) {
+    rbmoe_ctx* ctx = L->ctx;
+    const rbmoe_config& c = L->cfg;
+    if (!L->training) return fail(ctx, RBMOE_INVALID_CONFIG, "training is not enabled on this layer");
+    if (block && !L->norm_set) return fail(ctx, RBMOE_INVALID_CONFIG, "the feed-forward norm has not been set");
+    if (!block && L->last_T < 0) return fail(ctx, RBMOE_INVALID_INPUT, "no forward pass has run yet");
+    if (block && (L->last_T < 0 || !L->last_was_block))
+        return fail(ctx, RBMOE_INVALID_INPUT, "the last forward pass was not rbmoe_forward_block");
+    if (const int rc = backward_shape_problem(L, tokens, cols)) return rc;  // before any byte of the buffers is touched
+    if (io != c.act_dtype && io != RBMOE_F32) return fail(ctx, RBMOE_INVALID_CONFIG, "rows must be f32 or the layer's own dtype");
+    const int T = L->last_T;
+    if (T == 0) return RBMOE_OK;
+    if (!grad_output || !grad_input) return fail(ctx, RBMOE_NULL_POINTER, "grad_output or grad_input is NULL");
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    if (const int rc = host_forward_finish(L)) return rc;
+    const bool convert = io != c.act_dtype;
+    const size_t as = dtype_size(c.act_dtype), n = (size_t)T * c.d_model;
+    hipStream_t s = ctx->stream;
+    PendingOut po;
+    po.any = true;
+    po.stream = s;
+    if (!po.in.take(n * as)) return fail(ctx, RBMOE_OUT_OF_MEMORY, "no host memory for the rows");
+    int rc = host_rows_in(ctx, L->st_gout.p, grad_output, n, convert, as, po.in.p, po.in.pinned(), s);
+    if (rc == RBMOE_OK)
+        rc = block ? rbmoe_backward_block(L, L->st_gout.p, tokens, cols, L->st_gin.p)
+                   : rbmoe_backward(L, L->st_gout.p, tokens, cols, L->st_gin.p);
+    if (rc == RBMOE_OK) rc = host_rows_out(ctx, L->st_gin.p, grad_input, n, convert, as, po, s);
+    if (rc != RBMOE_OK) po.user = nullptr;
+    const int rc2 = host_out_finish(ctx, po);
+    return rc != RBMOE_OK ? rc : rc2;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1438,33 +1756,20 @@ int rbmoe_replay_stage(rbmoe_layer* L, int32_t stage, int32_t launches, float* m
 int rbmoe_forward_host(rbmoe_layer* L, const void* x, int32_t T, int32_t cols, const uint8_t* valid,
                        const float* router_bias, const void* residual, void* out) {
     if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
-    rbmoe_ctx* ctx = L->ctx;
-    const rbmoe_config& c = L->cfg;
-    if (cols != c.d_model) {
-        char buf[120];
-        std::snprintf(buf, sizeof buf, "input length %d does not match expected length %d", cols, c.d_model);
-        return fail(ctx, RBMOE_INVALID_INPUT, buf);
-    }
-    if (T < 0 || T > L->max_T) return fail(ctx, RBMOE_INVALID_INPUT, "token count outside [0, max_tokens]");
-    if (T > 0 && (!x || !out)) return fail(ctx, RBMOE_NULL_POINTER, "x or out is NULL");
-    HIP_TRY(ctx, hipSetDevice(ctx->device));
-    const size_t as = dtype_size(c.act_dtype);
-    const size_t nbytes = (size_t)T * c.d_model * as;
-    hipStream_t s = ctx->stream;
-    if (T > 0) {
-        HIP_TRY(ctx, hipMemcpyAsync(L->st_x.p, x, nbytes, hipMemcpyHostToDevice, s));
-        if (valid) HIP_TRY(ctx, hipMemcpyAsync(L->st_valid.p, valid, (size_t)T, hipMemcpyHostToDevice, s));
-        if (residual) HIP_TRY(ctx, hipMemcpyAsync(L->st_res.p, residual, nbytes, hipMemcpyHostToDevice, s));
-    }
-    if (router_bias)
-        HIP_TRY(ctx, hipMemcpyAsync(L->st_bias.p, router_bias, (size_t)c.num_experts * 4, hipMemcpyHostToDevice, s));
-    int rc = forward_impl(L, L->st_x.p, T, cols, valid ? (const uint8_t*)L->st_valid.p : nullptr,
-                          router_bias ? (const float*)L->st_bias.p : nullptr, residual ? L->st_res.p : nullptr,
-                          L->st_out.p, 0);
-    if (rc != RBMOE_OK) return rc;
-    if (T > 0) HIP_TRY(ctx, hipMemcpyAsync(out, L->st_out.p, nbytes, hipMemcpyDeviceToHost, s));
-    HIP_TRY(ctx, hipStreamSynchronize(s));
-    return RBMOE_OK;
+    const int rc = host_forward_begin(L, x, L->cfg.act_dtype, T, cols, valid, router_bias, residual, false, out, nullptr, nullptr);
+    return rc == RBMOE_OK ? host_forward_finish(L) : rc;
+}
+
+int rbmoe_forward_train_begin(rbmoe_layer* L, const void* x, int32_t x_dtype, int32_t T, int32_t cols, const uint8_t* valid,
+                              const float* router_bias, const void* residual, int32_t block, void* out,
+                              rbmoe_routing* routing, float* losses) {
+    if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
+    return host_forward_begin(L, x, x_dtype, T, cols, valid, router_bias, residual, block != 0, out, routing, losses);
+}
+
+int rbmoe_forward_train_finish(rbmoe_layer* L) {
+    if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
+    return host_forward_finish(L);
 }
 
 // ---------------------------------------------------------------------------
@@ -1520,31 +1825,8 @@ int rbmoe_forward_block(rbmoe_layer* L, const void* x, int32_t T, int32_t cols, 
 int rbmoe_forward_block_host(rbmoe_layer* L, const void* x, int32_t T, int32_t cols, const uint8_t* valid,
                              const float* router_bias, void* out) {
     if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
-    rbmoe_ctx* ctx = L->ctx;
-    const rbmoe_config& c = L->cfg;
-    if (!L->norm_set) return fail(ctx, RBMOE_INVALID_CONFIG, "the feed-forward norm has not been set");
-    if (cols != c.d_model) {
-        char buf[120];
-        std::snprintf(buf, sizeof buf, "input length %d does not match expected length %d", cols, c.d_model);
-        return fail(ctx, RBMOE_INVALID_INPUT, buf);
-    }
-    if (T < 0 || T > L->max_T) return fail(ctx, RBMOE_INVALID_INPUT, "token count outside [0, max_tokens]");
-    if (T > 0 && (!x || !out)) return fail(ctx, RBMOE_NULL_POINTER, "x or out is NULL");
-    HIP_TRY(ctx, hipSetDevice(ctx->device));
-    const size_t nbytes = (size_t)T * c.d_model * dtype_size(c.act_dtype);
-    hipStream_t s = ctx->stream;
-    if (T > 0) {
-        HIP_TRY(ctx, hipMemcpyAsync(L->st_x.p, x, nbytes, hipMemcpyHostToDevice, s));
-        if (valid) HIP_TRY(ctx, hipMemcpyAsync(L->st_valid.p, valid, (size_t)T, hipMemcpyHostToDevice, s));
-    }
-    if (router_bias)
-        HIP_TRY(ctx, hipMemcpyAsync(L->st_bias.p, router_bias, (size_t)c.num_experts * 4, hipMemcpyHostToDevice, s));
-    int rc = rbmoe_forward_block(L, L->st_x.p, T, cols, valid ? (const uint8_t*)L->st_valid.p : nullptr,
-                                 router_bias ? (const float*)L->st_bias.p : nullptr, L->st_out.p);
-    if (rc != RBMOE_OK) return rc;
-    if (T > 0) HIP_TRY(ctx, hipMemcpyAsync(out, L->st_out.p, nbytes, hipMemcpyDeviceToHost, s));
-    HIP_TRY(ctx, hipStreamSynchronize(s));
-    return RBMOE_OK;
+    const int rc = host_forward_begin(L, x, L->cfg.act_dtype, T, cols, valid, router_bias, nullptr, true, out, nullptr, nullptr);
+    return rc == RBMOE_OK ? host_forward_finish(L) : rc;
 }
 
 // ---------------------------------------------------------------------------
@@ -1699,24 +1981,6 @@ int rbmoe_zero_grads(rbmoe_layer* L) {
     HIP_TRY(ctx, launch_fill_f32((float*)L->g_router.p, 0.0f, (long long)(L->g_router.bytes / 4), ctx->stream));
     if (L->g_norm.p) HIP_TRY(ctx, launch_fill_f32((float*)L->g_norm.p, 0.0f, (long long)(L->g_norm.bytes / 4), ctx->stream));
     L->grads_clear = true;
-    return RBMOE_OK;
-}
-
-// The backward entry points differentiate the LAST forward, whose shape the reference takes from the cached input
-// (src/moe.rs:349-350).  Here the cache is the layer's own state, so the caller states the shape of its buffers
-// and a mismatch is refused before any of their bytes is read or written.
-static int backward_shape_problem(rbmoe_layer* L, int32_t tokens, int32_t cols) {
-    rbmoe_ctx* ctx = L->ctx;
-    char buf[160];
-    if (cols != L->cfg.d_model) {
-        std::snprintf(buf, sizeof buf, "gradient length %d does not match expected length %d", cols, L->cfg.d_model);
-        return fail(ctx, RBMOE_INVALID_INPUT, buf);
-    }
-    if (tokens != L->last_T) {
-        std::snprintf(buf, sizeof buf, "gradient rows %d do not match the %d rows of the last forward pass", tokens,
-                      L->last_T);
-        return fail(ctx, RBMOE_INVALID_INPUT, buf);
-    }
     return RBMOE_OK;
 }
 
@@ -1879,21 +2143,13 @@ int rbmoe_backward(rbmoe_layer* L, const void* grad_output, int32_t tokens, int3
 
 int rbmoe_backward_host(rbmoe_layer* L, const void* grad_output, int32_t tokens, int32_t cols, void* grad_input) {
     if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
-    rbmoe_ctx* ctx = L->ctx;
-    if (!L->training) return fail(ctx, RBMOE_INVALID_CONFIG, "training is not enabled on this layer");
-    if (L->last_T < 0) return fail(ctx, RBMOE_INVALID_INPUT, "no forward pass has run yet");
-    if (const int rc = backward_shape_problem(L, tokens, cols)) return rc;  // before any byte of the buffers is touched
-    const int T = L->last_T;
-    if (T == 0) return RBMOE_OK;
-    if (!grad_output || !grad_input) return fail(ctx, RBMOE_NULL_POINTER, "grad_output or grad_input is NULL");
-    const size_t nbytes = (size_t)T * L->cfg.d_model * dtype_size(L->cfg.act_dtype);
-    HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, hipMemcpyAsync(L->st_gout.p, grad_output, nbytes, hipMemcpyHostToDevice, ctx->stream));
-    int rc = rbmoe_backward(L, L->st_gout.p, tokens, cols, L->st_gin.p);
-    if (rc != RBMOE_OK) return rc;
-    HIP_TRY(ctx, hipMemcpyAsync(grad_input, L->st_gin.p, nbytes, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    return RBMOE_OK;
+    return host_backward(L, grad_output, L->cfg.act_dtype, tokens, cols, false, grad_input);
+}
+
+int rbmoe_backward_train_host(rbmoe_layer* L, const void* grad_output, int32_t dtype, int32_t tokens, int32_t cols,
+                              int32_t block, void* grad_input) {
+    if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
+    return host_backward(L, grad_output, dtype, tokens, cols, block != 0, grad_input);
 }
 
 int rbmoe_backward_block(rbmoe_layer* L, const void* grad_output, int32_t tokens, int32_t cols, void* grad_input) {
@@ -1920,23 +2176,7 @@ int rbmoe_backward_block(rbmoe_layer* L, const void* grad_output, int32_t tokens
 int rbmoe_backward_block_host(rbmoe_layer* L, const void* grad_output, int32_t tokens, int32_t cols,
                               void* grad_input) {
     if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
-    rbmoe_ctx* ctx = L->ctx;
-    if (!L->training) return fail(ctx, RBMOE_INVALID_CONFIG, "training is not enabled on this layer");
-    if (!L->norm_set) return fail(ctx, RBMOE_INVALID_CONFIG, "the feed-forward norm has not been set");
-    if (L->last_T < 0 || !L->last_was_block)
-        return fail(ctx, RBMOE_INVALID_INPUT, "the last forward pass was not rbmoe_forward_block");
-    if (const int rc = backward_shape_problem(L, tokens, cols)) return rc;  // before any byte of the buffers is touched
-    const int T = L->last_T;
-    if (T == 0) return RBMOE_OK;
-    if (!grad_output || !grad_input) return fail(ctx, RBMOE_NULL_POINTER, "grad_output or grad_input is NULL");
-    const size_t nbytes = (size_t)T * L->cfg.d_model * dtype_size(L->cfg.act_dtype);
-    HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, hipMemcpyAsync(L->st_gout.p, grad_output, nbytes, hipMemcpyHostToDevice, ctx->stream));
-    const int rc = rbmoe_backward_block(L, L->st_gout.p, tokens, cols, L->st_gin.p);
-    if (rc != RBMOE_OK) return rc;
-    HIP_TRY(ctx, hipMemcpyAsync(grad_input, L->st_gin.p, nbytes, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    return RBMOE_OK;
+    return host_backward(L, grad_output, L->cfg.act_dtype, tokens, cols, true, grad_input);
 }
 
 int rbmoe_get_weight_grad(rbmoe_layer* L, int32_t which, int32_t expert, float* host, int32_t rows, int32_t cols) {
@@ -1987,21 +2227,43 @@ int rbmoe_get_weight_grad(rbmoe_layer* L, int32_t which, int32_t expert, float* 
         std::memset(host, 0, want_rows * want_cols * 4);
         return RBMOE_OK;
     }
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    if (pitch == 0 || pitch == want_cols)
-        HIP_TRY(ctx, hipMemcpy(host, src, want_rows * want_cols * 4, hipMemcpyDeviceToHost));
+    hipStream_t s = ctx->stream;
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    const size_t bytes = want_rows * want_cols * 4;
+    if (pitch == 0) pitch = want_cols;
+    if (host_block_holds(host, bytes) && reinterpret_cast<uintptr_t>(host) % 4 == 0) {
+        // straight into the caller's pinned block, behind whatever the stream still has to do
+        if (pitch == want_cols) HIP_TRY(ctx, hipMemcpyAsync(host, src, bytes, hipMemcpyDeviceToHost, s));
+        else HIP_TRY(ctx, launch_copy_rows(src, pitch, host, (int)want_rows, (int)want_cols, s));
+        HIP_TRY(ctx, hipStreamSynchronize(s));
+        return RBMOE_OK;
+    }
+    HIP_TRY(ctx, hipStreamSynchronize(s));
+    if (pitch == want_cols)
+        HIP_TRY(ctx, hipMemcpy(host, src, bytes, hipMemcpyDeviceToHost));
     else
         HIP_TRY(ctx, hipMemcpy2D(host, want_cols * 4, src, pitch * 4, want_cols * 4, want_rows, hipMemcpyDeviceToHost));
     return RBMOE_OK;
 }
 
-int rbmoe_get_losses(rbmoe_layer* L, float* aux_loss, float* z_loss) {
-    if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
+// Both getters: one launch on the context's stream, one wait.
+static int get_tables(rbmoe_layer* L, const rbmoe_routing* r, float* losses) {
     rbmoe_ctx* ctx = L->ctx;
     if (L->last_T < 0) return fail(ctx, RBMOE_INVALID_INPUT, "no forward pass has run yet");
-    float v[2] = {0.f, 0.f};
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    Staging stage;
+    std::vector<TableCopy> after;
+    const int rc = fetch_tables(L, r, losses, stage, after, ctx->stream);
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    HIP_TRY(ctx, hipMemcpy(v, L->last.losses, 8, hipMemcpyDeviceToHost));
+    if (rc != RBMOE_OK) return rc;
+    for (const TableCopy& t : after) std::memcpy(t.dst, t.src, t.bytes);
+    return RBMOE_OK;
+}
+
+int rbmoe_get_losses(rbmoe_layer* L, float* aux_loss, float* z_loss) {
+    if (!L) return fail(nullptr, RBMOE_NULL_POINTER, "layer is NULL");
+    float v[2] = {0.f, 0.f};
+    if (const int rc = get_tables(L, nullptr, v)) return rc;
     if (aux_loss) *aux_loss = v[0];
     if (z_loss) *z_loss = v[1];
     return RBMOE_OK;
@@ -2009,23 +2271,7 @@ int rbmoe_get_losses(rbmoe_layer* L, float* aux_loss, float* z_loss) {
 
 int rbmoe_get_routing(rbmoe_layer* L, rbmoe_routing* r) {
     if (!L || !r) return fail(L ? L->ctx : nullptr, RBMOE_NULL_POINTER, "layer or routing is NULL");
-    rbmoe_ctx* ctx = L->ctx;
-    if (L->last_T < 0) return fail(ctx, RBMOE_INVALID_INPUT, "no forward pass has run yet");
-    const int T = L->last_T, E = L->cfg.num_experts, k = L->cfg.experts_per_token;
-    const size_t S = (size_t)T * k;
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    const Work& w = L->last;
-    if (r->counts) HIP_TRY(ctx, hipMemcpy(r->counts, w.counts, (size_t)E * 4, hipMemcpyDeviceToHost));
-    if (r->offsets) HIP_TRY(ctx, hipMemcpy(r->offsets, w.offsets, (size_t)(E + 1) * 4, hipMemcpyDeviceToHost));
-    if (S == 0) return RBMOE_OK;
-    if (r->expert_of) HIP_TRY(ctx, hipMemcpy(r->expert_of, w.expert_of, S * 4, hipMemcpyDeviceToHost));
-    if (r->gate_of) HIP_TRY(ctx, hipMemcpy(r->gate_of, w.gate_of, S * 4, hipMemcpyDeviceToHost));
-    if (r->perm_slot) HIP_TRY(ctx, hipMemcpy(r->perm_slot, w.perm_slot, S * 4, hipMemcpyDeviceToHost));
-    if (r->perm_token) HIP_TRY(ctx, hipMemcpy(r->perm_token, w.perm_token, S * 4, hipMemcpyDeviceToHost));
-    if (r->probabilities)
-        HIP_TRY(ctx, hipMemcpy(r->probabilities, w.P, (size_t)T * E * 4, hipMemcpyDeviceToHost));
-    if (r->log_sum_exp) HIP_TRY(ctx, hipMemcpy(r->log_sum_exp, w.lse, (size_t)T * 4, hipMemcpyDeviceToHost));
-    return RBMOE_OK;
+    return get_tables(L, r, nullptr);
 }
 
 int rbmoe_get_expert_rows(rbmoe_layer* L, float* hidden, float* expert_out) {
@@ -2088,6 +2334,18 @@ int rbmoe_device_free(rbmoe_ctx* ctx, void* ptr) {
     if (!ctx) return fail(nullptr, RBMOE_NULL_POINTER, "ctx is NULL");
     if (ptr) HIP_TRY(ctx, hipFree(ptr));
     return RBMOE_OK;
+}
+
+int rbmoe_host_alloc(rbmoe_ctx* ctx, size_t bytes, void** out) {
+    if (!ctx || !out) return fail(ctx, RBMOE_NULL_POINTER, "ctx or out is NULL");
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    *out = host_block_take(bytes ? bytes : 1);
+    if (!*out) return fail(ctx, RBMOE_OUT_OF_MEMORY, "the pool of pinned host memory is exhausted");
+    return RBMOE_OK;
+}
+
+void rbmoe_host_free(void* ptr) {
+    if (ptr) host_block_give(ptr);
 }
 
 int rbmoe_copy_to_device(rbmoe_ctx* ctx, void* dst, const void* src, size_t bytes) {

@@ -15,13 +15,14 @@ arrays (or raw device pointers) across the C ABI.
 from __future__ import annotations
 
 import ctypes as C
+import gc
+import weakref
 from dataclasses import dataclass, replace
 from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
 
 from . import _lib as L
-from .synth import bf16_bits_to_f32, f32_to_bf16_bits
 
 DEFAULT_AUX_LOSS_WEIGHT = 0.01       # reference src/moe.rs:20
 DEFAULT_ROUTER_Z_LOSS_WEIGHT = 1e-3  # reference src/moe.rs:23
@@ -163,6 +164,9 @@ class Layout:
 
 
 # --------------------------------------------------------------------------- device
+_PINNED_FROM = 16 << 10  # bytes: smaller results are cheaper to copy twice than to look after
+
+
 class Device:
     """One GPU with a memory budget: the role of the reference's ``CudaDevice``
     handle (src/param.rs:86-190).  Fails closed when no GPU is usable."""
@@ -182,6 +186,20 @@ class Device:
 
     def synchronize(self) -> None:
         _check(self._lib.rbmoe_synchronize(self.handle), self.handle)
+
+    def empty(self, shape, dtype) -> np.ndarray:
+        """An uninitialised array for results.  Large ones lie in pinned memory from the library's pool, which the GPU
+        fills directly; the block goes back to the pool with the last reference to the array or a view of it."""
+        dtype = np.dtype(dtype)
+        nbytes = int(np.prod(shape, dtype=np.int64)) * dtype.itemsize
+        if nbytes < _PINNED_FROM:
+            return np.empty(shape, dtype)
+        p = C.c_void_p()
+        if self._lib.rbmoe_host_alloc(self.handle, nbytes, C.byref(p)) != L.OK:
+            return np.empty(shape, dtype)  # the pool is exhausted
+        block = (C.c_ubyte * nbytes).from_address(p.value)
+        weakref.finalize(block, self._lib.rbmoe_host_free, p).atexit = False
+        return np.frombuffer(block, dtype).reshape(shape)
 
     def close(self) -> None:
         if self.handle:
@@ -232,6 +250,43 @@ class MoeCache:
     @property
     def expert_slots(self) -> List[np.ndarray]:
         return [self.perm_slot[self.offsets[e]:self.offsets[e + 1]] for e in range(len(self.counts))]
+
+
+class _Tables:
+    """The host arrays one forward's routing tables are fetched into, cut out of one allocation."""
+
+    def __init__(self, layer: "MoeLayer", tokens: int):
+        E, k = layer.config.num_experts, layer.config.experts_per_token
+        S = tokens * k
+        sizes = (S, S, E, E + 1, S, S, tokens * E, tokens, 2)
+        words = layer.device.empty((sum(sizes),), np.int32)
+        at, ptr, parts, ptrs = 0, words.ctypes.data, [], []
+        for n in sizes:
+            parts.append(words[at:at + n])
+            ptrs.append(ptr + 4 * at)
+            at += n
+        self.expert_of, gate_of, self.counts, self.offsets, self.perm_slot, self.perm_token, prob, lse, losses = parts
+        self.gate_of, self.log_sum_exp, self.losses = (a.view(np.float32) for a in (gate_of, lse, losses))
+        self.probabilities = prob.view(np.float32).reshape(tokens, E)
+        self.k = k
+        self.c = np.array(ptrs[:8], np.uint64)  # the words of an L.Routing
+        self.losses_ptr = ptrs[8]
+
+    def cache(self, valid_tokens: Optional[int]) -> MoeCache:
+        R = int(self.offsets[-1])
+        if valid_tokens is None:
+            valid_tokens = R // self.k
+        # (thousands of tuples in one go: the collector would walk the young ones several times over, for nothing)
+        collecting = gc.isenabled()
+        gc.disable()
+        try:
+            assignments = list(zip(self.expert_of.tolist(), self.gate_of.tolist()))
+        finally:
+            if collecting:
+                gc.enable()
+        aux, z = self.losses.tolist()
+        return MoeCache(assignments, self.expert_of, self.gate_of, self.counts, self.offsets, self.perm_slot[:R],
+                        self.perm_token[:R], self.probabilities, self.log_sum_exp, valid_tokens, aux, z)
 
 
 # --------------------------------------------------------------------------- layer
@@ -344,16 +399,15 @@ class MoeLayer:
                 self.set_shared(w["gate"], w["up"], w["down"])
 
     # ---- forward
-    def _to_act(self, a: np.ndarray) -> np.ndarray:
-        a = np.ascontiguousarray(a, dtype=np.float32)
-        return f32_to_bf16_bits(a).reshape(a.shape) if self.act_dtype == "bf16" else a
-
     def forward(self, input: np.ndarray) -> np.ndarray:
         return self.forward_train(input, Layout())[0]
 
     def forward_train(self, input: np.ndarray, layout: Layout = Layout(),
                       router_bias: Optional[np.ndarray] = None,
                       residual: Optional[np.ndarray] = None) -> Tuple[np.ndarray, MoeCache]:
+        return self._forward_host(input, layout, router_bias, residual, False)
+
+    def _forward_host(self, input, layout: Layout, router_bias, residual, block: bool) -> Tuple[np.ndarray, MoeCache]:
         input = np.asarray(input)
         if input.ndim != 2:
             raise InvalidInput("input must be a [tokens, d_model] matrix")
@@ -363,25 +417,28 @@ class MoeLayer:
             raise InvalidInput(f"input length {cols} does not match expected length {self._d_model}",
                                expected=self._d_model, actual=cols)
         layout.check(rows)
-        x = self._to_act(input)
-        out = np.empty_like(x)
+        x = np.ascontiguousarray(input, dtype=np.float32)  # (a bf16 layer's rows are rounded by the library)
+        out = self.device.empty((rows, cols), np.float32)
         vp = bp = rp = None
         valid = None
         if layout.valid is not None:
-            valid = np.ascontiguousarray(np.asarray(layout.valid, dtype=bool).astype(np.uint8))
-            vp = valid.ctypes.data_as(C.c_void_p)
+            valid = np.ascontiguousarray(np.asarray(layout.valid, dtype=bool).view(np.uint8))
+            vp = valid.ctypes.data
         if router_bias is not None:
             router_bias = np.ascontiguousarray(router_bias, dtype=np.float32)
-            bp = router_bias.ctypes.data_as(C.c_void_p)
+            bp = router_bias.ctypes.data
         if residual is not None:
-            residual = self._to_act(residual)
-            rp = residual.ctypes.data_as(C.c_void_p)
-        _check(self._lib.rbmoe_forward_host(self.handle, x.ctypes.data_as(C.c_void_p), rows, cols, vp, bp, rp,
-                                            out.ctypes.data_as(C.c_void_p)), self.device.handle)
-        if self.act_dtype == "bf16":
-            out = bf16_bits_to_f32(out).reshape(rows, cols)
-        valid_tokens = rows if valid is None else int(valid.sum())
-        return out, self.cache(rows, valid_tokens)
+            residual = np.ascontiguousarray(residual, dtype=np.float32)
+            rp = residual.ctypes.data
+        t = _Tables(self, rows)
+        _check(self._lib.rbmoe_forward_train_begin(self.handle, x.ctypes.data, L.F32, rows, cols, vp, bp, rp, int(block),
+                                                   out.ctypes.data, t.c.ctypes.data, t.losses_ptr), self.device.handle)
+        try:  # the tables are here; the expert products and the rows are still on their way
+            cache = t.cache(rows if valid is None else int(np.count_nonzero(valid)))
+        finally:
+            rc = self._lib.rbmoe_forward_train_finish(self.handle)
+        _check(rc, self.device.handle)
+        return out, cache
 
     def forward_device(self, x_ptr: int, tokens: int, out_ptr: int, valid_ptr: int = 0, bias_ptr: int = 0,
                        residual_ptr: int = 0) -> None:
@@ -443,28 +500,10 @@ class MoeLayer:
         return float(aux.value), float(z.value)
 
     def cache(self, tokens: int, valid_tokens: Optional[int] = None) -> MoeCache:
-        E, k = self.config.num_experts, self.config.experts_per_token
-        S = tokens * k
-        expert_of = np.full((S,), UNROUTED, np.int32)
-        gate_of = np.zeros((S,), np.float32)
-        counts = np.zeros((E,), np.int32)
-        offsets = np.zeros((E + 1,), np.int32)
-        perm_slot = np.full((S,), -1, np.int32)
-        perm_token = np.full((S,), -1, np.int32)
-        P = np.zeros((tokens, E), np.float32)
-        lse = np.zeros((tokens,), np.float32)
-        ip, fp = C.POINTER(C.c_int32), C.POINTER(C.c_float)
-        r = L.Routing(expert_of.ctypes.data_as(ip), gate_of.ctypes.data_as(fp), counts.ctypes.data_as(ip),
-                      offsets.ctypes.data_as(ip), perm_slot.ctypes.data_as(ip), perm_token.ctypes.data_as(ip),
-                      P.ctypes.data_as(fp), lse.ctypes.data_as(fp))
-        _check(self._lib.rbmoe_get_routing(self.handle, C.byref(r)), self.device.handle)
-        aux, z = self.losses()
-        R = int(offsets[E])
-        if valid_tokens is None:
-            valid_tokens = R // k
-        assignments = list(zip(expert_of.tolist(), gate_of.tolist()))
-        return MoeCache(assignments, expert_of, gate_of, counts, offsets, perm_slot[:R], perm_token[:R], P, lse,
-                        valid_tokens, aux, z)
+        t = _Tables(self, tokens)
+        _check(self._lib.rbmoe_get_routing(self.handle, t.c.ctypes.data), self.device.handle)
+        t.losses[:] = self.losses()
+        return t.cache(valid_tokens)
 
     def expert_rows(self, routed: int) -> Tuple[np.ndarray, np.ndarray]:
         """Hidden rows ``[routed, d_ff]`` and expert output rows ``[routed, d_model]``
@@ -487,30 +526,7 @@ class MoeLayer:
     def forward_block(self, residual: np.ndarray, layout: Layout = Layout(),
                       router_bias: Optional[np.ndarray] = None) -> Tuple[np.ndarray, MoeCache]:
         """``residual + forward_train(feed_forward_norm(residual))``; the cache describes the normed rows."""
-        residual = np.asarray(residual)
-        if residual.ndim != 2:
-            raise InvalidInput("input must be a [tokens, d_model] matrix")
-        rows, cols = residual.shape
-        if cols != self._d_model:
-            raise InvalidInput(f"input length {cols} does not match expected length {self._d_model}",
-                               expected=self._d_model, actual=cols)
-        layout.check(rows)
-        x = self._to_act(residual)
-        out = np.empty_like(x)
-        vp = bp = None
-        valid = None
-        if layout.valid is not None:
-            valid = np.ascontiguousarray(np.asarray(layout.valid, dtype=bool).astype(np.uint8))
-            vp = valid.ctypes.data_as(C.c_void_p)
-        if router_bias is not None:
-            router_bias = np.ascontiguousarray(router_bias, dtype=np.float32)
-            bp = router_bias.ctypes.data_as(C.c_void_p)
-        _check(self._lib.rbmoe_forward_block_host(self.handle, x.ctypes.data_as(C.c_void_p), rows, cols, vp, bp,
-                                                  out.ctypes.data_as(C.c_void_p)), self.device.handle)
-        if self.act_dtype == "bf16":
-            out = bf16_bits_to_f32(out).reshape(rows, cols)
-        valid_tokens = rows if valid is None else int(valid.sum())
-        return out, self.cache(rows, valid_tokens)
+        return self._forward_host(residual, layout, router_bias, None, True)
 
     def forward_block_device(self, x_ptr: int, tokens: int, out_ptr: int, valid_ptr: int = 0,
                              bias_ptr: int = 0) -> None:
@@ -531,12 +547,13 @@ class MoeLayer:
         if grad_output.ndim != 2 or grad_output.shape[1] != self._d_model:
             raise InvalidInput(f"grad_output must be [tokens, {self._d_model}]", expected=self._d_model,
                                actual=grad_output.shape[-1] if grad_output.ndim else 0)
-        g = self._to_act(grad_output)
-        out = np.empty_like(g)
-        _check(self._lib.rbmoe_backward_host(self.handle, g.ctypes.data_as(C.c_void_p), g.shape[0], g.shape[1],
-                                             out.ctypes.data_as(C.c_void_p)), self.device.handle)
-        if self.act_dtype == "bf16":
-            out = bf16_bits_to_f32(out).reshape(g.shape)
+        return self._backward_host(grad_output, False)
+
+    def _backward_host(self, grad_output: np.ndarray, block: bool) -> np.ndarray:
+        g = np.ascontiguousarray(grad_output, dtype=np.float32)
+        out = self.device.empty(g.shape, np.float32)
+        _check(self._lib.rbmoe_backward_train_host(self.handle, g.ctypes.data, L.F32, g.shape[0], g.shape[1], int(block),
+                                                   out.ctypes.data), self.device.handle)
         return out
 
     def backward_block(self, grad_output: np.ndarray) -> np.ndarray:
@@ -546,13 +563,7 @@ class MoeLayer:
         if grad_output.ndim != 2 or grad_output.shape[1] != self._d_model:
             raise InvalidInput(f"grad_output must be [tokens, {self._d_model}]", expected=self._d_model,
                                actual=grad_output.shape[-1] if grad_output.ndim else 0)
-        g = self._to_act(grad_output)
-        out = np.empty_like(g)
-        _check(self._lib.rbmoe_backward_block_host(self.handle, g.ctypes.data_as(C.c_void_p), g.shape[0], g.shape[1],
-                                                   out.ctypes.data_as(C.c_void_p)), self.device.handle)
-        if self.act_dtype == "bf16":
-            out = bf16_bits_to_f32(out).reshape(g.shape)
-        return out
+        return self._backward_host(grad_output, True)
 
     def backward_block_device(self, grad_output_ptr: int, tokens: int, grad_input_ptr: int) -> None:
         """Enqueue the block step's backward pass on device pointers (no synchronisation); both buffers are
@@ -574,7 +585,7 @@ class MoeLayer:
         F, d, Fs = self.config.d_ff, self._d_model, self.shared_d_ff
         shape = {L.W_ROUTER: (self.config.num_experts, d), L.W_GATE: (F, d), L.W_UP: (F, d), L.W_DOWN: (d, F),
                  L.W_SHARED_GATE: (Fs, d), L.W_SHARED_UP: (Fs, d), L.W_SHARED_DOWN: (d, Fs), L.W_NORM: (1, d)}[which]
-        g = np.zeros(shape, np.float32)
+        g = self.device.empty(shape, np.float32)
         _check(self._lib.rbmoe_get_weight_grad(self.handle, which, expert, g.ctypes.data_as(C.POINTER(C.c_float)),
                                                shape[0], shape[1]), self.device.handle)
         return g

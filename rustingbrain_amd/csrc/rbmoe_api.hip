@@ -279,6 +279,7 @@ struct rbmoe_layer {
     bool training = false;
     bool weights_set = false;
     Buf xc;                               // copy of the last input [T, d]
+    const void* x_saved = nullptr;        // the last input as the backward pass reads it: xc, or the normed rows
     Buf gu, gus;                          // pre-activations (gate | up): [S, 2F], shared [T, 2Fs]
     Buf dy, dgu, dxg;                     // [S, d], [S, 2F], [S, d]
     Buf g16;                              // [T, d] bf16 copy of an f32 upstream gradient (cast_rows)
@@ -577,7 +578,7 @@ int rbmoe_layer_create(rbmoe_ctx* ctx, const rbmoe_config* cfg, rbmoe_layer** ou
     L->cfg.shared_d_ff = L->Fs;
     L->max_T = cfg->max_tokens;
     L->max_S = cfg->max_tokens * cfg->experts_per_token;
-    L->max_nb = (cfg->max_tokens + kRouterTokens - 1) / kRouterTokens;
+    L->max_nb = (cfg->max_tokens + kMinRouterTokens - 1) / kMinRouterTokens;
     L->max_tiles = L->max_S / kGenericTileM + cfg->num_experts + 1;
     // (behaviour switches keep their defaults here: rbmoe_layer_set_option changes them)
     // bf16 matrix cores: bf16 activations, bf16 or int8 weights, widths that fit the packed layout
@@ -1066,7 +1067,29 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     }
     // the rows the expert products read
     const void* const xe = cast ? wk_.x16 : x;
-    if (norm_src && !norm_in_route)
+    RouterArgs ra{norm_src ? norm_src : x, (const float*)L->router.p, router_bias, valid, T, d, E, k,
+                  (float*)L->P.p, (float*)L->lse.p, (int*)L->expert_of.p, (float*)L->gate_of.p,
+                  (int*)L->rank_in_block.p, (int*)L->blockcnt.p, (float*)L->partial.p};
+    if (cast) ra.rows16 = L->x16.p;
+    ra.allow_fused = L->fused_router;
+    if (L->router_q8) {
+        ra.wq = (const int8_t*)L->router_q.p;
+        ra.wscale = (const float*)L->router_s.p;
+    }
+    if (norm_src) {
+        ra.norm_w = (const float*)L->norm_w.p;
+        ra.norm_eps = L->norm_eps;
+        ra.xn_out = L->xn.p;
+    }
+    const RouterPlan rplan = plan_router(ra, abf);
+    if (!rplan.takes_norm) {  // the norm runs by itself
+        ra.x = x;
+        ra.norm_w = nullptr;
+        ra.xn_out = nullptr;
+    }
+    const bool cast_apart = cast && L->router_q8 && !rplan.q8_writes_rows16;
+    if (cast_apart) ra.rows16 = nullptr;
+    if (norm_src && !norm_in_route && (decode_ok || !rplan.takes_norm))
         HIP_TRY(ctx, launch_rmsnorm(norm_src, (const float*)L->norm_w.p, L->norm_eps, T, d, L->xn.p, abf, s));
 
     // ---- a few tokens: route in one workgroup, then stream the touched weights once -------
@@ -1179,7 +1202,10 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         return RBMOE_OK;
     }
 
-    if (L->training && T > 0)  // MoeCache keeps the input (src/moe.rs:133-135)
+    // MoeCache keeps the input (src/moe.rs:133-135).  Behind the norm the input is the layer's own buffer of normed rows,
+    // which nothing writes before the next forward of the layer.
+    L->x_saved = norm_src ? L->xn.p : L->xc.p;
+    if (L->training && T > 0 && !norm_src)
         HIP_TRY(ctx, hipMemcpyAsync(L->xc.p, x, (size_t)T * d * dtype_size(c.act_dtype), hipMemcpyDeviceToDevice, s));
 
     for (auto& r : L->replay) r = nullptr;
@@ -1228,32 +1254,36 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         }
     } join_guard{ctx, s};
     bool shared_forked = false;
-    if (c.shared_expert && T >= 1024 && !timed && !cast && L->shared_beside && (mfma || f32mc) &&
-        ensure_side_stream(ctx) == RBMOE_OK) {
-        HIP_TRY(ctx, hipEventRecord(ctx->ev_fork, s));
-        HIP_TRY(ctx, hipStreamWaitEvent(ctx->side_stream, ctx->ev_fork, 0));
-        const hipError_t e = shared_expert(ctx->side_stream);
-        (void)hipEventRecord(ctx->ev_join, ctx->side_stream);  // recorded whatever happened: the join below always works
-        join_guard.armed = true;
-        shared_forked = true;
-        if (e != hipSuccess) return hip_fail(ctx, e, "shared expert on the side stream");
-    }
-
-    RouterArgs ra{x, (const float*)L->router.p, router_bias, valid, T, d, E, k,
-                  (float*)L->P.p, (float*)L->lse.p, (int*)L->expert_of.p, (float*)L->gate_of.p,
-                  (int*)L->rank_in_block.p, (int*)L->blockcnt.p, (float*)L->partial.p};
-    if (cast) ra.rows16 = L->x16.p;
-    ra.allow_fused = L->fused_router;
-    if (L->router_q8) {
-        ra.wq = (const int8_t*)L->router_q.p;
-        ra.wscale = (const float*)L->router_s.p;
-        if (cast) {  // the quantized router's kernel does not write the bf16 copy of f32 rows on its way
-            ra.rows16 = nullptr;
-            HIP_TRY(ctx, launch_cast_rows_bf16((const float*)x, L->x16.p, (long long)T * d, s));
+    auto fork_shared = [&]() -> int {
+        if (c.shared_expert && T >= 1024 && !timed && !cast && L->shared_beside && (mfma || f32mc) &&
+            ensure_side_stream(ctx) == RBMOE_OK) {
+            HIP_TRY(ctx, hipEventRecord(ctx->ev_fork, s));
+            HIP_TRY(ctx, hipStreamWaitEvent(ctx->side_stream, ctx->ev_fork, 0));
+            const hipError_t e = shared_expert(ctx->side_stream);
+            (void)hipEventRecord(ctx->ev_join, ctx->side_stream);  // recorded whatever happened: the join below always works
+            join_guard.armed = true;
+            shared_forked = true;
+            if (e != hipSuccess) return hip_fail(ctx, e, "shared expert on the side stream");
         }
-    }
+        return RBMOE_OK;
+    };
+    // (rows that the router's launch norms on its way are not there before it)
+    const bool shared_first = ra.norm_w == nullptr;
+    if (shared_first)
+        if (const int rc = fork_shared()) return rc;
+
+    if (cast_apart)
+        HIP_TRY(ctx, launch_cast_rows_bf16((const float*)x, L->x16.p, (long long)T * d, s));
     HIP_TRY(ctx, launch_router(ra, abf, s));
-    L->replay[RBMOE_STAGE_ROUTER] = [=](hipStream_t st) { return launch_router(ra, abf, st); };
+    if (!shared_first)
+        if (const int rc = fork_shared()) return rc;
+    RouterArgs again = ra;  // (the rows are normed by now; in an in-place block step the raw ones are gone)
+    if (again.norm_w) {
+        again.x = x;
+        again.norm_w = nullptr;
+        again.xn_out = nullptr;
+    }
+    L->replay[RBMOE_STAGE_ROUTER] = [=](hipStream_t st) { return launch_router(again, abf, st); };
     HIP_TRY(ctx, mark(1));
 
     HIP_TRY(ctx, mark(2));  // an interval with no work in it: the cost of one pair of event records
@@ -1266,6 +1296,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     da.partial = (const float*)L->partial.p;
     da.blockbase = (int*)L->blockbase.p;
     da.T = T; da.d = d; da.E = E; da.k = k;
+    da.block_tokens = rplan.block_tokens;
     da.w_aux = c.aux_loss_weight; da.w_z = c.router_z_loss_weight;
     da.tile_m = tile_m0;
     da.counts = (int*)L->counts.p; da.offsets = (int*)L->offsets.p;
@@ -2053,7 +2084,7 @@ int rbmoe_backward(rbmoe_layer* L, const void* grad_output, int32_t tokens, int3
     HIP_TRY(ctx, launch_route_backward((const float*)L->P.p, (const float*)L->lse.p, (const int*)L->expert_of.p,
                                        (const float*)L->grad_gates.p, counts, offsets, T, E, k, c.aux_loss_weight,
                                        c.router_z_loss_weight, (float*)L->dlogits.p, rs));
-    HIP_TRY(ctx, launch_router_grad((const float*)L->dlogits.p, L->xc.p, (const float*)L->router.p, T, d, E,
+    HIP_TRY(ctx, launch_router_grad((const float*)L->dlogits.p, L->x_saved, (const float*)L->router.p, T, d, E,
                                     (float*)L->rpartial.p, (float*)L->g_router.p, L->dxr.p, xbf, rs));
 
     // SwiGlu::backward over the routed rows (src/ffn.rs:87-120)
@@ -2122,7 +2153,7 @@ int rbmoe_backward(rbmoe_layer* L, const void* grad_output, int32_t tokens, int3
         sx.a = L->dgus.p; sx.w = L->swguT.p; sx.N = d; sx.K = 2 * Fs; sx.out = L->dxs.p;
         HIP_TRY(ctx, prod(sx));
         HIP_TRY(ctx, wgrad(2, gout, d, L->hs.p, nullptr, Fs, 1, T, T, (float*)L->g_sdown.p, 0));
-        HIP_TRY(ctx, wgrad(3, L->dgus.p, 2 * Fs, cast ? L->x16.p : L->xc.p, nullptr, d, 1, T, T, (float*)L->g_sgu.p, 0));
+        HIP_TRY(ctx, wgrad(3, L->dgus.p, 2 * Fs, cast ? L->x16.p : L->x_saved, nullptr, d, 1, T, T, (float*)L->g_sgu.p, 0));
     }
     // grad_input = sum over a token's slots of its expert rows + shared + router
     if (side) HIP_TRY(ctx, hipStreamWaitEvent(s, ctx->ev_join, 0));

@@ -109,6 +109,87 @@ __device__ __forceinline__ float rb_logf(float x) {
     return r;
 }
 
+__device__ __forceinline__ float inverse_rms_of(float sum, int d, float eps) {
+    const float mean_square = __fdiv_rn(sum, (float)d);
+    // The root must be the correctly rounded one (the reference's f32::sqrt): taken in double and rounded once,
+    // which is exact for a square root; the single-precision root instruction alone is not.
+    const float root = (float)sqrt((double)__fadd_rn(mean_square, eps));
+    return __fdiv_rn(1.0f, root);
+}
+
+// LDS reads of 16 bytes each that stay where they are written.
+template <typename V>
+__device__ __forceinline__ V lds_load_ahead(const unsigned char* p) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    static_assert(sizeof(V) % 16 == 0, "16-byte pieces");
+    struct Raw {
+        u32x4 v[sizeof(V) / 16];
+    } raw;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(V) / 16; ++i)
+        raw.v[i] = *(const volatile __attribute__((address_space(3))) u32x4*)(const __attribute__((address_space(3))) void*)(p + 16 * i);
+    return __builtin_bit_cast(V, raw);
+}
+
+// The sum, in index order, of the d squares that lie at `row_f` in LDS (d a multiple of 8, the row on a 16-byte boundary,
+// at least 256 readable bytes behind it): what RmsNorm::forward adds up element by element (src/norm.rs:128-131).  One
+// dependent chain of rounded adds, 4.8 cycles each on a wave of its own - the length of a row's norm.  So nothing else is
+// on it: the squares are taken beforehand by every thread of the workgroup, and the reads go out 48 elements ahead in
+// registers of their own, in an order the compiler does not change (left to itself it moves every read down to its use).
+__device__ __forceinline__ float ordered_sum(const float* row_f, int d) {
+    const unsigned char* row = reinterpret_cast<const unsigned char*>(row_f);
+    struct Part {
+        float4 q[4];
+    };
+    auto read = [&](Part& p, int at) {  // 16 elements
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p.q[u] = lds_load_ahead<float4>(row + 64 * at + 16 * u);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float sum = 0.0f;
+    auto add4 = [&](const float4& q) {
+        sum = __fadd_rn(sum, q.x);
+        sum = __fadd_rn(sum, q.y);
+        sum = __fadd_rn(sum, q.z);
+        sum = __fadd_rn(sum, q.w);
+    };
+    auto add = [&](const Part& p) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) add4(p.q[u]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Part p0, p1, p2, p3;
+    read(p0, 0);
+    read(p1, 1);
+    read(p2, 2);
+    int left = d;
+    for (; left >= 64; left -= 64) {
+        read(p3, 3);
+        add(p0);
+        read(p0, 4);
+        add(p1);
+        read(p1, 5);
+        add(p2);
+        read(p2, 6);
+        add(p3);
+        row += 256;
+    }
+    // up to 56 elements are left
+    read(p3, 3);
+    auto rest = [&](const Part& p) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (left > 0) add4(p.q[u]);
+            left -= 4;
+        }
+    };
+    rest(p0);
+    rest(p1);
+    rest(p2);
+    rest(p3);
+    return sum;
+}
+
 // silu(x) = x * (1 / (1 + exp(-x))), the reference's operation order
 // (src/ffn.rs:223-229).  Tolerance-checked, so the fast exponential is used.
 __device__ __forceinline__ float silu_f32(float x) { return x * (1.0f / (1.0f + __expf(-x))); }

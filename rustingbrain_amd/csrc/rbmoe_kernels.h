@@ -49,9 +49,11 @@ extern thread_local KernelTimer* g_kernel_timer;  // null (the default): plain l
         }                                                                                                       \
     } while (0)
 
-// Tokens owned by one router / dispatch block.  Slots are numbered
-// token * k + rank, so a block owns a contiguous slot range.
+// Tokens owned by one router / dispatch block: a block owns a contiguous slot range (slots are numbered
+// token * k + rank).  The kernels that take a whole batch's rows at once use 8, 16 or 32 tokens a block, by what fills
+// the chip (plan_router); the others 32.
 constexpr int kRouterTokens = 32;
+constexpr int kMinRouterTokens = 8;
 constexpr int kRouterThreads = 512;     // router_kernel workgroup
 constexpr int kRouterWaves = kRouterThreads / 64;
 
@@ -61,7 +63,6 @@ constexpr int kMaxTopK = 32;
 
 size_t router_lds_bytes(int E, int k);
 constexpr int kMaxRouterLds = 160 * 1024;  // LDS per workgroup on gfx950
-size_t dispatch_lds_bytes(int E, int k);
 
 struct RouterArgs {
     const void* x;       // [T, d] f32 or bf16
@@ -82,7 +83,20 @@ struct RouterArgs {
     // `wr` is then not read and the logits are (sum_c x[c] * f32(q[c]), in the reference's 32 lanes) * scale
     const int8_t* wq = nullptr;      // [E, d]
     const float* wscale = nullptr;   // [E]
+    // The norm in front of the layer (RmsNorm::forward, src/norm.rs:41-61), for calls whose plan says `takes_norm`: `x`
+    // holds the raw rows, the routing is decided on the normed ones, which are written to `xn_out` [T, d].
+    const float* norm_w = nullptr;
+    float norm_eps = 0.0f;
+    void* xn_out = nullptr;
 };
+// How a call is routed: tokens of a router block (what launch_dispatch needs to know), whether the launch applies the
+// norm that `a` asks for, and whether it writes the bf16 copy of f32 rows for a quantized router too.
+struct RouterPlan {
+    int block_tokens;
+    bool takes_norm;
+    bool q8_writes_rows16;
+};
+RouterPlan plan_router(const RouterArgs& a, bool bf16);
 hipError_t launch_router(const RouterArgs& a, bool bf16, hipStream_t s);
 
 struct DispatchArgs {
@@ -92,6 +106,7 @@ struct DispatchArgs {
     const int* blockcnt;   // [nb, E]    per-block histogram from the router kernel
     const float* partial;  // [nb, E+1]  per-block sums of probabilities and of lse^2
     int T, d, E, k;
+    int block_tokens;      // tokens of a router block (RouterPlan)
     float w_aux, w_z;
     int tile_m;            // rows per tile of the grouped products
     int* counts;           // [E]

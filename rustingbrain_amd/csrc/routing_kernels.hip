@@ -12,6 +12,7 @@
 //
 // Nothing here uses floating-point atomics: every sum has a fixed order, so two
 // runs give the same bits.
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <type_traits>
@@ -28,9 +29,9 @@ namespace rbmoe {
 //   lexp   [TB][k]    selected expert per local slot (-1 = unrouted)
 //   wcount [waves][E] per-wave match counts of one ranking round
 //   running[E]        slots already ranked per expert
-__host__ __device__ static size_t router_fixed_bytes(int E, int k) {
+__host__ __device__ static size_t router_fixed_bytes(int E, int k, int tokens = kRouterTokens) {
     const int ES = E | 1;
-    size_t n = (size_t)kRouterTokens * ES + kRouterTokens + 2 * (size_t)kRouterTokens * k + (size_t)kRouterWaves * E + E;
+    size_t n = (size_t)tokens * ES + tokens + 2 * (size_t)tokens * k + (size_t)kRouterWaves * E + E;
     return (n * 4 + 15) & ~(size_t)15;
 }
 
@@ -242,11 +243,10 @@ __global__ __launch_bounds__(NE * 64, (!AHEAD && sizeof(XT) == 2) ? 6 : 2) void 
 // greatest probability bits (probabilities are never negative, so the bits order like the values), then the
 // lowest expert index among the lanes that hold them.
 // NQ = turns a wave needs for its tokens (64 / G tokens a turn); the NQ turns share no data and run interleaved.
-template <int MAXJ, int NQ>
+template <int MAXJ, int NQ, int TB>
 __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __restrict__ lsev,
                                              float* __restrict__ gates, int* __restrict__ lexp, int G, int t0, int nt,
                                              int ES, const uint8_t* __restrict__ valid, int E, int k) {
-    constexpr int TB = kRouterTokens;
     constexpr int TW = TB / kRouterWaves;  // tokens of a wave
     const int lane_ = threadIdx.x & 63, wave_ = threadIdx.x >> 6;
     const int lig = lane_ & (G - 1);          // lane in group
@@ -404,16 +404,15 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
             for (int r = lig; r < k; r += G) gates[tok[q] * k + r] = __fdiv_rn(gates[tok[q] * k + r], total[q]);
 }
 
-// router_tail: everything behind the logits for the 32 tokens of router block `blk` - softmax, log-sum-exp, top-k,
+// router_tail: everything behind the logits for the TB tokens of router block `blk` - softmax, log-sum-exp, top-k,
 // gates, ranks, block histogram, partial sums of the losses.  LOADED = false: the logits are read from P;
 // true: the caller has put them into the `prob` array of `lds_raw` (row pitch E | 1) and met at a barrier.
 // MAXJ = experts a lane may own: 1 when E <= 64 (a lane owns one expert), kMaxExperts / 64 otherwise.
-template <int MAXJ, bool LOADED>
+template <int MAXJ, bool LOADED, int TB = kRouterTokens>
 __device__ __forceinline__ void router_tail(
     unsigned char* __restrict__ lds_raw, int blk, const uint8_t* __restrict__ valid, int T, int E, int k,
     float* __restrict__ P, float* __restrict__ lse, int* __restrict__ expert_of, float* __restrict__ gate_of,
     int* __restrict__ rank_in_block, int* __restrict__ blockcnt, float* __restrict__ partial) {
-    constexpr int TB = kRouterTokens;
     const int ES = E | 1;
     float* prob = reinterpret_cast<float*>(lds_raw);
     float* lsev = prob + TB * ES;
@@ -440,11 +439,12 @@ __device__ __forceinline__ void router_tail(
     {
         int G = 1;
         while (G < E && G < 64) G <<= 1;
-        // a wave's four tokens: all at once with up to 16 lanes per token, in two or four turns with 32 or 64 - the
+        // a wave's tokens (four of 32): all at once with up to 16 lanes per token, in more turns with 32 or 64 - the
         // turns are worked on side by side (one instruction stream), because each is a chain of dependent steps
-        if (G == 64) softmax_topk<MAXJ, 4>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
-        else if (G == 32) softmax_topk<MAXJ, 2>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
-        else softmax_topk<MAXJ, 1>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
+        constexpr int TW = TB / kRouterWaves;
+        if (G == 64) softmax_topk<MAXJ, TW, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
+        else if (G == 32) softmax_topk<MAXJ, (TW + 1) / 2, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
+        else softmax_topk<MAXJ, (TW + 3) / 4, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
     }
     __syncthreads();
 
@@ -587,20 +587,6 @@ __global__ __launch_bounds__(256) void logits_q8_kernel(const XT* __restrict__ x
 // ---------------------------------------------------------------------------
 __host__ __device__ static size_t fused_lds_bytes(int E, int k, int cols, size_t xsize) {
     return router_fixed_bytes(E, k) + (size_t)kRouterTokens * (cols * xsize + 16) + (size_t)E * (cols * 4 + 16);
-}
-
-// LDS reads of 16 bytes each that stay where they are written.
-template <typename V>
-__device__ __forceinline__ V lds_load_ahead(const unsigned char* p) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    static_assert(sizeof(V) % 16 == 0, "16-byte pieces");
-    struct Raw {
-        u32x4 v[sizeof(V) / 16];
-    } raw;
-#pragma unroll
-    for (size_t i = 0; i < sizeof(V) / 16; ++i)
-        raw.v[i] = *(const volatile __attribute__((address_space(3))) u32x4*)(const __attribute__((address_space(3))) void*)(p + 16 * i);
-    return __builtin_bit_cast(V, raw);
 }
 
 // WIDE (bf16 rows): the token rows are widened to f32 once, on their way into LDS, instead of by each of the 16
@@ -773,6 +759,278 @@ __global__ __launch_bounds__(kRouterThreads) void route_fused_kernel(
     router_tail<1, true>(lds_raw, blk, valid, T, E, k, P, lse, expert_of, gate_of, rank_in_block, blockcnt, partial);
 }
 
+// ---------------------------------------------------------------------------
+// route_rows_kernel: norm (optional), logits and everything behind them for TB = 8, 16 or 32 tokens a workgroup, with
+// the workgroup's whole rows in LDS at once.
+// What bounds routing up to some thousand tokens is not work but the length of one workgroup's chain: with 32 tokens a
+// workgroup and slices of columns staged in turn (route_fused_kernel) it takes 18 to 20 us whether 7 workgroups run or
+// 256.  So the tokens of a workgroup are chosen to spread the call over the chip, everything a workgroup reads is
+// requested in one batch, and a dot product is taken by NL neighbouring threads, thread j owning column lane j of the
+// reference's sum: a chain of d / NL rounded multiplies and adds.  A thread works on TT tokens x EE experts side by
+// side, so that TT + EE words read from LDS feed TT * EE products; its columns j, j + NL, ... lie side by side in LDS,
+// so that it reads four steps of the chain at a time.
+// NL = 8: `dot` (src/matrix.rs:26-40).  NL = 32: the quantized router's dot_lanes::<32> (src/quantized.rs:154-177), its
+// int8 rows widened on their way into LDS, the sum times the row's scale (:61).
+// The norm is RmsNorm::forward (src/norm.rs:41-61): the squares are laid down in column order beside the rows and one
+// thread a row adds them up in index order, as the reference does.
+// Measured, against route_fused_kernel (and the norm's launch in front of it): d 768, 203 tokens x 16 experts 9.5 us
+// against 18.1, with the norm 14.4 against 32.2; 4096 x 8 10.5 against 17.7; 8192 x 16 16.2 against 19.6.  Of the 14.4:
+// rows staged 2.8 us into the workgroup, normed at 6.8 (half of it the chain of 768 adds), logits at 9.1, softmax and
+// top-k at 11.2, end 12.3.
+// ---------------------------------------------------------------------------
+struct RouteRowsArgs {
+    const void* x;
+    const float* wr;
+    const int8_t* wq;
+    const float* wscale;
+    const float* bias;
+    const uint8_t* valid;
+    int T, d, E, k, EG;  // EG: experts whose router rows are in LDS together
+    float* P;
+    float* lse;
+    int* expert_of;
+    float* gate_of;
+    int* rank_in_block;
+    int* blockcnt;
+    float* partial;
+    bf16_t* rows16;
+    const float* norm_w;
+    float norm_eps;
+    void* xn_out;
+};
+// A staged row: column lane j's elements side by side, `lane_pitch` floats from one lane to the next - whole 16-byte
+// pieces (a last one short of four steps is filled up with zeros, which the sums do not see), and an odd number of
+// them, so that the lanes' pieces start in different banks.
+__host__ __device__ static int route_lane_pitch(int d, int NL) {
+    const int steps = (d / NL + 3) / 4;
+    return 4 * (steps | 1);
+}
+
+template <typename XT, int TB, int NL, int TT, int EE>
+__global__ __launch_bounds__(kRouterThreads, 2) void route_rows_kernel(RouteRowsArgs a) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    constexpr int NT = kRouterThreads;
+    const int T = a.T, d = a.d, E = a.E, k = a.k, EG = a.EG;
+    const int ES = E | 1;
+    float* const prob = reinterpret_cast<float*>(lds_raw);
+    const int lp = route_lane_pitch(d, NL), pitch = NL * lp;
+    float* const xs = reinterpret_cast<float*>(lds_raw + router_fixed_bytes(E, k, TB));
+    float* const ws = xs + TB * pitch;
+    float* const sq = ws + EG * pitch;   // with a norm: the squares [TB][d + 4], the norm's weights [d] (and 256 bytes of room)
+    const int sp = d + 4;                // (4: the rows' chains read from different banks)
+    float* const nws = sq + TB * sp;
+    const int tid = threadIdx.x;
+    const int t0 = blockIdx.x * TB;
+    const int nt = min(TB, T - t0);
+    const bool norm = a.norm_w != nullptr;
+
+    // Staging: 16-byte pieces of the router's rows and of the token rows, six of each a thread requested before the first
+    // is stored (96 KB a trip to memory; variables of their own: an array of them ends up in scratch memory).  A row's
+    // pieces are counted by a rounded-up reciprocal, exact for the few thousand there are.
+    constexpr int XN = Vec16<XT>::N;
+    const int wpr = NL == 32 ? d / 16 : d / 4, xpr = d / XN;
+    const uint32_t wrecip = (uint32_t)(0x100000000ull / (uint32_t)wpr) + 1u, xrecip = (uint32_t)(0x100000000ull / (uint32_t)xpr) + 1u;
+    auto put_router = [&](int i, const uint4& v) {
+        const int r = wpr == 1 ? i : (int)__umulhi((uint32_t)i, wrecip), c = i - r * wpr;
+        if constexpr (NL == 32) {
+            float* const to = ws + r * pitch + ((16 * c) % NL) * lp + (16 * c) / NL;
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int q = 0; q < 16; ++q) to[q * lp] = (float)(int8_t)(w[q >> 2] >> (8 * (q & 3)));
+        } else {
+            float* const to = ws + r * pitch + ((4 * c) % NL) * lp + (4 * c) / NL;
+            to[0] = __uint_as_float(v.x); to[lp] = __uint_as_float(v.y);
+            to[2 * lp] = __uint_as_float(v.z); to[3 * lp] = __uint_as_float(v.w);
+        }
+    };
+    auto put_row = [&](int i, const uint4& v) {
+        const int r = xpr == 1 ? i : (int)__umulhi((uint32_t)i, xrecip), c = i - r * xpr;
+        float f[XN];
+        Vec16<XT>::widen(v, f);
+        float* const to = xs + r * pitch + ((XN * c) % NL) * lp + (XN * c) / NL;
+#pragma unroll
+        for (int q = 0; q < XN; ++q) to[q * lp] = f[q];
+        if (norm) {
+            float4* const s4 = reinterpret_cast<float4*>(sq + r * sp + XN * c);
+#pragma unroll
+            for (int q = 0; q < XN / 4; ++q)
+                s4[q] = make_float4(__fmul_rn(f[4 * q], f[4 * q]), __fmul_rn(f[4 * q + 1], f[4 * q + 1]),
+                                    __fmul_rn(f[4 * q + 2], f[4 * q + 2]), __fmul_rn(f[4 * q + 3], f[4 * q + 3]));
+        }
+    };
+    auto stage = [&](int e0, int ne, auto with_rows) {
+        constexpr bool kRows = decltype(with_rows)::value;
+        const uint4* const wsrc = NL == 32 ? reinterpret_cast<const uint4*>(a.wq + (size_t)e0 * d)
+                                           : reinterpret_cast<const uint4*>(a.wr + (size_t)e0 * d);
+        const uint4* const xsrc = reinterpret_cast<const uint4*>(static_cast<const XT*>(a.x) + (size_t)t0 * d);
+        const int nw = ne * wpr, nx = kRows ? nt * xpr : 0;
+        for (int i = tid; i < max(nw, nx); i += 6 * NT) {
+            auto fw = [&](int u) -> uint4 { return wsrc[(uint32_t)min(i + u * NT, nw - 1)]; };
+            auto fx = [&](int u) -> uint4 { return xsrc[(uint32_t)min(i + u * NT, max(nx, 1) - 1)]; };
+            const uint4 w0 = fw(0), w1 = fw(1), w2 = fw(2), w3 = fw(3), w4 = fw(4), w5 = fw(5);
+            uint4 x0, x1, x2, x3, x4, x5;
+            if constexpr (kRows) { x0 = fx(0); x1 = fx(1); x2 = fx(2); x3 = fx(3); x4 = fx(4); x5 = fx(5); }
+            __builtin_amdgcn_sched_barrier(0);
+            auto pw = [&](int u, const uint4& v) { if (i + u * NT < nw) put_router(i + u * NT, v); };
+            auto px = [&](int u, const uint4& v) { if (i + u * NT < nx) put_row(i + u * NT, v); };
+            pw(0, w0); pw(1, w1); pw(2, w2); pw(3, w3); pw(4, w4); pw(5, w5);
+            if constexpr (kRows) { px(0, x0); px(1, x1); px(2, x2); px(3, x3); px(4, x4); px(5, x5); }
+        }
+    };
+    // (the short last pieces' zeros)
+    const int short_from = d / NL, short_n = (short_from + 3) / 4 * 4 - short_from;
+    if (short_n > 0)
+        for (int i = tid; i < (TB + EG) * NL * short_n; i += NT) xs[(i / short_n) * lp + short_from + i % short_n] = 0.0f;
+    if (norm)
+        for (int c = tid; c < d; c += NT) nws[c] = a.norm_w[c];
+    stage(0, min(EG, E), std::true_type{});
+    __syncthreads();
+    if (norm) {
+        if (tid < nt) {
+            const float f = inverse_rms_of(ordered_sum(sq + tid * sp, d), d, a.norm_eps);
+            sq[tid * sp] = f;  // (the row's squares are used up)
+        }
+        __syncthreads();
+    }
+    if (norm || a.rows16 != nullptr) {
+        // the normed rows, rounded to the layer's own type, replace the raw ones; they (and the bf16 copy of f32 rows
+        // for the expert products) are written out on the way
+        const int pieces = d / 8;
+        const uint32_t recip = (uint32_t)(0x100000000ull / (uint32_t)pieces) + 1u;
+        for (int i = tid; i < nt * pieces; i += NT) {
+            const int r = pieces == 1 ? i : (int)__umulhi((uint32_t)i, recip), c = (i - r * pieces) * 8;
+            float* const at = xs + r * pitch + (c % NL) * lp + c / NL;
+            float v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = at[q * lp];
+            if (norm) {
+                const float sc = sq[r * sp];
+                const float4 wa = *reinterpret_cast<const float4*>(nws + c), wb = *reinterpret_cast<const float4*>(nws + c + 4);
+                const float w[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
+                XT o[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    o[q] = from_f32<XT>(__fmul_rn(__fmul_rn(v[q], sc), w[q]));
+                    v[q] = to_f32(o[q]);
+                    at[q * lp] = v[q];
+                }
+                uint4* const to = reinterpret_cast<uint4*>(static_cast<XT*>(a.xn_out) + (size_t)(t0 + r) * d + c);
+#pragma unroll
+                for (int q = 0; q < 8 / XN; ++q) to[q] = reinterpret_cast<const uint4*>(o)[q];
+            }
+            if constexpr (sizeof(XT) == 4) {
+                if (a.rows16 != nullptr) {
+                    uint4 o;
+                    o.x = f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16);
+                    o.y = f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16);
+                    o.z = f32_to_bf16_bits(v[4]) | ((uint32_t)f32_to_bf16_bits(v[5]) << 16);
+                    o.w = f32_to_bf16_bits(v[6]) | ((uint32_t)f32_to_bf16_bits(v[7]) << 16);
+                    *reinterpret_cast<uint4*>(a.rows16 + (size_t)(t0 + r) * d + c) = o;
+                }
+            }
+        }
+        if (norm) __syncthreads();
+    }
+    // ---- logits -------------------------------------------------------------------
+    const int j = tid % NL;  // the thread's column lane
+    const int quads = (d / NL + 3) / 4;
+    for (int e0 = 0; e0 < E; e0 += EG) {
+        const int ne = min(EG, E - e0);
+        if (e0 > 0) {
+            __syncthreads();  // the group before has been consumed
+            stage(e0, ne, std::false_type{});
+            __syncthreads();
+        }
+        const int etiles = (ne + EE - 1) / EE;
+        const int tasks = (TB / TT) * etiles;
+        for (int g0 = 0; g0 < tasks; g0 += NT / NL) {
+            const int g = g0 + tid / NL;
+            if (g0 + (int)(threadIdx.x & ~63u) / NL >= tasks) break;  // none of the wave's groups has a tile
+            const int tt = min(g / etiles, TB / TT - 1), et = g - (g / etiles) * etiles;
+            const unsigned char *xp[TT], *wp[EE];  // (a token or expert past the end: the last one's sums again, dropped)
+#pragma unroll
+            for (int u = 0; u < TT; ++u)
+                xp[u] = reinterpret_cast<const unsigned char*>(xs + min(tt * TT + u, nt - 1) * pitch + j * lp);
+#pragma unroll
+            for (int u = 0; u < EE; ++u)
+                wp[u] = reinterpret_cast<const unsigned char*>(ws + min(et * EE + u, ne - 1) * pitch + j * lp);
+            float acc[TT][EE];
+#pragma unroll
+            for (int u = 0; u < TT; ++u)
+#pragma unroll
+                for (int v = 0; v < EE; ++v) acc[u][v] = 0.0f;
+            struct Operands {
+                float4 x[TT], w[EE];
+            };
+            // four steps of the chain a trip, the next trip's operands read before this one's products (two sets of
+            // registers take turns)
+            auto read = [&](Operands& o, int q) {
+#pragma unroll
+                for (int u = 0; u < TT; ++u) o.x[u] = lds_load_ahead<float4>(xp[u] + 16 * q);
+#pragma unroll
+                for (int u = 0; u < EE; ++u) o.w[u] = lds_load_ahead<float4>(wp[u] + 16 * q);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto multiply = [&](const Operands& o) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int u = 0; u < TT; ++u)
+#pragma unroll
+                        for (int v = 0; v < EE; ++v)
+                            acc[u][v] = __fadd_rn(acc[u][v], __fmul_rn(reinterpret_cast<const float*>(&o.x[u])[c],
+                                                                       reinterpret_cast<const float*>(&o.w[v])[c]));
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            Operands oa, ob;
+            read(oa, 0);
+            int q = 0;
+            for (; q + 2 <= quads; q += 2) {
+                read(ob, q + 1);
+                multiply(oa);
+                read(oa, min(q + 2, quads - 1));
+                multiply(ob);
+            }
+            if (q < quads) multiply(oa);
+            // the column lanes folded left to right: lane l of a group holds ((0 + a_0) + a_1) + ... + a_l after l steps
+            // of "take the lane below's sum, add your own" (see softmax_topk), the products side by side
+            float own[TT][EE];
+#pragma unroll
+            for (int u = 0; u < TT; ++u)
+#pragma unroll
+                for (int v = 0; v < EE; ++v) {
+                    own[u][v] = acc[u][v];
+                    acc[u][v] = __fadd_rn(0.0f, acc[u][v]);
+                }
+            for (int st = 1; st < NL; ++st) {
+#pragma unroll
+                for (int u = 0; u < TT; ++u)
+#pragma unroll
+                    for (int v = 0; v < EE; ++v) {
+                        const float below = __uint_as_float(lanes_from<0x138>(__float_as_uint(acc[u][v])));  // wave_shr:1
+                        const float next = __fadd_rn(below, own[u][v]);
+                        acc[u][v] = j == 0 ? acc[u][v] : next;
+                    }
+            }
+#pragma unroll
+            for (int u = 0; u < TT; ++u)
+#pragma unroll
+                for (int v = 0; v < EE; ++v) {
+                    const int t = tt * TT + u, el = et * EE + v, e = e0 + el;
+                    if (j == NL - 1 && g < tasks && t < nt && el < ne) {
+                        float y = __fadd_rn(acc[u][v], 0.0f);  // the reference adds its (empty) scalar rest: sum + 0
+                        if constexpr (NL == 32) y = __fmul_rn(y, a.wscale[e]);
+                        if (a.bias) y = __fadd_rn(y, a.bias[e]);
+                        prob[t * ES + e] = y;
+                    }
+                }
+        }
+    }
+    __syncthreads();
+    router_tail<1, true, TB>(lds_raw, blockIdx.x, a.valid, T, E, k, a.P, a.lse, a.expert_of, a.gate_of, a.rank_in_block,
+                             a.blockcnt, a.partial);
+}
+
 template <typename XT, int MAXJ>
 __global__ __launch_bounds__(kRouterThreads) void router_kernel(
     const XT* __restrict__ x, const float* __restrict__ wr, const float* __restrict__ bias,
@@ -785,7 +1043,7 @@ __global__ __launch_bounds__(kRouterThreads) void router_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// dispatch_kernel: block b owns the same 32 tokens as router block b.
+// dispatch_kernel: block b owns the same tokens as router block b.
 //
 // Prologue (every block, redundantly — the table is a few KB and sits in L2): column sums
 // of the per-block histogram give counts[e], their exclusive prefix gives offsets[e], and
@@ -804,21 +1062,20 @@ __global__ __launch_bounds__(kRouterThreads) void router_kernel(
 // dispatch launch: every block re-derives counts, offsets and its own base from all the block
 // histograms (O(blocks^2 x experts) reads in total, but one launch less on the critical path);
 // block 0 also writes counts, offsets and the tile table, the last block the losses.
-size_t dispatch_fused_lds_bytes(int E, int k) {
+size_t dispatch_fused_lds_bytes(int E, int k, int tokens) {
     const int parts = 256 / E;
-    return ((size_t)2 * parts * E + (size_t)parts * (E + 1) + 4 * (size_t)(E + 1) + (size_t)kRouterTokens * k) * 4;
+    return ((size_t)2 * parts * E + (size_t)parts * (E + 1) + 4 * (size_t)(E + 1) + (size_t)tokens * k) * 4;
 }
 
 template <typename XT>
 __global__ __launch_bounds__(256) void dispatch_fused_kernel(
     const XT* __restrict__ x, const int* __restrict__ expert_of, const int* __restrict__ rank_in_block,
-    const int* __restrict__ blockcnt, const float* __restrict__ partial, int T, int d, int E, int k,
+    const int* __restrict__ blockcnt, const float* __restrict__ partial, int T, int d, int E, int k, int TB,
     float w_aux, float w_z, int tile_m, int* __restrict__ counts, int* __restrict__ offsets,
     int* __restrict__ tile_expert, int* __restrict__ tile_row0, int* __restrict__ tile_rows,
     int* __restrict__ ntiles, float* __restrict__ losses, int* __restrict__ perm_slot,
     int* __restrict__ perm_token, int* __restrict__ inv_pos, XT* __restrict__ xg) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    constexpr int TB = kRouterTokens;
     const int parts = 256 / E;  // E <= 256
     int* part_all = reinterpret_cast<int*>(lds_raw);           // [parts][E]
     int* part_before = part_all + parts * E;                   // [parts][E]
@@ -1185,20 +1442,19 @@ __global__ __launch_bounds__(kScanThreads) void layout_scan_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// dispatch_kernel: block b owns the same 32 tokens as router block b:
+// dispatch_kernel: block b owns the same tokens as router block b:
 // position = offsets[e] + blockbase[b][e] + rank in block.
 // ---------------------------------------------------------------------------
-size_t dispatch_lds_bytes(int E, int k) {
-    return ((size_t)2 * (E + 1) + (size_t)kRouterTokens * k) * 4;
+size_t dispatch_lds_bytes(int E, int k, int tokens) {
+    return ((size_t)2 * (E + 1) + (size_t)tokens * k) * 4;
 }
 
 template <typename XT>
 __global__ __launch_bounds__(256) void dispatch_kernel(
     const XT* __restrict__ x, const int* __restrict__ expert_of, const int* __restrict__ rank_in_block,
-    const int* __restrict__ blockbase, const int* __restrict__ offsets, int T, int d, int E, int k,
+    const int* __restrict__ blockbase, const int* __restrict__ offsets, int T, int d, int E, int k, int TB,
     int* __restrict__ perm_slot, int* __restrict__ perm_token, int* __restrict__ inv_pos, XT* __restrict__ xg) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    constexpr int TB = kRouterTokens;
     int* base = reinterpret_cast<int*>(lds_raw);  // [E+1] slots of each expert routed by earlier blocks
     int* off = base + (E + 1);                    // [E+1] first row of each expert group
     int* lpos = off + (E + 1);                    // [TB * k]
@@ -1416,8 +1672,89 @@ static int fused_cols(const RouterArgs& a, size_t xsize) {
     return fused_lds_bytes(a.E, a.k, cols, xsize) <= 64 * 1024 ? cols : 0;
 }
 
+// Whether route_rows_kernel takes the call and with how many tokens a workgroup: the fewest that still give at most one
+// workgroup a compute unit (the chain of a workgroup is what a call waits for), more for larger batches.
+struct RowsPlan {
+    int tokens = 0;  // 0: not taken
+    int EG = 0;
+    size_t lds = 0;
+};
+static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
+    RowsPlan p;
+    const int unit = a.wq ? 32 : 8;  // whole turns of the column lanes, whole 16-byte pieces
+    if (!a.allow_fused || a.E > 64 || a.d % unit != 0 || a.d < unit || a.k > kMaxTopK) return p;
+    if ((reinterpret_cast<uintptr_t>(a.x) & 15) || ((size_t)a.d * xsize) % 16 != 0) return p;
+    if (reinterpret_cast<uintptr_t>(a.wq ? static_cast<const void*>(a.wq) : a.wr) & 15) return p;
+    if (a.norm_w && ((reinterpret_cast<uintptr_t>(a.xn_out) & 15) || a.d % 8 != 0)) return p;
+    const size_t row = (size_t)(a.wq ? 32 * route_lane_pitch(a.d, 32) : 8 * route_lane_pitch(a.d, 8)) * 4;
+    int tokens = kMinRouterTokens;
+    while (tokens < kRouterTokens && (a.T + tokens - 1) / tokens > 256) tokens *= 2;
+    for (; tokens >= kMinRouterTokens; tokens /= 2) {
+        const size_t fixed = router_fixed_bytes(a.E, a.k, tokens) + (size_t)tokens * row +
+                             (a.norm_w ? (size_t)(tokens + 1) * (a.d + 4) * 4 + 256 : 0);
+        if (fixed + std::min(a.E, 8) * row > (size_t)kMaxRouterLds) continue;
+        p.tokens = tokens;
+        p.EG = std::min<int>(a.E, (int)(((size_t)kMaxRouterLds - fixed) / row));
+        if (p.EG < a.E && p.EG > 2) p.EG &= ~1;  // whole pairs of experts
+        p.lds = fixed + (size_t)p.EG * row;
+        break;
+    }
+    if (!p.tokens) return p;
+    // above: the sequences tuned for launches that fill the chip several times over.  Rows so wide that fewer tokens fit
+    // than one workgroup a compute unit needs would take two rounds: route_fused_kernel's slices take one.
+    const int blocks = (a.T + p.tokens - 1) / p.tokens;
+    if ((long long)a.T * a.E > 256 * 1024 || blocks > (p.tokens == kRouterTokens ? 512 : 256)) p.tokens = 0;
+    return p;
+}
+
+RouterPlan plan_router(const RouterArgs& a, bool bf16) {
+    const RowsPlan p = plan_rows(a, bf16 ? 2 : 4);
+    if (a.norm_w && (!p.tokens || (a.T + p.tokens - 1) / p.tokens > 256)) {
+        // the squares' room costs tokens a workgroup, and a second round of workgroups costs more than the norm in a
+        // launch of its own (8192 tokens, d 768: 37.7 us in two rounds, 16.2 + 8 in two launches)
+        RouterArgs b = a;
+        b.norm_w = nullptr;
+        RouterPlan q = plan_router(b, bf16);
+        q.takes_norm = false;
+        return q;
+    }
+    return p.tokens ? RouterPlan{p.tokens, true, true} : RouterPlan{kRouterTokens, false, false};
+}
+
+template <typename XT>
+static hipError_t launch_rows_t(const RouterArgs& a, const RowsPlan& p, hipStream_t s) {
+    RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, p.EG, a.P, a.lse, a.expert_of, a.gate_of,
+                    a.rank_in_block, a.blockcnt, a.partial, static_cast<bf16_t*>(a.rows16), a.norm_w, a.norm_eps, a.xn_out};
+    const dim3 grid((a.T + p.tokens - 1) / p.tokens);
+    auto go = [&](auto kernel) -> hipError_t {
+        static std::atomic<unsigned long long> attr_set{0};  // one per kernel: the lambda's body is instantiated for each
+        const hipError_t e = once_per_device(attr_set, [&] {
+            return hipFuncSetAttribute(reinterpret_cast<const void*>(+kernel.value), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       kMaxRouterLds);
+        });
+        if (e != hipSuccess) return e;
+        RB_LAUNCH(kernel.value, grid, dim3(kRouterThreads), p.lds, s, r);
+        return hipGetLastError();
+    };
+#define RB_ROUTE_ROWS(TB, NL, TT, EE) \
+    go(std::integral_constant<void (*)(RouteRowsArgs), &route_rows_kernel<XT, TB, NL, TT, EE>>{})
+    // tokens x experts a thread: the largest tile that still has work for every thread (more sums a thread mean less
+    // traffic with LDS; the sums of 8 tokens x 16 experts take 2.3 us with 1 x 2 on eight waves, 2.9 with 2 x 2 on four)
+    if (a.wq) {
+        if (p.tokens == 8) return RB_ROUTE_ROWS(8, 32, 2, 2);
+        if (p.tokens == 16) return RB_ROUTE_ROWS(16, 32, 4, 2);
+        return RB_ROUTE_ROWS(32, 32, 4, 2);
+    }
+    if (p.tokens == 8) return RB_ROUTE_ROWS(8, 8, 1, 2);
+    if (p.tokens == 16) return a.E <= 8 ? RB_ROUTE_ROWS(16, 8, 1, 2) : RB_ROUTE_ROWS(16, 8, 2, 2);
+    return a.E <= 8 ? RB_ROUTE_ROWS(32, 8, 2, 2) : RB_ROUTE_ROWS(32, 8, 4, 2);
+#undef RB_ROUTE_ROWS
+}
+
 template <typename XT>
 static hipError_t launch_router_t(const RouterArgs& a, hipStream_t s) {
+    if (const RowsPlan p = plan_rows(a, sizeof(XT)); p.tokens) return launch_rows_t<XT>(a, p, s);
+    if (a.norm_w) return hipErrorInvalidValue;  // (the plan said so)
     const int nb = (a.T + kRouterTokens - 1) / kRouterTokens;
     if (const int cols = a.wq ? 0 : fused_cols(a, sizeof(XT))) {
         // bf16 rows staged as f32 where a slice of the same width then still fits
@@ -1491,11 +1828,11 @@ hipError_t launch_router(const RouterArgs& a, bool bf16, hipStream_t s) {
 
 template <typename XT>
 static hipError_t launch_dispatch_t(const DispatchArgs& a, hipStream_t s) {
-    const int nb = (a.T + kRouterTokens - 1) / kRouterTokens;
+    const int nb = (a.T + a.block_tokens - 1) / a.block_tokens;
     if ((long long)nb * a.E <= kFusedScanLimit) {
         RB_LAUNCH(dispatch_fused_kernel<XT>, dim3(nb > 0 ? nb : 1), dim3(256),
-                           dispatch_fused_lds_bytes(a.E, a.k), s, static_cast<const XT*>(a.x), a.expert_of,
-                           a.rank_in_block, a.blockcnt, a.partial, a.T, a.d, a.E, a.k, a.w_aux, a.w_z, a.tile_m,
+                           dispatch_fused_lds_bytes(a.E, a.k, a.block_tokens), s, static_cast<const XT*>(a.x), a.expert_of,
+                           a.rank_in_block, a.blockcnt, a.partial, a.T, a.d, a.E, a.k, a.block_tokens, a.w_aux, a.w_z, a.tile_m,
                            a.counts, a.offsets, a.tile_expert, a.tile_row0, a.tile_rows, a.ntiles, a.losses,
                            a.perm_slot, a.perm_token, a.inv_pos, static_cast<XT*>(a.xg));
         return hipGetLastError();
@@ -1514,9 +1851,9 @@ static hipError_t launch_dispatch_t(const DispatchArgs& a, hipStream_t s) {
                        a.tile_row0, a.tile_rows, a.ntiles, a.losses);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || nb == 0) return e;
-    RB_LAUNCH(dispatch_kernel<XT>, dim3(nb), dim3(256), dispatch_lds_bytes(a.E, a.k), s,
+    RB_LAUNCH(dispatch_kernel<XT>, dim3(nb), dim3(256), dispatch_lds_bytes(a.E, a.k, a.block_tokens), s,
                        static_cast<const XT*>(a.x), a.expert_of, a.rank_in_block, a.blockbase, a.offsets, a.T, a.d,
-                       a.E, a.k, a.perm_slot, a.perm_token, a.inv_pos, static_cast<XT*>(a.xg));
+                       a.E, a.k, a.block_tokens, a.perm_slot, a.perm_token, a.inv_pos, static_cast<XT*>(a.xg));
     return hipGetLastError();
 }
 
@@ -1554,57 +1891,50 @@ static hipError_t launch_combine_t(const CombineArgs& a, hipStream_t s) {
 // come out identical; the output is (value * inverse_rms) * weight, two separately rounded
 // products as in the reference.
 //
-// The chain of d dependent additions per row is the floor of this kernel.  To keep memory
-// latency off that chain, a block first copies its R rows into LDS with every lane's loads in
-// flight at once (the rows of a block are one contiguous range), then lane r of the first wave
-// walks row r in LDS (pitch padded by 16 bytes: lanes fall into different banks), then the whole
-// block writes the normed rows from the LDS copy - the input is read from memory once.
+// The chain of d dependent additions per row is the floor of this kernel (1.9 us for 768 columns).  To keep everything
+// else off that chain, a block copies its R rows into LDS with every lane's loads in flight at once (the rows of a block
+// are one contiguous range) and lays their squares beside them, lane r of the first wave adds up the squares of row r,
+// then the whole block writes the normed rows from the LDS copy - the input is read from memory once.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float inverse_rms_of(float sum, int d, float eps) {
-    const float mean_square = __fdiv_rn(sum, (float)d);
-    // The root must be the correctly rounded one (the reference's f32::sqrt): taken in double and rounded once,
-    // which is exact for a square root; the single-precision root instruction alone is not.
-    const float root = (float)sqrt((double)__fadd_rn(mean_square, eps));
-    return __fdiv_rn(1.0f, root);
-}
-
 template <typename XT>
 __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const XT* __restrict__ x, const float* __restrict__ weight,
-                                                           float eps, int T, int d, int R, int pitch,
-                                                           XT* __restrict__ out) {
+                                                           float eps, int T, int d, int R, XT* __restrict__ out) {
     constexpr int VN = Vec16<XT>::N;
-    extern __shared__ __attribute__((aligned(16))) char smem[];  // R rows of `pitch` bytes, then R floats
-    float* const inv = reinterpret_cast<float*>(smem + (size_t)R * pitch);
+    extern __shared__ __attribute__((aligned(16))) char smem[];  // R rows, R rows of squares d + 4 floats apart, 256 bytes
+    XT* const rows = reinterpret_cast<XT*>(smem);
+    float* const sq = reinterpret_cast<float*>(smem + (((size_t)R * d * sizeof(XT) + 15) & ~(size_t)15));
+    const int sp = d + 4;
     const int tid = threadIdx.x;
     const int row0 = blockIdx.x * R;
     const int nrows = min(R, T - row0);
-    const int pieces = d / VN;  // d is a multiple of VN (checked by the launcher)
+    const int pieces = d / VN;  // d is a multiple of 8 (checked by the launcher)
+    const uint32_t recip = (uint32_t)(0x100000000ull / (uint32_t)pieces) + 1u;  // idx / pieces, exact for a block's few thousand
     const XT* const src = x + (size_t)row0 * d;
+#pragma unroll 4
     for (int idx = tid; idx < nrows * pieces; idx += 256) {
-        const int r = idx / pieces, p = idx - r * pieces;
-        *reinterpret_cast<uint4*>(smem + (size_t)r * pitch + p * 16) =
-            *reinterpret_cast<const uint4*>(src + (size_t)idx * VN);
+        const int r = pieces == 1 ? idx : (int)__umulhi((uint32_t)idx, recip), p = idx - r * pieces;
+        const uint4 raw = *reinterpret_cast<const uint4*>(src + (size_t)idx * VN);
+        *reinterpret_cast<uint4*>(rows + (size_t)idx * VN) = raw;
+        float v[VN];
+        Vec16<XT>::widen(raw, v);
+        float4* const s4 = reinterpret_cast<float4*>(sq + r * sp + p * VN);
+#pragma unroll
+        for (int q = 0; q < VN / 4; ++q)
+            s4[q] = make_float4(__fmul_rn(v[4 * q], v[4 * q]), __fmul_rn(v[4 * q + 1], v[4 * q + 1]),
+                                __fmul_rn(v[4 * q + 2], v[4 * q + 2]), __fmul_rn(v[4 * q + 3], v[4 * q + 3]));
     }
     __syncthreads();
     if (tid < nrows) {
-        const XT* const row = reinterpret_cast<const XT*>(smem + (size_t)tid * pitch);
-        float sum = 0.0f;
-#pragma unroll 4
-        for (int c = 0; c < d; c += VN) {
-            float v[VN];
-            Vec16<XT>::load(row + c, v);
-#pragma unroll
-            for (int i = 0; i < VN; ++i) sum = __fadd_rn(sum, __fmul_rn(v[i], v[i]));
-        }
-        inv[tid] = inverse_rms_of(sum, d, eps);
+        const float f = inverse_rms_of(ordered_sum(sq + tid * sp, d), d, eps);
+        sq[tid * sp] = f;  // (the row's squares are used up)
     }
     __syncthreads();
     XT* const dst = out + (size_t)row0 * d;
     for (int idx = tid; idx < nrows * pieces; idx += 256) {
-        const int r = idx / pieces, p = idx - r * pieces;
+        const int r = pieces == 1 ? idx : (int)__umulhi((uint32_t)idx, recip), p = idx - r * pieces;
         float v[VN], o[VN];
-        Vec16<XT>::load(reinterpret_cast<const XT*>(smem + (size_t)r * pitch + p * 16), v);
-        const float s = inv[r];
+        Vec16<XT>::load(rows + (size_t)idx * VN, v);
+        const float s = sq[r * sp];
         const float4* w = reinterpret_cast<const float4*>(weight + p * VN);
 #pragma unroll
         for (int q = 0; q < VN / 4; ++q) {
@@ -1645,15 +1975,15 @@ __global__ __launch_bounds__(64) void rmsnorm_rows_direct_kernel(const XT* __res
 
 template <typename XT>
 hipError_t launch_rmsnorm_t(const XT* x, const float* weight, float eps, int T, int d, XT* out, hipStream_t s) {
-    constexpr int VN = Vec16<XT>::N;
-    const int pitch = d * (int)sizeof(XT) + 16;
-    const bool pieces_ok = d % VN == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+    const bool pieces_ok = d % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
                            (reinterpret_cast<uintptr_t>(out) & 15) == 0 && (reinterpret_cast<uintptr_t>(weight) & 15) == 0;
-    if (pieces_ok && pitch + 4 <= 40 * 1024) {
-        const int R = std::max(1, std::min(64, (32 * 1024) / pitch));
-        const size_t lds = (size_t)R * pitch + (size_t)R * 4;
-        RB_LAUNCH(rmsnorm_rows_kernel<XT>, dim3((T + R - 1) / R), dim3(256), lds, s, x, weight, eps, T, d, R,
-                           pitch, out);
+    // rows a block: few enough that the rows' chains spread over the chip (the chain of one row is the time of a small
+    // call), enough blocks a compute unit for the loads of one to cover the chain of another
+    auto lds_of = [&](int R) { return (((size_t)R * d * sizeof(XT) + 15) & ~(size_t)15) + (size_t)R * (d + 4) * 4 + 256; };
+    if (pieces_ok && lds_of(1) <= 64 * 1024) {
+        int R = std::max(1, std::min(16, (T + 1023) / 1024));
+        while (R > 1 && lds_of(R) > 40 * 1024) --R;
+        RB_LAUNCH(rmsnorm_rows_kernel<XT>, dim3((T + R - 1) / R), dim3(256), lds_of(R), s, x, weight, eps, T, d, R, out);
     } else {
         RB_LAUNCH(rmsnorm_rows_direct_kernel<XT>, dim3((T + 63) / 64), dim3(64), 0, s, x, weight, eps, T, d,
                            out);

@@ -1,0 +1,51 @@
+"""The routing launch that keeps a workgroup's whole rows in LDS: 8, 16 and 32 tokens a workgroup, router rows in one
+group and in several, both routers, with and without the norm, and the calls at the edges of its rule."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
+from oracle import rb_oracle as orc
+from rustingbrain_amd import Layout, synth
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    dict(d=64, E=5, k=2, T=33),       # 8 tokens a workgroup, the last one short
+    dict(d=64, E=16, k=3, T=2049),    # the first call with 16 tokens a workgroup
+    dict(d=64, E=9, k=2, T=4097),     # ... and with 32
+    dict(d=1024, E=64, k=6, T=40),    # router rows in groups
+    dict(d=1024, E=16, k=2, T=4100),  # 32 tokens do not fit, the norm takes a launch of its own
+    dict(d=320, E=12, k=2, T=300),    # lanes of 40 steps (8 lanes) and of 10: a last piece with zeros (32 lanes)
+    dict(d=1024, E=33, k=2, T=4200),  # block histograms past the limit of the fused layout scan
+]
+
+
+@pytest.mark.parametrize("act,quantized", [("bf16", False), ("f32", False), ("bf16", True), ("f32", True)])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "d{d}_E{E}_k{k}_T{T}".format(**s))
+def test_block_step_routes_like_the_oracle(device, shape, act, quantized):
+    t = synth.make(small_workload(F=64, seed=91, act=act, wt="int8" if quantized else "bf16", **shape))
+    T, d = shape["T"], shape["d"]
+    layer = gpu_layer(device, t)
+    ref_layer = oracle_layer(t)
+    if quantized:
+        q, s = synth.quantize_rows(t.router)
+        layer.set_router_q8(q, s)
+        ref_layer.router_q, ref_layer.router_s = q, s
+    w = (1.0 + 0.1 * synth.normal((d,), 1.0, 91, 97)).astype(np.float32)
+    layer.set_feed_forward_norm(w, 1e-6)
+    valid = (np.arange(T) % 7 != 3).astype(np.uint8)
+    out, cache = layer.forward_block(t.x, Layout(valid=[bool(v) for v in valid]))
+    normed = orc.rmsnorm(t.x, w, 1e-6)
+    if act == "bf16":
+        normed = synth.round_bf16(normed)
+    ref = ref_layer.forward(normed, valid=valid, threads=8)
+    assert_routing_identical(cache, ref)
+    assert rel_l2(out, ref.out + t.x) <= 2e-2
+    plain, cache = layer.forward_train(t.x)     # without the norm
+    ref = ref_layer.forward(t.x, threads=8)
+    assert_routing_identical(cache, ref)
+    assert rel_l2(plain, ref.out) <= 2e-2
+    assert abs(cache.aux_loss() - ref.aux_loss) <= 1e-5 * abs(ref.aux_loss)
+    assert abs(cache.z_loss() - ref.z_loss) <= 1e-5 * abs(ref.z_loss)
+    layer.close()

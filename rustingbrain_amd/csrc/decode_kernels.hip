@@ -14,9 +14,10 @@
 // workgroups per expert (decode_down_by_expert_kernel): two launches.  The products are spread over (tile,
 // 32-feature block) workgroups whose waves split the reduction dimension, so that a few hundred kilobytes of
 // weight fragments are in flight per CU and every byte of a touched expert is fetched exactly once per 32-row tile.
+#include <atomic>
 #include <type_traits>
 
-#include "rbmoe_kernels.h"
+#include "routing_device.h"
 
 namespace rbmoe {
 
@@ -32,11 +33,6 @@ constexpr int kStageBytes = 96 * 1024;  // LDS for the staged router and token r
 // LDS of the routing code behind the staging area: prob, lsev, sexp, cnt, off, aux_term (see route_small_body)
 constexpr int kRouteFixedBytes = (kSmallRouteMaxPairs + kSmallRouteMaxTokens + kSmallRouteMaxTokens * kMaxTopK +
                                   2 * (kMaxExperts + 1) + kMaxExperts) * 4 + 64;
-// The launch that runs the routing beside the gate/up products (decode_front_kernel) keeps two workgroups on a
-// compute unit: 80 KiB each, of which the routing workgroup stages rows in this much.
-constexpr int kFrontLdsBytes = 80 * 1024;
-constexpr int kFrontStageBytes = (kFrontLdsBytes - kRouteFixedBytes) / 16 * 16;
-
 // softmax_rows (src/moe.rs, softmax over one row) and route (src/moe.rs:553-593) of one token, by one
 // thread, the row used where it lies in LDS: the path for more experts than a wave has lanes.
 __device__ __forceinline__ void token_phase_serial(float* row, int t, int E, int k, const uint8_t* valid, float* P,
@@ -180,6 +176,212 @@ __device__ __forceinline__ void token_phase_lanes(float* row_lds, int t, int j, 
     }
 }
 
+// What a routed call leaves for its consumers (see Work).
+struct SmallTables {
+    int *counts, *offsets, *tile_expert, *tile_row0, *tile_rows, *ntiles;
+    float* losses;
+    int *perm_slot, *perm_token, *inv_pos;
+};
+
+// The bucket loop and the losses of a call of at most 32 tokens, by one workgroup of kSmallThreads: `prob` [T, E]
+// probabilities, `lsev` [T], `sexp` [T k] experts of the slots (-1: none), all in LDS and met at a barrier; `cnt`, `off`
+// [kMaxExperts + 1] and `aux_term` [kMaxExperts]: scratch in LDS.
+__device__ __forceinline__ void small_layout(const float* __restrict__ prob, const float* __restrict__ lsev, const int* __restrict__ sexp,
+                                             int* __restrict__ cnt, int* __restrict__ off, float* __restrict__ aux_term,
+                                             const uint8_t* __restrict__ valid, int T, int E, int k, float w_aux, float w_z,
+                                             int tile_m, const SmallTables& o) {
+    int* __restrict__ const counts = o.counts;
+    int* __restrict__ const offsets = o.offsets;
+    int* __restrict__ const tile_expert = o.tile_expert;
+    int* __restrict__ const tile_row0 = o.tile_row0;
+    int* __restrict__ const tile_rows = o.tile_rows;
+    int* __restrict__ const ntiles = o.ntiles;
+    float* __restrict__ const losses = o.losses;
+    int* __restrict__ const perm_slot = o.perm_slot;
+    int* __restrict__ const perm_token = o.perm_token;
+    int* __restrict__ const inv_pos = o.inv_pos;
+    const int tid = threadIdx.x;
+    const int S = T * k;
+    // ---- bucket loop: a stable counting sort of the slots by expert ----------------
+    // With at most 64 slots and 64 experts the first wave sorts and the second wave works out the two losses beside
+    // it (same formulas and orders as the general code at the end; the per-expert counts it needs are ballots of
+    // its own), and nothing is left to wait for.
+    const bool side_losses = S <= 64 && E <= 64;
+    if (side_losses && tid >= 64 && tid < 128) {
+        const int ln = tid - 64;
+        const int my = ln < S ? sexp[ln] : -1;
+        int c_mine = 0;  // lane e: slots of expert e
+        for (int e = 0; e < E; ++e) {
+            const int c = __popcll(__ballot(my == e));
+            if (ln == e) c_mine = c;
+        }
+        int V = 0;
+        for (int t = 0; t < T; ++t) V += ((valid == nullptr) || valid[t]) ? 1 : 0;
+        if (ln < E) {
+            float term = 0.0f;
+            if (V > 0) {
+                const float load = (float)c_mine / ((float)V * (float)k);
+                float mass = 0.0f;
+                for (int t = 0; t < T; ++t)
+                    if ((valid == nullptr) || valid[t]) mass = mass + prob[t * E + ln];
+                mass = mass / (float)V;
+                term = load * mass;
+            }
+            aux_term[ln] = term;
+        }
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's LDS writes have landed
+        __builtin_amdgcn_wave_barrier();
+        if (ln == 0) {
+            float aux = 0.0f, z = 0.0f;
+            if (V > 0) {
+                for (int e = 0; e < E; ++e) aux = aux + aux_term[e];
+                aux = aux * ((float)E * w_aux);
+                float zs = 0.0f;
+                for (int t = 0; t < T; ++t)
+                    if ((valid == nullptr) || valid[t]) zs = zs + lsev[t] * lsev[t];
+                z = w_z * zs / (float)V;
+            }
+            losses[0] = aux;
+            losses[1] = z;
+        }
+    }
+    if (S <= 64) {
+        // one wave, slot = lane: a ballot per expert gives its count and every slot's rank
+        if (tid < 64) {
+            const int my = tid < S ? sexp[tid] : -1;
+            int run = 0, tiles = 0;
+            if (E <= 64) {
+                // the loop keeps everything in registers - slot `tid` its position, lane e expert e's count, first
+                // position and first tile - and every store follows it, side by side
+                int pos = -1, e_cnt = 0, e_off = 0, e_tile0 = 0;
+                for (int e = 0; e < E; ++e) {
+                    const unsigned long long mask = __ballot(my == e);
+                    const int c = __popcll(mask);
+                    pos = my == e ? run + __popcll(mask & ((1ull << tid) - 1ull)) : pos;
+                    e_cnt = tid == e ? c : e_cnt;
+                    e_off = tid == e ? run : e_off;
+                    e_tile0 = tid == e ? tiles : e_tile0;
+                    run += c;
+                    tiles += c <= tile_m ? (c > 0 ? 1 : 0) : (c + tile_m - 1) / tile_m;
+                }
+                if (my >= 0) {
+                    perm_slot[pos] = tid;
+                    perm_token[pos] = tid / k;
+                    inv_pos[tid] = pos;
+                }
+                if (tid < E) {
+                    cnt[tid] = e_cnt;
+                    counts[tid] = e_cnt;
+                    offsets[tid] = e_off;
+                    for (int r0 = 0, ti = e_tile0; r0 < e_cnt; r0 += tile_m, ++ti) {
+                        tile_expert[ti] = tid;
+                        tile_row0[ti] = e_off + r0;
+                        tile_rows[ti] = min(tile_m, e_cnt - r0);
+                    }
+                }
+            } else
+            for (int e = 0; e < E; ++e) {
+                const unsigned long long mask = __ballot(my == e);
+                const int c = __popcll(mask);
+                if (my == e) {
+                    const int pos = run + __popcll(mask & ((1ull << tid) - 1ull));
+                    perm_slot[pos] = tid;
+                    perm_token[pos] = tid / k;
+                    inv_pos[tid] = pos;
+                }
+                if (tid == 0) {
+                    cnt[e] = c;
+                    counts[e] = c;
+                    offsets[e] = run;
+                    for (int r0 = 0; r0 < c; r0 += tile_m) {
+                        tile_expert[tiles] = e;
+                        tile_row0[tiles] = run + r0;
+                        tile_rows[tiles] = min(tile_m, c - r0);
+                        ++tiles;
+                    }
+                }
+                run += c;
+            }
+            if (tid < S && my < 0) inv_pos[tid] = -1;
+            if (tid == 0) {
+                offsets[E] = run;
+                ntiles[0] = tiles;
+            }
+        }
+    } else {
+        // one expert per thread, slots in increasing order
+        for (int e = tid; e < E; e += kSmallThreads) {
+            int c = 0;
+            for (int s = 0; s < S; ++s) c += (sexp[s] == e) ? 1 : 0;
+            cnt[e] = c;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            int run = 0, tiles = 0;
+            for (int e = 0; e < E; ++e) {
+                off[e] = run;
+                counts[e] = cnt[e];
+                offsets[e] = run;
+                for (int r0 = 0; r0 < cnt[e]; r0 += tile_m) {
+                    tile_expert[tiles] = e;
+                    tile_row0[tiles] = run + r0;
+                    tile_rows[tiles] = min(tile_m, cnt[e] - r0);
+                    ++tiles;
+                }
+                run += cnt[e];
+            }
+            off[E] = run;
+            offsets[E] = run;
+            ntiles[0] = tiles;
+        }
+        for (int s = tid; s < S; s += kSmallThreads)
+            if (sexp[s] < 0) inv_pos[s] = -1;
+        __syncthreads();
+        for (int e = tid; e < E; e += kSmallThreads) {
+            int pos = off[e];
+            for (int s = 0; s < S; ++s)
+                if (sexp[s] == e) {
+                    perm_slot[pos] = s;
+                    perm_token[pos] = s / k;
+                    inv_pos[s] = pos;
+                    ++pos;
+                }
+        }
+    }
+    if (side_losses) return;
+    __syncthreads();
+
+    // ---- auxiliary losses (src/moe.rs:325-337): per expert in token order ---------
+    int V = 0;
+    for (int t = 0; t < T; ++t) V += ((valid == nullptr) || valid[t]) ? 1 : 0;
+    for (int e = tid; e < E; e += kSmallThreads) {
+        float term = 0.0f;
+        if (V > 0) {
+            const float load = (float)cnt[e] / ((float)V * (float)k);
+            float mass = 0.0f;
+            for (int t = 0; t < T; ++t)
+                if ((valid == nullptr) || valid[t]) mass = mass + prob[t * E + e];
+            mass = mass / (float)V;
+            term = load * mass;
+        }
+        aux_term[e] = term;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        float aux = 0.0f, z = 0.0f;
+        if (V > 0) {
+            for (int e = 0; e < E; ++e) aux = aux + aux_term[e];
+            aux = aux * ((float)E * w_aux);
+            float zs = 0.0f;
+            for (int t = 0; t < T; ++t)
+                if ((valid == nullptr) || valid[t]) zs = zs + lsev[t] * lsev[t];
+            z = w_z * zs / (float)V;
+        }
+        losses[0] = aux;
+        losses[1] = z;
+    }
+}
+
 // STAGE = bytes of `smem` for the staged router and token rows; the routing arrays follow them.
 template <typename XT, int STAGE>
 __device__ __forceinline__ void route_small_body(
@@ -191,7 +393,7 @@ __device__ __forceinline__ void route_small_body(
     int* __restrict__ tile_row0, int* __restrict__ tile_rows, int* __restrict__ ntiles,
     float* __restrict__ losses, int* __restrict__ perm_slot, int* __restrict__ perm_token,
     int* __restrict__ inv_pos, const float* __restrict__ norm_w, float norm_eps, XT* __restrict__ xn_out,
-    bf16_t* __restrict__ rows16, unsigned int* __restrict__ expert_tokens = nullptr) {
+    bf16_t* __restrict__ rows16) {
     static_assert(STAGE % 16 == 0, "the arrays behind the staging area stay aligned");
     unsigned char* const stage = smem;
     float* const prob = reinterpret_cast<float*>(smem + STAGE);                 // [kSmallRouteMaxPairs]
@@ -203,7 +405,6 @@ __device__ __forceinline__ void route_small_body(
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int S = T * k;
 
     // ---- logits ---------------------------------------------------------------
     // When they fit, the router rows and the token rows are first copied to LDS with wide
@@ -384,198 +585,8 @@ __device__ __forceinline__ void route_small_body(
     }
     __syncthreads();
 
-    // ---- bucket loop: a stable counting sort of the slots by expert ----------------
-    // With at most 64 slots and 64 experts the first wave sorts and the second wave works out the two losses beside
-    // it (same formulas and orders as the general code at the end; the per-expert counts it needs are ballots of
-    // its own), and nothing is left to wait for.
-    const bool side_losses = S <= 64 && E <= 64;
-    if (side_losses && tid >= 64 && tid < 128) {
-        const int ln = tid - 64;
-        const int my = ln < S ? sexp[ln] : -1;
-        int c_mine = 0;  // lane e: slots of expert e
-        for (int e = 0; e < E; ++e) {
-            const int c = __popcll(__ballot(my == e));
-            if (ln == e) c_mine = c;
-        }
-        int V = 0;
-        for (int t = 0; t < T; ++t) V += ((valid == nullptr) || valid[t]) ? 1 : 0;
-        if (ln < E) {
-            float term = 0.0f;
-            if (V > 0) {
-                const float load = (float)c_mine / ((float)V * (float)k);
-                float mass = 0.0f;
-                for (int t = 0; t < T; ++t)
-                    if ((valid == nullptr) || valid[t]) mass = mass + prob[t * E + ln];
-                mass = mass / (float)V;
-                term = load * mass;
-            }
-            aux_term[ln] = term;
-        }
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's LDS writes have landed
-        __builtin_amdgcn_wave_barrier();
-        if (ln == 0) {
-            float aux = 0.0f, z = 0.0f;
-            if (V > 0) {
-                for (int e = 0; e < E; ++e) aux = aux + aux_term[e];
-                aux = aux * ((float)E * w_aux);
-                float zs = 0.0f;
-                for (int t = 0; t < T; ++t)
-                    if ((valid == nullptr) || valid[t]) zs = zs + lsev[t] * lsev[t];
-                z = w_z * zs / (float)V;
-            }
-            losses[0] = aux;
-            losses[1] = z;
-        }
-    }
-    if (S <= 64) {
-        // one wave, slot = lane: a ballot per expert gives its count and every slot's rank
-        if (tid < 64) {
-            const int my = tid < S ? sexp[tid] : -1;
-            int run = 0, tiles = 0;
-            if (expert_tokens != nullptr) {
-                // the tokens of every expert, one bit a token (its rows are these tokens in ascending order: the sort
-                // is stable and a token names an expert at most once), gathered in LDS (`off` is free on this path)
-                for (int e = tid; e < E; e += 64) off[e] = 0;
-                __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-                __builtin_amdgcn_wave_barrier();
-                if (my >= 0) atomicOr(reinterpret_cast<unsigned int*>(&off[my]), 1u << (tid / k));
-                __builtin_amdgcn_s_waitcnt(0xc07f);
-                __builtin_amdgcn_wave_barrier();
-                for (int e = tid; e < E; e += 64) expert_tokens[e] = (unsigned int)off[e];
-            }
-            if (E <= 64) {
-                // the loop keeps everything in registers - slot `tid` its position, lane e expert e's count, first
-                // position and first tile - and every store follows it, side by side
-                int pos = -1, e_cnt = 0, e_off = 0, e_tile0 = 0;
-                for (int e = 0; e < E; ++e) {
-                    const unsigned long long mask = __ballot(my == e);
-                    const int c = __popcll(mask);
-                    pos = my == e ? run + __popcll(mask & ((1ull << tid) - 1ull)) : pos;
-                    e_cnt = tid == e ? c : e_cnt;
-                    e_off = tid == e ? run : e_off;
-                    e_tile0 = tid == e ? tiles : e_tile0;
-                    run += c;
-                    tiles += c <= tile_m ? (c > 0 ? 1 : 0) : (c + tile_m - 1) / tile_m;
-                }
-                if (my >= 0) {
-                    perm_slot[pos] = tid;
-                    perm_token[pos] = tid / k;
-                    inv_pos[tid] = pos;
-                }
-                if (tid < E) {
-                    cnt[tid] = e_cnt;
-                    counts[tid] = e_cnt;
-                    offsets[tid] = e_off;
-                    for (int r0 = 0, ti = e_tile0; r0 < e_cnt; r0 += tile_m, ++ti) {
-                        tile_expert[ti] = tid;
-                        tile_row0[ti] = e_off + r0;
-                        tile_rows[ti] = min(tile_m, e_cnt - r0);
-                    }
-                }
-            } else
-            for (int e = 0; e < E; ++e) {
-                const unsigned long long mask = __ballot(my == e);
-                const int c = __popcll(mask);
-                if (my == e) {
-                    const int pos = run + __popcll(mask & ((1ull << tid) - 1ull));
-                    perm_slot[pos] = tid;
-                    perm_token[pos] = tid / k;
-                    inv_pos[tid] = pos;
-                }
-                if (tid == 0) {
-                    cnt[e] = c;
-                    counts[e] = c;
-                    offsets[e] = run;
-                    for (int r0 = 0; r0 < c; r0 += tile_m) {
-                        tile_expert[tiles] = e;
-                        tile_row0[tiles] = run + r0;
-                        tile_rows[tiles] = min(tile_m, c - r0);
-                        ++tiles;
-                    }
-                }
-                run += c;
-            }
-            if (tid < S && my < 0) inv_pos[tid] = -1;
-            if (tid == 0) {
-                offsets[E] = run;
-                ntiles[0] = tiles;
-            }
-        }
-    } else {
-        // one expert per thread, slots in increasing order
-        for (int e = tid; e < E; e += kSmallThreads) {
-            int c = 0;
-            for (int s = 0; s < S; ++s) c += (sexp[s] == e) ? 1 : 0;
-            cnt[e] = c;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            int run = 0, tiles = 0;
-            for (int e = 0; e < E; ++e) {
-                off[e] = run;
-                counts[e] = cnt[e];
-                offsets[e] = run;
-                for (int r0 = 0; r0 < cnt[e]; r0 += tile_m) {
-                    tile_expert[tiles] = e;
-                    tile_row0[tiles] = run + r0;
-                    tile_rows[tiles] = min(tile_m, cnt[e] - r0);
-                    ++tiles;
-                }
-                run += cnt[e];
-            }
-            off[E] = run;
-            offsets[E] = run;
-            ntiles[0] = tiles;
-        }
-        for (int s = tid; s < S; s += kSmallThreads)
-            if (sexp[s] < 0) inv_pos[s] = -1;
-        __syncthreads();
-        for (int e = tid; e < E; e += kSmallThreads) {
-            int pos = off[e];
-            unsigned int tokens = 0u;
-            for (int s = 0; s < S; ++s)
-                if (sexp[s] == e) {
-                    perm_slot[pos] = s;
-                    perm_token[pos] = s / k;
-                    inv_pos[s] = pos;
-                    tokens |= 1u << (s / k);
-                    ++pos;
-                }
-            if (expert_tokens != nullptr) expert_tokens[e] = tokens;
-        }
-    }
-    if (side_losses) return;
-    __syncthreads();
-
-    // ---- auxiliary losses (src/moe.rs:325-337): per expert in token order ---------
-    int V = 0;
-    for (int t = 0; t < T; ++t) V += ((valid == nullptr) || valid[t]) ? 1 : 0;
-    for (int e = tid; e < E; e += kSmallThreads) {
-        float term = 0.0f;
-        if (V > 0) {
-            const float load = (float)cnt[e] / ((float)V * (float)k);
-            float mass = 0.0f;
-            for (int t = 0; t < T; ++t)
-                if ((valid == nullptr) || valid[t]) mass = mass + prob[t * E + e];
-            mass = mass / (float)V;
-            term = load * mass;
-        }
-        aux_term[e] = term;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        float aux = 0.0f, z = 0.0f;
-        if (V > 0) {
-            for (int e = 0; e < E; ++e) aux = aux + aux_term[e];
-            aux = aux * ((float)E * w_aux);
-            float zs = 0.0f;
-            for (int t = 0; t < T; ++t)
-                if ((valid == nullptr) || valid[t]) zs = zs + lsev[t] * lsev[t];
-            z = w_z * zs / (float)V;
-        }
-        losses[0] = aux;
-        losses[1] = z;
-    }
+    small_layout(prob, lsev, sexp, cnt, off, aux_term, valid, T, E, k, w_aux, w_z, tile_m,
+                 SmallTables{counts, offsets, tile_expert, tile_row0, tile_rows, ntiles, losses, perm_slot, perm_token, inv_pos});
 }
 
 template <typename XT>
@@ -652,24 +663,39 @@ struct DecodeSide {
     // XCDs' L2 caches are not coherent with one another, so such rows are stored with device-scope stores, which
     // go through to memory, and read back with device-scope loads.
     bool coherent_out = false;
+    // rows behind a norm (RowForm with kNorm), in LDS: the norm's weights [K] and the rows' factors [32]
+    const float* norm_w = nullptr;
+    const float* row_factor = nullptr;
 };
 
-// NW = waves of a workgroup, each with 1 / NW of the reduction steps: 4 for the gate/up product, 8 for the
-// down product (a third of the workgroups and twice the reduction length: with 8 waves every weight byte of
-// the launch is requested before the first multiply there as well).
-// The rows of a routed expert as the routing leaves them for a launch with one workgroup row per expert
-// (decode_down_by_expert_kernel): the tokens the expert takes, one bit a token, and the position of its first row.
-// The words are fetched behind the first weight loads (LATE_ROWS): nothing the weights' addresses need waits for them.
+// The rows a product reads.  XT: bf16, or f32 rounded to bf16 on the way (the product's precision either way).  NORM: the
+// rows are raw and the product is taken of their normed form, value * factor * weight with the norm's own roundings
+// (src/norm.rs:41-61), as if the normed rows had been written out first.
+template <typename XT, bool NORM>
+struct RowForm {
+    typedef XT type;
+    static constexpr bool kNorm = NORM;
+    static constexpr bool kPlain = !NORM && sizeof(XT) == 2;
+};
+struct NoHook {
+    __device__ __forceinline__ void operator()() const {}
+};
+
+// For a launch with one row of workgroups per EXPERT (decode_down_by_expert_kernel): which rows the expert has is read off
+// the experts of the call's slots, fetched in front of the first weight loads and looked at behind them.
+constexpr int kLateRounds = 4;  // 64 slots a round: at most 8 slots a token
 struct LateRows {
-    const unsigned int* tokens;  // the expert's word
-    const int* first;            // the expert's word
-    const int* with_rows;        // experts with rows (one word for the launch)
-    bool routed;  // false: the side's rows are sd.row0 / sd.rows as they stand (the shared expert)
-    int with_rows_out = 0;
+    const int* expert_of;  // [S]
+    int S, k, expert;
+    int* row_slot;         // LDS [32]: the slot of every row of the side, ascending
+    bool routed;           // false: the side's rows are sd.row0 / sd.rows as they stand (the shared expert)
 };
 
-template <bool SWIGLU, bool I8, int NW, int BATCH, int TEAMS = 1, bool LATE_ROWS = false>
-__device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* red_raw, LateRows* late = nullptr);
+template <bool SWIGLU, bool I8, int NW, int BATCH, int TEAMS = 1, bool LATE_ROWS = false, typename ROWS = RowForm<bf16_t, false>,
+          typename HOOK = NoHook>
+__device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* red_raw, LateRows* late = nullptr, HOOK hook = HOOK{});
+
+constexpr int kCombineEarlySlots = 4;  // slots a token up to which a thread fetches what the combine needs beforehand
 
 // The combine of a decode-shaped call, for the 32 output features of block `fb` and every token: what
 // combine_vec_kernel computes, element by element in the same order (the token's expert rows by ascending position,
@@ -722,59 +748,68 @@ __device__ __forceinline__ void decode_combine_block(const DecodeGemmArgs& g, in
     }
 }
 
-// What a thread of the folded combine can fetch before its workgroup has multiplied anything: the positions of its
-// token's expert rows in ascending order with their gates (at most four slots a token), and the residual.
-constexpr int kCombineEarlySlots = 4;
+// What a thread of the folded combine can fetch before its workgroup has multiplied anything: where its token's expert rows
+// lie, in ascending expert order once sorted, their gates, and the residual.  BY_SLOT: the expert rows lie in slot order and
+// `key` is the slot's expert; otherwise it is the row's position.  M: slots a token at most.
+template <int M>
 struct CombineEarly {
-    int pos[kCombineEarlySlots];  // as the routing wrote them; slots past k repeat the last one
-    float gate[kCombineEarlySlots];
+    int key[M];  // as the routing wrote them; slots past k repeat the last one
+    float gate[M];
     uint32_t res[2];  // the residual's two elements as they lie in memory: one word of two bf16, or two f32
 };
 
-__device__ __forceinline__ void decode_combine_fetch(const DecodeGemmArgs& g, int fb, CombineEarly& ce) {
+template <int M>
+__device__ __forceinline__ void decode_combine_fetch(const DecodeGemmArgs& g, const int* keys, int fb, CombineEarly<M>& ce) {
     // loads only, none of them looked at here and no branch between them: they return while the weights stream in
     const int t = min((int)threadIdx.x >> 4, g.cmb_T - 1), c = fb * 32 + 2 * ((int)threadIdx.x & 15), k = g.cmb_k;
-    const int* const ip = g.cmb_inv_pos + (size_t)t * k;
+    const int* const ip = keys + (size_t)t * k;
     const float* const gp = g.cmb_gate_of + (size_t)t * k;
 #pragma unroll
-    for (int q = 0; q < kCombineEarlySlots; ++q) {
-        ce.pos[q] = ip[min(q, k - 1)];
+    for (int q = 0; q < M; ++q) {
+        ce.key[q] = ip[min(q, k - 1)];
         ce.gate[q] = gp[min(q, k - 1)];
     }
-    // (without a residual the words of the output's own place are fetched and never used; bf16: the second word is
-    // the first again)
+    // (without a residual the words of the routing's gates are fetched and never used; bf16: the second word is the first
+    // again)
     const int es = g.cmb_f32 ? 4 : 2;
-    const char* const base = static_cast<const char*>(g.cmb_residual ? g.cmb_residual : g.cmb_out);
-    const char* const at = base + ((size_t)t * g.N + c) * es;
+    const char* const at = g.cmb_residual ? static_cast<const char*>(g.cmb_residual) + ((size_t)t * g.N + c) * es
+                                          : reinterpret_cast<const char*>(g.cmb_gate_of);
     ce.res[0] = *reinterpret_cast<const uint32_t*>(at);
-    ce.res[1] = *reinterpret_cast<const uint32_t*>(at + (g.cmb_f32 ? 4 : 0));
+    ce.res[1] = *reinterpret_cast<const uint32_t*>(at + (g.cmb_f32 && g.cmb_residual ? 4 : 0));
 }
 
 // decode_combine_block for a workgroup of 512 threads (one element pair a thread) that fetched `ce` beforehand: the
 // expert rows' loads go out side by side, the sums are taken in the same order.
-template <typename XT>
-__device__ __forceinline__ void decode_combine_block_early(const DecodeGemmArgs& g, int fb, CombineEarly ce) {
+template <typename XT, bool BY_SLOT, int M>
+__device__ __forceinline__ void decode_combine_block_early(const DecodeGemmArgs& g, int fb, CombineEarly<M> ce) {
     const int t = (int)threadIdx.x >> 4, c = fb * 32 + 2 * ((int)threadIdx.x & 15);
     if (t >= g.cmb_T) return;
-    // ascending positions (they are distinct; a padding token's slots and the slots past k have no row): five
-    // exchanges sort four
+    // ascending keys (they are distinct; a padding token's slots and the slots past k have no row), each with its row
+    int row[M];
 #pragma unroll
-    for (int q = 0; q < kCombineEarlySlots; ++q)
-        if (q >= g.cmb_k || ce.pos[q] < 0) ce.pos[q] = 0x7fffffff;
+    for (int q = 0; q < M; ++q) {
+        row[q] = BY_SLOT ? t * g.cmb_k + q : ce.key[q];
+        if (q >= g.cmb_k || ce.key[q] < 0) ce.key[q] = 0x7fffffff;
+    }
     auto order = [&](int a, int b) {
-        if (ce.pos[b] < ce.pos[a]) {
-            const int p = ce.pos[a]; ce.pos[a] = ce.pos[b]; ce.pos[b] = p;
+        if (ce.key[b] < ce.key[a]) {
+            const int p = ce.key[a]; ce.key[a] = ce.key[b]; ce.key[b] = p;
+            const int r = row[a]; row[a] = row[b]; row[b] = r;
             const float w = ce.gate[a]; ce.gate[a] = ce.gate[b]; ce.gate[b] = w;
         }
     };
-    order(0, 1); order(2, 3); order(0, 2); order(1, 3); order(1, 2);
+    // (neighbours exchanged in M rounds, every other pair at a time)
+#pragma unroll
+    for (int round = 0; round < M; ++round)
+#pragma unroll
+        for (int q = round & 1; q + 1 < M; q += 2) order(q, q + 1);
     const bf16_t* const y = static_cast<const bf16_t*>(g.out);
     const int d = g.N;
-    uint32_t v[kCombineEarlySlots], vs = 0u;
+    uint32_t v[M], vs = 0u;
 #pragma unroll
-    for (int q = 0; q < kCombineEarlySlots; ++q)
-        v[q] = ce.pos[q] != 0x7fffffff
-                   ? __hip_atomic_load(reinterpret_cast<const uint32_t*>(y + (size_t)ce.pos[q] * d + c), __ATOMIC_RELAXED,
+    for (int q = 0; q < M; ++q)
+        v[q] = ce.key[q] != 0x7fffffff
+                   ? __hip_atomic_load(reinterpret_cast<const uint32_t*>(y + (size_t)row[q] * d + c), __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_AGENT)
                    : 0u;
     if (g.a_shared)
@@ -782,8 +817,8 @@ __device__ __forceinline__ void decode_combine_block_early(const DecodeGemmArgs&
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
-    for (int q = 0; q < kCombineEarlySlots; ++q)
-        if (ce.pos[q] != 0x7fffffff) {
+    for (int q = 0; q < M; ++q)
+        if (ce.key[q] != 0x7fffffff) {
             a0 = __fadd_rn(a0, __fmul_rn(ce.gate[q], __uint_as_float(v[q] << 16)));
             a1 = __fadd_rn(a1, __fmul_rn(ce.gate[q], __uint_as_float(v[q] & 0xffff0000u)));
         }
@@ -855,8 +890,8 @@ __global__ __launch_bounds__(NW * 64) void decode_gemm_kernel(DecodeGemmArgs g) 
         if (g.cmb_out != nullptr) {  // uniform over the launch
             // eight waves and at most four slots a token: what the combine needs of the routing is fetched now
             const bool early = NW == 8 && g.cmb_k <= kCombineEarlySlots;
-            CombineEarly ce;
-            if (early) decode_combine_fetch(g, fb, ce);
+            CombineEarly<kCombineEarlySlots> ce;
+            if (early) decode_combine_fetch(g, g.cmb_inv_pos, fb, ce);
             if (!works) {
                 // nothing to multiply here; with no writer at all (every row is padding and there is no shared
                 // expert) the first of these workgroups still owes the block its combine
@@ -880,8 +915,8 @@ __global__ __launch_bounds__(NW * 64) void decode_gemm_kernel(DecodeGemmArgs g) 
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
             }
             if (early) {
-                if (g.cmb_f32) decode_combine_block_early<float>(g, fb, ce);
-                else decode_combine_block_early<bf16_t>(g, fb, ce);
+                if (g.cmb_f32) decode_combine_block_early<float, false>(g, fb, ce);
+                else decode_combine_block_early<bf16_t, false>(g, fb, ce);
             } else {
                 if (g.cmb_f32) decode_combine_block<float>(g, fb, NW * 64);
                 else decode_combine_block<bf16_t>(g, fb, NW * 64);
@@ -895,27 +930,63 @@ __global__ __launch_bounds__(NW * 64) void decode_gemm_kernel(DecodeGemmArgs g) 
 
 // ---------------------------------------------------------------------------
 // decode_down_by_expert_kernel: the down product and the folded combine behind decode_front_kernel, blockIdx.y =
-// expert (then the shared expert's 32-row blocks).  decode_gemm_kernel learns its expert from the tile table and
-// its rows from the row index - two dependent trips to memory in front of the weight loads and the token loads;
-// here the weights' address follows from the grid, and the three words that say which rows the expert has (its
-// token bits, its first position, the number of experts with rows) are requested before the weights and looked at
-// behind them.  Every thread also fetches what the combine will need of the routing (positions, gates, residual)
-// before the product, so that the last workgroup of a block has only the expert rows left to load.
+// expert (then the shared expert's 32-row blocks, then one workgroup for the tables).  decode_gemm_kernel learns its
+// expert from the tile table and its rows from the row index - two dependent trips to memory in front of the weight
+// loads and the token loads; here the weights' address follows from the grid, and which rows the expert has is read off
+// the slots' experts, requested before the weights and looked at behind them.  Nothing of the launch waits for the
+// counting sort: expert rows are stored by slot and summed by slot, in ascending expert order, and the tables that
+// callers may ask for (and the losses) are made by a workgroup of their own beside the products.  Every thread also
+// fetches what the combine will need of the routing before the product, so that the last workgroup of a block has only
+// the expert rows left to load.  An expert without rows costs its weights' bytes.
 // Same products, same order of sums: the outputs are decode_gemm_kernel's bit for bit.
 // ---------------------------------------------------------------------------
-template <bool I8>
-__global__ __launch_bounds__(512) void decode_down_by_expert_kernel(DecodeGemmArgs g, const unsigned int* __restrict__ expert_tokens,
-                                                                    const int* __restrict__ offsets, int E) {
-    __shared__ float red[8 * 16 * 64];
+constexpr int kLayoutLdsFloats = kSmallRouteMaxPairs + kSmallRouteMaxTokens + kSmallRouteMaxTokens * kMaxTopK + 2 * (kMaxExperts + 1) +
+                                 kMaxExperts;
+
+// The tables of a call whose probabilities, log-sum-exps and experts lie in memory.
+__device__ __forceinline__ void layout_from_memory(float* lds, const DecodeLayoutArgs& a) {
+    float* const prob = lds;
+    float* const lsev = prob + kSmallRouteMaxPairs;
+    int* const sexp = reinterpret_cast<int*>(lsev + kSmallRouteMaxTokens);
+    int* const cnt = sexp + kSmallRouteMaxTokens * kMaxTopK;
+    int* const off = cnt + (kMaxExperts + 1);
+    float* const aux_term = reinterpret_cast<float*>(off + (kMaxExperts + 1));
+    for (int i = threadIdx.x; i < a.T * a.E; i += kSmallThreads) prob[i] = a.P[i];
+    for (int i = threadIdx.x; i < a.T * a.k; i += kSmallThreads) sexp[i] = a.expert_of[i];
+    for (int i = threadIdx.x; i < a.T; i += kSmallThreads) lsev[i] = a.lse[i];
+    __syncthreads();
+    small_layout(prob, lsev, sexp, cnt, off, aux_term, a.valid, a.T, a.E, a.k, a.w_aux, a.w_z, kDecodeTileM,
+                 SmallTables{a.counts, a.offsets, a.tile_expert, a.tile_row0, a.tile_rows, a.ntiles, a.losses, a.perm_slot,
+                             a.perm_token, a.inv_pos});
+}
+
+// ... in a launch of its own, for a caller that takes the tile-table launch behind decode_front_kernel
+__global__ __launch_bounds__(kSmallThreads) void decode_layout_kernel(DecodeLayoutArgs a) {
+    __shared__ float lds[kLayoutLdsFloats];
+    layout_from_memory(lds, a);
+}
+
+template <bool I8, int M>
+__global__ __launch_bounds__(512) void decode_down_by_expert_kernel(DecodeGemmArgs g, DecodeLayoutArgs t) {
+    constexpr int kRed = 8 * 16 * 64;
+    __shared__ float red[kRed > kLayoutLdsFloats ? kRed : kLayoutLdsFloats];
+    __shared__ int row_slot[32];
     __shared__ int last_of_block;
+    const int E = t.E;
     const int fb = blockIdx.x, side = blockIdx.y;
+    const int shared_tiles = g.a_shared ? (g.T_shared + 31) / 32 : 0;
     const bool routed = side < E;
+    if (side == E + shared_tiles) {
+        if (fb == 0) layout_from_memory(red, t);
+        return;
+    }
     LateRows late;
     late.routed = routed;
-    late.tokens = expert_tokens + (routed ? side : 0);
-    late.first = offsets + (routed ? side : 0);
-    late.with_rows = g.ntiles;  // one tile an expert: the experts with rows
-    const int shared_tiles = g.a_shared ? (g.T_shared + 31) / 32 : 0;
+    late.expert_of = t.expert_of;
+    late.S = t.T * t.k;
+    late.k = t.k;
+    late.expert = side;
+    late.row_slot = row_slot;
     DecodeSide sd;
     sd.row_index = nullptr;
     sd.a_row0 = 0;
@@ -942,28 +1013,22 @@ __global__ __launch_bounds__(512) void decode_down_by_expert_kernel(DecodeGemmAr
         sd.row0 = st * 32;
         sd.rows = min(32, g.T_shared - sd.row0);
     }
-    CombineEarly ce;
-    decode_combine_fetch(g, fb, ce);
+    CombineEarly<M> ce;
+    decode_combine_fetch(g, t.expert_of, fb, ce);
     decode_gemm_body<false, I8, 8, kBatch, 1, true>(sd, fb, red, &late);
-    const bool works = sd.rows > 0;
-    const int writers = late.with_rows_out + shared_tiles;
-    if (!works) {
-        // nothing to multiply here; with no writer at all (every row is padding and there is no shared expert) the
-        // first side's workgroups still owe their blocks the combine
-        if (writers != 0 || side != 0) return;
-    } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the row stores have been acknowledged
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const int before = atomicAdd(&g.cmb_counter[fb * kDecodeCombineCounterStride], 1);
-            last_of_block = before == writers - 1;
-            if (before == writers - 1) atomicExch(&g.cmb_counter[fb * kDecodeCombineCounterStride], 0);  // every writer has arrived: ready for the next launch
-        }
-        __syncthreads();
-        if (!last_of_block) return;
+    // every side of the block arrives, with rows or without
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the row stores have been acknowledged
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int writers = E + shared_tiles;
+        const int before = atomicAdd(&g.cmb_counter[fb * kDecodeCombineCounterStride], 1);
+        last_of_block = before == writers - 1;
+        if (before == writers - 1) atomicExch(&g.cmb_counter[fb * kDecodeCombineCounterStride], 0);  // every writer has arrived: ready for the next launch
     }
-    if (g.cmb_f32) decode_combine_block_early<float>(g, fb, ce);
-    else decode_combine_block_early<bf16_t>(g, fb, ce);
+    __syncthreads();
+    if (!last_of_block) return;
+    if (g.cmb_f32) decode_combine_block_early<float, true>(g, fb, ce);
+    else decode_combine_block_early<bf16_t, true>(g, fb, ce);
 }
 
 // red_raw: TEAMS * NW * (SWIGLU ? 2 : 1) * 1024 floats of LDS; BATCH: reduction steps whose loads a wave issues together.
@@ -971,9 +1036,11 @@ __global__ __launch_bounds__(512) void decode_down_by_expert_kernel(DecodeGemmAr
 // every team its block; a team without one has left the kernel before: the barrier below counts the waves that
 // are still there).
 // LATE_ROWS: which rows the side has is looked at behind the first weight loads (`late`); a side without rows leaves
-// with sd.rows == 0 and nothing stored.
-template <bool SWIGLU, bool I8, int NW, int BATCH, int TEAMS, bool LATE_ROWS>
-__device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* red_raw, LateRows* late) {
+// with sd.rows == 0 and nothing stored, and row r is stored at its slot.
+// hook(): what the workgroup does between the first weight loads and the first look at a row (every wave runs it once; it
+// leaves everything it puts into LDS behind a barrier, and `red_raw` free).
+template <bool SWIGLU, bool I8, int NW, int BATCH, int TEAMS, bool LATE_ROWS, typename ROWS, typename HOOK>
+__device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* red_raw, LateRows* late, HOOK hook) {
     const int team = TEAMS > 1 ? (int)threadIdx.x / (NW * 64) : 0;
     float (*red)[SWIGLU ? 2 : 1][16][64] =
         reinterpret_cast<float (*)[SWIGLU ? 2 : 1][16][64]>(red_raw + (size_t)team * NW * (SWIGLU ? 2 : 1) * 1024);
@@ -1009,13 +1076,20 @@ __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* 
     floatx16 acc0, acc1;
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc0[v] = acc1[v] = 0.0f;
+    float row_factor = 1.0f;  // ROWS::kNorm: of this lane's token
+    int slot_expert[LATE_ROWS ? kLateRounds : 1];  // lane l: the experts of slots l, l + 64, ... (past the last: nobody's)
+    if constexpr (LATE_ROWS) {
+#pragma unroll
+        for (int i = 0; i < kLateRounds; ++i) slot_expert[i] = late->expert_of[min(lane + 64 * i, late->S - 1)];
+    }
 
     // One batch of reduction steps.  The first batch stands in front of the loop over the others, as straight
     // code: at the head of a loop the compiler waits for every load still under way - the row index, what the
     // combine fetched early - before the first weight load could go out.  Returns true when the side has no rows.
     auto batch = [&](const int s0, auto first_tag) -> bool {
         constexpr bool kFirst = decltype(first_tag)::value;
-        bf16x8 wa[BATCH], wb[BATCH], tf[BATCH];
+        bf16x8 wa[BATCH], wb[BATCH];
+        uint4 raw[BATCH][ROWS::kPlain || sizeof(typename ROWS::type) == 2 ? 1 : 2];
         // the weights first: the address of a token row depends on a load of its own (the row index), and
         // loads are issued in order - nothing of the stream may queue up behind that wait
 #pragma unroll
@@ -1026,57 +1100,84 @@ __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* 
         }
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (LATE_ROWS && kFirst) {
-            {
-                // the three words, by scalar loads issued here and nowhere earlier (the compiler would fetch them
-                // in front of the weights, or with vector loads that queue up behind them)
-                unsigned int tokens;
-                int first, with_rows;
-                asm volatile(
-                    "s_load_dword %0, %3, 0x0\n\t"
-                    "s_load_dword %1, %4, 0x0\n\t"
-                    "s_load_dword %2, %5, 0x0\n\t"
-                    "s_waitcnt lgkmcnt(0)"
-                    : "=&s"(tokens), "=&s"(first), "=&s"(with_rows)
-                    : "s"(late->tokens), "s"(late->first), "s"(late->with_rows)
-                    : "memory");
-                late->with_rows_out = with_rows;
-                if (late->routed) {
-                    sd.rows = __popc(tokens);
-                    sd.row0 = first;
+            if (late->routed) {
+                // the expert's rows in slot order: a matching lane pushes its slot to the lane numbered by the row
+                int rows = 0, slot = 0;
+#pragma unroll
+                for (int i = 0; i < kLateRounds; ++i) {
+                    if (64 * i >= late->S) break;  // uniform
+                    const bool mine = lane + 64 * i < late->S && slot_expert[i] == late->expert;
+                    const unsigned long long m = __ballot(mine);
+                    const int rank = rows + __popcll(m & ((1ull << lane) - 1ull));  // below 32: a token names an expert once
+                    const int pushed = __builtin_amdgcn_ds_permute(4 * (mine ? rank : 63), lane + 64 * i);
+                    const int upto = rows + __popcll(m);
+                    slot = lane >= rows && lane < upto ? pushed : slot;
+                    rows = upto;
                 }
-                if (sd.rows <= 0) return true;  // the whole workgroup
-                const int trow = (lane & 31) < sd.rows ? (lane & 31) : 0;
-                int token = sd.row0 + trow;
-                if (late->routed) {  // row `trow` of the expert: the token of its set bit number `trow`
-                    unsigned int rest = tokens;
-                    for (int i = 0; i < trow; ++i) rest &= rest - 1u;
-                    token = __ffs(rest) - 1;
-                }
-                grow = token + sd.a_row0;
+                sd.rows = rows;
+                if (rows <= 0) return true;  // the whole workgroup
+                if (wave == 0 && lane < 32) late->row_slot[lane] = slot;
+                const int trow = (lane & 31) < rows ? (lane & 31) : 0;
+                const int mine_slot = __shfl(slot, trow);
+                grow = mine_slot / late->k + sd.a_row0;
+            } else {
+                if (sd.rows <= 0) return true;
+                grow = sd.row0 + ((lane & 31) < sd.rows ? (lane & 31) : 0);
             }
         }
         // (the empty statement pins the first use of the row index, and with it the wait for it, below the
         // weight loads; the barriers keep every load of the batch ahead of the first multiply)
         asm volatile("" : "+v"(grow));
-        const bf16_t* arow = sd.a + (size_t)grow * K + 8 * (lane >> 5);
+        const typename ROWS::type* arow = reinterpret_cast<const typename ROWS::type*>(sd.a) + (size_t)grow * K + 8 * (lane >> 5);
 #pragma unroll
         for (int u = 0; u < BATCH; ++u) {
             const int s = min(s0 + u, g1 - 1);
-            tf[u] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(arow + 16 * s));
+            const uint4* const from = reinterpret_cast<const uint4*>(arow + 16 * s);
+            raw[u][0] = from[0];
+            if constexpr (sizeof(typename ROWS::type) == 4) raw[u][1] = from[1];
         }
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kFirst && !std::is_same<HOOK, NoHook>::value) {
+            hook();
+            if constexpr (ROWS::kNorm) row_factor = sd.row_factor[lane & 31];
+        }
+        auto fragment = [&](int u) -> bf16x8 {
+            if constexpr (ROWS::kPlain) {
+                return __builtin_bit_cast(bf16x8, raw[u][0]);
+            } else {
+                float v[8];
+                if constexpr (sizeof(typename ROWS::type) == 2) {
+                    Vec16<bf16_t>::widen(raw[u][0], v);
+                } else {
+                    float lo[4], hi[4];
+                    Vec16<float>::widen(raw[u][0], lo);
+                    Vec16<float>::widen(raw[u][1], hi);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] = lo[q], v[4 + q] = hi[q];
+                }
+                if constexpr (ROWS::kNorm) {
+                    const float* const nw = sd.norm_w + 16 * (s0 + u) + 8 * (lane >> 5);
+                    const float4 na = *reinterpret_cast<const float4*>(nw), nb = *reinterpret_cast<const float4*>(nw + 4);
+                    const float n[8] = {na.x, na.y, na.z, na.w, nb.x, nb.y, nb.z, nb.w};
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) v[q] = __fmul_rn(__fmul_rn(v[q], row_factor), n[q]);
+                }
+                return __builtin_bit_cast(bf16x8, make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])));
+            }
+        };
 #pragma unroll
         for (int u = 0; u < BATCH; ++u) {
             if (s0 + u < g1) {
-                acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa[u], tf[u], acc0, 0, 0, 0);
-                if constexpr (SWIGLU) acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb[u], tf[u], acc1, 0, 0, 0);
+                const bf16x8 tf = fragment(u);
+                acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wa[u], tf, acc0, 0, 0, 0);
+                if constexpr (SWIGLU) acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb[u], tf, acc1, 0, 0, 0);
             }
         }
         return false;
     };
     // (LATE_ROWS: every wave takes the first batch, also one without a reduction step of its own, so that all of
     // them learn the rows and leave together when there are none)
-    if (LATE_ROWS || g0 < g1) {
+    if (LATE_ROWS || ROWS::kNorm || g0 < g1) {
         if (batch(g0, std::true_type{})) return;
     }
     for (int s0 = g0 + BATCH; s0 < g1; s0 += BATCH) batch(s0, std::false_type{});
@@ -1111,7 +1212,10 @@ __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* 
                 }
                 y4[h] = y;
             }
-            bf16_t* const where = sd.out + (size_t)(sd.out_row0 + sd.row0 + token) * sd.N + fb * 32 + f;
+            int out_row = sd.out_row0 + sd.row0 + token;
+            if constexpr (LATE_ROWS)
+                if (late->routed) out_row = late->row_slot[token];
+            bf16_t* const where = sd.out + (size_t)out_row * sd.N + fb * 32 + f;
             const unsigned long long four =
                 (unsigned long long)((uint32_t)f32_to_bf16_bits(y4[0]) | ((uint32_t)f32_to_bf16_bits(y4[1]) << 16)) |
                 ((unsigned long long)((uint32_t)f32_to_bf16_bits(y4[2]) | ((uint32_t)f32_to_bf16_bits(y4[3]) << 16)) << 32);
@@ -1124,33 +1228,62 @@ __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* 
 }
 
 // ---------------------------------------------------------------------------
-// decode_front_kernel: the routing and the gate/up products in ONE launch, side by side.
-// The routing is one workgroup walking a dependent chain for about ten microseconds; the gate/up
-// product of a routed expert needs nothing of it but WHICH rows the expert takes.  With at most 32
-// tokens an expert's rows are one tile whatever the routing says, so every expert's gate/up product
-// is taken over ALL the call's rows - hidden rows [E][T, F] - without waiting for the routing: an
-// expert that turns out unrouted costs its weights' bytes (the caller takes this launch only when
-// most experts will be touched), the rows nobody routed to an expert cost nothing (the tile is 32
-// rows either way).  Workgroup 0 routes; workgroup 1 + side * (N / 32) + fb takes feature block fb
-// of side `side`: experts 0 .. E-1, then the shared expert's 32-row blocks.  The down product then
-// picks the routed rows out of the per-expert hidden rows (DecodeGemmArgs::a_expert_rows).
+// decode_front_kernel: norm, routing and the gate/up products in ONE launch, side by side.
+// The gate/up product of a routed expert needs nothing of the routing but WHICH rows the expert takes.  With at most 32
+// tokens an expert's rows are one tile whatever the routing says, so every expert's gate/up product is taken over ALL
+// the call's rows - hidden rows [E][T, F] - without waiting for the routing: an expert that turns out unrouted costs its
+// weights' bytes (the caller weighs them against the launch and the chain that this saves), the rows nobody routed to an
+// expert cost nothing (the tile is 32 rows either way).  The first workgroups route, eight tokens each (route_rows_body);
+// the others take two feature blocks of one side each: experts 0 .. E-1, then the shared expert's 32-row blocks.  The
+// products read the call's own rows: a norm in front of the layer is applied on the way (RowForm), f32 rows are rounded.
+// The down product then picks the routed rows out of the per-expert hidden rows (DecodeGemmArgs::a_expert_rows).
 // ---------------------------------------------------------------------------
-template <bool I8>
-__global__ __launch_bounds__(kSmallThreads, 2) void decode_front_kernel(SmallRouteArgs r, DecodeGemmArgs g, int E, int T) {
-    __shared__ __align__(16) unsigned char smem[kFrontLdsBytes];
-    if (blockIdx.x == 0) {
-        route_small_body<bf16_t, kFrontStageBytes>(
-            smem, static_cast<const bf16_t*>(r.x), r.wr, r.bias, r.valid, r.T, r.d, r.E, r.k, r.w_aux, r.w_z, r.tile_m, r.P,
-            r.lse, r.expert_of, r.gate_of, r.counts, r.offsets, r.tile_expert, r.tile_row0, r.tile_rows, r.ntiles, r.losses,
-            r.perm_slot, r.perm_token, r.inv_pos, nullptr, 0.0f, nullptr, nullptr, r.expert_tokens);
+constexpr int kFrontTokens = 8;  // a routing workgroup's
+constexpr int kFrontTeams = 2;   // feature blocks of a product workgroup
+constexpr int kFrontRedFloats = kFrontTeams * 4 * 2 * 1024;  // a product workgroup's partial sums
+// ... which share their room with the rows' squares of a call behind a norm (d + 4 floats a row; 64: the chain reads ahead)
+__host__ __device__ static int front_room_floats(int T, int d, bool norm) {
+    const int squares = norm ? T * (d + 4) + 64 : 0;
+    return squares > kFrontRedFloats ? squares : kFrontRedFloats;
+}
+
+template <typename XT, bool I8, bool Q8, bool NORM>
+__global__ __launch_bounds__(kSmallThreads, 2) void decode_front_kernel(RouteRowsArgs r, DecodeGemmArgs g, int routers) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int E = r.E, T = r.T;
+    if ((int)blockIdx.x < routers) {
+        const int k = r.k, ES = E | 1;
+        const int t0 = blockIdx.x * kFrontTokens, nt = min(kFrontTokens, T - t0);
+        route_rows_body<XT, kFrontTokens, Q8 ? 32 : 8, Q8 ? 2 : 1, 2>(r, blockIdx.x, lds);
+        __syncthreads();
+        float* const prob = reinterpret_cast<float*>(lds);  // the arrays of router_fixed_bytes
+        float* const lsev = prob + kFrontTokens * ES;
+        float* const gates = lsev + kFrontTokens;
+        int* const lexp = reinterpret_cast<int*>(gates + kFrontTokens * k);
+        int G = 1;
+        while (G < E && G < 64) G <<= 1;
+        softmax_topk<1, 1, kFrontTokens>(prob, lsev, gates, lexp, G, t0, nt, ES, r.valid, E, k);
+        __syncthreads();
+        const int tid = threadIdx.x;
+        for (int i = tid; i < nt * E; i += kSmallThreads) {
+            const int t = i / E;
+            r.P[(size_t)t0 * E + i] = prob[t * ES + (i - t * E)];
+        }
+        if (tid < nt) r.lse[t0 + tid] = lsev[tid];
+        for (int i = tid; i < nt * k; i += kSmallThreads) {
+            r.expert_of[(size_t)t0 * k + i] = lexp[i];
+            r.gate_of[(size_t)t0 * k + i] = gates[i];
+        }
         return;
     }
     // a product workgroup is two teams of four waves, each with a block of 32 features of its own: the reduction is
     // split four ways as in the launch without the routing, and a compute unit has twice the weight bytes in flight
     const int widest = g.a_shared ? max(g.N, g.N_shared) : g.N;
-    const int nfb = widest / 32, npair = (nfb + 1) / 2;
-    const int idx = blockIdx.x - 1;
-    const int fb = 2 * (idx % npair) + (int)threadIdx.x / (kSmallThreads / 2), side = idx / npair;
+    const int nfb = widest / 32, npair = (nfb + kFrontTeams - 1) / kFrontTeams;
+    const int idx = blockIdx.x - routers;
+    const int side = idx / npair;
+    const int fb0 = kFrontTeams * (idx % npair);
+    int fb = fb0 + (int)threadIdx.x / (kSmallThreads / kFrontTeams);
     DecodeSide sd;
     sd.row_index = nullptr;
     sd.row0 = 0;
@@ -1176,52 +1309,144 @@ __global__ __launch_bounds__(kSmallThreads, 2) void decode_front_kernel(SmallRou
         sd.rows = min(32, g.T_shared - sd.row0);
         sd.out_row0 = 0;
     }
-    if (fb * 32 >= sd.N) return;
-    decode_gemm_body<true, I8, kSmallThreads / 128, kBatch, 2>(sd, fb, reinterpret_cast<float*>(smem));
+    if (fb0 * 32 >= sd.N) return;  // (the sides' widths differ)
+    float* const red = reinterpret_cast<float*>(lds);
+    if constexpr (NORM) {
+        // (a team without a block keeps the other company to the barriers: it takes the last block again and stores nothing)
+        if (fb * 32 >= sd.N) {
+            fb = sd.N / 32 - 1;
+            sd.rows = 0;
+        }
+        // The rows' factors are taken here as the routing takes them (route_rows_body), by every product workgroup for
+        // itself: the rows are requested in front of the weights, squared and summed in index order while those stream in.
+        const int d = r.d, sp = d + 4, xpr = d / Vec16<XT>::N, nx = T * xpr, tid = threadIdx.x;
+        float* const nw = red + front_room_floats(T, d, true);
+        float* const inv = nw + d;
+        const uint4* const xsrc = reinterpret_cast<const uint4*>(r.x);
+        constexpr int NT = kSmallThreads;
+        auto fetch = [&](int i) -> uint4 { return xsrc[(uint32_t)min(i, nx - 1)]; };
+        const float w0 = r.norm_w[min(tid, d - 1)], w1 = r.norm_w[min(tid + NT, d - 1)];
+        const uint4 v0 = fetch(tid), v1 = fetch(tid + NT), v2 = fetch(tid + 2 * NT), v3 = fetch(tid + 3 * NT),
+                    v4 = fetch(tid + 4 * NT), v5 = fetch(tid + 5 * NT);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t recip = (uint32_t)(0x100000000ull / (uint32_t)xpr) + 1u;
+        auto put = [&](int i, const uint4& v) {
+            if (i >= nx) return;
+            const int row = xpr == 1 ? i : (int)__umulhi((uint32_t)i, recip), c = (i - row * xpr) * Vec16<XT>::N;
+            float f[Vec16<XT>::N];
+            Vec16<XT>::widen(v, f);
+            float4* const s4 = reinterpret_cast<float4*>(red + row * sp + c);
+#pragma unroll
+            for (int q = 0; q < Vec16<XT>::N / 4; ++q)
+                s4[q] = make_float4(__fmul_rn(f[4 * q], f[4 * q]), __fmul_rn(f[4 * q + 1], f[4 * q + 1]),
+                                    __fmul_rn(f[4 * q + 2], f[4 * q + 2]), __fmul_rn(f[4 * q + 3], f[4 * q + 3]));
+        };
+        auto hook = [&]() {
+            put(tid, v0); put(tid + NT, v1); put(tid + 2 * NT, v2);
+            put(tid + 3 * NT, v3); put(tid + 4 * NT, v4); put(tid + 5 * NT, v5);
+            for (int i = tid + 6 * NT; i < nx; i += NT) put(i, fetch(i));
+            if (tid < d) nw[tid] = w0;
+            if (tid + NT < d) nw[tid + NT] = w1;
+            for (int c = tid + 2 * NT; c < d; c += NT) nw[c] = r.norm_w[c];
+            __syncthreads();
+            if (tid < T) inv[tid] = inverse_rms_of(ordered_sum(red + tid * sp, d), d, r.norm_eps);
+            else if (tid < 32) inv[tid] = 0.0f;
+            __syncthreads();
+        };
+        sd.norm_w = nw;
+        sd.row_factor = inv;
+        decode_gemm_body<true, I8, kSmallThreads / 64 / kFrontTeams, sizeof(XT) == 4 ? 8 : kBatch, kFrontTeams, false,
+                         RowForm<XT, NORM>>(sd, fb, red, nullptr, hook);
+    } else {
+        if (fb * 32 >= sd.N) return;
+        // (f32 rows take two registers a fragment's worth: a shorter batch keeps everything in registers)
+        decode_gemm_body<true, I8, kSmallThreads / 64 / kFrontTeams, sizeof(XT) == 4 ? 8 : kBatch, kFrontTeams, false,
+                         RowForm<XT, NORM>>(sd, fb, red);
+    }
 }
 
-bool decode_front_ok(const void* x, const float* wr, int T, int d, int E, int k) {
-    // the routing workgroup of the fused launch has a smaller staging area; rows that do not fit it are read from
-    // memory piecemeal, which takes longer than the products beside it: not worth it
-    const size_t ds = (size_t)d + 8;
-    const bool staged = d % 8 == 0 && (size_t)E * ds * 4 + (size_t)T * ds * 2 <= (size_t)kFrontStageBytes &&
-                        reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(wr) % 16 == 0;
-    // most experts must be about to be touched: an unrouted expert's gate/up weights are fetched for nothing
-    return staged && T <= 32 && (long long)T * k >= 2LL * E;
+// LDS of the launch; *EG: experts whose router rows a routing workgroup holds together.  0: the call does not fit.
+static size_t front_lds_bytes(int T, int E, int k, int d, bool q8, bool norm, int* EG) {
+    const size_t products = ((size_t)front_room_floats(T, d, norm) + (norm ? d + 32 : 0)) * 4;
+    int eg = E;
+    auto route = [&] { return route_rows_lds_bytes(E, k, d, kFrontTokens, q8 ? 32 : 8, eg, norm); };
+    while (eg > 8 && route() > (size_t)kMaxRouterLds) eg = (eg - 1) & ~1;
+    if (route() > (size_t)kMaxRouterLds || products > (size_t)kMaxRouterLds) return 0;
+    *EG = eg;
+    return products > route() ? products : route();
 }
 
-hipError_t launch_decode_front(const SmallRouteArgs& r, const DecodeGemmArgs& g, WeightKind wk, hipStream_t s) {
-    if (!small_route_ok(r.T, r.E, r.k) || r.norm_w || r.rows16 || !g.swiglu) return hipErrorInvalidValue;
+bool decode_front_ok(const RouterArgs& a, bool bf16) {
+    const int unit = a.wq ? 32 : 8;
+    const size_t xsize = bf16 ? 2 : 4;
+    int eg = 0;
+    return a.T >= 1 && a.T <= kSmallRouteMaxTokens && a.E <= 64 && a.k <= kMaxTopK && a.T * a.E <= kSmallRouteMaxPairs &&
+           a.d % unit == 0 && a.d % 32 == 0 && (size_t)a.d * xsize % 16 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(a.wq ? static_cast<const void*>(a.wq) : a.wr) % 16 == 0 &&
+           front_lds_bytes(a.T, a.E, a.k, a.d, a.wq != nullptr, a.norm_w != nullptr, &eg) != 0;
+}
+
+hipError_t launch_decode_front(const RouterArgs& a, const DecodeGemmArgs& g, bool bf16, WeightKind wk, bool products, hipStream_t s) {
+    if (!decode_front_ok(a, bf16) || !g.swiglu || wk == WeightKind::F32 || (a.wq && (!a.wscale || wk != WeightKind::I8)))
+        return hipErrorInvalidValue;
     const int shared_tiles = g.a_shared ? (g.T_shared + 31) / 32 : 0;
     const int widest = g.a_shared ? (g.N > g.N_shared ? g.N : g.N_shared) : g.N;
-    const int grid = 1 + (r.E + shared_tiles) * ((widest / 32 + 1) / 2);
-    if (wk == WeightKind::BF16)
-        RB_LAUNCH(decode_front_kernel<false>, dim3(grid), dim3(kSmallThreads), 0, s, r, g, r.E, r.T);
-    else if (wk == WeightKind::I8)
-        RB_LAUNCH(decode_front_kernel<true>, dim3(grid), dim3(kSmallThreads), 0, s, r, g, r.E, r.T);
-    else
-        return hipErrorInvalidValue;
+    const int routers = (a.T + kFrontTokens - 1) / kFrontTokens;
+    const int grid = routers + (products ? (a.E + shared_tiles) * ((widest / 32 + kFrontTeams - 1) / kFrontTeams) : 0);
+    int EG = 0;
+    const size_t lds = front_lds_bytes(a.T, a.E, a.k, a.d, a.wq != nullptr, a.norm_w != nullptr, &EG);
+    RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, EG, a.P, a.lse, a.expert_of, a.gate_of,
+                    nullptr, nullptr, nullptr, nullptr, a.norm_w, a.norm_eps, nullptr};
+    auto go = [&](auto kernel) -> hipError_t {
+        static std::atomic<unsigned long long> attr_set{0};  // one per kernel: the lambda's body is instantiated for each
+        const hipError_t e = once_per_device(attr_set, [&] {
+            return hipFuncSetAttribute(reinterpret_cast<const void*>(+kernel.value), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       kMaxRouterLds);
+        });
+        if (e != hipSuccess) return e;
+        RB_LAUNCH(kernel.value, dim3(grid), dim3(kSmallThreads), lds, s, r, g, routers);
+        return hipGetLastError();
+    };
+#define RB_FRONT(XT, I8, Q8, NORM) \
+    go(std::integral_constant<void (*)(RouteRowsArgs, DecodeGemmArgs, int), &decode_front_kernel<XT, I8, Q8, NORM>>{})
+#define RB_FRONT_W(XT, NORM)                                                   \
+    (wk == WeightKind::BF16 ? RB_FRONT(XT, false, false, NORM)                 \
+                            : a.wq ? RB_FRONT(XT, true, true, NORM) : RB_FRONT(XT, true, false, NORM))
+    if (bf16) return a.norm_w ? RB_FRONT_W(bf16_t, true) : RB_FRONT_W(bf16_t, false);
+    return a.norm_w ? RB_FRONT_W(float, true) : RB_FRONT_W(float, false);
+#undef RB_FRONT_W
+#undef RB_FRONT
+}
+
+hipError_t launch_decode_layout(const DecodeLayoutArgs& a, hipStream_t s) {
+    if (!small_route_ok(a.T, a.E, a.k)) return hipErrorInvalidValue;
+    RB_LAUNCH(decode_layout_kernel, dim3(1), dim3(kSmallThreads), 0, s, a);
     return hipGetLastError();
 }
 
+constexpr int kByExpertSlots = 8;  // slots a token: what a thread of the combine fetches beforehand, and 64 * kLateRounds / 32
+
 bool decode_down_by_expert_ok(const DecodeGemmArgs& g, int E, int T, int k) {
-    return !g.swiglu && g.cmb_out != nullptr && g.cmb_counter != nullptr && g.cmb_inv_pos != nullptr &&
-           g.cmb_gate_of != nullptr && g.a_expert_rows == T && T >= 1 && T <= 32 && k <= kCombineEarlySlots &&
-           g.cmb_T == T && g.cmb_k == k && (!g.a_shared || g.N_shared == g.N) && g.N / 32 <= kDecodeCombineMaxBlocks &&
-           g.N % 32 == 0 && E >= 1;
+    return !g.swiglu && g.cmb_out != nullptr && g.cmb_counter != nullptr && g.cmb_gate_of != nullptr && g.a_expert_rows == T &&
+           T >= 1 && T <= 32 && k <= kByExpertSlots && g.cmb_T == T && g.cmb_k == k && (!g.a_shared || g.N_shared == g.N) &&
+           g.N / 32 <= kDecodeCombineMaxBlocks && g.N % 32 == 0 && E >= 1;
 }
 
-hipError_t launch_decode_down_by_expert(const DecodeGemmArgs& g, const unsigned int* expert_tokens, const int* offsets,
-                                        int E, WeightKind wk, hipStream_t s) {
-    if (!expert_tokens || !offsets || !decode_down_by_expert_ok(g, E, g.cmb_T, g.cmb_k)) return hipErrorInvalidValue;
+hipError_t launch_decode_down_by_expert(const DecodeGemmArgs& g, const DecodeLayoutArgs& t, WeightKind wk, hipStream_t s) {
+    static_assert(kByExpertSlots * kSmallRouteMaxTokens <= 64 * kLateRounds, "every slot is looked at");
+    if (!decode_down_by_expert_ok(g, t.E, t.T, t.k) || !small_route_ok(t.T, t.E, t.k)) return hipErrorInvalidValue;
     const int shared_tiles = g.a_shared ? (g.T_shared + 31) / 32 : 0;
-    const dim3 grid(g.N / 32, E + shared_tiles);
-    if (wk == WeightKind::BF16)
-        RB_LAUNCH(decode_down_by_expert_kernel<false>, grid, dim3(512), 0, s, g, expert_tokens, offsets, E);
-    else if (wk == WeightKind::I8)
-        RB_LAUNCH(decode_down_by_expert_kernel<true>, grid, dim3(512), 0, s, g, expert_tokens, offsets, E);
-    else
+    const dim3 grid(g.N / 32, t.E + shared_tiles + 1);
+    const bool few = t.k <= 4;
+    if (wk == WeightKind::BF16) {
+        if (few) RB_LAUNCH((decode_down_by_expert_kernel<false, 4>), grid, dim3(512), 0, s, g, t);
+        else RB_LAUNCH((decode_down_by_expert_kernel<false, kByExpertSlots>), grid, dim3(512), 0, s, g, t);
+    } else if (wk == WeightKind::I8) {
+        if (few) RB_LAUNCH((decode_down_by_expert_kernel<true, 4>), grid, dim3(512), 0, s, g, t);
+        else RB_LAUNCH((decode_down_by_expert_kernel<true, kByExpertSlots>), grid, dim3(512), 0, s, g, t);
+    } else {
         return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 

@@ -180,7 +180,6 @@ struct Work {
     void* hall = nullptr;  // hidden rows of every expert over every row, [E][T, F] (decode_front launches), or null
     void* x16 = nullptr;   // bf16 copy of f32 rows [T, d] (layers with cast_rows), or null
     int* cmb_counter = nullptr;  // arrival counters of a combine folded into the decode-shaped down launch (all zero between launches)
-    unsigned int* expert_tokens = nullptr;  // [E] the tokens of every expert, one bit a token (decode_front launches), or null
 };
 
 // Host memory of a call that is still under way: a pinned block, or plain memory when the pool is exhausted.
@@ -243,6 +242,7 @@ struct rbmoe_layer {
     bool decode_fold = true;   // decode-shaped calls: the combine inside the down launch
     bool decode_down_by_expert = true;  // behind a decode_front launch: the down launch's workgroup rows are experts, not tile-table entries
     bool last_front = false;   // the last forward's hidden rows are per expert over all rows (Work::hall)
+    bool last_by_slot = false; // ... and its expert rows lie in slot order
     int group_m = 0;
     const char* kernel_name = "none";
     int last_T = -1;
@@ -266,7 +266,6 @@ struct rbmoe_layer {
     Buf xg, h, y, hs, ys;
     Buf x16;               // [max_T, d] bf16 copy of f32 rows (cast_rows)
     Buf hall;              // [E][min(max_T, 32), F] hidden rows of decode_front launches
-    Buf etok;              // [E] token bits of every expert (decode_front launches)
     Buf cmbcnt;            // [kDecodeCombineMaxBlocks] arrival counters of the folded decode combine
     // feed-forward norm in front of the layer (allocated by rbmoe_set_feed_forward_norm)
     Buf xn, norm_w;  // [max_T, d] activation dtype, [d] f32
@@ -406,11 +405,8 @@ Plan make_plan(rbmoe_layer* L) {
     p.add(&L->perm_token, S * 4);
     p.add(&L->inv_pos, S * 4);
     if (L->cast_rows) p.add(&L->x16, T * d * 2);
-    // decode_front launches need most experts touched (tokens * k >= 2 E, at most 32 tokens): none when E > 16 k
-    if (L->use_stream && E <= 16 * k) {
+    if (L->use_stream && E <= 64)  // decode_front launches
         p.add(&L->hall, E * std::min<size_t>(T, kSmallRouteMaxTokens) * F * 2);
-        p.add(&L->etok, E * 4);
-    }
     p.add(&L->cmbcnt, kDecodeCombineCounterBytes);
     p.add(&L->xg, S * d * as);
     p.add(&L->h, S * F * as);
@@ -925,15 +921,25 @@ Work work_of_layer(const rbmoe_layer* L) {
     w.perm_slot = (int*)L->perm_slot.p; w.perm_token = (int*)L->perm_token.p; w.inv_pos = (int*)L->inv_pos.p;
     w.h = L->h.p; w.y = L->y.p; w.hs = L->hs.p; w.ys = L->ys.p;
     w.hall = L->hall.p;
-    w.expert_tokens = (unsigned int*)L->etok.p;
     w.x16 = L->x16.p;
     w.cmb_counter = (int*)L->cmbcnt.p;
     return w;
 }
 
+// Whether a decode-shaped call of T tokens should take every expert's products without waiting for the routing: when most
+// experts are about to be touched, or when the weights fetched for nothing cost less than the launch and the chain in
+// front of the products that this saves (about 8 us: 24 MB at the 3 to 4 TB/s these launches reach).
+bool decode_front_pays(const rbmoe_layer* L, int T) {
+    const rbmoe_config& c = L->cfg;
+    const double E = c.num_experts, k = c.experts_per_token;
+    if (T * k >= 2 * E) return true;
+    const double untouched = E * std::pow(1.0 - k / E, T);
+    return untouched * 3.0 * L->Fw * c.d_model * dtype_size(c.weight_dtype) <= 24e6;
+}
+
 // The buffers of a decode-shaped forward of T tokens carved out of `base` (pieces of 256 bytes); returns the
 // bytes used.  With base == nullptr only the size is computed.
-size_t carve_decode_work(const rbmoe_layer* L, int T, unsigned char* base, Work* w) {
+size_t carve_decode_work(const rbmoe_layer* L, int T, bool front, unsigned char* base, Work* w) {
     const rbmoe_config& c = L->cfg;
     const size_t E = c.num_experts, d = c.d_model, F = L->Fw, k = c.experts_per_token, Fs = L->Fsw;
     const size_t S = (size_t)T * k, as = L->cast_rows ? 2 : dtype_size(c.act_dtype);
@@ -955,10 +961,7 @@ size_t carve_decode_work(const rbmoe_layer* L, int T, unsigned char* base, Work*
     v.ntiles = (int*)take(8); v.losses = (float*)take(8);
     v.perm_slot = (int*)take(S * 4); v.perm_token = (int*)take(S * 4); v.inv_pos = (int*)take(S * 4);
     v.h = take(S * F * as); v.y = take(S * d * as);
-    if ((size_t)T * k >= 2 * E) {  // (the condition of decode_front_ok)
-        v.hall = take(E * (size_t)T * F * 2);
-        v.expert_tokens = (unsigned int*)take(E * 4);
-    }
+    if (front) v.hall = take(E * (size_t)T * F * 2);
     if (c.shared_expert) {
         v.hs = take((size_t)T * Fs * as);
         v.ys = take((size_t)T * d * as);
@@ -1036,37 +1039,8 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // norm and write the bf16 copy of f32 rows
     const bool stages_rows = small_route_stages_rows(x, (const float*)L->router.p, T, d, E, abf) &&
                              (!norm_src || small_route_stages_rows(norm_src, (const float*)L->router.p, T, d, E, abf));
-    // (a quantized router has one kernel for its logits, on the large-batch sequence)
-    const bool decode_ok = mfma && L->decode_path && !L->training && !L->router_q8 && small_route_ok(T, E, k) &&
-                           decode_shape_ok(F, d) &&
-                           decode_shape_ok(d, F) &&
-                           (!c.shared_expert || (decode_shape_ok(Fs, d) && decode_shape_ok(d, Fs))) &&
-                           (!cast || stages_rows);
-    const bool norm_in_route = norm_src && decode_ok && stages_rows;
-    Work wk_ = work_of_layer(L);
-    if (static_scratch) {
-        if (!decode_ok) {
-            char buf[200];
-            std::snprintf(buf, sizeof buf,
-                          "rbmoe_forward_static takes decode-shaped calls only: 1 to %d tokens of a layer with bf16 or "
-                          "int8 weights on the matrix-core path, not in training mode (got %d tokens)",
-                          kSmallRouteMaxTokens, T);
-            return fail(ctx, RBMOE_UNSUPPORTED, buf);
-        }
-        const size_t need = carve_decode_work(L, T, nullptr, nullptr);
-        if (need > (size_t)RBMOE_STATIC_SCRATCH_BYTES) {
-            char buf[200];
-            std::snprintf(buf, sizeof buf, "this call needs %zu bytes of scratch, the static buffer holds %zu", need,
-                          (size_t)RBMOE_STATIC_SCRATCH_BYTES);
-            return fail(ctx, RBMOE_UNSUPPORTED, buf);
-        }
-        // Nothing of it is cleared: every word a kernel of this call reads was written by an earlier kernel of
-        // the same call (the tile-table entries past *ntiles, which the product kernels fetch and drop, may be
-        // a previous call's).
-        carve_decode_work(L, T, static_cast<unsigned char*>(static_scratch), &wk_);
-    }
-    // the rows the expert products read
-    const void* const xe = cast ? wk_.x16 : x;
+    const bool small = mfma && L->decode_path && !L->training && small_route_ok(T, E, k) && decode_shape_ok(F, d) &&
+                       decode_shape_ok(d, F) && (!c.shared_expert || (decode_shape_ok(Fs, d) && decode_shape_ok(d, Fs)));
     RouterArgs ra{norm_src ? norm_src : x, (const float*)L->router.p, router_bias, valid, T, d, E, k,
                   (float*)L->P.p, (float*)L->lse.p, (int*)L->expert_of.p, (float*)L->gate_of.p,
                   (int*)L->rank_in_block.p, (int*)L->blockcnt.p, (float*)L->partial.p};
@@ -1081,6 +1055,38 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         ra.norm_eps = L->norm_eps;
         ra.xn_out = L->xn.p;
     }
+    // the routing beside the gate/up products, in one launch
+    bool front = small && L->decode_front && L->hall.p != nullptr && decode_front_ok(ra, abf) &&
+                 (!L->router_q8 || wk == WeightKind::I8) && decode_front_pays(L, T);
+    if (static_scratch && front && carve_decode_work(L, T, true, nullptr, nullptr) > (size_t)RBMOE_STATIC_SCRATCH_BYTES)
+        front = false;
+    // (without it a quantized router takes the large-batch sequence)
+    const bool decode_ok = small && (front || (!L->router_q8 && (!cast || stages_rows)));
+    const bool norm_in_route = norm_src && decode_ok && (front || stages_rows);
+    Work wk_ = work_of_layer(L);
+    if (static_scratch) {
+        if (!decode_ok) {
+            char buf[200];
+            std::snprintf(buf, sizeof buf,
+                          "rbmoe_forward_static takes decode-shaped calls only: 1 to %d tokens of a layer with bf16 or "
+                          "int8 weights on the matrix-core path, not in training mode (got %d tokens)",
+                          kSmallRouteMaxTokens, T);
+            return fail(ctx, RBMOE_UNSUPPORTED, buf);
+        }
+        const size_t need = carve_decode_work(L, T, front, nullptr, nullptr);
+        if (need > (size_t)RBMOE_STATIC_SCRATCH_BYTES) {
+            char buf[200];
+            std::snprintf(buf, sizeof buf, "this call needs %zu bytes of scratch, the static buffer holds %zu", need,
+                          (size_t)RBMOE_STATIC_SCRATCH_BYTES);
+            return fail(ctx, RBMOE_UNSUPPORTED, buf);
+        }
+        // Nothing of it is cleared: every word a kernel of this call reads was written by an earlier kernel of
+        // the same call (the tile-table entries past *ntiles, which the product kernels fetch and drop, may be
+        // a previous call's).
+        carve_decode_work(L, T, front, static_cast<unsigned char*>(static_scratch), &wk_);
+    }
+    // the rows the expert products read
+    const void* const xe = cast ? wk_.x16 : x;
     const RouterPlan rplan = plan_router(ra, abf);
     if (!rplan.takes_norm) {  // the norm runs by itself
         ra.x = x;
@@ -1101,9 +1107,6 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
             sr.x = norm_src; sr.norm_w = (const float*)L->norm_w.p; sr.norm_eps = L->norm_eps; sr.xn_out = L->xn.p;
         }
         if (cast) sr.rows16 = wk_.x16;
-        // the routing beside the gate/up products, in one launch: bf16 rows as they are (no norm to apply first)
-        const bool front = L->decode_front && !norm_src && !cast && wk_.hall != nullptr &&
-                           decode_front_ok(x, (const float*)L->router.p, T, d, E, k);
         sr.T = T; sr.d = d; sr.E = E; sr.k = k;
         sr.w_aux = c.aux_loss_weight; sr.w_z = c.router_z_loss_weight;
         sr.tile_m = kDecodeTileM;
@@ -1114,6 +1117,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         sr.ntiles = wk_.ntiles; sr.losses = wk_.losses;
         sr.perm_slot = wk_.perm_slot; sr.perm_token = wk_.perm_token; sr.inv_pos = wk_.inv_pos;
         for (auto& r : L->replay) r = nullptr;
+        const bool named_front = front && !cast && T * k >= 2 * E;
         if (!front) {
             HIP_TRY(ctx, launch_route_small(sr, abf, s));
             L->replay[RBMOE_STAGE_ROUTER] = [=](hipStream_t st) { return launch_route_small(sr, abf, st); };
@@ -1137,17 +1141,24 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
             d1.scales_shared = wk == WeightKind::I8 ? (const float*)L->ssgu.p : nullptr;
             d1.N_shared = Fs; d1.K_shared = d; d1.T_shared = T; d1.out_shared = wk_.hs;
         }
+        DecodeLayoutArgs lay{wk_.P, wk_.lse, wk_.expert_of, valid, T, E, k, c.aux_loss_weight, c.router_z_loss_weight,
+                             wk_.counts, wk_.offsets, wk_.tile_expert, wk_.tile_row0, wk_.tile_rows, wk_.ntiles, wk_.losses,
+                             wk_.perm_slot, wk_.perm_token, wk_.inv_pos};
         if (front) {
+            RouterArgs fr = ra;  // (the products read the same rows: raw ones in front of a norm, f32 ones as they are)
+            fr.P = wk_.P; fr.lse = wk_.lse; fr.expert_of = wk_.expert_of; fr.gate_of = wk_.gate_of;
+            d1.a = fr.x;
+            if (c.shared_expert) d1.a_shared = fr.x;
             d1.row_index = nullptr;
             d1.out = wk_.hall;
-            sr.expert_tokens = wk_.expert_tokens;
-            HIP_TRY(ctx, launch_decode_front(sr, d1, wk, s));
-            L->replay[RBMOE_STAGE_GATE_UP] = [=](hipStream_t st) { return launch_decode_front(sr, d1, wk, st); };
+            HIP_TRY(ctx, launch_decode_front(fr, d1, abf, wk, true, s));
+            L->replay[RBMOE_STAGE_GATE_UP] = [=](hipStream_t st) { return launch_decode_front(fr, d1, abf, wk, true, st); };
+            if (!named_front)  // (not reported as routing beside the products: the routing alone is its stage then)
+                L->replay[RBMOE_STAGE_ROUTER] = [=](hipStream_t st) { return launch_decode_front(fr, d1, abf, wk, false, st); };
         } else {
             HIP_TRY(ctx, launch_decode_gemm(d1, wk, s));
             L->replay[RBMOE_STAGE_GATE_UP] = [=](hipStream_t st) { return launch_decode_gemm(d1, wk, st); };
         }
-        if (L->record_routed) HIP_TRY(ctx, hipEventRecord(L->record_routed, s));
         HIP_TRY(ctx, mark(4));
 
         DecodeGemmArgs d2 = d1;
@@ -1174,17 +1185,18 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
             d2.cmb_residual = residual; d2.cmb_out = out;
             d2.cmb_T = T; d2.cmb_k = k; d2.cmb_f32 = abf ? 0 : 1;
         }
-        // behind the routing-beside-the-products launch every expert's rows are known by its token bits: the down
-        // launch then has one row of workgroups per expert, whose weights go out before anything of the routing is read
-        if (front && fold && L->decode_down_by_expert && wk_.expert_tokens != nullptr && decode_down_by_expert_ok(d2, E, T, k)) {
-            const unsigned int* const etok = wk_.expert_tokens;
-            const int* const offs = wk_.offsets;
-            HIP_TRY(ctx, launch_decode_down_by_expert(d2, etok, offs, E, wk, s));
-            L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return launch_decode_down_by_expert(d2, etok, offs, E, wk, st); };
+        // behind the routing-beside-the-products launch the down launch has one row of workgroups per expert, whose weights
+        // go out before anything of the routing is read, and makes the tables beside them
+        const bool by_expert = front && fold && L->decode_down_by_expert && decode_down_by_expert_ok(d2, E, T, k);
+        if (by_expert) {
+            HIP_TRY(ctx, launch_decode_down_by_expert(d2, lay, wk, s));
+            L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return launch_decode_down_by_expert(d2, lay, wk, st); };
         } else {
+            if (front) HIP_TRY(ctx, launch_decode_layout(lay, s));
             HIP_TRY(ctx, launch_decode_gemm(d2, wk, s));
             L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return launch_decode_gemm(d2, wk, st); };
         }
+        if (L->record_routed) HIP_TRY(ctx, hipEventRecord(L->record_routed, s));
         HIP_TRY(ctx, mark(5));
         HIP_TRY(ctx, mark(6));
         if (!fold) {
@@ -1197,8 +1209,9 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         L->last_T = T;
         L->last = wk_;
         L->last_front = front;
-        L->kernel_name = front ? (wk == WeightKind::I8 ? "mfma_bf16_decode_front_int8w" : "mfma_bf16_decode_front")
-                               : L->kernel_name;
+        L->last_by_slot = by_expert;
+        if (named_front)
+            L->kernel_name = wk == WeightKind::I8 ? "mfma_bf16_decode_front_int8w" : "mfma_bf16_decode_front";
         return RBMOE_OK;
     }
 
@@ -1373,6 +1386,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     L->last_T = T;
     L->last = wk_;
     L->last_front = false;
+    L->last_by_slot = false;
     return RBMOE_OK;
 }
 
@@ -2349,6 +2363,16 @@ int rbmoe_get_expert_rows(rbmoe_layer* L, float* hidden, float* expert_out) {
         rc = fetch(hidden, L->last.h, (size_t)R * F);
     }
     if (rc != RBMOE_OK) return rc;
+    if (L->last_by_slot && expert_out && R > 0) {
+        const int S = L->last_T * L->cfg.experts_per_token;
+        std::vector<float> all((size_t)S * d);
+        std::vector<int> slots(R);
+        rc = fetch(all.data(), L->last.y, all.size());
+        if (rc != RBMOE_OK) return rc;
+        HIP_TRY(ctx, hipMemcpy(slots.data(), L->last.perm_slot, (size_t)R * 4, hipMemcpyDeviceToHost));
+        for (int pos = 0; pos < R; ++pos) std::memcpy(expert_out + (size_t)pos * d, all.data() + (size_t)slots[pos] * d, (size_t)d * 4);
+        return RBMOE_OK;
+    }
     return fetch(expert_out, L->last.y, (size_t)R * d);
 }
 

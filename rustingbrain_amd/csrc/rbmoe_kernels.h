@@ -287,9 +287,6 @@ struct SmallRouteArgs {
     // f32 rows only: a bf16 copy [T, d] of the rows the routing is decided on (after the norm, if any), for the
     // matrix-core products; only for calls whose rows are staged in LDS (small_route_stages_rows)
     void* rows16 = nullptr;
-    // launch_decode_front only, or null: [E] the tokens every expert takes, one bit a token (at most 32 tokens); the
-    // expert's rows are these tokens in ascending order
-    unsigned int* expert_tokens = nullptr;
 };
 bool small_route_stages_rows(const void* x, const float* wr, int T, int d, int E, bool bf16);
 bool small_route_ok(int T, int E, int k);
@@ -338,16 +335,31 @@ constexpr int kDecodeCombineCounterStride = 64;
 constexpr size_t kDecodeCombineCounterBytes = (size_t)kDecodeCombineMaxBlocks * kDecodeCombineCounterStride * 4;
 bool decode_shape_ok(int N, int K);
 hipError_t launch_decode_gemm(const DecodeGemmArgs& g, WeightKind wk, hipStream_t s);
-// Routing and gate/up products in one launch (bf16 rows, no norm): every expert's gate/up product over all T rows,
-// hidden rows to g.out as [E][T, N]; the shared expert as in launch_decode_gemm.  g.a / g.a_shared: the T rows.
-bool decode_front_ok(const void* x, const float* wr, int T, int d, int E, int k);
-hipError_t launch_decode_front(const SmallRouteArgs& r, const DecodeGemmArgs& g, WeightKind wk, hipStream_t s);
+// Routing and gate/up products in one launch: every expert's gate/up product over all T rows, hidden rows to g.out as
+// [E][T, N]; the shared expert as in launch_decode_gemm.  g.a / g.a_shared: the call's rows as they are (a.x), f32 or
+// bf16, raw when the routing applies a norm - the products then take the normed rows on the way.  P, lse, expert_of and
+// gate_of are written, nothing else of the routing (DecodeLayoutArgs).  products = false: the routing alone.
+bool decode_front_ok(const RouterArgs& a, bool bf16);
+hipError_t launch_decode_front(const RouterArgs& a, const DecodeGemmArgs& g, bool bf16, WeightKind wk, bool products, hipStream_t s);
+// The tables and losses of a call routed by launch_decode_front.
+struct DecodeLayoutArgs {
+    const float* P;
+    const float* lse;
+    const int* expert_of;
+    const uint8_t* valid;
+    int T, E, k;
+    float w_aux, w_z;
+    int *counts, *offsets, *tile_expert, *tile_row0, *tile_rows, *ntiles;
+    float* losses;
+    int *perm_slot, *perm_token, *inv_pos;
+};
+hipError_t launch_decode_layout(const DecodeLayoutArgs& a, hipStream_t s);
 // The down product behind launch_decode_front with the combine folded in (g as for launch_decode_gemm: cmb_* set,
-// a_expert_rows = tokens of the call), one row of workgroups per EXPERT instead of per entry of the tile table: a
-// workgroup knows its weights from its place in the grid and requests them at once, and learns its rows from
-// expert_tokens / offsets / g.ntiles behind them.  An expert without rows costs its weights' bytes.
+// a_expert_rows = tokens of the call; expert rows to g.out in SLOT order), one row of workgroups per EXPERT instead of per
+// entry of the tile table: a workgroup knows its weights from its place in the grid and requests them at once, and learns
+// its rows from t.expert_of behind them.  An expert without rows costs its weights' bytes.  The tables and losses of `t` are
+// made beside the products.
 bool decode_down_by_expert_ok(const DecodeGemmArgs& g, int E, int T, int k);
-hipError_t launch_decode_down_by_expert(const DecodeGemmArgs& g, const unsigned int* expert_tokens, const int* offsets,
-                                        int E, WeightKind wk, hipStream_t s);
+hipError_t launch_decode_down_by_expert(const DecodeGemmArgs& g, const DecodeLayoutArgs& t, WeightKind wk, hipStream_t s);
 
 }  // namespace rbmoe

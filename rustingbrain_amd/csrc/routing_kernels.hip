@@ -17,23 +17,10 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "rbmoe_kernels.h"
+#include "routing_device.h"
 
 namespace rbmoe {
 
-
-// Dynamic LDS layout of router_kernel (floats / ints, in this order):
-//   prob   [TB][ES]   logits, then exp, then probabilities   (ES = E | 1)
-//   lsev   [TB]       log-sum-exp per token
-//   gates  [TB][k]    selected probabilities, then gates
-//   lexp   [TB][k]    selected expert per local slot (-1 = unrouted)
-//   wcount [waves][E] per-wave match counts of one ranking round
-//   running[E]        slots already ranked per expert
-__host__ __device__ static size_t router_fixed_bytes(int E, int k, int tokens = kRouterTokens) {
-    const int ES = E | 1;
-    size_t n = (size_t)tokens * ES + tokens + 2 * (size_t)tokens * k + (size_t)kRouterWaves * E + E;
-    return (n * 4 + 15) & ~(size_t)15;
-}
 
 size_t router_lds_bytes(int E, int k) {
     return router_fixed_bytes(E, k);
@@ -230,178 +217,6 @@ __global__ __launch_bounds__(NE * 64, (!AHEAD && sizeof(XT) == 2) ? 6 : 2) void 
         if (bias) v = __fadd_rn(v, bias[e]);
         logits[(size_t)(t0 + lane) * E + e] = v;
     }
-}
-
-// softmax, log-sum-exp and the k argmax rounds for the tokens of one wave of a router block (see router_tail).
-// Everything order-sensitive keeps the reference's order: the maximum ignores NaN (f32::max), exp(v - max) is
-// summed one expert after the other in index order, the k argmax rounds prefer the lower index on equal
-// probabilities, and the gates are summed in rank order.
-// The sum: lane l of a group ends with ((ex_0 + ex_1) + ... ) + ex_l after l steps of "take the lane below's sum,
-// add your own value" (a shift of the whole wave by one lane inside the add; a group's first lane keeps the sum
-// carried over from the experts of the slices before) - the reference's chain, one rounded add per expert, with
-// no trip through LDS; lanes past the last expert add zeros.  An argmax round is two reductions of 32 bits: the
-// greatest probability bits (probabilities are never negative, so the bits order like the values), then the
-// lowest expert index among the lanes that hold them.
-// NQ = turns a wave needs for its tokens (64 / G tokens a turn); the NQ turns share no data and run interleaved.
-template <int MAXJ, int NQ, int TB>
-__device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __restrict__ lsev,
-                                             float* __restrict__ gates, int* __restrict__ lexp, int G, int t0, int nt,
-                                             int ES, const uint8_t* __restrict__ valid, int E, int k) {
-    constexpr int TW = TB / kRouterWaves;  // tokens of a wave
-    const int lane_ = threadIdx.x & 63, wave_ = threadIdx.x >> 6;
-    const int lig = lane_ & (G - 1);          // lane in group
-    const int gbase = lane_ & ~(G - 1);       // first lane of the group
-    const int tpw = 64 / G;                   // tokens a wave handles in one turn
-    const unsigned long long gmask = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << gbase;
-    const float neg_inf = __uint_as_float(0xff800000u);
-    int tok[NQ];
-    bool live[NQ], ok[NQ];
-    float* row[NQ];
-    float pv[NQ][MAXJ], mx[NQ], sum[NQ], total[NQ];
-    unsigned taken_bits[NQ];  // bit j: expert lig + G j is taken
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        tok[q] = wave_ * TW + q * tpw + lane_ / G;  // token of this group in turn q
-        live[q] = tok[q] < nt && tok[q] < (wave_ + 1) * TW && q * tpw < TW;
-        row[q] = prob + (live[q] ? tok[q] : 0) * ES;
-        mx[q] = neg_inf;
-#pragma unroll
-        for (int j = 0; j < MAXJ; ++j) {
-            const int e = lig + G * j;
-            pv[q][j] = (live[q] && e < E) ? row[q][e] : neg_inf;
-            const float vv = (pv[q][j] == pv[q][j]) ? pv[q][j] : neg_inf;  // a NaN never becomes the maximum
-            mx[q] = vv > mx[q] ? vv : mx[q];
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) mx[q] = group_fmax(mx[q], G);
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-#pragma unroll
-        for (int j = 0; j < MAXJ; ++j) {
-            const int e = lig + G * j;
-            // lanes without an expert carry +0 through the sums below
-            pv[q][j] = (live[q] && e < E) ? rb_expf(__fadd_rn(pv[q][j], -mx[q])) : 0.0f;
-        }
-    }
-    // the sums: one chain of adds per token in index order, slice after slice
-    {
-        float carry[NQ];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) carry[q] = 0.0f;
-#pragma unroll
-        for (int j = 0; j < MAXJ; ++j) {
-            if (G * j >= E) break;  // uniform
-            float acc[NQ], seed[NQ];
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-                seed[q] = __fadd_rn(carry[q], pv[q][j]);  // what a group's first lane holds: 0 + ex_0 = ex_0 in the first slice
-                acc[q] = lig == 0 ? seed[q] : pv[q][j];
-            }
-            for (int st = 1; st < G; ++st) {
-#pragma unroll
-                for (int q = 0; q < NQ; ++q) {
-                    const float below = __uint_as_float(lanes_from<0x138>(__float_as_uint(acc[q])));  // wave_shr:1
-                    const float next = __fadd_rn(below, pv[q][j]);
-                    acc[q] = lig == 0 ? seed[q] : next;
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) carry[q] = __shfl(acc[q], gbase + G - 1);
-        }
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) sum[q] = carry[q];
-    }
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        if (live[q] && lig == 0) lsev[tok[q]] = __fadd_rn(mx[q], rb_logf(sum[q]));
-#pragma unroll
-        for (int j = 0; j < MAXJ; ++j) {
-            const int e = lig + G * j;
-            if (live[q] && e < E) {
-                if (sum[q] > 0.0f) pv[q][j] = __fdiv_rn(pv[q][j], sum[q]);
-                row[q][e] = pv[q][j];
-            }
-        }
-        ok[q] = live[q] && ((valid == nullptr) || (valid[t0 + tok[q]] != 0));
-        taken_bits[q] = 0;
-        total[q] = 0.0f;
-    }
-    // ---- k rounds of argmax over the experts not yet taken ----
-    for (int r = 0; r < k; ++r) {
-        int first[NQ];
-        uint32_t lbits[NQ], le[NQ];  // this lane's best candidate: probability bits and expert index
-        bool has[NQ];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            // First expert not yet taken: the lowest set bit of a ballot over the group, taking
-            // the expert slices j in increasing order (slice j holds experts G j .. G j + G - 1).
-            first[q] = 0x7fffffff;
-#pragma unroll
-            for (int j = MAXJ - 1; j >= 0; --j) {
-                const int e = lig + G * j;
-                const unsigned long long m = __ballot(e < E && !((taken_bits[q] >> j) & 1u)) & gmask;
-                if (m != 0ull) first[q] = (__ffsll((long long)m) - 1 - gbase) + G * j;
-            }
-            // best candidate of this lane: not taken, not NaN; greater probability, then lower index
-            has[q] = false;
-            lbits[q] = 0;
-            le[q] = 0x7fffffffu;
-#pragma unroll
-            for (int j = 0; j < MAXJ; ++j) {
-                const int e = lig + G * j;
-                if (live[q] && e < E && !((taken_bits[q] >> j) & 1u) && pv[q][j] == pv[q][j]) {
-                    const uint32_t bits = __float_as_uint(pv[q][j]);
-                    if (!has[q] || bits > lbits[q]) {  // slices in increasing index order: a tie keeps the lower index
-                        lbits[q] = bits;
-                        le[q] = (uint32_t)e;
-                    }
-                    has[q] = true;
-                }
-            }
-        }
-        uint32_t mbits[NQ], ci[NQ];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) mbits[q] = group_umax(has[q] ? lbits[q] : 0u, G);
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) ci[q] = group_umin((has[q] && lbits[q] == mbits[q]) ? le[q] : 0x7fffffffu, G);
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            // the reference starts from the first untaken expert and replaces it only on a
-            // strictly greater probability: if that first one is NaN nothing replaces it
-            bool first_nan = false;
-#pragma unroll
-            for (int j = 0; j < MAXJ; ++j)
-                if (lig + G * j == first[q] && pv[q][j] != pv[q][j]) first_nan = true;
-            const bool nan_wins = (__ballot(first_nan) & gmask) != 0ull;
-            const bool use_first = nan_wins || ci[q] == 0x7fffffffu;
-            const int best = use_first ? first[q] : (int)ci[q];
-            float mine = 0.0f;
-#pragma unroll
-            for (int j = 0; j < MAXJ; ++j)
-                if (lig + G * j == best) {
-                    mine = pv[q][j];
-                    taken_bits[q] |= 1u << j;
-                }
-            // the winner's probability is the greatest bits themselves; only a NaN first expert has to be fetched
-            float bestv = __uint_as_float(mbits[q]);
-            if (__ballot(use_first) != 0ull) {  // uniform over the wave
-                const float fv = __shfl(mine, gbase + (best & (G - 1)));
-                if (use_first) bestv = fv;
-            }
-            total[q] = __fadd_rn(total[q], bestv);
-            if (live[q] && lig == 0) {
-                lexp[tok[q] * k + r] = ok[q] ? best : -1;
-                gates[tok[q] * k + r] = ok[q] ? bestv : 0.0f;
-            }
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-        if (ok[q] && total[q] > 0.0f)
-            for (int r = lig; r < k; r += G) gates[tok[q] * k + r] = __fdiv_rn(gates[tok[q] * k + r], total[q]);
 }
 
 // router_tail: everything behind the logits for the TB tokens of router block `blk` - softmax, log-sum-exp, top-k,
@@ -759,275 +574,13 @@ __global__ __launch_bounds__(kRouterThreads) void route_fused_kernel(
     router_tail<1, true>(lds_raw, blk, valid, T, E, k, P, lse, expert_of, gate_of, rank_in_block, blockcnt, partial);
 }
 
-// ---------------------------------------------------------------------------
-// route_rows_kernel: norm (optional), logits and everything behind them for TB = 8, 16 or 32 tokens a workgroup, with
-// the workgroup's whole rows in LDS at once.
-// What bounds routing up to some thousand tokens is not work but the length of one workgroup's chain: with 32 tokens a
-// workgroup and slices of columns staged in turn (route_fused_kernel) it takes 18 to 20 us whether 7 workgroups run or
-// 256.  So the tokens of a workgroup are chosen to spread the call over the chip, everything a workgroup reads is
-// requested in one batch, and a dot product is taken by NL neighbouring threads, thread j owning column lane j of the
-// reference's sum: a chain of d / NL rounded multiplies and adds.  A thread works on TT tokens x EE experts side by
-// side, so that TT + EE words read from LDS feed TT * EE products; its columns j, j + NL, ... lie side by side in LDS,
-// so that it reads four steps of the chain at a time.
-// NL = 8: `dot` (src/matrix.rs:26-40).  NL = 32: the quantized router's dot_lanes::<32> (src/quantized.rs:154-177), its
-// int8 rows widened on their way into LDS, the sum times the row's scale (:61).
-// The norm is RmsNorm::forward (src/norm.rs:41-61): the squares are laid down in column order beside the rows and one
-// thread a row adds them up in index order, as the reference does.
-// Measured, against route_fused_kernel (and the norm's launch in front of it): d 768, 203 tokens x 16 experts 9.5 us
-// against 18.1, with the norm 14.4 against 32.2; 4096 x 8 10.5 against 17.7; 8192 x 16 16.2 against 19.6.  Of the 14.4:
-// rows staged 2.8 us into the workgroup, normed at 6.8 (half of it the chain of 768 adds), logits at 9.1, softmax and
-// top-k at 11.2, end 12.3.
-// ---------------------------------------------------------------------------
-struct RouteRowsArgs {
-    const void* x;
-    const float* wr;
-    const int8_t* wq;
-    const float* wscale;
-    const float* bias;
-    const uint8_t* valid;
-    int T, d, E, k, EG;  // EG: experts whose router rows are in LDS together
-    float* P;
-    float* lse;
-    int* expert_of;
-    float* gate_of;
-    int* rank_in_block;
-    int* blockcnt;
-    float* partial;
-    bf16_t* rows16;
-    const float* norm_w;
-    float norm_eps;
-    void* xn_out;
-};
-// A staged row: column lane j's elements side by side, `lane_pitch` floats from one lane to the next - whole 16-byte
-// pieces (a last one short of four steps is filled up with zeros, which the sums do not see), and an odd number of
-// them, so that the lanes' pieces start in different banks.
-__host__ __device__ static int route_lane_pitch(int d, int NL) {
-    const int steps = (d / NL + 3) / 4;
-    return 4 * (steps | 1);
-}
-
+// Norm (optional), logits and everything behind them for TB tokens a workgroup (see route_rows_body).
 template <typename XT, int TB, int NL, int TT, int EE>
 __global__ __launch_bounds__(kRouterThreads, 2) void route_rows_kernel(RouteRowsArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    constexpr int NT = kRouterThreads;
-    const int T = a.T, d = a.d, E = a.E, k = a.k, EG = a.EG;
-    const int ES = E | 1;
-    float* const prob = reinterpret_cast<float*>(lds_raw);
-    const int lp = route_lane_pitch(d, NL), pitch = NL * lp;
-    float* const xs = reinterpret_cast<float*>(lds_raw + router_fixed_bytes(E, k, TB));
-    float* const ws = xs + TB * pitch;
-    float* const sq = ws + EG * pitch;   // with a norm: the squares [TB][d + 4], the norm's weights [d] (and 256 bytes of room)
-    const int sp = d + 4;                // (4: the rows' chains read from different banks)
-    float* const nws = sq + TB * sp;
-    const int tid = threadIdx.x;
-    const int t0 = blockIdx.x * TB;
-    const int nt = min(TB, T - t0);
-    const bool norm = a.norm_w != nullptr;
-
-    // Staging: 16-byte pieces of the router's rows and of the token rows, six of each a thread requested before the first
-    // is stored (96 KB a trip to memory; variables of their own: an array of them ends up in scratch memory).  A row's
-    // pieces are counted by a rounded-up reciprocal, exact for the few thousand there are.
-    constexpr int XN = Vec16<XT>::N;
-    const int wpr = NL == 32 ? d / 16 : d / 4, xpr = d / XN;
-    const uint32_t wrecip = (uint32_t)(0x100000000ull / (uint32_t)wpr) + 1u, xrecip = (uint32_t)(0x100000000ull / (uint32_t)xpr) + 1u;
-    auto put_router = [&](int i, const uint4& v) {
-        const int r = wpr == 1 ? i : (int)__umulhi((uint32_t)i, wrecip), c = i - r * wpr;
-        if constexpr (NL == 32) {
-            float* const to = ws + r * pitch + ((16 * c) % NL) * lp + (16 * c) / NL;
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int q = 0; q < 16; ++q) to[q * lp] = (float)(int8_t)(w[q >> 2] >> (8 * (q & 3)));
-        } else {
-            float* const to = ws + r * pitch + ((4 * c) % NL) * lp + (4 * c) / NL;
-            to[0] = __uint_as_float(v.x); to[lp] = __uint_as_float(v.y);
-            to[2 * lp] = __uint_as_float(v.z); to[3 * lp] = __uint_as_float(v.w);
-        }
-    };
-    auto put_row = [&](int i, const uint4& v) {
-        const int r = xpr == 1 ? i : (int)__umulhi((uint32_t)i, xrecip), c = i - r * xpr;
-        float f[XN];
-        Vec16<XT>::widen(v, f);
-        float* const to = xs + r * pitch + ((XN * c) % NL) * lp + (XN * c) / NL;
-#pragma unroll
-        for (int q = 0; q < XN; ++q) to[q * lp] = f[q];
-        if (norm) {
-            float4* const s4 = reinterpret_cast<float4*>(sq + r * sp + XN * c);
-#pragma unroll
-            for (int q = 0; q < XN / 4; ++q)
-                s4[q] = make_float4(__fmul_rn(f[4 * q], f[4 * q]), __fmul_rn(f[4 * q + 1], f[4 * q + 1]),
-                                    __fmul_rn(f[4 * q + 2], f[4 * q + 2]), __fmul_rn(f[4 * q + 3], f[4 * q + 3]));
-        }
-    };
-    auto stage = [&](int e0, int ne, auto with_rows) {
-        constexpr bool kRows = decltype(with_rows)::value;
-        const uint4* const wsrc = NL == 32 ? reinterpret_cast<const uint4*>(a.wq + (size_t)e0 * d)
-                                           : reinterpret_cast<const uint4*>(a.wr + (size_t)e0 * d);
-        const uint4* const xsrc = reinterpret_cast<const uint4*>(static_cast<const XT*>(a.x) + (size_t)t0 * d);
-        const int nw = ne * wpr, nx = kRows ? nt * xpr : 0;
-        for (int i = tid; i < max(nw, nx); i += 6 * NT) {
-            auto fw = [&](int u) -> uint4 { return wsrc[(uint32_t)min(i + u * NT, nw - 1)]; };
-            auto fx = [&](int u) -> uint4 { return xsrc[(uint32_t)min(i + u * NT, max(nx, 1) - 1)]; };
-            const uint4 w0 = fw(0), w1 = fw(1), w2 = fw(2), w3 = fw(3), w4 = fw(4), w5 = fw(5);
-            uint4 x0, x1, x2, x3, x4, x5;
-            if constexpr (kRows) { x0 = fx(0); x1 = fx(1); x2 = fx(2); x3 = fx(3); x4 = fx(4); x5 = fx(5); }
-            __builtin_amdgcn_sched_barrier(0);
-            auto pw = [&](int u, const uint4& v) { if (i + u * NT < nw) put_router(i + u * NT, v); };
-            auto px = [&](int u, const uint4& v) { if (i + u * NT < nx) put_row(i + u * NT, v); };
-            pw(0, w0); pw(1, w1); pw(2, w2); pw(3, w3); pw(4, w4); pw(5, w5);
-            if constexpr (kRows) { px(0, x0); px(1, x1); px(2, x2); px(3, x3); px(4, x4); px(5, x5); }
-        }
-    };
-    // (the short last pieces' zeros)
-    const int short_from = d / NL, short_n = (short_from + 3) / 4 * 4 - short_from;
-    if (short_n > 0)
-        for (int i = tid; i < (TB + EG) * NL * short_n; i += NT) xs[(i / short_n) * lp + short_from + i % short_n] = 0.0f;
-    if (norm)
-        for (int c = tid; c < d; c += NT) nws[c] = a.norm_w[c];
-    stage(0, min(EG, E), std::true_type{});
+    route_rows_body<XT, TB, NL, TT, EE>(a, blockIdx.x, lds_raw);
     __syncthreads();
-    if (norm) {
-        if (tid < nt) {
-            const float f = inverse_rms_of(ordered_sum(sq + tid * sp, d), d, a.norm_eps);
-            sq[tid * sp] = f;  // (the row's squares are used up)
-        }
-        __syncthreads();
-    }
-    if (norm || a.rows16 != nullptr) {
-        // the normed rows, rounded to the layer's own type, replace the raw ones; they (and the bf16 copy of f32 rows
-        // for the expert products) are written out on the way
-        const int pieces = d / 8;
-        const uint32_t recip = (uint32_t)(0x100000000ull / (uint32_t)pieces) + 1u;
-        for (int i = tid; i < nt * pieces; i += NT) {
-            const int r = pieces == 1 ? i : (int)__umulhi((uint32_t)i, recip), c = (i - r * pieces) * 8;
-            float* const at = xs + r * pitch + (c % NL) * lp + c / NL;
-            float v[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) v[q] = at[q * lp];
-            if (norm) {
-                const float sc = sq[r * sp];
-                const float4 wa = *reinterpret_cast<const float4*>(nws + c), wb = *reinterpret_cast<const float4*>(nws + c + 4);
-                const float w[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
-                XT o[8];
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    o[q] = from_f32<XT>(__fmul_rn(__fmul_rn(v[q], sc), w[q]));
-                    v[q] = to_f32(o[q]);
-                    at[q * lp] = v[q];
-                }
-                uint4* const to = reinterpret_cast<uint4*>(static_cast<XT*>(a.xn_out) + (size_t)(t0 + r) * d + c);
-#pragma unroll
-                for (int q = 0; q < 8 / XN; ++q) to[q] = reinterpret_cast<const uint4*>(o)[q];
-            }
-            if constexpr (sizeof(XT) == 4) {
-                if (a.rows16 != nullptr) {
-                    uint4 o;
-                    o.x = f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16);
-                    o.y = f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16);
-                    o.z = f32_to_bf16_bits(v[4]) | ((uint32_t)f32_to_bf16_bits(v[5]) << 16);
-                    o.w = f32_to_bf16_bits(v[6]) | ((uint32_t)f32_to_bf16_bits(v[7]) << 16);
-                    *reinterpret_cast<uint4*>(a.rows16 + (size_t)(t0 + r) * d + c) = o;
-                }
-            }
-        }
-        if (norm) __syncthreads();
-    }
-    // ---- logits -------------------------------------------------------------------
-    const int j = tid % NL;  // the thread's column lane
-    const int quads = (d / NL + 3) / 4;
-    for (int e0 = 0; e0 < E; e0 += EG) {
-        const int ne = min(EG, E - e0);
-        if (e0 > 0) {
-            __syncthreads();  // the group before has been consumed
-            stage(e0, ne, std::false_type{});
-            __syncthreads();
-        }
-        const int etiles = (ne + EE - 1) / EE;
-        const int tasks = (TB / TT) * etiles;
-        for (int g0 = 0; g0 < tasks; g0 += NT / NL) {
-            const int g = g0 + tid / NL;
-            if (g0 + (int)(threadIdx.x & ~63u) / NL >= tasks) break;  // none of the wave's groups has a tile
-            const int tt = min(g / etiles, TB / TT - 1), et = g - (g / etiles) * etiles;
-            const unsigned char *xp[TT], *wp[EE];  // (a token or expert past the end: the last one's sums again, dropped)
-#pragma unroll
-            for (int u = 0; u < TT; ++u)
-                xp[u] = reinterpret_cast<const unsigned char*>(xs + min(tt * TT + u, nt - 1) * pitch + j * lp);
-#pragma unroll
-            for (int u = 0; u < EE; ++u)
-                wp[u] = reinterpret_cast<const unsigned char*>(ws + min(et * EE + u, ne - 1) * pitch + j * lp);
-            float acc[TT][EE];
-#pragma unroll
-            for (int u = 0; u < TT; ++u)
-#pragma unroll
-                for (int v = 0; v < EE; ++v) acc[u][v] = 0.0f;
-            struct Operands {
-                float4 x[TT], w[EE];
-            };
-            // four steps of the chain a trip, the next trip's operands read before this one's products (two sets of
-            // registers take turns)
-            auto read = [&](Operands& o, int q) {
-#pragma unroll
-                for (int u = 0; u < TT; ++u) o.x[u] = lds_load_ahead<float4>(xp[u] + 16 * q);
-#pragma unroll
-                for (int u = 0; u < EE; ++u) o.w[u] = lds_load_ahead<float4>(wp[u] + 16 * q);
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            auto multiply = [&](const Operands& o) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-#pragma unroll
-                    for (int u = 0; u < TT; ++u)
-#pragma unroll
-                        for (int v = 0; v < EE; ++v)
-                            acc[u][v] = __fadd_rn(acc[u][v], __fmul_rn(reinterpret_cast<const float*>(&o.x[u])[c],
-                                                                       reinterpret_cast<const float*>(&o.w[v])[c]));
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            Operands oa, ob;
-            read(oa, 0);
-            int q = 0;
-            for (; q + 2 <= quads; q += 2) {
-                read(ob, q + 1);
-                multiply(oa);
-                read(oa, min(q + 2, quads - 1));
-                multiply(ob);
-            }
-            if (q < quads) multiply(oa);
-            // the column lanes folded left to right: lane l of a group holds ((0 + a_0) + a_1) + ... + a_l after l steps
-            // of "take the lane below's sum, add your own" (see softmax_topk), the products side by side
-            float own[TT][EE];
-#pragma unroll
-            for (int u = 0; u < TT; ++u)
-#pragma unroll
-                for (int v = 0; v < EE; ++v) {
-                    own[u][v] = acc[u][v];
-                    acc[u][v] = __fadd_rn(0.0f, acc[u][v]);
-                }
-            for (int st = 1; st < NL; ++st) {
-#pragma unroll
-                for (int u = 0; u < TT; ++u)
-#pragma unroll
-                    for (int v = 0; v < EE; ++v) {
-                        const float below = __uint_as_float(lanes_from<0x138>(__float_as_uint(acc[u][v])));  // wave_shr:1
-                        const float next = __fadd_rn(below, own[u][v]);
-                        acc[u][v] = j == 0 ? acc[u][v] : next;
-                    }
-            }
-#pragma unroll
-            for (int u = 0; u < TT; ++u)
-#pragma unroll
-                for (int v = 0; v < EE; ++v) {
-                    const int t = tt * TT + u, el = et * EE + v, e = e0 + el;
-                    if (j == NL - 1 && g < tasks && t < nt && el < ne) {
-                        float y = __fadd_rn(acc[u][v], 0.0f);  // the reference adds its (empty) scalar rest: sum + 0
-                        if constexpr (NL == 32) y = __fmul_rn(y, a.wscale[e]);
-                        if (a.bias) y = __fadd_rn(y, a.bias[e]);
-                        prob[t * ES + e] = y;
-                    }
-                }
-        }
-    }
-    __syncthreads();
-    router_tail<1, true, TB>(lds_raw, blockIdx.x, a.valid, T, E, k, a.P, a.lse, a.expert_of, a.gate_of, a.rank_in_block,
+    router_tail<1, true, TB>(lds_raw, blockIdx.x, a.valid, a.T, a.E, a.k, a.P, a.lse, a.expert_of, a.gate_of, a.rank_in_block,
                              a.blockcnt, a.partial);
 }
 
@@ -1686,18 +1239,17 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     if ((reinterpret_cast<uintptr_t>(a.x) & 15) || ((size_t)a.d * xsize) % 16 != 0) return p;
     if (reinterpret_cast<uintptr_t>(a.wq ? static_cast<const void*>(a.wq) : a.wr) & 15) return p;
     if (a.norm_w && ((reinterpret_cast<uintptr_t>(a.xn_out) & 15) || a.d % 8 != 0)) return p;
-    const size_t row = (size_t)(a.wq ? 32 * route_lane_pitch(a.d, 32) : 8 * route_lane_pitch(a.d, 8)) * 4;
+    const int NL = a.wq ? 32 : 8;
     int tokens = kMinRouterTokens;
     while (tokens < kRouterTokens && (a.T + tokens - 1) / tokens > 256) tokens *= 2;
-    for (; tokens >= kMinRouterTokens; tokens /= 2) {
-        const size_t fixed = router_fixed_bytes(a.E, a.k, tokens) + (size_t)tokens * row +
-                             (a.norm_w ? (size_t)(tokens + 1) * (a.d + 4) * 4 + 256 : 0);
-        if (fixed + std::min(a.E, 8) * row > (size_t)kMaxRouterLds) continue;
+    for (; tokens >= kMinRouterTokens && !p.tokens; tokens /= 2) {
+        int EG = a.E;  // as many experts' rows as fit together, whole pairs, at least 8 (or all of them)
+        auto lds = [&] { return route_rows_lds_bytes(a.E, a.k, a.d, tokens, NL, EG, a.norm_w != nullptr); };
+        while (EG > 8 && lds() > (size_t)kMaxRouterLds) EG = (EG - 1) & ~1;
+        if (lds() > (size_t)kMaxRouterLds) continue;
         p.tokens = tokens;
-        p.EG = std::min<int>(a.E, (int)(((size_t)kMaxRouterLds - fixed) / row));
-        if (p.EG < a.E && p.EG > 2) p.EG &= ~1;  // whole pairs of experts
-        p.lds = fixed + (size_t)p.EG * row;
-        break;
+        p.EG = EG;
+        p.lds = lds();
     }
     if (!p.tokens) return p;
     // above: the sequences tuned for launches that fill the chip several times over.  Rows so wide that fewer tokens fit

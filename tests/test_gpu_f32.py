@@ -59,3 +59,17 @@ def test_f32_matrix_core_and_generic_kernels_agree(device):
             os.environ.pop("RBMOE_FORCE_GENERIC", None)
         else:
             os.environ["RBMOE_FORCE_GENERIC"] = saved
+
+
+@pytest.mark.parametrize("shape", [dict(d=96, E=3, k=2, F=96, T=16411), dict(d=32, E=5, k=2, F=160, T=33001)],
+                         ids=lambda s: "d{d}_E{E}_k{k}_F{F}_T{T}".format(**s))
+def test_f32_tiles_of_64_rows(device, shape):
+    """Enough rows for 64-row tiles: ragged last tiles, partial feature tiles, reductions of one to five slices of 32."""
+    t = synth.make(small_workload(seed=44, act="f32", wt="f32", shared=True, shared_d_ff=64, **shape))
+    ref = oracle_layer(t).forward(t.x, threads=8)
+    layer = gpu_layer(device, t)
+    out, cache = layer.forward_train(t.x)
+    assert layer.kernel_name() == "mfma_f32"
+    assert_routing_identical(cache, ref)
+    assert rel_l2(out, ref.out) <= 1e-5
+    layer.close()

@@ -553,6 +553,277 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     RBMOE_TRACE_AT(blockIdx.x, 3);
 }
 
+
+// ---- the narrow kernel: launches with few tiles ------------------------------------------------------
+// Half the weight rows a workgroup (a wave owns 128 token rows x ONE block of 32 weight rows) and a deep weight ring.
+// With fewer workgroups than compute units the kernel above is bound by the latency of its weight loads: they run
+// three steps (0.3 us) ahead, a first touch of expert weights takes one to two microseconds, and a lone workgroup took
+// 1.1 us a slice of 64 columns whose multiplies last 0.43.  Half the accumulators leave registers for 16 steps of
+// weights under way, a fourth LDS stage lets the DMA run three slices ahead, and there are twice as many workgroups.
+// A full chip is better off with the kernel above: here each token fragment read from LDS serves one multiply instead
+// of two.
+//   gate/up: waves 0 and 1 take 64 gate rows, waves 2 and 3 the matching up rows, which meet in LDS at the end.
+//   down:    four blocks of 32 features side by side.
+// Issue order inside a step: the ring load, then (last step of a slice) the four DMA instructions.  Step g's ring load
+// was issued in step g - 15; younger are 14 ring loads and the DMA of the last steps among g - 15 .. g - 1: four of
+// them, three when g itself is one.  The DMA of slice kt + 1 was issued in the last step of slice kt - 2; when slice
+// kt waits for it behind its step KS - 2, seven ring loads and the DMA of slice kt + 2 are younger.
+constexpr int NRING = 16;
+constexpr int NSTAGES = 4;
+
+template <bool I8>
+struct Slot1;
+template <>
+struct Slot1<false> {
+    u32x4 f;
+    static __device__ __forceinline__ uint32_t offset(int g, uint32_t lane16) { return Slot<false>::offset(g, lane16); }
+    __device__ __forceinline__ bf16x8 frag() const { return __builtin_bit_cast(bf16x8, f); }
+};
+template <>
+struct Slot1<true> {
+    u32x2 f;
+    static __device__ __forceinline__ uint32_t offset(int g, uint32_t lane16) { return Slot<true>::offset(g, lane16); }
+    __device__ __forceinline__ bf16x8 frag() const { return widen_i8(make_uint2(f.x, f.y)); }
+};
+
+template <int N, typename V>
+__device__ __forceinline__ void wait_for1(V& a) {
+    asm volatile("s_waitcnt vmcnt(%1)" : "+v"(a) : "n"(N));
+}
+
+// As pipe_loop: before the call nothing is outstanding (slices 0 .. NSTAGES - 2 and ring steps 0 .. NRING - 2 have
+// landed) and the workgroup has met at a barrier; after it nothing is outstanding.
+template <bool I8, int NB>
+__device__ __forceinline__ void narrow_loop(const PipeCtx& c, floatx16 (&acc)[TT], Slot1<I8> (&ring)[NRING],
+                                            const uint32_t (&a_src)[DMA_PER_WAVE]) {
+    constexpr int D = NRING - 1;
+    static_assert(KS == 4 && NRING == 16 && NSTAGES == 4 && DMA_PER_WAVE == 4 && TT == 4, "the wait counts are derived for this");
+    const uint4* const As = c.As;
+    const uint32_t lds0 = c.lds0, lane16 = c.lane16;
+    const char* const a_base = c.a_base;
+    const char* const wp = c.wp0;
+    const int KT = c.KT, GS = KT * KS;
+    int frag0 = c.lrow * CPR + (c.lhalf ^ c.lxor);
+    bf16x8 tf[2][TT];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) tf[0][t] = lds_frag(As, t * 32 * CPR + frag0);
+    auto pslice = [&](int kt, auto idx_tag) {
+        constexpr int IDX = decltype(idx_tag)::value;  // kt % 4
+        constexpr int NEXT = (IDX + 1) % NSTAGES, FREE = (IDX + 3) % NSTAGES;
+        const uint4* const Ab = As + IDX * (BM * CPR);
+        const uint4* const An = As + NEXT * (BM * CPR);
+        asm volatile("" : "+v"(frag0));
+        static_for<0, KS>([&](auto s_tag) {
+            constexpr int s = decltype(s_tag)::value;
+            constexpr bool LAST = s == KS - 1;
+            constexpr int P = IDX * KS + s;  // ring position of step g
+            const int g = kt * KS + s;
+            wait_for1<(D - 1) + DMA_PER_WAVE * (LAST ? 3 : 4)>(ring[P].f);
+            const bf16x8 w = ring[P].frag();
+            const uint32_t woff = Slot1<I8>::offset(min(g + D, GS - 1), lane16);
+            const uint32_t aoff = (uint32_t)min(kt + 3, KT - 1) * (BK * 2);
+            const int frag = frag0 ^ (2 * ((s + 1) % KS));
+            constexpr int NOPS = 1 + (LAST ? DMA_PER_WAVE : NB);
+            auto op = [&](auto i_tag) {
+                constexpr int i = decltype(i_tag)::value;
+                if constexpr (i == 0) {
+                    issue_load(ring[(P + D) % NRING].f, woff, wp);
+                } else {
+                    constexpr int j = i - 1;
+                    if constexpr (LAST)
+                        issue_dma(lds0 + FREE * (BM * CPR * 16) + j * 8 * CPR * 16, a_src[j] + aoff, a_base);
+                    if constexpr (j < NB) tf[(s + 1) & 1][j] = lds_frag(LAST ? An : Ab, j * 32 * CPR + frag);
+                }
+            };
+            static_for<0, NB>([&](auto m_tag) {
+                constexpr int m = decltype(m_tag)::value;
+                acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, tf[s & 1][m], acc[m], 0, 0, 0);
+                if constexpr (m < NOPS) op(m_tag);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            static_for<NB, NOPS>(op);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (s == KS - 2) {
+                wait_outstanding<(2 * KS - 1) + DMA_PER_WAVE>();
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        });
+    };
+    int kt = 0;
+    for (; kt + 4 <= KT; kt += 4)
+        static_for<0, 4>([&](auto i) { pslice(kt + decltype(i)::value, i); });
+    static_while<0, 3>([&](auto i) {
+        if (kt + decltype(i)::value >= KT) return false;
+        pslice(kt + decltype(i)::value, i);
+        return true;
+    });
+    wait_outstanding<0>();
+#pragma unroll
+    for (int i = 0; i < NRING; ++i) asm volatile("" : : "v"(ring[i].f));
+}
+
+template <bool SWIGLU, bool I8>
+__global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
+    const bf16_t* __restrict__ a, const int* __restrict__ row_index, const void* __restrict__ wpacked,
+    size_t w_expert_stride_bytes, const float* __restrict__ scales, size_t s_expert_stride, int N, int K,
+    const int* __restrict__ tile_expert, const int* __restrict__ tile_row0, const int* __restrict__ tile_rows,
+    const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, int group_m) {
+    constexpr int BN = SWIGLU ? 64 : 128;  // output features per workgroup
+    __shared__ uint4 As[NSTAGES * BM * CPR];
+
+    const int tiles_n = (N + BN - 1) / BN;
+    const int tiles_m = dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles;
+    const int total = tiles_m * tiles_n;
+    const int per_xcd = (total + 7) / 8;
+    const int local = blockIdx.x >> 3;
+    if (local >= per_xcd) return;
+    const int pid = (blockIdx.x & 7) * per_xcd + local;
+    if (pid >= total) return;
+    const int per_group = group_m * tiles_n;
+    const int grp = pid / per_group;
+    const int first_m = grp * group_m;
+    const int gsize = min(group_m, tiles_m - first_m);
+    const int in_g = pid - grp * per_group;
+    const int tm_idx = first_m + in_g % gsize;
+    const int n0 = in_g / gsize * BN;
+
+    int expert, row0, rows;
+    if (dense_rows >= 0) {
+        expert = 0;
+        row0 = tm_idx * BM;
+        rows = min(BM, dense_rows - row0);
+    } else {
+        expert = tile_expert[tm_idx];
+        row0 = tile_row0[tm_idx];
+        rows = tile_rows[tm_idx];
+    }
+    const int nblk = (rows + 31) >> 5;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    // this wave's 32 weight rows; past N (ragged last feature tile) it runs the same loop on block 0 and stores nothing
+    const int fb = n0 + (SWIGLU ? wave & 1 : wave) * 32;  // its first output feature
+    const bool act = fb < N;
+    const int wrow = SWIGLU && wave >= 2 ? N + fb : fb;
+    const size_t block_bytes = (size_t)K * 32 * (I8 ? 1 : 2);
+    const char* const wp = static_cast<const char*>(wpacked) + (size_t)expert * w_expert_stride_bytes +
+                           (size_t)(act ? wrow / 32 : 0) * block_bytes;
+    const uint32_t lane16 = (uint32_t)lane * 16u;
+
+    // LDS-DMA of the activation slices: as in the kernel above
+    const char* const a_base = reinterpret_cast<const char*>(a);
+    uint32_t a_src[DMA_PER_WAVE];
+#pragma unroll
+    for (int j = 0; j < DMA_PER_WAVE; ++j) {
+        const int r = wave * (BM / NW) + j * 8 + (lane >> 3);
+        const int rr = r < rows ? r : 0;
+        const int grow = row_index ? row_index[row0 + rr] : row0 + rr;
+        a_src[j] = ((uint32_t)grow * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)As + wave * (BM / NW) * CPR * 16;
+    const int KT = K / BK, GS = KT * KS;
+
+    floatx16 acc[TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[t][v] = 0.0f;
+
+    Slot1<I8> ring[NRING];
+#pragma unroll
+    for (int g = 0; g < NRING - 1; ++g) issue_load(ring[g].f, Slot1<I8>::offset(min(g, GS - 1), lane16), wp);
+    static_for<0, NSTAGES - 1>([&](auto st) {
+        constexpr int ST = decltype(st)::value;
+#pragma unroll
+        for (int j = 0; j < DMA_PER_WAVE; ++j)
+            issue_dma(lds0 + ST * (BM * CPR * 16) + j * 8 * CPR * 16, a_src[j] + (uint32_t)min(ST, KT - 1) * (BK * 2), a_base);
+    });
+    wait_outstanding<0>();
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    {
+        const int lrow = lane & 31;
+        const PipeCtx pc{As, lds0, a_base, wp, nullptr, lane16, lrow, lane >> 5, (lrow >> 1) & 7, KT};
+        if (nblk >= 4) narrow_loop<I8, 4>(pc, acc, ring, a_src);
+        else if (nblk == 3) narrow_loop<I8, 3>(pc, acc, ring, a_src);
+        else if (nblk == 2) narrow_loop<I8, 2>(pc, acc, ring, a_src);
+        else narrow_loop<I8, 1>(pc, acc, ring, a_src);
+    }
+    __syncthreads();  // every wave's last DMA has landed and its last fragment reads are done
+
+    // ---- epilogue: accumulator element v of lane l is feature 8 (v / 4) + 4 (l / 32) + v % 4, token t * 32 + l % 32
+    char* const lds = reinterpret_cast<char*>(As);
+    const int lrow = lane & 31, lhalf = lane >> 5;
+    const float* const sc = I8 ? scales + (size_t)expert * s_expert_stride + (act ? wrow : 0) : nullptr;
+    if constexpr (I8) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[t][v] *= sc[8 * (v >> 2) + 4 * lhalf + (v & 3)];
+    }
+    constexpr int XCH = 2 * TT * 16 * 64 * 4;  // gate/up: the up waves' accumulators, 32 KiB; the output tile behind them
+    char* const stage = lds + (SWIGLU ? XCH : 0);
+    if constexpr (SWIGLU) {
+        float4* const xch = reinterpret_cast<float4*>(lds) + (wave & 1) * (TT * 4 * 64) + lane;
+        if (wave >= 2) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (t * 32 < rows)
+                        xch[(t * 4 + q) * 64] =
+                            make_float4(acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]);
+        }
+        __syncthreads();
+        if (wave < 2) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (t * 32 < rows) {
+                        const float4 u = xch[(t * 4 + q) * 64];
+                        acc[t][4 * q + 0] = silu_bf16_grade(acc[t][4 * q + 0]) * u.x;
+                        acc[t][4 * q + 1] = silu_bf16_grade(acc[t][4 * q + 1]) * u.y;
+                        acc[t][4 * q + 2] = silu_bf16_grade(acc[t][4 * q + 2]) * u.z;
+                        acc[t][4 * q + 3] = silu_bf16_grade(acc[t][4 * q + 3]) * u.w;
+                    }
+        }
+    }
+    // the output tile through LDS (16-byte pieces, piece p of row r at position p ^ (r % pieces)), then 16-byte stores
+    constexpr int PW = BN / 8;
+    if (act && (!SWIGLU || wave < 2)) {
+        const int w = SWIGLU ? wave & 1 : wave;
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+            if (t * 32 >= rows) continue;
+            const int m = t * 32 + lrow;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<uint2*>(stage + m * (BN * 2) + ((w * 4 + q) ^ (m & (PW - 1))) * 16 + lhalf * 8) =
+                    make_uint2(pack2(acc[t][4 * q], acc[t][4 * q + 1]), pack2(acc[t][4 * q + 2], acc[t][4 * q + 3]));
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < BM * PW / NT; ++i) {
+        const int idx = i * NT + tid;
+        const int r = idx / PW, p = idx % PW;
+        if (r < rows && n0 + 8 * p < N)
+            *reinterpret_cast<uint4*>(out + (size_t)(row0 + r) * N + n0 + 8 * p) =
+                *reinterpret_cast<const uint4*>(stage + r * (BN * 2) + ((p ^ (r & (PW - 1))) * 16));
+    }
+}
+
+// At most this many wide tiles take the narrow kernel.  Down: up to one a compute unit.  us, wide against narrow, at so
+// many tiles of d 768 (K 1408; * int8 weights): 57 (203 rows) 17.2 / 10.6, 72* 23.2 / 15.0, 93* 24.2 / 16.1, 216* 29.3 /
+// 27.0, 432 41.1 / 47.1; 80 of d 512 (K 384) 9.9 / 6.8.  Gate/up workgroups are twice as many per tile (64 features) and
+// their reductions short, so the line is lower: 120 tiles (K 512) 11.8 / 10.5, 209 (K 768) 15.0 / 16.5, 264* 18.3 / 19.6.
+// Launches that keep or read pre-activations (training) stay with the wide kernel's epilogue.
+constexpr int kNarrowDownTiles = 256;
+constexpr int kNarrowGateUpTiles = 128;
+
 template <bool SWIGLU, bool I8>
 hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
     constexpr int BN = SWIGLU ? NW * 32 : NW * 64;
@@ -561,6 +832,14 @@ hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
     if (tiles_m <= 0) return hipSuccess;
     const int total = tiles_m * tiles_n;
     const int grid = ((total + 7) / 8) * 8;
+    if (total <= (SWIGLU ? kNarrowGateUpTiles : kNarrowDownTiles) && !g.gu_out && !g.swiglu_grad_gu) {
+        const int narrow = (g.N + BN / 2 - 1) / (BN / 2) * tiles_m;
+        RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((narrow + 7) / 8 * 8), dim3(NT), 0, s,
+                  static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
+                  g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
+                  static_cast<bf16_t*>(g.out), g.group_m > 0 ? g.group_m : 8);
+        return hipGetLastError();
+    }
     RB_LAUNCH((grouped_stream_kernel<SWIGLU, I8>), dim3(grid), dim3(NT), 0, s,
                        static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
                        g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,

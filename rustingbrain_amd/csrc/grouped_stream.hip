@@ -418,35 +418,72 @@ __device__ __forceinline__ void pipe_loop(const PipeCtx& c, floatx16 (&acc)[2][T
     for (int i = 0; i < RING; ++i) asm volatile("" : : "v"(ring_ref[i].f0), "v"(ring_ref[i].f1));
 }
 
+// Which tile a workgroup takes.  Each XCD (workgroup number mod 8) walks a contiguous range of the launch's tiles, M
+// fastest inside a group of row tiles; the tiles of the second, dense group (the shared expert's, in the same launch)
+// come behind the routed ones, and its operands take the place of the routed experts' (all of it uniform over the
+// workgroup).  `tm` < 0: no tile.
+struct TileAt {
+    int tm, tn;
+    bool second;
+};
+template <int BN>
+__device__ __forceinline__ TileAt tile_at(int tiles_m, int N, int group_m, int rows2, int N2) {
+    int tiles_n = (N + BN - 1) / BN;
+    const int total1 = tiles_m * tiles_n;
+    const int tiles_n2 = (N2 + BN - 1) / BN, tiles_m2 = (rows2 + BM - 1) / BM;
+    const int total = total1 + tiles_m2 * tiles_n2;
+    const int per_xcd = (total + 7) / 8;
+    const int local = blockIdx.x >> 3;
+    int pid = (blockIdx.x & 7) * per_xcd + local;
+    if (local >= per_xcd || pid >= total) return {-1, 0, false};
+    const bool second = pid >= total1;
+    if (second) {
+        pid -= total1;
+        tiles_n = tiles_n2;
+        tiles_m = tiles_m2;
+    }
+    const int per_group = group_m * tiles_n;
+    const int grp = pid / per_group;
+    const int first_m = grp * group_m;
+    const int gsize = min(group_m, tiles_m - first_m);
+    const int in_g = pid - grp * per_group;
+    return {first_m + in_g % gsize, in_g / gsize, second};
+}
+
+struct DenseGroup {
+    const bf16_t* a;
+    const void* w;
+    const float* scales;
+    int N, K, rows;
+    bf16_t *out, *gu_out;
+};
+
 template <bool SWIGLU, bool I8>
 __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     const bf16_t* __restrict__ a, const int* __restrict__ row_index, const void* __restrict__ wpacked,
     size_t w_expert_stride_bytes, const float* __restrict__ scales, size_t s_expert_stride, int N, int K,
     const int* __restrict__ tile_expert, const int* __restrict__ tile_row0, const int* __restrict__ tile_rows,
     const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, bf16_t* __restrict__ gu_out,
-    const bf16_t* __restrict__ bw_gu,
-    int group_m) {
+    const bf16_t* __restrict__ bw_gu, int group_m, DenseGroup g2) {
     constexpr int BN = SWIGLU ? NW * 32 : NW * 64;  // output features per workgroup
     // LDS stages of one activation slice each; the epilogue reuses the first two as one
     // 128 x 128 staging tile for the output.
     __shared__ uint4 As[STAGES * BM * CPR];
 
-    // ---- which tile (each XCD walks a contiguous range, M fastest inside a group)
-    const int tiles_n = (N + BN - 1) / BN;
-    const int tiles_m = dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles;
-    const int total = tiles_m * tiles_n;
-    const int per_xcd = (total + 7) / 8;
-    const int local = blockIdx.x >> 3;
-    if (local >= per_xcd) return;
-    const int pid = (blockIdx.x & 7) * per_xcd + local;
-    if (pid >= total) return;
-    const int per_group = group_m * tiles_n;
-    const int grp = pid / per_group;
-    const int first_m = grp * group_m;
-    const int gsize = min(group_m, tiles_m - first_m);
-    const int in_g = pid - grp * per_group;
-    const int tm_idx = first_m + in_g % gsize;
-    const int tn_idx = in_g / gsize;
+    const TileAt at = tile_at<BN>(dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
+    if (at.tm < 0) return;
+    const int tm_idx = at.tm, tn_idx = at.tn;
+    if (at.second) {
+        a = g2.a;
+        row_index = nullptr;
+        wpacked = g2.w;
+        scales = g2.scales;
+        N = g2.N;
+        K = g2.K;
+        dense_rows = g2.rows;
+        out = g2.out;
+        gu_out = g2.gu_out;
+    }
 
     RBMOE_TRACE_AT(blockIdx.x, 0);
     int expert, row0, rows;
@@ -668,25 +705,24 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
     const bf16_t* __restrict__ a, const int* __restrict__ row_index, const void* __restrict__ wpacked,
     size_t w_expert_stride_bytes, const float* __restrict__ scales, size_t s_expert_stride, int N, int K,
     const int* __restrict__ tile_expert, const int* __restrict__ tile_row0, const int* __restrict__ tile_rows,
-    const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, int group_m) {
+    const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, int group_m, DenseGroup g2) {
     constexpr int BN = SWIGLU ? 64 : 128;  // output features per workgroup
     __shared__ uint4 As[NSTAGES * BM * CPR];
 
-    const int tiles_n = (N + BN - 1) / BN;
-    const int tiles_m = dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles;
-    const int total = tiles_m * tiles_n;
-    const int per_xcd = (total + 7) / 8;
-    const int local = blockIdx.x >> 3;
-    if (local >= per_xcd) return;
-    const int pid = (blockIdx.x & 7) * per_xcd + local;
-    if (pid >= total) return;
-    const int per_group = group_m * tiles_n;
-    const int grp = pid / per_group;
-    const int first_m = grp * group_m;
-    const int gsize = min(group_m, tiles_m - first_m);
-    const int in_g = pid - grp * per_group;
-    const int tm_idx = first_m + in_g % gsize;
-    const int n0 = in_g / gsize * BN;
+    const TileAt at = tile_at<BN>(dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
+    if (at.tm < 0) return;
+    const int tm_idx = at.tm, tn_idx = at.tn;
+    if (at.second) {
+        a = g2.a;
+        row_index = nullptr;
+        wpacked = g2.w;
+        scales = g2.scales;
+        N = g2.N;
+        K = g2.K;
+        dense_rows = g2.rows;
+        out = g2.out;
+    }
+    const int n0 = tn_idx * BN;
 
     int expert, row0, rows;
     if (dense_rows >= 0) {
@@ -827,24 +863,28 @@ constexpr int kNarrowGateUpTiles = 128;
 template <bool SWIGLU, bool I8>
 hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
     constexpr int BN = SWIGLU ? NW * 32 : NW * 64;
-    const int tiles_n = (g.N + BN - 1) / BN;
     const int tiles_m = g.dense_rows >= 0 ? (g.dense_rows + BM - 1) / BM : g.max_tiles;
-    if (tiles_m <= 0) return hipSuccess;
-    const int total = tiles_m * tiles_n;
-    const int grid = ((total + 7) / 8) * 8;
+    const GroupedArgs::Dense& d2 = g.dense2;
+    auto tiles = [&](int bn) {
+        return tiles_m * ((g.N + bn - 1) / bn) + (d2.rows + BM - 1) / BM * ((d2.N + bn - 1) / bn);
+    };
+    const int total = tiles(BN);
+    if (total <= 0) return hipSuccess;
+    const DenseGroup g2{static_cast<const bf16_t*>(d2.a), d2.w, d2.scales, d2.N, d2.K, d2.rows,
+                        static_cast<bf16_t*>(d2.out), static_cast<bf16_t*>(d2.gu_out)};
+    const int group_m = g.group_m > 0 ? g.group_m : 8;
     if (total <= (SWIGLU ? kNarrowGateUpTiles : kNarrowDownTiles) && !g.gu_out && !g.swiglu_grad_gu) {
-        const int narrow = (g.N + BN / 2 - 1) / (BN / 2) * tiles_m;
-        RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((narrow + 7) / 8 * 8), dim3(NT), 0, s,
+        RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((tiles(BN / 2) + 7) / 8 * 8), dim3(NT), 0, s,
                   static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
                   g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
-                  static_cast<bf16_t*>(g.out), g.group_m > 0 ? g.group_m : 8);
+                  static_cast<bf16_t*>(g.out), group_m, g2);
         return hipGetLastError();
     }
-    RB_LAUNCH((grouped_stream_kernel<SWIGLU, I8>), dim3(grid), dim3(NT), 0, s,
-                       static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
-                       g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
-                       static_cast<bf16_t*>(g.out), static_cast<bf16_t*>(g.gu_out), static_cast<const bf16_t*>(g.swiglu_grad_gu),
-                       g.group_m > 0 ? g.group_m : 8);
+    RB_LAUNCH((grouped_stream_kernel<SWIGLU, I8>), dim3((total + 7) / 8 * 8), dim3(NT), 0, s,
+              static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
+              g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
+              static_cast<bf16_t*>(g.out), static_cast<bf16_t*>(g.gu_out), static_cast<const bf16_t*>(g.swiglu_grad_gu),
+              group_m, g2);
     return hipGetLastError();
 }
 
@@ -858,6 +898,8 @@ bool stream_shape_ok(int N, int K) { return K % 64 == 0 && K >= 64 && N % 32 == 
 
 hipError_t launch_grouped_stream(const GroupedArgs& g, WeightKind wk, hipStream_t s) {
     if (!stream_shape_ok(g.N, g.K)) return hipErrorInvalidValue;
+    if (g.dense2.rows > 0 && (!stream_shape_ok(g.dense2.N, g.dense2.K) || !g.dense2.gu_out != !g.gu_out || g.swiglu_grad_gu))
+        return hipErrorInvalidValue;
     if (wk == WeightKind::BF16) return g.swiglu ? launch_t<true, false>(g, s) : launch_t<false, false>(g, s);
     if (wk == WeightKind::I8) return g.swiglu ? launch_t<true, true>(g, s) : launch_t<false, true>(g, s);
     return hipErrorInvalidValue;

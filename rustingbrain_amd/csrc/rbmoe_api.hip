@@ -1228,35 +1228,47 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         return launch_grouped_generic(g, abf, wk, kGenericTileM, st);
     };
     auto run = [&](const GroupedArgs& g, bool) -> hipError_t { return run_on(g, s); };
-    // The shared expert (src/moe.rs:313-319) takes every row and needs nothing of the routing: with a second stream
-    // its two products run beside the routing kernels, which are bound by the vector units and by latency and
-    // leave the matrix cores idle.  (Not when the stages are timed one by one, and not over f32 rows, whose bf16
-    // copy the logits kernel has yet to write.)
+    // The shared expert (src/moe.rs:313-319) takes every row and needs nothing of the routing: its products run in the
+    // routed experts' launches, or with a second stream beside the routing kernels, which are bound by the vector units
+    // and by latency and leave the matrix cores idle.  (Neither when the stages are timed one by one; not beside over f32
+    // rows, whose bf16 copy the logits kernel has yet to write.)
+    GroupedArgs s1{};  // gate/up, and (s2) the down product
+    s1.a = xe;
+    s1.w = L->swgu.p;
+    s1.scales = wk == WeightKind::I8 ? (const float*)L->ssgu.p : nullptr;
+    s1.N = Fs;
+    s1.K = d;
+    s1.dense_rows = T;
+    s1.out = L->hs.p;
+    s1.swiglu = true;
+    s1.group_m = L->group_m;
+    if (L->training) s1.gu_out = L->gus.p;
+    GroupedArgs s2 = s1;
+    s2.a = L->hs.p;
+    s2.w = L->swd.p;
+    s2.scales = wk == WeightKind::I8 ? (const float*)L->ssd.p : nullptr;
+    s2.gu_out = nullptr;
+    s2.N = d;
+    s2.K = Fs;
+    s2.out = L->ys.p;
+    s2.swiglu = false;
+    if (L->group_m == 0) s2.group_m = 4;
     auto shared_expert = [&](hipStream_t st) -> hipError_t {
-        GroupedArgs s1{};
-        s1.a = xe;
-        s1.w = L->swgu.p;
-        s1.scales = wk == WeightKind::I8 ? (const float*)L->ssgu.p : nullptr;
-        s1.N = Fs;
-        s1.K = d;
-        s1.dense_rows = T;
-        s1.out = L->hs.p;
-        s1.swiglu = true;
-        s1.group_m = L->group_m;
-        if (L->training) s1.gu_out = L->gus.p;
-        hipError_t e = run_on(s1, st);
-        if (e != hipSuccess) return e;
-        GroupedArgs s2 = s1;
-        s2.a = L->hs.p;
-        s2.w = L->swd.p;
-        s2.scales = wk == WeightKind::I8 ? (const float*)L->ssd.p : nullptr;
-        s2.gu_out = nullptr;
-        s2.N = d;
-        s2.K = Fs;
-        s2.out = L->ys.p;
-        s2.swiglu = false;
-        if (L->group_m == 0) s2.group_m = 4;
-        return run_on(s2, st);
+        const hipError_t e = run_on(s1, st);
+        return e != hipSuccess ? e : run_on(s2, st);
+    };
+    // Its tiles join the routed experts' launches where those do not fill the chip: below 1024 rows, where the products
+    // would otherwise follow one another, and up to kSharedInsideTiles gate/up tiles in all.  Above, it runs beside the
+    // routing kernels.  us a step, inside against beside (one behind the other below 1024 rows), at so many tiles: d 512,
+    // 8 experts of 352 and one shared, 64 rows 33.6 / 46.3, 2048 rows (168 tiles) 42.5 / 63.4, 4096 (312) 56.1 / 66.3, 8192
+    // (600) 79.6 / 86.2; d 768, 8 of 1408, 256 rows 43.2 / 63.2, 2048 (616) 76.5 / 80.4, 4096 (1144) 112.0 / 111.2; d 1024,
+    // 64 of 704, six a row, 1000 rows 126.5 / 139.0, 2048 (1136) 164.5 / 154.0.
+    constexpr int kSharedInsideTiles = 768;
+    const int gate_up_tiles = ((T * k) / tile_m0 + E) * ((F + 127) / 128) + (T + 127) / 128 * ((Fs + 127) / 128);
+    const bool shared_inside = c.shared_expert && mfma && !timed && T > 0 && (T < 1024 || gate_up_tiles <= kSharedInsideTiles);
+    auto with_shared = [&](GroupedArgs g, const GroupedArgs& sh) {
+        g.dense2 = {sh.a, sh.w, sh.scales, sh.N, sh.K, sh.dense_rows, sh.out, sh.gu_out};
+        return g;
     };
     struct JoinGuard {  // an error between fork and join must not leave the side stream forked (a capture could not end)
         rbmoe_ctx* ctx;
@@ -1268,7 +1280,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     } join_guard{ctx, s};
     bool shared_forked = false;
     auto fork_shared = [&]() -> int {
-        if (c.shared_expert && T >= 1024 && !timed && !cast && L->shared_beside && (mfma || f32mc) &&
+        if (c.shared_expert && !shared_inside && T >= 1024 && !timed && !cast && L->shared_beside && (mfma || f32mc) &&
             ensure_side_stream(ctx) == RBMOE_OK) {
             HIP_TRY(ctx, hipEventRecord(ctx->ev_fork, s));
             HIP_TRY(ctx, hipStreamWaitEvent(ctx->side_stream, ctx->ev_fork, 0));
@@ -1345,7 +1357,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     g1.swiglu = true;
     g1.group_m = L->group_m;
     if (L->training) g1.gu_out = L->gu.p;
-    HIP_TRY(ctx, run(g1, true));
+    HIP_TRY(ctx, run(shared_inside ? with_shared(g1, s1) : g1, true));
     L->replay[RBMOE_STAGE_GATE_UP] = [=](hipStream_t st) { return run_on(g1, st); };
     HIP_TRY(ctx, mark(4));
 
@@ -1366,11 +1378,11 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // rows, which are wider, for the down product (measured HBM-side traffic: 270 against 301 MB with groups of 8
     // against 4 for gate/up, 147 against 166 MB with 4 against 8 for down)
     if (L->group_m == 0) g2.group_m = 4;
-    HIP_TRY(ctx, run(g2, false));
+    HIP_TRY(ctx, run(shared_inside ? with_shared(g2, s2) : g2, false));
     L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return run_on(g2, st); };
     HIP_TRY(ctx, mark(5));
 
-    if (c.shared_expert && T > 0 && !shared_forked) HIP_TRY(ctx, shared_expert(s));
+    if (c.shared_expert && T > 0 && !shared_forked && !shared_inside) HIP_TRY(ctx, shared_expert(s));
     if (shared_forked) {
         HIP_TRY(ctx, hipStreamWaitEvent(s, ctx->ev_join, 0));
         join_guard.armed = false;

@@ -174,6 +174,16 @@ struct GroupedArgs {
     // gradients of the pre-activations go to `gu_out` [rows, 2N] and `out` is not written.
     const void* swiglu_grad_gu = nullptr;
     bool swiglu;
+    // bf16 matrix-core launches: a second, dense group in the same launch (the shared expert); rows 0: none.  Its weights
+    // are of the same kind; pre-activations are kept (`gu_out`) for both groups or for neither.
+    struct Dense {
+        const void* a = nullptr;  // [rows, K]
+        const void* w = nullptr;
+        const float* scales = nullptr;
+        int N = 0, K = 0, rows = 0;
+        void* out = nullptr;      // [rows, N]
+        void* gu_out = nullptr;   // [rows, 2N]
+    } dense2;
     int group_m;            // MFMA path: M-tiles per scheduling group (0 = default)
     int tile_m = 0;         // f32 matrix-core path: rows per tile of the tile table (64 or 32)
 };

@@ -393,7 +393,7 @@ Plan make_plan(rbmoe_layer* L) {
     p.add(&L->rank_in_block, S * 4);
     p.add(&L->blockcnt, nb * E * 4);
     p.add(&L->partial, nb * (E + 1) * 4);
-    p.add(&L->blockbase, nb * E * 4);
+    p.add(&L->blockbase, (nb * E + E + 1) * 4);
     p.add(&L->counts, E * 4);
     p.add(&L->offsets, (E + 1) * 4);
     p.add(&L->tile_expert, (size_t)L->max_tiles * 4);

@@ -116,7 +116,7 @@ struct DispatchArgs {
     int* tile_rows;
     int* ntiles;           // [1]
     float* losses;         // [2]
-    int* blockbase;        // [nb, E]  scratch: slots of expert e routed by the blocks before block b
+    int* blockbase;        // [nb, E]  scratch: slots of expert e routed by the blocks before block b; then E + 1 sums
     int* perm_slot;
     int* perm_token;
     int* inv_pos;

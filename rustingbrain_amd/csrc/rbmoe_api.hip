@@ -937,6 +937,27 @@ bool decode_front_pays(const rbmoe_layer* L, int T) {
     return untouched * 3.0 * L->Fw * c.d_model * dtype_size(c.weight_dtype) <= 24e6;
 }
 
+// Whether a few tokens' call is better off on the decode-shaped kernels than on the large-batch sequence, whose routing
+// takes a workgroup per eight tokens and whose launches a few microseconds each.  us, decode against large-batch:
+//   routing beside the products: its down launch sums slots one after the other.  Over 64 slots and 20 M weights a
+//     matrix: d 1024, 16 experts of 1408, four a row: 16 rows 38.7 / 47.5, 20 rows 52.0 / 47.5, 32 rows 63.0 / 47.8; 32
+//     experts of 704: 16 rows 42.3 / 51.3, 20 rows 57.2 / 52.6; 64 experts of 704, six a row, 32 rows 125.8 / 94.6.  Fewer
+//     weights, later: 32 rows, four a row, 16 experts, d 768 (17 M) 50.8 / 43.0, 8 experts, d 1024 (12 M) 44.4 / 41.2.
+//   routing alone in one workgroup, in front: its time grows with tokens x experts x width, steeply where the rows do not
+//     fit its LDS.  Staged: 32 experts, d 512, 8 rows (131 K) 30.0 / 40.0, 16 rows (262 K) 47.2 / 40.9; 16 experts, d 768, 8
+//     rows (98 K) 39.2 / 44.2, 12 rows (147 K) 44.8 / 43.3.  Not staged: 32 experts, d 768, 4 rows (98 K) 41.5 / 41.5, 8 rows
+//     (197 K) 79.5 / 48.5; 64 experts, d 1024, 1 row (66 K) 56.4 / 64.3, 2 rows 73.2 / 66.4, 16 rows 303 / 83.5.
+bool decode_front_beats_batch(const rbmoe_layer* L, int T) {
+    const rbmoe_config& c = L->cfg;
+    const int slots = T * c.experts_per_token;
+    const double weights = (double)c.num_experts * L->Fw * c.d_model;
+    return !(slots > 64 && weights > 20e6) && !(slots > 112 && weights > 11e6);
+}
+bool decode_alone_beats_batch(const rbmoe_layer* L, int T, bool stages_rows) {
+    const long long work = (long long)T * L->cfg.num_experts * L->cfg.d_model;
+    return work <= (stages_rows ? 160000 : 110000);
+}
+
 // The buffers of a decode-shaped forward of T tokens carved out of `base` (pieces of 256 bytes); returns the
 // bytes used.  With base == nullptr only the size is computed.
 size_t carve_decode_work(const rbmoe_layer* L, int T, bool front, unsigned char* base, Work* w) {
@@ -1058,10 +1079,15 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // the routing beside the gate/up products, in one launch
     bool front = small && L->decode_front && L->hall.p != nullptr && decode_front_ok(ra, abf) &&
                  (!L->router_q8 || wk == WeightKind::I8) && decode_front_pays(L, T);
+    // (a caller without allocations, or one who switched the combined launch off, asked for these kernels by name)
+    const bool choose = !static_scratch && L->decode_front;
+    const bool batch = choose && small &&
+                       (front ? !decode_front_beats_batch(L, T) : !decode_alone_beats_batch(L, T, stages_rows));
+    if (batch) front = false;
     if (static_scratch && front && carve_decode_work(L, T, true, nullptr, nullptr) > (size_t)RBMOE_STATIC_SCRATCH_BYTES)
         front = false;
     // (without it a quantized router takes the large-batch sequence)
-    const bool decode_ok = small && (front || (!L->router_q8 && (!cast || stages_rows)));
+    const bool decode_ok = small && !batch && (front || (!L->router_q8 && (!cast || stages_rows)));
     const bool norm_in_route = norm_src && decode_ok && (front || stages_rows);
     Work wk_ = work_of_layer(L);
     if (static_scratch) {

@@ -852,29 +852,32 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
     }
 }
 
-// At most this many wide tiles take the narrow kernel.  Down: up to one a compute unit.  us, wide against narrow, at so
-// many tiles of d 768 (K 1408; * int8 weights): 57 (203 rows) 17.2 / 10.6, 72* 23.2 / 15.0, 93* 24.2 / 16.1, 216* 29.3 /
-// 27.0, 432 41.1 / 47.1; 80 of d 512 (K 384) 9.9 / 6.8.  Gate/up workgroups are twice as many per tile (64 features) and
-// their reductions short, so the line is lower: 120 tiles (K 512) 11.8 / 10.5, 209 (K 768) 15.0 / 16.5, 264* 18.3 / 19.6.
+// Up to how many wide tiles (as many as are likely, not the upper bound of the grid) the narrow kernel takes a launch.
+// Down products, bf16, reductions over 512: as long as the narrow workgroups are about one a compute unit.  us a step, wide
+// against narrow, d 768, K 1408: 48 tiles (203 rows over 16 experts) 17.2 / 10.6 (the launch alone), 117 tiles (2000 rows)
+// 65.1 / 59.0, 129 (2500 rows over 8) 68.6 / 63.3, 141 (2500 rows over 16) 76.4 / 77.2, 165 (3000 rows) 78.8 / 79.8, 186 (3500)
+// 90.7 / 95.1.  Short reductions (the default model's 384) are mostly first loads and stores: 156 tiles 47.5 / 46.2, 244
+// tiles 69.4 / 67.4, 392 the same.  int8 weights: 129 tiles 71.2 / 62.8, 174 tiles 83.4 / 80.8, 204 tiles 90.1 / 87.6, 246
+// tiles 104.6 / 105.5.
+// Gate/up workgroups are twice as many per tile (64 features): 81 tiles (K 512) 39.9 / 38.9, 88 (int8, K 768) 43.9 / 41.7, 156
+// 42.5 / 46.0, 176 (K 768, the launch alone) 15.0 / 16.5.
 // Launches that keep or read pre-activations (training) stay with the wide kernel's epilogue.
-constexpr int kNarrowDownTiles = 256;
-constexpr int kNarrowGateUpTiles = 128;
+constexpr int narrow_tiles(bool swiglu, bool i8, int K) { return swiglu ? 128 : i8 ? 210 : K <= 512 ? 250 : 140; }
 
 template <bool SWIGLU, bool I8>
 hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
     constexpr int BN = SWIGLU ? NW * 32 : NW * 64;
     const int tiles_m = g.dense_rows >= 0 ? (g.dense_rows + BM - 1) / BM : g.max_tiles;
     const GroupedArgs::Dense& d2 = g.dense2;
-    auto tiles = [&](int bn) {
-        return tiles_m * ((g.N + bn - 1) / bn) + (d2.rows + BM - 1) / BM * ((d2.N + bn - 1) / bn);
-    };
-    const int total = tiles(BN);
+    auto tiles = [&](int m, int bn) { return m * ((g.N + bn - 1) / bn) + (d2.rows + BM - 1) / BM * ((d2.N + bn - 1) / bn); };
+    const int total = tiles(tiles_m, BN);
     if (total <= 0) return hipSuccess;
     const DenseGroup g2{static_cast<const bf16_t*>(d2.a), d2.w, d2.scales, d2.N, d2.K, d2.rows,
                         static_cast<bf16_t*>(d2.out), static_cast<bf16_t*>(d2.gu_out)};
     const int group_m = g.group_m > 0 ? g.group_m : 8;
-    if (total <= (SWIGLU ? kNarrowGateUpTiles : kNarrowDownTiles) && !g.gu_out && !g.swiglu_grad_gu) {
-        RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((tiles(BN / 2) + 7) / 8 * 8), dim3(NT), 0, s,
+    const int likely = g.dense_rows < 0 && g.likely_tiles > 0 ? tiles(g.likely_tiles, BN) : total;
+    if (likely <= narrow_tiles(SWIGLU, I8, g.K) && !g.gu_out && !g.swiglu_grad_gu) {
+        RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((tiles(tiles_m, BN / 2) + 7) / 8 * 8), dim3(NT), 0, s,
                   static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
                   g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
                   static_cast<bf16_t*>(g.out), group_m, g2);

@@ -1377,6 +1377,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     g1.tile_rows = (const int*)L->tile_rows.p;
     g1.ntiles = (const int*)L->ntiles.p;
     g1.max_tiles = T > 0 ? (T * k) / tile_m0 + E : 0;
+    g1.likely_tiles = std::max((T * k) / tile_m0 + E / 2, std::min(E, T * k));  // a last tile half full, or one tile each
     g1.tile_m = tile_m0;
     g1.dense_rows = -1;
     g1.out = L->h.p;

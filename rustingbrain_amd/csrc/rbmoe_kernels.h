@@ -166,6 +166,7 @@ struct GroupedArgs {
     const int* tile_rows;
     const int* ntiles;
     int max_tiles;
+    int likely_tiles = 0;   // what *ntiles will be about, for the choice of a kernel (0: max_tiles)
     int dense_rows;         // >= 0: one group of this many rows, no tile table (shared expert)
     void* out;              // [rows, N] activation dtype
     void* gu_out = nullptr; // gate/up launches: [rows, 2N] pre-activations (gate | up) kept for a backward pass

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [dict(d=64, E=4, k=1, F=64, T=33), dict(d=128, E=3, k=2, F=192, T=129), dict(d=320, E=5, k=2, F=448, T=97),
           dict(d=192, E=8, k=4, F=256, T=257), dict(d=384, E=2, k=1, F=384, T=223),
-          # 128 experts: over 128 gate/up and 256 down tiles, so the wide kernel, with the same odd shapes
+          # 128 experts: over 128 gate/up and 250 down tiles, so the wide kernel, with the same odd shapes
           dict(d=320, E=128, k=2, F=192, T=260)]
 
 

@@ -1113,15 +1113,11 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     }
     // the rows the expert products read
     const void* const xe = cast ? wk_.x16 : x;
-    const RouterPlan rplan = plan_router(ra, abf);
-    if (!rplan.takes_norm) {  // the norm runs by itself
-        ra.x = x;
-        ra.norm_w = nullptr;
-        ra.xn_out = nullptr;
-    }
+    bool norm_apart = false;  // the norm runs by itself
+    const RouterPlan rplan = plan_router_behind_norm(ra, x, abf, &norm_apart);
     const bool cast_apart = cast && L->router_q8 && !rplan.q8_writes_rows16;
     if (cast_apart) ra.rows16 = nullptr;
-    if (norm_src && !norm_in_route && (decode_ok || !rplan.takes_norm))
+    if (decode_ok ? norm_src && !norm_in_route : norm_apart)
         HIP_TRY(ctx, launch_rmsnorm(norm_src, (const float*)L->norm_w.p, L->norm_eps, T, d, L->xn.p, abf, s));
 
     // ---- a few tokens: route in one workgroup, then stream the touched weights once -------
@@ -1325,7 +1321,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
 
     if (cast_apart)
         HIP_TRY(ctx, launch_cast_rows_bf16((const float*)x, L->x16.p, (long long)T * d, s));
-    HIP_TRY(ctx, launch_router(ra, abf, s));
+    HIP_TRY(ctx, launch_router(ra, rplan, abf, s));
     if (!shared_first)
         if (const int rc = fork_shared()) return rc;
     RouterArgs again = ra;  // (the rows are normed by now; in an in-place block step the raw ones are gone)
@@ -1334,7 +1330,10 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         again.norm_w = nullptr;
         again.xn_out = nullptr;
     }
-    L->replay[RBMOE_STAGE_ROUTER] = [=](hipStream_t st) { return launch_router(again, abf, st); };
+    // (the same tokens a block with the norm and without: a norm that costs tokens is not taken along)
+    const RouterPlan again_plan = plan_router(again, abf);
+    if (again_plan.block_tokens == rplan.block_tokens)
+        L->replay[RBMOE_STAGE_ROUTER] = [=](hipStream_t st) { return launch_router(again, again_plan, abf, st); };
     HIP_TRY(ctx, mark(1));
 
     HIP_TRY(ctx, mark(2));  // an interval with no work in it: the cost of one pair of event records
@@ -2470,6 +2469,41 @@ int rbmoe_internal_weight_grad_slots(int32_t M, int32_t N, int32_t groups, int32
     const int rows = dense ? tokens : tokens * rows_per_token;
     *needed = (int64_t)(weight_grad_partial_bytes(M, N, groups, dense ? rows : -1, rows, bf16 != 0) / one);
     *held = (int64_t)(weight_grad_partial_bytes_upto(M, N, groups, dense != 0, max_tokens, rows_per_token, bf16 != 0) / one);
+    return RBMOE_OK;
+}
+
+// Test hook (not part of rbmoe.h), runs without a GPU: how a large-batch call on rows at address `x` (never read) is routed.
+// out[0]: tokens of a router block as the dispatch counts them, [1]: whether the norm takes a launch of its own, [2]: whether
+// the router's launch takes the plan with the arguments it gets, [3]: tokens of a block when the stage is replayed.
+int rbmoe_internal_router_plan(int32_t d, int32_t E, int32_t k, int32_t T, int32_t bf16, int32_t norm, int32_t quantized,
+                               int32_t fused, uint64_t x, int32_t* out) {
+    if (!out) return RBMOE_NULL_POINTER;
+    auto at = [](uint64_t address) { return reinterpret_cast<void*>((uintptr_t)address); };
+    void* const own = at(1 << 20);  // the layer's own buffers: on an allocation's boundary
+    RouterArgs a{};
+    a.x = at(x);
+    a.wr = static_cast<const float*>(own);
+    a.T = T; a.d = d; a.E = E; a.k = k;
+    a.allow_fused = fused != 0;
+    if (quantized) {
+        a.wq = static_cast<const int8_t*>(own);
+        a.wscale = static_cast<const float*>(own);
+    }
+    if (norm) {
+        a.norm_w = static_cast<const float*>(own);
+        a.xn_out = own;
+    }
+    bool apart = false;
+    const RouterPlan p = plan_router_behind_norm(a, own, bf16 != 0, &apart);
+    out[0] = p.block_tokens;
+    out[1] = apart ? 1 : 0;
+    out[2] = router_takes(a, p, bf16 != 0) ? 1 : 0;
+    if (a.norm_w) {
+        a.x = own;
+        a.norm_w = nullptr;
+        a.xn_out = nullptr;
+    }
+    out[3] = plan_router(a, bf16 != 0).block_tokens;
     return RBMOE_OK;
 }
 

@@ -90,14 +90,27 @@ struct RouterArgs {
     void* xn_out = nullptr;
 };
 // How a call is routed: tokens of a router block (what launch_dispatch needs to know), whether the launch applies the
-// norm that `a` asks for, and whether it writes the bf16 copy of f32 rows for a quantized router too.
+// norm that `a` asks for, and whether it writes the bf16 copy of f32 rows for a quantized router too.  Made once per call,
+// from the pointers that the launch will get: which kernel takes a call depends on their alignment, and the kernels'
+// blocks differ in tokens.
 struct RouterPlan {
-    int block_tokens;
-    bool takes_norm;
-    bool q8_writes_rows16;
+    int block_tokens = 0;
+    bool takes_norm = false;
+    bool q8_writes_rows16 = false;
+    // route_rows_kernel: experts whose router rows lie in LDS together (0: another kernel), LDS bytes
+    int row_experts = 0;
+    size_t row_lds = 0;
+    bool operator==(const RouterPlan& o) const {
+        return block_tokens == o.block_tokens && takes_norm == o.takes_norm && q8_writes_rows16 == o.q8_writes_rows16 &&
+               row_experts == o.row_experts && row_lds == o.row_lds;
+    }
 };
 RouterPlan plan_router(const RouterArgs& a, bool bf16);
-hipError_t launch_router(const RouterArgs& a, bool bf16, hipStream_t s);
+// The plan of a call behind a norm (a.x: the raw rows): where no launch takes the norm along, `a` is turned to the normed
+// rows, which the caller then makes first (`norm_apart`), and the plan is theirs.
+RouterPlan plan_router_behind_norm(RouterArgs& a, const void* normed, bool bf16, bool* norm_apart);
+bool router_takes(const RouterArgs& a, const RouterPlan& p, bool bf16);  // whether `p` is the plan of these arguments
+hipError_t launch_router(const RouterArgs& a, const RouterPlan& p, bool bf16, hipStream_t s);  // refuses any other plan
 
 struct DispatchArgs {
     const void* x;

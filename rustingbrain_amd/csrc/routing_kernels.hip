@@ -1233,23 +1233,36 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
 
 RouterPlan plan_router(const RouterArgs& a, bool bf16) {
     const RowsPlan p = plan_rows(a, bf16 ? 2 : 4);
-    if (a.norm_w && (!p.tokens || (a.T + p.tokens - 1) / p.tokens > 256)) {
-        // the squares' room costs tokens a workgroup, and a second round of workgroups costs more than the norm in a
-        // launch of its own (8192 tokens, d 768: 37.7 us in two rounds, 16.2 + 8 in two launches)
-        RouterArgs b = a;
-        b.norm_w = nullptr;
-        RouterPlan q = plan_router(b, bf16);
-        q.takes_norm = false;
-        return q;
-    }
-    return p.tokens ? RouterPlan{p.tokens, true, true} : RouterPlan{kRouterTokens, false, false};
+    RouterPlan q;
+    q.block_tokens = p.tokens ? p.tokens : kRouterTokens;
+    q.row_experts = p.tokens ? p.EG : 0;
+    q.row_lds = p.tokens ? p.lds : 0;
+    // the squares' room costs tokens a workgroup, and a second round of workgroups costs more than the norm in a
+    // launch of its own (8192 tokens, d 768: 37.7 us in two rounds, 16.2 + 8 in two launches)
+    q.takes_norm = a.norm_w && p.tokens && (a.T + p.tokens - 1) / p.tokens <= 256;
+    q.q8_writes_rows16 = p.tokens != 0;
+    return q;
+}
+
+RouterPlan plan_router_behind_norm(RouterArgs& a, const void* normed, bool bf16, bool* norm_apart) {
+    const RouterPlan p = plan_router(a, bf16);
+    *norm_apart = a.norm_w && !p.takes_norm;
+    if (!*norm_apart) return p;
+    a.x = normed;
+    a.norm_w = nullptr;
+    a.xn_out = nullptr;
+    return plan_router(a, bf16);
+}
+
+bool router_takes(const RouterArgs& a, const RouterPlan& p, bool bf16) {
+    return p == plan_router(a, bf16) && (!a.norm_w || p.takes_norm);
 }
 
 template <typename XT>
-static hipError_t launch_rows_t(const RouterArgs& a, const RowsPlan& p, hipStream_t s) {
-    RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, p.EG, a.P, a.lse, a.expert_of, a.gate_of,
+static hipError_t launch_rows_t(const RouterArgs& a, const RouterPlan& p, hipStream_t s) {
+    RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, p.row_experts, a.P, a.lse, a.expert_of, a.gate_of,
                     a.rank_in_block, a.blockcnt, a.partial, static_cast<bf16_t*>(a.rows16), a.norm_w, a.norm_eps, a.xn_out};
-    const dim3 grid((a.T + p.tokens - 1) / p.tokens);
+    const dim3 grid((a.T + p.block_tokens - 1) / p.block_tokens);
     auto go = [&](auto kernel) -> hipError_t {
         static std::atomic<unsigned long long> attr_set{0};  // one per kernel: the lambda's body is instantiated for each
         const hipError_t e = once_per_device(attr_set, [&] {
@@ -1257,7 +1270,7 @@ static hipError_t launch_rows_t(const RouterArgs& a, const RowsPlan& p, hipStrea
                                        kMaxRouterLds);
         });
         if (e != hipSuccess) return e;
-        RB_LAUNCH(kernel.value, grid, dim3(kRouterThreads), p.lds, s, r);
+        RB_LAUNCH(kernel.value, grid, dim3(kRouterThreads), p.row_lds, s, r);
         return hipGetLastError();
     };
 #define RB_ROUTE_ROWS(TB, NL, TT, EE) \
@@ -1265,20 +1278,19 @@ static hipError_t launch_rows_t(const RouterArgs& a, const RowsPlan& p, hipStrea
     // tokens x experts a thread: the largest tile that still has work for every thread (more sums a thread mean less
     // traffic with LDS; the sums of 8 tokens x 16 experts take 2.3 us with 1 x 2 on eight waves, 2.9 with 2 x 2 on four)
     if (a.wq) {
-        if (p.tokens == 8) return RB_ROUTE_ROWS(8, 32, 2, 2);
-        if (p.tokens == 16) return RB_ROUTE_ROWS(16, 32, 4, 2);
+        if (p.block_tokens == 8) return RB_ROUTE_ROWS(8, 32, 2, 2);
+        if (p.block_tokens == 16) return RB_ROUTE_ROWS(16, 32, 4, 2);
         return RB_ROUTE_ROWS(32, 32, 4, 2);
     }
-    if (p.tokens == 8) return RB_ROUTE_ROWS(8, 8, 1, 2);
-    if (p.tokens == 16) return a.E <= 8 ? RB_ROUTE_ROWS(16, 8, 1, 2) : RB_ROUTE_ROWS(16, 8, 2, 2);
+    if (p.block_tokens == 8) return RB_ROUTE_ROWS(8, 8, 1, 2);
+    if (p.block_tokens == 16) return a.E <= 8 ? RB_ROUTE_ROWS(16, 8, 1, 2) : RB_ROUTE_ROWS(16, 8, 2, 2);
     return a.E <= 8 ? RB_ROUTE_ROWS(32, 8, 2, 2) : RB_ROUTE_ROWS(32, 8, 4, 2);
 #undef RB_ROUTE_ROWS
 }
 
 template <typename XT>
-static hipError_t launch_router_t(const RouterArgs& a, hipStream_t s) {
-    if (const RowsPlan p = plan_rows(a, sizeof(XT)); p.tokens) return launch_rows_t<XT>(a, p, s);
-    if (a.norm_w) return hipErrorInvalidValue;  // (the plan said so)
+static hipError_t launch_router_t(const RouterArgs& a, const RouterPlan& p, hipStream_t s) {
+    if (p.row_experts) return launch_rows_t<XT>(a, p, s);
     const int nb = (a.T + kRouterTokens - 1) / kRouterTokens;
     if (const int cols = a.wq ? 0 : fused_cols(a, sizeof(XT))) {
         // bf16 rows staged as f32 where a slice of the same width then still fits
@@ -1344,10 +1356,11 @@ static hipError_t launch_router_t(const RouterArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_router(const RouterArgs& a, bool bf16, hipStream_t s) {
+hipError_t launch_router(const RouterArgs& a, const RouterPlan& p, bool bf16, hipStream_t s) {
     if (a.T <= 0) return hipSuccess;
+    if (!router_takes(a, p, bf16)) return hipErrorInvalidValue;  // (its blocks would not be those the dispatch counts)
     if (a.rows16 && (bf16 || a.d % 8 != 0)) return hipErrorInvalidValue;  // the copy rides on the 8-element pieces
-    return bf16 ? launch_router_t<bf16_t>(a, s) : launch_router_t<float>(a, s);
+    return bf16 ? launch_router_t<bf16_t>(a, p, s) : launch_router_t<float>(a, p, s);
 }
 
 template <typename XT>

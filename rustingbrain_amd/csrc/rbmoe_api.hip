@@ -1113,7 +1113,8 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     }
     // the rows the expert products read
     const void* const xe = cast ? wk_.x16 : x;
-    bool norm_apart = false;  // the norm runs by itself
+    const RouterArgs front_args = ra;  // (the routing beside the products has its own way with the norm)
+    bool norm_apart = false;           // the norm runs by itself
     const RouterPlan rplan = plan_router_behind_norm(ra, x, abf, &norm_apart);
     const bool cast_apart = cast && L->router_q8 && !rplan.q8_writes_rows16;
     if (cast_apart) ra.rows16 = nullptr;
@@ -1167,7 +1168,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
                              wk_.counts, wk_.offsets, wk_.tile_expert, wk_.tile_row0, wk_.tile_rows, wk_.ntiles, wk_.losses,
                              wk_.perm_slot, wk_.perm_token, wk_.inv_pos};
         if (front) {
-            RouterArgs fr = ra;  // (the products read the same rows: raw ones in front of a norm, f32 ones as they are)
+            RouterArgs fr = front_args;  // (the products read the same rows: raw ones in front of a norm, f32 ones as they are)
             fr.P = wk_.P; fr.lse = wk_.lse; fr.expert_of = wk_.expert_of; fr.gate_of = wk_.gate_of;
             d1.a = fr.x;
             if (c.shared_expert) d1.a_shared = fr.x;

@@ -1,5 +1,7 @@
 """The routing beside the gate/up products (at most 32 tokens): every combination of row type, weights, router and norm
 that the launch has a variant for, several routing workgroups, a k past the combine's first slots, ragged teams."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -7,6 +9,7 @@ from conftest import rel_l2
 from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
 from oracle import rb_oracle as orc
 from rustingbrain_amd import Layout, synth
+from rustingbrain_amd import _lib as L
 
 pytestmark = pytest.mark.gpu
 
@@ -49,4 +52,19 @@ def test_matches_the_oracle(device, shape, act, wt, q8, norm):
     h, y = layer.expert_rows(int(ref.offsets[-1]))
     assert rel_l2(h, ref.hidden) <= 2e-2 and rel_l2(y, ref.expert_out) <= 2e-2
     assert abs(cache.aux_loss() - ref.aux_loss) <= 1e-6 + 1e-5 * abs(ref.aux_loss)
+    layer.close()
+
+
+@pytest.mark.parametrize("act,wt", [("bf16", "bf16"), ("f32", "int8")])
+def test_block_step_with_the_fused_router_switched_off(device, act, wt):
+    """RBMOE_OPT_FUSED_ROUTER 0 speaks of the large-batch routing: a decode step still norms its rows on the way."""
+    t = synth.make(small_workload(d=64, E=6, k=2, F=64, T=9, seed=71, act=act, wt=wt))
+    layer = gpu_layer(device, t)
+    layer.set_feed_forward_norm((1.0 + 0.1 * synth.normal((64,), 1.0, 71, 97)).astype(np.float32), 1e-6)
+    out, cache = layer.forward_block(t.x)
+    layer.forward_block(t.x[::-1].copy())   # (what the layer's buffers hold afterwards is another call's)
+    layer.set_option(L.OPT_FUSED_ROUTER, 0)
+    again, cache_again = layer.forward_block(t.x)
+    assert_routing_identical(cache_again, SimpleNamespace(**{**vars(cache), "lse": cache.log_sum_exp}))
+    assert np.array_equal(again, out)
     layer.close()

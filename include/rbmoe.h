@@ -182,6 +182,7 @@ int rbmoe_set_weight(rbmoe_layer* layer, int32_t which, int32_t expert, const vo
  *   residual [T, d] act_dtype added to the result (the block's residual add,
  *            src/transformer_block.rs:221-222), or NULL
  *   out      [T, d] act_dtype
+ * Rows may start at any element; off a 16-byte boundary the matrix-core kernels work on a copy of them.
  * Auxiliary losses and routing tables stay on the device until fetched. */
 int rbmoe_forward(rbmoe_layer* layer, const void* x, int32_t T, int32_t cols, const uint8_t* valid,
                   const float* router_bias, const void* residual, void* out);

@@ -992,6 +992,10 @@ size_t carve_decode_work(const rbmoe_layer* L, int T, bool front, unsigned char*
     return used;
 }
 
+// The matrix-core products fetch their rows by LDS-DMA in 16-byte pieces (every row is a whole number of them).  A caller's
+// rows that start off such a boundary are copied to the layer's own memory first.
+bool starts_on_piece(const void* rows) { return reinterpret_cast<uintptr_t>(rows) % 16 == 0; }
+
 // `norm_src` (block step): the raw rows; `x` is then the layer's buffer of normed rows, filled here - by the
 // small-route kernel itself for a few tokens, by the norm kernel otherwise - before anything reads it.
 // `static_scratch` (rbmoe_forward_static): this device's copy of the static scratch array; the call must then be
@@ -1112,7 +1116,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         carve_decode_work(L, T, front, static_cast<unsigned char*>(static_scratch), &wk_);
     }
     // the rows the expert products read
-    const void* const xe = cast ? wk_.x16 : x;
+    const void* xe = cast ? wk_.x16 : x;
     const RouterArgs front_args = ra;  // (the routing beside the products has its own way with the norm)
     bool norm_apart = false;           // the norm runs by itself
     const RouterPlan rplan = plan_router_behind_norm(ra, x, abf, &norm_apart);
@@ -1243,6 +1247,12 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     L->x_saved = norm_src ? L->xn.p : L->xc.p;
     if (L->training && T > 0 && !norm_src)
         HIP_TRY(ctx, hipMemcpyAsync(L->xc.p, x, (size_t)T * d * dtype_size(c.act_dtype), hipMemcpyDeviceToDevice, s));
+
+    if ((mfma || f32mc) && !cast && T > 0 && !starts_on_piece(x)) {
+        if (!L->training)
+            HIP_TRY(ctx, hipMemcpyAsync(L->st_x.p, x, (size_t)T * d * dtype_size(c.act_dtype), hipMemcpyDeviceToDevice, s));
+        xe = L->training ? L->xc.p : L->st_x.p;
+    }
 
     for (auto& r : L->replay) r = nullptr;
     auto run_on = [=](const GroupedArgs& g, hipStream_t st) -> hipError_t {
@@ -2091,6 +2101,11 @@ int rbmoe_backward(rbmoe_layer* L, const void* grad_output, int32_t tokens, int3
     if (cast) {
         HIP_TRY(ctx, launch_cast_rows_bf16((const float*)grad_output, L->g16.p, (long long)T * d, s));
         gout = L->g16.p;
+    }
+
+    if (!cast && c.shared_expert && (L->use_stream || L->use_f32_mc) && !starts_on_piece(grad_output)) {
+        HIP_TRY(ctx, hipMemcpyAsync(L->st_gout.p, grad_output, (size_t)T * d * dtype_size(c.act_dtype), hipMemcpyDeviceToDevice, s));
+        gout = L->st_gout.p;
     }
 
     // upstream of every expert: gate * dOut[token]; gate gradient: dOut[token] . Y[row]

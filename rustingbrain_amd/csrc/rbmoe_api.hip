@@ -351,8 +351,11 @@ void choose_kernel_sets(rbmoe_layer* L) {
         if (rows * widest * 2 >= ((size_t)1 << 32)) L->use_stream = false;
     }
     if (cfg->act_dtype == RBMOE_F32 && L->use_stream) {
-        // the bf16 copy is written in 8-element pieces of 16-byte aligned rows
-        if (cfg->d_model % 8 == 0) L->cast_rows = true;
+        // the bf16 copy is written in 8-element pieces of 16-byte aligned rows.  Rounding a width would also round the
+        // rows: the any-shape kernels that such a layer has otherwise keep input, hidden and expert rows in f32 (1e-5
+        // against 3e-3), and the caller asked for f32 rows.
+        const bool whole = L->Fw == cfg->d_ff && (!cfg->shared_expert || L->Fsw == L->Fs);
+        if (cfg->d_model % 8 == 0 && whole) L->cast_rows = true;
         else L->use_stream = false;
     }
     if (!L->use_stream && !L->use_f32_mc) {  // the any-shape kernels take the widths as they are

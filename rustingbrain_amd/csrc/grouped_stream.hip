@@ -188,7 +188,6 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
     const float* const sc = o.sc;
     bf16_t* const out = o.out;
     bf16_t* const gu_out = o.gu_out;
-    const bf16_t* const bw_gu = o.bw_gu;
     // Accumulator element v of block (b, t): feature 8*(v/4) + 4*(lane/32) + v%4 of the
     // wave's row block b, token t*32 + lane%32 - a lane holds 4 consecutive features of a
     // token, so a direct store would scatter 8-byte pieces over 32 rows per instruction.
@@ -252,41 +251,6 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
             const int r = idx / PW, p = idx % PW;
             if (r < rows && col0 + 8 * p < N) {
                 const uint4 v = *reinterpret_cast<const uint4*>(stage + r * 256 + ((p ^ (r & 15)) * 16));
-                if constexpr (!SWIGLU) {
-                    if (bw_gu != nullptr) {  // uniform over the launch
-                        // SwiGlu::backward (src/ffn.rs:87-120) on the way out: the product rows are the
-                        // gradient of the hidden rows; with the gate and up pre-activations G | U of
-                        // the forward pass, dG = dH * U * silu'(G) and dU = dH * silu(G) go to `gu_out`
-                        // (both [rows, 2 N]) and the hidden gradient itself is never stored.
-                        const size_t off = (size_t)(row0 + r) * 2 * N + col0 + 8 * p;
-                        // (read once: fetched past the caches)
-                        typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-                        const u32x4_t g8 = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(bw_gu + off));
-                        const u32x4_t u8 = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(bw_gu + off + N));
-                        const uint32_t hw[4] = {v.x, v.y, v.z, v.w}, gw[4] = {g8.x, g8.y, g8.z, g8.w},
-                                       uw[4] = {u8.x, u8.y, u8.z, u8.w};
-                        uint32_t dg[4], du[4];
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            float dgv[2], duv[2];
-#pragma unroll
-                            for (int h = 0; h < 2; ++h) {
-                                const float dh = __uint_as_float(h ? hw[q] & 0xffff0000u : hw[q] << 16);
-                                const float gv = __uint_as_float(h ? gw[q] & 0xffff0000u : gw[q] << 16);
-                                const float uv = __uint_as_float(h ? uw[q] & 0xffff0000u : uw[q] << 16);
-                                const float sg = __builtin_amdgcn_rcpf(
-                                    1.0f + __builtin_amdgcn_exp2f(gv * -1.44269504088896340736f));
-                                dgv[h] = dh * uv * (sg * (1.0f + gv * (1.0f - sg)));  // silu', src/ffn.rs:235-238
-                                duv[h] = dh * (gv * sg);
-                            }
-                            dg[q] = pack2(dgv[0], dgv[1]);
-                            du[q] = pack2(duv[0], duv[1]);
-                        }
-                        *reinterpret_cast<uint4*>(gu_out + off) = make_uint4(dg[0], dg[1], dg[2], dg[3]);
-                        *reinterpret_cast<uint4*>(gu_out + off + N) = make_uint4(du[0], du[1], du[2], du[3]);
-                        continue;
-                    }
-                }
                 uint4* const where = reinterpret_cast<uint4*>(dst + (size_t)(row0 + r) * dstride + col0 + 8 * p);
                 if (SWIGLU && b > 0) {
                     // the pre-activations are not read again before the backward pass: stored past the caches,
@@ -297,6 +261,85 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
                     *where = v;
                 }
             }
+        }
+    }
+}
+
+// The same for a launch whose product rows are the gradient of the hidden rows, SwiGlu::backward (src/ffn.rs:87-120)
+// on the way out: with the gate and up pre-activations G | U of the forward pass, dG = dH * U * silu'(G) and
+// dU = dH * silu(G) go to `gu_out` (both [rows, 2 N]) and the hidden gradient itself is never stored.  It passes through
+// LDS in f32, 64 features at a time: rounded to bf16 first, as the tiles above are, it would cost the weight
+// gradients a rounding more than the any-shape kernels' have (3.12e-3 from 64 bits against 2.81e-3).  A pass's
+// pre-activations are requested in front of its barriers: 8192 tokens, d 768, 16 experts top-2 of 1408 take 80 us,
+// 90 with the rounded tile and the requests behind them.
+__device__ __forceinline__ void write_swiglu_backward(const TileOut& o, floatx16 (&acc)[2][TT], char* const stage) {
+    constexpr int BN = NW * 64;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lrow = lane & 31, lhalf = lane >> 5;
+    const int rows = o.rows, row0 = o.row0, N = o.N;
+    constexpr int TURNS = BM * 8 / NT;
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int bh = 0; bh < NW; ++bh) {
+        const int b = bh / (NW / 2), h = bh % (NW / 2);  // block index, pair of waves
+        const int col0 = o.tn_idx * BN + b * (NW * 32) + h * 64;
+        // this thread's pre-activations of the pass are under way while the tile is staged (read once: past the caches)
+        u32x4_t g8[TURNS], u8[TURNS];
+        auto offset_of = [&](int i, bool& in) {
+            const int r = (i * NT + tid) / 8, p = tid % 8;  // 8 features of a row
+            in = r < rows && col0 + 8 * p < N;
+            return (size_t)(row0 + (in ? r : 0)) * 2 * N + (in ? col0 + 8 * p : 0);
+        };
+#pragma unroll
+        for (int i = 0; i < TURNS; ++i) {
+            bool in;
+            const size_t off = offset_of(i, in);
+            g8[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(o.bw_gu + off));
+            u8[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(o.bw_gu + off + N));
+        }
+        if (bh) __syncthreads();  // the previous pass has been read out
+        if (wave / 2 == h && (b ? o.act1 : o.act0)) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                if (t * 32 >= rows) continue;
+                const int m = t * 32 + lrow;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<float4*>(stage + m * 256 + (((wave & 1) * 8 + 2 * q + lhalf) ^ (m & 15)) * 16) =
+                        make_float4(acc[b][t][4 * q], acc[b][t][4 * q + 1], acc[b][t][4 * q + 2], acc[b][t][4 * q + 3]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TURNS; ++i) {
+            bool in;
+            const size_t off = offset_of(i, in);
+            if (!in) continue;
+            const int r = (i * NT + tid) / 8, p = tid % 8;
+            const float4 lo = *reinterpret_cast<const float4*>(stage + r * 256 + ((2 * p) ^ (r & 15)) * 16);
+            const float4 hi = *reinterpret_cast<const float4*>(stage + r * 256 + ((2 * p + 1) ^ (r & 15)) * 16);
+            const float dh[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            const uint32_t gw[4] = {g8[i].x, g8[i].y, g8[i].z, g8[i].w}, uw[4] = {u8[i].x, u8[i].y, u8[i].z, u8[i].w};
+            uint32_t dg[4], du[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float dgv[2], duv[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const float gv = __uint_as_float(e ? gw[q] & 0xffff0000u : gw[q] << 16);
+                    const float uv = __uint_as_float(e ? uw[q] & 0xffff0000u : uw[q] << 16);
+                    const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gv * -1.44269504088896340736f));
+                    dgv[e] = dh[2 * q + e] * uv * (sg * (1.0f + gv * (1.0f - sg)));  // silu', src/ffn.rs:235-238
+                    duv[e] = dh[2 * q + e] * (gv * sg);
+                }
+                dg[q] = pack2(dgv[0], dgv[1]);
+                du[q] = pack2(duv[0], duv[1]);
+            }
+            *reinterpret_cast<uint4*>(o.gu_out + off) = make_uint4(dg[0], dg[1], dg[2], dg[3]);
+            *reinterpret_cast<uint4*>(o.gu_out + off + N) = make_uint4(du[0], du[1], du[2], du[3]);
         }
     }
 }
@@ -586,6 +629,13 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     __syncthreads();  // every wave's last DMA has landed and its last fragment reads are done
     const TileOut to{rows, row0, tn_idx, N, act0, act1, r0, r1, I8 ? scales + (size_t)expert * s_expert_stride : nullptr,
                      out, gu_out, bw_gu};
+    if constexpr (!SWIGLU && !I8) {
+        if (bw_gu != nullptr) {  // uniform over the launch
+            write_swiglu_backward(to, acc, reinterpret_cast<char*>(As));
+            RBMOE_TRACE_AT(blockIdx.x, 3);
+            return;
+        }
+    }
     write_tile<SWIGLU, I8>(to, acc, reinterpret_cast<char*>(As), [] {});
     RBMOE_TRACE_AT(blockIdx.x, 3);
 }
@@ -903,6 +953,7 @@ hipError_t launch_grouped_stream(const GroupedArgs& g, WeightKind wk, hipStream_
     if (!stream_shape_ok(g.N, g.K)) return hipErrorInvalidValue;
     if (g.dense2.rows > 0 && (!stream_shape_ok(g.dense2.N, g.dense2.K) || !g.dense2.gu_out != !g.gu_out || g.swiglu_grad_gu))
         return hipErrorInvalidValue;
+    if (g.swiglu_grad_gu && (g.swiglu || wk != WeightKind::BF16)) return hipErrorInvalidValue;
     if (wk == WeightKind::BF16) return g.swiglu ? launch_t<true, false>(g, s) : launch_t<false, false>(g, s);
     if (wk == WeightKind::I8) return g.swiglu ? launch_t<true, true>(g, s) : launch_t<false, true>(g, s);
     return hipErrorInvalidValue;

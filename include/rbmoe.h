@@ -130,7 +130,12 @@ const char* rbmoe_last_global_error(void);
 
 /* MoeLayer::new (src/moe.rs:215-231) + TransformerLm::to_cuda's upload of the
  * layer (src/transformer.rs:1263-1296): validates, checks the budget BEFORE
- * allocating (src/param.rs:172-189), allocates weights (zeroed) and workspace. */
+ * allocating (src/param.rs:172-189), allocates weights (zeroed) and workspace.
+ * Expert widths between two multiples of a matrix-core tile are stored rounded up (bf16 rows: to 64, at most four
+ * times the width; all-f32 layers: to 32, at most twice), which takes that much more memory.  A layer whose rounded
+ * widths are over the budget - here, or when the norm or training mode is added before the first weight - or over a limit
+ * of the backward products keeps its true widths and the any-shape kernels instead.  Layers that already hold
+ * weights stay as they are: a budget shared by several layers has to allow for their rounded widths. */
 int rbmoe_layer_create(rbmoe_ctx* ctx, const rbmoe_config* cfg, rbmoe_layer** out);
 void rbmoe_layer_destroy(rbmoe_layer* layer);
 

@@ -8,6 +8,7 @@
 // fallback: without a usable GPU every device entry point fails.
 #include "../../include/rbmoe.h"
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdio>
@@ -223,6 +224,10 @@ struct rbmoe_layer {
     // of the tile is rounded up and the extra gate and up rows and down columns are zero (their hidden values are
     // silu(0) * 0 = 0 and add nothing).  Equal to the true widths where nothing is rounded.
     int Fw = 0, Fsw = 0;
+    // Laid out as small as the kernels allow, because the memory budget, the memory or a limit of the rounded widths would
+    // refuse the layer otherwise: true widths, router blocks of one size, no room for the routing beside the products of
+    // a layer with many experts.
+    bool tight = false;
     int max_T = 0;
     int max_S = 0;
     int max_nb = 0;
@@ -318,7 +323,7 @@ struct Plan {
     }
 };
 
-// Which kernel sets the layer's shapes and dtypes allow (and `force_generic` does not rule out).
+// Which kernel sets the layer's shapes and dtypes allow (and `force_generic` and `tight` do not rule out).
 void choose_kernel_sets(rbmoe_layer* L) {
     const rbmoe_config* cfg = &L->cfg;
     L->use_stream = L->use_f32_mc = L->cast_rows = false;
@@ -326,9 +331,9 @@ void choose_kernel_sets(rbmoe_layer* L) {
     // for the packed bf16 / int8 kernels, 32 for the f32 ones.  The any-shape kernels run at a thirtieth of the bf16
     // matrix-core rate and a third of the f32 one, so rounding pays while it multiplies the work by less than that:
     // up to four times (bf16) and twice (f32).  d_ff 352 (the default model's) is 384 columns: 9 % more work.
-    auto rounded = [](int f, int unit, int most) {
+    auto rounded = [L](int f, int unit, int most) {
         const int up = (f + unit - 1) / unit * unit;
-        return up <= most * f ? up : f;
+        return up <= most * f && !L->tight ? up : f;
     };
     const int unit = cfg->weight_dtype == RBMOE_F32 ? 32 : 64, most = cfg->weight_dtype == RBMOE_F32 ? 2 : 4;
     L->Fw = rounded(cfg->d_ff, unit, most);
@@ -362,6 +367,25 @@ void choose_kernel_sets(rbmoe_layer* L) {
         L->Fw = cfg->d_ff;
         L->Fsw = L->Fs;
     }
+    const int block = L->tight ? kRouterTokens : kMinRouterTokens;  // tokens of the smallest router block
+    L->max_nb = (cfg->max_tokens + block - 1) / block;
+}
+
+// What stands against the backward pass of a layer with these widths ("": nothing).
+const char* training_widths_problem(const rbmoe_layer* L) {
+    const rbmoe_config& c = L->cfg;
+    const size_t d = c.d_model, F = L->Fw, Fs = L->Fsw, T = L->max_T, S = L->max_S;
+    if (L->use_stream && c.weight_dtype == RBMOE_BF16) {
+        if (!stream_shape_ok((int)d, (int)(2 * F)) || (c.shared_expert && !stream_shape_ok((int)d, (int)(2 * Fs))))
+            return "expert width not supported by the backward products";
+        // 32-bit byte offsets into the widest operand of the backward products: [S, 2F] bf16
+        if (std::max(S * 2 * F, T * 2 * Fs) * 2 >= ((size_t)1 << 32))
+            return "max_tokens x expert width too large for the backward products";
+    } else if (L->use_f32_mc &&
+               (!f32_shape_ok((int)d, (int)(2 * F)) || (c.shared_expert && !f32_shape_ok((int)d, (int)(2 * Fs))))) {
+        return "expert width not supported by the backward products";
+    }
+    return "";  // (any other layer - odd widths, mixed dtypes - takes the any-shape kernels in both directions)
 }
 
 Plan make_plan(rbmoe_layer* L) {
@@ -408,7 +432,7 @@ Plan make_plan(rbmoe_layer* L) {
     p.add(&L->perm_token, S * 4);
     p.add(&L->inv_pos, S * 4);
     if (L->cast_rows) p.add(&L->x16, T * d * 2);
-    if (L->use_stream && E <= 64)  // decode_front launches
+    if (L->use_stream && E <= (L->tight ? std::min<size_t>(64, 16 * k) : 64))  // decode_front launches
         p.add(&L->hall, E * std::min<size_t>(T, kSmallRouteMaxTokens) * F * 2);
     p.add(&L->cmbcnt, kDecodeCombineCounterBytes);
     p.add(&L->xg, S * d * as);
@@ -419,7 +443,6 @@ Plan make_plan(rbmoe_layer* L) {
     p.add(&L->st_res, T * d * as);
     p.add(&L->st_valid, T);
     p.add(&L->st_bias, E * 4);
-    (void)k;
     return p;
 }
 
@@ -433,6 +456,86 @@ void free_layer_buffers(rbmoe_layer* L) {
         }
     }
     L->all.clear();
+}
+
+// The buffers of a new layer, cleared.  A failure leaves none of them behind.
+int allocate_layer(rbmoe_layer* L) {
+    rbmoe_ctx* ctx = L->ctx;
+    Plan plan = make_plan(L);
+    // Refuse before allocating anything, as the reference's budget check does
+    // (src/param.rs:172-189).
+    if (ctx->budget_bytes && ctx->allocated + plan.total > ctx->budget_bytes) {
+        char buf[200];
+        std::snprintf(buf, sizeof buf, "memory budget exceeded: estimated %zu MiB exceeds budget %zu MiB",
+                      (ctx->allocated + plan.total + (1 << 20) - 1) >> 20, ctx->budget_bytes >> 20);
+        return fail(ctx, RBMOE_MEMORY_BUDGET, buf);
+    }
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    for (auto& it : plan.items) {
+        void* p = nullptr;
+        hipError_t e = hipMalloc(&p, it.second);
+        if (e != hipSuccess) {
+            size_t free_b = 0, total_b = 0;
+            (void)hipGetLastError();
+            (void)hipMemGetInfo(&free_b, &total_b);
+            char buf[200];
+            std::snprintf(buf, sizeof buf, "out of memory: an allocation of %zu MiB failed with %zu MiB free",
+                          it.second >> 20, free_b >> 20);
+            free_layer_buffers(L);
+            return fail(ctx, RBMOE_OUT_OF_MEMORY, buf);
+        }
+        it.first->p = p;
+        it.first->bytes = it.second;
+        ctx->allocated += it.second;
+        L->all.push_back(it.first);
+        e = hipMemsetAsync(p, 0, it.second, ctx->stream);
+        if (e != hipSuccess) {
+            free_layer_buffers(L);
+            return hip_fail(ctx, e, "hipMemsetAsync");
+        }
+    }
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (e != hipSuccess) {
+        free_layer_buffers(L);
+        return hip_fail(ctx, e, "hipStreamSynchronize");
+    }
+    return RBMOE_OK;
+}
+
+// A layer whose weights have not been set gives back what it holds beyond the tight layout, so that something further
+// fits.  Every buffer of that layout is at most as large as the one it replaces, and where the smaller one cannot be had
+// the layer keeps the larger.  A forward that has run on the zero weights is forgotten.
+void make_tight(rbmoe_layer* L) {
+    rbmoe_ctx* ctx = L->ctx;
+    const Plan roomy = make_plan(L);
+    L->tight = true;
+    choose_kernel_sets(L);
+    const Plan plan = make_plan(L);
+    (void)hipStreamSynchronize(ctx->stream);
+    L->last_T = -1;
+    for (auto& r : L->replay) r = nullptr;
+    for (const auto& was : roomy.items) {
+        Buf* const b = was.first;
+        size_t bytes = 0;
+        for (const auto& it : plan.items)
+            if (it.first == b) bytes = it.second;
+        if (bytes == b->bytes) continue;
+        void* p = nullptr;
+        if (bytes != 0) {
+            if (hipMalloc(&p, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                continue;
+            }
+            (void)hipMemsetAsync(p, 0, bytes, ctx->stream);
+        }
+        (void)hipFree(b->p);
+        ctx->allocated -= b->bytes;
+        ctx->allocated += bytes;
+        b->p = p;
+        b->bytes = bytes;
+        if (bytes == 0) L->all.erase(std::find(L->all.begin(), L->all.end(), b));
+    }
+    (void)hipStreamSynchronize(ctx->stream);
 }
 
 }  // namespace
@@ -577,59 +680,18 @@ int rbmoe_layer_create(rbmoe_ctx* ctx, const rbmoe_config* cfg, rbmoe_layer** ou
     L->cfg.shared_d_ff = L->Fs;
     L->max_T = cfg->max_tokens;
     L->max_S = cfg->max_tokens * cfg->experts_per_token;
-    L->max_nb = (cfg->max_tokens + kMinRouterTokens - 1) / kMinRouterTokens;
     L->max_tiles = L->max_S / kGenericTileM + cfg->num_experts + 1;
     // (behaviour switches keep their defaults here: rbmoe_layer_set_option changes them)
-    // bf16 matrix cores: bf16 activations, bf16 or int8 weights, widths that fit the packed layout
-    // (f32 rows with bf16 / int8 weights - what a caller with f32 matrices and a quantized or bf16 checkpoint has -
-    // take the same kernels over a bf16 copy of the rows)
-    choose_kernel_sets(L);
-
-    Plan plan = make_plan(L);
-    // Refuse before allocating anything, as the reference's budget check does
-    // (src/param.rs:172-189).
-    if (ctx->budget_bytes && ctx->allocated + plan.total > ctx->budget_bytes) {
-        char buf[200];
-        std::snprintf(buf, sizeof buf, "memory budget exceeded: estimated %zu MiB exceeds budget %zu MiB",
-                      (ctx->allocated + plan.total + (1 << 20) - 1) >> 20, ctx->budget_bytes >> 20);
-        delete L;
-        return fail(ctx, RBMOE_MEMORY_BUDGET, buf);
+    int rc = RBMOE_OK;
+    for (const bool tight : {false, true}) {
+        L->tight = tight;
+        choose_kernel_sets(L);
+        rc = allocate_layer(L);
+        if (rc != RBMOE_MEMORY_BUDGET && rc != RBMOE_OUT_OF_MEMORY) break;
     }
-    hipError_t e = hipSetDevice(ctx->device);
-    if (e != hipSuccess) {
+    if (rc != RBMOE_OK) {
         delete L;
-        return hip_fail(ctx, e, "hipSetDevice");
-    }
-    for (auto& it : plan.items) {
-        void* p = nullptr;
-        e = hipMalloc(&p, it.second);
-        if (e != hipSuccess) {
-            size_t free_b = 0, total_b = 0;
-            (void)hipGetLastError();
-            (void)hipMemGetInfo(&free_b, &total_b);
-            char buf[200];
-            std::snprintf(buf, sizeof buf, "out of memory: an allocation of %zu MiB failed with %zu MiB free",
-                          it.second >> 20, free_b >> 20);
-            free_layer_buffers(L);
-            delete L;
-            return fail(ctx, RBMOE_OUT_OF_MEMORY, buf);
-        }
-        it.first->p = p;
-        it.first->bytes = it.second;
-        ctx->allocated += it.second;
-        L->all.push_back(it.first);
-        e = hipMemsetAsync(p, 0, it.second, ctx->stream);
-        if (e != hipSuccess) {
-            free_layer_buffers(L);
-            delete L;
-            return hip_fail(ctx, e, "hipMemsetAsync");
-        }
-    }
-    e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) {
-        free_layer_buffers(L);
-        delete L;
-        return hip_fail(ctx, e, "hipStreamSynchronize");
+        return rc;
     }
     ++ctx->refs;
     *out = L;
@@ -1074,6 +1136,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
                   (int*)L->rank_in_block.p, (int*)L->blockcnt.p, (float*)L->partial.p};
     if (cast) ra.rows16 = L->x16.p;
     ra.allow_fused = L->fused_router;
+    if (L->tight) ra.min_tokens = kRouterTokens;
     if (L->router_q8) {
         ra.wq = (const int8_t*)L->router_q.p;
         ra.wscale = (const float*)L->router_s.p;
@@ -1488,19 +1551,107 @@ int allocate_plan(rbmoe_layer* L, Plan& p, const char* what) {
     return hip_fail(ctx, e, what);
 }
 
+// f(), as it would come out for the tight layout.
+template <typename F>
+auto when_tight(rbmoe_layer* L, F&& f) {
+    L->tight = true;
+    choose_kernel_sets(L);
+    auto r = f();
+    L->tight = false;
+    choose_kernel_sets(L);
+    return r;
+}
+
+// allocate_plan of `make()`; where budget or memory refuse it and the layer can still give something back, the layer is
+// made tight first.
+template <typename F>
+int allocate_or_tighten(rbmoe_layer* L, F&& make, const char* what) {
+    rbmoe_ctx* ctx = L->ctx;
+    {
+        Plan p = make();
+        const int rc = allocate_plan(L, p, what);
+        if ((rc != RBMOE_MEMORY_BUDGET && rc != RBMOE_OUT_OF_MEMORY) || L->tight || L->weights_set || L->training) return rc;
+        size_t held = 0;
+        for (const auto& it : make_plan(L).items) held += it.first->bytes;
+        const size_t needed = when_tight(L, [&] { return make_plan(L).total + make().total; });
+        if (rc == RBMOE_MEMORY_BUDGET && ctx->allocated - held + needed > ctx->budget_bytes) return rc;
+    }
+    make_tight(L);
+    Plan p = make();
+    return allocate_plan(L, p, what);
+}
+
 // Buffers of the backward pass through the norm: allocated by whichever of rbmoe_set_feed_forward_norm and
 // rbmoe_layer_enable_training comes second.
-int ensure_block_training_buffers(rbmoe_layer* L) {
-    if (!L->training || !L->norm_w.p || L->xraw.p) return RBMOE_OK;
+void add_block_training(rbmoe_layer* L, Plan& p) {
+    if (!L->norm_w.p || L->xraw.p) return;
     const rbmoe_config& c = L->cfg;
     const size_t T = L->max_T, d = c.d_model, as = dtype_size(c.act_dtype);
-    Plan p;
     p.add(&L->xraw, T * d * as);
     p.add(&L->dxn, T * d * as);
     p.add(&L->inv_rms, T * 4);
     p.add(&L->norm_partial, (size_t)rmsnorm_grad_tiles((int)T) * d * 4);
     p.add(&L->g_norm, d * 4);
+}
+int ensure_block_training_buffers(rbmoe_layer* L) {
+    if (!L->training || !L->norm_w.p || L->xraw.p) return RBMOE_OK;
+    Plan p;
+    add_block_training(L, p);
     return allocate_plan(L, p, "the norm's backward buffers");
+}
+
+Plan training_plan(rbmoe_layer* L) {
+    const rbmoe_config& c = L->cfg;
+    const size_t E = c.num_experts, d = c.d_model, F = L->Fw, Fs = L->Fsw, T = L->max_T, S = L->max_S;
+    const size_t ws = dtype_size(c.weight_dtype);  // bytes per element of the transposed weight copies
+    const size_t as = dtype_size(c.act_dtype);
+    const size_t ps = L->cast_rows ? 2 : as;       // bytes per element of the rows the products read and write
+    Plan p;
+    p.add(&L->xc, T * d * as);
+    if (L->cast_rows) p.add(&L->g16, T * d * 2);
+    p.add(&L->gu, S * 2 * F * ps);
+    p.add(&L->dy, S * d * ps);
+    p.add(&L->dgu, S * 2 * F * ps);
+    p.add(&L->dxg, S * d * ps);
+    p.add(&L->grad_gates, S * 4);
+    p.add(&L->ones, S * 4);
+    p.add(&L->dlogits, T * E * 4);
+    p.add(&L->dxr, T * d * as);
+    p.add(&L->rpartial, (size_t)router_grad_chunks((int)T) * E * d * 4);
+    p.add(&L->g_router, E * d * 4);
+    p.add(&L->g_gu, E * 2 * F * d * 4);
+    p.add(&L->g_down, E * d * F * 4);
+    p.add(&L->wdT, E * F * d * ws);
+    p.add(&L->wguT, E * d * 2 * F * ws);
+    // (four tables: down and gate/up gradients of the routed experts and of the shared one)
+    p.add(&L->wg_chunks, (size_t)4 * wgrad_table_ints(L) * 4);
+    // How the weight gradients treat an expert far above the average share (and the shared expert, whose one
+    // group of rows is always cut): in a fixed order by default (RBMOE_OPT_WGRAD_MODE for f32 atomics or no cut).
+    if (L->wgrad_split == WgradSplit::Ordered) {
+        const bool wbf = c.act_dtype == RBMOE_BF16 || L->cast_rows;
+        // sized for every token count up to max_tokens: a smaller batch can need more partial matrices than the
+        // largest one, because the cut limit follows the row count with a floor and a rounding
+        const int k = c.experts_per_token;
+        size_t need = std::max(weight_grad_partial_bytes_upto((int)d, (int)F, (int)E, false, (int)T, k, wbf),
+                               weight_grad_partial_bytes_upto((int)(2 * F), (int)d, (int)E, false, (int)T, k, wbf));
+        if (c.shared_expert)
+            need = std::max(need, std::max(weight_grad_partial_bytes_upto((int)d, (int)Fs, 1, true, (int)T, 1, wbf),
+                                           weight_grad_partial_bytes_upto((int)(2 * Fs), (int)d, 1, true, (int)T, 1, wbf)));
+        p.add(&L->wg_partial, need);
+    }
+    p.add(&L->st_gout, T * d * as);
+    p.add(&L->st_gin, T * d * as);
+    if (c.shared_expert) {
+        p.add(&L->gus, T * 2 * Fs * ps);
+        p.add(&L->dgus, T * 2 * Fs * ps);
+        p.add(&L->dxs, T * d * ps);
+        p.add(&L->g_sgu, 2 * Fs * d * 4);
+        p.add(&L->g_sdown, d * Fs * 4);
+        p.add(&L->swdT, Fs * d * ws);
+        p.add(&L->swguT, d * 2 * Fs * ws);
+    }
+    add_block_training(L, p);
+    return p;
 }
 
 // The backward entry points differentiate the LAST forward, whose shape the reference takes from the cached input
@@ -1886,10 +2037,13 @@ int rbmoe_set_feed_forward_norm(rbmoe_layer* L, const float* weight, int32_t col
     }
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     if (!L->norm_w.p) {
-        Plan p;
-        p.add(&L->xn, (size_t)L->max_T * c.d_model * dtype_size(c.act_dtype));
-        p.add(&L->norm_w, (size_t)c.d_model * 4);
-        if (const int rc = allocate_plan(L, p, "the normed rows")) return rc;
+        auto plan = [&] {
+            Plan p;
+            p.add(&L->xn, (size_t)L->max_T * c.d_model * dtype_size(c.act_dtype));
+            p.add(&L->norm_w, (size_t)c.d_model * 4);
+            return p;
+        };
+        if (const int rc = allocate_or_tighten(L, plan, "the normed rows")) return rc;
     }
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));  // no forward may still read the old weight
     HIP_TRY(ctx, hipMemcpy(L->norm_w.p, weight, (size_t)c.d_model * 4, hipMemcpyHostToDevice));
@@ -1944,82 +2098,24 @@ int rbmoe_layer_enable_training(rbmoe_layer* L) {
     // the matrix cores in both directions: the products read the bf16 copy of the rows that the forward writes
     // anyway and a bf16 copy of the upstream gradient that the backward pass writes first; the router's branch,
     // the norm and the sums that end in the caller's buffers stay f32)
-    const bool bf16_layer = L->use_stream && c.weight_dtype == RBMOE_BF16;
     if (L->max_T > router_grad_max_tokens()) {  // found here, not in the middle of a backward pass
         char buf[160];
         std::snprintf(buf, sizeof buf, "the backward pass takes at most %d tokens a call, the layer was created for %d",
                       router_grad_max_tokens(), L->max_T);
         return fail(ctx, RBMOE_UNSUPPORTED, buf);
     }
-    const size_t E = c.num_experts, d = c.d_model, F = L->Fw, Fs = L->Fsw, T = L->max_T, S = L->max_S;
-    if (bf16_layer) {
-        if (!stream_shape_ok((int)d, (int)(2 * F)) || (c.shared_expert && !stream_shape_ok((int)d, (int)(2 * Fs))))
-            return fail(ctx, RBMOE_UNSUPPORTED, "expert width not supported by the backward products");
-        // 32-bit byte offsets into the widest operand of the backward products: [S, 2F] bf16
-        if (std::max(S * 2 * F, T * 2 * Fs) * 2 >= ((size_t)1 << 32))
-            return fail(ctx, RBMOE_UNSUPPORTED, "max_tokens x expert width too large for the backward products");
-    } else if (L->use_f32_mc &&
-               (!f32_shape_ok((int)d, (int)(2 * F)) || (c.shared_expert && !f32_shape_ok((int)d, (int)(2 * Fs))))) {
-        return fail(ctx, RBMOE_UNSUPPORTED, "expert width not supported by the backward products");
-    }
-    // (any other layer - odd widths, mixed dtypes - takes the any-shape kernels in both directions)
-    const size_t ws = dtype_size(c.weight_dtype);  // bytes per element of the transposed weight copies
-    const size_t as = dtype_size(c.act_dtype);
-    const size_t ps = L->cast_rows ? 2 : as;       // bytes per element of the rows the products read and write
-    Plan p;
-    p.add(&L->xc, T * d * as);
-    if (L->cast_rows) p.add(&L->g16, T * d * 2);
-    p.add(&L->gu, S * 2 * F * ps);
-    p.add(&L->dy, S * d * ps);
-    p.add(&L->dgu, S * 2 * F * ps);
-    p.add(&L->dxg, S * d * ps);
-    p.add(&L->grad_gates, S * 4);
-    p.add(&L->ones, S * 4);
-    p.add(&L->dlogits, T * E * 4);
-    p.add(&L->dxr, T * d * as);
-    p.add(&L->rpartial, (size_t)router_grad_chunks((int)T) * E * d * 4);
-    p.add(&L->g_router, E * d * 4);
-    p.add(&L->g_gu, E * 2 * F * d * 4);
-    p.add(&L->g_down, E * d * F * 4);
-    p.add(&L->wdT, E * F * d * ws);
-    p.add(&L->wguT, E * d * 2 * F * ws);
-    // (four tables: down and gate/up gradients of the routed experts and of the shared one)
-    p.add(&L->wg_chunks, (size_t)4 * wgrad_table_ints(L) * 4);
-    // How the weight gradients treat an expert far above the average share (and the shared expert, whose one
-    // group of rows is always cut): in a fixed order by default (RBMOE_OPT_WGRAD_MODE for f32 atomics or no cut).
-    if (L->wgrad_split == WgradSplit::Ordered) {
-        const bool wbf = c.act_dtype == RBMOE_BF16 || L->cast_rows;
-        // sized for every token count up to max_tokens: a smaller batch can need more partial matrices than the
-        // largest one, because the cut limit follows the row count with a floor and a rounding
-        const int k = c.experts_per_token;
-        size_t need = std::max(weight_grad_partial_bytes_upto((int)d, (int)F, (int)E, false, (int)T, k, wbf),
-                               weight_grad_partial_bytes_upto((int)(2 * F), (int)d, (int)E, false, (int)T, k, wbf));
-        if (c.shared_expert)
-            need = std::max(need, std::max(weight_grad_partial_bytes_upto((int)d, (int)Fs, 1, true, (int)T, 1, wbf),
-                                           weight_grad_partial_bytes_upto((int)(2 * Fs), (int)d, 1, true, (int)T, 1, wbf)));
-        p.add(&L->wg_partial, need);
-    }
-    p.add(&L->st_gout, T * d * as);
-    p.add(&L->st_gin, T * d * as);
-    if (c.shared_expert) {
-        p.add(&L->gus, T * 2 * Fs * ps);
-        p.add(&L->dgus, T * 2 * Fs * ps);
-        p.add(&L->dxs, T * d * ps);
-        p.add(&L->g_sgu, 2 * Fs * d * 4);
-        p.add(&L->g_sdown, d * Fs * 4);
-        p.add(&L->swdT, Fs * d * ws);
-        p.add(&L->swguT, d * 2 * Fs * ws);
-    }
+    if (*training_widths_problem(L) && !L->tight && !*when_tight(L, [&] { return training_widths_problem(L); })) make_tight(L);
+    if (const char* const problem = training_widths_problem(L); *problem) return fail(ctx, RBMOE_UNSUPPORTED, problem);
     // (the second stream first: a failure there must not leave buffers behind that a second attempt would allocate again)
     if (L->shared_beside)
         if (const int rc = ensure_side_stream(ctx)) return rc;
-    if (const int rc = allocate_plan(L, p, "the training buffers")) return rc;
-    HIP_TRY(ctx, launch_fill_f32((float*)L->ones.p, 1.0f, (long long)S, ctx->stream));
+    if (const int rc = allocate_or_tighten(L, [&] { return training_plan(L); }, "the training buffers")) return rc;
+    HIP_TRY(ctx, launch_fill_f32((float*)L->ones.p, 1.0f, (long long)L->max_S, ctx->stream));
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     L->side_branch = L->shared_beside;
     L->training = true;
     L->grads_clear = true;
-    return ensure_block_training_buffers(L);
+    return RBMOE_OK;
 }
 
 int rbmoe_layer_set_option(rbmoe_layer* L, int32_t option, int32_t value) {
@@ -2488,6 +2584,28 @@ int rbmoe_internal_weight_grad_slots(int32_t M, int32_t N, int32_t groups, int32
     const int rows = dense ? tokens : tokens * rows_per_token;
     *needed = (int64_t)(weight_grad_partial_bytes(M, N, groups, dense ? rows : -1, rows, bf16 != 0) / one);
     *held = (int64_t)(weight_grad_partial_bytes_upto(M, N, groups, dense != 0, max_tokens, rows_per_token, bf16 != 0) / one);
+    return RBMOE_OK;
+}
+
+// Test hook (not part of rbmoe.h), runs without a GPU: the expert widths that the kernels of a layer see.  out[0]: routed,
+// [1]: shared, [2]: 0 any-shape kernels, 1 bf16 matrix cores, 2 f32 matrix cores; training != 0: after
+// rbmoe_layer_enable_training, RBMOE_UNSUPPORTED where that refuses the widths.
+int rbmoe_internal_widths(const rbmoe_config* cfg, int32_t training, int32_t* out) {
+    if (!cfg || !out) return RBMOE_NULL_POINTER;
+    rbmoe_layer L;
+    L.cfg = *cfg;
+    L.Fs = cfg->shared_d_ff > 0 ? cfg->shared_d_ff : cfg->d_ff;
+    L.max_T = cfg->max_tokens;
+    L.max_S = cfg->max_tokens * cfg->experts_per_token;
+    choose_kernel_sets(&L);
+    if (training && *training_widths_problem(&L)) {
+        L.tight = true;
+        choose_kernel_sets(&L);
+        if (*training_widths_problem(&L)) return RBMOE_UNSUPPORTED;
+    }
+    out[0] = L.Fw;
+    out[1] = L.Fsw;
+    out[2] = L.use_stream ? 1 : L.use_f32_mc ? 2 : 0;
     return RBMOE_OK;
 }
 

@@ -79,6 +79,7 @@ struct RouterArgs {
     float* partial;      // [nb, E+1]
     void* rows16 = nullptr;  // f32 rows only: [T, d] bf16 copy of x written on the way (d a multiple of 8), or null
     bool allow_fused = true; // logits and everything behind them in one launch where the shapes allow
+    int min_tokens = kMinRouterTokens;  // of a router block: the block tables are sized for these
     // a quantized router (Quantized::matmul_rhs_transposed, src/quantized.rs:55-62): int8 rows and one scale per row;
     // `wr` is then not read and the logits are (sum_c x[c] * f32(q[c]), in the reference's 32 lanes) * scale
     const int8_t* wq = nullptr;      // [E, d]

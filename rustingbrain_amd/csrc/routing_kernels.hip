@@ -1212,9 +1212,9 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     if (reinterpret_cast<uintptr_t>(a.wq ? static_cast<const void*>(a.wq) : a.wr) & 15) return p;
     if (a.norm_w && ((reinterpret_cast<uintptr_t>(a.xn_out) & 15) || a.d % 8 != 0)) return p;
     const int NL = a.wq ? 32 : 8;
-    int tokens = kMinRouterTokens;
+    int tokens = a.min_tokens;
     while (tokens < kRouterTokens && (a.T + tokens - 1) / tokens > 256) tokens *= 2;
-    for (; tokens >= kMinRouterTokens && !p.tokens; tokens /= 2) {
+    for (; tokens >= a.min_tokens && !p.tokens; tokens /= 2) {
         int EG = a.E;  // as many experts' rows as fit together, whole pairs, at least 8 (or all of them)
         auto lds = [&] { return route_rows_lds_bytes(a.E, a.k, a.d, tokens, NL, EG, a.norm_w != nullptr); };
         while (EG > 8 && lds() > (size_t)kMaxRouterLds) EG = (EG - 1) & ~1;

@@ -72,3 +72,35 @@ def test_weight_gradients_of_bf16_layers_round_no_more_often_than_the_plain_kern
         return rel_l2(got, ref)
 
     assert distance(False) <= 1.03 * distance(True)
+
+
+@pytest.mark.parametrize("training", [False, True])
+def test_a_memory_budget_that_holds_the_true_widths_is_enough(device, training):
+    """F 16 is stored as 64: four times the matrices.  A budget too small for that gets the any-shape kernels."""
+    E, d, F, T = 8, 1024, 16, 40
+    t = synth.make(small_workload(d=d, E=E, k=2, F=F, T=T, seed=64, act="bf16", wt="bf16"))
+    ref = oracle_layer(t).forward(t.x, threads=4)
+    gout = synth.round_bf16(synth.normal((T, d), 1.0, 64, 5))
+    want = oracle_layer(t).backward(t.x, gout, threads=4) if training else None
+    names = []
+    for mib in range(1, 64):
+        dev = rb.Device.open(0, budget_mib=mib)
+        try:
+            layer = rb.MoeLayer(d, rb.MoeConfig(E, 2, F), dev, act_dtype="bf16", weight_dtype="bf16", max_tokens=T)
+            if training:
+                layer.set_feed_forward_norm(np.ones(d, np.float32))   # (its buffers count too)
+                layer.enable_training()
+        except rb.MemoryBudget:
+            assert not names   # a larger budget is enough as well
+            continue
+        layer.load_tensors(t)
+        out, _ = layer.forward_train(t.x)
+        assert rel_l2(out, ref.out) <= 2e-2
+        if training:
+            assert rel_l2(layer.backward(gout), want.grad_input) <= 2e-2
+            assert rel_l2(layer.weight_grad(L.W_DOWN, 1), want.grad_down[1]) <= 2e-2
+        names.append(layer.kernel_name())
+        layer.close()
+        dev.close()
+    small = names.index("mfma_bf16_stream")
+    assert 0 < small and names == ["generic"] * small + ["mfma_bf16_stream"] * (len(names) - small)

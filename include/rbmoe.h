@@ -343,8 +343,10 @@ int rbmoe_forward_kernel_times(rbmoe_layer* layer, const void* x, int32_t T, int
  * rotation.  RBMOE_UNSUPPORTED when the last forward had no launch of its own for the stage. */
 int rbmoe_replay_stage(rbmoe_layer* layer, int32_t stage, int32_t launches, float* ms_per_launch);
 
-/* Name of the kernel variant the last forward used for the expert products
- * ("mfma_bf16", "generic", ...), for reports.  Static storage. */
+/* Name of the kernels the last forward used for the expert products, for reports: "mfma_bf16_stream" (large
+ * batches), "mfma_bf16_decode_front" (a few tokens, routing beside the gate/up products), "mfma_bf16_decode" (a few
+ * tokens, routing in a launch of its own), each with "_int8w" behind it for int8 weights, "mfma_f32", "generic"; "none"
+ * before the first.  Static storage. */
 const char* rbmoe_expert_kernel_name(const rbmoe_layer* layer);
 
 /* Device memory helpers for hosts without their own HIP binding. */

@@ -1386,13 +1386,13 @@ bool decode_front_ok(const RouterArgs& a, bool bf16) {
            front_lds_bytes(a.T, a.E, a.k, a.d, a.wq != nullptr, a.norm_w != nullptr, &eg) != 0;
 }
 
-hipError_t launch_decode_front(const RouterArgs& a, const DecodeGemmArgs& g, bool bf16, WeightKind wk, bool products, hipStream_t s) {
+hipError_t launch_decode_front(const RouterArgs& a, const DecodeGemmArgs& g, bool bf16, WeightKind wk, hipStream_t s) {
     if (!decode_front_ok(a, bf16) || !g.swiglu || wk == WeightKind::F32 || (a.wq && (!a.wscale || wk != WeightKind::I8)))
         return hipErrorInvalidValue;
     const int shared_tiles = g.a_shared ? (g.T_shared + 31) / 32 : 0;
     const int widest = g.a_shared ? (g.N > g.N_shared ? g.N : g.N_shared) : g.N;
     const int routers = (a.T + kFrontTokens - 1) / kFrontTokens;
-    const int grid = routers + (products ? (a.E + shared_tiles) * ((widest / 32 + kFrontTeams - 1) / kFrontTeams) : 0);
+    const int grid = routers + (a.E + shared_tiles) * ((widest / 32 + kFrontTeams - 1) / kFrontTeams);
     int EG = 0;
     const size_t lds = front_lds_bytes(a.T, a.E, a.k, a.d, a.wq != nullptr, a.norm_w != nullptr, &EG);
     RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, EG, a.P, a.lse, a.expert_of, a.gate_of,

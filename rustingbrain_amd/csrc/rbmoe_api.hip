@@ -1193,7 +1193,8 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
 
     // ---- a few tokens: route in one workgroup, then stream the touched weights once -------
     if (decode_ok) {
-        L->kernel_name = wk == WeightKind::I8 ? "mfma_bf16_decode_int8w" : "mfma_bf16_decode";
+        L->kernel_name = front ? (wk == WeightKind::I8 ? "mfma_bf16_decode_front_int8w" : "mfma_bf16_decode_front")
+                               : (wk == WeightKind::I8 ? "mfma_bf16_decode_int8w" : "mfma_bf16_decode");
         SmallRouteArgs sr{};
         sr.x = x; sr.wr = (const float*)L->router.p; sr.bias = router_bias; sr.valid = valid;
         if (norm_in_route) {
@@ -1210,7 +1211,6 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         sr.ntiles = wk_.ntiles; sr.losses = wk_.losses;
         sr.perm_slot = wk_.perm_slot; sr.perm_token = wk_.perm_token; sr.inv_pos = wk_.inv_pos;
         for (auto& r : L->replay) r = nullptr;
-        const bool named_front = front && !cast && T * k >= 2 * E;
         if (!front) {
             HIP_TRY(ctx, launch_route_small(sr, abf, s));
             L->replay[RBMOE_STAGE_ROUTER] = [=](hipStream_t st) { return launch_route_small(sr, abf, st); };
@@ -1244,10 +1244,8 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
             if (c.shared_expert) d1.a_shared = fr.x;
             d1.row_index = nullptr;
             d1.out = wk_.hall;
-            HIP_TRY(ctx, launch_decode_front(fr, d1, abf, wk, true, s));
-            L->replay[RBMOE_STAGE_GATE_UP] = [=](hipStream_t st) { return launch_decode_front(fr, d1, abf, wk, true, st); };
-            if (!named_front)  // (not reported as routing beside the products: the routing alone is its stage then)
-                L->replay[RBMOE_STAGE_ROUTER] = [=](hipStream_t st) { return launch_decode_front(fr, d1, abf, wk, false, st); };
+            HIP_TRY(ctx, launch_decode_front(fr, d1, abf, wk, s));
+            L->replay[RBMOE_STAGE_GATE_UP] = [=](hipStream_t st) { return launch_decode_front(fr, d1, abf, wk, st); };
         } else {
             HIP_TRY(ctx, launch_decode_gemm(d1, wk, s));
             L->replay[RBMOE_STAGE_GATE_UP] = [=](hipStream_t st) { return launch_decode_gemm(d1, wk, st); };
@@ -1303,8 +1301,6 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         L->last = wk_;
         L->last_front = front;
         L->last_by_slot = by_expert;
-        if (named_front)
-            L->kernel_name = wk == WeightKind::I8 ? "mfma_bf16_decode_front_int8w" : "mfma_bf16_decode_front";
         return RBMOE_OK;
     }
 

@@ -363,9 +363,9 @@ hipError_t launch_decode_gemm(const DecodeGemmArgs& g, WeightKind wk, hipStream_
 // Routing and gate/up products in one launch: every expert's gate/up product over all T rows, hidden rows to g.out as
 // [E][T, N]; the shared expert as in launch_decode_gemm.  g.a / g.a_shared: the call's rows as they are (a.x), f32 or
 // bf16, raw when the routing applies a norm - the products then take the normed rows on the way.  P, lse, expert_of and
-// gate_of are written, nothing else of the routing (DecodeLayoutArgs).  products = false: the routing alone.
+// gate_of are written, nothing else of the routing (DecodeLayoutArgs).
 bool decode_front_ok(const RouterArgs& a, bool bf16);
-hipError_t launch_decode_front(const RouterArgs& a, const DecodeGemmArgs& g, bool bf16, WeightKind wk, bool products, hipStream_t s);
+hipError_t launch_decode_front(const RouterArgs& a, const DecodeGemmArgs& g, bool bf16, WeightKind wk, hipStream_t s);
 // The tables and losses of a call routed by launch_decode_front.
 struct DecodeLayoutArgs {
     const float* P;

@@ -148,8 +148,9 @@ def test_routing_beside_the_products_changes_nothing_but_the_launch_count(device
     assert np.array_equal(cache_f.gate_of.view(np.uint32), cache_p.gate_of.view(np.uint32))
     assert cache_f.aux_loss() == cache_p.aux_loss() and cache_f.z_loss() == cache_p.z_loss()
     assert rel_l2(out_f, out_p) <= 5e-3
-    # few slots on many experts: the launches stay apart (an unrouted expert's weights would be fetched for nothing)
-    t = synth.make(small_workload(seed=41, act="bf16", wt=wt, d=64, E=16, k=2, F=64, T=4))
+    # few slots on many large experts: the launches stay apart (28 of 32 experts' weights, 44 or 88 MB, would be fetched
+    # for nothing)
+    t = synth.make(small_workload(seed=41, act="bf16", wt=wt, d=512, E=32, k=2, F=1024, T=2))
     env.pop("RBMOE_NO_DECODE_FRONT", None)
     name, _, _ = run(device, t)
     assert name.startswith("mfma_bf16_decode") and "front" not in name

@@ -109,7 +109,7 @@ def test_f32_rows_with_bf16_or_int8_weights_run_on_the_matrix_cores(device, wt, 
     t = synth.make(small_workload(d=768, E=8, k=2, F=1408, T=T, seed=29, act="f32", wt=wt, shared=True,
                                   shared_d_ff=704))
     name = run(device, t)
-    assert name == ("mfma_bf16_decode" if T <= 32 else "mfma_bf16_stream") + ("_int8w" if wt == "int8" else "")
+    assert name == ("mfma_bf16_decode_front" if T <= 32 else "mfma_bf16_stream") + ("_int8w" if wt == "int8" else "")
     valid = (np.arange(T) % 5 != 2).astype(np.uint8)
     bias = synth.normal((8,), 0.5, 29, 98)
     run(device, t, valid=valid, bias=bias)

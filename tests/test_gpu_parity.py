@@ -162,7 +162,7 @@ def test_rows_whose_logits_overflow_route_like_the_cpu_path(device, T, act):
     assert np.array_equal(cache.probabilities[finite], ref.probabilities[finite])
     assert cache.expert_of.reshape(T, 2)[2].tolist() == [0, 1]          # all-equal probabilities: lowest indices
     assert np.array_equal(cache.counts, ref.counts) and np.array_equal(cache.perm_slot, ref.perm_slot)
-    assert layer.kernel_name() == {"f32": "generic", "bf16": "mfma_bf16_decode" if T <= 32 else "mfma_bf16_stream"}[act]
+    assert layer.kernel_name() == {"f32": "generic", "bf16": "mfma_bf16_decode_front" if T <= 32 else "mfma_bf16_stream"}[act]
     layer.close()
 
 

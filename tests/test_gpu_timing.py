@@ -14,8 +14,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("shape", [dict(d=128, E=8, k=2, F=192, T=700, shared=True),     # large-batch kernels
                                    dict(d=128, E=8, k=2, F=192, T=16, shared=True),      # decode-shaped, routing beside
-                                   dict(d=64, E=40, k=2, F=64, T=8)],                    # decode-shaped, four launches
-                         ids=["batch", "decode_front", "decode"])
+                                   dict(d=256, E=40, k=2, F=640, T=8),                   # decode-shaped, routing in front
+                                   dict(d=64, E=40, k=2, F=64, T=8)],                    # few slots, little to fetch for nothing
+                         ids=["batch", "decode_front", "decode", "decode_front_few_slots"])
 def test_measuring_entry_points_leave_the_results_alone(device, shape):
     t = synth.make(small_workload(seed=91, act="bf16", wt="bf16", **shape))
     T = shape["T"]
@@ -58,6 +59,7 @@ def test_measuring_entry_points_leave_the_results_alone(device, shape):
         assert layer.enqueue_stage(stage, 2)
         assert same(snapshot(), plain), stage
     front = layer.kernel_name().startswith("mfma_bf16_decode_front")
+    assert front == (T <= 32 and shape["d"] * shape["F"] < 100_000)
     assert (layer.replay_stage("router", 2) is None) == front   # the routing has no launch of its own there
     assert (layer.replay_stage("dispatch", 2) is None) == ("decode" in layer.kernel_name())
     assert layer.replay_stage("empty", 2) is None

@@ -354,8 +354,7 @@ int rbmoe_device_alloc(rbmoe_ctx* ctx, size_t bytes, void** out);
 int rbmoe_device_free(rbmoe_ctx* ctx, void* ptr);
 /* Host memory the GPU writes to and reads from directly (57 GB/s over the link here, against 4 to 30 for a copy to or
  * from memory that is not pinned): every entry point above that fills or reads a host array recognises these blocks.
- * They come from a pool of at most 1 GiB that keeps freed blocks for the next caller and is emptied when the last
- * context goes; RBMOE_OUT_OF_MEMORY when it is exhausted (use ordinary memory then).  Any thread may free. */
+ * They come from a pool of at most 1 GiB that keeps freed blocks for the next caller while a context lives; RBMOE_OUT_OF_MEMORY when it is exhausted (use ordinary memory then).  Any thread may free. */
 int rbmoe_host_alloc(rbmoe_ctx* ctx, size_t bytes, void** out);
 void rbmoe_host_free(void* ptr);
 int rbmoe_copy_to_device(rbmoe_ctx* ctx, void* dst, const void* src, size_t bytes);

@@ -13,12 +13,15 @@ namespace rbmoe {
 // Pinning is slow (a millisecond for a few megabytes) and a copy to pageable memory that has not been touched yet
 // runs at 4 GB/s (page faults; warm pages 18, pinned 57), so blocks are kept for the next taker.  Blocks in use and
 // blocks kept together never exceed kHostPoolMax; above it host_block_take returns null and the caller uses pageable
-// memory.  host_pool_trim gives the kept blocks back to the system.  Any thread may call any of these.
+// memory.  Blocks are kept while a context lives (host_pool_hold, host_pool_release): the last one to go gives the kept
+// blocks back to the system, and those still in use follow when they are given back.  Any thread may call any of these.
 constexpr size_t kHostPoolMax = (size_t)1 << 30;
 void* host_block_take(size_t bytes);
 void host_block_give(void* p);
 bool host_block_holds(const void* p, size_t bytes);  // whether [p, p + bytes) lies inside a block in use
-void host_pool_trim();
+void host_pool_hold();
+void host_pool_release();
+void host_pool_sizes(size_t* used, size_t* kept);  // bytes
 
 // A block for the length of a scope (null when the pool is exhausted).
 struct HostBlock {

@@ -17,6 +17,7 @@ struct HostPool {
     std::map<uintptr_t, size_t> used;              // blocks in use, by address
     std::map<size_t, std::vector<void*>> kept;     // free blocks, by size
     size_t used_bytes = 0, kept_bytes = 0;
+    int holders = 0;                               // contexts that live
 };
 
 // (never destroyed: blocks may be given back while the process ends)
@@ -85,6 +86,10 @@ void host_block_give(void* block) {
     const size_t size = it->second;
     p.used.erase(it);
     p.used_bytes -= size;
+    if (p.holders == 0) {  // nobody is left to take it again
+        (void)hipHostFree(block);
+        return;
+    }
     p.kept[size].push_back(block);
     p.kept_bytes += size;
 }
@@ -98,9 +103,23 @@ bool host_block_holds(const void* ptr, size_t bytes) {
     return (uintptr_t)ptr + bytes <= it->first + it->second;
 }
 
-void host_pool_trim() {
+void host_pool_hold() {
     HostPool& p = pool();
     std::lock_guard<std::mutex> lock(p.mutex);
+    ++p.holders;
+}
+
+void host_pool_sizes(size_t* used, size_t* kept) {
+    HostPool& p = pool();
+    std::lock_guard<std::mutex> lock(p.mutex);
+    *used = p.used_bytes;
+    *kept = p.kept_bytes;
+}
+
+void host_pool_release() {
+    HostPool& p = pool();
+    std::lock_guard<std::mutex> lock(p.mutex);
+    if (--p.holders > 0) return;
     for (auto& k : p.kept)
         for (void* b : k.second) (void)hipHostFree(b);
     p.kept.clear();

@@ -9,7 +9,6 @@
 #include "../../include/rbmoe.h"
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -56,8 +55,6 @@ hipError_t static_scratch_of(int device, void** out) {
     *out = g_scratch_ptr[device];
     return hipSuccess;
 }
-
-std::atomic<int> g_live_contexts{0};  // the last one to go gives the kept pinned blocks back
 
 thread_local std::string g_global_error;
 
@@ -619,7 +616,7 @@ int rbmoe_ctx_create(int32_t device, size_t budget_mib, rbmoe_ctx** out) {
         return hip_fail(nullptr, se, "hipStreamCreateWithFlags");
     }
     ctx->stream = ctx->own_stream;
-    ++g_live_contexts;
+    host_pool_hold();
     *out = ctx;
     return RBMOE_OK;
 }
@@ -641,7 +638,7 @@ static void ctx_release(rbmoe_ctx* ctx) {
         (void)hipStreamDestroy(ctx->own_stream);
     }
     delete ctx;
-    if (--g_live_contexts == 0) host_pool_trim();
+    host_pool_release();
 }
 
 // Layers keep their context alive: destroying the context while layers exist
@@ -2580,6 +2577,16 @@ int rbmoe_internal_weight_grad_slots(int32_t M, int32_t N, int32_t groups, int32
     const int rows = dense ? tokens : tokens * rows_per_token;
     *needed = (int64_t)(weight_grad_partial_bytes(M, N, groups, dense ? rows : -1, rows, bf16 != 0) / one);
     *held = (int64_t)(weight_grad_partial_bytes_upto(M, N, groups, dense != 0, max_tokens, rows_per_token, bf16 != 0) / one);
+    return RBMOE_OK;
+}
+
+// Test hook (not part of rbmoe.h): bytes of the pinned pool in use and kept.
+int rbmoe_internal_host_pool(uint64_t* used, uint64_t* kept) {
+    if (!used || !kept) return RBMOE_NULL_POINTER;
+    size_t u = 0, k = 0;
+    host_pool_sizes(&u, &k);
+    *used = u;
+    *kept = k;
     return RBMOE_OK;
 }
 

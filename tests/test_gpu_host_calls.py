@@ -1,11 +1,14 @@
 """Host matrices through the pinned pool: results in pinned blocks, pageable ones, a pool that is given back to, rows
 longer than one piece of the copy, f32 rows of bf16 layers rounded by the library."""
 import ctypes as C
+import subprocess
+import sys
 import threading
 
 import numpy as np
 import pytest
 
+from conftest import ROOT
 from helpers import gpu_layer, small_workload
 from rustingbrain_amd import _lib as L
 from rustingbrain_amd import synth
@@ -76,3 +79,37 @@ def test_threads_take_and_give_blocks_at_once(device):
     [th.start() for th in threads]
     [th.join() for th in threads]
     assert not errors
+
+
+def test_blocks_outliving_the_last_context_are_not_kept():
+    """In a process of its own: this one's contexts live on."""
+    code = """
+import ctypes as C
+import subprocess
+import sys
+import numpy as np
+import rustingbrain_amd as rb
+from rustingbrain_amd import _lib as L
+def pool():
+    used, kept = C.c_uint64(), C.c_uint64()
+    assert L.load().rbmoe_internal_host_pool(C.byref(used), C.byref(kept)) == L.OK
+    return used.value, kept.value
+dev = rb.Device.open(0)
+a, b = dev.empty((1 << 20,), np.float32), dev.empty((1 << 20,), np.float32)
+del b
+assert pool() == (4 << 20, 4 << 20), pool()
+dev.close()
+assert pool() == (4 << 20, 0), pool()   # what was kept is gone, what is in use is not
+a[:] = 1
+del a
+assert pool() == (0, 0), pool()
+dev = rb.Device.open(0)
+c = dev.empty((1 << 20,), np.float32)
+del c
+assert pool() == (0, 4 << 20), pool()
+dev.close()
+assert pool() == (0, 0), pool()
+print("pool ok")
+"""
+    done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0 and "pool ok" in done.stdout, done.stderr[-2000:]

@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes as C
 import gc
+import math
 import weakref
 from dataclasses import dataclass, replace
 from typing import List, Optional, Sequence, Tuple
@@ -253,24 +254,29 @@ class MoeCache:
 
 
 class _Tables:
-    """The host arrays one forward's routing tables are fetched into, cut out of one allocation."""
+    """The host arrays one forward's routing tables are fetched into, each with memory of its own: a caller may keep one
+    of them for long."""
 
     def __init__(self, layer: "MoeLayer", tokens: int):
         E, k = layer.config.num_experts, layer.config.experts_per_token
         S = tokens * k
-        sizes = (S, S, E, E + 1, S, S, tokens * E, tokens, 2)
-        words = layer.device.empty((sum(sizes),), np.int32)
-        at, ptr, parts, ptrs = 0, words.ctypes.data, [], []
-        for n in sizes:
-            parts.append(words[at:at + n])
-            ptrs.append(ptr + 4 * at)
-            at += n
-        self.expert_of, gate_of, self.counts, self.offsets, self.perm_slot, self.perm_token, prob, lse, losses = parts
-        self.gate_of, self.log_sum_exp, self.losses = (a.view(np.float32) for a in (gate_of, lse, losses))
-        self.probabilities = prob.view(np.float32).reshape(tokens, E)
+
+        def table(shape, dtype):
+            # below 64 KB the library's own copy is cheaper than a pinned block (4 us), and it overlaps with the products
+            if math.prod(shape) < 16384:
+                return np.empty(shape, dtype)
+            return layer.device.empty(shape, dtype)
+
+        self.expert_of, self.gate_of = table((S,), np.int32), table((S,), np.float32)
+        self.counts, self.offsets = np.empty((E,), np.int32), np.empty((E + 1,), np.int32)
+        self.perm_slot, self.perm_token = table((S,), np.int32), table((S,), np.int32)
+        self.probabilities, self.log_sum_exp = table((tokens, E), np.float32), table((tokens,), np.float32)
+        self.losses = np.empty((2,), np.float32)
         self.k = k
-        self.c = np.array(ptrs[:8], np.uint64)  # the words of an L.Routing
-        self.losses_ptr = ptrs[8]
+        self.c = np.array([a.ctypes.data for a in (self.expert_of, self.gate_of, self.counts, self.offsets, self.perm_slot,
+                                                   self.perm_token, self.probabilities, self.log_sum_exp)],
+                          np.uint64)  # the words of an L.Routing
+        self.losses_ptr = self.losses.ctypes.data
 
     def cache(self, valid_tokens: Optional[int]) -> MoeCache:
         R = int(self.offsets[-1])

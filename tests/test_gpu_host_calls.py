@@ -113,3 +113,23 @@ print("pool ok")
 """
     done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=100)
     assert done.returncode == 0 and "pool ok" in done.stdout, done.stderr[-2000:]
+
+
+@pytest.mark.parametrize("T", [40, 9000])   # tables in ordinary memory, and in pinned blocks
+def test_a_table_that_is_kept_keeps_no_other_table(device, T):
+    t = synth.make(small_workload(d=64, E=8, k=2, F=64, T=T, seed=84))
+    layer = gpu_layer(device, t)
+    _, cache = layer.forward_train(t.x)
+
+    def memory(a):
+        while isinstance(a.base, np.ndarray):
+            a = a.base
+        return a.ctypes.data, a.ctypes.data + a.nbytes
+
+    names = ("expert_of", "gate_of", "counts", "offsets", "perm_slot", "perm_token", "probabilities", "log_sum_exp")
+    spans = sorted(memory(getattr(cache, n)) for n in names)
+    assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
+    for n in names:
+        lo, hi = memory(getattr(cache, n))
+        assert hi - lo <= 4 * max(T * 8, 9)   # a table's own bytes
+    layer.close()

@@ -206,7 +206,8 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
 // The norm is RmsNorm::forward (src/norm.rs:41-61): the squares are laid down in column order beside the rows and one
 // thread a row adds them up in index order, as the reference does.
 // Measured, against route_fused_kernel (and the norm's launch in front of it): d 768, 203 tokens x 16 experts 9.5 us
-// against 18.1, with the norm 14.4 against 32.2; 4096 x 8 10.5 against 17.7; 8192 x 16 16.2 against 19.6.  Of the 14.4:
+// against 18.1, with the norm 14.4 against 32.2; 4096 x 8 10.5 against 17.7; 8192 x 16 17.3 against 19.0 (median
+// inside a forward 20.9 against 22.8).  Of the 14.4:
 // rows staged 2.8 us into the workgroup, normed at 6.8 (half of it the chain of 768 adds), logits at 9.1, softmax and
 // top-k at 11.2, end 12.3.
 // ---------------------------------------------------------------------------

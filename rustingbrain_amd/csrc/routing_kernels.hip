@@ -1204,6 +1204,20 @@ struct RowsPlan {
     int EG = 0;
     size_t lds = 0;
 };
+// Where the other kernels are faster all the same (blocks of 8 tokens never lose).  Times are forwards of narrow experts,
+// other kernels / this one.
+//   quantized: a dot product is d / 32 steps on 32 threads and the folding of their 32 sums; the shorter the rows and the
+//     more products a workgroup has, the more of it is folding, which logits_q8_kernel (one thread a product) does not have.
+//     16 tokens: d 256, 16 experts 1.03 times as long, 8 experts 0.93; d 384, 32 experts 1.09 / 24 experts 1.00; d 512, 64
+//     experts 1.12, 48 experts 1.07 to 0.95; d 768, 64 experts 0.92.  32 tokens: d 256, 8 experts 1.05, 4 experts 0.96; d 384,
+//     16 experts 1.14 to 1.03; d 512, 24 experts 1.10 to 1.00, 16 experts 1.06 to 0.97; d 768, 32 experts 1.08 to 0.95.
+//   32 tokens, 12 to 24 experts (tiles of 4 x 2): short rows leave too little between the barriers.  bf16 rows, d 256 1.02
+//     to 1.04, d 384 0.98 to 1.02; f32 rows, d 512 1.02 to 1.03, d 768 1.00; 8 experts 1.00, 32 experts 0.7 to 1.0.
+static bool rows_lose(int d, int E, int tokens, bool quantized, bool f32) {
+    if (quantized) return tokens == 16 ? 6 * (E + 28) >= d : 16 * (E + 8) >= d;
+    return tokens == 32 && E > 8 && E < 32 && d <= (f32 ? 512 : 256);
+}
+
 static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     RowsPlan p;
     const int unit = a.wq ? 32 : 8;  // whole turns of the column lanes, whole 16-byte pieces
@@ -1224,10 +1238,13 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
         p.lds = lds();
     }
     if (!p.tokens) return p;
-    // above: the sequences tuned for launches that fill the chip several times over.  Rows so wide that fewer tokens fit
-    // than one workgroup a compute unit needs would take two rounds: route_fused_kernel's slices take one.
+    // above: the sequences tuned for launches that fill the chip several times over.  Below, one round of workgroups or
+    // none, for the chain of a second round is as long as the first's: 9000 tokens, d 512, 8 experts 60.0 us a forward in two
+    // rounds, 57.0 without; 16 experts 63.2 / 57.1, f32 rows 65.8 / 56.7; d 512, 4 experts, two workgroups a unit 55.5 / 61.0.
     const int blocks = (a.T + p.tokens - 1) / p.tokens;
-    if ((long long)a.T * a.E > 256 * 1024 || blocks > (p.tokens == kRouterTokens ? 512 : 256)) p.tokens = 0;
+    const int together = p.tokens == kRouterTokens && 2 * p.lds <= (size_t)kMaxRouterLds ? 512 : 256;
+    if ((long long)a.T * a.E > 256 * 1024 || blocks > together) p.tokens = 0;
+    if (p.tokens > kMinRouterTokens && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
     return p;
 }
 

@@ -14,6 +14,9 @@ SHAPES = [
     dict(d=64, E=5, k=2, T=33),       # 8 tokens a workgroup, the last one short
     dict(d=64, E=16, k=3, T=2049),    # the first call with 16 tokens a workgroup
     dict(d=64, E=9, k=2, T=4097),     # ... and with 32
+    dict(d=544, E=9, k=2, T=2049),    # ... rows long enough for the quantized router's 16 tokens
+    dict(d=544, E=9, k=2, T=4097),    # ... and 32
+    dict(d=544, E=9, k=2, T=8193),    # a second round of workgroups would start: another kernel
     dict(d=1024, E=64, k=6, T=40),    # router rows in groups
     dict(d=1024, E=16, k=2, T=4100),  # 32 tokens do not fit, the norm takes a launch of its own
     dict(d=320, E=12, k=2, T=300),    # lanes of 40 steps (8 lanes) and of 10: a last piece with zeros (32 lanes)

@@ -990,13 +990,22 @@ Work work_of_layer(const rbmoe_layer* L) {
 
 // Whether a decode-shaped call of T tokens should take every expert's products without waiting for the routing: when most
 // experts are about to be touched, or when the weights fetched for nothing cost less than the launch and the chain in
-// front of the products that this saves (about 8 us: 24 MB at the 3 to 4 TB/s these launches reach).
-bool decode_front_pays(const rbmoe_layer* L, int T) {
+// front of the products that this saves.  us, routing in front / beside, at so many MB expected for nothing (top-2 of 8 to
+// 32 experts):
+//   bf16: d 512, 26 18.0 / 12.4; d 768, 29 18.3 / 15.2, 39 18.0 / 15.0, 47 26.3 / 25.7, 61 23.6 / 24.3, 80 19.6 / 22.8; d 512,
+//     41 20.8 / 20.1, 46 19.9 / 20.0, 53 19.1 / 19.9; d 256, 41 24.5 / 25.0.
+//   int8 (widened on the way, so a byte takes longer): d 512, 27 19.5 / 16.1, 30 19.0 / 15.8; d 768, 40 20.1 / 18.6; d 1024,
+//     top-4, 22 25.8 / 25.7, 29 24.6 / 25.5, 39 23.8 / 25.3, 52 22.1 / 24.3.
+//   where the routing alone would not hold its rows in LDS its chain grows with the tokens.  32 experts: d 768 of 704, 1
+//     token, 97 23.7 / 25.6, 2, 91 24.8 / 25.4, 3, 86 31.2 / 25.5, 8, 62 37.0 / 27.6; d 1024, 2, 106 35.4 / 33.4, 3, 93 50.5 /
+//     33.9; d 768 of 1408, 3, 189 31.0 / 40.0; 64 experts, d 1024, top-6, 8, 126 72.2 / 75.7.
+bool decode_front_pays(const rbmoe_layer* L, int T, bool stages_rows) {
     const rbmoe_config& c = L->cfg;
     const double E = c.num_experts, k = c.experts_per_token;
     if (T * k >= 2 * E) return true;
     const double untouched = E * std::pow(1.0 - k / E, T);
-    return untouched * 3.0 * L->Fw * c.d_model * dtype_size(c.weight_dtype) <= 24e6;
+    const double cost = untouched * 3.0 * L->Fw * c.d_model * (c.weight_dtype == RBMOE_I8 ? 1.5 : 2.0);
+    return cost <= (stages_rows ? 42e6 : std::max(42e6, 36e6 * std::min(T, 3)));
 }
 
 // Whether a few tokens' call is better off on the decode-shaped kernels than on the large-batch sequence, whose routing
@@ -1145,7 +1154,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     }
     // the routing beside the gate/up products, in one launch
     bool front = small && L->decode_front && L->hall.p != nullptr && decode_front_ok(ra, abf) &&
-                 (!L->router_q8 || wk == WeightKind::I8) && decode_front_pays(L, T);
+                 (!L->router_q8 || wk == WeightKind::I8) && decode_front_pays(L, T, stages_rows);
     // (a caller without allocations, or one who switched the combined launch off, asked for these kernels by name)
     const bool choose = !static_scratch && L->decode_front;
     const bool batch = choose && small &&

@@ -8,10 +8,12 @@ from rustingbrain_amd import synth
 
 pytestmark = pytest.mark.gpu
 
-CASES = [  # routing alone in one workgroup: rows that do not fit its LDS, and rows that do
-    (dict(d=1024, E=32, k=1, F=256, T=3), "mfma_bf16_decode"), (dict(d=1024, E=32, k=1, F=256, T=4), "mfma_bf16_stream"),
-    (dict(d=1024, E=32, k=2, F=256, T=9), "mfma_bf16_stream"), (dict(d=512, E=32, k=1, F=1408, T=9), "mfma_bf16_decode"),
-    (dict(d=512, E=32, k=1, F=1408, T=10), "mfma_bf16_stream"),
+CASES = [  # weights expected to be fetched for nothing beside the routing
+    (dict(d=512, E=8, k=2, F=1408, T=1), "mfma_bf16_decode_front"), (dict(d=512, E=16, k=2, F=1408, T=3), "mfma_bf16_decode"),
+    (dict(d=512, E=16, k=2, F=1408, T=4), "mfma_bf16_decode_front"), (dict(d=1024, E=32, k=2, F=256, T=9), "mfma_bf16_decode_front"),
+    # routing alone in one workgroup: rows that do not fit its LDS, and rows that do
+    (dict(d=1024, E=32, k=1, F=640, T=3), "mfma_bf16_decode"), (dict(d=1024, E=32, k=1, F=640, T=4), "mfma_bf16_stream"),
+    (dict(d=512, E=32, k=1, F=1408, T=9), "mfma_bf16_decode"), (dict(d=512, E=32, k=1, F=1408, T=10), "mfma_bf16_stream"),
     # routing beside the products: slots and weights
     (dict(d=1024, E=16, k=4, F=704, T=28), "mfma_bf16_decode_front"), (dict(d=1024, E=16, k=4, F=704, T=29), "mfma_bf16_stream")]
 

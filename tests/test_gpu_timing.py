@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("shape", [dict(d=128, E=8, k=2, F=192, T=700, shared=True),     # large-batch kernels
                                    dict(d=128, E=8, k=2, F=192, T=16, shared=True),      # decode-shaped, routing beside
-                                   dict(d=256, E=40, k=2, F=640, T=8),                   # decode-shaped, routing in front
+                                   dict(d=256, E=40, k=2, F=1152, T=8),                  # decode-shaped, routing in front
                                    dict(d=64, E=40, k=2, F=64, T=8)],                    # few slots, little to fetch for nothing
                          ids=["batch", "decode_front", "decode", "decode_front_few_slots"])
 def test_measuring_entry_points_leave_the_results_alone(device, shape):

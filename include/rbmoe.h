@@ -132,7 +132,9 @@ const char* rbmoe_last_global_error(void);
  * layer (src/transformer.rs:1263-1296): validates, checks the budget BEFORE
  * allocating (src/param.rs:172-189), allocates weights (zeroed) and workspace.
  * Expert widths between two multiples of a matrix-core tile are stored rounded up (bf16 rows: to 64, at most four
- * times the width; all-f32 layers: to 32, at most twice), which takes that much more memory.  A layer whose rounded
+ * times the width; all-f32 layers: to 32, at most twice), which takes that much more memory.  f32 rows over bf16 or int8
+ * weights are not rounded: at widths off 64 they keep the any-shape kernels and f32 accuracy, at multiples of 64 the
+ * products take a bf16 copy of the rows (RBMOE_OPT_FORCE_GENERIC: f32 accuracy there too, at a thirtieth of the rate).  A layer whose rounded
  * widths are over the budget - here, or when the norm or training mode is added before the first weight - or over a limit
  * of the backward products keeps its true widths and the any-shape kernels instead.  Layers that already hold
  * weights stay as they are: a budget shared by several layers has to allow for their rounded widths. */
@@ -198,9 +200,10 @@ int rbmoe_forward(rbmoe_layer* layer, const void* x, int32_t T, int32_t cols, co
  * kernels run), but every intermediate buffer of the call (probabilities, routing tables, tile table, losses,
  * hidden and expert output rows) lies in a static device array of RBMOE_STATIC_SCRATCH_BYTES that is part of
  * the library's code object, instead of in the workspace that rbmoe_layer_create allocated.  The call makes
- * no hipMalloc, hipFree or other allocating call.
+ * no hipMalloc, hipFree or other allocating call.  (A few tokens over many or wide experts, which rbmoe_forward hands to
+ * the large-batch kernels, stay decode-shaped here: same routing bit for bit, rows equal to their rounding.)
  * Limits: decode-shaped calls only, i.e. 1 to 32 tokens with tokens * num_experts <= 2048 on a layer with bf16
- * or int8 weights whose widths are multiples of 64 (bf16 rows, or f32 rows whose bf16 copy then lies in the
+ * or int8 weights on the matrix-core path (bf16 rows, or f32 rows whose bf16 copy then lies in the
  * array as well), not in training mode; and the buffers of the call (about tokens * experts_per_token *
  * (d_ff + d_model) * 2 bytes, plus the shared expert's rows and the tables) must fit the array.  Anything else is RBMOE_UNSUPPORTED with a message that says which limit was hit.
  * Every call on one GPU, from any layer or context, uses that GPU's one array: calls that overlap in time on
@@ -261,10 +264,11 @@ int rbmoe_forward_block_host(rbmoe_layer* layer, const void* x, int32_t tokens, 
 /* ---- backward pass (MoeLayer::backward, src/moe.rs:348-489) ------------------------------
  * Training mode makes the forward keep what MoeCache keeps for the backward pass (the input,
  * src/moe.rs:133-135; gate and up pre-activations, src/ffn.rs:27-33) and allocates f32 gradient
- * accumulators, the role of Param.grad (src/param.rs).  For every f32 / bf16 layer: bf16 layers with
- * widths that are multiples of 64 and all-f32 layers (multiples of 32) differentiate on the matrix
- * cores, any other shape or dtype mix on plain kernels; int8 layers report RBMOE_UNSUPPORTED, as the
- * reference has no backward for quantized experts (src/ffn.rs:87-93).
+ * accumulators, the role of Param.grad (src/param.rs).  For every f32 / bf16 layer: bf16 layers with a d_model
+ * that is a multiple of 64 and all-f32 layers (32) differentiate on the matrix cores, their expert widths rounded up
+ * (rbmoe_layer_create); f32 rows over bf16 weights do where every width is a multiple of 64; any other shape or dtype
+ * mix on plain kernels; int8 layers report RBMOE_UNSUPPORTED, as the reference has no backward for quantized
+ * experts (src/ffn.rs:87-93).
  * Call it before the weights are set.  A training layer always takes the large-batch kernels. */
 int rbmoe_layer_enable_training(rbmoe_layer* layer);
 

@@ -9,8 +9,8 @@
 //   combine              (the same kernel as the large path)
 //
 // which the layer folds into fewer where the call allows it: the combine into the down launch (the last
-// workgroup of a block of output columns to finish sums it), and - when most experts are about to be touched -
-// the routing into the gate/up launch (decode_front_kernel), behind which the down launch has one row of
+// workgroup of a block of output columns to finish sums it), and - where fetching the untouched experts' weights too
+// costs less than it saves - the routing into the gate/up launch (decode_front_kernel), behind which the down launch has one row of
 // workgroups per expert (decode_down_by_expert_kernel): two launches.  The products are spread over (tile,
 // 32-feature block) workgroups whose waves split the reduction dimension, so that a few hundred kilobytes of
 // weight fragments are in flight per CU and every byte of a touched expert is fetched exactly once per 32-row tile.

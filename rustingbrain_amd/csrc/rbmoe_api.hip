@@ -237,8 +237,8 @@ struct rbmoe_layer {
     // write on the way, hidden and expert rows are bf16, and the combine sums them into f32 again
     bool cast_rows = false;
     bool use_f32_mc = false;   // all-f32 layer on the f32 matrix cores
-    bool decode_path = true;   // few tokens: four launches that stream every touched weight once
-    bool decode_front = true;  // ... three, with the routing beside the gate/up products, when most experts are touched
+    bool decode_path = true;   // few tokens: launches that stream every touched weight once
+    bool decode_front = true;  // ... the routing beside the gate/up products where that pays (decode_front_pays)
     bool shared_beside = true; // large batches: the shared expert's products on the side stream, beside the routing
     bool fused_router = true;  // logits and everything behind them in one launch where the shapes allow
     bool decode_fold = true;   // decode-shaped calls: the combine inside the down launch

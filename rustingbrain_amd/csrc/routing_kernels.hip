@@ -4,6 +4,7 @@
 //   logits_kernel   router logits in the reference's eight-lane `dot` order
 //   router_kernel   softmax, log-sum-exp, deterministic top-k, per-block ranks
 //                   and histogram, per-block partial sums for the auxiliary losses
+//   route_rows_kernel, route_fused_kernel   both in one launch, by calls of up to 256 K pairs (plan_router)
 //   dispatch_kernel prefix scan over blocks and experts, stable permutation
 //                   (slot -> position), optional row gather; block 0 also writes
 //                   the tile table of the grouped products and the two losses

@@ -210,7 +210,7 @@ BY_EXPERT_CASES = [
                          ids=lambda c: "{wt}_d{d}_E{E}_k{k}_F{F}_T{T}_pad-{pad}".format(**c))
 def test_down_launch_by_expert_gives_the_bits_of_the_tile_table_launch(device, env, case):
     """Behind the launch that routes beside the gate/up products, the down launch has one row of workgroups per
-    expert (weights requested at once, the expert's rows read off its token bits behind them, the combine's
+    expert (weights requested at once, the expert's rows read off the slots' experts behind them, the combine's
     positions and gates fetched early): routing tables, losses and outputs are those of the launch that walks the
     tile table, in every bit - three calls in a row, the last one with fewer tokens."""
     T, k, E, d = case["T"], case["k"], case["E"], case["d"]

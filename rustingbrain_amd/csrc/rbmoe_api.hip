@@ -999,13 +999,18 @@ Work work_of_layer(const rbmoe_layer* L) {
 //   where the routing alone would not hold its rows in LDS its chain grows with the tokens.  32 experts: d 768 of 704, 1
 //     token, 97 23.7 / 25.6, 2, 91 24.8 / 25.4, 3, 86 31.2 / 25.5, 8, 62 37.0 / 27.6; d 1024, 2, 106 35.4 / 33.4, 3, 93 50.5 /
 //     33.9; d 768 of 1408, 3, 189 31.0 / 40.0; 64 experts, d 1024, top-6, 8, 126 72.2 / 75.7.
-bool decode_front_pays(const rbmoe_layer* L, int T, bool stages_rows) {
+//   with an RMSNorm in front, which every workgroup of the one launch does again before its products: d 256, 32 experts of
+//     1408, 4 rows, 40 24.5 / 27.0, 8 rows, 41 28.0 / 30.8; d 512, 16 experts of 1408, 2 rows, 40 22.9 / 23.7, 4 rows, 41 24.4
+//     / 26.6, 8 experts, 26 21.7 / 15.4; rows not held: 32 experts, d 1024, 3, 70 52.4 / 38.4, d 768, 3, 86 38.9 / 35.8; 64
+//     experts, top-6, d 512, 4, 93 47.3 / 45.8, d 1024 with a shared expert, 8, 95 72.6 / 75.3, 7, 104 75.0 / 82.7.
+bool decode_front_pays(const rbmoe_layer* L, int T, bool stages_rows, bool normed) {
     const rbmoe_config& c = L->cfg;
     const double E = c.num_experts, k = c.experts_per_token;
     if (T * k >= 2 * E) return true;
     const double untouched = E * std::pow(1.0 - k / E, T);
     const double cost = untouched * 3.0 * L->Fw * c.d_model * (c.weight_dtype == RBMOE_I8 ? 1.5 : 2.0);
-    return cost <= (stages_rows ? 42e6 : std::max(42e6, 36e6 * std::min(T, 3)));
+    const double held = normed ? 38e6 : 42e6;  // what may be fetched for nothing where routing alone holds its rows
+    return cost <= (stages_rows ? held : std::max(held, (normed ? 30e6 : 36e6) * std::min(T, 3)));
 }
 
 // Whether a few tokens' call is better off on the decode-shaped kernels than on the large-batch sequence, whose routing
@@ -1154,7 +1159,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     }
     // the routing beside the gate/up products, in one launch
     bool front = small && L->decode_front && L->hall.p != nullptr && decode_front_ok(ra, abf) &&
-                 (!L->router_q8 || wk == WeightKind::I8) && decode_front_pays(L, T, stages_rows);
+                 (!L->router_q8 || wk == WeightKind::I8) && decode_front_pays(L, T, stages_rows, norm_src != nullptr);
     // (a caller without allocations, or one who switched the combined launch off, asked for these kernels by name)
     const bool choose = !static_scratch && L->decode_front;
     const bool batch = choose && small &&

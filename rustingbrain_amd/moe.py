@@ -253,6 +253,11 @@ class MoeCache:
         return [self.perm_slot[self.offsets[e]:self.offsets[e + 1]] for e in range(len(self.counts))]
 
 
+def _address(a: np.ndarray) -> int:
+    """Where a writable, contiguous array lies.  (``a.ctypes`` takes a microsecond, and a host call asks ten times.)"""
+    return C.addressof(C.c_char.from_buffer(a)) if a.size else 0
+
+
 class _Tables:
     """The host arrays one forward's routing tables are fetched into, each with memory of its own: a caller may keep one
     of them for long."""
@@ -273,10 +278,10 @@ class _Tables:
         self.probabilities, self.log_sum_exp = table((tokens, E), np.float32), table((tokens,), np.float32)
         self.losses = np.empty((2,), np.float32)
         self.k = k
-        self.c = np.array([a.ctypes.data for a in (self.expert_of, self.gate_of, self.counts, self.offsets, self.perm_slot,
-                                                   self.perm_token, self.probabilities, self.log_sum_exp)],
+        self.c = np.array([_address(a) for a in (self.expert_of, self.gate_of, self.counts, self.offsets, self.perm_slot,
+                                                self.perm_token, self.probabilities, self.log_sum_exp)],
                           np.uint64)  # the words of an L.Routing
-        self.losses_ptr = self.losses.ctypes.data
+        self.losses_ptr = _address(self.losses)
 
     def cache(self, valid_tokens: Optional[int]) -> MoeCache:
         R = int(self.offsets[-1])
@@ -438,7 +443,7 @@ class MoeLayer:
             rp = residual.ctypes.data
         t = _Tables(self, rows)
         _check(self._lib.rbmoe_forward_train_begin(self.handle, x.ctypes.data, L.F32, rows, cols, vp, bp, rp, int(block),
-                                                   out.ctypes.data, t.c.ctypes.data, t.losses_ptr), self.device.handle)
+                                                   out.ctypes.data, _address(t.c), t.losses_ptr), self.device.handle)
         try:  # the tables are here; the expert products and the rows are still on their way
             cache = t.cache(rows if valid is None else int(np.count_nonzero(valid)))
         finally:
@@ -507,7 +512,7 @@ class MoeLayer:
 
     def cache(self, tokens: int, valid_tokens: Optional[int] = None) -> MoeCache:
         t = _Tables(self, tokens)
-        _check(self._lib.rbmoe_get_routing(self.handle, t.c.ctypes.data), self.device.handle)
+        _check(self._lib.rbmoe_get_routing(self.handle, _address(t.c)), self.device.handle)
         t.losses[:] = self.losses()
         return t.cache(valid_tokens)
 

@@ -127,7 +127,7 @@ def cpu_baseline(t: synth.Tensors, budget_s: float = 20.0) -> dict:
     on the host cores of this machine.  Only this function touches oracle/."""
     sys.path.insert(0, os.path.join(ROOT, "tests"))
     from helpers import oracle_layer
-    threads = max(1, min(16, os.cpu_count() or 1))   # the GPU box gives one job 16 cores' worth
+    threads = max(1, min(16, os.cpu_count() or 1))   # 16 cores' worth beside one GPU
     layer = oracle_layer(t)
     T = t.x.shape[0]
     layer.forward(t.x, router_bias=t.router_bias, threads=threads)  # warm-up

@@ -1,6 +1,6 @@
-// Grouped expert products for any shape and dtype: the fallback when a shape
-// does not fit the MFMA kernels (tiny widths, odd sizes) and the path for f32
-// and f32-activation layers.  A 16x16 thread block computes a 16x16 output tile
+// Grouped expert products for any shape and dtype: the fallback of bf16 rows where a shape
+// does not fit the matrix-core kernels (model widths and tiny expert widths off the tile, f32
+// weights), and the plain kernels of RBMOE_OPT_FORCE_GENERIC.  A 16x16 thread block computes a 16x16 output tile
 // from 16-wide K slices staged in LDS; accumulation is f32 in index order.  Like the matrix-core
 // kernels, the gate/up launch can keep the pre-activations for a backward pass (`gu_out`), and a
 // down-shaped launch can apply SwiGLU's backward to its rows on the way out (`bw_gu`).

@@ -1,32 +1,36 @@
-// Grouped expert products for all-f32 layers on the f32 matrix cores of gfx950
-// (v_mfma_f32_32x32x2_f32: f32 products, f32 accumulation).
+// Grouped expert products over f32 rows on the bf16 matrix cores of gfx950, at f32 accuracy.
 //
 //   out[row, n] = sum_c a[row, c] * w[expert][n, c]                 (down product)
 //   out[row, n] = silu(a . wgate[n]) * (a . wup[n])                 (gate/up product)
 //
-// A workgroup owns 64 or 32 token rows x 64 output features; a wave owns 32 x 32 of them (gate/up: two
-// accumulators, the gate rows and the matching up rows).  Both operands go global -> LDS by LDS-DMA in slices of SK
-// reduction columns; one 16-byte LDS read per operand feeds four multiplies, the next fragments and the next slices
-// are under way while a fragment is multiplied.  With SPLIT = 2 the workgroup has two groups of 4 waves that take
-// the two halves of every slice and add their accumulators through LDS at the end (group 1 first, then group 0
-// on top: a fixed order): twice the waves for the same tiles, which is what a launch with few tiles needs.
+// An f32 value is the exact sum of three bf16 values, x = x1 + x2 + x3, each the nearest to what the ones before leave
+// (24 bits of mantissa in three times eight, signs included).  Products of bf16 values are exact in f32, so
+//   f32 weights    x w = x1 w1 + x1 w2 + x2 w1 + x1 w3 + x2 w2 + x3 w1 + (less than 2^-25 of |x w|): six multiplies on a
+//                  unit of sixteen times the rate of the f32 one
+//   bf16 weights   x w = x1 w + x2 w + x3 w, exactly: three
+//   int8 weights   the same, the values being exact in bf16; the row's scale multiplies the sum (src/quantized.rs:55-62)
+// with f32 accumulation.  A sum's error is that of its additions, and there are fewer of them than the f32 unit has (one
+// a step of 16 columns for the large terms, the small ones summed apart or with them where the groups share out the
+// steps): hidden rows against 64 bits, d 512, 8 experts of 1408, 1024 tokens, 1.9e-7 where v_mfma_f32_32x32x2 gave 4.3e-7,
+// products over given rows 2.4e-7 / 4.8e-7; bf16 weights, width 352, 3.6e-7 where a chain of fused adds gave 6.2e-7.
+// Rows and weights stay f32 in memory.
 //
-// Exactly two waves a SIMD (amdgpu_waves_per_eu): the kernel needs 86 registers at most, and where more waves may be
-// resident the hardware fills some SIMDs with three or more while others hold one - a kernel of nothing but multiplies
-// falls from 156 to 103 TFLOP/s that way (512 workgroups of 4 waves, one or two accumulators each).  One wave a SIMD
-// leaves a workgroup's first loads and its stores uncovered.  What remains is the clock: the launch runs at 2.16 GHz
-// (multiplies alone on random data: 130-141 TFLOP/s), and the last round of a launch.
-// 1024 tokens, d 512, 8 experts top-2 of width 1408: gate/up 76.6 -> 73.7 us, down 51.6 -> 43.7 us (68 TFLOP/s); 8192
-// tokens: 463 -> 451 and 256 -> 236 us (105 and 100 TFLOP/s).  Same box, against the kernel that staged through
-// registers with one LDS stage, 4-byte fragment reads and three workgroups a compute unit.  One wave a SIMD: 76.8 / 48.8
-// and 469 / 263 us; three: 77.1 / 47.8 and 470 / 244; 32 x 32 tiles with four wave groups 83.8 / 45.6.  A layer's output
-// against 64 bits: 6.46e-7 (6.48e-7 before), 9.16e-7 (the same) at 8192 tokens.
-// Rows are fetched through `row_index`, so the gather of
-// the routed rows (gather_rows, src/moe.rs:658-664) never materialises.  The weight fragment
-// is the matrix-core A operand and the token fragment B, so a lane ends with 4 consecutive
-// features of one token (one 16-byte store).  SiLU uses the exact division: this path is held
-// to 1e-5.  For a backward pass the gate/up launch can also keep the pre-activations (`gu_out`),
-// and a plain launch can apply SwiGLU's backward where it stores its rows (`swiglu_grad_gu`).
+// What bounds it.  A step of a 64 x 64 wave tile is 24 multiplies (768 cycles of the matrix core) and the splitting of two
+// weight fragments (88 vector instructions, 352 cycles).  The rows are split once per workgroup, on their way from registers
+// into three bf16 planes in LDS; weights go to LDS by LDS-DMA as they are and a wave splits its own fragments (nobody else
+// needs them), so they take 4 bytes a value on every path.  Everything of a step sits between its multiplies, one piece
+// behind each (see `step`).  Large launches run at the power limit: 8192 tokens, same layer, gate/up 451 -> 283 us (the
+// six bf16 products at 1000 TFLOP/s, where the library's large bf16 product reaches 1160), down 236 -> 160; 1024 tokens
+// 75 -> 46 and 44 -> 31, against the kernel on the f32 unit.  Small ones are a chain of slices and memory: see f32_tile.
+// f32 rows over bf16 or int8 weights at widths off 64 ran on the any-shape kernel's 20 TFLOP/s: 52 rows, d 768, 32 experts
+// of 352 and a shared one 154 -> 58 us a forward.
+//
+// Rows are fetched through `row_index`, so the gather of the routed rows (gather_rows, src/moe.rs:658-664) never
+// materialises.  The weight fragment is the matrix-core A operand and the token fragment B, so a lane ends with 4
+// consecutive features of one token.  SiLU uses the exact division: this path is held to 1e-5.  For a backward pass the
+// gate/up launch can also keep the pre-activations (`gu_out`), and a plain launch can apply SwiGLU's backward where it
+// stores its rows (`bw_gu`).
+#include <algorithm>
 #include <type_traits>
 
 #include "rbmoe_kernels.h"
@@ -35,42 +39,115 @@ namespace rbmoe {
 
 namespace {
 
-constexpr int FN = 64;   // output features per workgroup (two waves side by side)
-constexpr int FK = 32;   // reduction widths are multiples of this
+constexpr int RING = 3;   // LDS stages of weights
 
-// Loads go to LDS by LDS-DMA, issued from inline assembly: the compiler would drain every load in flight in front of
-// an LDS read otherwise.  A wave deposits 64 pieces of 16 bytes at consecutive LDS addresses.
-__device__ __forceinline__ void f32_issue_dma(uint32_t lds_addr, const float* src) {
+// Every load of the main loop is issued from inline assembly and awaited by a hand-counted vmcnt: the compiler would drain
+// all loads in flight in front of an LDS read otherwise.  An LDS-DMA deposits 64 pieces of 16 bytes at consecutive
+// addresses.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void f32_issue_dma(uint32_t lds_addr, const void* src) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_addr), "v"(src) : "memory");
 }
-template <int N>
-__device__ __forceinline__ void f32_wait_outstanding() {
-    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+__device__ __forceinline__ void f32_issue_load(u32x4& d, const void* src) {
+    asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(d) : "v"(src));
 }
 
-// FM = token rows per workgroup, 64 or 32 (FM / 32 x 2 waves per group); SPLIT = wave groups; SK = reduction columns of
-// a slice, SK / SPLIT of them multiplied by each wave group; STAGES = LDS stages of one slice each
-template <bool SWIGLU, int FM, int SPLIT, int SK, int STAGES>
-__global__ __launch_bounds__(FM * 4 * SPLIT) __attribute__((amdgpu_waves_per_eu(2, 2))) void grouped_f32_kernel(
-    const float* __restrict__ a, const int* __restrict__ row_index, const float* __restrict__ w,
-    size_t w_expert_stride, int N, int K, const int* __restrict__ tile_expert, const int* __restrict__ tile_row0,
-    const int* __restrict__ tile_rows, const int* __restrict__ ntiles, int dense_rows, float* __restrict__ out,
-    float* __restrict__ gu_out, const float* __restrict__ bw_gu) {
-    constexpr int WR = SWIGLU ? 2 * FN : FN;  // weight rows staged per slice
-    constexpr int WPG = FM / 32 * 2;          // waves per group
-    constexpr int NTH = 64 * WPG * SPLIT;     // threads
-    constexpr int NW = NTH / 64;
-    constexpr int PPR = SK / 4;               // 16-byte pieces per staged row: 4 or 8
-    constexpr int STAGE = (FM + WR) * SK;     // floats of a stage: token rows, then weight rows
-    constexpr int STEPS = SK / SPLIT / 8;     // fragment reads (four multiplies deep) per slice and wave
-    constexpr int DMA = (FM + WR) * PPR / 64 / NW;  // LDS-DMA instructions per wave and slice
-    static_assert(DMA * 64 * NW == (FM + WR) * PPR && STEPS % 2 == 0, "whole instructions, two fragment sets in turn");
-    __shared__ __attribute__((aligned(16))) float lds[STAGES * STAGE];
+template <int I, int N, typename F>
+__device__ __forceinline__ void f32_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        f32_for<I + 1, N>(f);
+    }
+}
+
+// Two f32 values as three pairs of bf16: nearest, nearest of the rest, the rest.
+__device__ __forceinline__ void split2(float x, float y, uint32_t& a, uint32_t& b, uint32_t& c) {
+    a = pack2(x, y);
+    const float x1 = x - __uint_as_float(a << 16), y1 = y - __uint_as_float(a & 0xffff0000u);
+    b = pack2(x1, y1);
+    c = pack2(x1 - __uint_as_float(b << 16), y1 - __uint_as_float(b & 0xffff0000u));
+}
+
+// Rows of 16 * PP bytes lie in LDS one behind the other; position p of row r holds piece p ^ row_swizzle<PP>(r), so that 16
+// lanes that read one logical piece of 16 rows touch distinct banks (256 bytes of them).
+template <int PP>
+__device__ __forceinline__ int row_swizzle(int r) {
+    static_assert((PP & (PP - 1)) == 0 && PP <= 16, "");
+    return (r / (16 / PP)) & (PP - 1);
+}
+
+// A wave's weight fragment of one step: READS 16-byte (int8: 8-byte) LDS reads of a row, PARTS bf16 operands out of CHUNKS
+// turns of conversion.
+template <typename WT>
+struct Weights;
+template <>
+struct Weights<float> {
+    static constexpr int PARTS = 3, PIECE = 4, READS = 2, CHUNKS = 4, COST = 11;
+    float v[8];
+    __device__ __forceinline__ void read(int i, const unsigned char* row, int step, int half, int sw) {
+        const float4 q = *reinterpret_cast<const float4*>(row + 16 * ((4 * step + 2 * half + i) ^ sw));
+        v[4 * i] = q.x; v[4 * i + 1] = q.y; v[4 * i + 2] = q.z; v[4 * i + 3] = q.w;
+    }
+    __device__ __forceinline__ void convert(int i, uint32_t (&o)[3][4]) const { split2(v[2 * i], v[2 * i + 1], o[0][i], o[1][i], o[2][i]); }
+};
+template <>
+struct Weights<bf16_t> {
+    static constexpr int PARTS = 1, PIECE = 8, READS = 1, CHUNKS = 1, COST = 0;
+    uint4 v;
+    __device__ __forceinline__ void read(int, const unsigned char* row, int step, int half, int sw) {
+        v = *reinterpret_cast<const uint4*>(row + 16 * ((2 * step + half) ^ sw));
+    }
+    __device__ __forceinline__ void convert(int, uint32_t (&o)[1][4]) const { o[0][0] = v.x; o[0][1] = v.y; o[0][2] = v.z; o[0][3] = v.w; }
+};
+template <>
+struct Weights<int8_t> {
+    static constexpr int PARTS = 1, PIECE = 16, READS = 1, CHUNKS = 2, COST = 6;
+    uint2 v;
+    __device__ __forceinline__ void read(int, const unsigned char* row, int step, int half, int sw) {
+        v = *reinterpret_cast<const uint2*>(row + 16 * (step ^ sw) + 8 * half);
+    }
+    __device__ __forceinline__ void convert(int i, uint32_t (&o)[1][4]) const {
+        const uint32_t q = i ? v.y : v.x;
+        o[0][2 * i] = widen2(q, 0);
+        o[0][2 * i + 1] = widen2(q, 16);
+    }
+};
+__device__ __forceinline__ float weight_value(float v) { return v; }
+__device__ __forceinline__ float weight_value(bf16_t v) { return to_f32(v); }
+__device__ __forceinline__ float weight_value(int8_t v) { return (float)v; }
+
+// `sub`: this kernel's tiles in one of the tile table's, 1 or 2.  TB = blocks of 32 token rows per workgroup; FW = waves along the features (the workgroup owns 32 FW of them, or with
+// SWIGLU as many gate and up rows each), STEPS = steps of 16 reduction columns a wave takes of a slice.  DMA: rows of whole
+// 16-byte pieces on 16-byte boundaries and whole slices; otherwise both operands travel element by element.
+template <typename WT, bool SWIGLU, int NW, int TB, int FW, int STEPS, bool DMA>
+__global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
+    const float* __restrict__ a, const int* __restrict__ row_index, const WT* __restrict__ w, size_t w_expert_stride,
+    const float* __restrict__ scales, size_t s_expert_stride, int N, int K, const int* __restrict__ tile_expert,
+    const int* __restrict__ tile_row0, const int* __restrict__ tile_rows, const int* __restrict__ ntiles, int sub, int dense_rows,
+    float* __restrict__ out, float* __restrict__ gu_out, const float* __restrict__ bw_gu) {
+    typedef Weights<WT> W;
+    constexpr int NTH = NW * 64;
+    constexpr int KG = NW / FW;                   // wave groups that share out a slice's steps
+    constexpr int FN = 32 * FW;
+    constexpr int NB = SWIGLU ? 2 : 1;            // blocks of 32 weight rows a wave: gate and up, or plain
+    constexpr int WR = NB * FN;                   // weight rows staged per slice
+    constexpr int BM = 32 * TB;
+    constexpr int SK = 16 * STEPS * KG;           // reduction columns of a slice
+    constexpr int WROW = SK * (int)sizeof(WT), WPP = WROW / 16, TPP = SK / 8;  // pieces of a weight row, of a row of a plane
+    constexpr int WSTAGE = WR * WROW, PLANE = BM * SK * 2, PBUF = 3 * PLANE;
+    constexpr int WINST = WSTAGE / 1024;          // LDS-DMA instructions of a slice
+    constexpr int DW = (WINST + NW - 1) / NW;     // ... a wave (waves left without one repeat another's)
+    constexpr int TPIECES = BM * SK / 4;          // 16-byte pieces of raw token rows of a slice
+    constexpr int NT = (TPIECES + NTH - 1) / NTH; // ... a thread (threads left without one repeat another's)
+    constexpr int LOOP_BYTES = RING * WSTAGE + 2 * PBUF, MEET_BYTES = KG > 1 ? NW * NB * TB * 16 * 64 * 4 : 0;
+    constexpr int LDS_BYTES = LOOP_BYTES > MEET_BYTES ? LOOP_BYTES : MEET_BYTES;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];
+    unsigned char* const planes = lds + RING * WSTAGE;
 
     // ---- which tile: each XCD (workgroup number mod 8) walks a contiguous range of tiles with one expert's row tiles
-    // innermost, so that a weight slice is fetched by one L2 (in grid order every slice was fetched by four or eight)
+    // innermost, so that a weight slice is fetched by one L2
     const int tiles_n = (N + FN - 1) / FN;
-    const int tiles_m = dense_rows >= 0 ? (dense_rows + FM - 1) / FM : *ntiles;
+    const int tiles_m = dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles * sub;
     const int total = tiles_m * tiles_n;
     const int per_xcd = (total + 7) / 8;
     const int local = blockIdx.x >> 3;
@@ -88,232 +165,528 @@ __global__ __launch_bounds__(FM * 4 * SPLIT) __attribute__((amdgpu_waves_per_eu(
     int expert, row0, rows;
     if (dense_rows >= 0) {
         expert = 0;
-        row0 = tm_idx * FM;
-        rows = min(FM, dense_rows - row0);
+        row0 = tm_idx * BM;
+        rows = min(BM, dense_rows - row0);
     } else {
-        expert = tile_expert[tm_idx];
-        row0 = tile_row0[tm_idx];
-        rows = tile_rows[tm_idx];
+        const int entry = sub == 2 ? tm_idx >> 1 : tm_idx, skip = sub == 2 ? (tm_idx & 1) * BM : 0;
+        expert = tile_expert[entry];
+        row0 = tile_row0[entry] + skip;
+        rows = min(BM, tile_rows[entry] - skip);
+        if (rows <= 0) return;
     }
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave = wv % WPG;
-    const int grp = wv / WPG;                 // wave group: which part of each slice it multiplies
-    const int wy = wave >> 1, wx = wave & 1;  // token half, feature half
-    const float* wbase = w + (size_t)expert * w_expert_stride;
+    const int fw = wv % FW, grp = wv / FW;    // which 32 features; which steps of every slice
+    const int lr = lane & 31, lh = lane >> 5;
+    const WT* const wbase = w + (size_t)expert * w_expert_stride;
+    // (rows past the end of the group, features past N: any valid one, products never stored)
+    auto token_row = [&](int r) {
+        const int rr = r < rows ? r : 0;
+        return a + (size_t)(row_index ? row_index[row0 + rr] : row0 + rr) * K;
+    };
+    auto weight_row = [&](int q) {  // q < FN: gate (or plain) feature n0 + q; q >= FN: the matching up row
+        const int feat = n0 + (q % FN);
+        const int fr = feat < N ? feat : 0;
+        return wbase + (size_t)((SWIGLU && q >= FN) ? N + fr : fr) * K;
+    };
 
-    // ---- staging: instruction i of a wave fills LDS pieces 64 (wv DMA + i) .. + 63 of the stage.  Rows cannot be
-    // padded apart, so position q of row r holds piece q ^ swz(r): the 16 rows that 16 lanes of a fragment read touch
-    // at one logical piece then lie in 64 distinct banks.
-    auto swz = [](int r) { return PPR == 8 ? ((r >> 1) & 7) : ((r >> 2) & 3); };
-    const float* src[DMA];
+    // ---- staging
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+    const WT* wsrc[DMA ? DW : 1];
+    const float* tsrc[NT];
+    int tcol[NT];
+    unsigned char* tdst[NT];
+    constexpr int NWE = DMA ? 1 : WR * SK / NTH;
+    WT pend_w[NWE];
+    u32x4 pend_t[2][NT];  // raw row values of two slices under way
+    if constexpr (DMA) {
 #pragma unroll
-    for (int i = 0; i < DMA; ++i) {
-        const int p = (wv * DMA + i) * 64 + lane;
-        const int r = p / PPR;                    // row of the stage
-        const int c = 4 * ((p % PPR) ^ swz(r));   // swz(FM + r) == swz(r): FM is a multiple of 16
-        if (r < FM) {
-            const int rr = r < rows ? r : 0;  // rows past the end of the group: products never stored
-            const int grow = row_index ? row_index[row0 + rr] : row0 + rr;
-            src[i] = a + (size_t)grow * K + c;
-        } else {
-            // weight row q < FN: gate (or plain) feature n0 + q; q >= FN: the matching up row
-            const int q = r - FM;
-            const int feat = n0 + (q % FN);
-            const int fr = feat < N ? feat : 0;
-            src[i] = wbase + (size_t)((SWIGLU && q >= FN) ? N + fr : fr) * K + c;
+        for (int i = 0; i < DW; ++i) {
+            const int p = ((wv * DW + i) % WINST) * 64 + lane, r = p / WPP;
+            wsrc[i] = weight_row(r) + W::PIECE * ((p % WPP) ^ row_swizzle<WPP>(r));
         }
     }
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + (uint32_t)wv * (DMA * 1024);
-    const int KT = K / SK;
-    auto dma = [&](int kt, int stage) {
-        const int k0 = min(kt, KT - 1) * SK;  // past the end: fetched again and never read, so that the wait counts hold
 #pragma unroll
-        for (int i = 0; i < DMA; ++i) f32_issue_dma(lds0 + (uint32_t)(stage * (STAGE * 4) + i * 1024), src[i] + k0);
+    for (int i = 0; i < NT; ++i) {
+        const int p = (i * NTH + tid) % TPIECES, r = p / (SK / 4), c = p % (SK / 4);
+        tsrc[i] = token_row(r);
+        tcol[i] = 4 * c;
+        tdst[i] = planes + r * (SK * 2) + 16 * ((c >> 1) ^ row_swizzle<TPP>(r)) + 8 * (c & 1);
+    }
+    const int KT = (K + SK - 1) / SK;
+    // (slices past the last only keep the wait counts: fetched again and never read)
+    auto dma_w = [&](int i, int kt, int slot) {
+        f32_issue_dma(lds0 + (uint32_t)(slot * WSTAGE + ((wv * DW + i) % WINST) * 1024), wsrc[i] + min(kt, KT - 1) * SK);
     };
-
-    floatx16 acc0, acc1;
+    auto load_t = [&](int i, int kt, u32x4& to) {
+        if constexpr (DMA) {
+            f32_issue_load(to, tsrc[i] + min(kt, KT - 1) * SK + tcol[i]);
+        } else {
+            const int c = kt * SK + tcol[i];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc0[v] = acc1[v] = 0.0f;
-
-    // ---- fragments: one 16-byte read per operand feeds four multiplies.  Lane l reads row l % 32 of the wave's block,
-    // the columns 8 s + 4 (l / 32) .. + 3 of the group's share of the slice; multiply j takes column j of both halves
-    // (both operands in the same order, so the product is the same sum).
-    const int frow = lane & 31, fhalf = lane >> 5;
-    const int fsw = swz(frow);
-    const float* const a_rows = lds + (wy * 32 + frow) * SK;
-    const float* const w_rows = lds + (FM + wx * 32 + frow) * SK;
-    struct Frag {
-        float4 t, g, u;
-    } fr[2];
-    auto read = [&](Frag& f, int stage, int s) {
-        const int o = stage * STAGE + 4 * ((grp * (PPR / SPLIT) + 2 * s + fhalf) ^ fsw);
-        f.t = *reinterpret_cast<const float4*>(a_rows + o);
-        f.g = *reinterpret_cast<const float4*>(w_rows + o);
-        if constexpr (SWIGLU) f.u = *reinterpret_cast<const float4*>(w_rows + FN * SK + o);
+            for (int q = 0; q < 4; ++q) {
+                const float v = tsrc[i][min(c + q, K - 1)];
+                to[q] = c + q < K ? __float_as_uint(v) : 0u;  // (columns past the end of a row count as zero)
+            }
+        }
     };
-    auto mul = [&](float g, float u, float t) {
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(g, t, acc0, 0, 0, 0);
-        if constexpr (SWIGLU) acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(u, t, acc1, 0, 0, 0);
+    auto load_w = [&](int kt) {
+        if constexpr (!DMA) {
+#pragma unroll
+            for (int i = 0; i < NWE; ++i) {
+                const int e = i * NTH + tid;
+                pend_w[i] = weight_row(e / SK)[min(kt * SK + e % SK, K - 1)];
+            }
+        }
+    };
+    auto put_w = [&](int slot) {
+        if constexpr (!DMA) {
+#pragma unroll
+            for (int i = 0; i < NWE; ++i) {
+                const int e = i * NTH + tid, r = e / SK, c = e % SK;
+                reinterpret_cast<WT*>(lds + slot * WSTAGE + r * WROW + 16 * ((c / W::PIECE) ^ row_swizzle<WPP>(r)))[c % W::PIECE] = pend_w[i];
+            }
+        }
+    };
+    // the rows' planes: [buffer][plane][row][SK / 8 pieces of 8 bf16]
+    uint32_t cv[3][2];
+    auto split_t = [&](int half, const u32x4& v) {
+        split2(__uint_as_float(half ? v.z : v.x), __uint_as_float(half ? v.w : v.y), cv[0][half], cv[1][half], cv[2][half]);
+    };
+    auto put_t = [&](int i, int buf) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(tdst[i] + buf * PBUF + p * PLANE) = make_uint2(cv[p][0], cv[p][1]);
     };
 
-    // ---- main loop.  The one barrier of a slice stands in front of its last step, whose fragments are in registers by
-    // then: before it a wave waits for its own DMA of the next slice (loads retire in order; STAGES - 2 younger slices
-    // may be in flight), behind it the next slice is complete, its first fragments are read during this slice's last
-    // multiplies, and this slice's stage, which nobody reads any more, takes the DMA of slice kt + STAGES.
-    for (int i = 0; i < STAGES; ++i) dma(i, i);
-    f32_wait_outstanding<(STAGES - 1) * DMA>();
+    // Six terms a step are six roundings of a sum where the f32 unit has eight; the five small ones are therefore summed
+    // apart, where a rounding is 2^-8 of one of the large sum's, unless the wave groups share out the steps anyway.
+    constexpr bool APART = W::PARTS == 3 && KG == 1;
+    floatx16 acc[NB][TB], low[NB][TB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int t = 0; t < TB; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[nb][t][v] = low[nb][t][v] = 0.0f;
+
+    // ---- fragments of one step
+    struct Operands {
+        uint4 t[TB][3];
+        uint32_t w[NB][W::PARTS][4];
+    };
+    W wraw[NB];
+    const int wsw = row_swizzle<WPP>(lr), tsw = row_swizzle<TPP>(lr);  // (32 rows on, the same)
+    const unsigned char* const wrow = lds + (fw * 32 + lr) * WROW;
+    const unsigned char* const trow = planes + lr * (SK * 2);
+    auto read_t = [&](Operands& o, int i, int buf, int s) {
+        const int t = i / 3, p = i % 3;
+        o.t[t][p] = *reinterpret_cast<const uint4*>(trow + buf * PBUF + p * PLANE + t * (32 * SK * 2) + 16 * ((2 * (grp * STEPS + s) + lh) ^ tsw));
+    };
+    auto read_w = [&](int i, int slot, int s) {
+        const int nb = i / W::READS;
+        wraw[nb].read(i % W::READS, wrow + slot * WSTAGE + nb * (FN * WROW), grp * STEPS + s, lh, wsw);
+    };
+    // term number i of a product, the smallest first: which part of the weight, which of the row
+    constexpr int TERMS = W::PARTS == 3 ? 6 : 3;
+    auto multiply = [&](auto m_tag, const Operands& o) {
+        constexpr int m = decltype(m_tag)::value, term = m / (NB * TB), nb = m / TB % NB, t = m % TB;
+        constexpr int wp = W::PARTS == 3 ? (term == 0 ? 2 : (term == 1 || term == 3) ? 1 : 0) : 0;
+        constexpr int tp = W::PARTS == 3 ? (term == 2 ? 2 : (term == 1 || term == 4) ? 1 : 0) : 2 - term;
+        const uint4 wf = make_uint4(o.w[nb][wp][0], o.w[nb][wp][1], o.w[nb][wp][2], o.w[nb][wp][3]);
+        floatx16& sum = APART && term < TERMS - 1 ? low[nb][t] : acc[nb][t];
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wf), __builtin_bit_cast(bf16x8, o.t[t][tp]), sum, 0, 0, 0);
+    };
+
+    // ---- one step: its multiplies with everything else between them, each piece behind a multiply of its own (the order is
+    // pinned): the reads of the next step's fragments; with FETCH the weights of slice kt + 3 under way; with CONV the rows
+    // of slice `ck` from registers to their planes and those of slice ck + 2 under way; the split of the next step's weights
+    auto step = [&](auto fetch_tag, auto conv_tag, const Operands& cur, Operands& nxt, int rslot, int rbuf, int rs, int kt,
+                    int fslot, int ck, u32x4 (&set)[NT]) {
+        constexpr bool FETCH = decltype(fetch_tag)::value, CONV = decltype(conv_tag)::value;
+        constexpr int NM = NB * TB * TERMS;
+        constexpr int RW = NB * W::READS, RT = 3 * TB, F = FETCH && DMA ? DW : 0, C = CONV ? 3 * NT : 0, X = NB * W::CHUNKS;
+        constexpr int OPS = RW + RT + F + C + X;
+        constexpr int COST = RW + RT + 4 * F + 10 * C + W::COST * X;
+        auto before = [](int i) constexpr {  // cost of what comes in front of operation i
+            int c = 0;
+            for (int j = 0; j < i; ++j)
+                c += j < RW + RT ? 1 : j < RW + RT + F ? 4 : j < RW + RT + F + C ? 10 : W::COST;
+            return c;
+        };
+        auto op = [&](auto i_tag) {
+            constexpr int i = decltype(i_tag)::value;
+            if constexpr (i < RW) {
+                read_w(i, rslot, rs);
+            } else if constexpr (i < RW + RT) {
+                read_t(nxt, i - RW, rbuf, rs);
+            } else if constexpr (i < RW + RT + F) {
+                dma_w(i - RW - RT, kt + 3, fslot);
+            } else if constexpr (i < RW + RT + F + C) {
+                constexpr int j = i - RW - RT - F, u = j / 3;
+                if constexpr (j % 3 < 2) {
+                    split_t(j % 3, set[u]);
+                } else {
+                    put_t(u, ck & 1);
+                    load_t(u, ck + 2, set[u]);
+                }
+            } else {
+                constexpr int j = i - RW - RT - F - C;
+                wraw[j / W::CHUNKS].convert(j % W::CHUNKS, nxt.w[j / W::CHUNKS]);
+            }
+        };
+        if constexpr (FETCH && !DMA) {
+            put_w(fslot == 0 ? 2 : fslot - 1);  // slice kt + 2
+            load_w(kt + 3);
+        }
+        f32_for<0, NM>([&](auto m_tag) {
+            constexpr int m = decltype(m_tag)::value;
+            multiply(m_tag, cur);
+            __builtin_amdgcn_sched_barrier(0);
+            f32_for<0, OPS>([&](auto i_tag) {
+                constexpr int at = COST == 0 ? 0 : before(decltype(i_tag)::value) * NM / (COST + 1);
+                if constexpr (at == m) op(i_tag);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+
+    // ---- pipeline.  The barrier of a slice stands in front of its last step: by then every wave has read all of the slice's
+    // fragments, and behind it the next slice is complete in LDS.  Loads retire in order: of what was issued since the last
+    // barrier nothing need have landed, of what was issued before that all must (weights of the next slice, row values of
+    // the next conversion).
+    constexpr bool ONE = STEPS == 1;
+    // Everything that the first slices need is requested at once: the rows of slices 0 and 1 (or 0 alone) in registers of
+    // their own, those of the next two where the loop takes them from - set p holds the slice that the conversions in the
+    // slices of parity p (or, with two steps, of the other parity) take next.
+    u32x4 first[2][NT];
+    f32_for<0, NT>([&](auto i) { load_t(i, 0, first[0][i]); });
+    if constexpr (ONE) f32_for<0, NT>([&](auto i) { load_t(i, 1, first[1][i]); });
+    auto first_w = [&](int k) {
+        if constexpr (DMA) {
+#pragma unroll
+            for (int i = 0; i < DW; ++i) dma_w(i, k, k);
+        } else {
+            load_w(k);
+            if (k < 2) put_w(k);
+        }
+    };
+    first_w(0);
+    f32_for<0, NT>([&](auto i) { load_t(i, 2, pend_t[0][i]); });
+    f32_for<0, NT>([&](auto i) { load_t(i, ONE ? 3 : 1, pend_t[1][i]); });
+    first_w(1);
+    first_w(2);
+    auto wait = [&](auto n_tag) {
+#pragma unroll
+        for (int i = 0; i < NT; ++i) asm volatile("" : "+v"(pend_t[0][i]), "+v"(pend_t[1][i]));
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(decltype(n_tag)::value) : "memory");
+#pragma unroll
+        for (int i = 0; i < NT; ++i) asm volatile("" : "+v"(pend_t[0][i]), "+v"(pend_t[1][i]));
+    };
+    typedef std::integral_constant<int, 0> All;
+    typedef std::integral_constant<int, DMA ? DW + NT : 63> Older;
+    wait(std::integral_constant<int, DMA ? 2 * NT + 2 * DW : 63>{});
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        asm volatile("" : "+v"(first[0][i]));
+        if constexpr (ONE) asm volatile("" : "+v"(first[1][i]));
+    }
+    auto convert_now = [&](int buf) {
+        f32_for<0, NT>([&](auto i) {
+            split_t(0, first[buf][i]);
+            split_t(1, first[buf][i]);
+            put_t(i, buf);
+        });
+    };
+    convert_now(0);
+    if constexpr (ONE) convert_now(1);
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    read(fr[0], 0, 0);
-    int st = 0;
-    for (int kt = 0; kt < KT; ++kt) {
-        const int nx = st + 1 == STAGES ? 0 : st + 1;
-#pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            Frag& cur = fr[s & 1];
-            if (s == STEPS - 1) {
-                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"((STAGES - 2) * DMA) : "memory");
-                __builtin_amdgcn_s_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-                read(fr[0], nx, 0);
-                dma(kt + STAGES, st);
-            } else {
-                read(fr[(s + 1) & 1], st, s + 1);
-            }
+    Operands oa, ob;
+    f32_for<0, NB * W::READS>([&](auto i) { read_w(i, 0, 0); });
+    f32_for<0, 3 * TB>([&](auto i) { read_t(oa, i, 0, 0); });
+    f32_for<0, NB * W::CHUNKS>([&](auto i) { wraw[i / W::CHUNKS].convert(i % W::CHUNKS, oa.w[i / W::CHUNKS]); });
+    wait(All{});
+    int s0 = 0;  // kt % RING
+    typedef std::true_type Yes;
+    typedef std::false_type No;
+    auto slice = [&](int kt, auto par_tag, Operands& c, Operands& n) {
+        constexpr int par = decltype(par_tag)::value;  // kt % 2
+        const int s1 = s0 == 2 ? 0 : s0 + 1;
+        if constexpr (ONE) {
+            wait(Older{});
+            __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
-            mul(cur.g.x, SWIGLU ? cur.u.x : 0.0f, cur.t.x);
-            mul(cur.g.y, SWIGLU ? cur.u.y : 0.0f, cur.t.y);
-            mul(cur.g.z, SWIGLU ? cur.u.z : 0.0f, cur.t.z);
-            mul(cur.g.w, SWIGLU ? cur.u.w : 0.0f, cur.t.w);
+            step(Yes{}, Yes{}, c, n, s1, par ^ 1, 0, kt, s0, kt + 2, pend_t[par]);
+        } else {
+            static_assert(STEPS <= 2, "one step in front of the barrier");
+            step(No{}, Yes{}, c, n, s0, par, 1, kt, 0, kt + 1, pend_t[par ^ 1]);
+            wait(Older{});
+            __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
+            step(Yes{}, No{}, n, c, s1, par ^ 1, 0, kt, s0, 0, pend_t[0]);
         }
-        st = nx;
+        s0 = s1;
+    };
+    typedef std::integral_constant<int, 0> Even;
+    typedef std::integral_constant<int, 1> Odd;
+    int kt = 0;
+    for (; kt + 2 <= KT; kt += 2) {
+        slice(kt, Even{}, oa, ob);
+        if constexpr (ONE) slice(kt + 1, Odd{}, ob, oa);
+        else slice(kt + 1, Odd{}, oa, ob);
     }
-    f32_wait_outstanding<0>();  // the LDS is used again below, and nothing may land after the workgroup has ended
+    if (kt < KT) slice(kt, Even{}, oa, ob);
+    wait(All{});  // the LDS is used again below, and nothing may land after the workgroup has ended
     __syncthreads();
 
-    if constexpr (SPLIT > 1) {
-        // the two groups' sums meet in LDS (the staging tiles are free: the loop's last barrier is behind us)
-        static_assert(STAGES * STAGE >= (SWIGLU ? 2 : 1) * WPG * 16 * 64, "room for the accumulators");
-        float* const r0 = lds + wave * (16 * 64) + lane;
-        float* const r1 = r0 + WPG * 16 * 64;
-        // groups SPLIT - 1 ... 1 hand their sums down one after the other; group 0 adds the last and stores
+    // ---- wave groups that share out the reduction meet in LDS: group g finishes quads (four values) g OQ .. + OQ - 1 of the
+    // wave's TB * 4, the groups' shares summed in their order
+    constexpr int OQ = TB * 4 / KG;
+    float mine[NB][OQ][4];
+    if constexpr (KG > 1) {
+        float4* const ex = reinterpret_cast<float4*>(lds);
 #pragma unroll
-        for (int gsrc = SPLIT - 1; gsrc >= 1; --gsrc) {
-            if (grp == gsrc) {
+        for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    r0[v * 64] = acc0[v];
-                    if constexpr (SWIGLU) r1[v * 64] = acc1[v];
+            for (int q = 0; q < TB * 4; ++q) {
+                const floatx16& v = acc[nb][q / 4];
+                ex[((wv * NB + nb) * (TB * 4) + q) * 64 + lane] =
+                    make_float4(v[4 * (q % 4)], v[4 * (q % 4) + 1], v[4 * (q % 4) + 2], v[4 * (q % 4) + 3]);
+            }
+        __syncthreads();
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int q = 0; q < OQ; ++q) {
+                float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+                for (int g = 0; g < KG; ++g) {
+                    const float4 v = ex[(((g * FW + fw) * NB + nb) * (TB * 4) + grp * OQ + q) * 64 + lane];
+                    sum.x += v.x;
+                    sum.y += v.y;
+                    sum.z += v.z;
+                    sum.w += v.w;
                 }
+                mine[nb][q][0] = sum.x; mine[nb][q][1] = sum.y; mine[nb][q][2] = sum.z; mine[nb][q][3] = sum.w;
             }
-            __syncthreads();
-            if (grp == gsrc - 1) {
+    } else {
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    acc0[v] += r0[v * 64];
-                    if constexpr (SWIGLU) acc1[v] += r1[v * 64];
-                }
-            }
-            if (gsrc > 1) __syncthreads();
-        }
-        if (grp != 0) return;
-    }
-
-    // accumulator element v of lane l: feature 8 (v / 4) + 4 (l / 32) + v % 4 of the wave's
-    // block, token l % 32
-    const int tok = wy * 32 + (lane & 31);
-    if (tok >= rows) return;
-    float* orow = out + (size_t)(row0 + tok) * N + n0 + wx * 32;
+        for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int f = 8 * q + 4 * (lane >> 5);
-        if (n0 + wx * 32 + f >= N) continue;  // N is a multiple of 4: a group of 4 is in or out as a whole
-        float4 y;
-        if constexpr (SWIGLU) {
-            y.x = silu_f32(acc0[4 * q + 0]) * acc1[4 * q + 0];
-            y.y = silu_f32(acc0[4 * q + 1]) * acc1[4 * q + 1];
-            y.z = silu_f32(acc0[4 * q + 2]) * acc1[4 * q + 2];
-            y.w = silu_f32(acc0[4 * q + 3]) * acc1[4 * q + 3];
-            if (gu_out != nullptr) {  // uniform: the pre-activations G | U [rows, 2 N] kept for a backward pass
-                float* const grow = gu_out + (size_t)(row0 + tok) * 2 * N + n0 + wx * 32 + f;
-                *reinterpret_cast<float4*>(grow) =
-                    make_float4(acc0[4 * q + 0], acc0[4 * q + 1], acc0[4 * q + 2], acc0[4 * q + 3]);
-                *reinterpret_cast<float4*>(grow + N) =
-                    make_float4(acc1[4 * q + 0], acc1[4 * q + 1], acc1[4 * q + 2], acc1[4 * q + 3]);
-            }
-        } else {
-            y = make_float4(acc0[4 * q + 0], acc0[4 * q + 1], acc0[4 * q + 2], acc0[4 * q + 3]);
-            if (bw_gu != nullptr) {  // uniform
-                // SwiGlu::backward (src/ffn.rs:87-120) on the way out: the product row is the gradient of the
-                // hidden row; dG = dH * U * silu'(G), dU = dH * silu(G) go to `gu_out`, `out` is not written.
-                const size_t off = (size_t)(row0 + tok) * 2 * N + n0 + wx * 32 + f;
-                const float4 g4 = *reinterpret_cast<const float4*>(bw_gu + off);
-                const float4 u4 = *reinterpret_cast<const float4*>(bw_gu + off + N);
-                const float dh[4] = {y.x, y.y, y.z, y.w}, gv[4] = {g4.x, g4.y, g4.z, g4.w}, uv[4] = {u4.x, u4.y, u4.z, u4.w};
-                float dg[4], du[4];
+            for (int q = 0; q < OQ; ++q)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float sg = 1.0f / (1.0f + __expf(-gv[i]));
-                    dg[i] = dh[i] * uv[i] * (sg * (1.0f + gv[i] * (1.0f - sg)));  // silu', src/ffn.rs:235-238
-                    du[i] = dh[i] * (gv[i] * sg);
+                    const float v = acc[nb][q / 4][4 * (q % 4) + i];
+                    mine[nb][q][i] = APART ? v + low[nb][q / 4][4 * (q % 4) + i] : v;
                 }
-                *reinterpret_cast<float4*>(gu_out + off) = make_float4(dg[0], dg[1], dg[2], dg[3]);
-                *reinterpret_cast<float4*>(gu_out + off + N) = make_float4(du[0], du[1], du[2], du[3]);
-                continue;
+    }
+
+    // Accumulator element v of lane l: feature 8 (v / 4) + 4 (l / 32) + v % 4 of the wave's block, token l % 32.
+    // finish: four features from `f` on of one row of the layer's tables, what becomes of the sums
+    auto finish = [&](auto whole_tag, size_t orow, int f, float (&g)[4], float (&u)[4]) {
+        constexpr bool WHOLE = decltype(whole_tag)::value;  // N a multiple of 4: in or out as a whole, on 16-byte boundaries
+        const int n = N - f;
+        auto store4 = [&](float* to, const float (&v)[4]) {
+            if constexpr (WHOLE) {
+                *reinterpret_cast<float4*>(to) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (i < n) to[i] = v[i];
+            }
+        };
+        if constexpr (sizeof(WT) == 1) {
+            const float* const sc = scales + (size_t)expert * s_expert_stride;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int fi = min(f + i, N - 1);
+                g[i] *= sc[fi];
+                if constexpr (SWIGLU) u[i] *= sc[N + fi];
             }
         }
-        *reinterpret_cast<float4*>(orow + f) = y;
-    }
+        float y[4];
+        if constexpr (SWIGLU) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = silu_f32(g[i]) * u[i];
+            if (gu_out != nullptr) {  // uniform: the pre-activations G | U [rows, 2 N] kept for a backward pass
+                float* const grow = gu_out + orow * 2 * N + f;
+                store4(grow, g);
+                store4(grow + N, u);
+            }
+        } else if (bw_gu != nullptr) {  // uniform
+            // SwiGlu::backward (src/ffn.rs:87-120) on the way out: the product row is the gradient of the
+            // hidden row; dG = dH * U * silu'(G), dU = dH * silu(G) go to `gu_out`, `out` is not written.
+            const size_t off = orow * 2 * N + f;
+            float gv[4], uv[4], dg[4], du[4];
+            if constexpr (WHOLE) {
+                const float4 g4 = *reinterpret_cast<const float4*>(bw_gu + off), u4 = *reinterpret_cast<const float4*>(bw_gu + off + N);
+                gv[0] = g4.x; gv[1] = g4.y; gv[2] = g4.z; gv[3] = g4.w;
+                uv[0] = u4.x; uv[1] = u4.y; uv[2] = u4.z; uv[3] = u4.w;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    gv[i] = bw_gu[off + min(i, n - 1)];
+                    uv[i] = bw_gu[off + N + min(i, n - 1)];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float sg = 1.0f / (1.0f + __expf(-gv[i]));
+                dg[i] = g[i] * uv[i] * (sg * (1.0f + gv[i] * (1.0f - sg)));  // silu', src/ffn.rs:235-238
+                du[i] = g[i] * (gv[i] * sg);
+            }
+            store4(gu_out + off, dg);
+            store4(gu_out + off + N, du);
+            return;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = g[i];
+        }
+        store4(out + orow * N + f, y);
+    };
+    auto token_of = [&](int q) { return (grp * OQ + q) / 4 * 32 + lr; };
+    auto feature_of = [&](int q) { return n0 + fw * 32 + 8 * ((grp * OQ + q) % 4) + 4 * lh; };
+    auto store_tile = [&](auto whole_tag) {
+        uint32_t odd = 0;  // quads with a sum that is not a number
+#pragma unroll
+        for (int q = 0; q < OQ; ++q) {
+            const int tok = token_of(q), f = feature_of(q);
+            if (tok >= rows || f >= N) continue;
+            float g[4], u[4];
+            bool nan = false;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                g[i] = mine[0][q][i];
+                u[i] = mine[NB - 1][q][i];
+                nan = nan || g[i] != g[i] || u[i] != u[i];
+            }
+            if (nan) odd |= 1u << q;
+            else finish(whole_tag, (size_t)(row0 + tok), f, g, u);
+        }
+        // An infinity (or a value within a rounding of the largest) splits into parts that cancel or meet a zero part of the
+        // other operand: the sum is then not a number where the product of the values themselves may well be one.  Such
+        // sums, and those that are not numbers anyway, are taken again from the values, one after the other.
+        if (odd == 0) return;
+#pragma unroll 1
+        for (int q = 0; q < OQ; ++q) {
+            if (!((odd >> q) & 1)) continue;
+            const int tok = token_of(q), f = feature_of(q);
+            const float* const ar = token_row(tok);
+            float g[4] = {0.0f, 0.0f, 0.0f, 0.0f}, u[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            const WT *wg[4], *wu[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int fi = min(f + i, N - 1);
+                wg[i] = wbase + (size_t)fi * K;
+                wu[i] = wbase + (size_t)(SWIGLU ? N + fi : fi) * K;
+            }
+#pragma unroll 1
+            for (int c = 0; c < K; ++c) {
+                const float av = ar[c];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    g[i] = fmaf(av, weight_value(wg[i][c]), g[i]);
+                    if constexpr (SWIGLU) u[i] = fmaf(av, weight_value(wu[i][c]), u[i]);
+                }
+            }
+            finish(whole_tag, (size_t)(row0 + tok), f, g, u);
+        }
+    };
+    if (N % 4 == 0) store_tile(Yes{});
+    else store_tile(No{});
 }
 
 }  // namespace
 
-// 64-row tiles; 32-row tiles when the launches of such a batch would have few tiles for the chip (their workgroups
-// cannot be spread evenly over 256 compute units: 320 tiles leave a quarter of them with twice the work)
-int f32_tile_m(int rows, int groups, int n_min) {
-    const long long tiles64 = (long long)(rows / 64 + groups) * ((n_min + 63) / 64);
-    return tiles64 < 4 * 256 ? 32 : 64;
+int f32_tile_m(int rows, int groups) { return rows <= 32 * groups ? 32 : 64; }
+
+// What the f32 matrix-core kernel set asks for: whole slices of the reduction, whole pieces of an output row
+bool f32_shape_ok(int N, int K) { return K % 32 == 0 && K >= 32 && N % 4 == 0 && N >= 4; }
+
+// Tokens x features of a workgroup, and its waves.  A launch is bound by the length of one workgroup's chain until there
+// are about as many workgroups as compute units, and by the multiplies from there on, which the larger tiles feed best.
+// So: the smallest tile of which there is at most one a compute unit (bf16 and int8 weights, a third of the multiplies
+// and of the LDS a tile: some more of them together), then 64 x 128.  us, all at 8 experts top-2, d 512:
+//   f32, gate/up of 1408     32x32 / 32x64 / 64x64 / 64x128 / the same on eight waves: 1 token 9.8 / 13.3 / 17.2 / 25.8 / -, 8
+//     tokens 14.0 / 12.7 / 17.6 / 26.2 / -, 128 20.2 / 19.7 / 17.6 / 25.8 / 23.9, 256 30.1 / 27.5 / 27.6 / 27.9 / 25.4, 1024
+//     71.1 / 59.6 / 52.9 / 46.4 / 50.1, 8192 499 / 374 / 301 / 284 / 319
+//   f32, down from 1408      128 tokens 13.0 / 17.0 / 22.8 / 34.6 / 29.6, 256 18.8 / 17.2 / 23.4 / 33.8 / 29.9, 512 24.3 / 25.4
+//     / 23.3 / 34.4 / 30.2, 1024 39.6 / 35.4 / 36.6 / 34.8 / 31.5, 8192 242 / 192 / 167 / 159 / 175
+//   bf16, gate/up of 682     32 tokens 8.9 / 8.5 / 11.6 / 14.5, 256 12.7 / 11.9 / 13.1 / 16.4, 1024 24.4 / 20.7 / 19.6 / 19.6,
+//     2048 40.7 / 32.0 / 31.2 / 29.4
+// A last feature tile that is mostly empty costs more than half as wide tiles do: 64 experts of 704 (five and a half tiles
+// of 128), d 1024, 2048 tokens, six a row: 268 us in 64x128, 248 in 64x64.
+enum class F32Tile { T32x32, T32x64, T64x64, T64x128, T64x128x8 };
+static F32Tile f32_tile(const GroupedArgs& g, bool f32_weights, bool small_slices) {
+    const int S = g.dense_rows >= 0 ? g.dense_rows : g.routed_rows, E = g.dense_rows >= 0 ? 1 : g.groups;
+    // tiles of a group's rows: a last one half full, or one tile for each group that gets any
+    const int hit = std::min(E, S);
+    auto tiles = [&](int rows, int features) {
+        return (long long)std::max(S / rows + (hit + 1) / 2, hit) * ((g.N + features - 1) / features);
+    };
+    if (tiles(32, 32) <= 256 && small_slices) return F32Tile::T32x32;
+    if (tiles(32, 64) <= (f32_weights ? 256 : 600) || (g.dense_rows < 0 && g.tile_m == 32)) return F32Tile::T32x64;
+    if (tiles(64, 64) <= 256) return F32Tile::T64x64;
+    if (f32_weights && tiles(64, 128) <= 256) return F32Tile::T64x128x8;
+    return (g.N + 127) / 128 * 128 * 20 > (g.N + 63) / 64 * 64 * 21 ? F32Tile::T64x64 : F32Tile::T64x128;
 }
 
-// reduction width a multiple of the slice, output width a multiple of 4 (16-byte stores)
-bool f32_shape_ok(int N, int K) { return K % FK == 0 && K >= FK && N % 4 == 0 && N >= 4; }
-
-hipError_t launch_grouped_f32(const GroupedArgs& g, hipStream_t s) {
-    // the tile table's tile height (a dense launch makes its own tiles: 64 rows, or 32 when that leaves few)
-    int fm = g.tile_m;
-    if (g.dense_rows >= 0) fm = f32_tile_m(g.dense_rows, 0, g.N);
-    if (fm != 32 && fm != 64) return hipErrorInvalidValue;
-    const int tiles_m = g.dense_rows >= 0 ? (g.dense_rows + fm - 1) / fm : g.max_tiles;
-    if (tiles_m <= 0) return hipSuccess;
-    const int total = (g.N + FN - 1) / FN * tiles_m;
-    const dim3 grid((total + 7) / 8 * 8);
-    auto go = [&](auto swiglu_tag, auto fm_tag, auto split_tag, auto sk_tag, auto stages_tag) {
+template <typename WT>
+static hipError_t launch_f32_t(const GroupedArgs& g, hipStream_t s) {
+    if (g.dense_rows < 0 && g.tile_m != 32 && g.tile_m != 64) return hipErrorInvalidValue;
+    constexpr bool F32 = sizeof(WT) == 4;
+    auto whole = [](const void* p, size_t pitch) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && pitch % 16 == 0; };
+    const bool aligned = g.K % 32 == 0 && whole(g.a, (size_t)g.K * 4) && whole(g.w, (size_t)g.K * sizeof(WT)) &&
+                         g.w_expert_stride * sizeof(WT) % 16 == 0;
+    auto go = [&](auto swiglu_tag, auto nw_tag, auto tb_tag, auto fw_tag, auto steps_tag) {
         constexpr bool SW = decltype(swiglu_tag)::value;
-        constexpr int FMv = decltype(fm_tag)::value, SP = decltype(split_tag)::value, SKv = decltype(sk_tag)::value,
-                      ST = decltype(stages_tag)::value;
-        RB_LAUNCH((grouped_f32_kernel<SW, FMv, SP, SKv, ST>), grid, dim3(FMv * 4 * SP), 0, s, static_cast<const float*>(g.a),
-                  g.row_index, static_cast<const float*>(g.w), g.w_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0,
-                  g.tile_rows, g.ntiles, g.dense_rows, static_cast<float*>(g.out), static_cast<float*>(g.gu_out),
-                  static_cast<const float*>(g.swiglu_grad_gu));
+        constexpr int FW = decltype(fw_tag)::value, FN = 32 * FW, BM = 32 * decltype(tb_tag)::value;
+        constexpr int NW = decltype(nw_tag)::value, STEPS = decltype(steps_tag)::value;
+        const int tiles_m = g.dense_rows >= 0 ? (g.dense_rows + BM - 1) / BM : g.max_tiles * (g.tile_m / BM);
+        const int total = (g.N + FN - 1) / FN * tiles_m;
+        if (total <= 0) return;
+        const int sub = g.tile_m / BM;
+        auto launch = [&](auto dma_tag) {
+            RB_LAUNCH((grouped_f32_kernel<WT, SW, NW, BM / 32, FW, STEPS, decltype(dma_tag)::value>), dim3((total + 7) / 8 * 8),
+                      dim3(64 * NW), 0, s, static_cast<const float*>(g.a), g.row_index, static_cast<const WT*>(g.w), g.w_expert_stride,
+                      g.scales, g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, sub, g.dense_rows,
+                      static_cast<float*>(g.out), static_cast<float*>(g.gu_out), static_cast<const float*>(g.swiglu_grad_gu));
+        };
+        constexpr int SK = 16 * STEPS * (NW / FW);
+        if (aligned && g.K % SK == 0) launch(std::true_type{});
+        else if constexpr (!(F32 && FW == 4)) launch(std::false_type{});  // (f32_tile does not ask for it)
     };
     typedef std::integral_constant<int, 1> One;
     typedef std::integral_constant<int, 2> Two;
-    typedef std::integral_constant<int, 3> Three;
-    typedef std::integral_constant<int, 16> K16;
-    typedef std::integral_constant<int, 32> K32;  // (and 32-row tiles)
-    typedef std::integral_constant<int, 64> M64;
-    // 32-row tiles have two waves per group: a second group brings the workgroup back to four
-    if (fm == 64) {
-        if (g.swiglu) go(std::true_type{}, M64{}, One{}, K16{}, Three{});
-        else go(std::false_type{}, M64{}, One{}, K16{}, Three{});
-    } else {
-        if (g.swiglu) go(std::true_type{}, K32{}, Two{}, K32{}, Two{});
-        else go(std::false_type{}, K32{}, Two{}, K32{}, Three{});
-    }
+    typedef std::integral_constant<int, 4> Four;
+    typedef std::integral_constant<int, 8> Eight;
+    auto pick = [&](auto swiglu_tag) {
+        typedef std::integral_constant<int, decltype(swiglu_tag)::value && F32 ? 1 : 2> Steps;
+        F32Tile tile = f32_tile(g, F32, !aligned || g.K % 64 == 0);
+        if (F32 && !aligned && (tile == F32Tile::T64x128 || tile == F32Tile::T64x128x8)) tile = F32Tile::T64x64;
+        switch (tile) {
+            case F32Tile::T32x32: return go(swiglu_tag, Four{}, One{}, One{}, One{});
+            case F32Tile::T32x64: return go(swiglu_tag, Four{}, One{}, Two{}, One{});
+            case F32Tile::T64x64: return go(swiglu_tag, Four{}, Two{}, Two{}, One{});
+            case F32Tile::T64x128: return go(swiglu_tag, Four{}, Two{}, Four{}, Steps{});
+            case F32Tile::T64x128x8:
+                if constexpr (F32) return go(swiglu_tag, Eight{}, Two{}, Four{}, One{});
+        }
+    };
+    if (g.swiglu) pick(std::true_type{});
+    else pick(std::false_type{});
     return hipGetLastError();
+}
+
+hipError_t launch_grouped_f32(const GroupedArgs& g, WeightKind wk, hipStream_t s) {
+    switch (wk) {
+        case WeightKind::F32: return launch_f32_t<float>(g, s);
+        case WeightKind::BF16: return launch_f32_t<bf16_t>(g, s);
+        case WeightKind::I8: return launch_f32_t<int8_t>(g, s);
+    }
+    return hipErrorInvalidValue;
 }
 
 }  // namespace rbmoe

@@ -236,7 +236,9 @@ struct rbmoe_layer {
     // products run on the bf16 matrix cores over a bf16 copy of the rows (nearest even) that the routing kernels
     // write on the way, hidden and expert rows are bf16, and the combine sums them into f32 again
     bool cast_rows = false;
-    bool use_f32_mc = false;   // all-f32 layer on the f32 matrix cores
+    bool use_f32_mc = false;   // all-f32 layer of whole tiles: the kernel set "mfma_f32"
+    bool f32_rows = false;     // products over f32 rows at f32 accuracy (launch_grouped_f32): with use_f32_mc, and on the
+                               // any-shape kernel set whatever the weights
     bool decode_path = true;   // few tokens: launches that stream every touched weight once
     bool decode_front = true;  // ... the routing beside the gate/up products where that pays (decode_front_pays)
     bool shared_beside = true; // large batches: the shared expert's products on the side stream, beside the routing
@@ -323,7 +325,7 @@ struct Plan {
 // Which kernel sets the layer's shapes and dtypes allow (and `force_generic` and `tight` do not rule out).
 void choose_kernel_sets(rbmoe_layer* L) {
     const rbmoe_config* cfg = &L->cfg;
-    L->use_stream = L->use_f32_mc = L->cast_rows = false;
+    L->use_stream = L->use_f32_mc = L->cast_rows = L->f32_rows = false;
     // Expert widths are rounded up to whole tiles (the model width is the caller's row pitch and is not): 64 columns
     // for the packed bf16 / int8 kernels, 32 for the f32 ones.  The any-shape kernels run at a thirtieth of the bf16
     // matrix-core rate and a third of the f32 one, so rounding pays while it multiplies the work by less than that:
@@ -364,6 +366,7 @@ void choose_kernel_sets(rbmoe_layer* L) {
         L->Fw = cfg->d_ff;
         L->Fsw = L->Fs;
     }
+    L->f32_rows = cfg->act_dtype == RBMOE_F32 && !L->use_stream && !L->force_generic;
     const int block = L->tight ? kRouterTokens : kMinRouterTokens;  // tokens of the smallest router block
     L->max_nb = (cfg->max_tokens + block - 1) / block;
 }
@@ -1129,12 +1132,12 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
 
     const bool mfma = L->use_stream;
     const bool f32mc = L->use_f32_mc;
-    const int tile_m0 = mfma ? stream_tile_m() : (f32mc ? f32_tile_m(T * k, E, std::min(F, d)) : kGenericTileM);
+    const int tile_m0 = mfma ? stream_tile_m() : (L->f32_rows ? f32_tile_m(T * k, E) : kGenericTileM);
     L->last_tile_m = tile_m0;
     L->kernel_name = mfma ? (wk == WeightKind::I8 ? "mfma_bf16_stream_int8w" : "mfma_bf16_stream")
                           : (f32mc ? "mfma_f32" : "generic");
     // a training layer keeps the gathered rows: the weight gradients of gate and up multiply by them
-    const bool gather_in_product = (mfma || f32mc) && !L->explicit_gather && !L->training;
+    const bool gather_in_product = (mfma || L->f32_rows) && !L->explicit_gather && !L->training;
 
     // whether the single-workgroup routing kernel would stage this call's rows in LDS: only then can it apply the
     // norm and write the bf16 copy of f32 rows
@@ -1330,7 +1333,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     for (auto& r : L->replay) r = nullptr;
     auto run_on = [=](const GroupedArgs& g, hipStream_t st) -> hipError_t {
         if (mfma) return launch_grouped_stream(g, wk, st);
-        if (f32mc) return launch_grouped_f32(g, st);
+        if (L->f32_rows) return launch_grouped_f32(g, wk, st);
         return launch_grouped_generic(g, abf, wk, kGenericTileM, st);
     };
     auto run = [&](const GroupedArgs& g, bool) -> hipError_t { return run_on(g, s); };
@@ -1386,7 +1389,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     } join_guard{ctx, s};
     bool shared_forked = false;
     auto fork_shared = [&]() -> int {
-        if (c.shared_expert && !shared_inside && T >= 1024 && !timed && !cast && L->shared_beside && (mfma || f32mc) &&
+        if (c.shared_expert && !shared_inside && T >= 1024 && !timed && !cast && L->shared_beside && (mfma || L->f32_rows) &&
             ensure_side_stream(ctx) == RBMOE_OK) {
             HIP_TRY(ctx, hipEventRecord(ctx->ev_fork, s));
             HIP_TRY(ctx, hipStreamWaitEvent(ctx->side_stream, ctx->ev_fork, 0));
@@ -1462,6 +1465,8 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     g1.max_tiles = T > 0 ? (T * k) / tile_m0 + E : 0;
     g1.likely_tiles = std::max((T * k) / tile_m0 + E / 2, std::min(E, T * k));  // a last tile half full, or one tile each
     g1.tile_m = tile_m0;
+    g1.routed_rows = T * k;
+    g1.groups = E;
     g1.dense_rows = -1;
     g1.out = L->h.p;
     g1.swiglu = true;
@@ -2269,6 +2274,8 @@ int rbmoe_backward(rbmoe_layer* L, const void* grad_output, int32_t tokens, int3
     g.ntiles = (const int*)L->ntiles.p;
     g.max_tiles = S / L->last_tile_m + E;  // the tile table of the last forward
     g.tile_m = L->last_tile_m;
+    g.routed_rows = S;
+    g.groups = E;
     g.dense_rows = -1;
     g.swiglu = false;
     g.group_m = L->group_m;
@@ -2278,7 +2285,7 @@ int rbmoe_backward(rbmoe_layer* L, const void* grad_output, int32_t tokens, int3
     const WeightKind wk = c.weight_dtype == RBMOE_F32 ? WeightKind::F32 : WeightKind::BF16;
     auto prod_on = [&](const GroupedArgs& a, hipStream_t st) -> hipError_t {
         if (L->use_stream) return launch_grouped_stream(a, WeightKind::BF16, st);
-        if (L->use_f32_mc) return launch_grouped_f32(a, st);
+        if (L->f32_rows) return launch_grouped_f32(a, wk, st);
         return launch_grouped_generic(a, abf, wk, kGenericTileM, st);
     };
     auto prod = [&](const GroupedArgs& a) -> hipError_t { return prod_on(a, s); };

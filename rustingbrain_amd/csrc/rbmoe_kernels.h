@@ -180,6 +180,7 @@ struct GroupedArgs {
     const int* tile_rows;
     const int* ntiles;
     int max_tiles;
+    int routed_rows = 0, groups = 0;  // f32 rows: rows in all and groups of the tile table, for the choice of a tile
     int likely_tiles = 0;   // what *ntiles will be about, for the choice of a kernel (0: max_tiles)
     int dense_rows;         // >= 0: one group of this many rows, no tile table (shared expert)
     void* out;              // [rows, N] activation dtype
@@ -200,7 +201,7 @@ struct GroupedArgs {
         void* gu_out = nullptr;   // [rows, 2N]
     } dense2;
     int group_m;            // MFMA path: M-tiles per scheduling group (0 = default)
-    int tile_m = 0;         // f32 matrix-core path: rows per tile of the tile table (64 or 32)
+    int tile_m = 0;         // rows per tile of the tile table
 };
 hipError_t launch_grouped_generic(const GroupedArgs& a, bool act_bf16, WeightKind wk, int tile_m,
                                   hipStream_t s);
@@ -215,10 +216,10 @@ hipError_t launch_grouped_stream(const GroupedArgs& a, WeightKind wk, hipStream_
 void pack_weight_bf16(const uint16_t* src, int rows, int cols, uint16_t* dst);
 void pack_weight_i8(const int8_t* src, int rows, int cols, int8_t* dst);
 
-// f32 matrix cores (all-f32 layers): 64-row tiles, plain row-major weights.
-int f32_tile_m(int rows, int groups, int n_min);  // tile height (64 or 32) for a batch of `rows` routed rows in `groups` groups; n_min: the narrower product's width
+// Products over f32 rows at f32 accuracy on the bf16 matrix cores: plain row-major weights of any kind, any shape.
+int f32_tile_m(int rows, int groups);  // rows of the tile table's tiles for so many routed rows: 32 or 64
 bool f32_shape_ok(int N, int K);
-hipError_t launch_grouped_f32(const GroupedArgs& a, hipStream_t s);
+hipError_t launch_grouped_f32(const GroupedArgs& a, WeightKind wk, hipStream_t s);
 
 // ---- backward pass: the kernels around the matrix products (backward_kernels.hip) --------
 // dy[pos] = gate * gout[token(pos)], grad_gates[slot] = gout[token] . y[pos]; row widths: multiples of 16 bytes

@@ -1,0 +1,74 @@
+"""Products over f32 rows at the sizes where a tile, a slice of the reduction or the way of the operands into LDS changes,
+and values that three bf16 parts do not hold."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
+from rustingbrain_amd import synth
+from test_gpu_row_pointers import run
+
+pytestmark = pytest.mark.gpu
+
+# One row up to several 64-row tiles an expert; widths of whole slices (64, 192), of half slices (96), of no whole pieces
+# (70, 37), a last tile of one feature (257) and more features than fit one round of small tiles (1408)
+SHAPES = [dict(d=64, E=4, k=2, F=192, T=1), dict(d=128, E=3, k=1, F=96, T=97), dict(d=96, E=4, k=2, F=257, T=65),
+          dict(d=70, E=5, k=2, F=37, T=40), dict(d=512, E=8, k=2, F=1408, T=130), dict(d=512, E=8, k=2, F=1408, T=515),
+          dict(d=256, E=3, k=2, F=682, T=1030), dict(d=192, E=2, k=2, F=1408, T=1500)]
+
+
+# 1e-5 is f32's: a chain of 1408 rounded additions is off by at most 1408 * 2^-24 = 8e-5 of the sum of magnitudes, and by its
+# root, 2e-6, on average; the mixed layers of test_gpu_ragged_widths.py are held to the same
+@pytest.mark.parametrize("wt", ["f32", "bf16", "int8"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "d{d}_F{F}_T{T}".format(**s))
+def test_tiles(device, shape, wt):
+    if wt != "f32" and shape["F"] % 64 == 0 and shape["d"] % 64 == 0:
+        shape = {**shape, "F": shape["F"] + 32}   # (such a layer's rows would be rounded to bf16)
+    t = synth.make(small_workload(seed=71, act="f32", wt=wt, shared=True, shared_d_ff=shape["F"], **shape))
+    ref = oracle_layer(t).forward(t.x, threads=8)
+    layer = gpu_layer(device, t)
+    out, cache = layer.forward_train(t.x)
+    assert_routing_identical(cache, ref)
+    h, y = layer.expert_rows(int(ref.offsets[-1]))
+    assert rel_l2(h, ref.hidden) <= 1e-5 and rel_l2(y, ref.expert_out) <= 1e-5
+    assert rel_l2(out, ref.out) <= 1e-5
+    layer.close()
+
+
+@pytest.mark.parametrize("T", [1, 150])
+@pytest.mark.parametrize("wt", ["bf16", "int8"])
+def test_rows_off_a_piece(device, wt, T):
+    """Rows of whole 16-byte pieces that do not start on one travel element by element."""
+    t = synth.make(small_workload(d=64, E=4, k=2, F=96, T=T, seed=73, act="f32", wt=wt))
+    layer = gpu_layer(device, t)
+    got, _, _ = run(device, layer, np.ascontiguousarray(t.x), 4, lambda x, o: layer.forward_device(x, T, o))
+    assert rel_l2(got.view(np.float32).reshape(T, 64), oracle_layer(t).forward(t.x, threads=4).out) <= 1e-5
+    layer.close()
+
+
+@pytest.mark.parametrize("T", [20, 300])
+@pytest.mark.parametrize("wt,F", [("f32", 64), ("f32", 45), ("bf16", 96), ("int8", 45)])
+def test_values_that_do_not_split(device, wt, F, T):
+    """Infinities, values within a rounding of the largest, NaN and subnormal values in the rows, infinities in f32 weights:
+    the hidden rows hold infinities and NaN where f32 arithmetic on the values themselves puts them."""
+    t = synth.make(small_workload(d=64, E=3, k=2, F=F, T=T, seed=72, act="f32", wt=wt))
+    x = t.x
+    x[1, 5], x[2, 9], x[3, 60] = np.inf, -np.inf, np.nan
+    x[4, 0], x[5, 63] = 3.4e38, -3.4e38        # rounded to bf16 these are infinities
+    x[6], x[7] = 1e-41, x[7] * 1e-36           # subnormal values, and values whose parts are
+    if wt == "f32":
+        t.experts[1]["gate"][3, 7] = np.inf
+        t.experts[2]["up"][0, 0] = -np.inf
+    with np.errstate(all="ignore"):
+        ref = oracle_layer(t).forward(x, threads=4)
+    layer = gpu_layer(device, t)
+    layer.forward_train(x)
+    R = int(ref.offsets[-1])
+    h, _ = layer.expert_rows(R)
+    want = np.asarray(ref.hidden[:R])
+    np.testing.assert_array_equal(np.isnan(h), np.isnan(want))
+    np.testing.assert_array_equal(np.where(np.isinf(h), h, 0), np.where(np.isinf(want), want, 0))
+    ok = np.isfinite(want) & (np.abs(want) < 1e30)
+    assert np.isinf(want).any() and np.isnan(want).any() and ok.any()
+    assert rel_l2(h[ok], want[ok]) <= 1e-5
+    layer.close()

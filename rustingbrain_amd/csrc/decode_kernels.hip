@@ -650,6 +650,10 @@ hipError_t launch_route_small(const SmallRouteArgs& a, bool bf16, hipStream_t s)
 // ---------------------------------------------------------------------------
 constexpr int kBatch = 12;
 
+// Partial sums meet in LDS as [wave][gate, up][16][64 lanes], the rows of 64 this far apart: the threads that add them up read
+// 8 neighbouring lanes of rows 0, 4, 8 and 12, which then lie in 64 different banks.  What follows the products of the int8
+// front launch at 32 tokens, d 768, 8 experts of 1408: 2.7 us 64 apart, 1.5 so, the scales requested in front of the products.
+constexpr int kRedPitch = 66;
 struct DecodeSide {
     const bf16_t* a;
     const int* row_index;
@@ -666,6 +670,7 @@ struct DecodeSide {
     // rows behind a norm (RowForm with kNorm), in LDS: the norm's weights [K] and the rows' factors [32]
     const float* norm_w = nullptr;
     const float* row_factor = nullptr;
+    bool widen_first = false;  // int8 weights of the first batch are widened in front of the hook
 };
 
 // The rows a product reads.  XT: bf16, or f32 rounded to bf16 on the way (the product's precision either way).  NORM: the
@@ -842,7 +847,7 @@ __device__ __forceinline__ void decode_combine_block_early(const DecodeGemmArgs&
 
 template <bool SWIGLU, bool I8, int NW>
 __global__ __launch_bounds__(NW * 64) void decode_gemm_kernel(DecodeGemmArgs g) {
-    __shared__ float red[NW * (SWIGLU ? 2 : 1) * 16 * 64];
+    __shared__ float red[NW * (SWIGLU ? 2 : 1) * 16 * kRedPitch];
     __shared__ int last_of_block;
     const int fb = blockIdx.x;
     const int ty = blockIdx.y;
@@ -968,7 +973,7 @@ __global__ __launch_bounds__(kSmallThreads) void decode_layout_kernel(DecodeLayo
 
 template <bool I8, int M>
 __global__ __launch_bounds__(512) void decode_down_by_expert_kernel(DecodeGemmArgs g, DecodeLayoutArgs t) {
-    constexpr int kRed = 8 * 16 * 64;
+    constexpr int kRed = 8 * 16 * kRedPitch;
     __shared__ float red[kRed > kLayoutLdsFloats ? kRed : kLayoutLdsFloats];
     __shared__ int row_slot[32];
     __shared__ int last_of_block;
@@ -1031,7 +1036,7 @@ __global__ __launch_bounds__(512) void decode_down_by_expert_kernel(DecodeGemmAr
     else decode_combine_block_early<bf16_t, true>(g, fb, ce);
 }
 
-// red_raw: TEAMS * NW * (SWIGLU ? 2 : 1) * 1024 floats of LDS; BATCH: reduction steps whose loads a wave issues together.
+// red_raw: TEAMS * NW * (SWIGLU ? 2 : 1) * 16 * kRedPitch floats of LDS; BATCH: reduction steps whose loads a wave issues together.
 // TEAMS > 1: the workgroup is TEAMS teams of NW waves, each with a feature block `fb` of its own (the caller hands
 // every team its block; a team without one has left the kernel before: the barrier below counts the waves that
 // are still there).
@@ -1042,8 +1047,8 @@ __global__ __launch_bounds__(512) void decode_down_by_expert_kernel(DecodeGemmAr
 template <bool SWIGLU, bool I8, int NW, int BATCH, int TEAMS, bool LATE_ROWS, typename ROWS, typename HOOK>
 __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* red_raw, LateRows* late, HOOK hook) {
     const int team = TEAMS > 1 ? (int)threadIdx.x / (NW * 64) : 0;
-    float (*red)[SWIGLU ? 2 : 1][16][64] =
-        reinterpret_cast<float (*)[SWIGLU ? 2 : 1][16][64]>(red_raw + (size_t)team * NW * (SWIGLU ? 2 : 1) * 1024);
+    float (*red)[SWIGLU ? 2 : 1][16][kRedPitch] =
+        reinterpret_cast<float (*)[SWIGLU ? 2 : 1][16][kRedPitch]>(red_raw + (size_t)team * NW * (SWIGLU ? 2 : 1) * 16 * kRedPitch);
     const int tid = (int)threadIdx.x - team * (NW * 64);
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1071,6 +1076,13 @@ __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* 
     if constexpr (!LATE_ROWS) {
         const int trow = (lane & 31) < sd.rows ? (lane & 31) : 0;
         grow = (sd.row_index ? sd.row_index[sd.row0 + trow] : sd.row0 + trow) + sd.a_row0;  // awaited after the weight loads
+    }
+
+    // int8: the scales of the four features this thread will finish, under way before the weights
+    float4 sc0 = make_float4(1.0f, 1.0f, 1.0f, 1.0f), sc1 = sc0;
+    if constexpr (I8) {
+        sc0 = *reinterpret_cast<const float4*>(sd.scales + fb * 32 + 4 * (tid & 7));
+        if constexpr (SWIGLU) sc1 = *reinterpret_cast<const float4*>(sd.scales + sd.N + fb * 32 + 4 * (tid & 7));
     }
 
     floatx16 acc0, acc1;
@@ -1138,6 +1150,15 @@ __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* 
         }
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (kFirst && !std::is_same<HOOK, NoHook>::value) {
+            if constexpr (I8) {
+                if (sd.widen_first) {  // uniform over the wave: it has nothing else to do before the rows are normed
+#pragma unroll
+                    for (int u = 0; u < BATCH; ++u) {
+                        asm volatile("" : "+v"(wa[u]));
+                        if constexpr (SWIGLU) asm volatile("" : "+v"(wb[u]));
+                    }
+                }
+            }
             hook();
             if constexpr (ROWS::kNorm) row_factor = sd.row_factor[lane & 31];
         }
@@ -1202,12 +1223,12 @@ __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* 
                 float y = red[0][0][v + h][l];
 #pragma unroll
                 for (int w = 1; w < NW; ++w) y += red[w][0][v + h][l];
-                if constexpr (I8) y *= sd.scales[fb * 32 + f + h];
+                if constexpr (I8) y *= h == 0 ? sc0.x : h == 1 ? sc0.y : h == 2 ? sc0.z : sc0.w;
                 if constexpr (SWIGLU) {
                     float u = red[0][1][v + h][l];
 #pragma unroll
                     for (int w = 1; w < NW; ++w) u += red[w][1][v + h][l];
-                    if constexpr (I8) u *= sd.scales[sd.N + fb * 32 + f + h];
+                    if constexpr (I8) u *= h == 0 ? sc1.x : h == 1 ? sc1.y : h == 2 ? sc1.z : sc1.w;
                     y = silu_bf16_grade(y) * u;
                 }
                 y4[h] = y;
@@ -1238,12 +1259,12 @@ __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* 
 // products read the call's own rows: a norm in front of the layer is applied on the way (RowForm), f32 rows are rounded.
 // The down product then picks the routed rows out of the per-expert hidden rows (DecodeGemmArgs::a_expert_rows).
 // ---------------------------------------------------------------------------
-constexpr int kFrontTokens = 8;  // a routing workgroup's
+constexpr int kFrontTokens = 8;  // a routing workgroup's (1, 2 or 4: the same times, the products take longer than the routing)
 constexpr int kFrontTeams = 2;   // feature blocks of a product workgroup
-constexpr int kFrontRedFloats = kFrontTeams * 4 * 2 * 1024;  // a product workgroup's partial sums
+constexpr int kFrontRedFloats = kFrontTeams * 4 * 2 * 16 * kRedPitch;  // a product workgroup's partial sums
 // ... which share their room with the rows' squares of a call behind a norm (d + 4 floats a row; 64: the chain reads ahead)
 __host__ __device__ static int front_room_floats(int T, int d, bool norm) {
-    const int squares = norm ? T * (d + 4) + 64 : 0;
+    const int squares = norm && !(T <= 8 && wave_norms(d)) ? T * (d + 4) + 64 : 0;
     return squares > kFrontRedFloats ? squares : kFrontRedFloats;
 }
 
@@ -1254,7 +1275,7 @@ __global__ __launch_bounds__(kSmallThreads, 2) void decode_front_kernel(RouteRow
     if ((int)blockIdx.x < routers) {
         const int k = r.k, ES = E | 1;
         const int t0 = blockIdx.x * kFrontTokens, nt = min(kFrontTokens, T - t0);
-        route_rows_body<XT, kFrontTokens, Q8 ? 32 : 8, Q8 ? 2 : 1, 2>(r, blockIdx.x, lds);
+        route_rows_body<XT, kFrontTokens, Q8 ? 32 : 8, Q8 ? 2 : 1, 2, NORM>(r, blockIdx.x, lds);
         __syncthreads();
         float* const prob = reinterpret_cast<float*>(lds);  // the arrays of router_fixed_bytes
         float* const lsev = prob + kFrontTokens * ES;
@@ -1319,44 +1340,98 @@ __global__ __launch_bounds__(kSmallThreads, 2) void decode_front_kernel(RouteRow
         }
         // The rows' factors are taken here as the routing takes them (route_rows_body), by every product workgroup for
         // itself: the rows are requested in front of the weights, squared and summed in index order while those stream in.
-        const int d = r.d, sp = d + 4, xpr = d / Vec16<XT>::N, nx = T * xpr, tid = threadIdx.x;
+        const int d = r.d, sp = d + 4, tid = threadIdx.x;
         float* const nw = red + front_room_floats(T, d, true);
         float* const inv = nw + d;
-        const uint4* const xsrc = reinterpret_cast<const uint4*>(r.x);
         constexpr int NT = kSmallThreads;
-        auto fetch = [&](int i) -> uint4 { return xsrc[(uint32_t)min(i, nx - 1)]; };
         const float w0 = r.norm_w[min(tid, d - 1)], w1 = r.norm_w[min(tid + NT, d - 1)];
-        const uint4 v0 = fetch(tid), v1 = fetch(tid + NT), v2 = fetch(tid + 2 * NT), v3 = fetch(tid + 3 * NT),
-                    v4 = fetch(tid + 4 * NT), v5 = fetch(tid + 5 * NT);
-        __builtin_amdgcn_sched_barrier(0);
-        const uint32_t recip = (uint32_t)(0x100000000ull / (uint32_t)xpr) + 1u;
-        auto put = [&](int i, const uint4& v) {
-            if (i >= nx) return;
-            const int row = xpr == 1 ? i : (int)__umulhi((uint32_t)i, recip), c = (i - row * xpr) * Vec16<XT>::N;
-            float f[Vec16<XT>::N];
-            Vec16<XT>::widen(v, f);
-            float4* const s4 = reinterpret_cast<float4*>(red + row * sp + c);
-#pragma unroll
-            for (int q = 0; q < Vec16<XT>::N / 4; ++q)
-                s4[q] = make_float4(__fmul_rn(f[4 * q], f[4 * q]), __fmul_rn(f[4 * q + 1], f[4 * q + 1]),
-                                    __fmul_rn(f[4 * q + 2], f[4 * q + 2]), __fmul_rn(f[4 * q + 3], f[4 * q + 3]));
-        };
-        auto hook = [&]() {
-            put(tid, v0); put(tid + NT, v1); put(tid + 2 * NT, v2);
-            put(tid + 3 * NT, v3); put(tid + 4 * NT, v4); put(tid + 5 * NT, v5);
-            for (int i = tid + 6 * NT; i < nx; i += NT) put(i, fetch(i));
+        auto put_norm_weights = [&]() {
             if (tid < d) nw[tid] = w0;
             if (tid + NT < d) nw[tid + NT] = w1;
             for (int c = tid + 2 * NT; c < d; c += NT) nw[c] = r.norm_w[c];
-            __syncthreads();
-            if (tid < T) inv[tid] = inverse_rms_of(ordered_sum(red + tid * sp, d), d, r.norm_eps);
-            else if (tid < 32) inv[tid] = 0.0f;
-            __syncthreads();
         };
         sd.norm_w = nw;
         sd.row_factor = inv;
-        decode_gemm_body<true, I8, kSmallThreads / 64 / kFrontTeams, sizeof(XT) == 4 ? 8 : kBatch, kFrontTeams, false,
-                         RowForm<XT, NORM>>(sd, fb, red, nullptr, hook);
+        auto products = [&](auto hook) {
+            decode_gemm_body<true, I8, kSmallThreads / 64 / kFrontTeams, sizeof(XT) == 4 ? 8 : kBatch, kFrontTeams, false,
+                             RowForm<XT, NORM>>(sd, fb, red, nullptr, hook);
+        };
+        if (T <= 8 && wave_norms(d)) {
+            // a wave a row (one token, d 512: the launch 7.6 us, 9.8 with a chain a thread; with four rows a wave, 32 tokens
+            // of d 768, it is slower than the chains, 18.9 us a call against 18.6, for eight waves' sums share four units)
+            const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+            typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+            const XT* const rows = static_cast<const XT*>(r.x);
+            constexpr int MOST = 32 / Vec16<XT>::N;  // pieces a lane at most; of a shorter row the last one again
+            const int most = d / 32 / Vec16<XT>::N - 1;
+            struct Ahead {
+                u32x4_t p[MOST];
+            };
+            auto fetch = [&](int row) {
+                const u32x4_t* const from = reinterpret_cast<const u32x4_t*>(rows + (size_t)min(row, T - 1) * d + (tid & 31) * (d / 32));
+                Ahead a;
+#pragma unroll
+                for (int p = 0; p < MOST; ++p) a.p[p] = from[min(p, most)];
+                return a;
+            };
+            const Ahead own = fetch(wave);
+            __builtin_amdgcn_sched_barrier(0);
+            products([&]() {
+                put_norm_weights();
+                if (tid >= T && tid < 32) inv[tid] = 0.0f;
+                if (wave < T)
+                    with_lane_elements(d, [&](auto l_tag) {
+                        LaneRow<XT, decltype(l_tag)::value> lr;
+#pragma unroll
+                        for (int p = 0; p < lr.P; ++p) lr.raw[p] = __builtin_bit_cast(uint4, own.p[p]);
+                        const float f = lr.inverse_rms(r.norm_eps);
+                        if ((tid & 63) == 0) inv[wave] = f;
+                    });
+                __syncthreads();
+            });
+            return;
+        }
+        // Squares in column order in LDS, a thread of the first wave a row.  The chain of additions is what the products wait
+        // for, so nothing stands in front of it: seven waves lay down their share of the squares before they ask for any
+        // weights, which then come in beside the chain, and the first wave asks for its own before its share (32 tokens, d 768,
+        // int8: the launch 12.5 us with what else is said at kRedPitch; 15.4 with every wave's weights in front).
+        const int xpr = d / Vec16<XT>::N, nx = T * xpr;
+        const uint4* const xsrc = reinterpret_cast<const uint4*>(r.x);
+        const uint32_t recip = (uint32_t)(0x100000000ull / (uint32_t)xpr) + 1u;
+        auto lay_squares = [&]() {
+            auto fetch = [&](int i) -> uint4 { return xsrc[(uint32_t)min(i, nx - 1)]; };
+            auto put = [&](int i, const uint4& v) {
+                if (i >= nx) return;
+                const int row = xpr == 1 ? i : (int)__umulhi((uint32_t)i, recip), c = (i - row * xpr) * Vec16<XT>::N;
+                float f[Vec16<XT>::N];
+                Vec16<XT>::widen(v, f);
+                float4* const s4 = reinterpret_cast<float4*>(red + row * sp + c);
+#pragma unroll
+                for (int q = 0; q < Vec16<XT>::N / 4; ++q)
+                    s4[q] = make_float4(__fmul_rn(f[4 * q], f[4 * q]), __fmul_rn(f[4 * q + 1], f[4 * q + 1]),
+                                        __fmul_rn(f[4 * q + 2], f[4 * q + 2]), __fmul_rn(f[4 * q + 3], f[4 * q + 3]));
+            };
+            for (int i = tid; i < nx; i += 6 * NT) {
+                const uint4 v0 = fetch(i), v1 = fetch(i + NT), v2 = fetch(i + 2 * NT), v3 = fetch(i + 3 * NT), v4 = fetch(i + 4 * NT),
+                            v5 = fetch(i + 5 * NT);
+                __builtin_amdgcn_sched_barrier(0);
+                put(i, v0); put(i + NT, v1); put(i + 2 * NT, v2);
+                put(i + 3 * NT, v3); put(i + 4 * NT, v4); put(i + 5 * NT, v5);
+            }
+            put_norm_weights();
+            __syncthreads();
+        };
+        const bool first_wave = __builtin_amdgcn_readfirstlane(tid >> 6) == 0;
+        if (!first_wave) lay_squares();
+        sd.widen_first = !first_wave;
+        products([&]() {
+            if (first_wave) {
+                lay_squares();
+                if (tid < T) inv[tid] = inverse_rms_of(ordered_sum(red + tid * sp, d), d, r.norm_eps);
+                else if (tid < 32) inv[tid] = 0.0f;
+            }
+            __syncthreads();
+        });
     } else {
         if (fb * 32 >= sd.N) return;
         // (f32 rows take two registers a fragment's worth: a shorter batch keeps everything in registers)

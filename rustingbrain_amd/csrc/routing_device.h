@@ -23,10 +23,11 @@ __host__ __device__ static size_t router_fixed_bytes(int E, int k, int tokens = 
 // Everything order-sensitive keeps the reference's order: the maximum ignores NaN (f32::max), exp(v - max) is
 // summed one expert after the other in index order, the k argmax rounds prefer the lower index on equal
 // probabilities, and the gates are summed in rank order.
-// The sum: lane l of a group ends with ((ex_0 + ex_1) + ... ) + ex_l after l steps of "take the lane below's sum,
-// add your own value" (a shift of the whole wave by one lane inside the add; a group's first lane keeps the sum
+// The sum: lane l of a group holds ((ex_0 + ex_1) + ... ) + ex_l after l steps of "take the lane below's sum,
+// add your own value" (a shift of the whole wave by one lane inside the add; a group's first lane starts from the sum
 // carried over from the experts of the slices before) - the reference's chain, one rounded add per expert, with
-// no trip through LDS; lanes past the last expert add zeros.  An argmax round is two reductions of 32 bits: the
+// no trip through LDS; lanes past the last expert add zeros.  What a group's first lane takes in from the group below
+// follows one lane behind and is overtaken by nobody: the last lane's sum after G - 1 steps is the chain's.  An argmax round is two reductions of 32 bits: the
 // greatest probability bits (probabilities are never negative, so the bits order like the values), then the
 // lowest expert index among the lanes that hold them.
 // NQ = turns a wave needs for its tokens (64 / G tokens a turn); the NQ turns share no data and run interleaved.
@@ -34,7 +35,7 @@ template <int MAXJ, int NQ, int TB>
 __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __restrict__ lsev,
                                              float* __restrict__ gates, int* __restrict__ lexp, int G, int t0, int nt,
                                              int ES, const uint8_t* __restrict__ valid, int E, int k) {
-    constexpr int TW = TB / kRouterWaves;  // tokens of a wave
+    constexpr int TW = TB < kRouterWaves ? 1 : TB / kRouterWaves;  // tokens of a wave
     const int lane_ = threadIdx.x & 63, wave_ = threadIdx.x >> 6;
     const int lig = lane_ & (G - 1);          // lane in group
     const int gbase = lane_ & ~(G - 1);       // first lane of the group
@@ -46,10 +47,12 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
     float* row[NQ];
     float pv[NQ][MAXJ], mx[NQ], sum[NQ], total[NQ];
     unsigned taken_bits[NQ];  // bit j: expert lig + G j is taken
+    uint8_t in_use[NQ];       // (asked for here, looked at behind the softmax)
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         tok[q] = wave_ * TW + q * tpw + lane_ / G;  // token of this group in turn q
         live[q] = tok[q] < nt && tok[q] < (wave_ + 1) * TW && q * tpw < TW;
+        in_use[q] = valid != nullptr ? valid[t0 + (live[q] ? tok[q] : 0)] : 1;
         row[q] = prob + (live[q] ? tok[q] : 0) * ES;
         mx[q] = neg_inf;
 #pragma unroll
@@ -79,19 +82,13 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
 #pragma unroll
         for (int j = 0; j < MAXJ; ++j) {
             if (G * j >= E) break;  // uniform
-            float acc[NQ], seed[NQ];
+            float acc[NQ];
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-                seed[q] = __fadd_rn(carry[q], pv[q][j]);  // what a group's first lane holds: 0 + ex_0 = ex_0 in the first slice
-                acc[q] = lig == 0 ? seed[q] : pv[q][j];
-            }
+            for (int q = 0; q < NQ; ++q) acc[q] = __fadd_rn(carry[q], pv[q][j]);  // in a group's first lane: 0 + ex_0 = ex_0 in the first slice
             for (int st = 1; st < G; ++st) {
 #pragma unroll
-                for (int q = 0; q < NQ; ++q) {
-                    const float below = __uint_as_float(lanes_from<0x138>(__float_as_uint(acc[q])));  // wave_shr:1
-                    const float next = __fadd_rn(below, pv[q][j]);
-                    acc[q] = lig == 0 ? seed[q] : next;
-                }
+                for (int q = 0; q < NQ; ++q)
+                    acc[q] = __fadd_rn(__uint_as_float(lanes_from<0x138>(__float_as_uint(acc[q]))), pv[q][j]);  // wave_shr:1
             }
 #pragma unroll
             for (int q = 0; q < NQ; ++q) carry[q] = __shfl(acc[q], gbase + G - 1);
@@ -110,11 +107,37 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
                 row[q][e] = pv[q][j];
             }
         }
-        ok[q] = live[q] && ((valid == nullptr) || (valid[t0 + tok[q]] != 0));
+        ok[q] = live[q] && in_use[q] != 0;
         taken_bits[q] = 0;
         total[q] = 0.0f;
     }
     // ---- k rounds of argmax over the experts not yet taken ----
+    // Without a NaN anywhere in the wave (with one expert a lane): the greatest probability bits among the untaken, then the
+    // lowest of the lanes that hold them.
+    bool any_nan = false;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) any_nan = any_nan || pv[q][0] != pv[q][0];
+    if (MAXJ == 1 && __ballot(any_nan) == 0ull) {  // uniform over the wave
+        bool open[NQ];  // this lane has an expert and it is not taken
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) open[q] = live[q] && lig < E;
+        for (int r = 0; r < k; ++r) {
+            uint32_t best[NQ];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) best[q] = group_umax(open[q] ? __float_as_uint(pv[q][0]) : 0u, G);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const unsigned long long holders = __ballot(open[q] && __float_as_uint(pv[q][0]) == best[q]) & gmask;
+                const bool mine = holders != 0ull && (holders & ((1ull << lane_) - 1ull)) == 0ull && ((holders >> lane_) & 1ull);
+                open[q] = open[q] && !mine;
+                total[q] = __fadd_rn(total[q], __uint_as_float(best[q]));
+                if (mine) {
+                    lexp[tok[q] * k + r] = ok[q] ? lig : -1;
+                    gates[tok[q] * k + r] = ok[q] ? __uint_as_float(best[q]) : 0.0f;
+                }
+            }
+        }
+    } else
     for (int r = 0; r < k; ++r) {
         int first[NQ];
         uint32_t lbits[NQ], le[NQ];  // this lane's best candidate: probability bits and expert index
@@ -203,13 +226,14 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
 // so that it reads four steps of the chain at a time.
 // NL = 8: `dot` (src/matrix.rs:26-40).  NL = 32: the quantized router's dot_lanes::<32> (src/quantized.rs:154-177), its
 // int8 rows widened on their way into LDS, the sum times the row's scale (:61).
-// The norm is RmsNorm::forward (src/norm.rs:41-61): the squares are laid down in column order beside the rows and one
-// thread a row adds them up in index order, as the reference does.
+// The norm is RmsNorm::forward (src/norm.rs:41-61), its squares added up in index order as the reference does: a wave a row
+// (ordered_sum_wave) straight from memory, which lays the normed row down - or, at widths that do not divide among its lanes,
+// squares in column order beside the rows and one thread a row.
 // Measured, against route_fused_kernel (and the norm's launch in front of it): d 768, 203 tokens x 16 experts 9.5 us
-// against 18.1, with the norm 14.4 against 32.2; 4096 x 8 10.5 against 17.7; 8192 x 16 17.3 against 19.0 (median
-// inside a forward 20.9 against 22.8).  Of the 14.4:
-// rows staged 2.8 us into the workgroup, normed at 6.8 (half of it the chain of 768 adds), logits at 9.1, softmax and
-// top-k at 11.2, end 12.3.
+// against 18.1, with the norm 11.2 (one chain a row 14.4) against 32.2; 4096 x 8 10.1 against 17.7; 8192 x 16 17.3 against
+// 19.0 (median inside a forward 20.9 against 22.8).  With the norm, 8 tokens of d 768 by a quantized router of 8 experts:
+// rows there 1.2 us into the workgroup, their sums at 2.6, normed rows at 3.1, router rows in place at 3.7, logits at 6.9,
+// softmax and top-k at 9.1, end 9.4.
 // ---------------------------------------------------------------------------
 struct RouteRowsArgs {
     const void* x;
@@ -245,18 +269,22 @@ __host__ __device__ static int route_shared_floats(int d, int TB, int EG, int pi
 }
 __host__ __device__ static size_t route_rows_lds_bytes(int E, int k, int d, int TB, int NL, int EG, bool norm) {
     const int pitch = NL * route_lane_pitch(d, NL);
+    const bool chain = norm && !wave_norms(d);
     return router_fixed_bytes(E, k, TB) +
-           ((size_t)TB * pitch + route_shared_floats(d, TB, EG, pitch, norm) + (norm ? d + TB : 0)) * 4;
+           ((size_t)TB * pitch + route_shared_floats(d, TB, EG, pitch, chain) + (chain ? d + TB : 0)) * 4;
 }
 
 // The logits of the TB tokens of block `blk` into the `prob` array (row pitch E | 1) of `lds_raw`, with everything in
-// front of them; the caller meets at a barrier before it reads them.
-template <typename XT, int TB, int NL, int TT, int EE>
+// front of them; the caller meets at a barrier before it reads them.  Kernels without the norm are compiled without its code:
+// with it they are 50 KB long instead of 25 and take 150 registers instead of 100, and 4096 tokens of d 768 by 8 experts are
+// routed in 10.4 us instead of 10.1.
+template <typename XT, int TB, int NL, int TT, int EE, bool NORM>
 __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk, unsigned char* __restrict__ lds_raw) {
     constexpr int NT = kRouterThreads;
     const int T = a.T, d = a.d, E = a.E, k = a.k, EG = a.EG;
     const int ES = E | 1;
-    const bool norm = a.norm_w != nullptr;
+    constexpr bool norm = NORM;
+    const bool wave_norm = norm && wave_norms(d);
     float* const prob = reinterpret_cast<float*>(lds_raw);
     const int lp = route_lane_pitch(d, NL), pitch = NL * lp;
     float* const xs = reinterpret_cast<float*>(lds_raw + router_fixed_bytes(E, k, TB));
@@ -329,7 +357,58 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
     if (short_n > 0)
         for (int i = tid; i < TB * NL * short_n; i += NT) xs[(i / short_n) * lp + short_from + i % short_n] = 0.0f;
     const int nw0 = min(EG, E) * wpr, nx = nt * xpr;
-    {
+    if (wave_norm) {
+        // a wave a row: the raw elements in registers, normed, rounded to the layer's own type and laid down; each half of the
+        // wave takes half of a lane's elements.  The router's rows are put into place meanwhile by whoever is free.
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = (tid >> 5) & 1;
+        const XT* const rows = static_cast<const XT*>(a.x) + (size_t)t0 * d;
+        with_lane_elements(d, [&](auto l_tag) {
+            constexpr int L = decltype(l_tag)::value, H = L / 2;
+            const int c0 = (tid & 31) * L + half * H;
+            LaneRow<XT, L> row;
+            row.load(rows + (size_t)min(wave, nt - 1) * d);
+            float4 nwv[H / 4];
+#pragma unroll
+            for (int i = 0; i < H / 4; ++i) nwv[i] = *reinterpret_cast<const float4*>(a.norm_w + c0 + 4 * i);
+            const Six w = request(router_src(0), nw0, tid);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+            for (int r = wave; r < nt; r += NT / 64) {
+                const float inv_r = row.inverse_rms(a.norm_eps);
+                float v[L];
+                row.widen(v);
+                if (r + NT / 64 < nt) row.load(rows + (size_t)(r + NT / 64) * d);
+                float* const to = xs + r * pitch;
+                XT o[H];
+#pragma unroll
+                for (int i = 0; i < H; ++i) {
+                    const float4 n4 = nwv[i / 4];
+                    const float n = i % 4 == 0 ? n4.x : i % 4 == 1 ? n4.y : i % 4 == 2 ? n4.z : n4.w;
+                    o[i] = from_f32<XT>(__fmul_rn(__fmul_rn(half ? v[H + i] : v[i], inv_r), n));
+                    const int c = c0 + i;
+                    to[(c % NL) * lp + c / NL] = to_f32(o[i]);
+                }
+                auto put4 = [&](auto* base, int i) {  // four neighbours of the row in memory
+                    typedef typename std::remove_pointer<decltype(base)>::type T;
+                    T* const at = base + (size_t)(t0 + r) * d + c0 + 4 * i;
+                    const float f[4] = {to_f32(o[4 * i]), to_f32(o[4 * i + 1]), to_f32(o[4 * i + 2]), to_f32(o[4 * i + 3])};
+                    if constexpr (sizeof(T) == 4)
+                        *reinterpret_cast<float4*>(at) = make_float4(f[0], f[1], f[2], f[3]);
+                    else
+                        *reinterpret_cast<uint2*>(at) = make_uint2(f32_to_bf16_bits(f[0]) | ((uint32_t)f32_to_bf16_bits(f[1]) << 16),
+                                                                   f32_to_bf16_bits(f[2]) | ((uint32_t)f32_to_bf16_bits(f[3]) << 16));
+                };
+#pragma unroll
+                for (int i = 0; i < H / 4; ++i) {
+                    if (a.xn_out != nullptr) put4(static_cast<XT*>(a.xn_out), i);
+                    if constexpr (sizeof(XT) == 4)
+                        if (a.rows16 != nullptr) put4(a.rows16, i);
+                }
+            }
+            deliver(w, nw0, tid, put_router);
+            rest_of_router(0, nw0, 6 * NT);
+        });
+    } else {
         const uint4* const xsrc = reinterpret_cast<const uint4*>(static_cast<const XT*>(a.x) + (size_t)t0 * d);
         const Six w = request(router_src(0), nw0, tid);
         const Six x = request(xsrc, nx, tid);
@@ -354,7 +433,7 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
         if (short_n > 0)
             for (int i = tid; i < EG * NL * short_n; i += NT) ws[(i / short_n) * lp + short_from + i % short_n] = 0.0f;
     }
-    if (norm || a.rows16 != nullptr) {
+    if (!wave_norm && (norm || a.rows16 != nullptr)) {
         if (!norm) __syncthreads();
         // the normed rows, rounded to the layer's own type, replace the raw ones; they (and the bf16 copy of f32 rows
         // for the expert products) are written out on the way
@@ -458,7 +537,8 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
             }
             if (q < quads) multiply(oa);
             // the column lanes folded left to right: lane l of a group holds ((0 + a_0) + a_1) + ... + a_l after l steps
-            // of "take the lane below's sum, add your own" (see softmax_topk), the products side by side
+            // of "take the lane below's sum, add your own" (see softmax_topk), the products side by side: one add a step,
+            // where keeping a group's first lane apart took three instructions (32 column lanes, 8 tokens x 8 experts: 0.5 us)
             float own[TT][EE];
 #pragma unroll
             for (int u = 0; u < TT; ++u)
@@ -471,11 +551,8 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
 #pragma unroll
                 for (int u = 0; u < TT; ++u)
 #pragma unroll
-                    for (int v = 0; v < EE; ++v) {
-                        const float below = __uint_as_float(lanes_from<0x138>(__float_as_uint(acc[u][v])));  // wave_shr:1
-                        const float next = __fadd_rn(below, own[u][v]);
-                        acc[u][v] = j == 0 ? acc[u][v] : next;
-                    }
+                    for (int v = 0; v < EE; ++v)
+                        acc[u][v] = __fadd_rn(__uint_as_float(lanes_from<0x138>(__float_as_uint(acc[u][v]))), own[u][v]);  // wave_shr:1
             }
 #pragma unroll
             for (int u = 0; u < TT; ++u)

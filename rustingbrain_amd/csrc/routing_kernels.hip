@@ -576,10 +576,10 @@ __global__ __launch_bounds__(kRouterThreads) void route_fused_kernel(
 }
 
 // Norm (optional), logits and everything behind them for TB tokens a workgroup (see route_rows_body).
-template <typename XT, int TB, int NL, int TT, int EE>
+template <typename XT, int TB, int NL, int TT, int EE, bool NORM>
 __global__ __launch_bounds__(kRouterThreads, 2) void route_rows_kernel(RouteRowsArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    route_rows_body<XT, TB, NL, TT, EE>(a, blockIdx.x, lds_raw);
+    route_rows_body<XT, TB, NL, TT, EE, NORM>(a, blockIdx.x, lds_raw);
     __syncthreads();
     router_tail<1, true, TB>(lds_raw, blockIdx.x, a.valid, a.T, a.E, a.k, a.P, a.lse, a.expert_of, a.gate_of, a.rank_in_block,
                              a.blockcnt, a.partial);
@@ -1255,8 +1255,9 @@ RouterPlan plan_router(const RouterArgs& a, bool bf16) {
     q.block_tokens = p.tokens ? p.tokens : kRouterTokens;
     q.row_experts = p.tokens ? p.EG : 0;
     q.row_lds = p.tokens ? p.lds : 0;
-    // the squares' room costs tokens a workgroup, and a second round of workgroups costs more than the norm in a
-    // launch of its own (8192 tokens, d 768: 37.7 us in two rounds, 16.2 + 8 in two launches)
+    // where the squares' room costs tokens a workgroup, a second round of workgroups costs more than the norm in a launch of
+    // its own (8192 tokens, d 768, squares in LDS: 37.7 us in two rounds, 16.2 + 8 in two launches; a wave a row leaves one
+    // round: 29 in one launch, 12.5 + 20 in two)
     q.takes_norm = a.norm_w && p.tokens && (a.T + p.tokens - 1) / p.tokens <= 256;
     q.q8_writes_rows16 = p.tokens != 0;
     return q;
@@ -1291,8 +1292,9 @@ static hipError_t launch_rows_t(const RouterArgs& a, const RouterPlan& p, hipStr
         RB_LAUNCH(kernel.value, grid, dim3(kRouterThreads), p.row_lds, s, r);
         return hipGetLastError();
     };
-#define RB_ROUTE_ROWS(TB, NL, TT, EE) \
-    go(std::integral_constant<void (*)(RouteRowsArgs), &route_rows_kernel<XT, TB, NL, TT, EE>>{})
+#define RB_ROUTE_ROWS(TB, NL, TT, EE)                                                                                    \
+    (a.norm_w ? go(std::integral_constant<void (*)(RouteRowsArgs), &route_rows_kernel<XT, TB, NL, TT, EE, true>>{})     \
+              : go(std::integral_constant<void (*)(RouteRowsArgs), &route_rows_kernel<XT, TB, NL, TT, EE, false>>{}))
     // tokens x experts a thread: the largest tile that still has work for every thread (more sums a thread mean less
     // traffic with LDS; the sums of 8 tokens x 16 experts take 2.3 us with 1 x 2 on eight waves, 2.9 with 2 x 2 on four)
     if (a.wq) {
@@ -1438,7 +1440,7 @@ static hipError_t launch_combine_t(const CombineArgs& a, hipStream_t s) {
 // come out identical; the output is (value * inverse_rms) * weight, two separately rounded
 // products as in the reference.
 //
-// The chain of d dependent additions per row is the floor of this kernel (1.9 us for 768 columns).  To keep everything
+// The chain of d dependent additions per row is the floor of this kernel (2.6 us for 768 columns).  To keep everything
 // else off that chain, a block copies its R rows into LDS with every lane's loads in flight at once (the rows of a block
 // are one contiguous range) and lays their squares beside them, lane r of the first wave adds up the squares of row r,
 // then the whole block writes the normed rows from the LDS copy - the input is read from memory once.
@@ -1524,9 +1526,10 @@ template <typename XT>
 hipError_t launch_rmsnorm_t(const XT* x, const float* weight, float eps, int T, int d, XT* out, hipStream_t s) {
     const bool pieces_ok = d % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
                            (reinterpret_cast<uintptr_t>(out) & 15) == 0 && (reinterpret_cast<uintptr_t>(weight) & 15) == 0;
-    // rows a block: few enough that the rows' chains spread over the chip (the chain of one row is the time of a small
-    // call), enough blocks a compute unit for the loads of one to cover the chain of another
     auto lds_of = [&](int R) { return (((size_t)R * d * sizeof(XT) + 15) & ~(size_t)15) + (size_t)R * (d + 4) * 4 + 256; };
+    // rows a block: few enough that the rows' chains spread over the chip (the chain of one row is the time of a small
+    // call), enough blocks a compute unit for the loads of one to cover the chain of another (a chain a lane is fewer
+    // instructions a row than ordered_sum_wave: 16384 rows, d 768 19 us, a wave a row 27)
     if (pieces_ok && lds_of(1) <= 64 * 1024) {
         int R = std::max(1, std::min(16, (T + 1023) / 1024));
         while (R > 1 && lds_of(R) > 40 * 1024) --R;

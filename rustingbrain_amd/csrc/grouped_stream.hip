@@ -8,8 +8,9 @@
 //                pack_weight_bf16 / pack_weight_i8); every wave streams its own
 //                fragments global -> VGPR through a 4-deep register ring, i.e.
 //                the load for reduction step g + 3 is issued while step g runs.
-//                int8 weights are widened to bf16 in registers right before the
-//                multiply; the per-row scale multiplies the accumulator.
+//                int8 weights are widened to bf16 in registers during the step
+//                before their multiplies; the per-row scale multiplies the
+//                accumulator.
 //   activations  128 token rows per workgroup (gathered through an index for
 //                the gate/up product) go global -> LDS with the LDS-DMA load
 //                (global_load_lds_dwordx4): lane l of a wave deposits its 16
@@ -151,8 +152,11 @@ struct Slot<true> {
     }
     __device__ __forceinline__ void load0(const char* p0, uint32_t off) { issue_load(f0, off, p0); }
     __device__ __forceinline__ void load1(const char* p1, uint32_t off) { issue_load(f1, off, p1); }
-    __device__ __forceinline__ bf16x8 a0() const { return widen_i8(make_uint2(f0.x, f0.y)); }
-    __device__ __forceinline__ bf16x8 a1() const { return widen_i8(make_uint2(f1.x, f1.y)); }
+    // pair i of the eight that the two fragments are, widened
+    __device__ __forceinline__ uint32_t pair(int i) const {
+        const u32x2& f = i < 4 ? f0 : f1;
+        return widen2((i & 2) ? f.y : f.x, 16 * (i & 1));
+    }
 };
 
 // ---- epilogue: the accumulators of one tile to memory -------------------------------------------------
@@ -361,6 +365,11 @@ __device__ __forceinline__ void write_swiglu_backward(const TileOut& o, floatx16
 // ring loads of step g when step g waits for them (they were issued in step g - D, D = 3): the DMA of that
 // step if it was a last step, then two ring loads per step in between and four DMA if one of them was a last
 // step - 8 in all for the steps 0 .. KS-2 of a slice, 4 for the last one.
+// int8 weights are widened a step ahead, a pair or two behind each multiply: 24 instructions of eight cycles, which in front
+// of the step's multiplies (256 cycles) left the matrix cores idle wherever the SIMD's other wave did not fill them.  So
+// step g waits for the weights of step g + 1, and the loads of step g + 4 take the registers that step g's have left: issued
+// in step g - 3 they have the same younger instructions.  A forward, d 768, 8 experts of 1408, widened in front / a step ahead:
+// 3000 tokens 85.1 / 82.3 us, 4096 94.4 / 92.6, 8192 153.5 / 150.2 (gate/up at 4096 43.8 / 40.9 before the clock falls).
 struct PipeCtx {
     const uint4* As;      // three LDS stages of one activation slice each
     uint32_t lds0;        // LDS byte address of this wave's rows in stage 0
@@ -378,8 +387,8 @@ struct PipeCtx {
 template <bool I8, int NB>
 __device__ __forceinline__ void pipe_loop(const PipeCtx& c, floatx16 (&acc)[2][TT], Slot<I8> (&ring)[KS],
                                           const uint32_t (&a_src)[DMA_PER_WAVE]) {
-    constexpr int D = RING - 1;
-    static_assert(KS == 4 && D == 3, "the wait counts below are derived for this configuration");
+    constexpr int D = I8 ? RING : RING - 1;
+    static_assert(KS == 4 && RING == 4, "the wait counts below are derived for this configuration");
     const uint4* const As = c.As;
     const uint32_t lds0 = c.lds0, lane16 = c.lane16;
     const char* const a_base = c.a_base;
@@ -395,6 +404,9 @@ __device__ __forceinline__ void pipe_loop(const PipeCtx& c, floatx16 (&acc)[2][T
     bf16x8 tf[2][TT];
 #pragma unroll
     for (int t = 0; t < NB; ++t) tf[0][t] = lds_frag(As, t * 32 * CPR + frag0);
+    u32x4 wide[2][2];  // int8: the step's two fragments, and the next step's as they are widened
+    if constexpr (I8)
+        static_for<0, 8>([&](auto i) { wide[0][decltype(i)::value >> 2][decltype(i)::value & 3] = ring[0].pair(decltype(i)::value); });
     auto pslice = [&](int kt, auto idx_tag) {
         constexpr int IDX = decltype(idx_tag)::value;
         constexpr int BUF = IDX % 3, NEXT = (IDX + 1) % 3, FREE = (IDX + 2) % 3;
@@ -405,11 +417,17 @@ __device__ __forceinline__ void pipe_loop(const PipeCtx& c, floatx16 (&acc)[2][T
             constexpr int s = decltype(s_tag)::value;
             constexpr bool LAST = s == KS - 1;
             const int g = kt * KS + s;
-            Slot<I8>& cur = ring[s % RING];
+            Slot<I8>& cur = ring[(I8 ? s + 1 : s) % RING];  // whose loads are awaited here
             Slot<I8>& nxt = ring[(s + D) % RING];
-            wait_for<LAST ? 2 * (D - 1) : 2 * (D - 1) + DMA_PER_WAVE>(cur.f0, cur.f1);
-            const bf16x8 w0 = cur.a0();
-            const bf16x8 w1 = cur.a1();
+            wait_for<LAST ? 2 * (RING - 2) : 2 * (RING - 2) + DMA_PER_WAVE>(cur.f0, cur.f1);
+            bf16x8 w0, w1;
+            if constexpr (I8) {
+                w0 = __builtin_bit_cast(bf16x8, wide[s & 1][0]);
+                w1 = __builtin_bit_cast(bf16x8, wide[s & 1][1]);
+            } else {
+                w0 = cur.a0();
+                w1 = cur.a1();
+            }
             const uint32_t woff = Slot<I8>::offset(min(g + D, GS - 1), lane16);
             const uint32_t aoff = (uint32_t)min(kt + 2, KT - 1) * (BK * 2);
             const int frag = frag0 ^ (2 * ((s + 1) % KS));
@@ -434,6 +452,11 @@ __device__ __forceinline__ void pipe_loop(const PipeCtx& c, floatx16 (&acc)[2][T
                 constexpr int b = m & 1, t = m >> 1;
                 acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b ? w1 : w0, tf[s & 1][t], acc[b][t], 0, 0, 0);
                 if constexpr (m < NOPS) op(m_tag);
+                if constexpr (I8)
+                    static_for<m * 8 / (2 * NB), (m + 1) * 8 / (2 * NB)>([&](auto i_tag) {
+                        constexpr int i = decltype(i_tag)::value;
+                        wide[(s + 1) & 1][i >> 2][i & 3] = cur.pair(i);
+                    });
                 __builtin_amdgcn_sched_barrier(0);
             });
             static_for<2 * NB, NOPS>(op);
@@ -601,7 +624,7 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
 
     const int KT = K / BK;
     const int GS = KT * KS;  // reduction steps in all
-    constexpr int D = RING - 1;  // the load for step g + D is issued while step g runs
+    constexpr int D = I8 ? RING : RING - 1;  // the load for step g + D is issued while step g runs
 
     // ---- prologue: the first STAGES - 1 activation slices, the first D weight steps; nothing is in flight
     // where the loop is entered (the compiler may copy registers there)
@@ -670,7 +693,7 @@ template <>
 struct Slot1<true> {
     u32x2 f;
     static __device__ __forceinline__ uint32_t offset(int g, uint32_t lane16) { return Slot<true>::offset(g, lane16); }
-    __device__ __forceinline__ bf16x8 frag() const { return widen_i8(make_uint2(f.x, f.y)); }
+    __device__ __forceinline__ uint32_t pair(int i) const { return widen2((i & 2) ? f.y : f.x, 16 * (i & 1)); }
 };
 
 template <int N, typename V>
@@ -678,12 +701,12 @@ __device__ __forceinline__ void wait_for1(V& a) {
     asm volatile("s_waitcnt vmcnt(%1)" : "+v"(a) : "n"(N));
 }
 
-// As pipe_loop: before the call nothing is outstanding (slices 0 .. NSTAGES - 2 and ring steps 0 .. NRING - 2 have
+// As pipe_loop: before the call nothing is outstanding (slices 0 .. NSTAGES - 2 and ring steps 0 .. D - 1 have
 // landed) and the workgroup has met at a barrier; after it nothing is outstanding.
 template <bool I8, int NB>
 __device__ __forceinline__ void narrow_loop(const PipeCtx& c, floatx16 (&acc)[TT], Slot1<I8> (&ring)[NRING],
                                             const uint32_t (&a_src)[DMA_PER_WAVE]) {
-    constexpr int D = NRING - 1;
+    constexpr int D = I8 ? NRING : NRING - 1;  // (int8 weights are widened a step ahead, as above)
     static_assert(KS == 4 && NRING == 16 && NSTAGES == 4 && DMA_PER_WAVE == 4 && TT == 4, "the wait counts are derived for this");
     const uint4* const As = c.As;
     const uint32_t lds0 = c.lds0, lane16 = c.lane16;
@@ -694,6 +717,9 @@ __device__ __forceinline__ void narrow_loop(const PipeCtx& c, floatx16 (&acc)[TT
     bf16x8 tf[2][TT];
 #pragma unroll
     for (int t = 0; t < NB; ++t) tf[0][t] = lds_frag(As, t * 32 * CPR + frag0);
+    u32x4 wide[2];
+    if constexpr (I8)
+        static_for<0, 4>([&](auto i) { wide[0][decltype(i)::value] = ring[0].pair(decltype(i)::value); });
     auto pslice = [&](int kt, auto idx_tag) {
         constexpr int IDX = decltype(idx_tag)::value;  // kt % 4
         constexpr int NEXT = (IDX + 1) % NSTAGES, FREE = (IDX + 3) % NSTAGES;
@@ -705,8 +731,11 @@ __device__ __forceinline__ void narrow_loop(const PipeCtx& c, floatx16 (&acc)[TT
             constexpr bool LAST = s == KS - 1;
             constexpr int P = IDX * KS + s;  // ring position of step g
             const int g = kt * KS + s;
-            wait_for1<(D - 1) + DMA_PER_WAVE * (LAST ? 3 : 4)>(ring[P].f);
-            const bf16x8 w = ring[P].frag();
+            Slot1<I8>& cur = ring[(I8 ? P + 1 : P) % NRING];  // whose load is awaited here
+            wait_for1<(NRING - 2) + DMA_PER_WAVE * (LAST ? 3 : 4)>(cur.f);
+            bf16x8 w;
+            if constexpr (I8) w = __builtin_bit_cast(bf16x8, wide[s & 1]);
+            else w = cur.frag();
             const uint32_t woff = Slot1<I8>::offset(min(g + D, GS - 1), lane16);
             const uint32_t aoff = (uint32_t)min(kt + 3, KT - 1) * (BK * 2);
             const int frag = frag0 ^ (2 * ((s + 1) % KS));
@@ -726,6 +755,11 @@ __device__ __forceinline__ void narrow_loop(const PipeCtx& c, floatx16 (&acc)[TT
                 constexpr int m = decltype(m_tag)::value;
                 acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, tf[s & 1][m], acc[m], 0, 0, 0);
                 if constexpr (m < NOPS) op(m_tag);
+                if constexpr (I8)
+                    static_for<m * 4 / NB, (m + 1) * 4 / NB>([&](auto i_tag) {
+                        constexpr int i = decltype(i_tag)::value;
+                        wide[(s + 1) & 1][i] = cur.pair(i);
+                    });
                 __builtin_amdgcn_sched_barrier(0);
             });
             static_for<NB, NOPS>(op);
@@ -819,7 +853,7 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
 
     Slot1<I8> ring[NRING];
 #pragma unroll
-    for (int g = 0; g < NRING - 1; ++g) issue_load(ring[g].f, Slot1<I8>::offset(min(g, GS - 1), lane16), wp);
+    for (int g = 0; g < (I8 ? NRING : NRING - 1); ++g) issue_load(ring[g].f, Slot1<I8>::offset(min(g, GS - 1), lane16), wp);
     static_for<0, NSTAGES - 1>([&](auto st) {
         constexpr int ST = decltype(st)::value;
 #pragma unroll
@@ -907,12 +941,12 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
 // against narrow, d 768, K 1408: 48 tiles (203 rows over 16 experts) 17.2 / 10.6 (the launch alone), 117 tiles (2000 rows)
 // 65.1 / 59.0, 129 (2500 rows over 8) 68.6 / 63.3, 141 (2500 rows over 16) 76.4 / 77.2, 165 (3000 rows) 78.8 / 79.8, 186 (3500)
 // 90.7 / 95.1.  Short reductions (the default model's 384) are mostly first loads and stores: 156 tiles 47.5 / 46.2, 244
-// tiles 69.4 / 67.4, 392 the same.  int8 weights: 129 tiles 71.2 / 62.8, 174 tiles 83.4 / 80.8, 204 tiles 90.1 / 87.6, 246
-// tiles 104.6 / 105.5.
+// tiles 69.4 / 67.4, 392 the same.  int8 weights: 129 tiles 65.6 / 66.0, 156 tiles 82.3 / 83.1, 180 tiles 83.9 / 84.2, 204 tiles
+// 92.6 / 92.2; 156 tiles of 16 experts 78.8 / 79.7.
 // Gate/up workgroups are twice as many per tile (64 features): 81 tiles (K 512) 39.9 / 38.9, 88 (int8, K 768) 43.9 / 41.7, 156
 // 42.5 / 46.0, 176 (K 768, the launch alone) 15.0 / 16.5.
 // Launches that keep or read pre-activations (training) stay with the wide kernel's epilogue.
-constexpr int narrow_tiles(bool swiglu, bool i8, int K) { return swiglu ? 128 : i8 ? 210 : K <= 512 ? 250 : 140; }
+constexpr int narrow_tiles(bool swiglu, int K) { return swiglu ? 128 : K <= 512 ? 250 : 140; }
 
 template <bool SWIGLU, bool I8>
 hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
@@ -926,7 +960,7 @@ hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
                         static_cast<bf16_t*>(d2.out), static_cast<bf16_t*>(d2.gu_out)};
     const int group_m = g.group_m > 0 ? g.group_m : 8;
     const int likely = g.dense_rows < 0 && g.likely_tiles > 0 ? tiles(g.likely_tiles, BN) : total;
-    if (likely <= narrow_tiles(SWIGLU, I8, g.K) && !g.gu_out && !g.swiglu_grad_gu) {
+    if (likely <= narrow_tiles(SWIGLU, g.K) && !g.gu_out && !g.swiglu_grad_gu) {
         RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((tiles(tiles_m, BN / 2) + 7) / 8 * 8), dim3(NT), 0, s,
                   static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
                   g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,

@@ -35,6 +35,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "layout_device.h"
 #include "rbmoe_kernels.h"
 
 // Hook for timeline studies of the kernels: a harness that includes this file may define it to record a time
@@ -530,13 +531,24 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     size_t w_expert_stride_bytes, const float* __restrict__ scales, size_t s_expert_stride, int N, int K,
     const int* __restrict__ tile_expert, const int* __restrict__ tile_row0, const int* __restrict__ tile_rows,
     const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, bf16_t* __restrict__ gu_out,
-    const bf16_t* __restrict__ bw_gu, int group_m, DenseGroup g2) {
+    const bf16_t* __restrict__ bw_gu, int group_m, DenseGroup g2, RoutedSlots slots) {
     constexpr int BN = SWIGLU ? NW * 32 : NW * 64;  // output features per workgroup
     // LDS stages of one activation slice each; the epilogue reuses the first two as one
     // 128 x 128 staging tile for the output.
     __shared__ uint4 As[STAGES * BM * CPR];
 
-    const TileAt at = tile_at<BN>(dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
+    // without tables: what the router left behind (RoutedSlots), worked out in the stages' room; the rows' tokens lie in the
+    // stage that is filled last, behind a barrier
+    const bool own = SWIGLU && slots.expert_of != nullptr;  // uniform over the launch
+    SlotsLds& sl = *reinterpret_cast<SlotsLds*>(As);
+    static_assert(sizeof(SlotsLds) <= (STAGES - 1) * BM * CPR * sizeof(uint4), "in front of the tokens");
+    int* const own_token = reinterpret_cast<int*>(As + (STAGES - 1) * BM * CPR);
+    RoutedCounts rc{};
+    if (own) {
+        if (blockIdx.x == gridDim.x - 1) return routed_rest(slots, reinterpret_cast<unsigned char*>(As));
+        rc = routed_counts<NT>(slots, sl);
+    }
+    const TileAt at = tile_at<BN>(own ? rc.ntiles : dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
     if (at.tm < 0) return;
     const int tm_idx = at.tm, tn_idx = at.tn;
     if (at.second) {
@@ -557,6 +569,11 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
         expert = 0;
         row0 = tm_idx * BM;
         rows = min(BM, dense_rows - row0);
+    } else if (own) {
+        const RoutedTile t = routed_tile<NT>(slots, rc, tm_idx, tn_idx == 0, sl, own_token);
+        expert = t.expert;
+        row0 = t.row0;
+        rows = t.rows;
     } else {
         expert = tile_expert[tm_idx];
         row0 = tile_row0[tm_idx];
@@ -599,7 +616,7 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     for (int j = 0; j < DMA_PER_WAVE; ++j) {
         const int r = wave * (BM / NW) + j * 8 + (lane >> 3);
         const int rr = r < rows ? r : 0;
-        const int grow = row_index ? row_index[row0 + rr] : row0 + rr;
+        const int grow = own && !at.second ? own_token[rr] : row_index ? row_index[row0 + rr] : row0 + rr;
         a_src[j] = ((uint32_t)grow * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)As + wave * (BM / NW) * CPR * 16;
@@ -789,11 +806,22 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
     const bf16_t* __restrict__ a, const int* __restrict__ row_index, const void* __restrict__ wpacked,
     size_t w_expert_stride_bytes, const float* __restrict__ scales, size_t s_expert_stride, int N, int K,
     const int* __restrict__ tile_expert, const int* __restrict__ tile_row0, const int* __restrict__ tile_rows,
-    const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, int group_m, DenseGroup g2) {
+    const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, int group_m, DenseGroup g2, RoutedSlots slots) {
     constexpr int BN = SWIGLU ? 64 : 128;  // output features per workgroup
     __shared__ uint4 As[NSTAGES * BM * CPR];
 
-    const TileAt at = tile_at<BN>(dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
+    // without tables: what the router left behind (RoutedSlots), worked out in the stages' room; the rows' tokens lie in the
+    // stage that is filled last, behind a barrier
+    const bool own = SWIGLU && slots.expert_of != nullptr;  // uniform over the launch
+    SlotsLds& sl = *reinterpret_cast<SlotsLds*>(As);
+    static_assert(sizeof(SlotsLds) <= (NSTAGES - 1) * BM * CPR * sizeof(uint4), "in front of the tokens");
+    int* const own_token = reinterpret_cast<int*>(As + (NSTAGES - 1) * BM * CPR);
+    RoutedCounts rc{};
+    if (own) {
+        if (blockIdx.x == gridDim.x - 1) return routed_rest(slots, reinterpret_cast<unsigned char*>(As));
+        rc = routed_counts<NT>(slots, sl);
+    }
+    const TileAt at = tile_at<BN>(own ? rc.ntiles : dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
     if (at.tm < 0) return;
     const int tm_idx = at.tm, tn_idx = at.tn;
     if (at.second) {
@@ -813,6 +841,11 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
         expert = 0;
         row0 = tm_idx * BM;
         rows = min(BM, dense_rows - row0);
+    } else if (own) {
+        const RoutedTile t = routed_tile<NT>(slots, rc, tm_idx, tn_idx == 0, sl, own_token);
+        expert = t.expert;
+        row0 = t.row0;
+        rows = t.rows;
     } else {
         expert = tile_expert[tm_idx];
         row0 = tile_row0[tm_idx];
@@ -839,7 +872,7 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
     for (int j = 0; j < DMA_PER_WAVE; ++j) {
         const int r = wave * (BM / NW) + j * 8 + (lane >> 3);
         const int rr = r < rows ? r : 0;
-        const int grow = row_index ? row_index[row0 + rr] : row0 + rr;
+        const int grow = own && !at.second ? own_token[rr] : row_index ? row_index[row0 + rr] : row0 + rr;
         a_src[j] = ((uint32_t)grow * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)As + wave * (BM / NW) * CPR * 16;
@@ -959,19 +992,20 @@ hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
     const DenseGroup g2{static_cast<const bf16_t*>(d2.a), d2.w, d2.scales, d2.N, d2.K, d2.rows,
                         static_cast<bf16_t*>(d2.out), static_cast<bf16_t*>(d2.gu_out)};
     const int group_m = g.group_m > 0 ? g.group_m : 8;
+    const int rest = SWIGLU && g.slots.expert_of ? 1 : 0;  // (routed_rest)
     const int likely = g.dense_rows < 0 && g.likely_tiles > 0 ? tiles(g.likely_tiles, BN) : total;
     if (likely <= narrow_tiles(SWIGLU, g.K) && !g.gu_out && !g.swiglu_grad_gu) {
-        RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((tiles(tiles_m, BN / 2) + 7) / 8 * 8), dim3(NT), 0, s,
+        RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((tiles(tiles_m, BN / 2) + 7) / 8 * 8 + rest), dim3(NT), 0, s,
                   static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
                   g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
-                  static_cast<bf16_t*>(g.out), group_m, g2);
+                  static_cast<bf16_t*>(g.out), group_m, g2, g.slots);
         return hipGetLastError();
     }
-    RB_LAUNCH((grouped_stream_kernel<SWIGLU, I8>), dim3((total + 7) / 8 * 8), dim3(NT), 0, s,
+    RB_LAUNCH((grouped_stream_kernel<SWIGLU, I8>), dim3((total + 7) / 8 * 8 + rest), dim3(NT), 0, s,
               static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
               g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
               static_cast<bf16_t*>(g.out), static_cast<bf16_t*>(g.gu_out), static_cast<const bf16_t*>(g.swiglu_grad_gu),
-              group_m, g2);
+              group_m, g2, g.slots);
     return hipGetLastError();
 }
 
@@ -987,6 +1021,7 @@ hipError_t launch_grouped_stream(const GroupedArgs& g, WeightKind wk, hipStream_
     if (!stream_shape_ok(g.N, g.K)) return hipErrorInvalidValue;
     if (g.dense2.rows > 0 && (!stream_shape_ok(g.dense2.N, g.dense2.K) || !g.dense2.gu_out != !g.gu_out || g.swiglu_grad_gu))
         return hipErrorInvalidValue;
+    if (g.slots.expert_of && (!g.swiglu || g.dense_rows >= 0 || g.slots.layout.tile_m != BM)) return hipErrorInvalidValue;
     if (g.swiglu_grad_gu && (g.swiglu || wk != WeightKind::BF16)) return hipErrorInvalidValue;
     if (wk == WeightKind::BF16) return g.swiglu ? launch_t<true, false>(g, s) : launch_t<false, false>(g, s);
     if (wk == WeightKind::I8) return g.swiglu ? launch_t<true, true>(g, s) : launch_t<false, true>(g, s);

@@ -1441,14 +1441,6 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     da.ntiles = (int*)L->ntiles.p; da.losses = (float*)L->losses.p;
     da.perm_slot = (int*)L->perm_slot.p; da.perm_token = (int*)L->perm_token.p; da.inv_pos = (int*)L->inv_pos.p;
     da.xg = gather_in_product ? nullptr : L->xg.p;
-    HIP_TRY(ctx, launch_dispatch(da, abf || cast, s));
-    if (L->record_routed) HIP_TRY(ctx, hipEventRecord(L->record_routed, s));
-    {
-        const bool rows_bf16 = abf || cast;
-        L->replay[RBMOE_STAGE_DISPATCH] = [=](hipStream_t st) { return launch_dispatch(da, rows_bf16, st); };
-    }
-    HIP_TRY(ctx, mark(3));
-
     GroupedArgs g1{};
     g1.a = gather_in_product ? xe : L->xg.p;
     g1.row_index = gather_in_product ? (const int*)L->perm_token.p : nullptr;
@@ -1472,7 +1464,27 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     g1.swiglu = true;
     g1.group_m = L->group_m;
     if (L->training) g1.gu_out = L->gu.p;
-    HIP_TRY(ctx, run(shared_inside ? with_shared(g1, s1) : g1, true));
+    // No launch for the dispatch: the gate/up product works its tiles out by itself and writes the tables on the way.  The
+    // launch and its chain (4 to 9 us) are saved, but every workgroup's own chain gets longer, so it pays for one round of
+    // workgroups, two a compute unit.  us a forward, without / with the launch, at so many gate/up tiles: d 256, 4 experts of 704,
+    // 40 rows 24.3 / 30.2, 8192 rows (396 tiles) 42.3 / 46.3; d 512, 8 experts of 352 and a shared one, 64 rows 26.8 / 30.9, 2048
+    // (156) 37.1 / 40.7, 6144 (444) 71.2 / 76.3, 8192 (588) 86.2 / 85.0; d 768, 8 of 1408, 64 rows 33.0 / 37.3, 2048 (396) 58.8 / 62.8,
+    // 4096 (748) 87.6 / 83.9; 16 of 1408, 512 rows 41.8 / 45.1, 3072 (616) 79.1 / 80.8, 8192 (1496) 151.0 / 139.4.
+    // (Not where a host call fetches the tables beside the products, nor where the stages are timed one by one.)
+    constexpr int kDispatchInsideTiles = 512;
+    GroupedArgs first = shared_inside ? with_shared(g1, s1) : g1;
+    const int workgroups = g1.likely_tiles * ((F + 127) / 128) + (first.dense2.rows + 127) / 128 * ((first.dense2.N + 127) / 128);
+    const bool dispatch_inside = mfma && gather_in_product && !timed && !L->record_routed && workgroups <= kDispatchInsideTiles &&
+                                 dispatch_in_product_ok(da);
+    if (dispatch_inside) first.slots = routed_slots(da);
+    if (!dispatch_inside) HIP_TRY(ctx, launch_dispatch(da, abf || cast, s));
+    if (L->record_routed) HIP_TRY(ctx, hipEventRecord(L->record_routed, s));
+    {
+        const bool rows_bf16 = abf || cast;
+        L->replay[RBMOE_STAGE_DISPATCH] = [=](hipStream_t st) { return launch_dispatch(da, rows_bf16, st); };
+    }
+    HIP_TRY(ctx, mark(3));
+    HIP_TRY(ctx, run(first, true));
     L->replay[RBMOE_STAGE_GATE_UP] = [=](hipStream_t st) { return run_on(g1, st); };
     HIP_TRY(ctx, mark(4));
 

@@ -138,6 +138,36 @@ struct DispatchArgs {
 };
 hipError_t launch_dispatch(const DispatchArgs& a, bool bf16, hipStream_t s);
 
+// What the router leaves behind and the tables that follow from it (layout_device.h)
+struct LayoutArgs {
+    const int* blockcnt;
+    const float* partial;
+    int T, E, k, TB;
+    float w_aux, w_z;
+    int tile_m;
+    int* counts;
+    int* offsets;
+    int* tile_expert;
+    int* tile_row0;
+    int* tile_rows;
+    int* ntiles;
+    float* losses;
+};
+// ... and the slots, for a gate/up launch that works out its own tiles and writes the tables on the way
+struct RoutedSlots {
+    const int* expert_of = nullptr;  // null: a dispatch launch has made the tables
+    const int* rank_in_block = nullptr;
+    int* perm_slot = nullptr;
+    int* perm_token = nullptr;
+    int* inv_pos = nullptr;
+    uint32_t k_recip = 0;  // 2^32 / k rounded up (k > 1)
+    int tb_shift = 0, tile_shift = 0;  // log2 of a router block's tokens, of a tile's rows
+    LayoutArgs layout{};
+};
+// Whether the gate/up product can do the dispatch's work for these arguments, and what it then takes
+bool dispatch_in_product_ok(const DispatchArgs& a);
+RoutedSlots routed_slots(const DispatchArgs& a);
+
 struct CombineArgs {
     const void* y;        // [R, d] expert output rows, activation dtype
     const void* yshared;  // [T, d] or null
@@ -202,6 +232,7 @@ struct GroupedArgs {
     } dense2;
     int group_m;            // MFMA path: M-tiles per scheduling group (0 = default)
     int tile_m = 0;         // rows per tile of the tile table
+    RoutedSlots slots;      // gate/up launches of the bf16 matrix-core kernels: in the place of tile table and row index
 };
 hipError_t launch_grouped_generic(const GroupedArgs& a, bool act_bf16, WeightKind wk, int tile_m,
                                   hipStream_t s);

@@ -18,6 +18,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "layout_device.h"
 #include "routing_device.h"
 
 namespace rbmoe {
@@ -617,40 +618,18 @@ __global__ __launch_bounds__(kRouterThreads) void router_kernel(
 // histograms (O(blocks^2 x experts) reads in total, but one launch less on the critical path);
 // block 0 also writes counts, offsets and the tile table, the last block the losses.
 size_t dispatch_fused_lds_bytes(int E, int k, int tokens) {
-    const int parts = 256 / E;
-    return ((size_t)2 * parts * E + (size_t)parts * (E + 1) + 4 * (size_t)(E + 1) + (size_t)tokens * k) * 4;
+    return layout_lds_bytes(E) + (size_t)tokens * k * 4;
 }
 
 template <typename XT>
 __global__ __launch_bounds__(256) void dispatch_fused_kernel(
-    const XT* __restrict__ x, const int* __restrict__ expert_of, const int* __restrict__ rank_in_block,
-    const int* __restrict__ blockcnt, const float* __restrict__ partial, int T, int d, int E, int k, int TB,
-    float w_aux, float w_z, int tile_m, int* __restrict__ counts, int* __restrict__ offsets,
-    int* __restrict__ tile_expert, int* __restrict__ tile_row0, int* __restrict__ tile_rows,
-    int* __restrict__ ntiles, float* __restrict__ losses, int* __restrict__ perm_slot,
-    int* __restrict__ perm_token, int* __restrict__ inv_pos, XT* __restrict__ xg) {
+    const XT* __restrict__ x, const int* __restrict__ expert_of, const int* __restrict__ rank_in_block, LayoutArgs l, int d,
+    int* __restrict__ perm_slot, int* __restrict__ perm_token, int* __restrict__ inv_pos, XT* __restrict__ xg) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    const int parts = 256 / E;  // E <= 256
-    int* part_all = reinterpret_cast<int*>(lds_raw);           // [parts][E]
-    int* part_before = part_all + parts * E;                   // [parts][E]
-    float* part_mass = reinterpret_cast<float*>(part_before + parts * E);  // [parts][E+1] (block 0)
-    int* cnt = reinterpret_cast<int*>(part_mass + parts * (E + 1));        // [E+1]
-    int* base = cnt + (E + 1);                                 // [E+1]
-    int* off = base + (E + 1);                                 // [E+1]
-    float* mass = reinterpret_cast<float*>(off + (E + 1));     // [E+1]
-    int* lpos = reinterpret_cast<int*>(mass + (E + 1));        // [TB * k]
-
+    const int T = l.T, E = l.E, k = l.k, TB = l.TB;
+    int* const lpos = reinterpret_cast<int*>(lds_raw + layout_lds_bytes(E));  // [TB * k]
     const int tid = threadIdx.x;
     const int blk = blockIdx.x;
-    const int nb = (T + TB - 1) / TB;
-    const int len = (nb + parts - 1) / parts;
-    const int p = tid / E;
-    const int e = tid - p * E;
-    const bool active = p < parts;
-    // Block 0 writes counts, offsets and the tile table; the two losses are the work of another block (the last
-    // one), so that neither of the two is the launch's long pole.  That block fetches the partial sums in the same
-    // batch of loads as the histograms.
-    const bool loss_blk = blk == nb - 1;
     // this thread's first slot does not depend on the scan: fetch it before anything else
     const int t0 = blk * TB;
     const int nt = min(TB, T - t0);
@@ -660,125 +639,12 @@ __global__ __launch_bounds__(256) void dispatch_fused_kernel(
         ex_first = expert_of[(size_t)t0 * k + tid];
         rank_first = rank_in_block[(size_t)t0 * k + tid];
     }
-    if (active) {
-        const int b0 = min(nb, p * len), b1 = min(nb, b0 + len);
-        // Loads in batches of 16 that do not depend on one another: one round trip to L2 per
-        // batch instead of one per block.
-        int s_all = 0, s_before = 0;
-        float m = 0.0f, zs = 0.0f;
-        for (int b = b0; b < b1; b += 16) {
-            int c[16];
-            float v[16], z[16];
-#pragma unroll
-            for (int u = 0; u < 16; ++u) c[u] = b + u < b1 ? blockcnt[(size_t)(b + u) * E + e] : 0;
-            if (loss_blk) {
-#pragma unroll
-                for (int u = 0; u < 16; ++u) {
-                    v[u] = b + u < b1 ? partial[(size_t)(b + u) * (E + 1) + e] : 0.0f;
-                    z[u] = (e == 0 && b + u < b1) ? partial[(size_t)(b + u) * (E + 1) + E] : 0.0f;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                s_all += c[u];
-                s_before += b + u < blk ? c[u] : 0;
-            }
-            if (loss_blk) {
-#pragma unroll
-                for (int u = 0; u < 16; ++u) {
-                    if (b + u < b1) {
-                        m += v[u];
-                        zs += z[u];
-                    }
-                }
-            }
-        }
-        part_all[p * E + e] = s_all;
-        part_before[p * E + e] = s_before;
-        if (loss_blk) {
-            part_mass[p * (E + 1) + e] = m;
-            if (e == 0) part_mass[p * (E + 1) + E] = zs;
-        }
-    }
-    __syncthreads();
-    if (tid < E) {
-        int ca = 0, cb = 0;
-        float m = 0.0f;
-        for (int q = 0; q < parts; ++q) {
-            ca += part_all[q * E + tid];
-            cb += part_before[q * E + tid];
-            if (loss_blk) m += part_mass[q * (E + 1) + tid];
-        }
-        cnt[tid] = ca;
-        base[tid] = cb;
-        mass[tid] = m;
-    }
-    // the sum of lse^2 over the parts: by the last thread of the workgroup, which exists for every expert count
-    // (a thread numbered E does not when E is the workgroup size) and owns no expert column unless E is 256
-    if (loss_blk && tid == 255) {
-        float zs = 0.0f;
-        for (int q = 0; q < parts; ++q) zs += part_mass[q * (E + 1) + E];
-        mass[E] = zs;
-    }
-    __syncthreads();
-    if (E <= 64) {  // exclusive prefix over the experts: one wave, log2(64) shuffle steps
-        if (tid < 64) {
-            const int c = tid < E ? cnt[tid] : 0;
-            int incl = c;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int up = __shfl_up(incl, o);
-                if (tid >= o) incl += up;
-            }
-            if (tid < E) off[tid] = incl - c;
-            if (tid == E - 1) off[E] = incl;
-        }
-    } else if (tid == 0) {
-        int run = 0;
-        for (int q = 0; q < E; ++q) {
-            off[q] = run;
-            run += cnt[q];
-        }
-        off[E] = run;
-    }
-    __syncthreads();
-    if (blk == 0) {
-        if (tid < E) {
-            counts[tid] = cnt[tid];
-            offsets[tid] = off[tid];
-            // tiles of this expert start after the tiles of the experts before it
-            int first = 0;
-            for (int q = 0; q < tid; ++q) first += (cnt[q] + tile_m - 1) / tile_m;
-            const int n = (cnt[tid] + tile_m - 1) / tile_m;
-            for (int i = 0; i < n; ++i) {
-                tile_expert[first + i] = tid;
-                tile_row0[first + i] = off[tid] + i * tile_m;
-                tile_rows[first + i] = min(tile_m, cnt[tid] - i * tile_m);
-            }
-            if (tid == E - 1) ntiles[0] = first + n;
-        }
-        if (tid == 0) offsets[E] = off[E];
-    }
-    if (loss_blk) {
-        // every valid token routes exactly k slots, so the valid-token count is routed / k.  The experts' terms
-        // (two divisions and a product each) side by side, then their sum in expert order by one thread.
-        const int V = off[E] / k;
-        const float tokens = (float)V;
-        const float slots = (float)V * (float)k;
-        float* const term = part_mass;  // [E]: the parts' sums are used up
-        if (tid < E && V > 0) term[tid] = ((float)cnt[tid] / slots) * (mass[tid] / tokens);
-        __syncthreads();
-        if (tid == 0) {
-            float aux = 0.0f, z = 0.0f;
-            if (V > 0) {
-                for (int q = 0; q < E; ++q) aux = aux + term[q];
-                aux = aux * ((float)E * w_aux);
-                z = w_z * mass[E] / tokens;
-            }
-            losses[0] = aux;
-            losses[1] = z;
-        }
-    }
+    // Block 0 writes counts, offsets and the tile table; the two losses are the work of another block (the last
+    // one), so that neither of the two is the launch's long pole.  That block fetches the partial sums in the same
+    // batch of loads as the histograms.
+    const LayoutSums sums = layout_scan(l, blk, blk == 0, blk == (T + TB - 1) / TB - 1, lds_raw);
+    const int* const off = sums.off;
+    const int* const base = sums.base;
 
     for (int ls = tid; ls < nls; ls += 256) {
         const int s = t0 * k + ls;
@@ -1383,15 +1249,38 @@ hipError_t launch_router(const RouterArgs& a, const RouterPlan& p, bool bf16, hi
     return bf16 ? launch_router_t<bf16_t>(a, p, s) : launch_router_t<float>(a, p, s);
 }
 
+static LayoutArgs layout_args(const DispatchArgs& a) {
+    return {a.blockcnt, a.partial, a.T, a.E, a.k, a.block_tokens, a.w_aux, a.w_z, a.tile_m, a.counts, a.offsets,
+            a.tile_expert, a.tile_row0, a.tile_rows, a.ntiles, a.losses};
+}
+
+bool dispatch_in_product_ok(const DispatchArgs& a) {
+    if (a.T <= 0 || a.xg != nullptr || a.E > 64 || (a.E & (a.E - 1)) != 0) return false;
+    const long long nb = (a.T + a.block_tokens - 1) / a.block_tokens;
+    return nb * a.E <= kSlotsMaxHistogram && nb <= kSlotsMaxBlocks && (a.block_tokens & (a.block_tokens - 1)) == 0 &&
+           (a.tile_m & (a.tile_m - 1)) == 0 && a.tile_m <= kSlotsTileM;
+}
+RoutedSlots routed_slots(const DispatchArgs& a) {
+    RoutedSlots r;
+    r.expert_of = a.expert_of;
+    r.rank_in_block = a.rank_in_block;
+    r.perm_slot = a.perm_slot;
+    r.perm_token = a.perm_token;
+    r.inv_pos = a.inv_pos;
+    r.k_recip = (uint32_t)(0x100000000ull / (uint32_t)a.k) + 1u;
+    for (int tb = a.block_tokens; tb > 1; tb >>= 1) ++r.tb_shift;
+    for (int m = a.tile_m; m > 1; m >>= 1) ++r.tile_shift;
+    r.layout = layout_args(a);
+    return r;
+}
+
 template <typename XT>
 static hipError_t launch_dispatch_t(const DispatchArgs& a, hipStream_t s) {
     const int nb = (a.T + a.block_tokens - 1) / a.block_tokens;
     if ((long long)nb * a.E <= kFusedScanLimit) {
         RB_LAUNCH(dispatch_fused_kernel<XT>, dim3(nb > 0 ? nb : 1), dim3(256),
                            dispatch_fused_lds_bytes(a.E, a.k, a.block_tokens), s, static_cast<const XT*>(a.x), a.expert_of,
-                           a.rank_in_block, a.blockcnt, a.partial, a.T, a.d, a.E, a.k, a.block_tokens, a.w_aux, a.w_z, a.tile_m,
-                           a.counts, a.offsets, a.tile_expert, a.tile_row0, a.tile_rows, a.ntiles, a.losses,
-                           a.perm_slot, a.perm_token, a.inv_pos, static_cast<XT*>(a.xg));
+                           a.rank_in_block, layout_args(a), a.d, a.perm_slot, a.perm_token, a.inv_pos, static_cast<XT*>(a.xg));
         return hipGetLastError();
     }
     float* const mass = reinterpret_cast<float*>(a.blockbase + (size_t)nb * a.E);  // [E + 1]

@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "layout_device.h"
 #include "rbmoe_kernels.h"
 
 namespace rbmoe {
@@ -116,6 +117,16 @@ __device__ __forceinline__ float weight_value(float v) { return v; }
 __device__ __forceinline__ float weight_value(bf16_t v) { return to_f32(v); }
 __device__ __forceinline__ float weight_value(int8_t v) { return (float)v; }
 
+// A second, dense group in the same launch (the shared expert); rows 0: none.
+template <typename WT>
+struct F32Dense {
+    const float* a;
+    const WT* w;
+    const float* scales;
+    int N, K, rows;
+    float *out, *gu_out;
+};
+
 // `sub`: this kernel's tiles in one of the tile table's, 1 or 2.  TB = blocks of 32 token rows per workgroup; FW = waves along the features (the workgroup owns 32 FW of them, or with
 // SWIGLU as many gate and up rows each), STEPS = steps of 16 reduction columns a wave takes of a slice.  DMA: rows of whole
 // 16-byte pieces on 16-byte boundaries and whole slices; otherwise both operands travel element by element.
@@ -124,7 +135,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     const float* __restrict__ a, const int* __restrict__ row_index, const WT* __restrict__ w, size_t w_expert_stride,
     const float* __restrict__ scales, size_t s_expert_stride, int N, int K, const int* __restrict__ tile_expert,
     const int* __restrict__ tile_row0, const int* __restrict__ tile_rows, const int* __restrict__ ntiles, int sub, int dense_rows,
-    float* __restrict__ out, float* __restrict__ gu_out, const float* __restrict__ bw_gu) {
+    float* __restrict__ out, float* __restrict__ gu_out, const float* __restrict__ bw_gu, F32Dense<WT> g2, RoutedSlots slots) {
     typedef Weights<WT> W;
     constexpr int NTH = NW * 64;
     constexpr int KG = NW / FW;                   // wave groups that share out a slice's steps
@@ -140,20 +151,47 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     constexpr int TPIECES = BM * SK / 4;          // 16-byte pieces of raw token rows of a slice
     constexpr int NT = (TPIECES + NTH - 1) / NTH; // ... a thread (threads left without one repeat another's)
     constexpr int LOOP_BYTES = RING * WSTAGE + 2 * PBUF, MEET_BYTES = KG > 1 ? NW * NB * TB * 16 * 64 * 4 : 0;
-    constexpr int LDS_BYTES = LOOP_BYTES > MEET_BYTES ? LOOP_BYTES : MEET_BYTES;
+    constexpr int USED_BYTES = LOOP_BYTES > MEET_BYTES ? LOOP_BYTES : MEET_BYTES;
+    constexpr int LDS_BYTES = !SWIGLU || USED_BYTES > (int)sizeof(SlotsLds) ? USED_BYTES : (int)sizeof(SlotsLds);
     __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];
+    __shared__ int own_token[SWIGLU ? 2 * kSlotsTileM : 1];  // (read once more behind the loop)
     unsigned char* const planes = lds + RING * WSTAGE;
 
     // ---- which tile: each XCD (workgroup number mod 8) walks a contiguous range of tiles with one expert's row tiles
     // innermost, so that a weight slice is fetched by one L2
-    const int tiles_n = (N + FN - 1) / FN;
-    const int tiles_m = dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles * sub;
-    const int total = tiles_m * tiles_n;
+    // (without tables: what the router left behind, see RoutedSlots; the second group's tiles come behind the routed ones)
+    const bool own = SWIGLU && slots.expert_of != nullptr;  // uniform over the launch
+    SlotsLds& sl = *reinterpret_cast<SlotsLds*>(lds);
+    RoutedCounts rc{};
+    if (own) {
+        if (blockIdx.x == gridDim.x - 1) return routed_rest(slots, lds);
+        rc = routed_counts<NTH>(slots, sl);
+    }
+    int tiles_n = (N + FN - 1) / FN;
+    int tiles_m = dense_rows >= 0 ? (dense_rows + BM - 1) / BM : (own ? rc.ntiles : *ntiles) * sub;
+    const int total1 = tiles_m * tiles_n;
+    const int tiles_n2 = (g2.N + FN - 1) / FN, tiles_m2 = (g2.rows + BM - 1) / BM;
+    const int total = total1 + tiles_m2 * tiles_n2;
     const int per_xcd = (total + 7) / 8;
     const int local = blockIdx.x >> 3;
     if (local >= per_xcd) return;
-    const int pid = (blockIdx.x & 7) * per_xcd + local;
+    int pid = (blockIdx.x & 7) * per_xcd + local;
     if (pid >= total) return;
+    const bool second = pid >= total1;
+    if (second) {  // (uniform over the workgroup)
+        pid -= total1;
+        tiles_n = tiles_n2;
+        tiles_m = tiles_m2;
+        a = g2.a;
+        row_index = nullptr;
+        w = g2.w;
+        scales = g2.scales;
+        N = g2.N;
+        K = g2.K;
+        dense_rows = g2.rows;
+        out = g2.out;
+        gu_out = g2.gu_out;
+    }
     constexpr int GROUP_M = 8;
     const int per_group = GROUP_M * tiles_n;
     const int first_m = pid / per_group * GROUP_M;
@@ -162,18 +200,27 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     const int tm_idx = first_m + in_g % gsize;
     const int n0 = in_g / gsize * FN;
 
-    int expert, row0, rows;
+    int expert, row0, rows, skip = 0;
     if (dense_rows >= 0) {
         expert = 0;
         row0 = tm_idx * BM;
         rows = min(BM, dense_rows - row0);
     } else {
-        const int entry = sub == 2 ? tm_idx >> 1 : tm_idx, skip = sub == 2 ? (tm_idx & 1) * BM : 0;
-        expert = tile_expert[entry];
-        row0 = tile_row0[entry] + skip;
-        rows = min(BM, tile_rows[entry] - skip);
+        const int entry = sub == 2 ? tm_idx >> 1 : tm_idx;
+        skip = sub == 2 ? (tm_idx & 1) * BM : 0;
+        if (own) {
+            const RoutedTile t = routed_tile<NTH>(slots, rc, entry, n0 == 0 && skip == 0, sl, own_token);
+            expert = t.expert;
+            row0 = t.row0 + skip;
+            rows = min(BM, t.rows - skip);
+        } else {
+            expert = tile_expert[entry];
+            row0 = tile_row0[entry] + skip;
+            rows = min(BM, tile_rows[entry] - skip);
+        }
         if (rows <= 0) return;
     }
+    const bool own_rows = own && !second;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -183,7 +230,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     // (rows past the end of the group, features past N: any valid one, products never stored)
     auto token_row = [&](int r) {
         const int rr = r < rows ? r : 0;
-        return a + (size_t)(row_index ? row_index[row0 + rr] : row0 + rr) * K;
+        return a + (size_t)(own_rows ? own_token[skip + rr] : row_index ? row_index[row0 + rr] : row0 + rr) * K;
     };
     auto weight_row = [&](int q) {  // q < FN: gate (or plain) feature n0 + q; q >= FN: the matching up row
         const int feat = n0 + (q % FN);
@@ -618,14 +665,16 @@ bool f32_shape_ok(int N, int K) { return K % 32 == 0 && K >= 32 && N % 4 == 0 &&
 //     2048 40.7 / 32.0 / 31.2 / 29.4
 // A last feature tile that is mostly empty costs more than half as wide tiles do: 64 experts of 704 (five and a half tiles
 // of 128), d 1024, 2048 tokens, six a row: 268 us in 64x128, 248 in 64x64.
-enum class F32Tile { T32x32, T32x64, T64x64, T64x128, T64x128x8 };
-static F32Tile f32_tile(const GroupedArgs& g, bool f32_weights, bool small_slices) {
+static long long f32_tiles(const GroupedArgs& g, int rows, int features) {
     const int S = g.dense_rows >= 0 ? g.dense_rows : g.routed_rows, E = g.dense_rows >= 0 ? 1 : g.groups;
     // tiles of a group's rows: a last one half full, or one tile for each group that gets any
     const int hit = std::min(E, S);
-    auto tiles = [&](int rows, int features) {
-        return (long long)std::max(S / rows + (hit + 1) / 2, hit) * ((g.N + features - 1) / features);
-    };
+    return (long long)std::max(S / rows + (hit + 1) / 2, hit) * ((g.N + features - 1) / features) +
+           (long long)((g.dense2.rows + rows - 1) / rows) * ((g.dense2.N + features - 1) / features);
+}
+enum class F32Tile { T32x32, T32x64, T64x64, T64x128, T64x128x8 };
+static F32Tile f32_tile(const GroupedArgs& g, bool f32_weights, bool small_slices) {
+    auto tiles = [&](int rows, int features) { return f32_tiles(g, rows, features); };
     if (tiles(32, 32) <= 256 && small_slices) return F32Tile::T32x32;
     if (tiles(32, 64) <= (f32_weights ? 256 : 600) || (g.dense_rows < 0 && g.tile_m == 32)) return F32Tile::T32x64;
     if (tiles(64, 64) <= 256) return F32Tile::T64x64;
@@ -633,29 +682,62 @@ static F32Tile f32_tile(const GroupedArgs& g, bool f32_weights, bool small_slice
     return (g.N + 127) / 128 * 128 * 20 > (g.N + 63) / 64 * 64 * 21 ? F32Tile::T64x64 : F32Tile::T64x128;
 }
 
+struct F32Plan {
+    F32Tile tile;
+    bool aligned;
+    int workgroups;  // about as many
+};
+static F32Plan f32_plan(const GroupedArgs& g, int weight_size) {
+    auto whole = [](const void* p, size_t pitch) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && pitch % 16 == 0; };
+    auto group = [&](const void* a, const void* w, int K) { return K % 32 == 0 && whole(a, (size_t)K * 4) && whole(w, (size_t)K * weight_size); };
+    const GroupedArgs::Dense& d2 = g.dense2;
+    const bool f32 = weight_size == 4;
+    F32Plan p;
+    p.aligned = group(g.a, g.w, g.K) && g.w_expert_stride * weight_size % 16 == 0 && (d2.rows == 0 || group(d2.a, d2.w, d2.K));
+    p.tile = f32_tile(g, f32, !p.aligned || (g.K % 64 == 0 && d2.K % 64 == 0));
+    if (f32 && !p.aligned && (p.tile == F32Tile::T64x128 || p.tile == F32Tile::T64x128x8)) p.tile = F32Tile::T64x64;
+    const int rows = p.tile == F32Tile::T32x32 || p.tile == F32Tile::T32x64 ? 32 : 64;
+    const int features = p.tile == F32Tile::T32x32 ? 32 : p.tile == F32Tile::T32x64 || p.tile == F32Tile::T64x64 ? 64 : 128;
+    p.workgroups = (int)std::min<long long>(f32_tiles(g, rows, features), 1 << 30);
+    return p;
+}
+
+int f32_workgroups(const GroupedArgs& g, WeightKind wk) {
+    return f32_plan(g, wk == WeightKind::F32 ? 4 : wk == WeightKind::BF16 ? 2 : 1).workgroups;
+}
+
+// Whole slices of both down products, or of neither: the routed experts' kernel stays the one they have by themselves.
+bool f32_joins(int F, int Fs) { return F == Fs || (F % 64 == 0 && Fs % 64 == 0); }
+
 template <typename WT>
 static hipError_t launch_f32_t(const GroupedArgs& g, hipStream_t s) {
     if (g.dense_rows < 0 && g.tile_m != 32 && g.tile_m != 64) return hipErrorInvalidValue;
+    if (g.slots.expert_of && (!g.swiglu || g.dense_rows >= 0 || g.slots.layout.tile_m != g.tile_m)) return hipErrorInvalidValue;
+    if (g.dense2.rows > 0 && (g.dense_rows >= 0 || !g.dense2.gu_out != !g.gu_out || g.swiglu_grad_gu)) return hipErrorInvalidValue;
     constexpr bool F32 = sizeof(WT) == 4;
-    auto whole = [](const void* p, size_t pitch) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && pitch % 16 == 0; };
-    const bool aligned = g.K % 32 == 0 && whole(g.a, (size_t)g.K * 4) && whole(g.w, (size_t)g.K * sizeof(WT)) &&
-                         g.w_expert_stride * sizeof(WT) % 16 == 0;
+    const F32Plan plan = f32_plan(g, sizeof(WT));
+    const bool aligned = plan.aligned;
+    const GroupedArgs::Dense& d2 = g.dense2;
+    const F32Dense<WT> g2{static_cast<const float*>(d2.a), static_cast<const WT*>(d2.w), d2.scales, d2.N, d2.K, d2.rows,
+                          static_cast<float*>(d2.out), static_cast<float*>(d2.gu_out)};
     auto go = [&](auto swiglu_tag, auto nw_tag, auto tb_tag, auto fw_tag, auto steps_tag) {
         constexpr bool SW = decltype(swiglu_tag)::value;
         constexpr int FW = decltype(fw_tag)::value, FN = 32 * FW, BM = 32 * decltype(tb_tag)::value;
         constexpr int NW = decltype(nw_tag)::value, STEPS = decltype(steps_tag)::value;
         const int tiles_m = g.dense_rows >= 0 ? (g.dense_rows + BM - 1) / BM : g.max_tiles * (g.tile_m / BM);
-        const int total = (g.N + FN - 1) / FN * tiles_m;
+        const int total = (g.N + FN - 1) / FN * tiles_m + (d2.N + FN - 1) / FN * ((d2.rows + BM - 1) / BM);
         if (total <= 0) return;
+        const int rest = SW && g.slots.expert_of ? 1 : 0;  // (routed_rest)
         const int sub = g.tile_m / BM;
         auto launch = [&](auto dma_tag) {
-            RB_LAUNCH((grouped_f32_kernel<WT, SW, NW, BM / 32, FW, STEPS, decltype(dma_tag)::value>), dim3((total + 7) / 8 * 8),
+            RB_LAUNCH((grouped_f32_kernel<WT, SW, NW, BM / 32, FW, STEPS, decltype(dma_tag)::value>), dim3((total + 7) / 8 * 8 + rest),
                       dim3(64 * NW), 0, s, static_cast<const float*>(g.a), g.row_index, static_cast<const WT*>(g.w), g.w_expert_stride,
                       g.scales, g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, sub, g.dense_rows,
-                      static_cast<float*>(g.out), static_cast<float*>(g.gu_out), static_cast<const float*>(g.swiglu_grad_gu));
+                      static_cast<float*>(g.out), static_cast<float*>(g.gu_out), static_cast<const float*>(g.swiglu_grad_gu), g2,
+                      g.slots);
         };
         constexpr int SK = 16 * STEPS * (NW / FW);
-        if (aligned && g.K % SK == 0) launch(std::true_type{});
+        if (aligned && g.K % SK == 0 && d2.K % SK == 0) launch(std::true_type{});
         else if constexpr (!(F32 && FW == 4)) launch(std::false_type{});  // (f32_tile does not ask for it)
     };
     typedef std::integral_constant<int, 1> One;
@@ -664,9 +746,7 @@ static hipError_t launch_f32_t(const GroupedArgs& g, hipStream_t s) {
     typedef std::integral_constant<int, 8> Eight;
     auto pick = [&](auto swiglu_tag) {
         typedef std::integral_constant<int, decltype(swiglu_tag)::value && F32 ? 1 : 2> Steps;
-        F32Tile tile = f32_tile(g, F32, !aligned || g.K % 64 == 0);
-        if (F32 && !aligned && (tile == F32Tile::T64x128 || tile == F32Tile::T64x128x8)) tile = F32Tile::T64x64;
-        switch (tile) {
+        switch (plan.tile) {
             case F32Tile::T32x32: return go(swiglu_tag, Four{}, One{}, One{}, One{});
             case F32Tile::T32x64: return go(swiglu_tag, Four{}, One{}, Two{}, One{});
             case F32Tile::T64x64: return go(swiglu_tag, Four{}, Two{}, Two{}, One{});

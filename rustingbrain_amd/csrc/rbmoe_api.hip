@@ -1374,7 +1374,16 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // 64 of 704, six a row, 1000 rows 126.5 / 139.0, 2048 (1136) 164.5 / 154.0.
     constexpr int kSharedInsideTiles = 768;
     const int gate_up_tiles = ((T * k) / tile_m0 + E) * ((F + 127) / 128) + (T + 127) / 128 * ((Fs + 127) / 128);
-    const bool shared_inside = c.shared_expert && mfma && !timed && T > 0 && (T < 1024 || gate_up_tiles <= kSharedInsideTiles);
+    // Over f32 rows (their kernels have tiles of 64 x 128 where a launch is large) the same below 1024 rows, and up to 400 such
+    // tiles: us a step, inside / one behind the other (from 1024 rows on beside), d 512, 8 of 352, bf16 weights, 4 rows 32.6 /
+    // 44.1, 512 39.2 / 49.7, 1024 (156 tiles) 45.8 / 61.2, 2048 (300) 63.1 / 72.0; f32 weights, 200 rows 35.2 / 50.3, 2048 84.1 / 83.0,
+    // 4096 (588) 132.7 / 127.5; d 1024, 4 of 910, 24 rows 46.5 / 70.0, 1024 (272) 114.0 / 114.1, 2048 (528) 188.7 / 177.2; d 768,
+    // 8 of 1408, 512 rows 111 / 123, 1024 (572) 179 / 158.
+    constexpr int kSharedInsideF32Tiles = 400;
+    const int f32_tiles = ((T * k) / 64 + (E + 1) / 2) * ((F + 127) / 128) + (T + 63) / 64 * ((Fs + 127) / 128);
+    const bool shared_inside = c.shared_expert && !timed && T > 0 &&
+                               (mfma ? T < 1024 || gate_up_tiles <= kSharedInsideTiles
+                                     : L->f32_rows && f32_joins(F, Fs) && (T < 1024 || f32_tiles <= kSharedInsideF32Tiles));
     auto with_shared = [&](GroupedArgs g, const GroupedArgs& sh) {
         g.dense2 = {sh.a, sh.w, sh.scales, sh.N, sh.K, sh.dense_rows, sh.out, sh.gu_out};
         return g;
@@ -1471,11 +1480,15 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // (156) 37.1 / 40.7, 6144 (444) 71.2 / 76.3, 8192 (588) 86.2 / 85.0; d 768, 8 of 1408, 64 rows 33.0 / 37.3, 2048 (396) 58.8 / 62.8,
     // 4096 (748) 87.6 / 83.9; 16 of 1408, 512 rows 41.8 / 45.1, 3072 (616) 79.1 / 80.8, 8192 (1496) 151.0 / 139.4.
     // (Not where a host call fetches the tables beside the products, nor where the stages are timed one by one.)
-    constexpr int kDispatchInsideTiles = 512;
+    // Over f32 rows, workgroups as f32_workgroups counts them: d 512, 8 experts of 352 and a shared one, bf16 weights, 64 rows
+    // 27.3 / 31.2, 1024 (600 workgroups) 42.6 / 45.8, 4096 (588) 91.0 / 93.0, 8192 (1164) 148.0 / 145.5; f32 weights, 8 of 1408, 1024
+    // (396) 90.2 / 95.5, 4096 (1452) 260.7 / 261.6; d 768, 16 of 682, four a row, 512 (288) 91.9 / 95.2, 2048 (816) 205.5 / 202.8.
+    constexpr int kDispatchInsideTiles = 512, kDispatchInsideF32 = 620;
     GroupedArgs first = shared_inside ? with_shared(g1, s1) : g1;
-    const int workgroups = g1.likely_tiles * ((F + 127) / 128) + (first.dense2.rows + 127) / 128 * ((first.dense2.N + 127) / 128);
-    const bool dispatch_inside = mfma && gather_in_product && !timed && !L->record_routed && workgroups <= kDispatchInsideTiles &&
-                                 dispatch_in_product_ok(da);
+    const int workgroups = mfma ? g1.likely_tiles * ((F + 127) / 128) + (first.dense2.rows + 127) / 128 * ((first.dense2.N + 127) / 128)
+                                : L->f32_rows ? f32_workgroups(first, wk) : 0;
+    const bool dispatch_inside = (mfma || L->f32_rows) && gather_in_product && !timed && !L->record_routed &&
+                                 workgroups <= (mfma ? kDispatchInsideTiles : kDispatchInsideF32) && dispatch_in_product_ok(da);
     if (dispatch_inside) first.slots = routed_slots(da);
     if (!dispatch_inside) HIP_TRY(ctx, launch_dispatch(da, abf || cast, s));
     if (L->record_routed) HIP_TRY(ctx, hipEventRecord(L->record_routed, s));

@@ -220,7 +220,7 @@ struct GroupedArgs {
     // gradients of the pre-activations go to `gu_out` [rows, 2N] and `out` is not written.
     const void* swiglu_grad_gu = nullptr;
     bool swiglu;
-    // bf16 matrix-core launches: a second, dense group in the same launch (the shared expert); rows 0: none.  Its weights
+    // matrix-core launches: a second, dense group in the same launch (the shared expert); rows 0: none.  Its weights
     // are of the same kind; pre-activations are kept (`gu_out`) for both groups or for neither.
     struct Dense {
         const void* a = nullptr;  // [rows, K]
@@ -232,7 +232,7 @@ struct GroupedArgs {
     } dense2;
     int group_m;            // MFMA path: M-tiles per scheduling group (0 = default)
     int tile_m = 0;         // rows per tile of the tile table
-    RoutedSlots slots;      // gate/up launches of the bf16 matrix-core kernels: in the place of tile table and row index
+    RoutedSlots slots;      // gate/up launches of the matrix-core kernels: in the place of tile table and row index
 };
 hipError_t launch_grouped_generic(const GroupedArgs& a, bool act_bf16, WeightKind wk, int tile_m,
                                   hipStream_t s);
@@ -250,6 +250,8 @@ void pack_weight_i8(const int8_t* src, int rows, int cols, int8_t* dst);
 // Products over f32 rows at f32 accuracy on the bf16 matrix cores: plain row-major weights of any kind, any shape.
 int f32_tile_m(int rows, int groups);  // rows of the tile table's tiles for so many routed rows: 32 or 64
 bool f32_shape_ok(int N, int K);
+int f32_workgroups(const GroupedArgs& a, WeightKind wk);  // about as many as the launch has
+bool f32_joins(int F, int Fs);  // whether a shared expert of width Fs may go into the launches of experts of width F
 hipError_t launch_grouped_f32(const GroupedArgs& a, WeightKind wk, hipStream_t s);
 
 // ---- backward pass: the kernels around the matrix products (backward_kernels.hip) --------

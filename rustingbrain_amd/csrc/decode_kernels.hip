@@ -1275,7 +1275,7 @@ __global__ __launch_bounds__(kSmallThreads, 2) void decode_front_kernel(RouteRow
     if ((int)blockIdx.x < routers) {
         const int k = r.k, ES = E | 1;
         const int t0 = blockIdx.x * kFrontTokens, nt = min(kFrontTokens, T - t0);
-        route_rows_body<XT, kFrontTokens, Q8 ? 32 : 8, Q8 ? 2 : 1, 2, NORM>(r, blockIdx.x, lds);
+        route_rows_body<XT, kFrontTokens, Q8 ? 32 : 8, Q8 ? 2 : 1, 2, NORM>(r, blockIdx.x, 0, r.E, lds);
         __syncthreads();
         float* const prob = reinterpret_cast<float*>(lds);  // the arrays of router_fixed_bytes
         float* const lsev = prob + kFrontTokens * ES;

@@ -1019,22 +1019,27 @@ bool decode_front_pays(const rbmoe_layer* L, int T, bool stages_rows, bool norme
 // Whether a few tokens' call is better off on the decode-shaped kernels than on the large-batch sequence, whose routing
 // takes a workgroup per eight tokens and whose launches a few microseconds each.  us, decode against large-batch:
 //   routing beside the products: its down launch sums slots one after the other.  Over 64 slots and 20 M weights a
-//     matrix: d 1024, 16 experts of 1408, four a row: 16 rows 38.7 / 47.5, 20 rows 52.0 / 47.5, 32 rows 63.0 / 47.8; 32
-//     experts of 704: 16 rows 42.3 / 51.3, 20 rows 57.2 / 52.6; 64 experts of 704, six a row, 32 rows 125.8 / 94.6.  Fewer
-//     weights, later: 32 rows, four a row, 16 experts, d 768 (17 M) 50.8 / 43.0, 8 experts, d 1024 (12 M) 44.4 / 41.2.
+//     matrix: d 1024, 16 experts of 1408, four a row, 17 rows 1.07 times as long as the large-batch launches, 32 rows 1.38;
+//     32 experts of 1408, d 512, 1.11 / 1.42.  Fewer weights, later: 32 rows, four a row, 16 experts, d 768 (17 M) 50.8 / 43.0,
+//     8 experts, d 1024 (12 M) 44.4 / 41.2.
+//     Its routing workgroup takes every expert's row, the large-batch routing shares them out (plan_rows): from 32 K router
+//     weights on and with 20 M weights a matrix, 32 experts of 704, d 1024, 4 to 32 rows 0.98 to 1.18, behind a norm 1.09 to
+//     1.24; 64 experts of 704, d 512, 1.00 to 1.19, behind a norm 1.15 to 1.33, d 1024 with a shared expert 1.36 to 1.65; 24 K
+//     (32 of 1408, d 768) 0.77 to 0.87, behind a norm 0.98 to 1.04.
 //   routing alone in one workgroup, in front: its time grows with tokens x experts x width, steeply where the rows do not
-//     fit its LDS.  Staged: 32 experts, d 512, 8 rows (131 K) 30.0 / 40.0, 16 rows (262 K) 47.2 / 40.9; 16 experts, d 768, 8
-//     rows (98 K) 39.2 / 44.2, 12 rows (147 K) 44.8 / 43.3.  Not staged: 32 experts, d 768, 4 rows (98 K) 41.5 / 41.5, 8 rows
-//     (197 K) 79.5 / 48.5; 64 experts, d 1024, 1 row (66 K) 56.4 / 64.3, 2 rows 73.2 / 66.4, 16 rows 303 / 83.5.
+//     fit its LDS.  d 1024, 16 experts of 1408: 1 row 0.68, 4 rows 0.83, 8 rows 0.97, behind a norm 0.84, 0.99, 1.08; 32 experts,
+//     d 512, 4 rows 0.87 / 0.99, 6 rows 1.06 / 1.12; staged: 16 experts, d 768, 12 rows (147 K) 44.8 us / 43.3.  Over 32 experts
+//     and 32 K router weights the routing that shares them out is ahead sooner: 64 experts, d 512, 1 row 0.89 / 0.99, 2 rows
+//     1.05 / 1.19, 4 rows - / 1.56; d 1024, 1 row 1.38 / 1.54, 8 rows 3.2.
 bool decode_front_beats_batch(const rbmoe_layer* L, int T) {
     const rbmoe_config& c = L->cfg;
-    const int slots = T * c.experts_per_token;
-    const double weights = (double)c.num_experts * L->Fw * c.d_model;
-    return !(slots > 64 && weights > 20e6) && !(slots > 112 && weights > 11e6);
+    const int slots = T * c.experts_per_token, E = c.num_experts;
+    const double weights = (double)E * L->Fw * c.d_model;
+    return !((slots > 64 || E * c.d_model >= 32 * 1024) && weights > 20e6) && !(slots > 112 && weights > 11e6);
 }
 bool decode_alone_beats_batch(const rbmoe_layer* L, int T, bool stages_rows) {
-    const long long work = (long long)T * L->cfg.num_experts * L->cfg.d_model;
-    return work <= (stages_rows ? 160000 : 110000);
+    const long long E = L->cfg.num_experts, work = T * E * L->cfg.d_model;
+    return work <= (E > 32 && E * L->cfg.d_model >= 32 * 1024 ? 40000 : stages_rows ? 160000 : 110000);
 }
 
 // The buffers of a decode-shaped forward of T tokens carved out of `base` (pieces of 256 bytes); returns the
@@ -1150,6 +1155,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
                   (int*)L->rank_in_block.p, (int*)L->blockcnt.p, (float*)L->partial.p};
     if (cast) ra.rows16 = L->x16.p;
     ra.allow_fused = L->fused_router;
+    ra.arrive = (int*)L->cmbcnt.p;
     if (L->tight) ra.min_tokens = kRouterTokens;
     if (L->router_q8) {
         ra.wq = (const int8_t*)L->router_q.p;

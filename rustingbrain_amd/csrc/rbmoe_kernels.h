@@ -89,6 +89,9 @@ struct RouterArgs {
     const float* norm_w = nullptr;
     float norm_eps = 0.0f;
     void* xn_out = nullptr;
+    // Arrival counters, all zero between launches (kDecodeCombineCounterStride apart, one a block of tokens), or null: where
+    // a few tokens have many experts, several workgroups then share a block's experts out.
+    int* arrive = nullptr;
 };
 // How a call is routed: tokens of a router block (what launch_dispatch needs to know), whether the launch applies the
 // norm that `a` asks for, and whether it writes the bf16 copy of f32 rows for a quantized router too.  Made once per call,
@@ -101,9 +104,10 @@ struct RouterPlan {
     // route_rows_kernel: experts whose router rows lie in LDS together (0: another kernel), LDS bytes
     int row_experts = 0;
     size_t row_lds = 0;
+    int row_slice = 0;  // ... and experts of a workgroup, where a block's experts are shared out (0: they are not)
     bool operator==(const RouterPlan& o) const {
         return block_tokens == o.block_tokens && takes_norm == o.takes_norm && q8_writes_rows16 == o.q8_writes_rows16 &&
-               row_experts == o.row_experts && row_lds == o.row_lds;
+               row_experts == o.row_experts && row_lds == o.row_lds && row_slice == o.row_slice;
     }
 };
 RouterPlan plan_router(const RouterArgs& a, bool bf16);

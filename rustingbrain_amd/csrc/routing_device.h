@@ -254,6 +254,8 @@ struct RouteRowsArgs {
     const float* norm_w;
     float norm_eps;
     void* xn_out;
+    int slice = 0;          // route_rows_kernel: experts of a workgroup (0: all of them)
+    int* arrive = nullptr;  // ... and, with a slice, a token block's arrival counter, kDecodeCombineCounterStride apart
 };
 // A staged row: column lane j's elements side by side, `lane_pitch` floats from one lane to the next - whole 16-byte
 // pieces (a last one short of four steps is filled up with zeros, which the sums do not see), and an odd number of
@@ -274,12 +276,13 @@ __host__ __device__ static size_t route_rows_lds_bytes(int E, int k, int d, int 
            ((size_t)TB * pitch + route_shared_floats(d, TB, EG, pitch, chain) + (chain ? d + TB : 0)) * 4;
 }
 
-// The logits of the TB tokens of block `blk` into the `prob` array (row pitch E | 1) of `lds_raw`, with everything in
+// The logits of the TB tokens of block `blk` for the experts [e_from, e_to) into the `prob` array (row pitch E | 1) of `lds_raw`, with everything in
 // front of them; the caller meets at a barrier before it reads them.  Kernels without the norm are compiled without its code:
 // with it they are 50 KB long instead of 25 and take 150 registers instead of 100, and 4096 tokens of d 768 by 8 experts are
 // routed in 10.4 us instead of 10.1.
 template <typename XT, int TB, int NL, int TT, int EE, bool NORM>
-__device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk, unsigned char* __restrict__ lds_raw) {
+__device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk, int e_from, int e_to,
+                                                unsigned char* __restrict__ lds_raw) {
     constexpr int NT = kRouterThreads;
     const int T = a.T, d = a.d, E = a.E, k = a.k, EG = a.EG;
     const int ES = E | 1;
@@ -356,7 +359,7 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
     const int short_from = d / NL, short_n = (short_from + 3) / 4 * 4 - short_from;
     if (short_n > 0)
         for (int i = tid; i < TB * NL * short_n; i += NT) xs[(i / short_n) * lp + short_from + i % short_n] = 0.0f;
-    const int nw0 = min(EG, E) * wpr, nx = nt * xpr;
+    const int nw0 = min(EG, e_to - e_from) * wpr, nx = nt * xpr;
     if (wave_norm) {
         // a wave a row: the raw elements in registers, normed, rounded to the layer's own type and laid down; each half of the
         // wave takes half of a lane's elements.  The router's rows are put into place meanwhile by whoever is free.
@@ -370,7 +373,7 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
             float4 nwv[H / 4];
 #pragma unroll
             for (int i = 0; i < H / 4; ++i) nwv[i] = *reinterpret_cast<const float4*>(a.norm_w + c0 + 4 * i);
-            const Six w = request(router_src(0), nw0, tid);
+            const Six w = request(router_src(e_from), nw0, tid);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
             for (int r = wave; r < nt; r += NT / 64) {
@@ -406,11 +409,11 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
                 }
             }
             deliver(w, nw0, tid, put_router);
-            rest_of_router(0, nw0, 6 * NT);
+            rest_of_router(e_from, nw0, 6 * NT);
         });
     } else {
         const uint4* const xsrc = reinterpret_cast<const uint4*>(static_cast<const XT*>(a.x) + (size_t)t0 * d);
-        const Six w = request(router_src(0), nw0, tid);
+        const Six w = request(router_src(e_from), nw0, tid);
         const Six x = request(xsrc, nx, tid);
         float nwv[2] = {0.0f, 0.0f};
         if (norm) {
@@ -429,7 +432,7 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
             __syncthreads();
         }
         deliver(w, nw0, tid, put_router);
-        rest_of_router(0, nw0, 6 * NT);
+        rest_of_router(e_from, nw0, 6 * NT);
         if (short_n > 0)
             for (int i = tid; i < EG * NL * short_n; i += NT) ws[(i / short_n) * lp + short_from + i % short_n] = 0.0f;
     }
@@ -478,9 +481,9 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
     // ---- logits -------------------------------------------------------------------
     const int j = tid % NL;  // the thread's column lane
     const int quads = (d / NL + 3) / 4;
-    for (int e0 = 0; e0 < E; e0 += EG) {
-        const int ne = min(EG, E - e0);
-        if (e0 > 0) {
+    for (int e0 = e_from; e0 < e_to; e0 += EG) {
+        const int ne = min(EG, e_to - e0);
+        if (e0 > e_from) {
             __syncthreads();  // the group before has been consumed
             rest_of_router(e0, ne * wpr, 0);
             __syncthreads();

@@ -576,12 +576,53 @@ __global__ __launch_bounds__(kRouterThreads) void route_fused_kernel(
     router_tail<1, true>(lds_raw, blk, valid, T, E, k, P, lse, expert_of, gate_of, rank_in_block, blockcnt, partial);
 }
 
+// A token block's experts shared out over workgroups: each leaves its logits in P; the last to arrive fetches the others' into
+// its own array and goes on.  Device-scope stores and loads: the workgroups may sit on different XCDs, whose L2s do not see
+// each other's lines; a workgroup's stores are acknowledged before its arrival is counted.
+template <int TB>
+__device__ __forceinline__ bool last_slice(const RouteRowsArgs& a, int from, int to, unsigned char* lds_raw) {
+    float* const prob = reinterpret_cast<float*>(lds_raw);
+    const int E = a.E, ES = E | 1, tid = threadIdx.x;
+    int& last = *reinterpret_cast<int*>(prob + TB * ES);  // (where router_tail will keep the log-sum-exps)
+    const int t0 = blockIdx.x * TB, nt = min(TB, a.T - t0), n = to - from;
+    for (int i = tid; i < nt * n; i += kRouterThreads) {
+        const int t = i / n, e = from + i - t * n;
+        __hip_atomic_store(a.P + (size_t)(t0 + t) * E + e, prob[t * ES + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+        int* const counter = a.arrive + blockIdx.x * kDecodeCombineCounterStride;
+        const int before = atomicAdd(counter, 1);
+        last = before == (int)gridDim.y - 1;
+        if (before == (int)gridDim.y - 1) atomicExch(counter, 0);  // everyone has arrived: ready for the next launch
+    }
+    __syncthreads();
+    if (!last) return false;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    for (int i = tid; i < nt * E; i += kRouterThreads) {
+        const int t = i / E, e = i - t * E;
+        if (e < from || e >= to)
+            prob[t * ES + e] = __hip_atomic_load(a.P + (size_t)t0 * E + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return true;  // (router_tail begins with a barrier)
+}
+
 // Norm (optional), logits and everything behind them for TB tokens a workgroup (see route_rows_body).
 template <typename XT, int TB, int NL, int TT, int EE, bool NORM>
 __global__ __launch_bounds__(kRouterThreads, 2) void route_rows_kernel(RouteRowsArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    route_rows_body<XT, TB, NL, TT, EE, NORM>(a, blockIdx.x, lds_raw);
-    __syncthreads();
+    if (a.slice == 0) {  // uniform over the launch
+        route_rows_body<XT, TB, NL, TT, EE, NORM>(a, blockIdx.x, 0, a.E, lds_raw);
+        __syncthreads();
+    } else {
+        const int from = blockIdx.y * a.slice, to = min(a.E, from + a.slice);
+        RouteRowsArgs own = a;
+        if (blockIdx.y != 0) own.xn_out = own.rows16 = nullptr;  // (the first slice writes the rows)
+        route_rows_body<XT, TB, NL, TT, EE, NORM>(own, blockIdx.x, from, to, lds_raw);
+        __syncthreads();
+        if (!last_slice<TB>(a, from, to, lds_raw)) return;
+    }
     router_tail<1, true, TB>(lds_raw, blockIdx.x, a.valid, a.T, a.E, a.k, a.P, a.lse, a.expert_of, a.gate_of, a.rank_in_block,
                              a.blockcnt, a.partial);
 }
@@ -1070,6 +1111,7 @@ struct RowsPlan {
     int tokens = 0;  // 0: not taken
     int EG = 0;
     size_t lds = 0;
+    int slice = 0;
 };
 // Where the other kernels are faster all the same (blocks of 8 tokens never lose).  Times are forwards of narrow experts,
 // other kernels / this one.
@@ -1112,6 +1154,19 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     const int together = p.tokens == kRouterTokens && 2 * p.lds <= (size_t)kMaxRouterLds ? 512 : 256;
     if ((long long)a.T * a.E > 256 * 1024 || blocks > together) p.tokens = 0;
     if (p.tokens > kMinRouterTokens && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
+    // A few tokens by many experts: one workgroup a block would take the experts' rows through its own LDS one group after the
+    // other (64 experts of d 1024: 27 us, whatever the tokens).  So the block's experts are shared out, eight to a workgroup
+    // or as many as leave at most one round of workgroups; the last to arrive does the rest.  us a forward, one workgroup / shared
+    // out: 64 experts, d 1024, 1 row 52.5 / 40.2, 256 rows 100.7 / 87.4, 512 rows 106.3 / 93.9; 32 experts, d 1024, f32, 24 rows
+    // 59.6 / 53.7; d 768 38.2 / 36.4; d 512, 128 rows 34.4 / 33.2, but d 256, 128 rows 27.1 / 27.2, 512 rows 29.1 / 29.5; 16 experts,
+    // d 768, 64 rows 38.4 / 39.2.
+    if (p.tokens == kMinRouterTokens && a.arrive && a.E >= 32 && a.E * a.d >= 16 * 1024)
+        for (int slice = 8; slice < a.E && !p.slice; slice *= 2)
+            if (blocks * ((a.E + slice - 1) / slice) <= 256) {
+                p.slice = slice;
+                p.EG = std::min(p.EG, slice);
+                p.lds = route_rows_lds_bytes(a.E, a.k, a.d, p.tokens, NL, p.EG, a.norm_w != nullptr);
+            }
     return p;
 }
 
@@ -1121,6 +1176,7 @@ RouterPlan plan_router(const RouterArgs& a, bool bf16) {
     q.block_tokens = p.tokens ? p.tokens : kRouterTokens;
     q.row_experts = p.tokens ? p.EG : 0;
     q.row_lds = p.tokens ? p.lds : 0;
+    q.row_slice = p.tokens ? p.slice : 0;
     // where the squares' room costs tokens a workgroup, a second round of workgroups costs more than the norm in a launch of
     // its own (8192 tokens, d 768, squares in LDS: 37.7 us in two rounds, 16.2 + 8 in two launches; a wave a row leaves one
     // round: 29 in one launch, 12.5 + 20 in two)
@@ -1146,8 +1202,9 @@ bool router_takes(const RouterArgs& a, const RouterPlan& p, bool bf16) {
 template <typename XT>
 static hipError_t launch_rows_t(const RouterArgs& a, const RouterPlan& p, hipStream_t s) {
     RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, p.row_experts, a.P, a.lse, a.expert_of, a.gate_of,
-                    a.rank_in_block, a.blockcnt, a.partial, static_cast<bf16_t*>(a.rows16), a.norm_w, a.norm_eps, a.xn_out};
-    const dim3 grid((a.T + p.block_tokens - 1) / p.block_tokens);
+                    a.rank_in_block, a.blockcnt, a.partial, static_cast<bf16_t*>(a.rows16), a.norm_w, a.norm_eps, a.xn_out,
+                    p.row_slice, a.arrive};
+    const dim3 grid((a.T + p.block_tokens - 1) / p.block_tokens, p.row_slice ? (a.E + p.row_slice - 1) / p.row_slice : 1);
     auto go = [&](auto kernel) -> hipError_t {
         static std::atomic<unsigned long long> attr_set{0};  // one per kernel: the lambda's body is instantiated for each
         const hipError_t e = once_per_device(attr_set, [&] {

@@ -255,7 +255,7 @@ struct rbmoe_layer {
 
     // weights
     Buf router;            // f32 [E, d]
-    Buf router_q, router_s; // a quantized router: int8 [E, d], f32 scales [E]
+    Buf router_q, router_s; // a quantized router: int8 [E, d], f32 scales [E] (`router` then holds the int8 values as f32)
     bool router_q8 = false; // the layer routes with the quantized product (src/quantized.rs:55-62)
     bool quantize_router = false;  // f32 router data is quantized at upload (TransformerLm::quantize reaches the router too)
     int quant_rule = 0;     // f32 -> int8 at upload: 0 the checkpoint writer's rule, 1 the in-memory rule
@@ -836,6 +836,10 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
         if (router_to_i8) {
             HIP_TRY(ctx, hipMemcpy(L->router_q.p, src, n_given, hipMemcpyHostToDevice));
             HIP_TRY(ctx, hipMemcpy(L->router_s.p, scales, (size_t)rows * 4, hipMemcpyHostToDevice));
+            // ... and widened, for the products of large calls (logits_kernel)
+            const int8_t* const q = static_cast<const int8_t*>(src);
+            const std::vector<float> wide(q, q + n_given);
+            HIP_TRY(ctx, hipMemcpy(L->router.p, wide.data(), n_given * 4, hipMemcpyHostToDevice));
         } else {
             HIP_TRY(ctx, hipMemcpy(L->router.p, src, n_given * 4, hipMemcpyHostToDevice));
         }

@@ -76,13 +76,22 @@ struct XPiece<float> {
 // WIDE (bf16 rows): the rows are widened to f32 once, on their way into LDS, instead of by each of the NE waves
 // that read them (one of the three vector instructions per element); a slice is then half as many columns, so
 // that a workgroup takes no more LDS and as many of them fit a compute unit.
-template <typename XT, int NE, bool AHEAD, bool WIDE = false>
+// NL = 32: the logits of a quantized router, in the order of dot_lanes::<32> (src/quantized.rs:154-177): lanes[c % 32] +=
+// x[c] * f32(q[c]), the scalar rest from the last multiple of 32 on, and the whole times the row's `scale` (:61).  `wr` then
+// holds the int8 weights widened once, at their upload: a whole number in f32 is fetched like any other router weight.
+// For bf16 rows; bound by the vector units like the other order.  us a forward with a thread a product over the int8 rows
+// (logits_q8_kernel: 64 lines of them a load) / with this: 64 experts of 704, d 1024, 16384 tokens 734.6 / 639.7, 4096
+// 209.0 / 202.3; 16 experts of 256, d 1024, 16384 tokens 171.9 / 140.4; 32 of 256, 5000 tokens 107.1 / 85.5; 8 of 256, d 768,
+// 12000 tokens 107.1 / 95.1; 128 of 64, d 512, one token 55.7 / 51.6, 64 tokens 61.1 / 58.0.
+template <typename XT, int NE, bool AHEAD, bool WIDE = false, int NL = 8>
 __global__ __launch_bounds__(NE * 64, (!AHEAD && sizeof(XT) == 2) ? 6 : 2) void logits_kernel(const XT* __restrict__ x,
                                                                 const float* __restrict__ wr,
                                                                 const float* __restrict__ bias, int T, int d, int E,
                                                                 float* __restrict__ logits,
-                                                                bf16_t* __restrict__ rows16) {
+                                                                bf16_t* __restrict__ rows16,
+                                                                const float* __restrict__ scale) {
     static_assert(!WIDE || sizeof(XT) == 2, "only bf16 rows are widened");
+    static_assert(NL == 8 || (NL == 32 && sizeof(XT) == 2), "32 lanes: bf16 rows");
     typedef typename XPiece<XT>::raw_t piece_t;
     typedef typename std::conditional<WIDE, float, XT>::type ST;  // the element type of the staged rows
     typedef typename XPiece<ST>::raw_t spiece_t;
@@ -114,11 +123,14 @@ __global__ __launch_bounds__(NE * 64, (!AHEAD && sizeof(XT) == 2) ? 6 : 2) void 
     const int e = blockIdx.y * NE + wave;  // this wave's expert
     const bool has = e < E;
     const float* w0 = wr + (size_t)(has ? e : 0) * d;
-    const int tail = d - d % 8;
-    float la[8];
+    const int tail = d - d % NL;
+    float la[NL];
 #pragma unroll
-    for (int l = 0; l < 8; ++l) la[l] = 0.0f;
-    const bool vec = d % 8 == 0;
+    for (int l = 0; l < NL; ++l) la[l] = 0.0f;
+    const bool vec = d % 8 == 0 && (NL == 8 || (reinterpret_cast<uintptr_t>(x) & 15) == 0);
+    constexpr int TURN = NL / 8;                                // pieces of one turn of the column lanes
+    constexpr int BATCH = NL == 8 ? kLogitBatch : TURN;         // (32 sums leave registers for half a batch)
+    static_assert(PIECES % BATCH == 0 && BATCH % TURN == 0, "a slice is whole turns");
     // A slice's pieces travel global -> registers -> LDS.  AHEAD: the loads of the next slice are issued
     // before the products of the current one, so their latency is covered by arithmetic - for launches of few
     // workgroups; with several workgroups on a compute unit they cover for each other, and the registers the
@@ -184,28 +196,33 @@ __global__ __launch_bounds__(NE * 64, (!AHEAD && sizeof(XT) == 2) ? 6 : 2) void 
         if (has) {
             const float* wa = w0 + c0;
             int q = 0;
-            for (; q + kLogitBatch <= np; q += kLogitBatch) {
-                // one batch: 32 router weights into scalar registers, 4 token pieces from LDS
-                float wv[8 * kLogitBatch];
+            for (; q + BATCH <= np; q += BATCH) {
+                // one batch: its router weights into scalar registers, its token pieces from LDS
+                float wv[8 * BATCH];
 #pragma unroll
-                for (int j = 0; j < 8 * kLogitBatch; ++j) wv[j] = wa[8 * q + j];
-                spiece_t xp[kLogitBatch];
+                for (int j = 0; j < 8 * BATCH; ++j) wv[j] = wa[8 * q + j];
+                spiece_t xp[BATCH];
 #pragma unroll
-                for (int b = 0; b < kLogitBatch; ++b) xp[b] = *staged(lane, q + b);
+                for (int b = 0; b < BATCH; ++b) xp[b] = *staged(lane, q + b);
 #pragma unroll
-                for (int b = 0; b < kLogitBatch; ++b) {
+                for (int b = 0; b < BATCH; ++b) {
                     float xv[8];
                     XPiece<ST>::widen(xp[b], xv);
 #pragma unroll
-                    for (int l = 0; l < 8; ++l) la[l] = __fadd_rn(la[l], __fmul_rn(xv[l], wv[8 * b + l]));
+                    for (int l = 0; l < 8; ++l) {
+                        float& sum = la[8 * (b % TURN) + l];
+                        sum = __fadd_rn(sum, __fmul_rn(xv[l], wv[8 * b + l]));
+                    }
                 }
             }
-            for (; q < np; ++q) {
-                float xv[8];
-                XPiece<ST>::widen(*staged(lane, q), xv);
+            if constexpr (BATCH > TURN)
+                for (; q < np; ++q) {
+                    static_assert(TURN == 1, "one piece a turn");
+                    float xv[8];
+                    XPiece<ST>::widen(*staged(lane, q), xv);
 #pragma unroll
-                for (int l = 0; l < 8; ++l) la[l] = __fadd_rn(la[l], __fmul_rn(xv[l], wa[8 * q + l]));
-            }
+                    for (int l = 0; l < 8; ++l) la[l] = __fadd_rn(la[l], __fmul_rn(xv[l], wa[8 * q + l]));
+                }
         }
     }
     if (lane < nt && has) {
@@ -214,8 +231,9 @@ __global__ __launch_bounds__(NE * 64, (!AHEAD && sizeof(XT) == 2) ? 6 : 2) void 
         for (int c = tail; c < d; ++c) rest = __fadd_rn(rest, __fmul_rn(to_f32(xr[c]), w0[c]));
         float sum = 0.0f;
 #pragma unroll
-        for (int l = 0; l < 8; ++l) sum = __fadd_rn(sum, la[l]);
+        for (int l = 0; l < NL; ++l) sum = __fadd_rn(sum, la[l]);
         float v = __fadd_rn(sum, rest);
+        if constexpr (NL == 32) v = __fmul_rn(v, scale[e]);
         if (bias) v = __fadd_rn(v, bias[e]);
         logits[(size_t)(t0 + lane) * E + e] = v;
     }
@@ -359,8 +377,10 @@ __device__ __forceinline__ void router_tail(
 // logits_q8_kernel: the logits of a quantized router, one thread per (token, expert).  The reference's order
 // (dot_lanes::<32>, src/quantized.rs:154-177, taken on machines with AVX2, :179-196): lanes[c % 32] += x[c] * f32(q[c])
 // over the whole chunks of 32 columns, a scalar rest over the tail, the lanes folded from 0.0 in lane order, plus the
-// rest, times the row's scale (:61); every product and every sum rounded by itself.  Any width; not tuned (a
-// quantized layer's router is a few hundred kilobytes and this kernel a few percent of its forward).
+// rest, times the row's scale (:61); every product and every sum rounded by itself.  Any width.  For f32 rows: there
+// logits_kernel's own order of lanes is no faster in large launches (us a forward, this / logits_kernel<NL = 32>: 12000
+// tokens, d 768, 8 experts 115.6 / 120.8; 5000, d 1024, 32 experts 113.5 / 135.5; 3000, d 512, 64 experts 69.6 / 79.9; 8192,
+// d 768, 16 experts 169.9 / 163.0); bf16 rows are routed there.
 // ---------------------------------------------------------------------------
 template <typename XT>
 __global__ __launch_bounds__(256) void logits_q8_kernel(const XT* __restrict__ x, const int8_t* __restrict__ q,
@@ -1116,7 +1136,8 @@ struct RowsPlan {
 // Where the other kernels are faster all the same (blocks of 8 tokens never lose).  Times are forwards of narrow experts,
 // other kernels / this one.
 //   quantized: a dot product is d / 32 steps on 32 threads and the folding of their 32 sums; the shorter the rows and the
-//     more products a workgroup has, the more of it is folding, which logits_q8_kernel (one thread a product) does not have.
+//     more products a workgroup has, the more of it is folding, which the kernels with a lane a product
+//     (logits_q8_kernel; logits_kernel for bf16 rows) do not have; the line was drawn against the former.
 //     16 tokens: d 256, 16 experts 1.03 times as long, 8 experts 0.93; d 384, 32 experts 1.09 / 24 experts 1.00; d 512, 64
 //     experts 1.12, 48 experts 1.07 to 0.95; d 768, 64 experts 0.92.  32 tokens: d 256, 8 experts 1.05, 4 experts 0.96; d 384,
 //     16 experts 1.14 to 1.03; d 512, 24 experts 1.10 to 1.00, 16 experts 1.06 to 0.97; d 768, 32 experts 1.08 to 0.95.
@@ -1275,17 +1296,25 @@ static hipError_t launch_router_t(const RouterArgs& a, const RouterPlan& p, hipS
     constexpr int NE = 8;
     const int tiles_t = (a.T + kLogitTokens - 1) / kLogitTokens;
     const dim3 lgrid(tiles_t, (a.E + NE - 1) / NE);
-    if (a.wq) {
-        if (a.rows16 || !a.wscale) return hipErrorInvalidValue;  // (the caller casts f32 rows itself on this path)
+    if (a.wq && (a.rows16 || !a.wscale)) return hipErrorInvalidValue;  // (the caller casts f32 rows itself on this path)
+    auto logits = [&](auto lanes) {
+        constexpr int NL = decltype(lanes)::value;
+        if ((long long)lgrid.x * lgrid.y <= 512)  // at most two workgroups on a compute unit
+            RB_LAUNCH((logits_kernel<XT, NE, true, false, NL>), lgrid, dim3(NE * 64), 0, s, static_cast<const XT*>(a.x),
+                      a.wr, a.bias, a.T, a.d, a.E, a.P, static_cast<bf16_t*>(a.rows16), a.wscale);
+        else
+            RB_LAUNCH((logits_kernel<XT, NE, false, sizeof(XT) == 2, NL>), lgrid, dim3(NE * 64), 0, s,
+                      static_cast<const XT*>(a.x), a.wr, a.bias, a.T, a.d, a.E, a.P, static_cast<bf16_t*>(a.rows16), a.wscale);
+    };
+    if (!a.wq) {
+        logits(std::integral_constant<int, 8>{});
+    } else if constexpr (sizeof(XT) == 2) {
+        logits(std::integral_constant<int, 32>{});
+    } else {
         const long long pairs = (long long)a.T * a.E;
         RB_LAUNCH(logits_q8_kernel<XT>, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, s,
                   static_cast<const XT*>(a.x), a.wq, a.wscale, a.bias, a.T, a.d, a.E, a.P);
-    } else if ((long long)lgrid.x * lgrid.y <= 512)  // at most two workgroups on a compute unit
-        RB_LAUNCH((logits_kernel<XT, NE, true>), lgrid, dim3(NE * 64), 0, s, static_cast<const XT*>(a.x),
-                           a.wr, a.bias, a.T, a.d, a.E, a.P, static_cast<bf16_t*>(a.rows16));
-    else
-        RB_LAUNCH((logits_kernel<XT, NE, false, sizeof(XT) == 2>), lgrid, dim3(NE * 64), 0, s, static_cast<const XT*>(a.x),
-                           a.wr, a.bias, a.T, a.d, a.E, a.P, static_cast<bf16_t*>(a.rows16));
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (a.E <= 64)

@@ -75,7 +75,8 @@ struct XPiece<float> {
 // have every piece of their rows in hand anyway (widths that are multiples of 8).
 // WIDE (bf16 rows): the rows are widened to f32 once, on their way into LDS, instead of by each of the NE waves
 // that read them (one of the three vector instructions per element); a slice is then half as many columns, so
-// that a workgroup takes no more LDS and as many of them fit a compute unit.
+// that a workgroup takes no more LDS and as many of them fit a compute unit.  So it is for f32 rows in launches of many
+// workgroups: four on a compute unit instead of two (64 experts of 704, d 1024, 16384 f32 rows 823.7 -> 803 us a forward).
 // NL = 32: the logits of a quantized router, in the order of dot_lanes::<32> (src/quantized.rs:154-177): lanes[c % 32] +=
 // x[c] * f32(q[c]), the scalar rest from the last multiple of 32 on, and the whole times the row's `scale` (:61).  `wr` then
 // holds the int8 weights widened once, at their upload: a whole number in f32 is fetched like any other router weight.
@@ -95,7 +96,7 @@ __global__ __launch_bounds__(NE * 64, (!AHEAD && sizeof(XT) == 2) ? 6 : 2) void 
     typedef typename XPiece<XT>::raw_t piece_t;
     typedef typename std::conditional<WIDE, float, XT>::type ST;  // the element type of the staged rows
     typedef typename XPiece<ST>::raw_t spiece_t;
-    constexpr int kChunk = WIDE ? kLogitChunk / 2 : kLogitChunk;
+    constexpr int kChunk = !AHEAD && sizeof(ST) == 4 ? kLogitChunk / 2 : kLogitChunk;
     constexpr int PIECES = kChunk / 8;  // pieces per row per slice
     constexpr int ROWB = PIECES * (int)sizeof(spiece_t) + 16;  // bytes of a staged row: 16 of padding, so that the lanes' rows start in different banks
     __shared__ __align__(16) unsigned char xs_raw[kLogitTokens * ROWB];

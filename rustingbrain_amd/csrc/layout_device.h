@@ -197,7 +197,8 @@ struct RoutedTile {
     int expert, row0, rows, first;  // first: the tile's first row among its expert's
 };
 // The histograms and the tile table's length; the rest (lane = expert: its slots, the slots and tiles up to and with it) is for
-// routed_tile.  Called by all NTH threads of the workgroup.
+// routed_tile.  Called by all NTH threads of the workgroup; when it returns every wave has the sums, so that a workgroup that
+// does not go on to routed_tile (a dense tile) may use the LDS for something else.
 struct RoutedCounts {
     int count, rows, tiles, ntiles;
 };
@@ -227,6 +228,7 @@ __device__ __forceinline__ RoutedCounts routed_counts(const RoutedSlots& r, Slot
     c.count = 0;
 #pragma unroll
     for (int w = 0; w < NTH / 64; ++w) c.count += lds.wave_sum[w][lane];
+    __syncthreads();
     c.count = lane < E ? c.count : 0;
     c.rows = sum_up_to_lane(c.count);
     c.tiles = sum_up_to_lane((c.count + l.tile_m - 1) >> r.tile_shift);

@@ -78,8 +78,8 @@ def split_kernels(asm: str) -> Dict[str, List[str]]:
     return kernels
 
 
-def check_kernel(lines: List[str], max_states: int = 200000) -> List[str]:
-    """Returns a list of hazard descriptions (empty = clean)."""
+def parse(lines: List[str]) -> Tuple[List[Inst], Dict[str, int]]:
+    """The instructions of a kernel, and which of them its labels stand in front of."""
     insts: List[Inst] = []
     label_at: Dict[str, int] = {}
     for n, raw in enumerate(lines):
@@ -91,6 +91,12 @@ def check_kernel(lines: List[str], max_states: int = 200000) -> List[str]:
         if not t or t.startswith((";", ".")) or not raw.startswith("\t"):
             continue
         insts.append(Inst(n, t))
+    return insts, label_at
+
+
+def check_kernel(lines: List[str], max_states: int = 200000) -> List[str]:
+    """Returns a list of hazard descriptions (empty = clean)."""
+    insts, label_at = parse(lines)
     hazards: Dict[Tuple[int, int], str] = {}
     # state: tuple of destination sets (frozenset, line) of outstanding vector-memory ops, oldest first
     start: Tuple = ()
@@ -133,6 +139,36 @@ def check_kernel(lines: List[str], max_states: int = 200000) -> List[str]:
                 work.append((label_at[ins.target], state))
             pc += 1
     return [hazards[k] for k in sorted(hazards)]
+
+
+def barriers_before_dma(lines: List[str]) -> Optional[int]:
+    """The fewest barriers on any path from a wave's first write to the LDS to the first load it issues straight into it
+    (`global_load_lds_*`); None where no path has both."""
+    insts, label_at = parse(lines)
+    fewest: Optional[int] = None
+    seen = set()
+    work: List[Tuple[int, bool, int]] = [(0, False, 0)]
+    while work:
+        pc, used, barriers = work.pop()
+        while pc < len(insts) and (pc, used, barriers) not in seen:
+            seen.add((pc, used, barriers))
+            ins = insts[pc]
+            if ins.mnemonic.startswith("global_load_lds"):
+                if used:
+                    fewest = barriers if fewest is None else min(fewest, barriers)
+                break
+            used = used or ins.mnemonic.startswith(("ds_write", "ds_store"))
+            if ins.mnemonic == "s_barrier":
+                barriers = min(barriers + 1, 8)
+            if ins.kind == "end":
+                break
+            if ins.kind == "jump":
+                pc = label_at[ins.target]
+                continue
+            if ins.kind == "cond":
+                work.append((label_at[ins.target], used, barriers))
+            pc += 1
+    return fewest
 
 
 def check_asm(asm: str, name_filter: Optional[str] = None) -> Dict[str, List[str]]:

@@ -1,6 +1,7 @@
 """The streaming kernel waits for its inline-assembly loads by hand; this compiles it to
 assembly with the library's own flags and checks, over every path of every instantiation,
 that no instruction touches a register whose load can still be outstanding."""
+import functools
 import os
 import shutil
 import subprocess
@@ -12,7 +13,18 @@ import isa_check
 from rustingbrain_amd import build as rb_build
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SRC = os.path.join(HERE, "..", "rustingbrain_amd", "csrc", "grouped_stream.hip")
+CSRC = os.path.join(HERE, "..", "rustingbrain_amd", "csrc")
+needs_hipcc = pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
+
+
+@functools.lru_cache(maxsize=None)
+def assembly(source: str) -> str:
+    with tempfile.TemporaryDirectory() as tmp:
+        out = os.path.join(tmp, "kernels.s")
+        cmd = [rb_build.HIPCC] + [f for f in rb_build.FLAGS if f != "-fPIC"] + ["-S", "--cuda-device-only", "-o", out,
+                                                                              os.path.join(CSRC, source)]
+        subprocess.run(cmd, check=True, capture_output=True)
+        return open(out).read()
 
 
 def test_checker_flags_a_use_before_the_wait():
@@ -30,30 +42,34 @@ def test_checker_follows_loops():
     assert any("v_mov_b32_e32 v2, v9" in h for h in res)
 
 
-@pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
+@needs_hipcc
 def test_streaming_kernel_has_no_use_of_outstanding_loads():
-    with tempfile.TemporaryDirectory() as tmp:
-        out = os.path.join(tmp, "grouped_stream.s")
-        cmd = [rb_build.HIPCC] + [f for f in rb_build.FLAGS if f != "-fPIC"] + ["-S", "--cuda-device-only", "-o", out, SRC]
-        subprocess.run(cmd, check=True, capture_output=True)
-        res = isa_check.check_asm(open(out).read(), "grouped_stream_kernel")
+    res = isa_check.check_asm(assembly("grouped_stream.hip"), "grouped_stream_kernel")
     assert len(res) >= 4, "expected every instantiation of the kernel in the assembly"
     bad = {k: v[:5] for k, v in res.items() if v}
     assert not bad, bad
 
 
-@pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
+@needs_hipcc
+@pytest.mark.parametrize("source,kernel", [("grouped_stream.hip", "grouped_stream_kernel"), ("grouped_f32.hip", "grouped_f32_kernel")])
+def test_a_dense_tile_starts_when_every_wave_has_the_routed_counts(source, kernel):
+    """A gate/up launch that works out its own tiles sums the router's histograms through the LDS that its main loop fills by
+    LDS-DMA.  One barrier stands in front of the sums; a workgroup whose tile is a dense one fills the LDS right after, and
+    a fast wave of it would overwrite the sums of a slow one without a second."""
+    kernels = {n: k for n, k in isa_check.split_kernels(assembly(source)).items() if kernel in n}
+    found = {n: isa_check.barriers_before_dma(k) for n, k in kernels.items()}
+    found = {n: v for n, v in found.items() if v is not None}
+    assert len(found) >= 4, "expected the gate/up instantiations among the kernels"
+    assert all(v >= 2 for v in found.values()), found
+
+
+@needs_hipcc
 def test_static_scratch_array_is_a_symbol_the_runtime_can_look_up():
     # rbmoe_forward_static's scratch is a static device array whose address the host asks the runtime for by name
     # (hipGetSymbolAddress).  The runtime searches the code object's global symbols, and a missing one ends the
     # process rather than returning an error - so the array must come out of the device compilation as a global
     # object of the declared size, not as a local one.
-    src = os.path.join(HERE, "..", "rustingbrain_amd", "csrc", "rbmoe_api.hip")
-    with tempfile.TemporaryDirectory() as tmp:
-        out = os.path.join(tmp, "rbmoe_api.s")
-        cmd = [rb_build.HIPCC] + [f for f in rb_build.FLAGS if f != "-fPIC"] + ["-S", "--cuda-device-only", "-o", out, src]
-        subprocess.run(cmd, check=True, capture_output=True)
-        lines = [ln.strip() for ln in open(out) if "rbmoe_static_scratch" in ln]
+    lines = [ln.strip() for ln in assembly("rbmoe_api.hip").splitlines() if "rbmoe_static_scratch" in ln]
     name = next(ln.split()[1].split(",")[0] for ln in lines if ln.startswith(".type"))
     assert f".globl {name}" in [" ".join(ln.split()) for ln in lines], lines
     assert not any(ln.startswith(".local") for ln in lines), lines

@@ -117,6 +117,26 @@ __device__ __forceinline__ float weight_value(float v) { return v; }
 __device__ __forceinline__ float weight_value(bf16_t v) { return to_f32(v); }
 __device__ __forceinline__ float weight_value(int8_t v) { return (float)v; }
 
+// Columns c .. c + 3 of a row of K, in f32.  WHOLE: rows of whole 16-byte pieces on 16-byte boundaries; otherwise columns past
+// the end count as zero.
+template <bool WHOLE, typename T>
+__device__ __forceinline__ void load4_f32(const T* row, int c, int K, float (&v)[4]) {
+    struct __attribute__((aligned(4 * sizeof(T)))) Four {
+        T v[4];
+    };
+    if constexpr (WHOLE) {
+        const Four f = *reinterpret_cast<const Four*>(row + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = weight_value(f.v[i]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float w = weight_value(row[min(c + i, K - 1)]);
+            v[i] = c + i < K ? w : 0.0f;
+        }
+    }
+}
+
 // A second, dense group in the same launch (the shared expert); rows 0: none.
 template <typename WT>
 struct F32Dense {
@@ -155,6 +175,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     constexpr int LDS_BYTES = !SWIGLU || USED_BYTES > (int)sizeof(SlotsLds) ? USED_BYTES : (int)sizeof(SlotsLds);
     __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];
     __shared__ int own_token[SWIGLU ? 2 * kSlotsTileM : 1];  // (read once more behind the loop)
+    __shared__ int row_nan[BM];                              // rows that hold a NaN
     unsigned char* const planes = lds + RING * WSTAGE;
 
     // ---- which tile: each XCD (workgroup number mod 8) walks a contiguous range of tiles with one expert's row tiles
@@ -244,6 +265,9 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     const float* tsrc[NT];
     int tcol[NT];
     unsigned char* tdst[NT];
+    bool nan[NT];  // ... of the row of piece i
+    auto piece_row = [&](int i) { return (i * NTH + tid) % TPIECES / (SK / 4); };
+    if (tid < BM) row_nan[tid] = 0;
     constexpr int NWE = DMA ? 1 : WR * SK / NTH;
     WT pend_w[NWE];
     u32x4 pend_t[2][NT];  // raw row values of two slices under way
@@ -256,7 +280,8 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     }
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
-        const int p = (i * NTH + tid) % TPIECES, r = p / (SK / 4), c = p % (SK / 4);
+        const int r = piece_row(i), c = (i * NTH + tid) % (SK / 4);
+        nan[i] = false;
         tsrc[i] = token_row(r);
         tcol[i] = 4 * c;
         tdst[i] = planes + r * (SK * 2) + 16 * ((c >> 1) ^ row_swizzle<TPP>(r)) + 8 * (c & 1);
@@ -298,8 +323,10 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     };
     // the rows' planes: [buffer][plane][row][SK / 8 pieces of 8 bf16]
     uint32_t cv[3][2];
-    auto split_t = [&](int half, const u32x4& v) {
-        split2(__uint_as_float(half ? v.z : v.x), __uint_as_float(half ? v.w : v.y), cv[0][half], cv[1][half], cv[2][half]);
+    auto split_t = [&](int i, int half, const u32x4& v) {
+        const float x = __uint_as_float(half ? v.z : v.x), y = __uint_as_float(half ? v.w : v.y);
+        nan[i] = nan[i] || __builtin_isunordered(x, y);
+        split2(x, y, cv[0][half], cv[1][half], cv[2][half]);
     };
     auto put_t = [&](int i, int buf) {
 #pragma unroll
@@ -372,7 +399,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
             } else if constexpr (i < RW + RT + F + C) {
                 constexpr int j = i - RW - RT - F, u = j / 3;
                 if constexpr (j % 3 < 2) {
-                    split_t(j % 3, set[u]);
+                    split_t(u, j % 3, set[u]);
                 } else {
                     put_t(u, ck & 1);
                     load_t(u, ck + 2, set[u]);
@@ -440,8 +467,8 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     }
     auto convert_now = [&](int buf) {
         f32_for<0, NT>([&](auto i) {
-            split_t(0, first[buf][i]);
-            split_t(1, first[buf][i]);
+            split_t(i, 0, first[buf][i]);
+            split_t(i, 1, first[buf][i]);
             put_t(i, buf);
         });
     };
@@ -486,6 +513,9 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     }
     if (kt < KT) slice(kt, Even{}, oa, ob);
     wait(All{});  // the LDS is used again below, and nothing may land after the workgroup has ended
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+        if (nan[i]) row_nan[piece_row(i)] = 1;
     __syncthreads();
 
     // ---- wave groups that share out the reduction meet in LDS: group g finishes quads (four values) g OQ .. + OQ - 1 of the
@@ -595,48 +625,79 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     };
     auto token_of = [&](int q) { return (grp * OQ + q) / 4 * 32 + lr; };
     auto feature_of = [&](int q) { return n0 + fw * 32 + 8 * ((grp * OQ + q) % 4) + 4 * lh; };
+    // An infinity (or a value within a rounding of the largest) splits into parts that cancel or meet a zero part of the other
+    // operand: the sum is then not a number where the product of the values themselves may well be one.  Sums that are not
+    // numbers, those of rows with a NaN in them aside, are therefore taken again from the values, by the f32 matrix unit, the
+    // whole wave block at once and straight from memory.  Only they take the new sums: what a row comes out as does not depend
+    // on its neighbours.  us a forward, 1024 rows, d 512, 8 experts of 1408 in f32, plain rows 93: a row of NaN among them 94, all
+    // NaN 86, all infinite 156; one lane after the other 1231, 2935 and 2934, and 126, 115 and 115 with every product on the f32
+    // unit.  8 experts of 352 and a shared one, bf16 weights, plain 41: 41, 40 and 103.
+    uint32_t odd = 0;
+#pragma unroll
+    for (int q = 0; q < OQ; ++q) {
+        if (token_of(q) >= rows || feature_of(q) >= N || row_nan[token_of(q)]) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (__builtin_isunordered(mine[0][q][i], mine[NB - 1][q][i])) odd |= 1u << q;
+    }
+    if (__ballot(odd != 0) != 0ull) {
+        constexpr int OT = OQ >= 4 ? OQ / 4 : 1;  // blocks of 32 rows that this wave finishes
+        const float* tr[OT];
+        const WT* wr[NB];
+        floatx16 sum[NB][OT];
+#pragma unroll
+        for (int t = 0; t < OT; ++t) tr[t] = token_row((grp * OQ / 4 + t) * 32 + lr);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            wr[nb] = weight_row(nb * FN + fw * 32 + lr);
+#pragma unroll
+            for (int t = 0; t < OT; ++t)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sum[nb][t][v] = 0.0f;
+        }
+        // multiply j of a step takes column 4 (l / 32) + j of lane l in both operands
+#pragma unroll 1
+        for (int c0 = 0; c0 < K; c0 += 32) {
+            float tv[4][OT][4], wv4[4][NB][4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int c = c0 + 8 * u + 4 * lh;
+#pragma unroll
+                for (int t = 0; t < OT; ++t) load4_f32<DMA>(tr[t], c, K, tv[u][t]);
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) load4_f32<DMA>(wr[nb], c, K, wv4[u][nb]);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                        for (int t = 0; t < OT; ++t)
+                            sum[nb][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv4[u][nb][j], tv[u][t][j], sum[nb][t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < OQ; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {  // (which quad of its block q is, is known at compile time where the wave has whole blocks)
+                if (!((odd >> q) & 1) || v != (grp * OQ + q) % 4) continue;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) mine[nb][q][i] = sum[nb][OQ >= 4 ? q / 4 : 0][4 * v + i];
+            }
+    }
     auto store_tile = [&](auto whole_tag) {
-        uint32_t odd = 0;  // quads with a sum that is not a number
 #pragma unroll
         for (int q = 0; q < OQ; ++q) {
             const int tok = token_of(q), f = feature_of(q);
             if (tok >= rows || f >= N) continue;
             float g[4], u[4];
-            bool nan = false;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 g[i] = mine[0][q][i];
                 u[i] = mine[NB - 1][q][i];
-                nan = nan || g[i] != g[i] || u[i] != u[i];
-            }
-            if (nan) odd |= 1u << q;
-            else finish(whole_tag, (size_t)(row0 + tok), f, g, u);
-        }
-        // An infinity (or a value within a rounding of the largest) splits into parts that cancel or meet a zero part of the
-        // other operand: the sum is then not a number where the product of the values themselves may well be one.  Such
-        // sums, and those that are not numbers anyway, are taken again from the values, one after the other.
-        if (odd == 0) return;
-#pragma unroll 1
-        for (int q = 0; q < OQ; ++q) {
-            if (!((odd >> q) & 1)) continue;
-            const int tok = token_of(q), f = feature_of(q);
-            const float* const ar = token_row(tok);
-            float g[4] = {0.0f, 0.0f, 0.0f, 0.0f}, u[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            const WT *wg[4], *wu[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int fi = min(f + i, N - 1);
-                wg[i] = wbase + (size_t)fi * K;
-                wu[i] = wbase + (size_t)(SWIGLU ? N + fi : fi) * K;
-            }
-#pragma unroll 1
-            for (int c = 0; c < K; ++c) {
-                const float av = ar[c];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    g[i] = fmaf(av, weight_value(wg[i][c]), g[i]);
-                    if constexpr (SWIGLU) u[i] = fmaf(av, weight_value(wu[i][c]), u[i]);
-                }
             }
             finish(whole_tag, (size_t)(row0 + tok), f, g, u);
         }

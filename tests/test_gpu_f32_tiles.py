@@ -1,8 +1,11 @@
 """Products over f32 rows at the sizes where a tile, a slice of the reduction or the way of the operands into LDS changes,
 and values that three bf16 parts do not hold."""
+import time
+
 import numpy as np
 import pytest
 
+from bench import DeviceBuffer
 from conftest import rel_l2
 from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
 from rustingbrain_amd import synth
@@ -71,4 +74,37 @@ def test_values_that_do_not_split(device, wt, F, T):
     ok = np.isfinite(want) & (np.abs(want) < 1e30)
     assert np.isinf(want).any() and np.isnan(want).any() and ok.any()
     assert rel_l2(h[ok], want[ok]) <= 1e-5
+    layer.close()
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("wt,F", [("f32", 704), ("bf16", 352), ("int8", 352)])
+def test_sums_taken_again_cost_little_and_leave_the_neighbours_alone(device, wt, F, value):
+    """Sums that are not numbers are taken again on the f32 matrix unit.  A sixteenth of the bf16 unit's rate by three or six
+    products is at most five times the products' time; one lane at a time it was thirty times that of the whole call."""
+    T = 1024
+    t = synth.make(small_workload(d=512, E=8, k=2, F=F, T=T, seed=74, act="f32", wt=wt))
+    layer = gpu_layer(device, t)
+    x = np.ascontiguousarray(t.x)
+    some = x.copy()
+    some[::7, 100] = value
+    outs, times = [], []
+    for rows in (x, some, np.full_like(x, value)):
+        xb, ob = DeviceBuffer(device, x.nbytes).upload(rows), DeviceBuffer(device, x.nbytes)
+        best = 1e9
+        for _ in range(6):
+            device.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(10):
+                layer.forward_device(xb.ptr, T, ob.ptr)
+            device.synchronize()
+            best = min(best, time.perf_counter() - t0)
+        outs.append(ob.download(np.empty_like(x)).copy())
+        times.append(best)
+        xb.free()
+        ob.free()
+    same = np.arange(T) % 7 != 0
+    np.testing.assert_array_equal(outs[0][same].view(np.uint32), outs[1][same].view(np.uint32))
+    assert not np.isfinite(outs[1][~same]).all(axis=1).any()
+    assert max(times[1:]) <= 5 * times[0], times
     layer.close()

@@ -626,8 +626,9 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     auto token_of = [&](int q) { return (grp * OQ + q) / 4 * 32 + lr; };
     auto feature_of = [&](int q) { return n0 + fw * 32 + 8 * ((grp * OQ + q) % 4) + 4 * lh; };
     // An infinity (or a value within a rounding of the largest) splits into parts that cancel or meet a zero part of the other
-    // operand: the sum is then not a number where the product of the values themselves may well be one.  Sums that are not
-    // numbers, those of rows with a NaN in them aside, are therefore taken again from the values, by the f32 matrix unit, the
+    // operand: the sum is then not a number where the product of the values themselves may well be one.  And a product of two
+    // first parts may be larger than that of the values by 2^-7, and past the largest f32 where that is not.  Sums that are not
+    // finite, those of rows with a NaN in them aside, are therefore taken again from the values, by the f32 matrix unit, the
     // whole wave block at once and straight from memory.  Only they take the new sums: what a row comes out as does not depend
     // on its neighbours.  us a forward, 1024 rows, d 512, 8 experts of 1408 in f32, plain rows 93: a row of NaN among them 94, all
     // NaN 86, all infinite 156; one lane after the other 1231, 2935 and 2934, and 126, 115 and 115 with every product on the f32
@@ -638,7 +639,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
         if (token_of(q) >= rows || feature_of(q) >= N || row_nan[token_of(q)]) continue;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (__builtin_isunordered(mine[0][q][i], mine[NB - 1][q][i])) odd |= 1u << q;
+            if (!__builtin_isfinite(mine[0][q][i]) || !__builtin_isfinite(mine[NB - 1][q][i])) odd |= 1u << q;
     }
     if (__ballot(odd != 0) != 0ull) {
         constexpr int OT = OQ >= 4 ? OQ / 4 : 1;  // blocks of 32 rows that this wave finishes

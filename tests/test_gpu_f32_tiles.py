@@ -77,6 +77,41 @@ def test_values_that_do_not_split(device, wt, F, T):
     layer.close()
 
 
+@pytest.mark.parametrize("T", [1, 40, 300])
+@pytest.mark.parametrize("wt,F", [("f32", 64), ("f32", 45), ("bf16", 96), ("int8", 45)])
+def test_products_next_to_the_largest_value(device, wt, F, T):
+    """x w is within f32, the product of the nearest bf16 values of both is not: the hidden rows are finite, as the oracle's."""
+    v, w = (1.99 * 2.0 ** 126, 2 * 1.004) if wt == "f32" else (2.0 ** 127 * (1 - 2.0 ** -10), 2.0)
+    v, w = np.float32(v), np.float32(w)
+    assert np.isfinite(v * w)
+    with np.errstate(over="ignore"):
+        assert np.isinf(np.float32(synth.round_bf16(np.array([v]))[0] * synth.round_bf16(np.array([w]))[0]))
+    t = synth.make(small_workload(d=64, E=3, k=1, F=F, T=T, seed=75, act="f32", wt=wt))
+    t.router[:, 0] = 0
+    for e in t.experts:
+        gate, up = (e["gate_q"], e["up_q"]) if wt == "int8" else (e["gate"], e["up"])
+        gate[::3], up[::3] = 0, 0
+        gate[::3, 0], up[::3, 1] = w, 1
+        gate[1::3, 0] = 0   # (what else they multiply stays as it is)
+        gate[2::3, 0] = 0
+        up[1::3, 0] = 0
+        up[2::3, 0] = 0
+        if wt == "int8":
+            e["gate_s"][:], e["up_s"][:] = 1, 1
+    t.x[:, 0], t.x[:, 1] = v, np.float32(2.0 ** -3)
+    ref = oracle_layer(t).forward(t.x, threads=4)
+    layer = gpu_layer(device, t)
+    layer.forward_train(t.x)
+    h, _ = layer.expert_rows(T)
+    want = np.asarray(ref.hidden[:T])
+    assert np.isfinite(want).all() and (np.abs(want[:, ::3]) > 4e37).all()
+    assert np.isfinite(h).all()
+    np.testing.assert_allclose(h[:, ::3], want[:, ::3], rtol=2.0 ** -22)   # one product, one halving
+    rest = np.arange(F) % 3 != 0
+    assert rel_l2(h[:, rest], want[:, rest]) <= 1e-5
+    layer.close()
+
+
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 @pytest.mark.parametrize("wt,F", [("f32", 704), ("bf16", 352), ("int8", 352)])
 def test_sums_taken_again_cost_little_and_leave_the_neighbours_alone(device, wt, F, value):

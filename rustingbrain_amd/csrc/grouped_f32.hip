@@ -3,8 +3,8 @@
 //   out[row, n] = sum_c a[row, c] * w[expert][n, c]                 (down product)
 //   out[row, n] = silu(a . wgate[n]) * (a . wup[n])                 (gate/up product)
 //
-// An f32 value is the exact sum of three bf16 values, x = x1 + x2 + x3, each the nearest to what the ones before leave
-// (24 bits of mantissa in three times eight, signs included).  Products of bf16 values are exact in f32, so
+// An f32 value of 2^-110 or more is the exact sum of three bf16 values, x = x1 + x2 + x3, each the nearest to what the ones
+// before leave (24 bits of mantissa in three times eight, signs included).  Products of bf16 values are exact in f32, so
 //   f32 weights    x w = x1 w1 + x1 w2 + x2 w1 + x1 w3 + x2 w2 + x3 w1 + (less than 2^-25 of |x w|): six multiplies on a
 //                  unit of sixteen times the rate of the f32 one
 //   bf16 weights   x w = x1 w + x2 w + x3 w, exactly: three
@@ -14,6 +14,10 @@
 // steps): hidden rows against 64 bits, d 512, 8 experts of 1408, 1024 tokens, 1.9e-7 where v_mfma_f32_32x32x2 gave 4.3e-7,
 // products over given rows 2.4e-7 / 4.8e-7; bf16 weights, width 352, 3.6e-7 where a chain of fused adds gave 6.2e-7.
 // Rows and weights stay f32 in memory.
+// bf16's smallest value is 2^-133: of a smaller f32 value than 2^-110 up to 2^-134 is lost, of the largest ones the first part
+// rounds to infinity, and a product of first parts may be past the largest f32 where that of the values is not.  Sums that
+// this could show in are taken again on the f32 unit (see `odd`): what is lost stays below 2^-44 of the row's largest value
+// a product.  f32 weights below 2^-110 lose as much wherever their sum is 2^-90 or more, or zero.
 //
 // What bounds it.  A step of a 64 x 64 wave tile is 24 multiplies (768 cycles of the matrix core) and the splitting of two
 // weight fragments (88 vector instructions, 352 cycles).  The rows are split once per workgroup, on their way from registers
@@ -68,6 +72,12 @@ __device__ __forceinline__ void split2(float x, float y, uint32_t& a, uint32_t& 
     b = pack2(x1, y1);
     c = pack2(x1 - __uint_as_float(b << 16), y1 - __uint_as_float(b & 0xffff0000u));
 }
+
+// Magnitudes in the order of their values, a NaN above all of them.
+__device__ __forceinline__ uint32_t magnitude(float v) { return __float_as_uint(v) << 1; }
+constexpr uint32_t kInfinite = 0xff000000u;
+// 2^-90: below it the parts of a split value may be missing (see the top of the file)
+constexpr uint32_t kSplitsFrom = (uint32_t)(127 - 90) << 24;
 
 // Rows of 16 * PP bytes lie in LDS one behind the other; position p of row r holds piece p ^ row_swizzle<PP>(r), so that 16
 // lanes that read one logical piece of 16 rows touch distinct banks (256 bytes of them).
@@ -175,7 +185,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     constexpr int LDS_BYTES = !SWIGLU || USED_BYTES > (int)sizeof(SlotsLds) ? USED_BYTES : (int)sizeof(SlotsLds);
     __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];
     __shared__ int own_token[SWIGLU ? 2 * kSlotsTileM : 1];  // (read once more behind the loop)
-    __shared__ int row_nan[BM];                              // rows that hold a NaN
+    __shared__ uint32_t row_top[BM];                         // the rows' largest magnitudes
     unsigned char* const planes = lds + RING * WSTAGE;
 
     // ---- which tile: each XCD (workgroup number mod 8) walks a contiguous range of tiles with one expert's row tiles
@@ -265,9 +275,9 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     const float* tsrc[NT];
     int tcol[NT];
     unsigned char* tdst[NT];
-    bool nan[NT];  // ... of the row of piece i
+    float top[NT];  // the largest value so far of the row of piece i, signs aside (NaN: there is one)
     auto piece_row = [&](int i) { return (i * NTH + tid) % TPIECES / (SK / 4); };
-    if (tid < BM) row_nan[tid] = 0;
+    if (tid < BM) row_top[tid] = 0;
     constexpr int NWE = DMA ? 1 : WR * SK / NTH;
     WT pend_w[NWE];
     u32x4 pend_t[2][NT];  // raw row values of two slices under way
@@ -281,7 +291,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const int r = piece_row(i), c = (i * NTH + tid) % (SK / 4);
-        nan[i] = false;
+        top[i] = 0.0f;
         tsrc[i] = token_row(r);
         tcol[i] = 4 * c;
         tdst[i] = planes + r * (SK * 2) + 16 * ((c >> 1) ^ row_swizzle<TPP>(r)) + 8 * (c & 1);
@@ -325,7 +335,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     uint32_t cv[3][2];
     auto split_t = [&](int i, int half, const u32x4& v) {
         const float x = __uint_as_float(half ? v.z : v.x), y = __uint_as_float(half ? v.w : v.y);
-        nan[i] = nan[i] || __builtin_isunordered(x, y);
+        top[i] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(top[i], __builtin_fabsf(x)), __builtin_fabsf(y));
         split2(x, y, cv[0][half], cv[1][half], cv[2][half]);
     };
     auto put_t = [&](int i, int buf) {
@@ -514,8 +524,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     if (kt < KT) slice(kt, Even{}, oa, ob);
     wait(All{});  // the LDS is used again below, and nothing may land after the workgroup has ended
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
-        if (nan[i]) row_nan[piece_row(i)] = 1;
+    for (int i = 0; i < NT; ++i) atomicMax(&row_top[piece_row(i)], magnitude(top[i]));
     __syncthreads();
 
     // ---- wave groups that share out the reduction meet in LDS: group g finishes quads (four values) g OQ .. + OQ - 1 of the
@@ -627,19 +636,44 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     auto feature_of = [&](int q) { return n0 + fw * 32 + 8 * ((grp * OQ + q) % 4) + 4 * lh; };
     // An infinity (or a value within a rounding of the largest) splits into parts that cancel or meet a zero part of the other
     // operand: the sum is then not a number where the product of the values themselves may well be one.  And a product of two
-    // first parts may be larger than that of the values by 2^-7, and past the largest f32 where that is not.  Sums that are not
-    // finite, those of rows with a NaN in them aside, are therefore taken again from the values, by the f32 matrix unit, the
-    // whole wave block at once and straight from memory.  Only they take the new sums: what a row comes out as does not depend
-    // on its neighbours.  us a forward, 1024 rows, d 512, 8 experts of 1408 in f32, plain rows 93: a row of NaN among them 94, all
-    // NaN 86, all infinite 156; one lane after the other 1231, 2935 and 2934, and 126, 115 and 115 with every product on the f32
-    // unit.  8 experts of 352 and a shared one, bf16 weights, plain 41: 41, 40 and 103.
-    uint32_t odd = 0;
+    // first parts may be larger than that of the values by 2^-7, and past the largest f32 where that is not.  At the other end
+    // parts are missing (see the top of the file).  Taken again from the values, by the f32 matrix unit, the whole wave block
+    // at once and straight from memory, are therefore sums that are not finite, those of rows with a NaN in them aside; sums
+    // below 2^-90 that are not zero; and all sums of a row whose largest value is below 2^-90 and not zero.  Only they take
+    // the new sums: what a row comes out as does not depend on its neighbours.  us a forward, 1024 rows, d 512, 8 experts of
+    // 1408 in f32, plain rows 93 (92.5 without a look at small values): a row of NaN among them 94, all NaN 86, all infinite
+    // 156; one lane after the other 1231, 2935 and 2934, and 126, 115 and 115 with every product on the f32 unit.  8 experts of
+    // 352 and a shared one, bf16 weights, plain 41: 41, 40 and 103.
+    // (the whole lane at once first: hardly ever is there more to find out)
+    float most = 0.0f, least = HUGE_VALF;
+    bool tiny = false;
 #pragma unroll
     for (int q = 0; q < OQ; ++q) {
-        if (token_of(q) >= rows || feature_of(q) >= N || row_nan[token_of(q)]) continue;
+        tiny = tiny || row_top[token_of(q)] - 1 < kSplitsFrom - 1;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (!__builtin_isfinite(mine[0][q][i]) || !__builtin_isfinite(mine[NB - 1][q][i])) odd |= 1u << q;
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                most = __builtin_elementwise_maximum(most, __builtin_fabsf(mine[nb][q][i]));
+                least = __builtin_elementwise_minimum(least, __builtin_fabsf(mine[nb][q][i]));
+            }
+    }
+    uint32_t odd = 0;  // quads to take again
+    if (__ballot(tiny || !(most < HUGE_VALF && least >= 0x1p-90f)) != 0ull) {
+#pragma unroll
+        for (int q = 0; q < OQ; ++q) {
+            const uint32_t largest = row_top[token_of(q)];
+            if (token_of(q) >= rows || feature_of(q) >= N || largest > kInfinite) continue;
+            bool again = largest - 1 < kSplitsFrom - 1;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t m = magnitude(mine[nb][q][i]);
+                    again = again || m >= kInfinite || m - 1 < kSplitsFrom - 1;
+                }
+            if (again) odd |= 1u << q;
+        }
     }
     if (__ballot(odd != 0) != 0ull) {
         constexpr int OT = OQ >= 4 ? OQ / 4 : 1;  // blocks of 32 rows that this wave finishes

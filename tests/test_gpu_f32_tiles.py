@@ -112,6 +112,64 @@ def test_products_next_to_the_largest_value(device, wt, F, T):
     layer.close()
 
 
+# A product is off by 2^-24 of itself; each of a row's K terms next to the smallest value is rounded to a multiple of 2^-149.
+# Rows of 2^-122 in three bf16 parts, the last of which would be below 2^-133, are off by 1e-4.
+SCALES = [80, 89, 91, 100, 108, 112, 118, 122]
+
+
+def assert_rows_close(got, want, K):
+    got, want = got.astype(np.float64), want.astype(np.float64)
+    err, size = np.sqrt(((got - want) ** 2).mean(axis=1)), np.sqrt((want ** 2).mean(axis=1))
+    assert (size > 0).all()
+    np.testing.assert_array_less(err, 1e-5 * size + K * 2.0 ** -150)
+
+
+@pytest.mark.parametrize("T", [8, 40, 300])
+@pytest.mark.parametrize("wt,F", [("f32", 64), ("f32", 45), ("bf16", 96), ("int8", 45)])
+def test_rows_of_tiny_values(device, wt, F, T):
+    """Tiny sums over rows that hold a large value too, and rows of nothing but tiny values: each row by itself."""
+    t = synth.make(small_workload(d=64, E=3, k=1, F=F, T=T, seed=76, act="f32", wt=wt))
+    dense = []
+    for e in t.experts:
+        if wt == "int8":
+            e["up_q"][:, 0] = 0
+            m = [e[n + "_q"].astype(np.float64) * e[n + "_s"].astype(np.float64)[:, None] for n in ("gate", "up", "down")]
+        else:
+            e["up"][:, 0] = 0
+            m = [e[n].astype(np.float64) for n in ("gate", "up", "down")]
+        dense.append(m)
+    t.x[:, 1:] *= np.ldexp(np.float32(1), -np.resize(SCALES, T))[:, None].astype(np.float32)
+    t.x[:, 0] = 1
+    layer = gpu_layer(device, t)
+    _, cache = layer.forward_train(t.x)
+    h, y = layer.expert_rows(T)
+    tok = np.asarray(cache.perm_token[:T])
+    x = t.x[tok].astype(np.float64)
+    expert = np.asarray(cache.expert_of).reshape(-1)[tok]
+    for e, (gate, up, down) in enumerate(dense):
+        of = expert == e
+        if not of.any():
+            continue
+        g = x[of] @ gate.T
+        assert_rows_close(h[of], g / (1 + np.exp(-g)) * (x[of] @ up.T), 64)
+        assert_rows_close(y[of], h[of].astype(np.float64) @ down.T, F)
+    layer.close()
+
+
+@pytest.mark.parametrize("wt,F,T", [("f32", 64, 40), ("f32", 96, 300), ("bf16", 45, 70)])
+def test_gradients_of_tiny_rows(device, wt, F, T):
+    """Gradients are proportional to what comes in: rows of 2^-80 to 2^-122 as rows of one."""
+    t = synth.make(small_workload(d=64, E=4, k=2, F=F, T=T, seed=77, act="f32", wt=wt))
+    layer = gpu_layer(device, t, training=True, aux_w=0, z_w=0)
+    gout = np.random.default_rng(5).standard_normal(t.x.shape).astype(np.float32)
+    scale = np.ldexp(np.float32(1), -np.resize(SCALES, T))[:, None].astype(np.float32)
+    layer.forward_train(t.x)
+    whole = layer.backward(gout).astype(np.float64)
+    tiny = layer.backward(gout * scale)
+    assert_rows_close(tiny, whole * scale, 64 + 2 * F)
+    layer.close()
+
+
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 @pytest.mark.parametrize("wt,F", [("f32", 704), ("bf16", 352), ("int8", 352)])
 def test_sums_taken_again_cost_little_and_leave_the_neighbours_alone(device, wt, F, value):

@@ -277,7 +277,6 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     unsigned char* tdst[NT];
     float top[NT];  // the largest value so far of the row of piece i, signs aside (NaN: there is one)
     auto piece_row = [&](int i) { return (i * NTH + tid) % TPIECES / (SK / 4); };
-    if (tid < BM) row_top[tid] = 0;
     constexpr int NWE = DMA ? 1 : WR * SK / NTH;
     WT pend_w[NWE];
     u32x4 pend_t[2][NT];  // raw row values of two slices under way
@@ -460,6 +459,7 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     f32_for<0, NT>([&](auto i) { load_t(i, ONE ? 3 : 1, pend_t[1][i]); });
     first_w(1);
     first_w(2);
+    if (tid < BM) row_top[tid] = 0;  // (every wave passes a barrier before it is read)
     auto wait = [&](auto n_tag) {
 #pragma unroll
         for (int i = 0; i < NT; ++i) asm volatile("" : "+v"(pend_t[0][i]), "+v"(pend_t[1][i]));

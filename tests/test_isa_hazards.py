@@ -1,8 +1,9 @@
-"""The streaming kernel waits for its inline-assembly loads by hand; this compiles it to
+"""The product kernels wait for their inline-assembly loads by hand; this compiles them to
 assembly with the library's own flags and checks, over every path of every instantiation,
 that no instruction touches a register whose load can still be outstanding."""
 import functools
 import os
+import re
 import shutil
 import subprocess
 import tempfile
@@ -48,6 +49,35 @@ def test_streaming_kernel_has_no_use_of_outstanding_loads():
     assert len(res) >= 4, "expected every instantiation of the kernel in the assembly"
     bad = {k: v[:5] for k, v in res.items() if v}
     assert not bad, bad
+
+
+def f32_kernels():
+    """The instantiations over f32 rows with loads of their own: the last template argument says that rows and weights travel by
+    them (the others leave every load and its wait to the compiler)."""
+    return {n: k for n, k in isa_check.split_kernels(assembly("grouped_f32.hip")).items()
+            if n.startswith("_ZN") and "grouped_f32_kernel" in n and "Lb1EEEv" in n}
+
+
+@needs_hipcc
+def test_f32_kernels_have_no_use_of_outstanding_loads():
+    kernels = f32_kernels()
+    assert len(kernels) == 26, "three weight types, gate/up and plain, four tiles (f32 weights: five)"
+    bad = {n: h[:5] for n, h in ((n, isa_check.check_kernel(k)) for n, k in kernels.items()) if h}
+    assert not bad, bad
+
+
+@needs_hipcc
+def test_a_wait_that_lets_two_more_loads_be_outstanding_is_found():
+    """The check sees the f32 kernels' row loads: of the waits that leave some outstanding (the prologue's and the loop's), at
+    least two of each kernel are flagged when they let two more be (the others stand for loads straight into the LDS only)."""
+    for name, lines in f32_kernels().items():
+        found = 0
+        for i, line in enumerate(lines):
+            m = re.search(r"vmcnt\(([1-9]\d*)\) lgkmcnt\(0\)", line)
+            if m:
+                looser = line.replace(m.group(0), f"vmcnt({int(m.group(1)) + 2}) lgkmcnt(0)")
+                found += bool(isa_check.check_kernel(lines[:i] + [looser] + lines[i + 1:]))
+        assert found >= 2, name
 
 
 @needs_hipcc

@@ -309,6 +309,9 @@ int rbmoe_backward_block_host(rbmoe_layer* layer, const void* grad_output, int32
 
 /* Per-stage timing of one forward with HIP events on the context's stream.
  * `ms` receives RBMOE_NUM_STAGES durations in milliseconds.  Synchronises.
+ * Every stage has launches of its own here, one behind the other: a call that is not timed may have the dispatch inside the
+ * gate/up launch, and the shared expert's products inside the routed experts' launches or beside them on a second stream,
+ * and is then shorter than the stages' sum.
  * Stage 1 brackets no work at all: it reads what one pair of event records adds to
  * every other stage (about 5 us), so callers can subtract it. */
 #define RBMOE_NUM_STAGES 8
@@ -330,8 +333,10 @@ int rbmoe_forward_timed(rbmoe_layer* layer, const void* x, int32_t T, int32_t co
  * start and stop events, which receive the begin and end time stamps of that dispatch itself (no launch gap, no
  * event-pair overhead, no events between the stages).  `ms` receives RBMOE_NUM_STAGES values in milliseconds: per
  * stage the sum over its launches (RBMOE_STAGE_EMPTY: 0), RBMOE_STAGE_TOTAL: their sum - the time the device spent
- * inside kernels, which is less than the forward took by the gaps between the launches.  Synchronises.  Like
- * rbmoe_forward_timed, the call runs the shared expert on the main stream. */
+ * inside kernels, which is less than the forward took by the gaps between the launches.  Synchronises.  Where the
+ * gate/up launch does the dispatch's work, RBMOE_STAGE_DISPATCH is 0.  A large-batch call's shared expert has launches of its
+ * own on the main stream here, like rbmoe_forward_timed's; one that is not timed may have it inside the routed experts'
+ * launches or beside them. */
 int rbmoe_forward_kernel_times(rbmoe_layer* layer, const void* x, int32_t T, int32_t cols,
                                const uint8_t* valid, const float* router_bias, const void* residual,
                                void* out, float* ms);
@@ -344,7 +349,8 @@ int rbmoe_forward_kernel_times(rbmoe_layer* layer, const void* x, int32_t T, int
  * what a kernel trace shows for the launch; the operands a stage shares with its neighbours in a forward may sit
  * in other cache levels here.  With ms_per_launch == NULL the launches are only enqueued (no warm-up, no events, no
  * synchronisation): for a caller that times a sequence of its own, e.g. the same stage of several layers in
- * rotation.  RBMOE_UNSUPPORTED when the last forward had no launch of its own for the stage. */
+ * rotation.  RBMOE_UNSUPPORTED when the last forward had nothing to do for the stage, or did it in a decode-shaped launch; a
+ * dispatch inside a gate/up launch is replayed as the launch it would be, and gate/up and down as the routed experts' alone. */
 int rbmoe_replay_stage(rbmoe_layer* layer, int32_t stage, int32_t launches, float* ms_per_launch);
 
 /* Name of the kernels the last forward used for the expert products, for reports: "mfma_bf16_stream" (large

@@ -1489,7 +1489,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // 40 rows 24.3 / 30.2, 8192 rows (396 tiles) 42.3 / 46.3; d 512, 8 experts of 352 and a shared one, 64 rows 26.8 / 30.9, 2048
     // (156) 37.1 / 40.7, 6144 (444) 71.2 / 76.3, 8192 (588) 86.2 / 85.0; d 768, 8 of 1408, 64 rows 33.0 / 37.3, 2048 (396) 58.8 / 62.8,
     // 4096 (748) 87.6 / 83.9; 16 of 1408, 512 rows 41.8 / 45.1, 3072 (616) 79.1 / 80.8, 8192 (1496) 151.0 / 139.4.
-    // (Not where a host call fetches the tables beside the products, nor where the stages are timed one by one.)
+    // (Not where a host call fetches the tables beside the products, nor with events between the stages.)
     // Over f32 rows, workgroups as f32_workgroups counts them: d 512, 8 experts of 352 and a shared one, bf16 weights, 64 rows
     // 27.3 / 31.2, 1024 (600 workgroups) 42.6 / 45.8, 4096 (588) 91.0 / 93.0, 8192 (1164) 148.0 / 145.5; f32 weights, 8 of 1408, 1024
     // (396) 90.2 / 95.5, 4096 (1452) 260.7 / 261.6; d 768, 16 of 682, four a row, 512 (288) 91.9 / 95.2, 2048 (816) 205.5 / 202.8.
@@ -1497,7 +1497,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     GroupedArgs first = shared_inside ? with_shared(g1, s1) : g1;
     const int workgroups = mfma ? g1.likely_tiles * ((F + 127) / 128) + (first.dense2.rows + 127) / 128 * ((first.dense2.N + 127) / 128)
                                 : L->f32_rows ? f32_workgroups(first, wk) : 0;
-    const bool dispatch_inside = (mfma || L->f32_rows) && gather_in_product && !timed && !L->record_routed &&
+    const bool dispatch_inside = (mfma || L->f32_rows) && gather_in_product && timing != 1 && !L->record_routed &&
                                  workgroups <= (mfma ? kDispatchInsideTiles : kDispatchInsideF32) && dispatch_in_product_ok(da);
     if (dispatch_inside) first.slots = routed_slots(da);
     if (!dispatch_inside) HIP_TRY(ctx, launch_dispatch(da, abf || cast, s));

@@ -66,3 +66,19 @@ def test_measuring_entry_points_leave_the_results_alone(device, shape):
     layer.close()
     xb.free()
     ob.free()
+
+
+@pytest.mark.parametrize("act,E,inside", [("bf16", 8, True), ("f32", 8, True), ("bf16", 6, False)])
+def test_kernel_times_are_those_of_the_calls_own_launches(device, act, E, inside):
+    """A gate/up launch that does the dispatch's work does it here too: no time for a launch that the call does not have (six
+    experts: it has one)."""
+    t = synth.make(small_workload(seed=92, act=act, wt=act, d=64, E=E, k=2, F=64, T=300))
+    layer = gpu_layer(device, t)
+    x = synth.f32_to_bf16_bits(t.x) if act == "bf16" else t.x
+    xb, ob = DeviceBuffer(device, x.nbytes).upload(x), DeviceBuffer(device, x.nbytes)
+    kt = layer.forward_kernel_times(xb.ptr, 300, ob.ptr)
+    assert (kt["dispatch"] == 0) == inside and min(kt["router"], kt["gate_up"], kt["down"], kt["combine"]) > 0
+    assert layer.forward_timed(xb.ptr, 300, ob.ptr)["dispatch"] > 0
+    layer.close()
+    xb.free()
+    ob.free()

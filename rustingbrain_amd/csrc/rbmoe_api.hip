@@ -2703,6 +2703,23 @@ int rbmoe_internal_router_plan(int32_t d, int32_t E, int32_t k, int32_t T, int32
     return RBMOE_OK;
 }
 
+// Test hook (not part of rbmoe.h), runs without a GPU: experts of a routing workgroup of a large-batch call on aligned rows, 0
+// where a block's experts are not shared out.
+int rbmoe_internal_router_slice(int32_t d, int32_t E, int32_t k, int32_t T, int32_t bf16, int32_t norm, int32_t quantized) {
+    RouterArgs a{};
+    a.T = T; a.d = d; a.E = E; a.k = k;
+    a.allow_fused = true;
+    a.x = reinterpret_cast<void*>((uintptr_t)1 << 20);  // (never read)
+    a.wr = static_cast<const float*>(a.x);
+    if (quantized) {
+        a.wq = static_cast<const int8_t*>(a.x);
+        a.wscale = a.wr;
+    }
+    if (norm) a.norm_w = a.wr;
+    a.arrive = reinterpret_cast<int*>((uintptr_t)1 << 20);
+    return plan_router(a, bf16 != 0).row_slice;
+}
+
 int rbmoe_copy_device(rbmoe_ctx* ctx, void* dst, const void* src, size_t bytes) {
     if (!ctx) return fail(nullptr, RBMOE_NULL_POINTER, "ctx is NULL");
     if (bytes == 0) return RBMOE_OK;

@@ -9,17 +9,27 @@ from conftest import rel_l2
 from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
 from oracle import rb_oracle as orc
 from rustingbrain_amd import synth
+from test_router_plan import router_slice
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [dict(E=64, k=6, T=33), dict(E=64, k=2, T=256), dict(E=64, k=2, T=257), dict(E=64, k=4, T=1020), dict(E=32, k=4, T=40),
-          dict(E=32, k=1, T=512), dict(E=32, k=2, T=513), dict(E=44, k=3, T=77), dict(E=33, k=2, T=41)]
+# (experts, choices, tokens) -> experts of a workgroup
+SHAPES = [dict(E=64, k=6, T=33, n=8), dict(E=64, k=2, T=256, n=8), dict(E=64, k=2, T=257, n=16), dict(E=64, k=4, T=1020, n=32),
+          dict(E=32, k=4, T=40, n=8), dict(E=32, k=1, T=512, n=8), dict(E=32, k=2, T=513, n=16), dict(E=44, k=3, T=77, n=8),
+          dict(E=33, k=2, T=41, n=8), dict(E=44, k=3, T=1020, n=32), dict(E=40, k=2, T=420, n=16)]
+# 512 columns: a wave takes the norm of a row; 544 (17 steps of 32 columns): a thread does
+CASES = [(512, s) for s in SHAPES] + [(544, SHAPES[i]) for i in (0, 2, 3, 9)]
 
 
 @pytest.mark.parametrize("act,wt,quantized", [("bf16", "bf16", False), ("f32", "bf16", False), ("f32", "f32", False), ("bf16", "int8", True)])
-@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "E{E}_k{k}_T{T}".format(**s))
-def test_experts_of_a_block_shared_out(device, shape, act, wt, quantized):
-    t = synth.make(small_workload(seed=67, act=act, wt=wt, d=192, F=64, **shape))
+@pytest.mark.parametrize("d,shape", CASES, ids=["d{}_E{E}_k{k}_T{T}".format(d, **s) for d, s in CASES])
+def test_experts_of_a_block_shared_out(device, d, shape, act, wt, quantized):
+    shape = dict(shape)
+    slice_ = shape.pop("n")
+    for norm in (0, 1):
+        if not (norm and quantized):
+            assert router_slice(d, shape["E"], shape["k"], shape["T"], act == "bf16", norm, quantized) == slice_
+    t = synth.make(small_workload(seed=67, act=act, wt=wt, d=d, F=64, **shape))
     T, E = shape["T"], shape["E"]
     layer = gpu_layer(device, t)
     oracle = oracle_layer(t)

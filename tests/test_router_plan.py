@@ -19,6 +19,13 @@ def plan(d, E, k, T, bf16, norm, quantized, fused, x):
     return tuple(out)
 
 
+def router_slice(d, E, k, T, bf16, norm, quantized):
+    fn = L.load().rbmoe_internal_router_slice
+    fn.restype = C.c_int
+    fn.argtypes = [C.c_int32] * 7
+    return fn(d, E, k, T, bf16, norm, quantized)
+
+
 @pytest.mark.parametrize("quantized", [0, 1])
 @pytest.mark.parametrize("norm", [0, 1])
 @pytest.mark.parametrize("bf16", [0, 1])
@@ -39,3 +46,10 @@ def test_the_launch_takes_the_plan_the_dispatch_counts_by(offset, bf16, norm, qu
 def test_small_blocks_serve_calls_that_would_not_fill_the_chip():
     assert [plan(768, 16, 2, T, 1, 0, 0, 1, ALIGNED)[0] for T in (40, 203, 2048, 2049, 4096, 4097)] == [8, 8, 8, 16, 16, 32]
     assert plan(768, 16, 2, 203, 1, 0, 0, 1, ALIGNED + 2)[0] == 32   # rows off a 16-byte boundary without a norm in front
+
+
+def test_experts_of_a_block_are_shared_out_to_at_most_one_round_of_workgroups():
+    assert [router_slice(512, 64, 2, T, 1, 0, 0) for T in (5, 256, 257, 512, 513, 1020, 1024)] == [8, 8, 16, 16, 32, 32, 32]
+    assert [router_slice(512, E, 2, 40, 1, 0, 0) for E in (8, 31, 32, 33, 44)] == [0, 0, 8, 8, 8]
+    assert [router_slice(d, 32, 2, 40, 1, 0, 0) for d in (256, 504, 512, 544, 1024)] == [0, 0, 8, 8, 8]
+    assert router_slice(512, 64, 2, 2048, 1, 0, 0) == 0   # a round of workgroups as it is

@@ -1,11 +1,13 @@
 """Gate/up products that work out their own tiles and write the routing tables on the way, against the oracle's tables and,
-bit for bit, against the same call with a dispatch launch (which the timed forward keeps): first and last tile of an
-expert, experts without rows, a histogram of the largest size, blocks and batches with remainders, padding, padding only."""
+bit for bit, against the same call with a dispatch launch (which the timed forward keeps, and a call that writes the gathered
+rows out): first and last tile of an expert, experts without rows, a histogram of the largest size, blocks and batches with
+remainders, padding, padding only."""
 import numpy as np
 import pytest
 import torch
 
 from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
+from rustingbrain_amd import _lib as L
 from rustingbrain_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -15,11 +17,14 @@ SHAPES = [dict(E=8, k=2, T=33), dict(E=1, k=1, T=300), dict(E=2, k=2, T=257), di
           dict(E=6, k=2, T=130)]  # (six experts: the dispatch launch)
 
 
-@pytest.mark.parametrize("act,wt,shared", [("bf16", "bf16", False), ("bf16", "int8", True), ("f32", "bf16", True),
-                                           ("f32", "f32", False)])
+# widths off 64 (96): rows stay f32 over bf16 and int8 weights too; at 64 those rows are rounded to bf16
+@pytest.mark.parametrize("act,wt,shared,F,kernel", [
+    ("bf16", "bf16", False, 64, "mfma_bf16_stream"), ("bf16", "int8", True, 64, "mfma_bf16_stream_int8w"),
+    ("f32", "bf16", True, 64, "mfma_bf16_stream"), ("f32", "f32", False, 64, "mfma_f32"), ("f32", "f32", True, 64, "mfma_f32"),
+    ("f32", "bf16", True, 96, "generic"), ("f32", "int8", True, 96, "generic")])
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "E{E}_k{k}_T{T}".format(**s))
-def test_tables_and_outputs_without_a_dispatch_launch(device, shape, act, wt, shared):
-    t = synth.make(small_workload(seed=61, act=act, wt=wt, shared=shared, shared_d_ff=128, d=64, F=64, **shape))
+def test_tables_and_outputs_without_a_dispatch_launch(device, shape, act, wt, shared, F, kernel):
+    t = synth.make(small_workload(seed=61, act=act, wt=wt, shared=shared, shared_d_ff=128 if F == 64 else F, d=64, F=F, **shape))
     T, E = shape["T"], shape["E"]
     dt = torch.bfloat16 if act == "bf16" else torch.float32
     x = torch.from_numpy(np.ascontiguousarray(t.x)).to(dt).cuda()
@@ -31,12 +36,19 @@ def test_tables_and_outputs_without_a_dispatch_launch(device, shape, act, wt, sh
         layer = gpu_layer(device, t)
         dv, db = torch.from_numpy(valid).cuda(), torch.from_numpy(bias).cuda()
         got = {}
-        for way, call in (("inside", layer.forward_device), ("launch", layer.forward_timed)):
+        f32_joined = shared and kernel in ("mfma_f32", "generic")
+        for way, call in (("inside", layer.forward_device), ("launch", layer.forward_device if f32_joined else layer.forward_timed)):
+            if way == "launch" and f32_joined:   # (the timed forward's f32 shared expert, in launches of its own, has other tiles)
+                layer.set_option(L.OPT_EXPLICIT_GATHER, 1)
             out = torch.full_like(x, 7.0)
             torch.cuda.synchronize()
             call(x.data_ptr(), T, out.data_ptr(), dv.data_ptr(), db.data_ptr())
             device.synchronize()
             got[way] = (out.cpu(), layer.cache(T, int(valid.sum())), layer.losses())
+        assert layer.kernel_name() == kernel
+        layer.set_option(L.OPT_EXPLICIT_GATHER, 0)
+        if T <= 1000:   # (the call by itself: larger ones may have a launch, by the number of their tiles)
+            assert (layer.forward_kernel_times(x.data_ptr(), T, out.data_ptr(), dv.data_ptr(), db.data_ptr())["dispatch"] == 0) == (E != 6)
         (out, cache, losses), (out2, cache2, losses2) = got["inside"], got["launch"]
         assert_routing_identical(cache, cache_as_ref(cache2))
         assert losses == losses2

@@ -136,7 +136,7 @@ const char* rbmoe_last_global_error(void);
  * weights are not rounded: at widths off 64 they keep those widths and f32 accuracy, at multiples of 64 the
  * products take a bf16 copy of the rows (RBMOE_OPT_FORCE_GENERIC: f32 accuracy there too, at a thirtieth of the rate).  A layer whose rounded
  * widths are over the budget - here, or when the norm or training mode is added before the first weight - or over a limit
- * of the backward products keeps its true widths and the any-shape kernels instead.  Layers that already hold
+ * of the backward products keeps its true widths instead (bf16 rows then take the any-shape kernels).  Layers that already hold
  * weights stay as they are: a budget shared by several layers has to allow for their rounded widths. */
 int rbmoe_layer_create(rbmoe_ctx* ctx, const rbmoe_config* cfg, rbmoe_layer** out);
 void rbmoe_layer_destroy(rbmoe_layer* layer);
@@ -355,8 +355,9 @@ int rbmoe_replay_stage(rbmoe_layer* layer, int32_t stage, int32_t launches, floa
 
 /* Name of the kernels the last forward used for the expert products, for reports: "mfma_bf16_stream" (large
  * batches), "mfma_bf16_decode_front" (a few tokens, routing beside the gate/up products), "mfma_bf16_decode" (a few
- * tokens, routing in a launch of its own), each with "_int8w" behind it for int8 weights, "mfma_f32", "generic"; "none"
- * before the first.  Static storage. */
+ * tokens, routing in a launch of its own), each with "_int8w" behind it for int8 weights, "mfma_f32" (all-f32 layers
+ * at widths of whole slices), "generic" (every other layer: f32 rows, whose products run on the matrix cores like mfma_f32's
+ * unless RBMOE_OPT_FORCE_GENERIC is set, and bf16 rows on the any-shape kernels); "none" before the first.  Static storage. */
 const char* rbmoe_expert_kernel_name(const rbmoe_layer* layer);
 
 /* Device memory helpers for hosts without their own HIP binding. */

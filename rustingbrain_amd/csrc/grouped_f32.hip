@@ -23,9 +23,10 @@
 // weight fragments (88 vector instructions, 352 cycles).  The rows are split once per workgroup, on their way from registers
 // into three bf16 planes in LDS; weights go to LDS by LDS-DMA as they are and a wave splits its own fragments (nobody else
 // needs them), so they take 4 bytes a value on every path.  Everything of a step sits between its multiplies, one piece
-// behind each (see `step`).  Large launches run at the power limit: 8192 tokens, same layer, gate/up 451 -> 283 us (the
-// six bf16 products at 1000 TFLOP/s, where the library's large bf16 product reaches 1160), down 236 -> 160; 1024 tokens
-// 75 -> 46 and 44 -> 31, against the kernel on the f32 unit.  Small ones are a chain of slices and memory: see f32_tile.
+// behind each (see `step`).  Large launches run at the power limit: 8192 tokens, same layer, gate/up 451 -> 288 us (the
+// six bf16 products at 985 TFLOP/s, where the library's large bf16 product reaches 1160), down 236 -> 163; 1024 tokens
+// 75 -> 47 and 44 -> 31, against the kernel on the f32 unit (of the large launches 1 % is the look at the rows' largest values
+// and the sums' sizes, of the smallest 0.2 us).  Small ones are a chain of slices and memory: see f32_tile.
 // f32 rows over bf16 or int8 weights at widths off 64 ran on the any-shape kernel's 20 TFLOP/s: 52 rows, d 768, 32 experts
 // of 352 and a shared one 154 -> 58 us a forward.
 //
@@ -751,7 +752,8 @@ bool f32_shape_ok(int N, int K) { return K % 32 == 0 && K >= 32 && N % 4 == 0 &&
 // Tokens x features of a workgroup, and its waves.  A launch is bound by the length of one workgroup's chain until there
 // are about as many workgroups as compute units, and by the multiplies from there on, which the larger tiles feed best.
 // So: the smallest tile of which there is at most one a compute unit (bf16 and int8 weights, a third of the multiplies
-// and of the LDS a tile: some more of them together), then 64 x 128.  us, all at 8 experts top-2, d 512:
+// and of the LDS a tile: some more of them together), then 64 x 128.  us, all at 8 experts top-2, d 512 (swept before
+// the rows' largest values were looked at: the large ones take 1 % more now, whichever the tile):
 //   f32, gate/up of 1408     32x32 / 32x64 / 64x64 / 64x128 / the same on eight waves: 1 token 9.8 / 13.3 / 17.2 / 25.8 / -, 8
 //     tokens 14.0 / 12.7 / 17.6 / 26.2 / -, 128 20.2 / 19.7 / 17.6 / 25.8 / 23.9, 256 30.1 / 27.5 / 27.6 / 27.9 / 25.4, 1024
 //     71.1 / 59.6 / 52.9 / 46.4 / 50.1, 8192 499 / 374 / 301 / 284 / 319

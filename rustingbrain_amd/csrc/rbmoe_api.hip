@@ -237,8 +237,8 @@ struct rbmoe_layer {
     // write on the way, hidden and expert rows are bf16, and the combine sums them into f32 again
     bool cast_rows = false;
     bool use_f32_mc = false;   // all-f32 layer of whole tiles: the kernel set "mfma_f32"
-    bool f32_rows = false;     // products over f32 rows at f32 accuracy (launch_grouped_f32): with use_f32_mc, and on the
-                               // any-shape kernel set whatever the weights
+    bool f32_rows = false;     // products over f32 rows at f32 accuracy (launch_grouped_f32): with use_f32_mc, and without it
+                               // (the kernel name is then "generic") whatever the weights and widths
     bool decode_path = true;   // few tokens: launches that stream every touched weight once
     bool decode_front = true;  // ... the routing beside the gate/up products where that pays (decode_front_pays)
     bool shared_beside = true; // large batches: the shared expert's products on the side stream, beside the routing
@@ -327,9 +327,11 @@ void choose_kernel_sets(rbmoe_layer* L) {
     const rbmoe_config* cfg = &L->cfg;
     L->use_stream = L->use_f32_mc = L->cast_rows = L->f32_rows = false;
     // Expert widths are rounded up to whole tiles (the model width is the caller's row pitch and is not): 64 columns
-    // for the packed bf16 / int8 kernels, 32 for the f32 ones.  The any-shape kernels run at a thirtieth of the bf16
-    // matrix-core rate and a third of the f32 one, so rounding pays while it multiplies the work by less than that:
-    // up to four times (bf16) and twice (f32).  d_ff 352 (the default model's) is 384 columns: 9 % more work.
+    // for the packed bf16 / int8 kernels, 32 for the f32 ones.  bf16 rows at other widths take the any-shape kernels, a
+    // thirtieth of the matrix-core rate, so rounding pays up to four times the work and beyond.  All-f32 products at other
+    // widths (launch_grouped_f32) fetch both operands element by element, and twice the work is still ahead: us a forward, d 512,
+    // 8 experts, rounded / as they are: 682 (704) 64 rows 30.7 / 41.9, 1024 58.0 / 80.6, 4096 158 / 194; 130 (160) 1024 rows 36.6 /
+    // 44.3; 40 (64) 32.0 / 36.9; 33 (64) 64 rows 27.6 / 31.6, 4096 52.4 / 59.0.
     auto rounded = [L](int f, int unit, int most) {
         const int up = (f + unit - 1) / unit * unit;
         return up <= most * f && !L->tight ? up : f;
@@ -356,13 +358,13 @@ void choose_kernel_sets(rbmoe_layer* L) {
     }
     if (cfg->act_dtype == RBMOE_F32 && L->use_stream) {
         // the bf16 copy is written in 8-element pieces of 16-byte aligned rows.  Rounding a width would also round the
-        // rows: the any-shape kernels that such a layer has otherwise keep input, hidden and expert rows in f32 (1e-5
+        // rows: the products that such a layer has otherwise (f32_rows) keep input, hidden and expert rows in f32 (1e-5
         // against 3e-3), and the caller asked for f32 rows.
         const bool whole = L->Fw == cfg->d_ff && (!cfg->shared_expert || L->Fsw == L->Fs);
         if (cfg->d_model % 8 == 0 && whole) L->cast_rows = true;
         else L->use_stream = false;
     }
-    if (!L->use_stream && !L->use_f32_mc) {  // the any-shape kernels take the widths as they are
+    if (!L->use_stream && !L->use_f32_mc) {  // the other products take the widths as they are
         L->Fw = cfg->d_ff;
         L->Fsw = L->Fs;
     }
@@ -385,7 +387,8 @@ const char* training_widths_problem(const rbmoe_layer* L) {
                (!f32_shape_ok((int)d, (int)(2 * F)) || (c.shared_expert && !f32_shape_ok((int)d, (int)(2 * Fs))))) {
         return "expert width not supported by the backward products";
     }
-    return "";  // (any other layer - odd widths, mixed dtypes - takes the any-shape kernels in both directions)
+    return "";  // (any other layer - odd widths, mixed dtypes - takes its widths as they are in both directions: f32 rows
+                // through launch_grouped_f32, bf16 rows on the any-shape kernels)
 }
 
 Plan make_plan(rbmoe_layer* L) {
@@ -2647,7 +2650,7 @@ int rbmoe_internal_host_pool(uint64_t* used, uint64_t* kept) {
 }
 
 // Test hook (not part of rbmoe.h), runs without a GPU: the expert widths that the kernels of a layer see.  out[0]: routed,
-// [1]: shared, [2]: 0 any-shape kernels, 1 bf16 matrix cores, 2 f32 matrix cores; training != 0: after
+// [1]: shared, [2]: 1 mfma_bf16_*, 2 mfma_f32, 0 generic; training != 0: after
 // rbmoe_layer_enable_training, RBMOE_UNSUPPORTED where that refuses the widths.
 int rbmoe_internal_widths(const rbmoe_config* cfg, int32_t training, int32_t* out) {
     if (!cfg || !out) return RBMOE_NULL_POINTER;

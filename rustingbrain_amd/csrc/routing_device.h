@@ -278,8 +278,10 @@ __host__ __device__ static size_t route_rows_lds_bytes(int E, int k, int d, int 
 
 // The logits of the TB tokens of block `blk` for the experts [e_from, e_to) into the `prob` array (row pitch E | 1) of `lds_raw`, with everything in
 // front of them; the caller meets at a barrier before it reads them.  Kernels without the norm are compiled without its code:
-// with it they are 50 KB long instead of 25 and take 150 registers instead of 100, and 4096 tokens of d 768 by 8 experts are
-// routed in 10.4 us instead of 10.1.
+// with it (a wave's row at four widths, a thread's at any) they are 90 to 126 KB long instead of 35 to 63 and take 139 to 152
+// registers instead of 71 to 92, and 4096 tokens of d 768 by 8 experts are routed in 10.4 us instead of 10.1.  Both hold the
+// body twice, with all experts and with some; a launch runs one of them.  From swept caches, where code is fetched too, 203
+// tokens of d 768 by 16 experts are routed in 10.1 us, by the kernels of 26 KB with everything in one body in 10.8.
 template <typename XT, int TB, int NL, int TT, int EE, bool NORM>
 __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk, int e_from, int e_to,
                                                 unsigned char* __restrict__ lds_raw) {

@@ -1275,7 +1275,13 @@ __global__ __launch_bounds__(kSmallThreads, 2) void decode_front_kernel(RouteRow
     if ((int)blockIdx.x < routers) {
         const int k = r.k, ES = E | 1;
         const int t0 = blockIdx.x * kFrontTokens, nt = min(kFrontTokens, T - t0);
-        route_rows_body<XT, kFrontTokens, Q8 ? 32 : 8, Q8 ? 2 : 1, 2, NORM>(r, blockIdx.x, 0, r.E, lds);
+        bool routed = false;
+        if constexpr (sizeof(XT) == 2)
+            if (r.exact) {  // uniform over the launch
+                route_exact_body<kFrontTokens, Q8 ? 32 : 8, NORM>(r, blockIdx.x, 0, r.E, lds);
+                routed = true;
+            }
+        if (!routed) route_rows_body<XT, kFrontTokens, Q8 ? 32 : 8, Q8 ? 2 : 1, 2, NORM>(r, blockIdx.x, 0, r.E, lds);
         __syncthreads();
         float* const prob = reinterpret_cast<float*>(lds);  // the arrays of router_fixed_bytes
         float* const lsev = prob + kFrontTokens * ES;
@@ -1441,10 +1447,15 @@ __global__ __launch_bounds__(kSmallThreads, 2) void decode_front_kernel(RouteRow
 }
 
 // LDS of the launch; *EG: experts whose router rows a routing workgroup holds together.  0: the call does not fit.
-static size_t front_lds_bytes(int T, int E, int k, int d, bool q8, bool norm, int* EG) {
+static size_t front_lds_bytes(const RouterArgs& a, bool bf16, int* EG) {
+    const int T = a.T, E = a.E, k = a.k, d = a.d;
+    const bool q8 = a.wq != nullptr, norm = a.norm_w != nullptr, exact = route_exact_ok(a, bf16);
     const size_t products = ((size_t)front_room_floats(T, d, norm) + (norm ? d + 32 : 0)) * 4;
     int eg = E;
-    auto route = [&] { return route_rows_lds_bytes(E, k, d, kFrontTokens, q8 ? 32 : 8, eg, norm); };
+    auto route = [&] {
+        return exact ? route_exact_lds_bytes(E, k, d, kFrontTokens, q8 ? 32 : 8, eg)
+                     : route_rows_lds_bytes(E, k, d, kFrontTokens, q8 ? 32 : 8, eg, norm);
+    };
     while (eg > 8 && route() > (size_t)kMaxRouterLds) eg = (eg - 1) & ~1;
     if (route() > (size_t)kMaxRouterLds || products > (size_t)kMaxRouterLds) return 0;
     *EG = eg;
@@ -1458,7 +1469,7 @@ bool decode_front_ok(const RouterArgs& a, bool bf16) {
     return a.T >= 1 && a.T <= kSmallRouteMaxTokens && a.E <= 64 && a.k <= kMaxTopK && a.T * a.E <= kSmallRouteMaxPairs &&
            a.d % unit == 0 && a.d % 32 == 0 && (size_t)a.d * xsize % 16 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0 &&
            reinterpret_cast<uintptr_t>(a.wq ? static_cast<const void*>(a.wq) : a.wr) % 16 == 0 &&
-           front_lds_bytes(a.T, a.E, a.k, a.d, a.wq != nullptr, a.norm_w != nullptr, &eg) != 0;
+           front_lds_bytes(a, bf16, &eg) != 0;
 }
 
 hipError_t launch_decode_front(const RouterArgs& a, const DecodeGemmArgs& g, bool bf16, WeightKind wk, hipStream_t s) {
@@ -1469,9 +1480,9 @@ hipError_t launch_decode_front(const RouterArgs& a, const DecodeGemmArgs& g, boo
     const int routers = (a.T + kFrontTokens - 1) / kFrontTokens;
     const int grid = routers + (a.E + shared_tiles) * ((widest / 32 + kFrontTeams - 1) / kFrontTeams);
     int EG = 0;
-    const size_t lds = front_lds_bytes(a.T, a.E, a.k, a.d, a.wq != nullptr, a.norm_w != nullptr, &EG);
+    const size_t lds = front_lds_bytes(a, bf16, &EG);
     RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, EG, a.P, a.lse, a.expert_of, a.gate_of,
-                    nullptr, nullptr, nullptr, nullptr, a.norm_w, a.norm_eps, nullptr};
+                    nullptr, nullptr, nullptr, nullptr, a.norm_w, a.norm_eps, nullptr, route_exact_ok(a, bf16)};
     auto go = [&](auto kernel) -> hipError_t {
         static std::atomic<unsigned long long> attr_set{0};  // one per kernel: the lambda's body is instantiated for each
         const hipError_t e = once_per_device(attr_set, [&] {

@@ -67,6 +67,16 @@ uint16_t host_f32_to_bf16(float f) {
     b += 0x7fffu + ((b >> 16) & 1u);
     return (uint16_t)(b >> 16);
 }
+// RouterArgs::exact: bf16 values, zeros or of magnitudes from 2^-40 to below 2^20.
+bool router_weights_exact(const float* w, size_t n) {
+    for (size_t i = 0; i < n; ++i) {
+        uint32_t b;
+        std::memcpy(&b, w + i, 4);
+        const uint32_t exponent = (b >> 23) & 0xffu;
+        if ((b & 0xffffu) != 0 || ((b & 0x7fffffffu) != 0 && (exponent < 127 - 40 || exponent >= 127 + 20))) return false;
+    }
+    return true;
+}
 float host_bf16_to_f32(uint16_t h) {
     uint32_t b = (uint32_t)h << 16;
     float f;
@@ -256,6 +266,7 @@ struct rbmoe_layer {
     // weights
     Buf router;            // f32 [E, d]
     Buf router_q, router_s; // a quantized router: int8 [E, d], f32 scales [E] (`router` then holds the int8 values as f32)
+    bool router_exact = false;  // RouterArgs::exact of the router that is set
     bool router_q8 = false; // the layer routes with the quantized product (src/quantized.rs:55-62)
     bool quantize_router = false;  // f32 router data is quantized at upload (TransformerLm::quantize reaches the router too)
     int quant_rule = 0;     // f32 -> int8 at upload: 0 the checkpoint writer's rule, 1 the in-memory rule
@@ -847,6 +858,7 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
             HIP_TRY(ctx, hipMemcpy(L->router.p, src, n_given * 4, hipMemcpyHostToDevice));
         }
         L->router_q8 = router_to_i8;
+        L->router_exact = router_to_i8 || router_weights_exact(static_cast<const float*>(src), n_given);
         L->weights_set = true;
         return RBMOE_OK;
     }
@@ -1164,6 +1176,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     ra.allow_fused = L->fused_router;
     ra.arrive = (int*)L->cmbcnt.p;
     if (L->tight) ra.min_tokens = kRouterTokens;
+    ra.exact = L->router_exact;
     if (L->router_q8) {
         ra.wq = (const int8_t*)L->router_q.p;
         ra.wscale = (const float*)L->router_s.p;

@@ -84,6 +84,10 @@ struct RouterArgs {
     // `wr` is then not read and the logits are (sum_c x[c] * f32(q[c]), in the reference's 32 lanes) * scale
     const int8_t* wq = nullptr;      // [E, d]
     const float* wscale = nullptr;   // [E]
+    // Whether every router weight - of a quantized router: its whole number - is zero or a bf16 value of a magnitude from 2^-40 to
+    // below 2^20.  Times a bf16 element from 2^-72 to below 2^80 it is then exact in f32, and no sum of such products overflows
+    // or falls below 2^-126 on the way: the logits of bf16 rows may be taken by fused multiply-adds.
+    bool exact = false;
     // The norm in front of the layer (RmsNorm::forward, src/norm.rs:41-61), for calls whose plan says `takes_norm`: `x`
     // holds the raw rows, the routing is decided on the normed ones, which are written to `xn_out` [T, d].
     const float* norm_w = nullptr;
@@ -104,10 +108,11 @@ struct RouterPlan {
     // route_rows_kernel: experts whose router rows lie in LDS together (0: another kernel), LDS bytes
     int row_experts = 0;
     size_t row_lds = 0;
+    bool row_exact = false;  // ... route_exact_kernel in its place
     int row_slice = 0;  // ... and experts of a workgroup, where a block's experts are shared out (0: they are not)
     bool operator==(const RouterPlan& o) const {
         return block_tokens == o.block_tokens && takes_norm == o.takes_norm && q8_writes_rows16 == o.q8_writes_rows16 &&
-               row_experts == o.row_experts && row_lds == o.row_lds && row_slice == o.row_slice;
+               row_experts == o.row_experts && row_lds == o.row_lds && row_slice == o.row_slice && row_exact == o.row_exact;
     }
 };
 RouterPlan plan_router(const RouterArgs& a, bool bf16);

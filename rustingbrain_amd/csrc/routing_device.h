@@ -254,6 +254,7 @@ struct RouteRowsArgs {
     const float* norm_w;
     float norm_eps;
     void* xn_out;
+    bool exact = false;     // route_exact_body takes the rows
     int slice = 0;          // route_rows_kernel: experts of a workgroup (0: all of them)
     int* arrive = nullptr;  // ... and, with a slice, a token block's arrival counter, kDecodeCombineCounterStride apart
 };
@@ -574,5 +575,503 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
         }
     }
 }
+
+// ---------------------------------------------------------------------------
+// route_exact_body: what route_rows_body does, for bf16 rows and router weights whose products with them are exact
+// (RouterArgs::exact, RowRange): there one fused multiply-add rounds as the reference's multiply and add do, and the f32
+// matrix product of 16 x 16 x 4 is just that - its four columns one after the other, in index order, a fused multiply-add
+// each (held against fmaf in every bit for bf16 and f32 operands, 5e4 sums) - so a column lane's sums run on the matrix cores, at
+// four times the rate of a multiply and an add on the vector units and a sixteenth of their reads from LDS.
+// Rows and router rows lie in LDS in bf16, column lane by column lane, and within one the 16 steps of a block so that lane
+// (row, q) of the product finds its steps q, q + 4, q + 8, q + 12 in one 8-byte piece; who moves four pieces of a row there turns
+// them over in registers.  Wave w owns the column lanes w NL / 8 ..; the lanes' sums meet in LDS and are folded left to right by
+// a thread a logit.
+// A workgroup whose rows hold an element out of RowRange takes the same sums one multiply and one add at a time.
+// Bound by the length of a workgroup's chain, not by work: 203 tokens, d 768, 16 experts, behind a norm, from the kernel's start:
+// normed rows laid down at 2.6 us, every wave's rows and weights at 3.8, sums 5.2, folded 5.8, softmax and top-k 7.7, end 8.8
+// (route_rows_body 10.1); 8192 tokens without a norm 4.0, 6.4, 7.4, 9.2, 10.4 (11.7).  us a call, route_rows_body / this: the two
+// 48.4 / 47.6 and 157.3 / 153.3, 4096 tokens by 8 experts (int8) 91.3 / 89.8, 2048 of d 512 behind a norm 36.5 / 35.8.
+// ---------------------------------------------------------------------------
+// Elements of bf16 rows: nothing but zeros and magnitudes from 2^-72 to below 2^80.  Two at a time, as the bits lie in memory.
+struct RowRange {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 most = {0, 0}, least = {0xffff, 0xffff};  // of the magnitudes' bits; of the same less one, zeros aside
+    __device__ __forceinline__ void see(uint32_t two) {
+        const u16x2 m = __builtin_bit_cast(u16x2, two & 0x7fff7fffu);
+        most = __builtin_elementwise_max(most, m);
+        least = __builtin_elementwise_min(least, m - (u16x2){1, 1});
+    }
+    __device__ __forceinline__ void see(const uint4& v) { see(v.x); see(v.y); see(v.z); see(v.w); }
+    __device__ __forceinline__ bool left() const {
+        return max(most.x, most.y) >= ((127 + 80) << 7) || min(least.x, least.y) < ((127 - 72) << 7) - 1;
+    }
+};
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+__host__ __device__ static int exact_lane_steps(int d, int NL) { return (d / NL + 15) & ~15; }
+// Bytes of a staged row: 16 rows' pieces of the same step start in different banks.
+__host__ __device__ static int exact_row_bytes(int d, int NL) { return NL * exact_lane_steps(d, NL) * 2 + 16; }
+// Experts whose column lanes' sums meet in LDS at a time.
+__host__ __device__ constexpr int exact_round(int TB, int NL) { return TB * NL > 512 ? 8 : 16; }
+// Whether route_exact_body takes the call's rows (which lie on 16-byte boundaries, in whole turns of the column lanes).
+__host__ static inline bool route_exact_ok(const RouterArgs& a, bool bf16) {
+    return bf16 && a.exact && a.rows16 == nullptr && (!a.norm_w || wave_norms(a.d));
+}
+__host__ __device__ static size_t route_exact_lds_bytes(int E, int k, int d, int TB, int NL, int EG) {
+    return router_fixed_bytes(E, k, TB) + 4 * kRouterWaves + (size_t)NL * TB * exact_round(TB, NL) * 4 +
+           (size_t)(TB + EG) * exact_row_bytes(d, NL);
+}
+
+template <int TB, int NL, bool NORM>
+__device__ __forceinline__ void route_exact_body(const RouteRowsArgs& a, int blk, int e_from, int e_to,
+                                                 unsigned char* __restrict__ lds_raw) {
+    constexpr int NT = kRouterThreads, LW = NL / 8, MB = (TB + 15) / 16, RE = exact_round(TB, NL);
+    const int T = a.T, d = a.d, E = a.E, k = a.k, EG = a.EG, ES = E | 1;
+    float* const prob = reinterpret_cast<float*>(lds_raw);
+    int* const left = reinterpret_cast<int*>(lds_raw + router_fixed_bytes(E, k, TB));  // [waves] elements out of RowRange
+    float* const part = reinterpret_cast<float*>(left + kRouterWaves);                 // [NL][TB][RE]
+    const int S = d / NL, Sp = exact_lane_steps(d, NL), pitch = exact_row_bytes(d, NL);
+    unsigned char* const xs = reinterpret_cast<unsigned char*>(part + NL * TB * RE);
+    unsigned char* const ws = xs + TB * pitch;
+    const int tid = threadIdx.x, t0 = blk * TB, nt = min(TB, T - t0);
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+    // Staging.  A piece is eight neighbouring columns; a task four pieces of a row, the steps 16 Q + 4 i + q.  (Past the end of
+    // a row: zeros, which sums do not see.)
+    constexpr int JB = NL / 8;  // pieces of a step
+    const int per_row = Sp / 4 * JB;
+    const uint32_t recip = (uint32_t)(0x100000000ull / (uint32_t)per_row) + 1u;  // exact for the few thousand tasks there are
+    struct Task {
+        int row, step, jb;  // its first step
+        unsigned at;        // bytes from the row's start in LDS
+    };
+    auto task = [&](int i) {
+        Task t;
+        t.row = (int)__umulhi((uint32_t)i, recip);
+        const int r = i - t.row * per_row, q = r / JB;  // 4 Q + q
+        t.jb = r % JB;
+        t.step = 16 * (q >> 2) + (q & 3);
+        t.at = (unsigned)(8 * t.jb * Sp * 2 + 8 * q);
+        return t;
+    };
+    auto turn = [&](unsigned char* to, const uint4 (&p)[4]) {  // p[i]: eight columns of step i, as bf16
+        const uint32_t w[4][4] = {{p[0].x, p[0].y, p[0].z, p[0].w}, {p[1].x, p[1].y, p[1].z, p[1].w},
+                                  {p[2].x, p[2].y, p[2].z, p[2].w}, {p[3].x, p[3].y, p[3].z, p[3].w}};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t pick = j & 1 ? 0x07060302u : 0x05040100u;
+            const uint2 v = make_uint2(__builtin_amdgcn_perm(w[1][j >> 1], w[0][j >> 1], pick),
+                                       __builtin_amdgcn_perm(w[3][j >> 1], w[2][j >> 1], pick));
+            *reinterpret_cast<uint2*>(to + j * Sp * 2) = v;
+        }
+    };
+    const uint4 zero = make_uint4(0, 0, 0, 0);
+    struct Weights {  // a task's columns as they lie in memory
+        uint4 v[NL == 32 ? 2 : 8];
+    };
+    auto weights_of = [&](int e0, int n, int i) {  // (past the end: the last task again)
+        const Task t = task(min(i, n - 1));
+        Weights w;
+        if constexpr (NL == 32) {
+            uint2 h[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                h[u] = *reinterpret_cast<const uint2*>(a.wq + (size_t)(e0 + t.row) * d + 32 * min(t.step + 4 * u, S - 1) + 8 * t.jb);
+            w.v[0] = make_uint4(h[0].x, h[0].y, h[1].x, h[1].y);
+            w.v[1] = make_uint4(h[2].x, h[2].y, h[3].x, h[3].y);
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint4* const from = reinterpret_cast<const uint4*>(a.wr + (size_t)(e0 + t.row) * d + 8 * min(t.step + 4 * u, S - 1));
+                w.v[2 * u] = from[0];
+                w.v[2 * u + 1] = from[1];
+            }
+        }
+        return w;
+    };
+    auto put_weights = [&](int n, int i, const Weights& w) {
+        if (i >= n) return;
+        const Task t = task(i);
+        uint4 p[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if constexpr (NL == 32) {
+                const uint4& v = w.v[u >> 1];
+                const uint2 h = u & 1 ? make_uint2(v.z, v.w) : make_uint2(v.x, v.y);
+                p[u] = make_uint4(widen2(h.x, 0), widen2(h.x, 16), widen2(h.y, 0), widen2(h.y, 16));
+            } else {
+                const uint4 &lo = w.v[2 * u], &hi = w.v[2 * u + 1];  // (bf16 values: the lower halves are zero)
+                p[u] = make_uint4(__builtin_amdgcn_perm(lo.y, lo.x, 0x07060302u), __builtin_amdgcn_perm(lo.w, lo.z, 0x07060302u),
+                                  __builtin_amdgcn_perm(hi.y, hi.x, 0x07060302u), __builtin_amdgcn_perm(hi.w, hi.z, 0x07060302u));
+            }
+            if (t.step + 4 * u >= S) p[u] = zero;
+        }
+        turn(ws + t.row * pitch + t.at, p);
+    };
+    auto rest_of_router = [&](int e0, int n, int from) {
+        for (int i = from + tid; i < n; i += NT) put_weights(n, i, weights_of(e0, n, i));
+    };
+    const int nw0 = min(EG, e_to - e_from) * per_row;
+    RowRange range;
+    if constexpr (NORM) {
+        // as in route_rows_body: a wave a row, each half of the wave half of a lane's elements (the widths of wave_norms)
+        const int half = (tid >> 5) & 1;
+        const bf16_t* const rows = static_cast<const bf16_t*>(a.x) + (size_t)t0 * d;
+        with_lane_elements(d, [&](auto l_tag) {
+            constexpr int L = decltype(l_tag)::value, H = L / 2;
+            const int c0 = (tid & 31) * L + half * H;
+            LaneRow<bf16_t, L> row;
+            row.load(rows + (size_t)min(wave, nt - 1) * d);
+            float4 nwv[H / 4];
+#pragma unroll
+            for (int i = 0; i < H / 4; ++i) nwv[i] = *reinterpret_cast<const float4*>(a.norm_w + c0 + 4 * i);
+            const Weights w = weights_of(e_from, nw0, tid);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+            for (int r = wave; r < nt; r += NT / 64) {
+                const float inv_r = row.inverse_rms(a.norm_eps);
+                float v[L];
+                row.widen(v);
+                if (r + NT / 64 < nt) row.load(rows + (size_t)(r + NT / 64) * d);
+                uint32_t o[H / 2];
+#pragma unroll
+                for (int i = 0; i < H; i += 2) {
+                    uint32_t two = 0;
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const float4 n4 = nwv[(i + u) / 4];
+                        const float n = (i + u) % 4 == 0 ? n4.x : (i + u) % 4 == 1 ? n4.y : (i + u) % 4 == 2 ? n4.z : n4.w;
+                        const uint32_t b = f32_to_bf16_bits(__fmul_rn(__fmul_rn(half ? v[H + i + u] : v[i + u], inv_r), n));
+                        two |= b << (16 * u);
+                        const int c = c0 + i + u, t = c / NL, j = c % NL;
+                        *reinterpret_cast<uint16_t*>(xs + r * pitch + (j * Sp + (t & ~15) + (t & 3) * 4 + ((t >> 2) & 3)) * 2) = (uint16_t)b;
+                    }
+                    range.see(two);
+                    o[i / 2] = two;
+                }
+                if (a.xn_out != nullptr) {
+                    bf16_t* const to = static_cast<bf16_t*>(a.xn_out) + (size_t)(t0 + r) * d + c0;
+#pragma unroll
+                    for (int i = 0; i < H / 4; ++i) *reinterpret_cast<uint2*>(to + 4 * i) = make_uint2(o[2 * i], o[2 * i + 1]);
+                }
+            }
+            put_weights(nw0, tid, w);
+        });
+        // (a row's steps past its end)
+        if (S < Sp)
+            for (int i = tid; i < TB * NL * (Sp - S); i += NT) {
+                const int q = i / (Sp - S), t = S + i % (Sp - S);
+                *reinterpret_cast<uint16_t*>(xs + (q / NL) * pitch + ((q % NL) * Sp + (t & ~15) + (t & 3) * 4 + ((t >> 2) & 3)) * 2) = 0;
+            }
+    } else {
+        const bf16_t* const rows = static_cast<const bf16_t*>(a.x) + (size_t)t0 * d;
+        const int nx = nt * per_row;
+        struct Rows {
+            uint4 v[4];
+        };
+        auto rows_of = [&](int i) {
+            const Task t = task(min(i, nx - 1));
+            Rows r;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                r.v[u] = *reinterpret_cast<const uint4*>(rows + (size_t)t.row * d + NL * min(t.step + 4 * u, S - 1) + 8 * t.jb);
+            return r;
+        };
+        auto put_rows = [&](int i, Rows r) {
+            if (i >= nx) return;
+            const Task t = task(i);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (t.step + 4 * u >= S) r.v[u] = zero;
+                range.see(r.v[u]);
+            }
+            turn(xs + t.row * pitch + t.at, r.v);
+        };
+        // (two tasks a thread requested before the first is turned over, then the router's)
+        Rows r0 = rows_of(tid), r1 = r0;
+        if (NT < nx) r1 = rows_of(tid + NT);
+        const Weights w = weights_of(e_from, nw0, tid);
+        __builtin_amdgcn_sched_barrier(0);
+        put_rows(tid, r0);
+        put_rows(tid + NT, r1);
+        for (int i = tid + 2 * NT; i < nx; i += NT) put_rows(i, rows_of(i));
+        put_weights(nw0, tid, w);
+    }
+    rest_of_router(e_from, nw0, NT);
+    {
+        const bool any = __ballot(range.left()) != 0ull;
+        if (lane == 0) left[wave] = any;
+    }
+    __syncthreads();
+    bool exact = true;
+#pragma unroll
+    for (int w = 0; w < kRouterWaves; ++w) exact = exact && left[w] == 0;
+    // ---- the column lanes' sums, 16 (RE) experts at a time ----------------------------
+    const int blocks = (S + 15) / 16, last = (S - 16 * (blocks - 1) + 3) / 4;  // products of the last block of steps
+    for (int e0 = e_from; e0 < e_to; e0 += EG) {
+        const int ng = min(EG, e_to - e0);
+        if (e0 > e_from) {  // (every wave is behind the barrier in front of the last round's fold)
+            rest_of_router(e0, ng * per_row, 0);
+            __syncthreads();
+        }
+        for (int r0 = 0; r0 < ng; r0 += RE) {
+            const int ne = min(RE, ng - r0);
+            if (r0 > 0 || e0 > e_from) __syncthreads();  // the round before has been folded
+            const unsigned char* const wr = ws + r0 * pitch;
+            if (exact) {  // uniform over the workgroup
+                const unsigned char* x[MB];
+                const unsigned at = (unsigned)(wave * LW * Sp * 2 + 8 * (lane >> 4));
+#pragma unroll
+                for (int b = 0; b < MB; ++b) x[b] = xs + min(16 * b + (lane & 15), nt - 1) * pitch + at;
+                const unsigned char* const w = wr + min(lane & 15, ne - 1) * pitch + at;
+                floatx4 acc[LW][MB];
+#pragma unroll
+                for (int u = 0; u < LW; ++u)
+#pragma unroll
+                    for (int b = 0; b < MB; ++b) acc[u][b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                struct Operands {
+                    uint2 x[LW][MB], w[LW];
+                };
+                auto read = [&](int Q) {
+                    Operands o;
+#pragma unroll
+                    for (int u = 0; u < LW; ++u) {
+                        o.w[u] = *reinterpret_cast<const uint2*>(w + u * Sp * 2 + 32 * Q);
+#pragma unroll
+                        for (int b = 0; b < MB; ++b) o.x[u][b] = *reinterpret_cast<const uint2*>(x[b] + u * Sp * 2 + 32 * Q);
+                    }
+                    return o;
+                };
+                auto multiply = [&](const Operands& o, int n) {
+                    auto value = [](const uint2& v, int i) {
+                        const uint32_t two = i < 2 ? v.x : v.y;
+                        return __uint_as_float(i & 1 ? two & 0xffff0000u : two << 16);
+                    };
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (i < n)
+#pragma unroll
+                            for (int u = 0; u < LW; ++u)
+#pragma unroll
+                                for (int b = 0; b < MB; ++b)
+                                    acc[u][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(value(o.x[u][b], i), value(o.w[u], i), acc[u][b], 0, 0, 0);
+                };
+                Operands o = read(0);
+                for (int Q = 0; Q + 1 < blocks; ++Q) {
+                    const Operands next = read(Q + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    multiply(o, 4);
+                    o = next;
+                }
+                multiply(o, last);
+                // lane l holds the sums of the tokens 4 (l / 16) .. + 3 (of a block of 16) and expert l % 16
+#pragma unroll
+                for (int u = 0; u < LW; ++u)
+#pragma unroll
+                    for (int b = 0; b < MB; ++b)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int t = 16 * b + 4 * (lane >> 4) + i, e = lane & 15;
+                            if (t < TB && e < ne) part[((wave * LW + u) * TB + t) * RE + e] = acc[u][b][i];
+                        }
+            } else {
+                for (int i = tid; i < nt * ne * NL; i += NT) {
+                    const int j = i % NL, t = i / NL / ne, e = i / NL - t * ne;
+                    const uint16_t* const xr = reinterpret_cast<const uint16_t*>(xs + t * pitch) + j * Sp;
+                    const uint16_t* const er = reinterpret_cast<const uint16_t*>(wr + e * pitch) + j * Sp;
+                    float sum = 0.0f;
+                    for (int s = 0; s < S; ++s) {
+                        const int p = (s & ~15) + (s & 3) * 4 + ((s >> 2) & 3);
+                        sum = __fadd_rn(sum, __fmul_rn(bf16_bits_to_f32(xr[p]), bf16_bits_to_f32(er[p])));
+                    }
+                    part[(j * TB + t) * RE + e] = sum;
+                }
+            }
+            __syncthreads();
+            for (int i = tid; i < nt * RE; i += NT) {
+                const int t = i / RE, e = e0 + r0 + i % RE;
+                if (i % RE >= ne) continue;
+                float v[NL], y = 0.0f;
+#pragma unroll
+                for (int l = 0; l < NL; ++l) v[l] = part[l * TB * RE + i];
+#pragma unroll
+                for (int l = 0; l < NL; ++l) y = __fadd_rn(y, v[l]);
+                y = __fadd_rn(y, 0.0f);  // the reference adds its (empty) scalar rest: sum + 0
+                if constexpr (NL == 32) y = __fmul_rn(y, a.wscale[e]);
+                if (a.bias) y = __fadd_rn(y, a.bias[e]);
+                prob[t * ES + e] = y;
+            }
+        }
+    }
+}
+
+// router_tail: everything behind the logits for the TB tokens of router block `blk` - softmax, log-sum-exp, top-k,
+// gates, ranks, block histogram, partial sums of the losses.  LOADED = false: the logits are read from P;
+// true: the caller has put them into the `prob` array of `lds_raw` (row pitch E | 1) and met at a barrier.
+// MAXJ = experts a lane may own: 1 when E <= 64 (a lane owns one expert), kMaxExperts / 64 otherwise.
+template <int MAXJ, bool LOADED, int TB = kRouterTokens>
+__device__ __forceinline__ void router_tail(
+    unsigned char* __restrict__ lds_raw, int blk, const uint8_t* __restrict__ valid, int T, int E, int k,
+    float* __restrict__ P, float* __restrict__ lse, int* __restrict__ expert_of, float* __restrict__ gate_of,
+    int* __restrict__ rank_in_block, int* __restrict__ blockcnt, float* __restrict__ partial) {
+    const int ES = E | 1;
+    float* prob = reinterpret_cast<float*>(lds_raw);
+    float* lsev = prob + TB * ES;
+    float* gates = lsev + TB;
+    int* lexp = reinterpret_cast<int*>(gates + TB * k);
+    int* wcount = lexp + TB * k;
+    int* running = wcount + kRouterWaves * E;
+
+    const int tid = threadIdx.x;
+    const int t0 = blk * TB;
+    const int nt = min(TB, T - t0);
+
+    // ---- logits were written to P by logits_kernel ------------------------------
+    if constexpr (!LOADED) {
+        for (int idx = tid; idx < nt * E; idx += kRouterThreads) {
+            const int i = idx / E;
+            prob[i * ES + (idx - i * E)] = P[(size_t)t0 * E + idx];
+        }
+    }
+    for (int idx = tid; idx < E; idx += kRouterThreads) running[idx] = 0;
+    __syncthreads();
+
+    // ---- softmax + top-k: G lanes per token, lane j of a group owns experts j, j + G, ... ----
+    {
+        int G = 1;
+        while (G < E && G < 64) G <<= 1;
+        // a wave's tokens (four of 32): all at once with up to 16 lanes per token, in more turns with 32 or 64 - the
+        // turns are worked on side by side (one instruction stream), because each is a chain of dependent steps
+        constexpr int TW = TB / kRouterWaves;
+        if (G == 64) softmax_topk<MAXJ, TW, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
+        else if (G == 32) softmax_topk<MAXJ, (TW + 1) / 2, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
+        else softmax_topk<MAXJ, (TW + 3) / 4, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
+    }
+    __syncthreads();
+
+    // ---- write probabilities, lse, assignments (coalesced) ----------------
+    for (int idx = tid; idx < nt * E; idx += kRouterThreads) {
+        const int i = idx / E;
+        const int e = idx - i * E;
+        P[(size_t)t0 * E + idx] = prob[i * ES + e];
+    }
+    if (tid < nt) lse[t0 + tid] = lsev[tid];
+    const int nls = nt * k;
+    for (int ls = tid; ls < nls; ls += kRouterThreads) {
+        expert_of[(size_t)t0 * k + ls] = lexp[ls];
+        gate_of[(size_t)t0 * k + ls] = gates[ls];
+    }
+
+    // ---- partial sums for the auxiliary losses (fixed order): the waves behind the first, which ranks the slots
+    // at the same time -----------------------------------------------------------
+    const bool one_wave_ranks = nls <= 64;
+    const int pfirst = one_wave_ranks ? 64 : 0;  // first thread that takes partial sums
+    for (int e = tid - pfirst; e >= 0 && e <= E; e += kRouterThreads - pfirst) {
+        float s = 0.0f;
+        for (int i0 = 0; i0 < nt; i0 += 8) {
+            float pvv[8];
+            int okv[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int i = min(i0 + u, nt - 1);
+                okv[u] = lexp[i * k];
+                pvv[u] = e < E ? prob[i * ES + e] : lsev[i] * lsev[i];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (i0 + u < nt && okv[u] >= 0) s += pvv[u];
+        }
+        partial[(size_t)blk * (E + 1) + e] = s;
+    }
+
+    // ---- rank of every local slot among earlier slots of the same expert --
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    int ebits = 0;
+    while ((1 << ebits) < E) ++ebits;
+    if (one_wave_ranks) {
+        // every slot of the block in one wave: a slot's rank is the number of lower lanes with its expert, an
+        // expert's count the size of its group - no barrier, no second pass
+        if (wave == 0) {
+            const int e = (lane < nls) ? lexp[lane] : -1;
+            unsigned long long mask = __ballot(e >= 0);
+            for (int b = 0; b < ebits; ++b) {
+                const bool bit = (e >> b) & 1;
+                const unsigned long long bb = __ballot(bit);
+                mask &= bit ? bb : ~bb;
+            }
+            const int rank_w = __popcll(mask & ((1ull << lane) - 1ull));
+            if (e >= 0) {
+                rank_in_block[(size_t)t0 * k + lane] = rank_w;
+                if (rank_w == 0) running[e] = __popcll(mask);  // zero so far (cleared at the top)
+            }
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's LDS writes have landed
+            __builtin_amdgcn_wave_barrier();
+            for (int idx = lane; idx < E; idx += 64) blockcnt[(size_t)blk * E + idx] = running[idx];
+        }
+        return;
+    }
+    const int rounds = (nls + kRouterThreads - 1) / kRouterThreads;
+    for (int rd = 0; rd < rounds; ++rd) {
+        for (int idx = tid; idx < kRouterWaves * E; idx += kRouterThreads) wcount[idx] = 0;
+        __syncthreads();
+        const int ls = rd * kRouterThreads + tid;
+        const int e = (ls < nls) ? lexp[ls] : -1;
+        unsigned long long mask = __ballot(e >= 0);
+        for (int b = 0; b < ebits; ++b) {
+            const bool bit = (e >> b) & 1;
+            const unsigned long long bb = __ballot(bit);
+            mask &= bit ? bb : ~bb;
+        }
+        const int rank_w = __popcll(mask & ((1ull << lane) - 1ull));
+        if (e >= 0 && rank_w == 0) wcount[wave * E + e] = __popcll(mask);
+        __syncthreads();
+        if (e >= 0) {
+            int pre = running[e];
+            for (int w = 0; w < wave; ++w) pre += wcount[w * E + e];
+            rank_in_block[(size_t)t0 * k + ls] = pre + rank_w;
+        }
+        __syncthreads();
+        for (int idx = tid; idx < E; idx += kRouterThreads)
+            for (int w = 0; w < kRouterWaves; ++w) running[idx] += wcount[w * E + idx];
+        __syncthreads();
+    }
+    for (int idx = tid; idx < E; idx += kRouterThreads) blockcnt[(size_t)blk * E + idx] = running[idx];
+}
+
+// A token block's experts shared out over workgroups: each leaves its logits in P; the last to arrive fetches the others' into
+// its own array and goes on.  Device-scope stores and loads: the workgroups may sit on different XCDs, whose L2s do not see
+// each other's lines; a workgroup's stores are acknowledged before its arrival is counted.
+template <int TB>
+__device__ __forceinline__ bool last_slice(const RouteRowsArgs& a, int from, int to, unsigned char* lds_raw) {
+    float* const prob = reinterpret_cast<float*>(lds_raw);
+    const int E = a.E, ES = E | 1, tid = threadIdx.x;
+    int& last = *reinterpret_cast<int*>(prob + TB * ES);  // (where router_tail will keep the log-sum-exps)
+    const int t0 = blockIdx.x * TB, nt = min(TB, a.T - t0), n = to - from;
+    for (int i = tid; i < nt * n; i += kRouterThreads) {
+        const int t = i / n, e = from + i - t * n;
+        __hip_atomic_store(a.P + (size_t)(t0 + t) * E + e, prob[t * ES + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+        int* const counter = a.arrive + blockIdx.x * kDecodeCombineCounterStride;
+        const int before = atomicAdd(counter, 1);
+        last = before == (int)gridDim.y - 1;
+        if (before == (int)gridDim.y - 1) atomicExch(counter, 0);  // everyone has arrived: ready for the next launch
+    }
+    __syncthreads();
+    if (!last) return false;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    for (int i = tid; i < nt * E; i += kRouterThreads) {
+        const int t = i / E, e = i - t * E;
+        if (e < from || e >= to)
+            prob[t * ES + e] = __hip_atomic_load(a.P + (size_t)t0 * E + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return true;  // (router_tail begins with a barrier)
+}
+
+hipError_t launch_route_exact(const RouterArgs& a, const RouterPlan& p, hipStream_t s);  // (route_exact.hip)
 
 }  // namespace rbmoe

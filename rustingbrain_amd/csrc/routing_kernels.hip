@@ -240,140 +240,6 @@ __global__ __launch_bounds__(NE * 64, (!AHEAD && sizeof(XT) == 2) ? 6 : 2) void 
     }
 }
 
-// router_tail: everything behind the logits for the TB tokens of router block `blk` - softmax, log-sum-exp, top-k,
-// gates, ranks, block histogram, partial sums of the losses.  LOADED = false: the logits are read from P;
-// true: the caller has put them into the `prob` array of `lds_raw` (row pitch E | 1) and met at a barrier.
-// MAXJ = experts a lane may own: 1 when E <= 64 (a lane owns one expert), kMaxExperts / 64 otherwise.
-template <int MAXJ, bool LOADED, int TB = kRouterTokens>
-__device__ __forceinline__ void router_tail(
-    unsigned char* __restrict__ lds_raw, int blk, const uint8_t* __restrict__ valid, int T, int E, int k,
-    float* __restrict__ P, float* __restrict__ lse, int* __restrict__ expert_of, float* __restrict__ gate_of,
-    int* __restrict__ rank_in_block, int* __restrict__ blockcnt, float* __restrict__ partial) {
-    const int ES = E | 1;
-    float* prob = reinterpret_cast<float*>(lds_raw);
-    float* lsev = prob + TB * ES;
-    float* gates = lsev + TB;
-    int* lexp = reinterpret_cast<int*>(gates + TB * k);
-    int* wcount = lexp + TB * k;
-    int* running = wcount + kRouterWaves * E;
-
-    const int tid = threadIdx.x;
-    const int t0 = blk * TB;
-    const int nt = min(TB, T - t0);
-
-    // ---- logits were written to P by logits_kernel ------------------------------
-    if constexpr (!LOADED) {
-        for (int idx = tid; idx < nt * E; idx += kRouterThreads) {
-            const int i = idx / E;
-            prob[i * ES + (idx - i * E)] = P[(size_t)t0 * E + idx];
-        }
-    }
-    for (int idx = tid; idx < E; idx += kRouterThreads) running[idx] = 0;
-    __syncthreads();
-
-    // ---- softmax + top-k: G lanes per token, lane j of a group owns experts j, j + G, ... ----
-    {
-        int G = 1;
-        while (G < E && G < 64) G <<= 1;
-        // a wave's tokens (four of 32): all at once with up to 16 lanes per token, in more turns with 32 or 64 - the
-        // turns are worked on side by side (one instruction stream), because each is a chain of dependent steps
-        constexpr int TW = TB / kRouterWaves;
-        if (G == 64) softmax_topk<MAXJ, TW, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
-        else if (G == 32) softmax_topk<MAXJ, (TW + 1) / 2, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
-        else softmax_topk<MAXJ, (TW + 3) / 4, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
-    }
-    __syncthreads();
-
-    // ---- write probabilities, lse, assignments (coalesced) ----------------
-    for (int idx = tid; idx < nt * E; idx += kRouterThreads) {
-        const int i = idx / E;
-        const int e = idx - i * E;
-        P[(size_t)t0 * E + idx] = prob[i * ES + e];
-    }
-    if (tid < nt) lse[t0 + tid] = lsev[tid];
-    const int nls = nt * k;
-    for (int ls = tid; ls < nls; ls += kRouterThreads) {
-        expert_of[(size_t)t0 * k + ls] = lexp[ls];
-        gate_of[(size_t)t0 * k + ls] = gates[ls];
-    }
-
-    // ---- partial sums for the auxiliary losses (fixed order): the waves behind the first, which ranks the slots
-    // at the same time -----------------------------------------------------------
-    const bool one_wave_ranks = nls <= 64;
-    const int pfirst = one_wave_ranks ? 64 : 0;  // first thread that takes partial sums
-    for (int e = tid - pfirst; e >= 0 && e <= E; e += kRouterThreads - pfirst) {
-        float s = 0.0f;
-        for (int i0 = 0; i0 < nt; i0 += 8) {
-            float pvv[8];
-            int okv[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int i = min(i0 + u, nt - 1);
-                okv[u] = lexp[i * k];
-                pvv[u] = e < E ? prob[i * ES + e] : lsev[i] * lsev[i];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (i0 + u < nt && okv[u] >= 0) s += pvv[u];
-        }
-        partial[(size_t)blk * (E + 1) + e] = s;
-    }
-
-    // ---- rank of every local slot among earlier slots of the same expert --
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    int ebits = 0;
-    while ((1 << ebits) < E) ++ebits;
-    if (one_wave_ranks) {
-        // every slot of the block in one wave: a slot's rank is the number of lower lanes with its expert, an
-        // expert's count the size of its group - no barrier, no second pass
-        if (wave == 0) {
-            const int e = (lane < nls) ? lexp[lane] : -1;
-            unsigned long long mask = __ballot(e >= 0);
-            for (int b = 0; b < ebits; ++b) {
-                const bool bit = (e >> b) & 1;
-                const unsigned long long bb = __ballot(bit);
-                mask &= bit ? bb : ~bb;
-            }
-            const int rank_w = __popcll(mask & ((1ull << lane) - 1ull));
-            if (e >= 0) {
-                rank_in_block[(size_t)t0 * k + lane] = rank_w;
-                if (rank_w == 0) running[e] = __popcll(mask);  // zero so far (cleared at the top)
-            }
-            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's LDS writes have landed
-            __builtin_amdgcn_wave_barrier();
-            for (int idx = lane; idx < E; idx += 64) blockcnt[(size_t)blk * E + idx] = running[idx];
-        }
-        return;
-    }
-    const int rounds = (nls + kRouterThreads - 1) / kRouterThreads;
-    for (int rd = 0; rd < rounds; ++rd) {
-        for (int idx = tid; idx < kRouterWaves * E; idx += kRouterThreads) wcount[idx] = 0;
-        __syncthreads();
-        const int ls = rd * kRouterThreads + tid;
-        const int e = (ls < nls) ? lexp[ls] : -1;
-        unsigned long long mask = __ballot(e >= 0);
-        for (int b = 0; b < ebits; ++b) {
-            const bool bit = (e >> b) & 1;
-            const unsigned long long bb = __ballot(bit);
-            mask &= bit ? bb : ~bb;
-        }
-        const int rank_w = __popcll(mask & ((1ull << lane) - 1ull));
-        if (e >= 0 && rank_w == 0) wcount[wave * E + e] = __popcll(mask);
-        __syncthreads();
-        if (e >= 0) {
-            int pre = running[e];
-            for (int w = 0; w < wave; ++w) pre += wcount[w * E + e];
-            rank_in_block[(size_t)t0 * k + ls] = pre + rank_w;
-        }
-        __syncthreads();
-        for (int idx = tid; idx < E; idx += kRouterThreads)
-            for (int w = 0; w < kRouterWaves; ++w) running[idx] += wcount[w * E + idx];
-        __syncthreads();
-    }
-    for (int idx = tid; idx < E; idx += kRouterThreads) blockcnt[(size_t)blk * E + idx] = running[idx];
-}
-
 // ---------------------------------------------------------------------------
 // logits_q8_kernel: the logits of a quantized router, one thread per (token, expert).  The reference's order
 // (dot_lanes::<32>, src/quantized.rs:154-177, taken on machines with AVX2, :179-196): lanes[c % 32] += x[c] * f32(q[c])
@@ -595,38 +461,6 @@ __global__ __launch_bounds__(kRouterThreads) void route_fused_kernel(
     }
     __syncthreads();
     router_tail<1, true>(lds_raw, blk, valid, T, E, k, P, lse, expert_of, gate_of, rank_in_block, blockcnt, partial);
-}
-
-// A token block's experts shared out over workgroups: each leaves its logits in P; the last to arrive fetches the others' into
-// its own array and goes on.  Device-scope stores and loads: the workgroups may sit on different XCDs, whose L2s do not see
-// each other's lines; a workgroup's stores are acknowledged before its arrival is counted.
-template <int TB>
-__device__ __forceinline__ bool last_slice(const RouteRowsArgs& a, int from, int to, unsigned char* lds_raw) {
-    float* const prob = reinterpret_cast<float*>(lds_raw);
-    const int E = a.E, ES = E | 1, tid = threadIdx.x;
-    int& last = *reinterpret_cast<int*>(prob + TB * ES);  // (where router_tail will keep the log-sum-exps)
-    const int t0 = blockIdx.x * TB, nt = min(TB, a.T - t0), n = to - from;
-    for (int i = tid; i < nt * n; i += kRouterThreads) {
-        const int t = i / n, e = from + i - t * n;
-        __hip_atomic_store(a.P + (size_t)(t0 + t) * E + e, prob[t * ES + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (tid == 0) {
-        int* const counter = a.arrive + blockIdx.x * kDecodeCombineCounterStride;
-        const int before = atomicAdd(counter, 1);
-        last = before == (int)gridDim.y - 1;
-        if (before == (int)gridDim.y - 1) atomicExch(counter, 0);  // everyone has arrived: ready for the next launch
-    }
-    __syncthreads();
-    if (!last) return false;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    for (int i = tid; i < nt * E; i += kRouterThreads) {
-        const int t = i / E, e = i - t * E;
-        if (e < from || e >= to)
-            prob[t * ES + e] = __hip_atomic_load(a.P + (size_t)t0 * E + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    return true;  // (router_tail begins with a barrier)
 }
 
 // Norm (optional), logits and everything behind them for TB tokens a workgroup (see route_rows_body).
@@ -1133,6 +967,7 @@ struct RowsPlan {
     int EG = 0;
     size_t lds = 0;
     int slice = 0;
+    bool exact = false;  // route_exact_kernel
 };
 // Where the other kernels are faster all the same (blocks of 8 tokens never lose).  Times are forwards of narrow experts,
 // other kernels / this one.
@@ -1149,6 +984,12 @@ static bool rows_lose(int d, int E, int tokens, bool quantized, bool f32) {
     return tokens == 32 && E > 8 && E < 32 && d <= (f32 ? 512 : 256);
 }
 
+static size_t rows_lds(const RouterArgs& a, bool exact, int tokens, int EG) {
+    const int NL = a.wq ? 32 : 8;
+    return exact ? route_exact_lds_bytes(a.E, a.k, a.d, tokens, NL, EG)
+                 : route_rows_lds_bytes(a.E, a.k, a.d, tokens, NL, EG, a.norm_w != nullptr);
+}
+
 static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     RowsPlan p;
     const int unit = a.wq ? 32 : 8;  // whole turns of the column lanes, whole 16-byte pieces
@@ -1156,12 +997,12 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     if ((reinterpret_cast<uintptr_t>(a.x) & 15) || ((size_t)a.d * xsize) % 16 != 0) return p;
     if (reinterpret_cast<uintptr_t>(a.wq ? static_cast<const void*>(a.wq) : a.wr) & 15) return p;
     if (a.norm_w && ((reinterpret_cast<uintptr_t>(a.xn_out) & 15) || a.d % 8 != 0)) return p;
-    const int NL = a.wq ? 32 : 8;
+    p.exact = route_exact_ok(a, xsize == 2);
     int tokens = a.min_tokens;
     while (tokens < kRouterTokens && (a.T + tokens - 1) / tokens > 256) tokens *= 2;
     for (; tokens >= a.min_tokens && !p.tokens; tokens /= 2) {
         int EG = a.E;  // as many experts' rows as fit together, whole pairs, at least 8 (or all of them)
-        auto lds = [&] { return route_rows_lds_bytes(a.E, a.k, a.d, tokens, NL, EG, a.norm_w != nullptr); };
+        auto lds = [&] { return rows_lds(a, p.exact, tokens, EG); };
         while (EG > 8 && lds() > (size_t)kMaxRouterLds) EG = (EG - 1) & ~1;
         if (lds() > (size_t)kMaxRouterLds) continue;
         p.tokens = tokens;
@@ -1173,9 +1014,9 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     // none, for the chain of a second round is as long as the first's: 9000 tokens, d 512, 8 experts 60.0 us a forward in two
     // rounds, 57.0 without; 16 experts 63.2 / 57.1, f32 rows 65.8 / 56.7; d 512, 4 experts, two workgroups a unit 55.5 / 61.0.
     const int blocks = (a.T + p.tokens - 1) / p.tokens;
-    const int together = p.tokens == kRouterTokens && 2 * p.lds <= (size_t)kMaxRouterLds ? 512 : 256;
+    const int together = p.tokens == kRouterTokens ? 256 * std::min(4, (int)((size_t)kMaxRouterLds / p.lds)) : 256;
     if ((long long)a.T * a.E > 256 * 1024 || blocks > together) p.tokens = 0;
-    if (p.tokens > kMinRouterTokens && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
+    if (p.tokens > kMinRouterTokens && !p.exact && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
     // A few tokens by many experts: one workgroup a block would take the experts' rows through its own LDS one group after the
     // other (64 experts of d 1024: 27 us, whatever the tokens).  So the block's experts are shared out, eight to a workgroup
     // or as many as leave at most one round of workgroups; the last to arrive does the rest.  us a forward, one workgroup / shared
@@ -1187,7 +1028,7 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
             if (blocks * ((a.E + slice - 1) / slice) <= 256) {
                 p.slice = slice;
                 p.EG = std::min(p.EG, slice);
-                p.lds = route_rows_lds_bytes(a.E, a.k, a.d, p.tokens, NL, p.EG, a.norm_w != nullptr);
+                p.lds = rows_lds(a, p.exact, p.tokens, p.EG);
             }
     return p;
 }
@@ -1199,6 +1040,7 @@ RouterPlan plan_router(const RouterArgs& a, bool bf16) {
     q.row_experts = p.tokens ? p.EG : 0;
     q.row_lds = p.tokens ? p.lds : 0;
     q.row_slice = p.tokens ? p.slice : 0;
+    q.row_exact = p.tokens && p.exact;
     // where the squares' room costs tokens a workgroup, a second round of workgroups costs more than the norm in a launch of
     // its own (8192 tokens, d 768, squares in LDS: 37.7 us in two rounds, 16.2 + 8 in two launches; a wave a row leaves one
     // round: 29 in one launch, 12.5 + 20 in two)
@@ -1225,7 +1067,7 @@ template <typename XT>
 static hipError_t launch_rows_t(const RouterArgs& a, const RouterPlan& p, hipStream_t s) {
     RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, p.row_experts, a.P, a.lse, a.expert_of, a.gate_of,
                     a.rank_in_block, a.blockcnt, a.partial, static_cast<bf16_t*>(a.rows16), a.norm_w, a.norm_eps, a.xn_out,
-                    p.row_slice, a.arrive};
+                    false, p.row_slice, a.arrive};
     const dim3 grid((a.T + p.block_tokens - 1) / p.block_tokens, p.row_slice ? (a.E + p.row_slice - 1) / p.row_slice : 1);
     auto go = [&](auto kernel) -> hipError_t {
         static std::atomic<unsigned long long> attr_set{0};  // one per kernel: the lambda's body is instantiated for each
@@ -1255,6 +1097,7 @@ static hipError_t launch_rows_t(const RouterArgs& a, const RouterPlan& p, hipStr
 
 template <typename XT>
 static hipError_t launch_router_t(const RouterArgs& a, const RouterPlan& p, hipStream_t s) {
+    if (p.row_exact) return launch_route_exact(a, p, s);
     if (p.row_experts) return launch_rows_t<XT>(a, p, s);
     const int nb = (a.T + kRouterTokens - 1) / kRouterTokens;
     if (const int cols = a.wq ? 0 : fused_cols(a, sizeof(XT))) {

@@ -1275,32 +1275,21 @@ __global__ __launch_bounds__(kSmallThreads, 2) void decode_front_kernel(RouteRow
     if ((int)blockIdx.x < routers) {
         const int k = r.k, ES = E | 1;
         const int t0 = blockIdx.x * kFrontTokens, nt = min(kFrontTokens, T - t0);
-        bool routed = false;
-        if constexpr (sizeof(XT) == 2)
-            if (r.exact) {  // uniform over the launch
-                route_exact_body<kFrontTokens, Q8 ? 32 : 8, NORM>(r, blockIdx.x, 0, r.E, lds);
-                routed = true;
-            }
-        if (!routed) route_rows_body<XT, kFrontTokens, Q8 ? 32 : 8, Q8 ? 2 : 1, 2, NORM>(r, blockIdx.x, 0, r.E, lds);
-        __syncthreads();
         float* const prob = reinterpret_cast<float*>(lds);  // the arrays of router_fixed_bytes
         float* const lsev = prob + kFrontTokens * ES;
-        float* const gates = lsev + kFrontTokens;
-        int* const lexp = reinterpret_cast<int*>(gates + kFrontTokens * k);
-        int G = 1;
-        while (G < E && G < 64) G <<= 1;
-        softmax_topk<1, 1, kFrontTokens>(prob, lsev, gates, lexp, G, t0, nt, ES, r.valid, E, k);
+        int* const lexp = reinterpret_cast<int*>(lsev + kFrontTokens);
+        const RouteOut out{r.P, r.lse, r.expert_of, r.gate_of};
+        if constexpr (sizeof(XT) == 2)
+            if (r.exact) {  // uniform over the launch
+                ExactLogits<kFrontTokens, Q8 ? 32 : 8> logits(r, lds);
+                logits.folded = !route_exact_body<kFrontTokens, Q8 ? 32 : 8, NORM>(r, blockIdx.x, 0, E, true, lds);
+                if (logits.folded) __syncthreads();
+                block_softmax_topk<1, kFrontTokens>(prob, lsev, lexp, t0, nt, r.valid, E, k, out, logits);
+                return;
+            }
+        route_rows_body<XT, kFrontTokens, Q8 ? 32 : 8, Q8 ? 2 : 1, 2, NORM>(r, blockIdx.x, 0, E, lds);
         __syncthreads();
-        const int tid = threadIdx.x;
-        for (int i = tid; i < nt * E; i += kSmallThreads) {
-            const int t = i / E;
-            r.P[(size_t)t0 * E + i] = prob[t * ES + (i - t * E)];
-        }
-        if (tid < nt) r.lse[t0 + tid] = lsev[tid];
-        for (int i = tid; i < nt * k; i += kSmallThreads) {
-            r.expert_of[(size_t)t0 * k + i] = lexp[i];
-            r.gate_of[(size_t)t0 * k + i] = gates[i];
-        }
+        block_softmax_topk<1, kFrontTokens>(prob, lsev, lexp, t0, nt, r.valid, E, k, out, [&](int i, int e) { return prob[i * ES + e]; });
         return;
     }
     // a product workgroup is two teams of four waves, each with a block of 32 features of its own: the reduction is

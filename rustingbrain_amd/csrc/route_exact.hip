@@ -12,11 +12,12 @@ __global__ __launch_bounds__(kRouterThreads, 2) void route_exact_kernel(RouteRow
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int from = blockIdx.y * a.slice, to = a.slice ? min(a.E, from + a.slice) : a.E;  // (no slice: one row of workgroups)
     if (blockIdx.y != 0) a.xn_out = nullptr;                                               // (the first slice writes the rows)
-    route_exact_body<TB, NL, NORM>(a, blockIdx.x, from, to, lds_raw);
-    __syncthreads();
+    ExactLogits<TB, NL> logits(a, lds_raw);
+    logits.folded = !route_exact_body<TB, NL, NORM>(a, blockIdx.x, from, to, a.slice == 0, lds_raw);
+    if (logits.folded) __syncthreads();
     if (a.slice && !last_slice<TB>(a, from, to, lds_raw)) return;
-    router_tail<1, true, TB>(lds_raw, blockIdx.x, a.valid, a.T, a.E, a.k, a.P, a.lse, a.expert_of, a.gate_of, a.rank_in_block,
-                             a.blockcnt, a.partial);
+    router_tail<1, TB>(lds_raw, blockIdx.x, a.valid, a.T, a.E, a.k, RouteOut{a.P, a.lse, a.expert_of, a.gate_of}, a.rank_in_block,
+                       a.blockcnt, a.partial, logits);
 }
 
 hipError_t launch_route_exact(const RouterArgs& a, const RouterPlan& p, hipStream_t s) {

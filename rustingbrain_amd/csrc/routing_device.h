@@ -7,134 +7,148 @@
 namespace rbmoe {
 
 // Dynamic LDS layout of router_kernel (floats / ints, in this order):
-//   prob   [TB][ES]   logits, then exp, then probabilities   (ES = E | 1)
+//   prob   [TB][ES]   logits, then probabilities   (ES = E | 1)
 //   lsev   [TB]       log-sum-exp per token
-//   gates  [TB][k]    selected probabilities, then gates
 //   lexp   [TB][k]    selected expert per local slot (-1 = unrouted)
 //   wcount [waves][E] per-wave match counts of one ranking round
 //   running[E]        slots already ranked per expert
 __host__ __device__ static size_t router_fixed_bytes(int E, int k, int tokens = kRouterTokens) {
     const int ES = E | 1;
-    size_t n = (size_t)tokens * ES + tokens + 2 * (size_t)tokens * k + (size_t)kRouterWaves * E + E;
+    size_t n = (size_t)tokens * ES + tokens + (size_t)tokens * k + (size_t)kRouterWaves * E + E;
     return (n * 4 + 15) & ~(size_t)15;
 }
 
-// softmax, log-sum-exp and the k argmax rounds for the tokens of one wave of a router block (see router_tail).
+// The arrays that softmax and top-k leave for a block's tokens: in memory (of the whole call), and in LDS for what follows.
+struct RouteOut {
+    float* P;
+    float* lse;
+    int* expert_of;
+    float* gate_of;
+};
+
+template <int I>
+__device__ __forceinline__ float from_row_lane(float v) {  // lane I of each row of 16
+    return __uint_as_float(lanes_from<0x150 + I>(__float_as_uint(v)));
+}
+// ((sum + v_FROM) + ...) + v_(TO - 1), v_i of lane i of the row, in every lane of the row
+template <int FROM, int TO>
+__device__ __forceinline__ float add_row_lanes(float sum, float v) {
+    if constexpr (FROM == TO) return sum;
+    else return add_row_lanes<FROM + 1, TO>(__fadd_rn(sum, from_row_lane<FROM>(v)), v);
+}
+
+// softmax, log-sum-exp and the k argmax rounds for the tokens of one wave of a router block (see router_tail), G lanes a
+// token (16, 32 or 64: the least that E fits; lane j owns the experts j, j + G, ...).  `logit(token, expert)` gives the logits; probabilities, lse,
+// experts and gates go to memory from the lanes that have them, and to `prob`, `lsev` and `lexp` for the ranks and losses.
 // Everything order-sensitive keeps the reference's order: the maximum ignores NaN (f32::max), exp(v - max) is
 // summed one expert after the other in index order, the k argmax rounds prefer the lower index on equal
 // probabilities, and the gates are summed in rank order.
-// The sum: lane l of a group holds ((ex_0 + ex_1) + ... ) + ex_l after l steps of "take the lane below's sum,
-// add your own value" (a shift of the whole wave by one lane inside the add; a group's first lane starts from the sum
-// carried over from the experts of the slices before) - the reference's chain, one rounded add per expert, with
-// no trip through LDS; lanes past the last expert add zeros.  What a group's first lane takes in from the group below
-// follows one lane behind and is overtaken by nobody: the last lane's sum after G - 1 steps is the chain's.  An argmax round is two reductions of 32 bits: the
-// greatest probability bits (probabilities are never negative, so the bits order like the values), then the
-// lowest expert index among the lanes that hold them.
+// The sum: a row of 16 lanes adds its lanes' exponentials one after the other, each handed to the whole row by the
+// lane-permuting operand of the addition itself (row_newbcast); the next row goes on from there (lanes past the last expert
+// add zeros).  An argmax round is a reduction of 32 bits - the greatest probability bits (probabilities are never negative, so the
+// bits order like the values) - and a ballot for the lowest lane that holds them; a lane remembers the round that took it.
 // NQ = turns a wave needs for its tokens (64 / G tokens a turn); the NQ turns share no data and run interleaved.
-template <int MAXJ, int NQ, int TB>
-__device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __restrict__ lsev,
-                                             float* __restrict__ gates, int* __restrict__ lexp, int G, int t0, int nt,
-                                             int ES, const uint8_t* __restrict__ valid, int E, int k) {
+// A dependent chain from end to end.  G is a compile-time constant: with one of run time every step of a reduction was a branch,
+// and with the sums shifted from lane to lane, gates divided in LDS and the results copied out behind a barrier the phase took
+// 1.9 us for 8 experts and 2.2 for 16; now 1.0 and 1.1.  us a call, before / after: one row of the default model 12.8 / 12.2,
+// 203 rows by 16 experts 47.6 / 46.9, 2048 rows of the default model 35.8 / 34.7, 8192 rows skewed 153.3 / 150.3.
+template <int MAXJ, int NQ, int TB, int G, typename LOGIT>
+__device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __restrict__ lsev, int* __restrict__ lexp, int t0,
+                                             int nt, int ES, const uint8_t* __restrict__ valid, int E, int k, const RouteOut& out,
+                                             LOGIT&& logit) {
     constexpr int TW = TB < kRouterWaves ? 1 : TB / kRouterWaves;  // tokens of a wave
     const int lane_ = threadIdx.x & 63, wave_ = threadIdx.x >> 6;
     const int lig = lane_ & (G - 1);          // lane in group
     const int gbase = lane_ & ~(G - 1);       // first lane of the group
-    const int tpw = 64 / G;                   // tokens a wave handles in one turn
-    const unsigned long long gmask = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << gbase;
+    constexpr int tpw = 64 / G;               // tokens a wave handles in one turn
+    const unsigned long long gmask = (G == 64 ? ~0ull : ((1ull << (G & 63)) - 1ull)) << gbase;
+    const unsigned long long below = gmask & ((1ull << lane_) - 1ull);  // the group's lower lanes
     const float neg_inf = __uint_as_float(0xff800000u);
     int tok[NQ];
     bool live[NQ], ok[NQ];
-    float* row[NQ];
-    float pv[NQ][MAXJ], mx[NQ], sum[NQ], total[NQ];
-    unsigned taken_bits[NQ];  // bit j: expert lig + G j is taken
-    uint8_t in_use[NQ];       // (asked for here, looked at behind the softmax)
+    float pv[NQ][MAXJ], mx[NQ], sum[NQ], total[NQ], lse[NQ];
+    int taken[NQ][MAXJ];  // the round that took expert lig + G j, or -1
+    uint8_t in_use[NQ];   // (asked for here, looked at behind the softmax)
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         tok[q] = wave_ * TW + q * tpw + lane_ / G;  // token of this group in turn q
         live[q] = tok[q] < nt && tok[q] < (wave_ + 1) * TW && q * tpw < TW;
         in_use[q] = valid != nullptr ? valid[t0 + (live[q] ? tok[q] : 0)] : 1;
-        row[q] = prob + (live[q] ? tok[q] : 0) * ES;
         mx[q] = neg_inf;
 #pragma unroll
         for (int j = 0; j < MAXJ; ++j) {
             const int e = lig + G * j;
-            pv[q][j] = (live[q] && e < E) ? row[q][e] : neg_inf;
+            pv[q][j] = (live[q] && e < E) ? logit(tok[q], e) : neg_inf;
             const float vv = (pv[q][j] == pv[q][j]) ? pv[q][j] : neg_inf;  // a NaN never becomes the maximum
             mx[q] = vv > mx[q] ? vv : mx[q];
+            taken[q][j] = -1;
         }
     }
 #pragma unroll
     for (int q = 0; q < NQ; ++q) mx[q] = group_fmax(mx[q], G);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
+        sum[q] = 0.0f;
 #pragma unroll
         for (int j = 0; j < MAXJ; ++j) {
             const int e = lig + G * j;
             // lanes without an expert carry +0 through the sums below
-            pv[q][j] = (live[q] && e < E) ? rb_expf(__fadd_rn(pv[q][j], -mx[q])) : 0.0f;
+            const float ex = rb_expf(__fadd_rn(pv[q][j], -mx[q]));
+            pv[q][j] = (live[q] && e < E) ? ex : 0.0f;
         }
     }
-    // the sums: one chain of adds per token in index order, slice after slice
-    {
-        float carry[NQ];
+    // the sums: one chain of adds per token in index order, row after row, slice after slice
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) carry[q] = 0.0f;
+    for (int j = 0; j < MAXJ; ++j) {
+        if (MAXJ > 1 && G * j >= E) break;  // uniform
 #pragma unroll
-        for (int j = 0; j < MAXJ; ++j) {
-            if (G * j >= E) break;  // uniform
-            float acc[NQ];
+        for (int r = 0; r < G / 16; ++r) {
+            if (r > 0 && G * j + 16 * r >= E) break;  // uniform
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) acc[q] = __fadd_rn(carry[q], pv[q][j]);  // in a group's first lane: 0 + ex_0 = ex_0 in the first slice
-            for (int st = 1; st < G; ++st) {
+            for (int q = 0; q < NQ; ++q) sum[q] = add_row_lanes<0, 8>(sum[q], pv[q][j]);
+            if (G * j + 16 * r + 8 < E)
 #pragma unroll
-                for (int q = 0; q < NQ; ++q)
-                    acc[q] = __fadd_rn(__uint_as_float(lanes_from<0x138>(__float_as_uint(acc[q]))), pv[q][j]);  // wave_shr:1
-            }
+                for (int q = 0; q < NQ; ++q) sum[q] = add_row_lanes<8, 16>(sum[q], pv[q][j]);
+            if constexpr (G > 16)
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) carry[q] = __shfl(acc[q], gbase + G - 1);
+                for (int q = 0; q < NQ; ++q) {  // row r's, to the whole group
+                    const uint32_t lo = __builtin_amdgcn_readlane(__float_as_uint(sum[q]), 16 * r);
+                    const uint32_t hi = G == 64 ? lo : __builtin_amdgcn_readlane(__float_as_uint(sum[q]), 32 + 16 * r);
+                    sum[q] = __uint_as_float(G == 32 && (lane_ & 32) ? hi : lo);
+                }
         }
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) sum[q] = carry[q];
     }
+    bool any_nan = false;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        if (live[q] && lig == 0) lsev[tok[q]] = __fadd_rn(mx[q], rb_logf(sum[q]));
+        lse[q] = __fadd_rn(mx[q], rb_logf(sum[q]));
 #pragma unroll
         for (int j = 0; j < MAXJ; ++j) {
-            const int e = lig + G * j;
-            if (live[q] && e < E) {
-                if (sum[q] > 0.0f) pv[q][j] = __fdiv_rn(pv[q][j], sum[q]);
-                row[q][e] = pv[q][j];
-            }
+            const float share = __fdiv_rn(pv[q][j], sum[q]);
+            pv[q][j] = sum[q] > 0.0f ? share : pv[q][j];
+            any_nan = any_nan || pv[q][j] != pv[q][j];
         }
         ok[q] = live[q] && in_use[q] != 0;
-        taken_bits[q] = 0;
         total[q] = 0.0f;
     }
     // ---- k rounds of argmax over the experts not yet taken ----
     // Without a NaN anywhere in the wave (with one expert a lane): the greatest probability bits among the untaken, then the
     // lowest of the lanes that hold them.
-    bool any_nan = false;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) any_nan = any_nan || pv[q][0] != pv[q][0];
     if (MAXJ == 1 && __ballot(any_nan) == 0ull) {  // uniform over the wave
-        bool open[NQ];  // this lane has an expert and it is not taken
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) open[q] = live[q] && lig < E;
         for (int r = 0; r < k; ++r) {
             uint32_t best[NQ];
-#pragma unroll
-            for (int q = 0; q < NQ; ++q) best[q] = group_umax(open[q] ? __float_as_uint(pv[q][0]) : 0u, G);
+            bool open[NQ];  // this lane has an expert and it is not taken
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-                const unsigned long long holders = __ballot(open[q] && __float_as_uint(pv[q][0]) == best[q]) & gmask;
-                const bool mine = holders != 0ull && (holders & ((1ull << lane_) - 1ull)) == 0ull && ((holders >> lane_) & 1ull);
-                open[q] = open[q] && !mine;
+                open[q] = live[q] && lig < E && taken[q][0] < 0;
+                best[q] = group_umax(open[q] ? __float_as_uint(pv[q][0]) : 0u, G);
+            }
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const bool holds = open[q] && __float_as_uint(pv[q][0]) == best[q];
+                const unsigned long long holders = __ballot(holds);
+                taken[q][0] = holds && (holders & below) == 0ull ? r : taken[q][0];
                 total[q] = __fadd_rn(total[q], __uint_as_float(best[q]));
-                if (mine) {
-                    lexp[tok[q] * k + r] = ok[q] ? lig : -1;
-                    gates[tok[q] * k + r] = ok[q] ? __uint_as_float(best[q]) : 0.0f;
-                }
             }
         }
     } else
@@ -150,7 +164,7 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
 #pragma unroll
             for (int j = MAXJ - 1; j >= 0; --j) {
                 const int e = lig + G * j;
-                const unsigned long long m = __ballot(e < E && !((taken_bits[q] >> j) & 1u)) & gmask;
+                const unsigned long long m = __ballot(e < E && taken[q][j] < 0) & gmask;
                 if (m != 0ull) first[q] = (__ffsll((long long)m) - 1 - gbase) + G * j;
             }
             // best candidate of this lane: not taken, not NaN; greater probability, then lower index
@@ -160,7 +174,7 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
 #pragma unroll
             for (int j = 0; j < MAXJ; ++j) {
                 const int e = lig + G * j;
-                if (live[q] && e < E && !((taken_bits[q] >> j) & 1u) && pv[q][j] == pv[q][j]) {
+                if (live[q] && e < E && taken[q][j] < 0 && pv[q][j] == pv[q][j]) {
                     const uint32_t bits = __float_as_uint(pv[q][j]);
                     if (!has[q] || bits > lbits[q]) {  // slices in increasing index order: a tie keeps the lower index
                         lbits[q] = bits;
@@ -191,7 +205,7 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
             for (int j = 0; j < MAXJ; ++j)
                 if (lig + G * j == best) {
                     mine = pv[q][j];
-                    taken_bits[q] |= 1u << j;
+                    taken[q][j] = r;
                 }
             // the winner's probability is the greatest bits themselves; only a NaN first expert has to be fetched
             float bestv = __uint_as_float(mbits[q]);
@@ -200,18 +214,42 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
                 if (use_first) bestv = fv;
             }
             total[q] = __fadd_rn(total[q], bestv);
-            if (live[q] && lig == 0) {
-                lexp[tok[q] * k + r] = ok[q] ? best : -1;
-                gates[tok[q] * k + r] = ok[q] ? bestv : 0.0f;
-            }
         }
     }
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
-        if (ok[q] && total[q] > 0.0f)
-            for (int r = lig; r < k; r += G) gates[tok[q] * k + r] = __fdiv_rn(gates[tok[q] * k + r], total[q]);
+    for (int q = 0; q < NQ; ++q) {
+        if (live[q] && lig == 0) {
+            lsev[tok[q]] = lse[q];
+            out.lse[t0 + tok[q]] = lse[q];
+        }
+#pragma unroll
+        for (int j = 0; j < MAXJ; ++j) {
+            const int e = lig + G * j;
+            if (!live[q] || e >= E) continue;
+            prob[tok[q] * ES + e] = pv[q][j];
+            out.P[(size_t)(t0 + tok[q]) * E + e] = pv[q][j];
+            if (taken[q][j] < 0) continue;
+            const int slot = tok[q] * k + taken[q][j];
+            const float gate = total[q] > 0.0f ? __fdiv_rn(pv[q][j], total[q]) : pv[q][j];
+            const int to = ok[q] ? e : -1;
+            lexp[slot] = to;
+            out.expert_of[(size_t)t0 * k + slot] = to;
+            out.gate_of[(size_t)t0 * k + slot] = ok[q] ? gate : 0.0f;
+        }
+    }
+}
+
+// ... for the tokens of a whole block of TB, MAXJ = experts a lane may own: 1 when E <= 64
+template <int MAXJ, int TB, typename LOGIT>
+__device__ __forceinline__ void block_softmax_topk(float* prob, float* lsev, int* lexp, int t0, int nt, const uint8_t* valid, int E,
+                                                   int k, const RouteOut& out, LOGIT&& logit) {
+    // a wave's tokens (four of 32): all at once with 16 lanes per token, in more turns with 32 or 64 - the
+    // turns are worked on side by side (one instruction stream), because each is a chain of dependent steps
+    constexpr int TW = TB < kRouterWaves ? 1 : TB / kRouterWaves;
+    const int ES = E | 1;
+    if (MAXJ == 1 && E <= 16) softmax_topk<1, (TW + 3) / 4, TB, 16>(prob, lsev, lexp, t0, nt, ES, valid, E, k, out, logit);
+    else if (MAXJ == 1 && E <= 32) softmax_topk<1, (TW + 1) / 2, TB, 32>(prob, lsev, lexp, t0, nt, ES, valid, E, k, out, logit);
+    else softmax_topk<MAXJ, TW, TB, 64>(prob, lsev, lexp, t0, nt, ES, valid, E, k, out, logit);
 }
 
 // ---------------------------------------------------------------------------
@@ -588,9 +626,10 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
 // a thread a logit.
 // A workgroup whose rows hold an element out of RowRange takes the same sums one multiply and one add at a time.
 // Bound by the length of a workgroup's chain, not by work: 203 tokens, d 768, 16 experts, behind a norm, from the kernel's start:
-// normed rows laid down at 2.6 us, every wave's rows and weights at 3.8, sums 5.2, folded 5.8, softmax and top-k 7.7, end 8.8
-// (route_rows_body 10.1); 8192 tokens without a norm 4.0, 6.4, 7.4, 9.2, 10.4 (11.7).  us a call, route_rows_body / this: the two
-// 48.4 / 47.6 and 157.3 / 153.3, 4096 tokens by 8 experts (int8) 91.3 / 89.8, 2048 of d 512 behind a norm 36.5 / 35.8.
+// normed rows laid down at 2.6 us, every wave's rows and weights at 3.7, sums 5.2, met 5.6, softmax and top-k 6.8, end 7.6; 8192
+// tokens without a norm 3.2, 3.7, 6.0, 6.7, 7.9, 8.7 (route_rows_body, with the same tail: 10.1 less the tail's 1.2; 11.7).  us a
+// call, route_rows_body / this: the two 48.4 / 47.6 and 157.3 / 153.3, 4096 tokens by 8 experts (int8) 91.3 / 89.8, 2048 of d 512
+// behind a norm 36.5 / 35.8.
 // ---------------------------------------------------------------------------
 // Elements of bf16 rows: nothing but zeros and magnitudes from 2^-72 to below 2^80.  Two at a time, as the bits lie in memory.
 struct RowRange {
@@ -623,8 +662,21 @@ __host__ __device__ static size_t route_exact_lds_bytes(int E, int k, int d, int
            (size_t)(TB + EG) * exact_row_bytes(d, NL);
 }
 
+// The column lanes' sums of one token and expert, folded left to right; `part`: lane 0's.
+template <int TB, int NL>
+__device__ __forceinline__ float fold_lanes(const float* part) {
+    float v[NL], y = 0.0f;
+#pragma unroll
+    for (int l = 0; l < NL; ++l) v[l] = part[l * TB * exact_round(TB, NL)];
+#pragma unroll
+    for (int l = 0; l < NL; ++l) y = __fadd_rn(y, v[l]);
+    return __fadd_rn(y, 0.0f);  // the reference adds its (empty) scalar rest: sum + 0
+}
+
+// With `fold_later` and one round of experts the sums are left where they meet (behind a barrier), for ExactLogits, and the result is
+// true; otherwise the logits lie in `prob` and the caller meets at a barrier before it reads them.
 template <int TB, int NL, bool NORM>
-__device__ __forceinline__ void route_exact_body(const RouteRowsArgs& a, int blk, int e_from, int e_to,
+__device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk, int e_from, int e_to, bool fold_later,
                                                  unsigned char* __restrict__ lds_raw) {
     constexpr int NT = kRouterThreads, LW = NL / 8, MB = (TB + 15) / 16, RE = exact_round(TB, NL);
     const int T = a.T, d = a.d, E = a.E, k = a.k, EG = a.EG, ES = E | 1;
@@ -889,80 +941,67 @@ __device__ __forceinline__ void route_exact_body(const RouteRowsArgs& a, int blk
                 }
             }
             __syncthreads();
+            if (fold_later && e_to - e_from <= min(RE, EG)) return true;
             for (int i = tid; i < nt * RE; i += NT) {
                 const int t = i / RE, e = e0 + r0 + i % RE;
                 if (i % RE >= ne) continue;
-                float v[NL], y = 0.0f;
-#pragma unroll
-                for (int l = 0; l < NL; ++l) v[l] = part[l * TB * RE + i];
-#pragma unroll
-                for (int l = 0; l < NL; ++l) y = __fadd_rn(y, v[l]);
-                y = __fadd_rn(y, 0.0f);  // the reference adds its (empty) scalar rest: sum + 0
+                float y = fold_lanes<TB, NL>(part + i);
                 if constexpr (NL == 32) y = __fmul_rn(y, a.wscale[e]);
                 if (a.bias) y = __fadd_rn(y, a.bias[e]);
                 prob[t * ES + e] = y;
             }
         }
     }
+    return false;
 }
 
+// The logits behind route_exact_body, for a wave whose lane 16 g + e asks for expert e (or, folded already, any): what is added to or
+// multiplied with the sums is asked for when the object is made.
+template <int TB, int NL>
+struct ExactLogits {
+    const float *part, *prob;
+    int ES;
+    float scale = 1.0f, bias = 0.0f;
+    bool has_bias, folded = false;
+    __device__ __forceinline__ ExactLogits(const RouteRowsArgs& a, unsigned char* lds_raw) {
+        prob = reinterpret_cast<const float*>(lds_raw);
+        part = reinterpret_cast<const float*>(lds_raw + router_fixed_bytes(a.E, a.k, TB)) + kRouterWaves;
+        ES = a.E | 1;
+        const int e = min((int)threadIdx.x & 15, a.E - 1);
+        has_bias = a.bias != nullptr;
+        if (has_bias) bias = a.bias[e];
+        if constexpr (NL == 32) scale = a.wscale[e];
+    }
+    __device__ __forceinline__ float operator()(int t, int e) const {
+        if (folded) return prob[t * ES + e];  // uniform over the workgroup
+        float y = fold_lanes<TB, NL>(part + t * exact_round(TB, NL) + e);
+        if constexpr (NL == 32) y = __fmul_rn(y, scale);
+        return has_bias ? __fadd_rn(y, bias) : y;
+    }
+};
+
 // router_tail: everything behind the logits for the TB tokens of router block `blk` - softmax, log-sum-exp, top-k,
-// gates, ranks, block histogram, partial sums of the losses.  LOADED = false: the logits are read from P;
-// true: the caller has put them into the `prob` array of `lds_raw` (row pitch E | 1) and met at a barrier.
+// gates, ranks, block histogram, partial sums of the losses.  `logit(token, expert)` may be read already.
 // MAXJ = experts a lane may own: 1 when E <= 64 (a lane owns one expert), kMaxExperts / 64 otherwise.
-template <int MAXJ, bool LOADED, int TB = kRouterTokens>
-__device__ __forceinline__ void router_tail(
-    unsigned char* __restrict__ lds_raw, int blk, const uint8_t* __restrict__ valid, int T, int E, int k,
-    float* __restrict__ P, float* __restrict__ lse, int* __restrict__ expert_of, float* __restrict__ gate_of,
-    int* __restrict__ rank_in_block, int* __restrict__ blockcnt, float* __restrict__ partial) {
+template <int MAXJ, int TB, typename LOGIT>
+__device__ __forceinline__ void router_tail(unsigned char* __restrict__ lds_raw, int blk, const uint8_t* __restrict__ valid, int T,
+                                            int E, int k, const RouteOut& out, int* __restrict__ rank_in_block,
+                                            int* __restrict__ blockcnt, float* __restrict__ partial, LOGIT&& logit) {
     const int ES = E | 1;
     float* prob = reinterpret_cast<float*>(lds_raw);
     float* lsev = prob + TB * ES;
-    float* gates = lsev + TB;
-    int* lexp = reinterpret_cast<int*>(gates + TB * k);
+    int* lexp = reinterpret_cast<int*>(lsev + TB);
     int* wcount = lexp + TB * k;
     int* running = wcount + kRouterWaves * E;
 
     const int tid = threadIdx.x;
     const int t0 = blk * TB;
     const int nt = min(TB, T - t0);
-
-    // ---- logits were written to P by logits_kernel ------------------------------
-    if constexpr (!LOADED) {
-        for (int idx = tid; idx < nt * E; idx += kRouterThreads) {
-            const int i = idx / E;
-            prob[i * ES + (idx - i * E)] = P[(size_t)t0 * E + idx];
-        }
-    }
     for (int idx = tid; idx < E; idx += kRouterThreads) running[idx] = 0;
+    block_softmax_topk<MAXJ, TB>(prob, lsev, lexp, t0, nt, valid, E, k, out, logit);
     __syncthreads();
 
-    // ---- softmax + top-k: G lanes per token, lane j of a group owns experts j, j + G, ... ----
-    {
-        int G = 1;
-        while (G < E && G < 64) G <<= 1;
-        // a wave's tokens (four of 32): all at once with up to 16 lanes per token, in more turns with 32 or 64 - the
-        // turns are worked on side by side (one instruction stream), because each is a chain of dependent steps
-        constexpr int TW = TB / kRouterWaves;
-        if (G == 64) softmax_topk<MAXJ, TW, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
-        else if (G == 32) softmax_topk<MAXJ, (TW + 1) / 2, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
-        else softmax_topk<MAXJ, (TW + 3) / 4, TB>(prob, lsev, gates, lexp, G, t0, nt, ES, valid, E, k);
-    }
-    __syncthreads();
-
-    // ---- write probabilities, lse, assignments (coalesced) ----------------
-    for (int idx = tid; idx < nt * E; idx += kRouterThreads) {
-        const int i = idx / E;
-        const int e = idx - i * E;
-        P[(size_t)t0 * E + idx] = prob[i * ES + e];
-    }
-    if (tid < nt) lse[t0 + tid] = lsev[tid];
     const int nls = nt * k;
-    for (int ls = tid; ls < nls; ls += kRouterThreads) {
-        expert_of[(size_t)t0 * k + ls] = lexp[ls];
-        gate_of[(size_t)t0 * k + ls] = gates[ls];
-    }
-
     // ---- partial sums for the auxiliary losses (fixed order): the waves behind the first, which ranks the slots
     // at the same time -----------------------------------------------------------
     const bool one_wave_ranks = nls <= 64;
@@ -1069,7 +1108,8 @@ __device__ __forceinline__ bool last_slice(const RouteRowsArgs& a, int from, int
         if (e < from || e >= to)
             prob[t * ES + e] = __hip_atomic_load(a.P + (size_t)t0 * E + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    return true;  // (router_tail begins with a barrier)
+    __syncthreads();
+    return true;
 }
 
 hipError_t launch_route_exact(const RouterArgs& a, const RouterPlan& p, hipStream_t s);  // (route_exact.hip)

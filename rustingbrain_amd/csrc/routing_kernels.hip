@@ -460,7 +460,8 @@ __global__ __launch_bounds__(kRouterThreads) void route_fused_kernel(
         }
     }
     __syncthreads();
-    router_tail<1, true>(lds_raw, blk, valid, T, E, k, P, lse, expert_of, gate_of, rank_in_block, blockcnt, partial);
+    router_tail<1, kRouterTokens>(lds_raw, blk, valid, T, E, k, RouteOut{P, lse, expert_of, gate_of}, rank_in_block, blockcnt, partial,
+                                  [&](int i, int e) { return prob[i * ES + e]; });
 }
 
 // Norm (optional), logits and everything behind them for TB tokens a workgroup (see route_rows_body).
@@ -478,19 +479,22 @@ __global__ __launch_bounds__(kRouterThreads, 2) void route_rows_kernel(RouteRows
         __syncthreads();
         if (!last_slice<TB>(a, from, to, lds_raw)) return;
     }
-    router_tail<1, true, TB>(lds_raw, blockIdx.x, a.valid, a.T, a.E, a.k, a.P, a.lse, a.expert_of, a.gate_of, a.rank_in_block,
-                             a.blockcnt, a.partial);
+    const float* const prob = reinterpret_cast<const float*>(lds_raw);
+    const int ES = a.E | 1;
+    router_tail<1, TB>(lds_raw, blockIdx.x, a.valid, a.T, a.E, a.k, RouteOut{a.P, a.lse, a.expert_of, a.gate_of}, a.rank_in_block,
+                       a.blockcnt, a.partial, [&](int i, int e) { return prob[i * ES + e]; });
 }
 
 template <typename XT, int MAXJ>
 __global__ __launch_bounds__(kRouterThreads) void router_kernel(
     const XT* __restrict__ x, const float* __restrict__ wr, const float* __restrict__ bias,
-    const uint8_t* __restrict__ valid, int T, int d, int E, int k, float* __restrict__ P,
+    const uint8_t* __restrict__ valid, int T, int d, int E, int k, float* P,
     float* __restrict__ lse, int* __restrict__ expert_of, float* __restrict__ gate_of,
     int* __restrict__ rank_in_block, int* __restrict__ blockcnt, float* __restrict__ partial) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    router_tail<MAXJ, false>(lds_raw, blockIdx.x, valid, T, E, k, P, lse, expert_of, gate_of, rank_in_block, blockcnt,
-                             partial);
+    // (the logits are where the probabilities go: a lane has read its own before it writes them)
+    router_tail<MAXJ, kRouterTokens>(lds_raw, blockIdx.x, valid, T, E, k, RouteOut{P, lse, expert_of, gate_of}, rank_in_block, blockcnt,
+                                     partial, [&](int i, int e) { return P[((size_t)blockIdx.x * kRouterTokens + i) * E + e]; });
 }
 
 // ---------------------------------------------------------------------------

@@ -1445,7 +1445,8 @@ static size_t front_lds_bytes(const RouterArgs& a, bool bf16, int* EG) {
         return exact ? route_exact_lds_bytes(E, k, d, kFrontTokens, q8 ? 32 : 8, eg)
                      : route_rows_lds_bytes(E, k, d, kFrontTokens, q8 ? 32 : 8, eg, norm);
     };
-    while (eg > 8 && route() > (size_t)kMaxRouterLds) eg = (eg - 1) & ~1;
+    while (eg > (exact ? 16 : 8) && route() > (size_t)kMaxRouterLds)
+        eg = exact ? exact_fewer(eg, kFrontTokens, q8 ? 32 : 8) : (eg - 1) & ~1;
     if (route() > (size_t)kMaxRouterLds || products > (size_t)kMaxRouterLds) return 0;
     *EG = eg;
     return products > route() ? products : route();

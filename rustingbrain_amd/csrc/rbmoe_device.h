@@ -273,7 +273,7 @@ struct Vec16<bf16_t> {
 
 // Reductions over the G neighbouring lanes of a group (G a power of two up to 64, the same for the whole wave)
 // without LDS: inside a row of 16 lanes through the lane-permuting operand of the instruction itself (every lane of
-// the row ends with the result), across rows through four scalar reads.
+// the row ends with the result), across rows by handing a row's last lane to the next rows and one or two scalar reads.
 template <int CTRL>
 __device__ __forceinline__ uint32_t lanes_from(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
@@ -284,11 +284,15 @@ __device__ __forceinline__ uint32_t group_reduce(uint32_t v, int G, Op op) {
     if (G >= 4) v = op(v, lanes_from<0x4E>(v));   // quad_perm [2,3,0,1]
     if (G >= 8) v = op(v, lanes_from<0x141>(v));  // row_half_mirror
     if (G >= 16) v = op(v, lanes_from<0x140>(v)); // row_mirror
-    if (G >= 32) {
-        const uint32_t r0 = __builtin_amdgcn_readlane(v, 0), r1 = __builtin_amdgcn_readlane(v, 16);
-        const uint32_t r2 = __builtin_amdgcn_readlane(v, 32), r3 = __builtin_amdgcn_readlane(v, 48);
-        const uint32_t lo = op(r0, r1), hi = op(r2, r3);
-        v = G == 64 ? op(lo, hi) : ((threadIdx.x & 32) ? hi : lo);
+    if (G >= 32) {  // (rows 1 and 3, then rows 2 and 3; the others keep what they have)
+        v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+        if (G == 64) {
+            v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+            v = __builtin_amdgcn_readlane(v, 63);
+        } else {
+            const uint32_t lo = __builtin_amdgcn_readlane(v, 31), hi = __builtin_amdgcn_readlane(v, 63);
+            v = (threadIdx.x & 32) ? hi : lo;
+        }
     }
     return v;
 }

@@ -101,9 +101,7 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
 #pragma unroll
     for (int j = 0; j < MAXJ; ++j) {
         if (MAXJ > 1 && G * j >= E) break;  // uniform
-#pragma unroll
-        for (int r = 0; r < G / 16; ++r) {
-            if (r > 0 && G * j + 16 * r >= E) break;  // uniform
+        auto row = [&](int r) {
 #pragma unroll
             for (int q = 0; q < NQ; ++q) sum[q] = add_row_lanes<0, 8>(sum[q], pv[q][j]);
             if (G * j + 16 * r + 8 < E)
@@ -115,8 +113,12 @@ __device__ __forceinline__ void softmax_topk(float* __restrict__ prob, float* __
                     const uint32_t lo = __builtin_amdgcn_readlane(__float_as_uint(sum[q]), 16 * r);
                     const uint32_t hi = G == 64 ? lo : __builtin_amdgcn_readlane(__float_as_uint(sum[q]), 32 + 16 * r);
                     sum[q] = __uint_as_float(G == 32 && (lane_ & 32) ? hi : lo);
+                    asm("" : "+v"(sum[q]));  // (known to be the same in every lane it would be taken through scalar registers)
                 }
-        }
+        };
+        const int rows = min(G / 16, (E - G * j + 15) / 16);
+#pragma unroll 1
+        for (int r = 0; r < rows; ++r) row(r);
     }
     bool any_nan = false;
 #pragma unroll
@@ -657,6 +659,8 @@ __host__ __device__ constexpr int exact_round(int TB, int NL) { return TB * NL >
 __host__ static inline bool route_exact_ok(const RouterArgs& a, bool bf16) {
     return bf16 && a.exact && a.rows16 == nullptr && (!a.norm_w || wave_norms(a.d));
 }
+// The next smaller number of experts whose rows may lie in LDS together: whole rounds.
+__host__ static inline int exact_fewer(int EG, int TB, int NL) { return (EG - 1) / exact_round(TB, NL) * exact_round(TB, NL); }
 __host__ __device__ static size_t route_exact_lds_bytes(int E, int k, int d, int TB, int NL, int EG) {
     return router_fixed_bytes(E, k, TB) + 4 * kRouterWaves + (size_t)NL * TB * exact_round(TB, NL) * 4 +
            (size_t)(TB + EG) * exact_row_bytes(d, NL);
@@ -742,7 +746,7 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
         }
         return w;
     };
-    auto put_weights = [&](int n, int i, const Weights& w) {
+    auto put_weights = [&](int n, int i, unsigned char* to, const Weights& w) {
         if (i >= n) return;
         const Task t = task(i);
         uint4 p[4];
@@ -759,10 +763,10 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
             }
             if (t.step + 4 * u >= S) p[u] = zero;
         }
-        turn(ws + t.row * pitch + t.at, p);
+        turn(to + t.row * pitch + t.at, p);
     };
-    auto rest_of_router = [&](int e0, int n, int from) {
-        for (int i = from + tid; i < n; i += NT) put_weights(n, i, weights_of(e0, n, i));
+    auto rest_of_router = [&](int e0, int n, int from, unsigned char* to) {
+        for (int i = from + tid; i < n; i += NT) put_weights(n, i, to, weights_of(e0, n, i));
     };
     const int nw0 = min(EG, e_to - e_from) * per_row;
     RowRange range;
@@ -808,7 +812,7 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
                     for (int i = 0; i < H / 4; ++i) *reinterpret_cast<uint2*>(to + 4 * i) = make_uint2(o[2 * i], o[2 * i + 1]);
                 }
             }
-            put_weights(nw0, tid, w);
+            put_weights(nw0, tid, ws, w);
         });
         // (a row's steps past its end)
         if (S < Sp)
@@ -848,9 +852,9 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
         put_rows(tid, r0);
         put_rows(tid + NT, r1);
         for (int i = tid + 2 * NT; i < nx; i += NT) put_rows(i, rows_of(i));
-        put_weights(nw0, tid, w);
+        put_weights(nw0, tid, ws, w);
     }
-    rest_of_router(e_from, nw0, NT);
+    rest_of_router(e_from, nw0, NT, ws);
     {
         const bool any = __ballot(range.left()) != 0ull;
         if (lane == 0) left[wave] = any;
@@ -860,17 +864,25 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
 #pragma unroll
     for (int w = 0; w < kRouterWaves; ++w) exact = exact && left[w] == 0;
     // ---- the column lanes' sums, 16 (RE) experts at a time ----------------------------
+    // Experts past the EG whose rows lie in LDS follow round by round, into the place of the round that is done with, asked for in
+    // front of its products.
     const int blocks = (S + 15) / 16, last = (S - 16 * (blocks - 1) + 3) / 4;  // products of the last block of steps
-    for (int e0 = e_from; e0 < e_to; e0 += EG) {
-        const int ng = min(EG, e_to - e0);
-        if (e0 > e_from) {  // (every wave is behind the barrier in front of the last round's fold)
-            rest_of_router(e0, ng * per_row, 0);
-            __syncthreads();
+    const int n = e_to - e_from;
+    int room = 0;  // where the round's router rows lie
+    for (int r0 = 0; r0 < n; r0 += RE) {
+        const int ne = min(RE, n - r0), next = min(RE, n - r0 - EG);  // (next: experts that follow into its place)
+        if (r0 > 0) __syncthreads();  // the round before has been folded, this one's rows are there
+        Weights follow;
+        if (next > 0) follow = weights_of(e_from + r0 + EG, next * per_row, tid);
+        float scale = 1.0f, bias = 0.0f;  // of the expert whose logits this thread folds
+        {
+            const int e = min(e_from + r0 + tid % RE, e_to - 1);
+            if constexpr (NL == 32) scale = a.wscale[e];
+            if (a.bias) bias = a.bias[e];
         }
-        for (int r0 = 0; r0 < ng; r0 += RE) {
-            const int ne = min(RE, ng - r0);
-            if (r0 > 0 || e0 > e_from) __syncthreads();  // the round before has been folded
-            const unsigned char* const wr = ws + r0 * pitch;
+        __builtin_amdgcn_sched_barrier(0);
+        unsigned char* const wr = ws + room * pitch;
+        {
             if (exact) {  // uniform over the workgroup
                 const unsigned char* x[MB];
                 const unsigned at = (unsigned)(wave * LW * Sp * 2 + 8 * (lane >> 4));
@@ -941,13 +953,19 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
                 }
             }
             __syncthreads();
-            if (fold_later && e_to - e_from <= min(RE, EG)) return true;
+            if (fold_later && n <= RE) return true;
+            if (next > 0) {
+                put_weights(next * per_row, tid, wr, follow);
+                rest_of_router(e_from + r0 + EG, next * per_row, NT, wr);
+            }
+            room = room + RE < EG ? room + RE : 0;
+            static_assert(NT % RE == 0, "a thread folds one expert");
             for (int i = tid; i < nt * RE; i += NT) {
-                const int t = i / RE, e = e0 + r0 + i % RE;
+                const int t = i / RE, e = e_from + r0 + i % RE;
                 if (i % RE >= ne) continue;
                 float y = fold_lanes<TB, NL>(part + i);
-                if constexpr (NL == 32) y = __fmul_rn(y, a.wscale[e]);
-                if (a.bias) y = __fadd_rn(y, a.bias[e]);
+                if constexpr (NL == 32) y = __fmul_rn(y, scale);
+                if (a.bias) y = __fadd_rn(y, bias);
                 prob[t * ES + e] = y;
             }
         }
@@ -997,74 +1015,87 @@ __device__ __forceinline__ void router_tail(unsigned char* __restrict__ lds_raw,
     const int tid = threadIdx.x;
     const int t0 = blk * TB;
     const int nt = min(TB, T - t0);
+    const int nls = nt * k, rank_waves = (nls + 63) >> 6;
     for (int idx = tid; idx < E; idx += kRouterThreads) running[idx] = 0;
+    if (rank_waves < kRouterWaves)
+        for (int idx = tid; idx < rank_waves * E; idx += kRouterThreads) wcount[idx] = 0;
     block_softmax_topk<MAXJ, TB>(prob, lsev, lexp, t0, nt, valid, E, k, out, logit);
     __syncthreads();
 
-    const int nls = nt * k;
-    // ---- partial sums for the auxiliary losses (fixed order): the waves behind the first, which ranks the slots
-    // at the same time -----------------------------------------------------------
-    const bool one_wave_ranks = nls <= 64;
-    const int pfirst = one_wave_ranks ? 64 : 0;  // first thread that takes partial sums
-    for (int e = tid - pfirst; e >= 0 && e <= E; e += kRouterThreads - pfirst) {
-        float s = 0.0f;
-        for (int i0 = 0; i0 < nt; i0 += 8) {
-            float pvv[8];
-            int okv[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int i = min(i0 + u, nt - 1);
-                okv[u] = lexp[i * k];
-                pvv[u] = e < E ? prob[i * ES + e] : lsev[i] * lsev[i];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (i0 + u < nt && okv[u] >= 0) s += pvv[u];
-        }
-        partial[(size_t)blk * (E + 1) + e] = s;
-    }
-
-    // ---- rank of every local slot among earlier slots of the same expert --
     const int lane = tid & 63;
     const int wave = tid >> 6;
     int ebits = 0;
     while ((1 << ebits) < E) ++ebits;
-    if (one_wave_ranks) {
-        // every slot of the block in one wave: a slot's rank is the number of lower lanes with its expert, an
-        // expert's count the size of its group - no barrier, no second pass
-        if (wave == 0) {
-            const int e = (lane < nls) ? lexp[lane] : -1;
-            unsigned long long mask = __ballot(e >= 0);
-            for (int b = 0; b < ebits; ++b) {
-                const bool bit = (e >> b) & 1;
-                const unsigned long long bb = __ballot(bit);
-                mask &= bit ? bb : ~bb;
-            }
-            const int rank_w = __popcll(mask & ((1ull << lane) - 1ull));
-            if (e >= 0) {
-                rank_in_block[(size_t)t0 * k + lane] = rank_w;
-                if (rank_w == 0) running[e] = __popcll(mask);  // zero so far (cleared at the top)
-            }
-            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's LDS writes have landed
-            __builtin_amdgcn_wave_barrier();
-            for (int idx = lane; idx < E; idx += 64) blockcnt[(size_t)blk * E + idx] = running[idx];
-        }
-        return;
-    }
-    const int rounds = (nls + kRouterThreads - 1) / kRouterThreads;
-    for (int rd = 0; rd < rounds; ++rd) {
-        for (int idx = tid; idx < kRouterWaves * E; idx += kRouterThreads) wcount[idx] = 0;
-        __syncthreads();
-        const int ls = rd * kRouterThreads + tid;
-        const int e = (ls < nls) ? lexp[ls] : -1;
+    // the slot's lower lanes with its expert, and (in the first of them) how many lanes have it
+    auto rank_in_wave = [&](int e, int& group) {
         unsigned long long mask = __ballot(e >= 0);
         for (int b = 0; b < ebits; ++b) {
             const bool bit = (e >> b) & 1;
             const unsigned long long bb = __ballot(bit);
             mask &= bit ? bb : ~bb;
         }
-        const int rank_w = __popcll(mask & ((1ull << lane) - 1ull));
-        if (e >= 0 && rank_w == 0) wcount[wave * E + e] = __popcll(mask);
+        group = __popcll(mask);
+        return __popcll(mask & ((1ull << lane) - 1ull));
+    };
+    // ---- partial sums for the auxiliary losses (fixed order), by the threads from `first` on ----
+    auto partial_sums = [&](int first) {
+        for (int e = tid - first; e >= 0 && e <= E; e += kRouterThreads - first) {
+            float s = 0.0f;
+            for (int i0 = 0; i0 < nt; i0 += 8) {
+                float pvv[8];
+                int okv[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int i = min(i0 + u, nt - 1);
+                    okv[u] = lexp[i * k];
+                    pvv[u] = e < E ? prob[i * ES + e] : lsev[i] * lsev[i];
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (i0 + u < nt && okv[u] >= 0) s += pvv[u];
+            }
+            partial[(size_t)blk * (E + 1) + e] = s;
+        }
+    };
+    // ---- rank of every local slot among earlier slots of the same expert: the block's slots in a few waves, the others take
+    // the partial sums meanwhile (64 experts, six a token: 5.3 us behind the softmax with one after the other) ----
+    if (rank_waves < kRouterWaves) {
+        const int ls = tid, e = ls < nls ? lexp[ls] : -1;
+        int group = 0, rank = 0;
+        if (wave < rank_waves) {  // uniform over the wave
+            rank = rank_in_wave(e, group);
+            if (e >= 0 && rank == 0) wcount[wave * E + e] = group;
+        } else {
+            partial_sums(64 * rank_waves);
+        }
+        if (rank_waves > 1) {
+            __syncthreads();
+        } else {
+            if (wave != 0) return;
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's LDS writes have landed
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (e >= 0) {
+            for (int w = 0; w < wave; ++w) rank += wcount[w * E + e];
+            rank_in_block[(size_t)t0 * k + ls] = rank;
+        }
+        for (int idx = tid; idx < E; idx += rank_waves > 1 ? kRouterThreads : 64) {
+            int count = 0;
+            for (int w = 0; w < rank_waves; ++w) count += wcount[w * E + idx];
+            blockcnt[(size_t)blk * E + idx] = count;
+        }
+        return;
+    }
+    partial_sums(0);
+    const int rounds = (nls + kRouterThreads - 1) / kRouterThreads;
+    for (int rd = 0; rd < rounds; ++rd) {
+        for (int idx = tid; idx < kRouterWaves * E; idx += kRouterThreads) wcount[idx] = 0;
+        __syncthreads();
+        const int ls = rd * kRouterThreads + tid;
+        const int e = (ls < nls) ? lexp[ls] : -1;
+        int group;
+        const int rank_w = rank_in_wave(e, group);
+        if (e >= 0 && rank_w == 0) wcount[wave * E + e] = group;
         __syncthreads();
         if (e >= 0) {
             int pre = running[e];

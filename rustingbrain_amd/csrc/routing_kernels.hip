@@ -23,7 +23,6 @@
 
 namespace rbmoe {
 
-
 size_t router_lds_bytes(int E, int k) {
     return router_fixed_bytes(E, k);
 }
@@ -1001,25 +1000,33 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     if ((reinterpret_cast<uintptr_t>(a.x) & 15) || ((size_t)a.d * xsize) % 16 != 0) return p;
     if (reinterpret_cast<uintptr_t>(a.wq ? static_cast<const void*>(a.wq) : a.wr) & 15) return p;
     if (a.norm_w && ((reinterpret_cast<uintptr_t>(a.xn_out) & 15) || a.d % 8 != 0)) return p;
+    const int NL = a.wq ? 32 : 8;
     p.exact = route_exact_ok(a, xsize == 2);
     int tokens = a.min_tokens;
     while (tokens < kRouterTokens && (a.T + tokens - 1) / tokens > 256) tokens *= 2;
     for (; tokens >= a.min_tokens && !p.tokens; tokens /= 2) {
         int EG = a.E;  // as many experts' rows as fit together, whole pairs, at least 8 (or all of them)
         auto lds = [&] { return rows_lds(a, p.exact, tokens, EG); };
-        while (EG > 8 && lds() > (size_t)kMaxRouterLds) EG = (EG - 1) & ~1;
+        const int least = p.exact ? exact_round(tokens, NL) : 8;
+        while (EG > least && lds() > (size_t)kMaxRouterLds) EG = p.exact ? exact_fewer(EG, tokens, NL) : (EG - 1) & ~1;
         if (lds() > (size_t)kMaxRouterLds) continue;
         p.tokens = tokens;
         p.EG = EG;
         p.lds = lds();
     }
     if (!p.tokens) return p;
-    // above: the sequences tuned for launches that fill the chip several times over.  Below, one round of workgroups or
+    // Above 256 K pairs: the sequences tuned for launches that fill the chip several times over.  Below, one round of workgroups or
     // none, for the chain of a second round is as long as the first's: 9000 tokens, d 512, 8 experts 60.0 us a forward in two
     // rounds, 57.0 without; 16 experts 63.2 / 57.1, f32 rows 65.8 / 56.7; d 512, 4 experts, two workgroups a unit 55.5 / 61.0.
     const int blocks = (a.T + p.tokens - 1) / p.tokens;
     const int together = p.tokens == kRouterTokens ? 256 * std::min(4, (int)((size_t)kMaxRouterLds / p.lds)) : 256;
-    if ((long long)a.T * a.E > 256 * 1024 || blocks > together) p.tokens = 0;
+    // On the matrix cores more than 16 experts in any number of rounds, ahead of a logit a lane and a launch for the rest: us a
+    // forward, logits_kernel + router_kernel / route_exact_kernel, 64 experts of 704, d 1024, 16384 rows 672.6 / 651.8, of 64, d 256,
+    // 30000 rows 110.0 / 92.3; 32 of 256, d 1024, 9000 rows 121.9 / 111.9, 16384 195.7 / 181.1; quantized, 64 of 704 751 / 747.  Up
+    // to 16 experts a chain less per round outweighs it: 16 of 256, d 768, 16384 rows 112.1 / 111.3, quantized 40000 rows 194.7 /
+    // 199.3; 8 of 64, d 512, 60000 rows 162.7 / 170.0.
+    const bool any_size = p.exact && a.E > 16;
+    if (!any_size && ((long long)a.T * a.E > 256 * 1024 || blocks > together)) p.tokens = 0;
     if (p.tokens > kMinRouterTokens && !p.exact && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
     // A few tokens by many experts: one workgroup a block would take the experts' rows through its own LDS one group after the
     // other (64 experts of d 1024: 27 us, whatever the tokens).  So the block's experts are shared out, eight to a workgroup

@@ -192,7 +192,10 @@ class Device:
         """An uninitialised array for results.  Large ones lie in pinned memory from the library's pool, which the GPU
         fills directly; the block goes back to the pool with the last reference to the array or a view of it."""
         dtype = np.dtype(dtype)
-        nbytes = int(np.prod(shape, dtype=np.int64)) * dtype.itemsize
+        # (np.prod takes 4 us an array, and the link is idle between two gradients: 24 of 2.9 MB fetched behind a step of 1024
+        # rows 2333 / 2293 us, 48 of 4.3 MB behind one of 4 x 8192 rows 6964 / 6863)
+        elements = math.prod(map(int, shape)) if isinstance(shape, tuple) else int(np.prod(shape, dtype=np.int64))
+        nbytes = elements * dtype.itemsize
         if nbytes < _PINNED_FROM:
             return np.empty(shape, dtype)
         p = C.c_void_p()

@@ -806,7 +806,7 @@ __global__ __launch_bounds__(256) void dispatch_kernel(
 // src/moe.rs:294-311), then + shared[t,:] (src/moe.rs:313-319), then
 // + residual[t,:].  Ascending expert order is ascending position order.
 // One thread per (token, 16-byte column piece); the token's slots are sorted
-// by position in registers when k <= KMAX, otherwise found by repeated search.
+// by position in registers when k <= KMAX (an unused slot is sorted behind them), otherwise found by repeated search.
 // ---------------------------------------------------------------------------
 // VN consecutive elements of an expert row, as raw bits and widened: the rows are of the layer's activation type, or
 // bf16 under f32 activations (a layer whose bf16 / int8 expert products run on the matrix cores).
@@ -826,57 +826,62 @@ struct RowPiece<bf16_t, float> {  // four bf16 elements beside four f32 ones
     }
 };
 
-template <typename XT, typename YT, int KMAX>
+// Bound by memory, 268 MB for 16384 tokens of d 1024 with six slots and a shared expert - as long as its vector instructions are
+// few: every lane sorting eight (position, gate) pairs by insertion made the kernel 1582 of them long; sorted as a network
+// of neighbours, for the least even number of slots, it has 530.
+// ROW: a row is whole waves of pieces (d a multiple of 512 in bf16, of 256 in f32), so that a wave's token is known to all its
+// lanes, and its positions and gates are fetched and sorted once a wave in scalar registers: 290.  us a forward, before / after: 64
+// experts of 704, six a token, d 1024, 16384 rows 673.3 / 665.2 (another box 712.0 / 701.0); 2048 rows of the default model 34.2 /
+// 33.9; without whole waves (d 768) 8192 rows by 16 experts, two a token, 147.2 / 146.4, 4096 rows int8 the same.
+template <typename XT, typename YT, int KMAX, bool ROW>
 __global__ __launch_bounds__(256) void combine_vec_kernel(
     const YT* __restrict__ y, const YT* __restrict__ yshared, const XT* __restrict__ residual,
-    const int* __restrict__ inv_pos, const float* __restrict__ gate_of, int T, int d, int k,
+    const int* __restrict__ inv_pos, const float* __restrict__ gate_of, int T, int d, int k, uint32_t recip,
     XT* __restrict__ out) {
     constexpr int VN = Vec16<XT>::N;
     typedef RowPiece<YT, XT> YP;
     const int pieces = d / VN;
-    const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (long long)T * pieces) return;
-    const int t = (int)(idx / pieces);
-    const int c = (int)(idx - (long long)t * pieces) * VN;
-    // the token's routed slots, sorted by position (insertion sort on registers)
-    int pos[KMAX];
-    float gate[KMAX];
+    int t, c;
+    if constexpr (ROW) {
+        const unsigned wave = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), per = (unsigned)pieces / 64u;
+        t = __builtin_amdgcn_readfirstlane((int)(wave / per));
+        if (t >= T) return;
+        c = (int)((wave - (unsigned)t * per) * 64u + (threadIdx.x & 63)) * VN;
+    } else {
+        const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
+        if (idx >= (long long)T * pieces) return;
+        t = recip ? (int)__umulhi((uint32_t)idx, recip) : (int)(idx / pieces);  // (uniform over the launch)
+        c = (int)(idx - (long long)t * pieces) * VN;
+    }
+    // The token's routed slots, sorted by position; those without one (-1) and those past k are the largest numbers.  All are requested
+    // before the first is looked at, from addresses that do not depend on one another - a slot past k repeats the last one:
+    // loads under a branch would follow one another, two trips to memory a slot in front of the rows'.  (Gates as bits: the
+    // compiler chooses between floats in vector registers.)
+    uint32_t pos[KMAX], gate[KMAX];
     int n = 0;
 #pragma unroll
     for (int r = 0; r < KMAX; ++r) {
-        pos[r] = 0x7fffffff;
-        gate[r] = 0.0f;
-    }
-    // (all positions and gates are requested before the first is looked at, from addresses that do not depend on
-    // one another - a slot past k repeats the last one: loads under a branch would follow one another, two trips to
-    // memory a slot in front of the rows')
-    int p_in[KMAX];
-    float g_in[KMAX];
-#pragma unroll
-    for (int r = 0; r < KMAX; ++r) {
         const int rr = r < k ? r : k - 1;
-        p_in[r] = inv_pos[(size_t)t * k + rr];
-        g_in[r] = gate_of[(size_t)t * k + rr];
+        pos[r] = (uint32_t)inv_pos[(size_t)t * k + rr];
+        gate[r] = reinterpret_cast<const uint32_t*>(gate_of)[(size_t)t * k + rr];
     }
 #pragma unroll
     for (int r = 0; r < KMAX; ++r) {
-        int p = p_in[r];
-        float g = g_in[r];
-        if (r < k && p >= 0) {
-            ++n;
-#pragma unroll
-            for (int q = 0; q < KMAX; ++q) {
-                if (p < pos[q]) {
-                    const int tp = pos[q];
-                    const float tg = gate[q];
-                    pos[q] = p;
-                    gate[q] = g;
-                    p = tp;
-                    g = tg;
-                }
-            }
-        }
+        if (r >= k) pos[r] = 0xffffffffu;
+        n += (int32_t)pos[r] >= 0 ? 1 : 0;
     }
+#pragma unroll
+    for (int round = 0; round < KMAX; ++round)  // neighbours in turn
+#pragma unroll
+        for (int q = round & 1; q + 1 < KMAX; q += 2) {
+            // (named values: a choice between array elements would be a choice of an index)
+            const uint32_t pa = pos[q], pb = pos[q + 1], ga = gate[q], gb = gate[q + 1];
+            const bool swap = pa > pb;
+            pos[q] = swap ? pb : pa;
+            pos[q + 1] = swap ? pa : pb;
+            gate[q] = swap ? gb : ga;
+            gate[q + 1] = swap ? ga : gb;
+        }
     float acc[VN];
 #pragma unroll
     for (int i = 0; i < VN; ++i) acc[i] = 0.0f;
@@ -894,7 +899,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(
             float v[VN];
             YP::widen(raw[r], v);
 #pragma unroll
-            for (int i = 0; i < VN; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn(gate[r], v[i]));
+            for (int i = 0; i < VN; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn(__uint_as_float(gate[r]), v[i]));
         }
     }
     if (yshared) {
@@ -1250,12 +1255,22 @@ static hipError_t launch_combine_t(const CombineArgs& a, hipStream_t s) {
     if (a.d % VN == 0 && a.k <= 8) {
         const long long total = (long long)a.T * (a.d / VN);
         const dim3 grid((unsigned)((total + 255) / 256)), block(256);
-        if (a.k <= 2)
-            RB_LAUNCH((combine_vec_kernel<XT, YT, 2>), grid, block, 0, s, y, ys, res, a.inv_pos, a.gate_of, a.T, a.d, a.k, out);
-        else if (a.k <= 4)
-            RB_LAUNCH((combine_vec_kernel<XT, YT, 4>), grid, block, 0, s, y, ys, res, a.inv_pos, a.gate_of, a.T, a.d, a.k, out);
-        else
-            RB_LAUNCH((combine_vec_kernel<XT, YT, 8>), grid, block, 0, s, y, ys, res, a.inv_pos, a.gate_of, a.T, a.d, a.k, out);
+        // 2^32 / pieces rounded up, which counts a row's pieces exactly as long as threads x pieces stays below 2^32 (0: divide)
+        const int pieces = a.d / VN;
+        const uint32_t recip = pieces > 1 && (total + 256) * pieces < (1ll << 32) ? (uint32_t)(0x100000000ull / (uint32_t)pieces) + 1u : 0u;
+        auto go = [&](auto kmax, auto row) {
+            RB_LAUNCH((combine_vec_kernel<XT, YT, decltype(kmax)::value, decltype(row)::value>), grid, block, 0, s, y, ys, res,
+                      a.inv_pos, a.gate_of, a.T, a.d, a.k, recip, out);
+        };
+        auto pick = [&](auto row) {
+            if (a.k <= 2) go(std::integral_constant<int, 2>{}, row);
+            else if (a.k <= 4) go(std::integral_constant<int, 4>{}, row);
+            else if (a.k <= 6) go(std::integral_constant<int, 6>{}, row);
+            else go(std::integral_constant<int, 8>{}, row);
+        };
+        // (waves are counted in 32 bits)
+        if (a.d / VN % 64 == 0 && total / 64 < (1ll << 31)) pick(std::true_type{});
+        else pick(std::false_type{});
     } else {
         RB_LAUNCH((combine_any_kernel<XT, YT>), dim3((a.T + 3) / 4), dim3(256), 0, s, y, ys, res, a.inv_pos,
                            a.gate_of, a.T, a.d, a.k, out);

@@ -1472,7 +1472,8 @@ hipError_t launch_decode_front(const RouterArgs& a, const DecodeGemmArgs& g, boo
     int EG = 0;
     const size_t lds = front_lds_bytes(a, bf16, &EG);
     RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, EG, a.P, a.lse, a.expert_of, a.gate_of,
-                    nullptr, nullptr, nullptr, nullptr, a.norm_w, a.norm_eps, nullptr, route_exact_ok(a, bf16)};
+                    nullptr, nullptr, nullptr, nullptr, a.norm_w, a.norm_eps, nullptr, route_exact_ok(a, bf16), 0, nullptr,
+                    a.exact_now};
     auto go = [&](auto kernel) -> hipError_t {
         static std::atomic<unsigned long long> attr_set{0};  // one per kernel: the lambda's body is instantiated for each
         const hipError_t e = once_per_device(attr_set, [&] {

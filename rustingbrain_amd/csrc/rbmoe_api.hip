@@ -266,7 +266,7 @@ struct rbmoe_layer {
     // weights
     Buf router;            // f32 [E, d]
     Buf router_q, router_s; // a quantized router: int8 [E, d], f32 scales [E] (`router` then holds the int8 values as f32)
-    bool router_exact = false;  // RouterArgs::exact of the router that is set
+    bool router_exact = false;  // RouterArgs::exact of the router that is set (a copy for the device: kRouterExactWord)
     bool router_q8 = false; // the layer routes with the quantized product (src/quantized.rs:55-62)
     bool quantize_router = false;  // f32 router data is quantized at upload (TransformerLm::quantize reaches the router too)
     int quant_rule = 0;     // f32 -> int8 at upload: 0 the checkpoint writer's rule, 1 the in-memory rule
@@ -281,7 +281,7 @@ struct rbmoe_layer {
     Buf xg, h, y, hs, ys;
     Buf x16;               // [max_T, d] bf16 copy of f32 rows (cast_rows)
     Buf hall;              // [E][min(max_T, 32), F] hidden rows of decode_front launches
-    Buf cmbcnt;            // [kDecodeCombineMaxBlocks] arrival counters of the folded decode combine
+    Buf cmbcnt;            // [kDecodeCombineMaxBlocks] arrival counters of the folded decode combine, kRouterExactWord
     // feed-forward norm in front of the layer (allocated by rbmoe_set_feed_forward_norm)
     Buf xn, norm_w;  // [max_T, d] activation dtype, [d] f32
     float norm_eps = 0.0f;
@@ -859,6 +859,8 @@ int rbmoe_set_weight(rbmoe_layer* L, int32_t which, int32_t expert, const void* 
         }
         L->router_q8 = router_to_i8;
         L->router_exact = router_to_i8 || router_weights_exact(static_cast<const float*>(src), n_given);
+        const int exact_now = L->router_exact;
+        HIP_TRY(ctx, hipMemcpy((int*)L->cmbcnt.p + kRouterExactWord, &exact_now, 4, hipMemcpyHostToDevice));
         L->weights_set = true;
         return RBMOE_OK;
     }
@@ -1177,7 +1179,9 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     ra.arrive = (int*)L->cmbcnt.p;
     if (L->tight) ra.min_tokens = kRouterTokens;
     ra.exact = L->router_exact;
+    ra.exact_now = (const int*)L->cmbcnt.p + kRouterExactWord;
     if (L->router_q8) {
+        ra.exact_now = nullptr;
         ra.wq = (const int8_t*)L->router_q.p;
         ra.wscale = (const float*)L->router_s.p;
     }

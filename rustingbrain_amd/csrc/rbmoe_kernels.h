@@ -86,8 +86,11 @@ struct RouterArgs {
     const float* wscale = nullptr;   // [E]
     // Whether every router weight - of a quantized router: its whole number - is zero or a bf16 value of a magnitude from 2^-40 to
     // below 2^20.  Times a bf16 element from 2^-72 to below 2^80 it is then exact in f32, and no sum of such products overflows
-    // or falls below 2^-126 on the way: the logits of bf16 rows may be taken by fused multiply-adds.
+    // or falls below 2^-126 on the way: the logits of bf16 rows may be taken by fused multiply-adds.  What the host knew when it chose
+    // the launch, and no more: a launch recorded into a graph or kept for a replay runs again when other weights lie in `wr`.
     bool exact = false;
+    // The same of the weights that lie there when the launch runs, beside them on the device (null: always true, as of whole numbers).
+    const int* exact_now = nullptr;
     // The norm in front of the layer (RmsNorm::forward, src/norm.rs:41-61), for calls whose plan says `takes_norm`: `x`
     // holds the raw rows, the routing is decided on the normed ones, which are written to `xn_out` [T, d].
     const float* norm_w = nullptr;
@@ -401,6 +404,8 @@ constexpr int kDecodeCombineMaxBlocks = 1024;  // feature blocks a folded combin
 // (side by side in one line, the atomics of a launch's two hundred workgroups queue up behind one another)
 constexpr int kDecodeCombineCounterStride = 64;
 constexpr size_t kDecodeCombineCounterBytes = (size_t)kDecodeCombineMaxBlocks * kDecodeCombineCounterStride * 4;
+// ... whose last word, in a cache line that no counter shares, is the layer's RouterArgs::exact_now
+constexpr int kRouterExactWord = kDecodeCombineMaxBlocks * kDecodeCombineCounterStride - 1;
 bool decode_shape_ok(int N, int K);
 hipError_t launch_decode_gemm(const DecodeGemmArgs& g, WeightKind wk, hipStream_t s);
 // Routing and gate/up products in one launch: every expert's gate/up product over all T rows, hidden rows to g.out as

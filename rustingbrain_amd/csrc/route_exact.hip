@@ -22,7 +22,8 @@ __global__ __launch_bounds__(kRouterThreads, 2) void route_exact_kernel(RouteRow
 
 hipError_t launch_route_exact(const RouterArgs& a, const RouterPlan& p, hipStream_t s) {
     RouteRowsArgs r{a.x, a.wr, a.wq, a.wscale, a.bias, a.valid, a.T, a.d, a.E, a.k, p.row_experts, a.P, a.lse, a.expert_of, a.gate_of,
-                    a.rank_in_block, a.blockcnt, a.partial, nullptr, a.norm_w, a.norm_eps, a.xn_out, true, p.row_slice, a.arrive};
+                    a.rank_in_block, a.blockcnt, a.partial, nullptr, a.norm_w, a.norm_eps, a.xn_out, true, p.row_slice, a.arrive,
+                    a.exact_now};
     const dim3 grid((a.T + p.block_tokens - 1) / p.block_tokens, p.row_slice ? (a.E + p.row_slice - 1) / p.row_slice : 1);
     auto go = [&](auto kernel) -> hipError_t {
         static std::atomic<unsigned long long> attr_set{0};  // one per kernel: the lambda's body is instantiated for each

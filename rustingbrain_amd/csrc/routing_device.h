@@ -297,6 +297,7 @@ struct RouteRowsArgs {
     bool exact = false;     // route_exact_body takes the rows
     int slice = 0;          // route_rows_kernel: experts of a workgroup (0: all of them)
     int* arrive = nullptr;  // ... and, with a slice, a token block's arrival counter, kDecodeCombineCounterStride apart
+    const int* exact_now = nullptr;  // RouterArgs::exact_now
 };
 // A staged row: column lane j's elements side by side, `lane_pitch` floats from one lane to the next - whole 16-byte
 // pieces (a last one short of four steps is filled up with zeros, which the sums do not see), and an odd number of
@@ -626,7 +627,9 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
 // (row, q) of the product finds its steps q, q + 4, q + 8, q + 12 in one 8-byte piece; who moves four pieces of a row there turns
 // them over in registers.  Wave w owns the column lanes w NL / 8 ..; the lanes' sums meet in LDS and are folded left to right by
 // a thread a logit.
-// A workgroup whose rows hold an element out of RowRange takes the same sums one multiply and one add at a time.
+// A workgroup whose rows hold an element out of RowRange takes the same sums one multiply and one add at a time.  So does every
+// workgroup of a launch that finds RouterArgs::exact_now unset, which a launch recorded under other weights does - over the weights in
+// memory (rounded_sums), for what is staged of them are bf16 parts.
 // Bound by the length of a workgroup's chain, not by work: 203 tokens, d 768, 16 experts, behind a norm, from the kernel's start:
 // normed rows laid down at 2.6 us, every wave's rows and weights at 3.7, sums 5.2, met 5.6, softmax and top-k 6.8, end 7.6; 8192
 // tokens without a norm 3.2, 3.7, 6.0, 6.7, 7.9, 8.7 (route_rows_body, with the same tail: 10.1 less the tail's 1.2; 11.7).  us a
@@ -677,6 +680,49 @@ __device__ __forceinline__ float fold_lanes(const float* part) {
     return __fadd_rn(y, 0.0f);  // the reference adds its (empty) scalar rest: sum + 0
 }
 
+// The column lanes' sums of `ne` experts from e0 on into `part`, for the tokens whose bits are set, one multiply and one add at a
+// time: token rows as they are staged, the router's weights from memory - a thread's sixteen of a block of steps serve four tokens.
+template <int TB, int NL>
+__device__ __forceinline__ void rounded_sums(const RouteRowsArgs& a, const unsigned char* xs, float* part, uint32_t tokens, int nt, int e0,
+                                             int ne) {
+    constexpr int RE = exact_round(TB, NL), TT = 4;
+    const int S = a.d / NL, Sp = exact_lane_steps(a.d, NL), pitch = exact_row_bytes(a.d, NL);
+#pragma unroll 1
+    for (int i = threadIdx.x; i < (TB / TT) * RE * NL; i += kRouterThreads) {
+        const int j = i % NL, e = i / NL % RE, t = i / (NL * RE) * TT;
+        if (e >= ne || ((tokens >> t) & ((1u << TT) - 1)) == 0) continue;
+        const unsigned char* x[TT];
+#pragma unroll
+        for (int u = 0; u < TT; ++u) x[u] = xs + min(t + u, nt - 1) * pitch + j * Sp * 2;
+        float sum[TT] = {};
+#pragma unroll 1
+        for (int s0 = 0; s0 < S; s0 += 16) {
+            float w[16];
+#pragma unroll
+            for (int s = 0; s < 16; ++s) {
+                const size_t at = (size_t)(e0 + e) * a.d + NL * min(s0 + s, S - 1) + j;
+                if constexpr (NL == 32) w[s] = (float)a.wq[at];
+                else w[s] = a.wr[at];
+            }
+#pragma unroll
+            for (int u = 0; u < TT; ++u) {
+                const uint4 lo = *reinterpret_cast<const uint4*>(x[u] + 2 * s0), hi = *reinterpret_cast<const uint4*>(x[u] + 2 * s0 + 16);
+                const uint32_t two[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+                for (int s = 0; s < 16; ++s) {
+                    if (s0 + s >= S) break;  // uniform
+                    const int p = (s & 3) * 4 + (s >> 2);
+                    const float v = __uint_as_float(p & 1 ? two[p >> 1] & 0xffff0000u : two[p >> 1] << 16);
+                    sum[u] = __fadd_rn(sum[u], __fmul_rn(v, w[s]));
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < TT; ++u)
+            if ((tokens >> (t + u)) & 1u) part[(j * TB + t + u) * RE + e] = sum[u];
+    }
+}
+
 // With `fold_later` and one round of experts the sums are left where they meet (behind a barrier), for ExactLogits, and the result is
 // true; otherwise the logits lie in `prob` and the caller meets at a barrier before it reads them.
 template <int TB, int NL, bool NORM>
@@ -692,6 +738,7 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
     unsigned char* const ws = xs + TB * pitch;
     const int tid = threadIdx.x, t0 = blk * TB, nt = min(TB, T - t0);
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool router_exact = NL == 32 || a.exact_now == nullptr || *a.exact_now != 0;  // (asked for here, looked at behind the staging)
 
     // Staging.  A piece is eight neighbouring columns; a task four pieces of a row, the steps 16 Q + 4 i + q.  (Past the end of
     // a row: zeros, which sums do not see.)
@@ -883,7 +930,9 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
         __builtin_amdgcn_sched_barrier(0);
         unsigned char* const wr = ws + room * pitch;
         {
-            if (exact) {  // uniform over the workgroup
+            if (!router_exact) {  // uniform over the launch
+                rounded_sums<TB, NL>(a, xs, part, 0xffffffffu, nt, e_from + r0, ne);
+            } else if (exact) {   // uniform over the workgroup
                 const unsigned char* x[MB];
                 const unsigned at = (unsigned)(wave * LW * Sp * 2 + 8 * (lane >> 4));
 #pragma unroll

@@ -128,3 +128,72 @@ def test_training_step_replays_identically(device, hip, monkeypatch):
     for b in (x, g, out, gin):
         b.free()
     layer.close()
+
+
+def general(router, seed):
+    """A router whose weights are no bf16 values, which routes other rows to other experts."""
+    return (router + 0.05 * np.random.default_rng(seed).standard_normal(router.shape)).astype(np.float32)
+
+
+def routing_of(layer, T):
+    c = layer.cache(T)
+    return {n: np.ascontiguousarray(getattr(c, n)).copy() for n in
+            ("expert_of", "counts", "offsets", "perm_slot", "perm_token", "probabilities", "log_sum_exp", "gate_of")}
+
+
+ROUTERS = [
+    (dict(d=768, E=8, k=2, F=128, T=8, shared=True), False),     # the routing beside the decode-shaped products
+    (dict(d=768, E=8, k=2, F=128, T=9, shared=True), True),      # ... behind the norm, two routing workgroups
+    (dict(d=704, E=16, k=2, F=64, T=203), True),                 # blocks of 8 tokens, the norm in the launch
+    (dict(d=512, E=33, k=3, F=64, T=40), False),                 # ... a block's experts shared out over workgroups
+    (dict(d=320, E=12, k=2, F=64, T=2100), False),               # blocks of 16
+    (dict(d=1024, E=64, k=2, F=64, T=4500), False),              # blocks of 32, more pairs than the other launches take
+]
+
+
+@pytest.mark.parametrize("shape,block", ROUTERS)
+def test_a_replay_routes_with_the_weights_of_its_own_time(device, hip, shape, block):
+    """A graph captured with a router of bf16 values, whose products with bf16 rows are exact, follows the router to weights that
+    are none and back; so does the routing stage launched again by itself."""
+    t = synth.make(small_workload(seed=63, act="bf16", wt="bf16", **shape))
+    T = shape["T"]
+    exact = synth.round_bf16(t.router)
+    layer = gpu_layer(device, t, max_tokens=T)
+    layer.set_feed_forward_norm(np.linspace(0.5, 1.5, shape["d"]).astype(np.float32), 1e-6)
+    xh = bits(t, t.x)
+    x = DeviceBuffer(device, xh.nbytes).upload(xh)
+    out = DeviceBuffer(device, xh.nbytes)
+    run = lambda: (layer.forward_block_device if block else layer.forward_device)(x.ptr, T, out.ptr)
+
+    def eager(router):
+        layer.set_router(router)
+        run()
+        device.synchronize()
+        return dict(routing_of(layer, T), out=out.download(np.empty_like(xh)).copy())
+
+    routers = [exact, general(exact, 1), exact * np.float32(2.0 ** 30), general(exact, 2)]
+    want = [eager(r) for r in routers]
+    assert not np.array_equal(want[0]["expert_of"], want[1]["expert_of"])
+    layer.set_router(exact)
+    cap = Capture(hip, device, run)
+    for i in (0, 1, 0, 2, 3):
+        layer.set_router(routers[i])
+        out.upload(np.zeros_like(xh))
+        cap.replay()
+        got = dict(routing_of(layer, T), out=out.download(np.empty_like(xh)))
+        for name, a in want[i].items():
+            assert np.array_equal(a, got[name], equal_nan=a.dtype == np.float32), (i, name)
+    cap.close()
+    # the stage by itself
+    if not block and "front" not in layer.kernel_name():
+        layer.set_router(exact)
+        run()
+        layer.set_router(routers[1])
+        assert layer.enqueue_stage("router") and layer.enqueue_stage("dispatch")
+        device.synchronize()
+        got = routing_of(layer, T)
+        for name in got:
+            assert np.array_equal(got[name], want[1][name]), name
+    for b in (x, out):
+        b.free()
+    layer.close()

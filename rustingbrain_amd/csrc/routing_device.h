@@ -627,9 +627,13 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
 // (row, q) of the product finds its steps q, q + 4, q + 8, q + 12 in one 8-byte piece; who moves four pieces of a row there turns
 // them over in registers.  Wave w owns the column lanes w NL / 8 ..; the lanes' sums meet in LDS and are folded left to right by
 // a thread a logit.
-// A workgroup whose rows hold an element out of RowRange takes the same sums one multiply and one add at a time.  So does every
-// workgroup of a launch that finds RouterArgs::exact_now unset, which a launch recorded under other weights does - over the weights in
-// memory (rounded_sums), for what is staged of them are bf16 parts.
+// A token whose row holds an element out of RowRange gets its sums one multiply and one add at a time (rounded_sums), beside the
+// products of its block.  So does every token of a launch that finds RouterArgs::exact_now unset, which a launch recorded under other
+// weights does - over the weights in memory, for what is staged of them are bf16 parts.
+// us a call with no such element / one in one row / one in every row: 203 tokens, d 768, 16 experts, behind a norm 27.1 / 29.4 / 30.8; 8192
+// of them without 46.0 / 49.8 / 55.4; 16384, d 1024, 64 experts 220 / 232 / 347 (route_rows_body or logits_kernel: 28.8, 50.4, 270, whatever
+// the elements).  The routing alone under weights that were set after the launch was recorded, beside a launch chosen for them: 9.3
+// against 8.0, 17.8 against 14.3, 153 against 89.
 // Bound by the length of a workgroup's chain, not by work: 203 tokens, d 768, 16 experts, behind a norm, from the kernel's start:
 // normed rows laid down at 2.6 us, every wave's rows and weights at 3.7, sums 5.2, met 5.6, softmax and top-k 6.8, end 7.6; 8192
 // tokens without a norm 3.2, 3.7, 6.0, 6.7, 7.9, 8.7 (route_rows_body, with the same tail: 10.1 less the tail's 1.2; 11.7).  us a
@@ -681,11 +685,13 @@ __device__ __forceinline__ float fold_lanes(const float* part) {
 }
 
 // The column lanes' sums of `ne` experts from e0 on into `part`, for the tokens whose bits are set, one multiply and one add at a
-// time: token rows as they are staged, the router's weights from memory - a thread's sixteen of a block of steps serve four tokens.
+// time: token rows as they are staged, the router's weights from memory - a thread's sixteen of a block of steps serve up to eight
+// tokens, the same for a whole wave, which leaves out a pair without a bit.  Bound by the vector units and the wait for the weights (asked
+// for a block ahead they made the kernels 150 to 190 registers, room for one workgroup on a compute unit instead of two).
 template <int TB, int NL>
 __device__ __forceinline__ void rounded_sums(const RouteRowsArgs& a, const unsigned char* xs, float* part, uint32_t tokens, int nt, int e0,
                                              int ne) {
-    constexpr int RE = exact_round(TB, NL), TT = 4;
+    constexpr int RE = exact_round(TB, NL), TT = TB * RE * NL / kRouterThreads < 8 ? TB * RE * NL / kRouterThreads : 8;
     const int S = a.d / NL, Sp = exact_lane_steps(a.d, NL), pitch = exact_row_bytes(a.d, NL);
 #pragma unroll 1
     for (int i = threadIdx.x; i < (TB / TT) * RE * NL; i += kRouterThreads) {
@@ -695,27 +701,49 @@ __device__ __forceinline__ void rounded_sums(const RouteRowsArgs& a, const unsig
 #pragma unroll
         for (int u = 0; u < TT; ++u) x[u] = xs + min(t + u, nt - 1) * pitch + j * Sp * 2;
         float sum[TT] = {};
-#pragma unroll 1
-        for (int s0 = 0; s0 < S; s0 += 16) {
+        struct Steps {
             float w[16];
+        };
+        const size_t row = (size_t)(e0 + e) * a.d + j;
+        auto weight = [&](size_t at) -> float {
+            if constexpr (NL == 32) return (float)a.wq[at];
+            else return a.wr[at];
+        };
+        auto add = [&](const Steps& v, int s0) {
 #pragma unroll
-            for (int s = 0; s < 16; ++s) {
-                const size_t at = (size_t)(e0 + e) * a.d + NL * min(s0 + s, S - 1) + j;
-                if constexpr (NL == 32) w[s] = (float)a.wq[at];
-                else w[s] = a.wr[at];
-            }
+            for (int h = 0; h < TT / 2; ++h) {  // two tokens at a time
+                if (((tokens >> (t + 2 * h)) & 3u) == 0) continue;
+                uint32_t two[2][8];
 #pragma unroll
-            for (int u = 0; u < TT; ++u) {
-                const uint4 lo = *reinterpret_cast<const uint4*>(x[u] + 2 * s0), hi = *reinterpret_cast<const uint4*>(x[u] + 2 * s0 + 16);
-                const uint32_t two[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                for (int u = 0; u < 2; ++u) {
+                    const uint4 lo = *reinterpret_cast<const uint4*>(x[2 * h + u] + 2 * s0);
+                    const uint4 hi = *reinterpret_cast<const uint4*>(x[2 * h + u] + 2 * s0 + 16);
+                    two[u][0] = lo.x; two[u][1] = lo.y; two[u][2] = lo.z; two[u][3] = lo.w;
+                    two[u][4] = hi.x; two[u][5] = hi.y; two[u][6] = hi.z; two[u][7] = hi.w;
+                }
 #pragma unroll
                 for (int s = 0; s < 16; ++s) {
-                    if (s0 + s >= S) break;  // uniform
                     const int p = (s & 3) * 4 + (s >> 2);
-                    const float v = __uint_as_float(p & 1 ? two[p >> 1] & 0xffff0000u : two[p >> 1] << 16);
-                    sum[u] = __fadd_rn(sum[u], __fmul_rn(v, w[s]));
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const float f = __uint_as_float(p & 1 ? two[u][p >> 1] & 0xffff0000u : two[u][p >> 1] << 16);
+                        sum[2 * h + u] = __fadd_rn(sum[2 * h + u], __fmul_rn(f, v.w[s]));
+                    }
                 }
             }
+        };
+#pragma unroll 1
+        for (int s0 = 0; s0 < S; s0 += 16) {
+            Steps v;
+            const size_t from = row + NL * s0;
+            if (s0 + 16 <= S) {
+#pragma unroll
+                for (int s = 0; s < 16; ++s) v.w[s] = weight(from + NL * s);
+            } else {  // (rows hold zeros past their end)
+#pragma unroll
+                for (int s = 0; s < 16; ++s) v.w[s] = s0 + s < S ? weight(from + NL * s) : 0.0f;
+            }
+            add(v, s0);
         }
 #pragma unroll
         for (int u = 0; u < TT; ++u)
@@ -907,9 +935,25 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
         if (lane == 0) left[wave] = any;
     }
     __syncthreads();
-    bool exact = true;
+    bool exact = router_exact;
 #pragma unroll
     for (int w = 0; w < kRouterWaves; ++w) exact = exact && left[w] == 0;
+    uint32_t rounded = 0;  // the tokens whose sums are taken one rounding at a time
+    if (!exact) {          // uniform over the workgroup
+        __syncthreads();   // everyone has read the votes
+        uint32_t mine = router_exact ? 0u : 0xffffffffu;
+        if (router_exact)
+            for (int t = wave; t < nt; t += kRouterWaves) {
+                RowRange of_row;
+                for (int i = lane; i < NL * Sp / 8; i += 64) of_row.see(*reinterpret_cast<const uint4*>(xs + t * pitch + 16 * i));
+                mine |= __ballot(of_row.left()) != 0ull ? 1u << t : 0u;
+            }
+        if (lane == 0) left[wave] = (int)mine;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kRouterWaves; ++w) rounded |= (uint32_t)left[w];
+        rounded = __builtin_amdgcn_readfirstlane(rounded);
+    }
     // ---- the column lanes' sums, 16 (RE) experts at a time ----------------------------
     // Experts past the EG whose rows lie in LDS follow round by round, into the place of the round that is done with, asked for in
     // front of its products.
@@ -930,9 +974,7 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
         __builtin_amdgcn_sched_barrier(0);
         unsigned char* const wr = ws + room * pitch;
         {
-            if (!router_exact) {  // uniform over the launch
-                rounded_sums<TB, NL>(a, xs, part, 0xffffffffu, nt, e_from + r0, ne);
-            } else if (exact) {   // uniform over the workgroup
+            if (router_exact) {  // uniform over the launch
                 const unsigned char* x[MB];
                 const unsigned at = (unsigned)(wave * LW * Sp * 2 + 8 * (lane >> 4));
 #pragma unroll
@@ -988,18 +1030,10 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
                             const int t = 16 * b + 4 * (lane >> 4) + i, e = lane & 15;
                             if (t < TB && e < ne) part[((wave * LW + u) * TB + t) * RE + e] = acc[u][b][i];
                         }
-            } else {
-                for (int i = tid; i < nt * ne * NL; i += NT) {
-                    const int j = i % NL, t = i / NL / ne, e = i / NL - t * ne;
-                    const uint16_t* const xr = reinterpret_cast<const uint16_t*>(xs + t * pitch) + j * Sp;
-                    const uint16_t* const er = reinterpret_cast<const uint16_t*>(wr + e * pitch) + j * Sp;
-                    float sum = 0.0f;
-                    for (int s = 0; s < S; ++s) {
-                        const int p = (s & ~15) + (s & 3) * 4 + ((s >> 2) & 3);
-                        sum = __fadd_rn(sum, __fmul_rn(bf16_bits_to_f32(xr[p]), bf16_bits_to_f32(er[p])));
-                    }
-                    part[(j * TB + t) * RE + e] = sum;
-                }
+            }
+            if (rounded != 0) {  // uniform over the workgroup
+                if (router_exact) __syncthreads();  // these take the place of the products' sums
+                rounded_sums<TB, NL>(a, xs, part, rounded, nt, e_from + r0, ne);
             }
             __syncthreads();
             if (fold_later && n <= RE) return true;

@@ -52,3 +52,25 @@ def test_routing_of_bf16_rows(device, shape, form, quantized):
     _, cache = layer.forward_train(x, rb.Layout())
     assert_routing_identical(cache, ref)
     layer.close()
+
+
+@pytest.mark.parametrize("quantized", [False, True])
+@pytest.mark.parametrize("which", ["one", "all"])
+def test_rows_out_of_range_do_not_hold_up_the_others(device, which, quantized):
+    """One tiny element in one row, and one in every row.  A row's exact sums are 2 x 64 x 1024 operations on the vector units instead of
+    the matrix cores, a 32nd of a block's for one of its rows: four times the routing's time is far above either, the fifteen that a
+    whole block's sums took one after the other are far beyond."""
+    t = synth.make(small_workload(d=1024, E=64, k=2, F=64, T=4200, seed=38, act="bf16", wt="int8"))
+    layer = gpu_layer(device, t)
+    if quantized:
+        layer.set_router_q8(*synth.quantize_rows(t.router))
+
+    def routing(x):
+        layer.forward_train(x)
+        return min(layer.replay_stage("router", 10) for _ in range(3))
+
+    plain = routing(t.x)
+    x = t.x.copy()
+    x[:1 if which == "one" else None, 3] = synth.round_bf16(np.full(1, 1e-30, np.float32))
+    assert routing(x) < 4 * plain
+    layer.close()

@@ -630,10 +630,10 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
 // A token whose row holds an element out of RowRange gets its sums one multiply and one add at a time (rounded_sums), beside the
 // products of its block.  So does every token of a launch that finds RouterArgs::exact_now unset, which a launch recorded under other
 // weights does - over the weights in memory, for what is staged of them are bf16 parts.
-// us a call with no such element / one in one row / one in every row: 203 tokens, d 768, 16 experts, behind a norm 27.1 / 29.4 / 30.8; 8192
-// of them without 46.0 / 49.8 / 55.4; 16384, d 1024, 64 experts 220 / 232 / 347 (route_rows_body or logits_kernel: 28.8, 50.4, 270, whatever
-// the elements).  The routing alone under weights that were set after the launch was recorded, beside a launch chosen for them: 9.3
-// against 8.0, 17.8 against 14.3, 153 against 89.
+// us a call with no such element / one in one row / one in every row: 203 tokens, d 768, 16 experts, behind a norm 27.2 / 29.3 / 32.3; 8192
+// of them without 45.8 / 49.1 / 59.5; 16384, d 1024, 64 experts 213 / 225 / 346 (route_rows_body or logits_kernel: 28.8, 50.4, 270, whatever
+// the elements).  The routing alone under weights that were set after the launch was recorded, beside a launch chosen for them: 10.7
+// against 8.0, 22.3 against 14.2, 165 against 89.
 // Bound by the length of a workgroup's chain, not by work: 203 tokens, d 768, 16 experts, behind a norm, from the kernel's start:
 // normed rows laid down at 2.6 us, every wave's rows and weights at 3.7, sums 5.2, met 5.6, softmax and top-k 6.8, end 7.6; 8192
 // tokens without a norm 3.2, 3.7, 6.0, 6.7, 7.9, 8.7 (route_rows_body, with the same tail: 10.1 less the tail's 1.2; 11.7).  us a
@@ -685,13 +685,15 @@ __device__ __forceinline__ float fold_lanes(const float* part) {
 }
 
 // The column lanes' sums of `ne` experts from e0 on into `part`, for the tokens whose bits are set, one multiply and one add at a
-// time: token rows as they are staged, the router's weights from memory - a thread's sixteen of a block of steps serve up to eight
-// tokens, the same for a whole wave, which leaves out a pair without a bit.  Bound by the vector units and the wait for the weights (asked
-// for a block ahead they made the kernels 150 to 190 registers, room for one workgroup on a compute unit instead of two).
+// time: token rows as they are staged, the router's weights from memory - a thread's sixteen of a block of steps serve up to four
+// tokens, the same for a whole wave, which leaves out those without a bit.  Bound by the vector units and the wait for the weights.
+// What counts first is that the kernels around it stay small: with eight tokens a thread (37.5 KB and 118 registers instead of 35.8 and
+// 106) 16384 tokens of d 1024 by 64 experts are rounded 6 % faster, but 9000 of d 512 by 8, none of them rounded, are routed in 13.1 us
+// instead of 12.5; with the weights asked for a block ahead the kernels take 150 to 190 registers.
 template <int TB, int NL>
 __device__ __forceinline__ void rounded_sums(const RouteRowsArgs& a, const unsigned char* xs, float* part, uint32_t tokens, int nt, int e0,
                                              int ne) {
-    constexpr int RE = exact_round(TB, NL), TT = TB * RE * NL / kRouterThreads < 8 ? TB * RE * NL / kRouterThreads : 8;
+    constexpr int RE = exact_round(TB, NL), TT = TB * RE * NL / kRouterThreads < 4 ? 2 : 4;
     const int S = a.d / NL, Sp = exact_lane_steps(a.d, NL), pitch = exact_row_bytes(a.d, NL);
 #pragma unroll 1
     for (int i = threadIdx.x; i < (TB / TT) * RE * NL; i += kRouterThreads) {
@@ -711,24 +713,15 @@ __device__ __forceinline__ void rounded_sums(const RouteRowsArgs& a, const unsig
         };
         auto add = [&](const Steps& v, int s0) {
 #pragma unroll
-            for (int h = 0; h < TT / 2; ++h) {  // two tokens at a time
-                if (((tokens >> (t + 2 * h)) & 3u) == 0) continue;
-                uint32_t two[2][8];
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const uint4 lo = *reinterpret_cast<const uint4*>(x[2 * h + u] + 2 * s0);
-                    const uint4 hi = *reinterpret_cast<const uint4*>(x[2 * h + u] + 2 * s0 + 16);
-                    two[u][0] = lo.x; two[u][1] = lo.y; two[u][2] = lo.z; two[u][3] = lo.w;
-                    two[u][4] = hi.x; two[u][5] = hi.y; two[u][6] = hi.z; two[u][7] = hi.w;
-                }
+            for (int u = 0; u < TT; ++u) {
+                if (((tokens >> (t + u)) & 1u) == 0) continue;
+                const uint4 lo = *reinterpret_cast<const uint4*>(x[u] + 2 * s0), hi = *reinterpret_cast<const uint4*>(x[u] + 2 * s0 + 16);
+                const uint32_t two[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
                 for (int s = 0; s < 16; ++s) {
                     const int p = (s & 3) * 4 + (s >> 2);
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        const float f = __uint_as_float(p & 1 ? two[u][p >> 1] & 0xffff0000u : two[u][p >> 1] << 16);
-                        sum[2 * h + u] = __fadd_rn(sum[2 * h + u], __fmul_rn(f, v.w[s]));
-                    }
+                    const float f = __uint_as_float(p & 1 ? two[p >> 1] & 0xffff0000u : two[p >> 1] << 16);
+                    sum[u] = __fadd_rn(sum[u], __fmul_rn(f, v.w[s]));
                 }
             }
         };
@@ -766,7 +759,14 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
     unsigned char* const ws = xs + TB * pitch;
     const int tid = threadIdx.x, t0 = blk * TB, nt = min(TB, T - t0);
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool router_exact = NL == 32 || a.exact_now == nullptr || *a.exact_now != 0;  // (asked for here, looked at behind the staging)
+    int exact_now = 1;
+    // (a vector load among the rows': a scalar one would be waited for with the kernel's arguments)
+    auto ask_router = [&] {
+        int zero = 0;
+        asm("" : "+v"(zero));
+        if constexpr (NL == 8)
+            if (a.exact_now != nullptr) exact_now = a.exact_now[zero];
+    };
 
     // Staging.  A piece is eight neighbouring columns; a task four pieces of a row, the steps 16 Q + 4 i + q.  (Past the end of
     // a row: zeros, which sums do not see.)
@@ -858,6 +858,7 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
 #pragma unroll
             for (int i = 0; i < H / 4; ++i) nwv[i] = *reinterpret_cast<const float4*>(a.norm_w + c0 + 4 * i);
             const Weights w = weights_of(e_from, nw0, tid);
+            ask_router();
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
             for (int r = wave; r < nt; r += NT / 64) {
@@ -923,6 +924,7 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
         Rows r0 = rows_of(tid), r1 = r0;
         if (NT < nx) r1 = rows_of(tid + NT);
         const Weights w = weights_of(e_from, nw0, tid);
+        ask_router();
         __builtin_amdgcn_sched_barrier(0);
         put_rows(tid, r0);
         put_rows(tid + NT, r1);
@@ -931,15 +933,16 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
     }
     rest_of_router(e_from, nw0, NT, ws);
     {
-        const bool any = __ballot(range.left()) != 0ull;
+        const bool any = __ballot(range.left() || exact_now == 0) != 0ull;
         if (lane == 0) left[wave] = any;
     }
     __syncthreads();
-    bool exact = router_exact;
+    const bool router_exact = __builtin_amdgcn_readfirstlane(exact_now) != 0;
+    bool exact = true;
 #pragma unroll
     for (int w = 0; w < kRouterWaves; ++w) exact = exact && left[w] == 0;
     uint32_t rounded = 0;  // the tokens whose sums are taken one rounding at a time
-    if (!exact) {          // uniform over the workgroup
+    if (__builtin_expect(!exact, 0)) {  // uniform over the workgroup
         __syncthreads();   // everyone has read the votes
         uint32_t mine = router_exact ? 0u : 0xffffffffu;
         if (router_exact)
@@ -1031,7 +1034,7 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
                             if (t < TB && e < ne) part[((wave * LW + u) * TB + t) * RE + e] = acc[u][b][i];
                         }
             }
-            if (rounded != 0) {  // uniform over the workgroup
+            if (__builtin_expect(rounded != 0, 0)) {  // uniform over the workgroup
                 if (router_exact) __syncthreads();  // these take the place of the products' sums
                 rounded_sums<TB, NL>(a, xs, part, rounded, nt, e_from + r0, ne);
             }

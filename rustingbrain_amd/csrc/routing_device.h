@@ -938,11 +938,11 @@ __device__ __forceinline__ bool route_exact_body(const RouteRowsArgs& a, int blk
     }
     __syncthreads();
     const bool router_exact = __builtin_amdgcn_readfirstlane(exact_now) != 0;
-    bool exact = true;
+    int votes = 0;  // (all of them asked for before the first is looked at)
 #pragma unroll
-    for (int w = 0; w < kRouterWaves; ++w) exact = exact && left[w] == 0;
+    for (int w = 0; w < kRouterWaves; ++w) votes |= left[w];
     uint32_t rounded = 0;  // the tokens whose sums are taken one rounding at a time
-    if (__builtin_expect(!exact, 0)) {  // uniform over the workgroup
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(votes) != 0, 0)) {  // uniform over the workgroup
         __syncthreads();   // everyone has read the votes
         uint32_t mine = router_exact ? 0u : 0xffffffffu;
         if (router_exact)

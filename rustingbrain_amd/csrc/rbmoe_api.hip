@@ -2690,8 +2690,9 @@ int rbmoe_internal_widths(const rbmoe_config* cfg, int32_t training, int32_t* ou
 
 // Test hook (not part of rbmoe.h), runs without a GPU: how a large-batch call on rows at address `x` (never read) is routed.
 // out[0]: tokens of a router block as the dispatch counts them, [1]: whether the norm takes a launch of its own, [2]: whether
-// the router's launch takes the plan with the arguments it gets, [3]: tokens of a block when the stage is replayed.
-int rbmoe_internal_router_plan(int32_t d, int32_t E, int32_t k, int32_t T, int32_t bf16, int32_t norm, int32_t quantized,
+// the router's launch takes the plan with the arguments it gets, [3]: tokens of a block when the stage is replayed, [4]: whether
+// the sums are taken on the matrix cores (`exact`: RouterArgs::exact; a quantized router's values always are).
+int rbmoe_internal_router_plan(int32_t d, int32_t E, int32_t k, int32_t T, int32_t bf16, int32_t norm, int32_t quantized, int32_t exact,
                                int32_t fused, uint64_t x, int32_t* out) {
     if (!out) return RBMOE_NULL_POINTER;
     auto at = [](uint64_t address) { return reinterpret_cast<void*>((uintptr_t)address); };
@@ -2701,6 +2702,7 @@ int rbmoe_internal_router_plan(int32_t d, int32_t E, int32_t k, int32_t T, int32
     a.wr = static_cast<const float*>(own);
     a.T = T; a.d = d; a.E = E; a.k = k;
     a.allow_fused = fused != 0;
+    a.exact = exact != 0;
     if (quantized) {
         a.wq = static_cast<const int8_t*>(own);
         a.wscale = static_cast<const float*>(own);
@@ -2714,6 +2716,7 @@ int rbmoe_internal_router_plan(int32_t d, int32_t E, int32_t k, int32_t T, int32
     out[0] = p.block_tokens;
     out[1] = apart ? 1 : 0;
     out[2] = router_takes(a, p, bf16 != 0) ? 1 : 0;
+    out[4] = p.row_exact ? 1 : 0;
     if (a.norm_w) {
         a.x = own;
         a.norm_w = nullptr;
@@ -2725,10 +2728,11 @@ int rbmoe_internal_router_plan(int32_t d, int32_t E, int32_t k, int32_t T, int32
 
 // Test hook (not part of rbmoe.h), runs without a GPU: experts of a routing workgroup of a large-batch call on aligned rows, 0
 // where a block's experts are not shared out.
-int rbmoe_internal_router_slice(int32_t d, int32_t E, int32_t k, int32_t T, int32_t bf16, int32_t norm, int32_t quantized) {
+int rbmoe_internal_router_slice(int32_t d, int32_t E, int32_t k, int32_t T, int32_t bf16, int32_t norm, int32_t quantized, int32_t exact) {
     RouterArgs a{};
     a.T = T; a.d = d; a.E = E; a.k = k;
     a.allow_fused = true;
+    a.exact = exact != 0;
     a.x = reinterpret_cast<void*>((uintptr_t)1 << 20);  // (never read)
     a.wr = static_cast<const float*>(a.x);
     if (quantized) {

@@ -998,7 +998,7 @@ static size_t rows_lds(const RouterArgs& a, bool exact, int tokens, int EG) {
                  : route_rows_lds_bytes(a.E, a.k, a.d, tokens, NL, EG, a.norm_w != nullptr);
 }
 
-static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
+static RowsPlan plan_rows(const RouterArgs& a, size_t xsize, bool exact) {
     RowsPlan p;
     const int unit = a.wq ? 32 : 8;  // whole turns of the column lanes, whole 16-byte pieces
     if (!a.allow_fused || a.E > 64 || a.d % unit != 0 || a.d < unit || a.k > kMaxTopK) return p;
@@ -1006,7 +1006,7 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     if (reinterpret_cast<uintptr_t>(a.wq ? static_cast<const void*>(a.wq) : a.wr) & 15) return p;
     if (a.norm_w && ((reinterpret_cast<uintptr_t>(a.xn_out) & 15) || a.d % 8 != 0)) return p;
     const int NL = a.wq ? 32 : 8;
-    p.exact = route_exact_ok(a, xsize == 2);
+    p.exact = exact;
     int tokens = a.min_tokens;
     while (tokens < kRouterTokens && (a.T + tokens - 1) / tokens > 256) tokens *= 2;
     for (; tokens >= a.min_tokens && !p.tokens; tokens /= 2) {
@@ -1023,13 +1023,19 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
     // Above 256 K pairs: the sequences tuned for launches that fill the chip several times over.  Below, one round of workgroups or
     // none, for the chain of a second round is as long as the first's: 9000 tokens, d 512, 8 experts 60.0 us a forward in two
     // rounds, 57.0 without; 16 experts 63.2 / 57.1, f32 rows 65.8 / 56.7; d 512, 4 experts, two workgroups a unit 55.5 / 61.0.
+    // Blocks of 32 tokens lie on a compute unit as its LDS and its registers allow: of route_rows_kernel three up to 8 experts (up to 76
+    // registers), two beyond (92); of route_exact_kernel two (106), over a quantized router one (135).  d 256, 8 experts of 64, 20000
+    // rows: three of the former 54.7, without 56.8; f32 rows 87.4 / 90.1; short rows the other way round, d 128, 20000 rows 45.5 / 43.8.
+    // On the matrix cores a round more all the same where rows are long enough: d 384, 20000 rows 68.0 / 69.6, d 256 57.0 / 54.7, d 128
+    // 48.5 / 43.8; quantized, d 512, 8193 rows 47.3 / 50.4, d 256, 12000 rows 51.4 / 49.6.
     const int blocks = (a.T + p.tokens - 1) / p.tokens;
-    const int together = p.tokens == kRouterTokens ? 256 * std::min(4, (int)((size_t)kMaxRouterLds / p.lds)) : 256;
+    const int in_lds = (int)((size_t)kMaxRouterLds / p.lds);
+    const int a_unit = p.exact ? (a.wq ? (a.d >= 512 ? 2 : 1) : (a.d >= 384 ? 3 : 2)) : (a.wq || a.E > 8 || a.d < 256 ? 2 : 3);
+    const int together = p.tokens == kRouterTokens ? 256 * std::min(a_unit, in_lds) : 256;
     // On the matrix cores more than 16 experts in any number of rounds, ahead of a logit a lane and a launch for the rest: us a
     // forward, logits_kernel + router_kernel / route_exact_kernel, 64 experts of 704, d 1024, 16384 rows 672.6 / 651.8, of 64, d 256,
-    // 30000 rows 110.0 / 92.3; 32 of 256, d 1024, 9000 rows 121.9 / 111.9, 16384 195.7 / 181.1; quantized, 64 of 704 751 / 747.  Up
-    // to 16 experts a chain less per round outweighs it: 16 of 256, d 768, 16384 rows 112.1 / 111.3, quantized 40000 rows 194.7 /
-    // 199.3; 8 of 64, d 512, 60000 rows 162.7 / 170.0.
+    // 30000 rows 110.0 / 92.3; 32 of 256, d 1024, 9000 rows 121.9 / 111.9, 16384 195.7 / 181.1; quantized, 64 of 704 751 / 747.  Up to 16 experts a chain less per round outweighs it: 16 of 256, d 768, 16384 rows 112.1 / 111.3, quantized
+    // 40000 rows 194.7 / 199.3; 8 of 64, d 512, 60000 rows 162.7 / 170.0.
     const bool any_size = p.exact && a.E > 16;
     if (!any_size && ((long long)a.T * a.E > 256 * 1024 || blocks > together)) p.tokens = 0;
     if (p.tokens > kMinRouterTokens && !p.exact && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
@@ -1050,7 +1056,8 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize) {
 }
 
 RouterPlan plan_router(const RouterArgs& a, bool bf16) {
-    const RowsPlan p = plan_rows(a, bf16 ? 2 : 4);
+    RowsPlan p = plan_rows(a, bf16 ? 2 : 4, route_exact_ok(a, bf16));
+    if (!p.tokens && p.exact) p = plan_rows(a, bf16 ? 2 : 4, false);
     RouterPlan q;
     q.block_tokens = p.tokens ? p.tokens : kRouterTokens;
     q.row_experts = p.tokens ? p.EG : 0;

@@ -94,6 +94,19 @@ def test_a_dense_tile_starts_when_every_wave_has_the_routed_counts(source, kerne
 
 
 @needs_hipcc
+def test_registers_hold_as_many_routing_workgroups_as_the_plan_counts_on():
+    """Two workgroups of eight waves on a compute unit where bf16 rows are routed on the matrix cores without a norm, four waves on
+    each of its SIMDs with 512 registers; one over a quantized router."""
+    asm = assembly("route_exact.hip")
+    registers = {n: (int(r), int(lds)) for n, lds, r in re.findall(
+        r"\.amdhsa_kernel (\S+)\n.*?\.amdhsa_private_segment_fixed_size (\d+)\n.*?\.amdhsa_next_free_vgpr (\d+)\n", asm, re.S)}
+    assert len(registers) == 12
+    for name, (vgprs, scratch) in registers.items():
+        assert scratch == 0, name
+        assert vgprs <= (128 if "ILi32ELi8ELb0E" in name else 256), name
+
+
+@needs_hipcc
 def test_static_scratch_array_is_a_symbol_the_runtime_can_look_up():
     # rbmoe_forward_static's scratch is a static device array whose address the host asks the runtime for by name
     # (hipGetSymbolAddress).  The runtime searches the code object's global symbols, and a missing one ends the

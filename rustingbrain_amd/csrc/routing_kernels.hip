@@ -998,6 +998,26 @@ static size_t rows_lds(const RouterArgs& a, bool exact, int tokens, int EG) {
                  : route_rows_lds_bytes(a.E, a.k, a.d, tokens, NL, EG, a.norm_w != nullptr);
 }
 
+// Calls of more than 16 experts on the matrix cores, which route_exact_kernel takes in any number of rounds otherwise.  Times are
+// forwards of experts of 64, this kernel / the others.
+//   8 tokens (rows of 2300 elements and more): every router row again for eight tokens, which loses once the logits kernel fills the
+//     chip.  d 2560, 32 experts, 9000 rows 169 / 169, 10240 180 / 173, 16384 306 / 267; 64 experts 16384 423 / 387.
+//   quantized, 32 tokens: a workgroup's chain is a round of sums for eight experts after the other, one workgroup on a compute unit, and
+//     as long whether the launch fills the chip or not.  One round of workgroups: d 256, 64 experts, 4100 rows 50.7 / 45.0, 8192 59.3 /
+//     61.8; d 768, 48 experts, 5000 rows 68.4 / 64.1, 5500 69.1 / 71.6; d 1024 74.6 / 71.7, 75.7 / 82.5; d 128, 32 experts 37.7 / 36.4.
+//     More: d 256, 32 experts, 9000 rows 61.2 / 49.1; d 512, 17 experts, 16384 rows 88.0 / 81.4; 32 experts, 12000 rows 75.9 / 66.7, 14500
+//     81.0 / 84.5, 16384 93.4 / 97.7, 30000 145 / 135; d 768, 12000 rows 95.6 / 86.8, 20000 139 / 133, 24000 150 / 166; d 1024, 12000
+//     rows 107 / 100, 20000 163 / 165; d 1280, 9000 rows 117 / 110, 64 experts 127 / 155.
+static bool exact_loses(int d, int E, int tokens, int blocks, bool quantized) {
+    if (E <= 16) return false;
+    if (tokens == kMinRouterTokens) return blocks > 1200;
+    if (!quantized || tokens < kRouterTokens) return false;
+    if (blocks <= 256) return d < 256 || (E > 32 && 4 * blocks < (d < 768 ? 15 : d < 1024 ? 14 : 12) * E);
+    if (d > 1024 && E >= 48) return false;
+    const int places = (blocks + 255) / 256 * 256;  // workgroups of that many rounds: an eighth or a fifth of them may be missing
+    return d < 512 || E <= 24 || (d < 768 && blocks > 512) || (places - blocks) * (d < 896 ? 8 : 5) > places;
+}
+
 static RowsPlan plan_rows(const RouterArgs& a, size_t xsize, bool exact) {
     RowsPlan p;
     const int unit = a.wq ? 32 : 8;  // whole turns of the column lanes, whole 16-byte pieces
@@ -1034,10 +1054,12 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize, bool exact) {
     const int together = p.tokens == kRouterTokens ? 256 * std::min(a_unit, in_lds) : 256;
     // On the matrix cores more than 16 experts in any number of rounds, ahead of a logit a lane and a launch for the rest: us a
     // forward, logits_kernel + router_kernel / route_exact_kernel, 64 experts of 704, d 1024, 16384 rows 672.6 / 651.8, of 64, d 256,
-    // 30000 rows 110.0 / 92.3; 32 of 256, d 1024, 9000 rows 121.9 / 111.9, 16384 195.7 / 181.1; quantized, 64 of 704 751 / 747.  Up to 16 experts a chain less per round outweighs it: 16 of 256, d 768, 16384 rows 112.1 / 111.3, quantized
+    // 30000 rows 110.0 / 92.3; 32 of 256, d 1024, 9000 rows 121.9 / 111.9, 16384 195.7 / 181.1; of 64, d 2048, 16384 rows 304 / 247 (where
+    // not: exact_loses).  Up to 16 experts a chain less per round outweighs it: 16 of 256, d 768, 16384 rows 112.1 / 111.3, quantized
     // 40000 rows 194.7 / 199.3; 8 of 64, d 512, 60000 rows 162.7 / 170.0.
     const bool any_size = p.exact && a.E > 16;
     if (!any_size && ((long long)a.T * a.E > 256 * 1024 || blocks > together)) p.tokens = 0;
+    if (p.exact && exact_loses(a.d, a.E, p.tokens, blocks, a.wq != nullptr)) p.tokens = 0;
     if (p.tokens > kMinRouterTokens && !p.exact && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
     // A few tokens by many experts: one workgroup a block would take the experts' rows through its own LDS one group after the
     // other (64 experts of d 1024: 27 us, whatever the tokens).  So the block's experts are shared out, eight to a workgroup

@@ -85,6 +85,13 @@ LINES = [
     (256, 8, 8192, 1, True), (256, 8, 8193, 1, False), (512, 8, 8193, 1, True), (512, 8, 16384, 1, True), (512, 8, 16385, 1, False),
     # more: any number of rounds
     (256, 17, 9000, 0, True), (1024, 64, 16384, 0, True), (1024, 64, 100000, 0, True), (2048, 64, 16384, 0, True),
+    # ... but not with eight tokens a workgroup in many rounds
+    (3072, 32, 9600, 0, True), (3072, 32, 9601, 0, False),
+    # ... nor under a quantized router with the last round far from full, one round of few workgroups by many experts, short rows
+    (512, 32, 14336, 1, True), (512, 32, 14335 - 31, 1, False), (512, 32, 16385, 1, False), (768, 32, 12000, 1, False),
+    (768, 32, 24000, 1, True), (1024, 32, 20000, 1, True), (1024, 32, 12000, 1, False), (1024, 24, 16384, 1, False),
+    (1280, 32, 9000, 1, False), (1280, 48, 9000, 1, True), (256, 32, 8192, 1, True), (256, 32, 8193, 1, False),
+    (512, 48, 5760, 1, True), (512, 48, 5728, 1, False), (128, 17, 8192, 1, False), (128, 16, 8192, 1, True),
 ]
 
 

@@ -7,25 +7,30 @@ import pytest
 
 import rustingbrain_amd as rb
 from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
+from oracle import rb_oracle as orc
 from rustingbrain_amd import synth
+from test_router_plan import routes_on_matrix_cores
 
 pytestmark = pytest.mark.gpu
 
 SHAPES = [dict(d=64, E=4, k=2, T=1), dict(d=192, E=17, k=2, T=9), dict(d=320, E=16, k=1, T=47), dict(d=64, E=15, k=3, T=2063),
           dict(d=704, E=8, k=2, T=2065), dict(d=192, E=33, k=2, T=4129), dict(d=1024, E=48, k=2, T=2100)]
+OFF_QUANTIZED = [s for s in SHAPES if s["E"] == 33]   # (short rows under a quantized router of many experts: other kernels)
 FORMS = ["plain", "range", "tiny", "huge", "infinite", "f32 router", "tiny router"]
+# (a quantized router holds whole numbers)
+FORMS_AND_ROUTERS = [(form, quantized) for form in FORMS for quantized in (False, True) if not (quantized and "router" in form)]
 
 
-@pytest.mark.parametrize("quantized", [False, True])
-@pytest.mark.parametrize("form", FORMS)
-@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "d{d}_E{E}_k{k}_T{T}".format(**s))
-def test_routing_of_bf16_rows(device, shape, form, quantized):
-    if quantized and "router" in form:
-        pytest.skip("whole numbers")
-    t = synth.make(small_workload(F=64, seed=37, act="bf16", wt="int8", **shape))
+def shape_id(s):
+    return "d{d}_E{E}_k{k}_T{T}".format(**s)
+
+
+def rows_and_router(t, form):
     x, router = t.x.copy(), t.router.copy()
     rows = slice(x.shape[0] // 2, None)          # (the first blocks stay on the matrix cores)
-    if form == "range":                          # the least and the greatest magnitudes that stay there, and zeros
+    if form == "one in a block":                 # ... and a row or two of each of the others leave them
+        x[rows.start::29, 7] = 2.0 ** -80
+    elif form == "range":                          # the least and the greatest magnitudes that stay there, and zeros
         x[rows, ::3] = 2.0 ** -72
         x[rows, 1::3] = -(2.0 ** 80 - 2.0 ** 72)
         x[rows, 2::3] = 0.0
@@ -39,6 +44,10 @@ def test_routing_of_bf16_rows(device, shape, form, quantized):
         router += np.float32(1e-5) * synth.normal(router.shape, 1.0, 37, 5)
     elif form == "tiny router":
         router[0, :8] = 2.0 ** -41
+    return x, router
+
+
+def layers(device, t, router, quantized):
     layer, oracle = gpu_layer(device, t), oracle_layer(t)
     oracle.router = router
     if quantized:
@@ -47,10 +56,50 @@ def test_routing_of_bf16_rows(device, shape, form, quantized):
         oracle.router_q, oracle.router_s = q, s
     else:
         layer.set_router(router)
+    return layer, oracle
+
+
+@pytest.mark.parametrize("form,quantized", FORMS_AND_ROUTERS)
+@pytest.mark.parametrize("shape", SHAPES, ids=shape_id)
+def test_routing_of_bf16_rows(device, shape, form, quantized):
+    t = synth.make(small_workload(F=64, seed=37, act="bf16", wt="int8", **shape))
+    x, router = rows_and_router(t, form)
+    layer, oracle = layers(device, t, router, quantized)
+    # (up to 32 tokens the routing runs beside the products, by the same body)
+    assert shape["T"] <= 32 or routes_on_matrix_cores(**shape, quantized=quantized) != (quantized and shape in OFF_QUANTIZED)
     with np.errstate(all="ignore"):
         ref = oracle.forward(x, threads=8)
     _, cache = layer.forward_train(x, rb.Layout())
     assert_routing_identical(cache, ref)
+    layer.close()
+
+
+# Calls of more than 16 experts in several rounds of workgroups and of more than 256 K pairs, and rounds of 16 and of 8 experts whose
+# router rows follow one another into the same place.
+LARGE = [(dict(d=64, E=64, k=2, T=4200), False), (dict(d=256, E=33, k=3, T=9000), False), (dict(d=1280, E=40, k=2, T=2100), False),
+         (dict(d=1024, E=48, k=2, T=8200), False), (dict(d=1024, E=48, k=2, T=8190), True), (dict(d=1536, E=40, k=2, T=2100), True),
+         (dict(d=512, E=25, k=2, T=14340), True), (dict(d=2048, E=64, k=2, T=300), True)]
+
+
+@pytest.mark.parametrize("form", ["plain", "one in a block", "tiny"])
+@pytest.mark.parametrize("shape,quantized", LARGE, ids=lambda s: shape_id(s) if isinstance(s, dict) else str(s))
+def test_large_calls(device, shape, quantized, form):
+    assert routes_on_matrix_cores(**shape, quantized=quantized)
+    t = synth.make(small_workload(F=64, seed=39, act="bf16", wt="int8", **shape))
+    x, router = rows_and_router(t, form)
+    layer, oracle = layers(device, t, router, quantized)
+    T, E = shape["T"], shape["E"]
+    valid = np.arange(T) % 7 != 3
+    bias = synth.normal((E,), 0.5, 39, 98)
+    ref = oracle.forward(x, valid=valid.astype(np.uint8), router_bias=bias, threads=8)
+    _, cache = layer.forward_train(x, rb.Layout(valid=valid), router_bias=bias)
+    assert_routing_identical(cache, ref)
+    if form == "plain":   # behind a norm, in the launch or in front of it
+        w = (1.0 + 0.1 * synth.normal((shape["d"],), 1.0, 39, 97)).astype(np.float32)
+        layer.set_feed_forward_norm(w, 1e-6)
+        ref = oracle.forward(synth.round_bf16(orc.rmsnorm(x, w, 1e-6)), threads=8)
+        _, cache = layer.forward_block(x)
+        assert_routing_identical(cache, ref)
     layer.close()
 
 

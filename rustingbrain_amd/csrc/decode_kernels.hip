@@ -96,8 +96,10 @@ __device__ __forceinline__ void token_phase_serial(float* row, int t, int E, int
 // index wins, as the reference's strict `>` scan does); a taken expert's key is 0, and so is a NaN's, which the
 // scan never prefers to anything and never replaces once it is the candidate.
 // softmax_rows and route of one token by a group of G lanes (16 or 64), lane j owning expert j: the reductions
-// run through lane-permuting operands and the ordered sum as a lane-shift chain (see softmax_topk in
-// routing_kernels.hip for both), so the phase makes two trips to LDS instead of dozens.
+// run through lane-permuting operands (group_reduce) and the ordered sum as a lane-shift chain, so the phase makes two trips to LDS
+// instead of dozens.  The chain: in every step a lane takes the sum of the lane below (a shift of the whole wave by one lane inside
+// the add) and adds its own exponential, a group's first lane keeps its own, so that after l steps lane l holds ((ex_0 + ex_1) + ...)
+// + ex_l; lanes past the last expert add zeros, and the last lane's sum is the token's.
 template <int G>
 __device__ __forceinline__ void token_phase_lanes(float* row_lds, int t, int j, int E, int k, const uint8_t* valid,
                                                   float* P, float* lse, float* lsev, int* sexp, int* expert_of,
@@ -1259,7 +1261,9 @@ __device__ __forceinline__ void decode_gemm_body(DecodeSide& sd, int fb, float* 
 // products read the call's own rows: a norm in front of the layer is applied on the way (RowForm), f32 rows are rounded.
 // The down product then picks the routed rows out of the per-expert hidden rows (DecodeGemmArgs::a_expert_rows).
 // ---------------------------------------------------------------------------
-constexpr int kFrontTokens = 8;  // a routing workgroup's (1, 2 or 4: the same times, the products take longer than the routing)
+// A routing workgroup's tokens.  (1, 2 or 4: the same times with 8 rows by bf16 weights, where the products take longer than the
+// routing.  Over int8 weights behind a norm the routing is the longer part, 12.8 us of a launch whose products end before; not timed.)
+constexpr int kFrontTokens = 8;
 constexpr int kFrontTeams = 2;   // feature blocks of a product workgroup
 constexpr int kFrontRedFloats = kFrontTeams * 4 * 2 * 16 * kRedPitch;  // a product workgroup's partial sums
 // ... which share their room with the rows' squares of a call behind a norm (d + 4 floats a row; 64: the chain reads ahead)

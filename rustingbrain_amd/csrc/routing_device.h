@@ -584,8 +584,10 @@ __device__ __forceinline__ void route_rows_body(const RouteRowsArgs& a, int blk,
             }
             if (q < quads) multiply(oa);
             // the column lanes folded left to right: lane l of a group holds ((0 + a_0) + a_1) + ... + a_l after l steps
-            // of "take the lane below's sum, add your own" (see softmax_topk), the products side by side: one add a step,
-            // where keeping a group's first lane apart took three instructions (32 column lanes, 8 tokens x 8 experts: 0.5 us)
+            // of "take the lane below's sum, add your own" (a shift of the whole wave by one lane inside the add), the products side
+            // by side.  A group's first lane takes in what the group below hands up, and wrong sums follow from there - one lane
+            // behind the right ones, which nothing overtakes: after NL - 1 steps the last lane's is right.  One add a step, where
+            // keeping a group's first lane apart took three instructions (32 column lanes, 8 tokens x 8 experts: 0.5 us)
             float own[TT][EE];
 #pragma unroll
             for (int u = 0; u < TT; ++u)

@@ -103,13 +103,14 @@ def test_large_calls(device, shape, quantized, form):
     layer.close()
 
 
-@pytest.mark.parametrize("quantized", [False, True])
+@pytest.mark.parametrize("shape,quantized", [(dict(d=1024, E=64, k=2, T=4200), False), (dict(d=1024, E=48, k=2, T=8190), True)])
 @pytest.mark.parametrize("which", ["one", "all"])
-def test_rows_out_of_range_do_not_hold_up_the_others(device, which, quantized):
-    """One tiny element in one row, and one in every row.  A row's exact sums are 2 x 64 x 1024 operations on the vector units instead of
-    the matrix cores, a 32nd of a block's for one of its rows: four times the routing's time is far above either, the fifteen that a
-    whole block's sums took one after the other are far beyond."""
-    t = synth.make(small_workload(d=1024, E=64, k=2, F=64, T=4200, seed=38, act="bf16", wt="int8"))
+def test_rows_out_of_range_do_not_hold_up_the_others(device, which, shape, quantized):
+    """One tiny element in one row, and one in every row.  A row's exact sums are 2 x E x 1024 operations on the vector units instead of
+    the matrix cores: times the routing without any, 1.5 and 3.6 (quantized 1.3 and 2.7), and 16.5 to 18.7 where one element holds up its
+    block's sums, one after the other.  The line lies as many times above the former as below the latter."""
+    assert routes_on_matrix_cores(**shape, quantized=quantized)
+    t = synth.make(small_workload(F=64, seed=38, act="bf16", wt="int8", **shape))
     layer = gpu_layer(device, t)
     if quantized:
         layer.set_router_q8(*synth.quantize_rows(t.router))
@@ -121,5 +122,5 @@ def test_rows_out_of_range_do_not_hold_up_the_others(device, which, quantized):
     plain = routing(t.x)
     x = t.x.copy()
     x[:1 if which == "one" else None, 3] = synth.round_bf16(np.full(1, 1e-30, np.float32))
-    assert routing(x) < 4 * plain
+    assert routing(x) < 8 * plain
     layer.close()

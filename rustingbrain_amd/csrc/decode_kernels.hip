@@ -11,9 +11,11 @@
 // which the layer folds into fewer where the call allows it: the combine into the down launch (the last
 // workgroup of a block of output columns to finish sums it), and - where fetching the untouched experts' weights too
 // costs less than it saves - the routing into the gate/up launch (decode_front_kernel), behind which the down launch has one row of
-// workgroups per expert (decode_down_by_expert_kernel): two launches.  The products are spread over (tile,
+// workgroups per expert (decode_down_by_expert_kernel) or, for a row or two, takes a column block's rows in one workgroup
+// (decode_down_few_kernel): two launches.  The products are spread over (tile,
 // 32-feature block) workgroups whose waves split the reduction dimension, so that a few hundred kilobytes of
 // weight fragments are in flight per CU and every byte of a touched expert is fetched exactly once per 32-row tile.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -1038,6 +1040,163 @@ __global__ __launch_bounds__(512) void decode_down_by_expert_kernel(DecodeGemmAr
     else decode_combine_block_early<bf16_t, true>(g, fb, ce);
 }
 
+// ---------------------------------------------------------------------------
+// decode_down_few_kernel: the down product and the combine of a call of a row or two, without a hand-over between workgroups.
+// A workgroup owns 8 output features and takes every PAIR of a row and a side of it (a slot's expert, or the shared expert), up
+// to four: a 32 x 32 x 16 multiply holds them all, 8 weight rows and one hidden row each (rows 8 j .. 8 j + 7 of one operand,
+// column j of the other; the products of different pairs are dropped), so that a wave fetches whole kilobytes.  The waves
+// split the reduction as in decode_gemm_body and their sums meet in LDS in the same order, so the rows are those of
+// the other down launches bit for bit; the wave that adds them up has all of a token's rows and sums it on the spot.  Expert rows
+// are stored for who asks for them and not waited for.
+// Bound by its chain: the slots' experts, then weights and hidden rows side by side, then the sums.  decode_down_by_expert_kernel
+// requests an expert's weights at once, but its rows go to memory, are counted in and come back to be summed, which takes longer
+// than the one trip; and here nothing is fetched of experts without rows.  us a call, before / now: one row of the default model
+// 12.25 / 11.2, without the norm 11.1 / 10.1; d 768, 8 experts of 1408, two rows 14.9 / 13.65, one row with a shared expert 15.9 /
+// 14.1; int8, d 1024, two rows 16.1 / 15.5.  Behind route_small_kernel 25.4 / 24.8 (one row, 16 experts).
+// As many steps are requested at once as the wave has, and no more (BATCH): with room for 12 where there are 3, the last one
+// asked for over and over, one row of the default model took 12.4.
+// ---------------------------------------------------------------------------
+constexpr int kFewPairs = 4;  // pairs of a call at most
+
+template <bool I8, int BATCH>
+__global__ __launch_bounds__(512) void decode_down_few_kernel(DecodeGemmArgs g, DecodeLayoutArgs t) {
+    constexpr int M = kFewPairs, kRed = 8 * M * 8;
+    __shared__ __align__(16) float red[kRed > kLayoutLdsFloats ? kRed : kLayoutLdsFloats];
+    const int blk = blockIdx.x;
+    if (blk == g.N / 8) return layout_from_memory(red, t);  // (behind decode_front_kernel)
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int T = t.T, k = t.k, S = T * k, P = S + (g.a_shared ? T : 0);
+    const bool front = g.a_expert_rows != 0;  // hidden rows per expert and expert rows by slot, or both by position
+
+    // ---- the pairs of this lane's operands: 8 weight rows of one, the hidden row of one
+    const int a_pair = (lane & 31) >> 3, b_pair = min(lane & 31, M - 1);
+    const int a_expert = t.expert_of[min(a_pair, S - 1)], b_expert = t.expert_of[min(b_pair, S - 1)];
+    const int b_pos = front ? 0 : t.inv_pos[min(b_pair, S - 1)];
+    // what this thread will finish: pair and feature, and as token and feature
+    const int f = tid & 7, n = blk * 8 + f, pair = min(tid >> 3, P - 1), token = min(tid >> 3, T - 1);
+    const int my_expert = t.expert_of[min(pair, S - 1)], my_pos = front ? pair : t.inv_pos[min(pair, S - 1)];
+    int key[M], slot[M];
+    float gate[M];
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        key[q] = t.expert_of[token * k + min(q, k - 1)];
+        gate[q] = g.cmb_gate_of[token * k + min(q, k - 1)];
+    }
+    float residual = 0.0f;
+    if (g.cmb_residual)  // uniform
+        residual = g.cmb_f32 ? static_cast<const float*>(g.cmb_residual)[(size_t)token * g.N + n]
+                             : to_f32(static_cast<const bf16_t*>(g.cmb_residual)[(size_t)token * g.N + n]);
+    float scale_shared = 1.0f;
+    if (I8 && g.a_shared) scale_shared = g.scales_shared[n];
+
+    struct Share {  // this wave's steps of a reduction
+        int first, count, last;
+    };
+    auto share = [&](int K) {
+        const int steps = K / 16, chunk = (steps + 7) / 8;
+        Share s;
+        s.first = min(steps - 1, wave * chunk);  // (a wave without a step: a valid one, not used)
+        s.count = min(chunk, max(steps - wave * chunk, 0));
+        s.last = s.first + max(s.count - 1, 0);
+        return s;
+    };
+    const Share sr = share(g.K), ss = g.a_shared ? share(g.K_shared) : sr;
+    const int most = max(sr.count, ss.count), least = min(sr.count, ss.count);
+    const bool ra = a_pair < S || !g.a_shared, rb = b_pair < S || !g.a_shared;
+    const Share sa = ra ? sr : ss, sb = rb ? sr : ss;
+    const char* const wa = (ra ? static_cast<const char*>(g.w) + (size_t)max(a_expert, 0) * g.w_expert_stride * (I8 ? 1 : 2)
+                               : static_cast<const char*>(g.w_shared)) +
+                           (size_t)(blk >> 2) * (ra ? g.K : g.K_shared) * 32 * (I8 ? 1 : 2) + (half * 32 + (blk & 3) * 8 + (lane & 7)) * 16;
+    const int p = min(b_pair, P - 1);
+    const int row = front ? max(b_expert, 0) * T + p / k : max(b_pos, 0);
+    const bf16_t* const xb = (rb ? static_cast<const bf16_t*>(g.a) + (size_t)row * g.K
+                                 : static_cast<const bf16_t*>(g.a_shared) + (size_t)(p - S) * g.K_shared) + 8 * half;
+    floatx16 acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+    // (a step past a pair's share: a valid address, and zeros in its place)
+    auto batch = [&](const int u0) {
+        uint4 w[BATCH], x[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            x[u] = *reinterpret_cast<const uint4*>(xb + 16 * min(sb.first + u0 + u, sb.last));
+            const int s = min(sa.first + u0 + u, sa.last);
+            if constexpr (I8) {
+                const uint2 v = *reinterpret_cast<const uint2*>(wa + (size_t)(s >> 1) * 1024 + (s & 1) * 8);
+                w[u].x = v.x;
+                w[u].y = v.y;
+            } else {
+                w[u] = *reinterpret_cast<const uint4*>(wa + (size_t)s * 1024);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            if (u0 + u >= most) break;  // uniform
+            bf16x8 wv, xv = __builtin_bit_cast(bf16x8, x[u]);
+            if constexpr (I8) wv = widen_i8(make_uint2(w[u].x, w[u].y));
+            else wv = __builtin_bit_cast(bf16x8, w[u]);
+            if (u0 + u >= least) {  // uniform
+                const bf16x8 zero = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
+                if (u0 + u >= sa.count) wv = zero;
+                if (u0 + u >= sb.count) xv = zero;
+            }
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, xv, acc, 0, 0, 0);
+        }
+    };
+    batch(0);
+    for (int u0 = BATCH; u0 < most; u0 += BATCH) batch(u0);
+    // accumulator element v of lane l: weight row 8 (v / 4) + 4 (l / 32) + v % 4, hidden row l % 32
+    const int j = lane & 31;
+    if (j < M) {
+        float y[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) y[m] = j == 0 ? acc[m] : j == 1 ? acc[4 + m] : j == 2 ? acc[8 + m] : acc[12 + m];
+        *reinterpret_cast<float4*>(red + (wave * M + j) * 8 + 4 * half) = make_float4(y[0], y[1], y[2], y[3]);
+    }
+    // ascending experts; a padding token's slots and the slots past k have no row
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        slot[q] = token * k + q;
+        if (q >= k || key[q] < 0) key[q] = 0x7fffffff;
+    }
+#pragma unroll
+    for (int round = 0; round < M; ++round)
+#pragma unroll
+        for (int q = round & 1; q + 1 < M; q += 2)
+            if (key[q + 1] < key[q]) {
+                const int a = key[q]; key[q] = key[q + 1]; key[q + 1] = a;
+                const int b = slot[q]; slot[q] = slot[q + 1]; slot[q + 1] = b;
+                const float c = gate[q]; gate[q] = gate[q + 1]; gate[q + 1] = c;
+            }
+    const bool routed = pair < S;
+    float scale = scale_shared;
+    if (I8 && wave == 0 && routed) scale = g.scales[(size_t)max(my_expert, 0) * g.s_expert_stride + n];
+    __syncthreads();
+    if (wave != 0) return;
+    float y = red[pair * 8 + f];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) y += red[(w * M + pair) * 8 + f];
+    if constexpr (I8) y *= scale;
+    const uint32_t bits = f32_to_bf16_bits(y);
+    if (tid < 8 * P && (!routed || my_expert >= 0))
+        reinterpret_cast<uint16_t*>(routed ? g.out : g.out_shared)[(size_t)(routed ? my_pos : pair - S) * g.N + n] = (uint16_t)bits;
+    auto row_value = [&](int q) { return __uint_as_float((uint32_t)__shfl((int)bits, (8 * q + f) & 63) << 16); };
+    float sum = 0.0f;
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        const float v = row_value(slot[q]);
+        if (key[q] != 0x7fffffff) sum = __fadd_rn(sum, __fmul_rn(gate[q], v));
+    }
+    if (g.a_shared) sum = __fadd_rn(sum, row_value(S + token));
+    if (g.cmb_residual) sum = __fadd_rn(sum, residual);
+    if (tid < 8 * T) {
+        if (g.cmb_f32) static_cast<float*>(g.cmb_out)[(size_t)token * g.N + n] = sum;
+        else static_cast<bf16_t*>(g.cmb_out)[(size_t)token * g.N + n] = from_f32<bf16_t>(sum);
+    }
+}
+
 // red_raw: TEAMS * NW * (SWIGLU ? 2 : 1) * 16 * kRedPitch floats of LDS; BATCH: reduction steps whose loads a wave issues together.
 // TEAMS > 1: the workgroup is TEAMS teams of NW waves, each with a feature block `fb` of its own (the caller hands
 // every team its block; a team without one has left the kernel before: the barrier below counts the waves that
@@ -1528,6 +1687,31 @@ hipError_t launch_decode_down_by_expert(const DecodeGemmArgs& g, const DecodeLay
     } else {
         return hipErrorInvalidValue;
     }
+    return hipGetLastError();
+}
+
+// Up to four pairs.  (Eight, in two multiplies a step, were slower: two rows of the default model 14.5 against 13.8 us, four rows by
+// 8 experts of 1408 19.2 against 15.0.)  int8 weights behind route_small_kernel stay with the tile table, which requests the weights
+// no later: d 1024, 16 experts of 1408, 3 and 4 rows 30.7 and 31.4 us here, 30.4 and 31.1 there.
+bool decode_down_few_ok(const DecodeGemmArgs& g, WeightKind wk, int T, int k) {
+    const int pairs = T * (k + (g.a_shared ? 1 : 0));
+    if (wk == WeightKind::F32 || (wk == WeightKind::I8 && g.a_expert_rows == 0)) return false;
+    return !g.swiglu && g.cmb_out != nullptr && g.cmb_gate_of != nullptr && (g.a_expert_rows == 0 || g.a_expert_rows == T) && T >= 1 &&
+           g.cmb_T == T && g.cmb_k == k && (!g.a_shared || g.N_shared == g.N) && g.N % 32 == 0 && pairs <= kFewPairs;
+}
+
+hipError_t launch_decode_down_few(const DecodeGemmArgs& g, const DecodeLayoutArgs& t, WeightKind wk, hipStream_t s) {
+    if (!decode_down_few_ok(g, wk, t.T, t.k) || !small_route_ok(t.T, t.E, t.k)) return hipErrorInvalidValue;
+    const dim3 grid(g.N / 8 + (g.a_expert_rows ? 1 : 0));
+    auto go = [&](auto i8_tag) {
+        constexpr bool I8 = decltype(i8_tag)::value;
+        const int K = g.a_shared ? std::max(g.K, g.K_shared) : g.K, steps = (K / 16 + 7) / 8;
+        if (steps <= 3) RB_LAUNCH((decode_down_few_kernel<I8, 3>), grid, dim3(512), 0, s, g, t);
+        else if (steps <= 6) RB_LAUNCH((decode_down_few_kernel<I8, 6>), grid, dim3(512), 0, s, g, t);
+        else RB_LAUNCH((decode_down_few_kernel<I8, 11>), grid, dim3(512), 0, s, g, t);
+    };
+    if (wk == WeightKind::I8) go(std::true_type{});
+    else go(std::false_type{});
     return hipGetLastError();
 }
 

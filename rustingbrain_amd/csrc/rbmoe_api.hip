@@ -1321,9 +1321,14 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
             d2.cmb_T = T; d2.cmb_k = k; d2.cmb_f32 = abf ? 0 : 1;
         }
         // behind the routing-beside-the-products launch the down launch has one row of workgroups per expert, whose weights
-        // go out before anything of the routing is read, and makes the tables beside them
+        // go out before anything of the routing is read, and makes the tables beside them; with a row or two, a workgroup
+        // takes all rows of its columns (`few`)
         const bool by_expert = front && fold && L->decode_down_by_expert && decode_down_by_expert_ok(d2, E, T, k);
-        if (by_expert) {
+        const bool few = fold && L->decode_down_by_expert && decode_down_few_ok(d2, wk, T, k);
+        if (few) {
+            HIP_TRY(ctx, launch_decode_down_few(d2, lay, wk, s));
+            L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return launch_decode_down_few(d2, lay, wk, st); };
+        } else if (by_expert) {
             HIP_TRY(ctx, launch_decode_down_by_expert(d2, lay, wk, s));
             L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return launch_decode_down_by_expert(d2, lay, wk, st); };
         } else {
@@ -1344,7 +1349,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         L->last_T = T;
         L->last = wk_;
         L->last_front = front;
-        L->last_by_slot = by_expert;
+        L->last_by_slot = front && (few || by_expert);
         return RBMOE_OK;
     }
 

@@ -434,5 +434,9 @@ hipError_t launch_decode_layout(const DecodeLayoutArgs& a, hipStream_t s);
 // made beside the products.
 bool decode_down_by_expert_ok(const DecodeGemmArgs& g, int E, int T, int k);
 hipError_t launch_decode_down_by_expert(const DecodeGemmArgs& g, const DecodeLayoutArgs& t, WeightKind wk, hipStream_t s);
+// The same for a call of a row or two, where a workgroup takes all of a column block's rows; also behind launch_route_small
+// (a_expert_rows 0: hidden rows by position, expert rows too, and the tables are there already).
+bool decode_down_few_ok(const DecodeGemmArgs& g, WeightKind wk, int T, int k);
+hipError_t launch_decode_down_few(const DecodeGemmArgs& g, const DecodeLayoutArgs& t, WeightKind wk, hipStream_t s);
 
 }  // namespace rbmoe

@@ -1061,6 +1061,25 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize, bool exact) {
     if (!any_size && ((long long)a.T * a.E > 256 * 1024 || blocks > together)) p.tokens = 0;
     if (p.exact && exact_loses(a.d, a.E, p.tokens, blocks, a.wq != nullptr)) p.tokens = 0;
     if (p.tokens > kMinRouterTokens && !p.exact && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
+    // In several rounds a workgroup's loads, sums and softmax follow one another with nothing beside them where it fills a compute
+    // unit's LDS by itself.  So blocks and router rows are made smaller until two lie there together, if they can be: experts past
+    // those whose rows lie in LDS follow through the place of the ones before, and blocks of 16 tokens take the router's rows twice as
+    // often, which is the smaller loss; and beside a shared expert's products there is room for one of their workgroups.  us a
+    // forward, experts of 64, one workgroup a unit / two: blocks of 32, d 512, 32 experts, 8200, 12000, 20000 rows 54.8 / 48.4, 61.5 / 55.5,
+    // 93.1 / 83.8, 64 experts 67.6 / 59.4, 75.2 / 67.0, 115 / 104; of 16, d 768, 24 experts 63.1 / 59.2, 77.6 / 71.3, 114 / 106, d 1024,
+    // 32 experts 75.7 / 72.9, 93.1 / 87.1, 139 / 130, 64 experts 101 / 91, 115 / 105, 172 / 156; quantized, d 512, 48 experts, 16384 rows
+    // 104 / 91; 64 experts of 704, six a row, and a shared one, d 1024, 16384 rows 658 / 648.  (In one round, 5000 rows: 1 to 2 %,
+    // not taken; narrower rows lie there twice as they are, wider ones do not fit.)
+    if (p.exact && p.tokens == kRouterTokens && blocks > 256 && p.lds > (size_t)kMaxRouterLds / 2)
+        for (int t = p.tokens; t >= std::max(a.min_tokens, p.tokens / 2); t /= 2) {
+            int EG = a.E;
+            while (EG > exact_round(t, NL) && rows_lds(a, true, t, EG) > (size_t)kMaxRouterLds / 2) EG = exact_fewer(EG, t, NL);
+            if (rows_lds(a, true, t, EG) > (size_t)kMaxRouterLds / 2) continue;
+            p.tokens = t;
+            p.EG = EG;
+            p.lds = rows_lds(a, true, t, EG);
+            break;
+        }
     // A few tokens by many experts: one workgroup a block would take the experts' rows through its own LDS one group after the
     // other (64 experts of d 1024: 27 us, whatever the tokens).  So the block's experts are shared out, eight to a workgroup
     // or as many as leave at most one round of workgroups; the last to arrive does the rest.  us a forward, one workgroup / shared

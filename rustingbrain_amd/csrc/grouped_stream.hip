@@ -165,6 +165,8 @@ struct TileOut {
     int rows, row0, tn_idx, N;
     bool act0, act1;      // whether the wave's two row blocks lie inside N
     int r0, r1;           // their first weight rows
+    int t0, blocks;       // the wave's token blocks: the first of them, and how many
+    int column;           // the wave's 32 features in the tile
     const float* sc;      // int8: the expert's scales, one per weight row
     bf16_t* out;
     bf16_t* gu_out;
@@ -190,6 +192,7 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
     const int lhalf = lane >> 5;
     const int rows = o.rows, row0 = o.row0, tn_idx = o.tn_idx, N = o.N, r0 = o.r0, r1 = o.r1;
     const bool act0 = o.act0, act1 = o.act1;
+    const int column = SWIGLU ? o.column : wave;
     const float* const sc = o.sc;
     bf16_t* const out = o.out;
     bf16_t* const gu_out = o.gu_out;
@@ -217,8 +220,8 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
             const int rb = b ? r1 : r0;
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
-                if (t * 32 >= rows) continue;
-                const int m = t * 32 + lrow;
+                if (SWIGLU ? t >= o.blocks : t * 32 >= rows) continue;
+                const int m = (SWIGLU ? o.t0 + t : t) * 32 + lrow;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int f = 8 * q + 4 * lhalf;  // first of 4 consecutive features inside the row block
@@ -237,7 +240,7 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
                             if constexpr (I8) y[i] *= sc[rb + f + i];
                         }
                     }
-                    const int piece = ((wave % WH) * 4 + q) ^ (m & 15);
+                    const int piece = ((column % WH) * 4 + q) ^ (m & 15);
                     *reinterpret_cast<uint2*>(stage + m * 256 + piece * 16 + lhalf * 8) =
                         make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
                 }
@@ -592,7 +595,13 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     // gate/up: gate rows nw .. nw + 31 and the matching up rows; down: rows nw .. nw + 31 and
     // the rows 128 further on, so that each block index covers 128 consecutive features of
     // the workgroup's tile.
-    const int nw = tn_idx * BN + wave * 32;
+    // A last gate/up tile of at most 64 features leaves two waves without any: there the waves share out the token blocks as well,
+    // two blocks of features by two halves of the rows.  us a forward, without / with: 64 experts of 704 (five and a half tiles), six a
+    // row, and a shared one of 1408, d 1024, 16384 rows 648 / 642; 32 of 704, int8, four a row, 8192 rows 205 / 200.
+    const bool halves = SWIGLU && NW == 4 && nblk > 2 && N - tn_idx * BN <= 64;  // uniform over the workgroup
+    const int column = halves ? wave & 1 : wave;
+    const int tb0 = halves ? wave & 2 : 0, tbs = halves ? min(nblk - tb0, 2) : nblk;  // the wave's token blocks
+    const int nw = tn_idx * BN + column * 32;
     const int r0 = nw, r1 = SWIGLU ? N + nw : nw + NW * 32;
     const bool act0 = nw < N;
     const bool act1 = SWIGLU ? act0 : (nw + NW * 32 < N);
@@ -657,18 +666,18 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     // The loop is specialised at compile time for the number of token blocks that hold rows: a run-time branch per
     // block between the multiplies costs far more than the skipped multiplies save.
     {
-        const PipeCtx pc{As, lds0, a_base, wp0, wp1, lane16, lrow, lhalf, lxor, KT};
+        const PipeCtx pc{As + tb0 * 32 * CPR, lds0, a_base, wp0, wp1, lane16, lrow, lhalf, lxor, KT};
         static_assert(TT >= 2 && TT <= 4, "one specialisation per possible block count");
-        if (TT >= 4 && nblk >= 4) pipe_loop<I8, (TT >= 4 ? 4 : TT)>(pc, acc, ring, a_src);
-        else if (TT >= 3 && nblk == 3) pipe_loop<I8, (TT >= 3 ? 3 : TT)>(pc, acc, ring, a_src);
-        else if (nblk == 2) pipe_loop<I8, 2>(pc, acc, ring, a_src);
+        if (TT >= 4 && tbs >= 4) pipe_loop<I8, (TT >= 4 ? 4 : TT)>(pc, acc, ring, a_src);
+        else if (TT >= 3 && tbs == 3) pipe_loop<I8, (TT >= 3 ? 3 : TT)>(pc, acc, ring, a_src);
+        else if (tbs == 2) pipe_loop<I8, 2>(pc, acc, ring, a_src);
         else pipe_loop<I8, 1>(pc, acc, ring, a_src);
     }
     RBMOE_TRACE_AT(blockIdx.x, 2);
     // ---- epilogue -------------------------------------------------------------
     __syncthreads();  // every wave's last DMA has landed and its last fragment reads are done
-    const TileOut to{rows, row0, tn_idx, N, act0, act1, r0, r1, I8 ? scales + (size_t)expert * s_expert_stride : nullptr,
-                     out, gu_out, bw_gu};
+    const TileOut to{rows, row0, tn_idx, N, act0, act1, r0, r1, tb0, tbs, column,
+                     I8 ? scales + (size_t)expert * s_expert_stride : nullptr, out, gu_out, bw_gu};
     if constexpr (!SWIGLU && !I8) {
         if (bw_gu != nullptr) {  // uniform over the launch
             write_swiglu_backward(to, acc, reinterpret_cast<char*>(As));

@@ -33,6 +33,7 @@
 // that lie beyond the end of a group are skipped, so a ragged group costs at
 // most 31 rows of padding.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "layout_device.h"
@@ -49,13 +50,9 @@ namespace rbmoe {
 
 namespace {
 
-#ifndef RBMOE_STREAM_BM
-#define RBMOE_STREAM_BM 128
-#endif
 #ifndef RBMOE_STREAM_OCC
 #define RBMOE_STREAM_OCC 2
 #endif
-constexpr int BM = RBMOE_STREAM_BM;   // token rows per workgroup
 constexpr int BK = 64;    // reduction slice held in one LDS stage
 #ifndef RBMOE_STREAM_NW
 #define RBMOE_STREAM_NW 4
@@ -63,9 +60,10 @@ constexpr int BK = 64;    // reduction slice held in one LDS stage
 constexpr int NW = RBMOE_STREAM_NW;     // waves per workgroup (4, or 8: one activation slice for twice the features)
 constexpr int NT = NW * 64;
 constexpr int CPR = BK / 8;            // 16-byte pieces per LDS row
-constexpr int TT = BM / 32;            // token blocks per wave
 constexpr int KS = BK / 16;            // matrix-core steps per slice
-constexpr int DMA_PER_WAVE = BM * CPR / 64 / NW;  // LDS-DMA instructions per wave per slice
+constexpr int TALL = 5;                // token blocks of a tall tile (see stream_tile_m; four otherwise)
+constexpr int rows_of(int TT) { return 32 * TT; }                           // token rows per workgroup
+constexpr int dma_per_wave(int TT) { return rows_of(TT) * CPR / 64 / NW; }  // LDS-DMA instructions per wave per slice
 constexpr int RING = KS;    // weight-fragment steps in flight per wave (register ring depth)
 constexpr int STAGES = 3;   // LDS stages of one activation slice each
 
@@ -76,6 +74,13 @@ __device__ __forceinline__ bf16x8 lds_frag(const uint4* __restrict__ base, int i
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// A pointer that is the same all over the wave, where the compiler does not see that it is.
+__device__ __forceinline__ const char* scalar_pointer(const char* p) {
+    const unsigned long long v = reinterpret_cast<unsigned long long>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)v), hi = __builtin_amdgcn_readfirstlane((int)(v >> 32));
+    return reinterpret_cast<const char*>(((unsigned long long)hi << 32) | lo);
+}
 
 // Every vector-memory instruction of the main loop is issued from inline assembly and waited
 // for by hand.  Left to the compiler, any wait that falls while an LDS-DMA is in flight
@@ -176,10 +181,10 @@ struct TileOut {
 // `stage`: 32 KiB of LDS that no wave of the workgroup reads or writes any more (the caller has made sure of
 // that with a barrier).  `before_stores()` is called once, when the first pass has been converted and staged and
 // before its first store to memory is issued.
-template <bool SWIGLU, bool I8, typename F>
+template <bool SWIGLU, bool I8, int TT, typename F>
 __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][TT], char* const stage,
                                            F&& before_stores) {
-    constexpr int BN = SWIGLU ? NW * 32 : NW * 64;
+    constexpr int BN = SWIGLU ? NW * 32 : NW * 64, BM = rows_of(TT);
     // The thread index is made opaque here: everything derived from it below (LDS and row offsets, two dozen
     // values per lane) is then worked out where it is used.  Otherwise a caller that writes tile after tile has
     // them computed once, in front of its tile loop, and carried through the main loop in registers that the
@@ -193,6 +198,7 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
     const int rows = o.rows, row0 = o.row0, tn_idx = o.tn_idx, N = o.N, r0 = o.r0, r1 = o.r1;
     const bool act0 = o.act0, act1 = o.act1;
     const int column = SWIGLU ? o.column : wave;
+    const int m0 = (SWIGLU ? o.t0 * 32 : 0) + lrow;  // the row of this lane's tokens in the wave's first block
     const float* const sc = o.sc;
     bf16_t* const out = o.out;
     bf16_t* const gu_out = o.gu_out;
@@ -221,7 +227,6 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
                 if (SWIGLU ? t >= o.blocks : t * 32 >= rows) continue;
-                const int m = (SWIGLU ? o.t0 + t : t) * 32 + lrow;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int f = 8 * q + 4 * lhalf;  // first of 4 consecutive features inside the row block
@@ -240,8 +245,8 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
                             if constexpr (I8) y[i] *= sc[rb + f + i];
                         }
                     }
-                    const int piece = ((column % WH) * 4 + q) ^ (m & 15);
-                    *reinterpret_cast<uint2*>(stage + m * 256 + piece * 16 + lhalf * 8) =
+                    const int piece = ((column % WH) * 4 + q) ^ (lrow & 15);
+                    *reinterpret_cast<uint2*>(stage + m0 * 256 + t * (32 * 256) + piece * 16 + lhalf * 8) =
                         make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
                 }
             }
@@ -280,6 +285,7 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
 // gradients a rounding more than the any-shape kernels' have (3.12e-3 from 64 bits against 2.81e-3).  A pass's
 // pre-activations are requested in front of its barriers: 8192 tokens, d 768, 16 experts top-2 of 1408 take 80 us,
 // 90 with the rounded tile and the requests behind them.
+template <int TT>
 __device__ __forceinline__ void write_swiglu_backward(const TileOut& o, floatx16 (&acc)[2][TT], char* const stage) {
     constexpr int BN = NW * 64;
     int tid = threadIdx.x;
@@ -288,7 +294,7 @@ __device__ __forceinline__ void write_swiglu_backward(const TileOut& o, floatx16
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lrow = lane & 31, lhalf = lane >> 5;
     const int rows = o.rows, row0 = o.row0, N = o.N;
-    constexpr int TURNS = BM * 8 / NT;
+    constexpr int TURNS = rows_of(TT) * 8 / NT;
     typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 #pragma unroll
     for (int bh = 0; bh < NW; ++bh) {
@@ -381,17 +387,17 @@ struct PipeCtx {
     const char* wp0;      // this wave's two blocks of packed weight rows
     const char* wp1;
     uint32_t lane16;
-    int lrow, lhalf, lxor;
+    int lrow, lhalf, lxor;  // this lane's row in the wave's first token block
     int KT;               // slices of the reduction
 };
 
 // Before the call: the DMA of slices 0 and 1 (stages 0 and 1) and the ring loads of steps 0 .. D-1 have been issued
 // and have landed, and the workgroup has met at a barrier.  After it: nothing is outstanding; every wave may
 // still be reading the stages until the next barrier.
-template <bool I8, int NB>
+template <bool I8, int TT, int NB>
 __device__ __forceinline__ void pipe_loop(const PipeCtx& c, floatx16 (&acc)[2][TT], Slot<I8> (&ring)[KS],
-                                          const uint32_t (&a_src)[DMA_PER_WAVE]) {
-    constexpr int D = I8 ? RING : RING - 1;
+                                          const uint32_t (&a_src)[dma_per_wave(TT)]) {
+    constexpr int D = I8 ? RING : RING - 1, BM = rows_of(TT), DMA_PER_WAVE = dma_per_wave(TT);
     static_assert(KS == 4 && RING == 4, "the wait counts below are derived for this configuration");
     const uint4* const As = c.As;
     const uint32_t lds0 = c.lds0, lane16 = c.lane16;
@@ -496,7 +502,7 @@ struct TileAt {
     int tm, tn;
     bool second;
 };
-template <int BN>
+template <int BN, int BM>
 __device__ __forceinline__ TileAt tile_at(int tiles_m, int N, int group_m, int rows2, int N2) {
     int tiles_n = (N + BN - 1) / BN;
     const int total1 = tiles_m * tiles_n;
@@ -528,7 +534,7 @@ struct DenseGroup {
     bf16_t *out, *gu_out;
 };
 
-template <bool SWIGLU, bool I8>
+template <bool SWIGLU, bool I8, int TT>
 __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     const bf16_t* __restrict__ a, const int* __restrict__ row_index, const void* __restrict__ wpacked,
     size_t w_expert_stride_bytes, const float* __restrict__ scales, size_t s_expert_stride, int N, int K,
@@ -536,13 +542,14 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, bf16_t* __restrict__ gu_out,
     const bf16_t* __restrict__ bw_gu, int group_m, DenseGroup g2, RoutedSlots slots) {
     constexpr int BN = SWIGLU ? NW * 32 : NW * 64;  // output features per workgroup
+    constexpr int BM = rows_of(TT), DMA_PER_WAVE = dma_per_wave(TT);
     // LDS stages of one activation slice each; the epilogue reuses the first two as one
-    // 128 x 128 staging tile for the output.
+    // BM x 128 staging tile for the output.
     __shared__ uint4 As[STAGES * BM * CPR];
 
     // without tables: what the router left behind (RoutedSlots), worked out in the stages' room; the rows' tokens lie in the
     // stage that is filled last, behind a barrier
-    const bool own = SWIGLU && slots.expert_of != nullptr;  // uniform over the launch
+    const bool own = SWIGLU && TT < TALL && slots.expert_of != nullptr;  // uniform over the launch
     SlotsLds& sl = *reinterpret_cast<SlotsLds*>(As);
     static_assert(sizeof(SlotsLds) <= (STAGES - 1) * BM * CPR * sizeof(uint4), "in front of the tokens");
     int* const own_token = reinterpret_cast<int*>(As + (STAGES - 1) * BM * CPR);
@@ -551,7 +558,7 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
         if (blockIdx.x == gridDim.x - 1) return routed_rest(slots, reinterpret_cast<unsigned char*>(As));
         rc = routed_counts<NT>(slots, sl);
     }
-    const TileAt at = tile_at<BN>(own ? rc.ntiles : dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
+    const TileAt at = tile_at<BN, BM>(own ? rc.ntiles : dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
     if (at.tm < 0) return;
     const int tm_idx = at.tm, tn_idx = at.tn;
     if (at.second) {
@@ -600,15 +607,16 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     // row, and a shared one of 1408, d 1024, 16384 rows 648 / 642; 32 of 704, int8, four a row, 8192 rows 205 / 200.
     const bool halves = SWIGLU && NW == 4 && nblk > 2 && N - tn_idx * BN <= 64;  // uniform over the workgroup
     const int column = halves ? wave & 1 : wave;
-    const int tb0 = halves ? wave & 2 : 0, tbs = halves ? min(nblk - tb0, 2) : nblk;  // the wave's token blocks
+    // the wave's token blocks
+    const int half = (nblk + 1) / 2, tb0 = halves ? (wave >> 1) * half : 0, tbs = halves ? min(half, nblk - tb0) : nblk;
     const int nw = tn_idx * BN + column * 32;
     const int r0 = nw, r1 = SWIGLU ? N + nw : nw + NW * 32;
     const bool act0 = nw < N;
     const bool act1 = SWIGLU ? act0 : (nw + NW * 32 < N);
     const size_t block_bytes = (size_t)K * 32 * (I8 ? 1 : 2);  // one block of 32 weight rows over all of K
     const char* wexp = static_cast<const char*>(wpacked) + (size_t)expert * w_expert_stride_bytes;
-    const char* wp0 = wexp + (size_t)(act0 ? r0 / 32 : 0) * block_bytes;
-    const char* wp1 = wexp + (size_t)(act1 ? r1 / 32 : 0) * block_bytes;
+    const char* wp0 = scalar_pointer(wexp + (size_t)(act0 ? r0 / 32 : 0) * block_bytes);
+    const char* wp1 = scalar_pointer(wexp + (size_t)(act1 ? r1 / 32 : 0) * block_bytes);
     const uint32_t lane16 = (uint32_t)lane * 16u;
 
     // ---- LDS-DMA of the activation slice --------------------------------------
@@ -666,12 +674,13 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     // The loop is specialised at compile time for the number of token blocks that hold rows: a run-time branch per
     // block between the multiplies costs far more than the skipped multiplies save.
     {
-        const PipeCtx pc{As + tb0 * 32 * CPR, lds0, a_base, wp0, wp1, lane16, lrow, lhalf, lxor, KT};
-        static_assert(TT >= 2 && TT <= 4, "one specialisation per possible block count");
-        if (TT >= 4 && tbs >= 4) pipe_loop<I8, (TT >= 4 ? 4 : TT)>(pc, acc, ring, a_src);
-        else if (TT >= 3 && tbs == 3) pipe_loop<I8, (TT >= 3 ? 3 : TT)>(pc, acc, ring, a_src);
-        else if (tbs == 2) pipe_loop<I8, 2>(pc, acc, ring, a_src);
-        else pipe_loop<I8, 1>(pc, acc, ring, a_src);
+        const PipeCtx pc{As, lds0, a_base, wp0, wp1, lane16, tb0 * 32 + lrow, lhalf, lxor, KT};
+        static_assert(TT >= 4 && TT <= 5, "one specialisation per possible block count");
+        if (TT >= 5 && tbs >= 5) pipe_loop<I8, TT, (TT >= 5 ? 5 : TT)>(pc, acc, ring, a_src);
+        else if (tbs >= 4) pipe_loop<I8, TT, 4>(pc, acc, ring, a_src);
+        else if (tbs == 3) pipe_loop<I8, TT, 3>(pc, acc, ring, a_src);
+        else if (tbs == 2) pipe_loop<I8, TT, 2>(pc, acc, ring, a_src);
+        else pipe_loop<I8, TT, 1>(pc, acc, ring, a_src);
     }
     RBMOE_TRACE_AT(blockIdx.x, 2);
     // ---- epilogue -------------------------------------------------------------
@@ -680,12 +689,12 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
                      I8 ? scales + (size_t)expert * s_expert_stride : nullptr, out, gu_out, bw_gu};
     if constexpr (!SWIGLU && !I8) {
         if (bw_gu != nullptr) {  // uniform over the launch
-            write_swiglu_backward(to, acc, reinterpret_cast<char*>(As));
+            write_swiglu_backward<TT>(to, acc, reinterpret_cast<char*>(As));
             RBMOE_TRACE_AT(blockIdx.x, 3);
             return;
         }
     }
-    write_tile<SWIGLU, I8>(to, acc, reinterpret_cast<char*>(As), [] {});
+    write_tile<SWIGLU, I8, TT>(to, acc, reinterpret_cast<char*>(As), [] {});
     RBMOE_TRACE_AT(blockIdx.x, 3);
 }
 
@@ -706,6 +715,8 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
 // kt waits for it behind its step KS - 2, seven ring loads and the DMA of slice kt + 2 are younger.
 constexpr int NRING = 16;
 constexpr int NSTAGES = 4;
+constexpr int TT = 4, BM = rows_of(TT), DMA_PER_WAVE = dma_per_wave(TT);  // (this kernel's tiles are never tall)
+static_assert(BM == kStreamTileM, "");
 
 template <bool I8>
 struct Slot1;
@@ -830,7 +841,7 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
         if (blockIdx.x == gridDim.x - 1) return routed_rest(slots, reinterpret_cast<unsigned char*>(As));
         rc = routed_counts<NT>(slots, sl);
     }
-    const TileAt at = tile_at<BN>(own ? rc.ntiles : dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
+    const TileAt at = tile_at<BN, BM>(own ? rc.ntiles : dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
     if (at.tm < 0) return;
     const int tm_idx = at.tm, tn_idx = at.tn;
     if (at.second) {
@@ -993,9 +1004,11 @@ constexpr int narrow_tiles(bool swiglu, int K) { return swiglu ? 128 : K <= 512 
 template <bool SWIGLU, bool I8>
 hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
     constexpr int BN = SWIGLU ? NW * 32 : NW * 64;
-    const int tiles_m = g.dense_rows >= 0 ? (g.dense_rows + BM - 1) / BM : g.max_tiles;
     const GroupedArgs::Dense& d2 = g.dense2;
-    auto tiles = [&](int m, int bn) { return m * ((g.N + bn - 1) / bn) + (d2.rows + BM - 1) / BM * ((d2.N + bn - 1) / bn); };
+    const bool tall = g.dense_rows < 0 && g.tile_m == rows_of(TALL);
+    const int bm = tall ? rows_of(TALL) : BM;
+    const int tiles_m = g.dense_rows >= 0 ? (g.dense_rows + bm - 1) / bm : g.max_tiles;
+    auto tiles = [&](int m, int bn) { return m * ((g.N + bn - 1) / bn) + (d2.rows + bm - 1) / bm * ((d2.N + bn - 1) / bn); };
     const int total = tiles(tiles_m, BN);
     if (total <= 0) return hipSuccess;
     const DenseGroup g2{static_cast<const bf16_t*>(d2.a), d2.w, d2.scales, d2.N, d2.K, d2.rows,
@@ -1003,25 +1016,48 @@ hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
     const int group_m = g.group_m > 0 ? g.group_m : 8;
     const int rest = SWIGLU && g.slots.expert_of ? 1 : 0;  // (routed_rest)
     const int likely = g.dense_rows < 0 && g.likely_tiles > 0 ? tiles(g.likely_tiles, BN) : total;
-    if (likely <= narrow_tiles(SWIGLU, g.K) && !g.gu_out && !g.swiglu_grad_gu) {
+    if (!tall && likely <= narrow_tiles(SWIGLU, g.K) && !g.gu_out && !g.swiglu_grad_gu) {
         RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((tiles(tiles_m, BN / 2) + 7) / 8 * 8 + rest), dim3(NT), 0, s,
                   static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
                   g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
                   static_cast<bf16_t*>(g.out), group_m, g2, g.slots);
         return hipGetLastError();
     }
-    RB_LAUNCH((grouped_stream_kernel<SWIGLU, I8>), dim3((total + 7) / 8 * 8 + rest), dim3(NT), 0, s,
-              static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
-              g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
-              static_cast<bf16_t*>(g.out), static_cast<bf16_t*>(g.gu_out), static_cast<const bf16_t*>(g.swiglu_grad_gu),
-              group_m, g2, g.slots);
+    auto go = [&](auto tt) {
+        RB_LAUNCH((grouped_stream_kernel<SWIGLU, I8, decltype(tt)::value>), dim3((total + 7) / 8 * 8 + rest), dim3(NT), 0, s,
+                  static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
+                  g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
+                  static_cast<bf16_t*>(g.out), static_cast<bf16_t*>(g.gu_out), static_cast<const bf16_t*>(g.swiglu_grad_gu),
+                  group_m, g2, g.slots);
+    };
+    if (tall) go(std::integral_constant<int, TALL>{});
+    else go(std::integral_constant<int, TT>{});
     return hipGetLastError();
 }
 
 
 }  // namespace
 
-int stream_tile_m() { return BM; }
+// Rows of the tiles of a call of so many routed rows: 128, or 160 (TALL).  A tall tile takes 1.19 times as long for 1.25 times the
+// rows: a wave's weight fragments, which are two thirds of what passes a compute unit's L1, serve five multiplies instead of four, and
+// there are fewer first loads and last stores.  Against that, launches end in whole tiles, and one table serves both products.  So
+// the lengths are estimated - tiles a compute unit, 0.3 of the way to the next whole number, by the tile's reduction and 800 columns
+// for its ends - and the tall tiles taken where they gain 1 %, above the sizes that the narrow kernel, a shared expert in the
+// launch and gate/up launches that make the tables take.  us a forward, 128 / 160, measured (estimated gain): d 768, 8 experts of 1408, 6000
+// rows 113.2 / 108.1 (8 %), 10000 155.7 / 157.6 (1 %, not taken), 16384 235.3 / 224.2 (7 %); 16 of them, 6000 121.2 / 112.7 (8 %),
+// 16384 251.4 / 246.1 (4 %); d 512, 8 of 352, 16384 90.5 / 83.4 (9 %); d 1024, 32 of 1408, four a row, 6000 256.6 / 244.8 (2 %),
+// 16384 592 / 567 (4 %); 64 of 704, six a row, 6000 237.7 / 231.0 (2 %), 16384 522 / 508 (3 %); d 256, 32 of 704, four a row, 10000 104.1 /
+// 104.7 (3 %), 16384 143.9 / 135.9 (5 %).  Not taken: d 1024, 32 of 352, four a row, 10000 164.9 / 167.3, d 512, 8 of 1408, 6000 88.9 / 89.6.
+int stream_tile_m(int rows, int groups, int F, int d) {
+    auto tiles = [&](int bm) { return std::max((double)rows / bm + 0.5 * groups, (double)std::min(groups, rows)); };
+    const int gate_up = (F + 127) / 128, down = (d + 255) / 256;
+    if (tiles(BM) * gate_up <= 768) return BM;
+    auto length = [&](int bm) {
+        auto units = [&](double n) { return n <= 256 ? 1.0 : 0.3 * std::ceil(n / 256) + 0.7 * n / 256; };
+        return (d + 800) * units(tiles(bm) * gate_up) + (F + 800) * units(tiles(bm) * down);
+    };
+    return length(BM) > 1.01 * 1.19 * length(rows_of(TALL)) ? rows_of(TALL) : BM;
+}
 
 // K a multiple of 64 (one LDS slice), N a multiple of 32 (row blocks of the packed weights)
 bool stream_shape_ok(int N, int K) { return K % 64 == 0 && K >= 64 && N % 32 == 0 && N >= 32; }
@@ -1031,6 +1067,7 @@ hipError_t launch_grouped_stream(const GroupedArgs& g, WeightKind wk, hipStream_
     if (g.dense2.rows > 0 && (!stream_shape_ok(g.dense2.N, g.dense2.K) || !g.dense2.gu_out != !g.gu_out || g.swiglu_grad_gu))
         return hipErrorInvalidValue;
     if (g.slots.expert_of && (!g.swiglu || g.dense_rows >= 0 || g.slots.layout.tile_m != BM)) return hipErrorInvalidValue;
+    if (g.dense_rows < 0 && g.tile_m != BM && g.tile_m != rows_of(TALL)) return hipErrorInvalidValue;
     if (g.swiglu_grad_gu && (g.swiglu || wk != WeightKind::BF16)) return hipErrorInvalidValue;
     if (wk == WeightKind::BF16) return g.swiglu ? launch_t<true, false>(g, s) : launch_t<false, false>(g, s);
     if (wk == WeightKind::I8) return g.swiglu ? launch_t<true, true>(g, s) : launch_t<false, true>(g, s);

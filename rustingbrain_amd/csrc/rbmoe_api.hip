@@ -1158,7 +1158,9 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
 
     const bool mfma = L->use_stream;
     const bool f32mc = L->use_f32_mc;
-    const int tile_m0 = mfma ? stream_tile_m() : (L->f32_rows ? f32_tile_m(T * k, E) : kGenericTileM);
+    // (training: no gain from tall tiles where gate/up also stores the pre-activations)
+    const int tile_m0 = mfma ? (L->training ? kStreamTileM : stream_tile_m(T * k, E, F, d))
+                             : (L->f32_rows ? f32_tile_m(T * k, E) : kGenericTileM);
     L->last_tile_m = tile_m0;
     L->kernel_name = mfma ? (wk == WeightKind::I8 ? "mfma_bf16_stream_int8w" : "mfma_bf16_stream")
                           : (f32mc ? "mfma_f32" : "generic");
@@ -1408,7 +1410,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // (600) 79.6 / 86.2; d 768, 8 of 1408, 256 rows 43.2 / 63.2, 2048 (616) 76.5 / 80.4, 4096 (1144) 112.0 / 111.2; d 1024,
     // 64 of 704, six a row, 1000 rows 126.5 / 139.0, 2048 (1136) 164.5 / 154.0.
     constexpr int kSharedInsideTiles = 768;
-    const int gate_up_tiles = ((T * k) / tile_m0 + E) * ((F + 127) / 128) + (T + 127) / 128 * ((Fs + 127) / 128);
+    const int gate_up_tiles = ((T * k) / kStreamTileM + E) * ((F + 127) / 128) + (T + 127) / 128 * ((Fs + 127) / 128);
     // Over f32 rows (their kernels have tiles of 64 x 128 where a launch is large) the same below 1024 rows, and up to 400 such
     // tiles: us a step, inside / one behind the other (from 1024 rows on beside), d 512, 8 of 352, bf16 weights, 4 rows 32.6 /
     // 44.1, 512 39.2 / 49.7, 1024 (156 tiles) 45.8 / 61.2, 2048 (300) 63.1 / 72.0; f32 weights, 200 rows 35.2 / 50.3, 2048 84.1 / 83.0,
@@ -2748,6 +2750,9 @@ int rbmoe_internal_router_slice(int32_t d, int32_t E, int32_t k, int32_t T, int3
     a.arrive = reinterpret_cast<int*>((uintptr_t)1 << 20);
     return plan_router(a, bf16 != 0).row_slice;
 }
+
+// Test hook (not part of rbmoe.h), runs without a GPU: rows of the tiles of a matrix-core call of so many routed rows.
+int rbmoe_internal_stream_tile(int32_t rows, int32_t E, int32_t F, int32_t d) { return stream_tile_m(rows, E, F, d); }
 
 int rbmoe_copy_device(rbmoe_ctx* ctx, void* dst, const void* src, size_t bytes) {
     if (!ctx) return fail(nullptr, RBMOE_NULL_POINTER, "ctx is NULL");

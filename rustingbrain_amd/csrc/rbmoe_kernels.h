@@ -253,7 +253,8 @@ constexpr int kGenericTileM = 16;
 // bf16 matrix-core path (bf16 activations; bf16 or int8 weights): weights repacked into
 // matrix-core operand order (pack_weight_*) and streamed global -> registers, activations
 // global -> LDS by DMA.  `w` must have been packed matrix by matrix.
-int stream_tile_m();
+constexpr int kStreamTileM = 128;
+int stream_tile_m(int rows, int groups, int F, int d);  // rows of the tile table's tiles for so many routed rows: 128 or 160
 bool stream_shape_ok(int N, int K);
 hipError_t launch_grouped_stream(const GroupedArgs& a, WeightKind wk, hipStream_t s);
 void pack_weight_bf16(const uint16_t* src, int rows, int cols, uint16_t* dst);

@@ -75,7 +75,8 @@ struct XPiece<float> {
 // WIDE (bf16 rows): the rows are widened to f32 once, on their way into LDS, instead of by each of the NE waves
 // that read them (one of the three vector instructions per element); a slice is then half as many columns, so
 // that a workgroup takes no more LDS and as many of them fit a compute unit.  So it is for f32 rows in launches of many
-// workgroups: four on a compute unit instead of two (64 experts of 704, d 1024, 16384 f32 rows 823.7 -> 803 us a forward).
+// workgroups: four on a compute unit instead of two (64 experts of 704, d 1024, 16384 f32 rows 823.7 -> 803 us a forward, while
+// those were routed here).
 // NL = 32: the logits of a quantized router, in the order of dot_lanes::<32> (src/quantized.rs:154-177): lanes[c % 32] +=
 // x[c] * f32(q[c]), the scalar rest from the last multiple of 32 on, and the whole times the row's `scale` (:61).  `wr` then
 // holds the int8 weights widened once, at their upload: a whole number in f32 is fetched like any other router weight.
@@ -1057,7 +1058,16 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize, bool exact) {
     // 30000 rows 110.0 / 92.3; 32 of 256, d 1024, 9000 rows 121.9 / 111.9, 16384 195.7 / 181.1; of 64, d 2048, 16384 rows 304 / 247 (where
     // not: exact_loses).  Up to 16 experts a chain less per round outweighs it: 16 of 256, d 768, 16384 rows 112.1 / 111.3, quantized
     // 40000 rows 194.7 / 199.3; 8 of 64, d 512, 60000 rows 162.7 / 170.0.
-    const bool any_size = p.exact && a.E > 16;
+    // So do f32 rows on the vector units: a thread's tile of tokens and experts reads LDS once for several products, where the other
+    // kernels read it for each and take the rows once for every eight experts.  us a forward, experts of 64, the others / this one:
+    // d 256, 32 experts, 8500 rows 64.5 / 52.3, 30000 128 / 90; 64 experts, 4500 rows 62.1 / 50.2, 8192 82.8 / 54.7; d 512, 32 experts,
+    // 8500 rows 94.6 / 71.2, 48 experts, 16384 160 / 113; d 768, 32 experts, 12000 rows 137 / 108, 64 experts, 8192 170 / 92; d 1024, 32
+    // experts, 4500 rows 115 / 82, 64 experts, 16384 337 / 248; d 2048, 32 experts, 12000 rows 316 / 308; quantized, d 768, 32 experts,
+    // 16384 rows 184 / 155, d 1024, 64 experts, 8500 rows 220 / 164.  Not where route_fused_kernel has long rows: d 768, 20 experts,
+    // 12000 rows 93.5 / 97.4, d 1024, 24 experts, 8500 rows 105 / 113 (d 512, 20 experts, 8500 rows 65.7 / 65.5).  Up to 16 experts as
+    // above: d 768, 16 experts, 16384 rows 123 / 133.
+    const bool any_f32 = !p.exact && xsize == 4 && a.E > 16 && (a.wq || a.d <= 512 || fused_cols(a, xsize) == 0);
+    const bool any_size = (p.exact && a.E > 16) || any_f32;
     if (!any_size && ((long long)a.T * a.E > 256 * 1024 || blocks > together)) p.tokens = 0;
     if (p.exact && exact_loses(a.d, a.E, p.tokens, blocks, a.wq != nullptr)) p.tokens = 0;
     if (p.tokens > kMinRouterTokens && !p.exact && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
@@ -1070,14 +1080,18 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize, bool exact) {
     // 32 experts 75.7 / 72.9, 93.1 / 87.1, 139 / 130, 64 experts 101 / 91, 115 / 105, 172 / 156; quantized, d 512, 48 experts, 16384 rows
     // 104 / 91; 64 experts of 704, six a row, and a shared one, d 1024, 16384 rows 658 / 648.  (In one round, 5000 rows: 1 to 2 %,
     // not taken; narrower rows lie there twice as they are, wider ones do not fit.)
-    if (p.exact && p.tokens == kRouterTokens && blocks > 256 && p.lds > (size_t)kMaxRouterLds / 2)
+    // f32 rows: d 512, 32 experts of 256, 12000 rows 93.9 / 88.1; d 1024, 64 experts of 704, six a row, 6000 rows 300 / 285, 16384 635 / 627,
+    // but 32 experts of 256, 12000 rows 165.4 / 171.1.
+    if (((p.exact && p.tokens == kRouterTokens) || (any_f32 && p.tokens)) && blocks > 256 && p.lds > (size_t)kMaxRouterLds / 2)
         for (int t = p.tokens; t >= std::max(a.min_tokens, p.tokens / 2); t /= 2) {
+            const int least = p.exact ? exact_round(t, NL) : 8;
             int EG = a.E;
-            while (EG > exact_round(t, NL) && rows_lds(a, true, t, EG) > (size_t)kMaxRouterLds / 2) EG = exact_fewer(EG, t, NL);
-            if (rows_lds(a, true, t, EG) > (size_t)kMaxRouterLds / 2) continue;
+            while (EG > least && rows_lds(a, p.exact, t, EG) > (size_t)kMaxRouterLds / 2)
+                EG = p.exact ? exact_fewer(EG, t, NL) : (EG - 1) & ~1;
+            if (rows_lds(a, p.exact, t, EG) > (size_t)kMaxRouterLds / 2) continue;
             p.tokens = t;
             p.EG = EG;
-            p.lds = rows_lds(a, true, t, EG);
+            p.lds = rows_lds(a, p.exact, t, EG);
             break;
         }
     // A few tokens by many experts: one workgroup a block would take the experts' rows through its own LDS one group after the

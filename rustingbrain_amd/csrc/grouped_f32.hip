@@ -158,6 +158,7 @@ struct F32Dense {
     float *out, *gu_out;
 };
 
+// `parts`: GroupedArgs::parts (DMA, plain launches; otherwise 1).
 // `sub`: this kernel's tiles in one of the tile table's, 1 or 2.  TB = blocks of 32 token rows per workgroup; FW = waves along the features (the workgroup owns 32 FW of them, or with
 // SWIGLU as many gate and up rows each), STEPS = steps of 16 reduction columns a wave takes of a slice.  DMA: rows of whole
 // 16-byte pieces on 16-byte boundaries and whole slices; otherwise both operands travel element by element.
@@ -166,7 +167,8 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     const float* __restrict__ a, const int* __restrict__ row_index, const WT* __restrict__ w, size_t w_expert_stride,
     const float* __restrict__ scales, size_t s_expert_stride, int N, int K, const int* __restrict__ tile_expert,
     const int* __restrict__ tile_row0, const int* __restrict__ tile_rows, const int* __restrict__ ntiles, int sub, int dense_rows,
-    float* __restrict__ out, float* __restrict__ gu_out, const float* __restrict__ bw_gu, F32Dense<WT> g2, RoutedSlots slots) {
+    float* __restrict__ out, float* __restrict__ gu_out, const float* __restrict__ bw_gu, int parts, int part_rows, F32Dense<WT> g2,
+    RoutedSlots slots) {
     typedef Weights<WT> W;
     constexpr int NTH = NW * 64;
     constexpr int KG = NW / FW;                   // wave groups that share out a slice's steps
@@ -203,12 +205,14 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     int tiles_m = dense_rows >= 0 ? (dense_rows + BM - 1) / BM : (own ? rc.ntiles : *ntiles) * sub;
     const int total1 = tiles_m * tiles_n;
     const int tiles_n2 = (g2.N + FN - 1) / FN, tiles_m2 = (g2.rows + BM - 1) / BM;
-    const int total = total1 + tiles_m2 * tiles_n2;
+    const int whole = total1 + tiles_m2 * tiles_n2, total = SWIGLU ? whole : whole * parts;
     const int per_xcd = (total + 7) / 8;
     const int local = blockIdx.x >> 3;
     if (local >= per_xcd) return;
     int pid = (blockIdx.x & 7) * per_xcd + local;
     if (pid >= total) return;
+    const int part = SWIGLU || parts == 1 ? 0 : pid / whole;  // (uniform over the workgroup, like all of this)
+    pid -= part * whole;
     const bool second = pid >= total1;
     if (second) {  // (uniform over the workgroup)
         pid -= total1;
@@ -223,6 +227,15 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
         dense_rows = g2.rows;
         out = g2.out;
         gu_out = g2.gu_out;
+        part_rows = g2.rows;
+    }
+    const int pitch = K;  // of the rows of both operands
+    if (DMA && !SWIGLU && parts > 1) {  // this workgroup's slices
+        const int from = K / SK * part / parts * SK, to = K / SK * (part + 1) / parts * SK;
+        a += from;
+        w += from;
+        K = to - from;
+        out += (size_t)part * part_rows * N;
     }
     constexpr int GROUP_M = 8;
     const int per_group = GROUP_M * tiles_n;
@@ -262,12 +275,12 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     // (rows past the end of the group, features past N: any valid one, products never stored)
     auto token_row = [&](int r) {
         const int rr = r < rows ? r : 0;
-        return a + (size_t)(own_rows ? own_token[skip + rr] : row_index ? row_index[row0 + rr] : row0 + rr) * K;
+        return a + (size_t)(own_rows ? own_token[skip + rr] : row_index ? row_index[row0 + rr] : row0 + rr) * pitch;
     };
     auto weight_row = [&](int q) {  // q < FN: gate (or plain) feature n0 + q; q >= FN: the matching up row
         const int feat = n0 + (q % FN);
         const int fr = feat < N ? feat : 0;
-        return wbase + (size_t)((SWIGLU && q >= FN) ? N + fr : fr) * K;
+        return wbase + (size_t)((SWIGLU && q >= FN) ? N + fr : fr) * pitch;
     };
 
     // ---- staging
@@ -804,6 +817,23 @@ int f32_workgroups(const GroupedArgs& g, WeightKind wk) {
     return f32_plan(g, wk == WeightKind::F32 ? 4 : wk == WeightKind::BF16 ? 2 : 1).workgroups;
 }
 
+// A tile's chain of slices is what a small down launch waits for, so its reduction is shared out until there is a workgroup for
+// every compute unit: in halves or quarters, whose sums the combine adds up.  us a forward, whole / 2 parts / 4 parts, f32 weights: d 512,
+// 8 experts of 1408, 1 row (32 tiles) 32.8 / 29.2 / 28.0, 2 rows (64) 32.8 / 29.8 / 27.9, 8 rows (128) 36.6 / 33.2 / 33.8, 64 rows 37.7 /
+// 35.0 / 35.5; d 256, 4 experts of 1408, all four a row, 20 rows (32) 32.5 / 29.1 / 28.1; d 768, 8 of 1408 and a shared one, 2 rows (120)
+// 36.6 / 33.8 / 35.0, 16 rows (216) 42.4 / 42.8 / 44.2.  A second workgroup on some of the compute units takes back what the shorter
+// chain gives: d 512, 8 of 1408, 1024 rows (144) 94.5 / 101.1 / 98.5.
+// Errors against 64 bits become smaller (d 512, 8 of 1408, 1 row 4.0e-7 / 3.1e-7, 64 rows 4.7e-7 / 4.2e-7).  What is taken again (see
+// `odd`) is so part by part: infinities and NaN meet in the combine's sum as they would in the whole one.
+int f32_parts(const GroupedArgs& g, WeightKind wk) {
+    const F32Plan p = f32_plan(g, wk == WeightKind::F32 ? 4 : wk == WeightKind::BF16 ? 2 : 1);
+    const int slice = p.tile == F32Tile::T32x32 ? 64 : 32, K = g.dense2.rows > 0 ? std::min(g.K, g.dense2.K) : g.K;
+    if (!p.aligned || g.K % slice != 0 || (g.dense2.rows > 0 && g.dense2.K % slice != 0)) return 1;
+    int parts = 1;
+    while (parts < 4 && 2 * parts * p.workgroups <= 256 && 2 * parts * slice <= K) parts *= 2;
+    return parts;
+}
+
 // Whole slices of both down products, or of neither: the routed experts' kernel stays the one they have by themselves.
 bool f32_joins(int F, int Fs) { return F == Fs || (F % 64 == 0 && Fs % 64 == 0); }
 
@@ -818,12 +848,13 @@ static hipError_t launch_f32_t(const GroupedArgs& g, hipStream_t s) {
     const GroupedArgs::Dense& d2 = g.dense2;
     const F32Dense<WT> g2{static_cast<const float*>(d2.a), static_cast<const WT*>(d2.w), d2.scales, d2.N, d2.K, d2.rows,
                           static_cast<float*>(d2.out), static_cast<float*>(d2.gu_out)};
+    bool refused = false;
     auto go = [&](auto swiglu_tag, auto nw_tag, auto tb_tag, auto fw_tag, auto steps_tag) {
         constexpr bool SW = decltype(swiglu_tag)::value;
         constexpr int FW = decltype(fw_tag)::value, FN = 32 * FW, BM = 32 * decltype(tb_tag)::value;
         constexpr int NW = decltype(nw_tag)::value, STEPS = decltype(steps_tag)::value;
         const int tiles_m = g.dense_rows >= 0 ? (g.dense_rows + BM - 1) / BM : g.max_tiles * (g.tile_m / BM);
-        const int total = (g.N + FN - 1) / FN * tiles_m + (d2.N + FN - 1) / FN * ((d2.rows + BM - 1) / BM);
+        const int total = ((g.N + FN - 1) / FN * tiles_m + (d2.N + FN - 1) / FN * ((d2.rows + BM - 1) / BM)) * g.parts;
         if (total <= 0) return;
         const int rest = SW && g.slots.expert_of ? 1 : 0;  // (routed_rest)
         const int sub = g.tile_m / BM;
@@ -831,11 +862,12 @@ static hipError_t launch_f32_t(const GroupedArgs& g, hipStream_t s) {
             RB_LAUNCH((grouped_f32_kernel<WT, SW, NW, BM / 32, FW, STEPS, decltype(dma_tag)::value>), dim3((total + 7) / 8 * 8 + rest),
                       dim3(64 * NW), 0, s, static_cast<const float*>(g.a), g.row_index, static_cast<const WT*>(g.w), g.w_expert_stride,
                       g.scales, g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, sub, g.dense_rows,
-                      static_cast<float*>(g.out), static_cast<float*>(g.gu_out), static_cast<const float*>(g.swiglu_grad_gu), g2,
-                      g.slots);
+                      static_cast<float*>(g.out), static_cast<float*>(g.gu_out), static_cast<const float*>(g.swiglu_grad_gu), g.parts,
+                      g.part_rows, g2, g.slots);
         };
         constexpr int SK = 16 * STEPS * (NW / FW);
         if (aligned && g.K % SK == 0 && d2.K % SK == 0) launch(std::true_type{});
+        else if (g.parts > 1) refused = true;  // (f32_parts does not ask for it)
         else if constexpr (!(F32 && FW == 4)) launch(std::false_type{});  // (f32_tile does not ask for it)
     };
     typedef std::integral_constant<int, 1> One;
@@ -855,7 +887,7 @@ static hipError_t launch_f32_t(const GroupedArgs& g, hipStream_t s) {
     };
     if (g.swiglu) pick(std::true_type{});
     else pick(std::false_type{});
-    return hipGetLastError();
+    return refused ? hipErrorInvalidValue : hipGetLastError();
 }
 
 hipError_t launch_grouped_f32(const GroupedArgs& g, WeightKind wk, hipStream_t s) {

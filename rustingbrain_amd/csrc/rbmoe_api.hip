@@ -257,6 +257,7 @@ struct rbmoe_layer {
     bool decode_down_by_expert = true;  // behind a decode_front launch: the down launch's workgroup rows are experts, not tile-table entries
     bool last_front = false;   // the last forward's hidden rows are per expert over all rows (Work::hall)
     bool last_by_slot = false; // ... and its expert rows lie in slot order
+    int last_parts = 1;          // ... the parts that the last forward's expert rows lie in (CombineArgs::parts)
     int group_m = 0;
     const char* kernel_name = "none";
     int last_T = -1;
@@ -1351,6 +1352,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         L->last_T = T;
         L->last = wk_;
         L->last_front = front;
+        L->last_parts = 1;
         L->last_by_slot = front && (few || by_expert);
         return RBMOE_OK;
     }
@@ -1555,8 +1557,19 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // rows, which are wider, for the down product (measured HBM-side traffic: 270 against 301 MB with groups of 8
     // against 4 for gate/up, 147 against 166 MB with 4 against 8 for down)
     if (L->group_m == 0) g2.group_m = 4;
-    HIP_TRY(ctx, run(shared_inside ? with_shared(g2, s2) : g2, false));
-    L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return run_on(g2, st); };
+    GroupedArgs second = shared_inside ? with_shared(g2, s2) : g2;
+    if (L->f32_rows && !L->training && T > 0 && d % 4 == 0 && k <= 8) {
+        second.parts = f32_parts(second, wk);
+        // (where the buffers hold as many rows)
+        while (second.parts > 1 && ((size_t)second.parts * T * k * d * 4 > L->y.bytes ||
+                                    (shared_inside && (size_t)second.parts * T * d * 4 > L->ys.bytes)))
+            second.parts /= 2;
+        second.part_rows = T * k;
+    }
+    HIP_TRY(ctx, run(second, false));
+    GroupedArgs down = second;
+    if (down.parts == 1) down = g2;
+    L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return run_on(down, st); };
     HIP_TRY(ctx, mark(5));
 
     if (c.shared_expert && T > 0 && !shared_forked && !shared_inside) HIP_TRY(ctx, shared_expert(s));
@@ -1569,11 +1582,15 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     CombineArgs ca{L->y.p, c.shared_expert ? L->ys.p : nullptr, residual, (const int*)L->inv_pos.p,
                    (const float*)L->gate_of.p, T, d, k, out};
     ca.rows_bf16 = cast;
+    ca.parts = second.parts;
+    ca.parts_shared = shared_inside ? second.parts : 1;
+    ca.part_rows = second.part_rows;
     HIP_TRY(ctx, launch_combine(ca, abf, s));
     L->replay[RBMOE_STAGE_COMBINE] = [=](hipStream_t st) { return launch_combine(ca, abf, st); };
     HIP_TRY(ctx, mark(7));
     L->last_T = T;
     L->last = wk_;
+    L->last_parts = second.parts;
     L->last_front = false;
     L->last_by_slot = false;
     return RBMOE_OK;
@@ -2602,7 +2619,16 @@ int rbmoe_get_expert_rows(rbmoe_layer* L, float* hidden, float* expert_out) {
         for (int pos = 0; pos < R; ++pos) std::memcpy(expert_out + (size_t)pos * d, all.data() + (size_t)slots[pos] * d, (size_t)d * 4);
         return RBMOE_OK;
     }
-    return fetch(expert_out, L->last.y, (size_t)R * d);
+    rc = fetch(expert_out, L->last.y, (size_t)R * d);
+    if (rc != RBMOE_OK || !expert_out || R == 0) return rc;
+    std::vector<float> more(L->last_parts > 1 ? (size_t)R * d : 0);
+    for (int p = 1; p < L->last_parts; ++p) {  // a row is the sum of its parts in order
+        const size_t from = (size_t)p * L->last_T * L->cfg.experts_per_token * d;
+        rc = fetch(more.data(), static_cast<const float*>(L->last.y) + from, more.size());
+        if (rc != RBMOE_OK) return rc;
+        for (size_t i = 0; i < more.size(); ++i) expert_out[i] += more[i];
+    }
+    return RBMOE_OK;
 }
 
 const char* rbmoe_expert_kernel_name(const rbmoe_layer* L) { return L ? L->kernel_name : "none"; }

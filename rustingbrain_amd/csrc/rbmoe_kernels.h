@@ -188,6 +188,9 @@ struct CombineArgs {
     const float* gate_of; // [T*k]
     int T, d, k;
     void* out;            // [T, d]
+    // f32 rows: y and yshared lie in so many parts (1, 2 or 4), part_rows and T rows apart, each row the sum of its parts in order
+    int parts = 1, parts_shared = 1;
+    int part_rows = 0;
     bool rows_bf16 = false;  // under f32 activations: y and yshared are bf16 (matrix-core products of a bf16 / int8 layer)
 };
 hipError_t launch_combine(const CombineArgs& a, bool bf16, hipStream_t s);
@@ -245,6 +248,10 @@ struct GroupedArgs {
     int group_m;            // MFMA path: M-tiles per scheduling group (0 = default)
     int tile_m = 0;         // rows per tile of the tile table
     RoutedSlots slots;      // gate/up launches of the matrix-core kernels: in the place of tile table and row index
+    // plain launches over f32 rows: the reduction shared out over so many workgroups a tile.  Part p of a row of `out` lies p * part_rows
+    // rows on (of dense2.out p * dense2.rows), and the row is their sum in order.
+    int parts = 1;
+    int part_rows = 0;
 };
 hipError_t launch_grouped_generic(const GroupedArgs& a, bool act_bf16, WeightKind wk, int tile_m,
                                   hipStream_t s);
@@ -264,6 +271,7 @@ void pack_weight_i8(const int8_t* src, int rows, int cols, int8_t* dst);
 int f32_tile_m(int rows, int groups);  // rows of the tile table's tiles for so many routed rows: 32 or 64
 bool f32_shape_ok(int N, int K);
 int f32_workgroups(const GroupedArgs& a, WeightKind wk);  // about as many as the launch has
+int f32_parts(const GroupedArgs& a, WeightKind wk);  // GroupedArgs::parts for a plain launch where there is room for them
 bool f32_joins(int F, int Fs);  // whether a shared expert of width Fs may go into the launches of experts of width F
 hipError_t launch_grouped_f32(const GroupedArgs& a, WeightKind wk, hipStream_t s);
 

@@ -834,11 +834,11 @@ struct RowPiece<bf16_t, float> {  // four bf16 elements beside four f32 ones
 // lanes, and its positions and gates are fetched and sorted once a wave in scalar registers: 290.  us a forward, before / after: 64
 // experts of 704, six a token, d 1024, 16384 rows 673.3 / 665.2 (another box 712.0 / 701.0); 2048 rows of the default model 34.2 /
 // 33.9; without whole waves (d 768) 8192 rows by 16 experts, two a token, 147.2 / 146.4, 4096 rows int8 the same.
-template <typename XT, typename YT, int KMAX, bool ROW>
+template <typename XT, typename YT, int KMAX, bool ROW, int PARTS>
 __global__ __launch_bounds__(256) void combine_vec_kernel(
     const YT* __restrict__ y, const YT* __restrict__ yshared, const XT* __restrict__ residual,
-    const int* __restrict__ inv_pos, const float* __restrict__ gate_of, int T, int d, int k, uint32_t recip,
-    XT* __restrict__ out) {
+    const int* __restrict__ inv_pos, const float* __restrict__ gate_of, int T, int d, int k, uint32_t recip, int part_rows,
+    int parts_shared, XT* __restrict__ out) {
     constexpr int VN = Vec16<XT>::N;
     typedef RowPiece<YT, XT> YP;
     const int pieces = d / VN;
@@ -888,24 +888,45 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(
     for (int i = 0; i < VN; ++i) acc[i] = 0.0f;
     // every row piece is fetched before the first add (no branch around a load: an unused slot
     // re-reads row 0), so the k loads of a token are one round trip instead of k
-    typename YP::raw_t raw[KMAX], raw_s = {};
+    typename YP::raw_t raw[PARTS][KMAX], raw_s[PARTS] = {};
     uint4 raw_r = make_uint4(0, 0, 0, 0);
 #pragma unroll
-    for (int r = 0; r < KMAX; ++r) raw[r] = YP::load_raw(y + (size_t)(r < n ? pos[r] : 0) * d + c);
-    if (yshared) raw_s = YP::load_raw(yshared + (size_t)t * d + c);    // uniform over the launch
+    for (int p = 0; p < PARTS; ++p)
+#pragma unroll
+        for (int r = 0; r < KMAX; ++r) raw[p][r] = YP::load_raw(y + ((size_t)p * part_rows + (r < n ? pos[r] : 0)) * d + c);
+    if (yshared) {  // uniform over the launch
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p)
+            if (p == 0 || p < parts_shared) raw_s[p] = YP::load_raw(yshared + ((size_t)p * T + t) * d + c);
+    }
     if (residual) raw_r = Vec16<XT>::load_raw(residual + (size_t)t * d + c);
 #pragma unroll
     for (int r = 0; r < KMAX; ++r) {
         if (r < n) {
             float v[VN];
-            YP::widen(raw[r], v);
+            YP::widen(raw[0][r], v);
+#pragma unroll
+            for (int p = 1; p < PARTS; ++p) {
+                float more[VN];
+                YP::widen(raw[p][r], more);
+#pragma unroll
+                for (int i = 0; i < VN; ++i) v[i] = __fadd_rn(v[i], more[i]);
+            }
 #pragma unroll
             for (int i = 0; i < VN; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn(__uint_as_float(gate[r]), v[i]));
         }
     }
     if (yshared) {
         float v[VN];
-        YP::widen(raw_s, v);
+        YP::widen(raw_s[0], v);
+#pragma unroll
+        for (int p = 1; p < PARTS; ++p) {
+            if (p >= parts_shared) break;
+            float more[VN];
+            YP::widen(raw_s[p], more);
+#pragma unroll
+            for (int i = 0; i < VN; ++i) v[i] = __fadd_rn(v[i], more[i]);
+        }
 #pragma unroll
         for (int i = 0; i < VN; ++i) acc[i] = __fadd_rn(acc[i], v[i]);
     }
@@ -1314,15 +1335,25 @@ static hipError_t launch_combine_t(const CombineArgs& a, hipStream_t s) {
     const XT* res = static_cast<const XT*>(a.residual);
     XT* out = static_cast<XT*>(a.out);
     constexpr int VN = Vec16<XT>::N;
-    if (a.d % VN == 0 && a.k <= 8) {
+    const bool pieces_ok = a.d % VN == 0 && a.k <= 8;
+    if ((a.parts != 1 && (!pieces_ok || sizeof(YT) != 4 || (a.parts != 2 && a.parts != 4))) || a.parts_shared < 1 || a.parts_shared > a.parts)
+        return hipErrorInvalidValue;
+    if (pieces_ok) {
         const long long total = (long long)a.T * (a.d / VN);
         const dim3 grid((unsigned)((total + 255) / 256)), block(256);
         // 2^32 / pieces rounded up, which counts a row's pieces exactly as long as threads x pieces stays below 2^32 (0: divide)
         const int pieces = a.d / VN;
         const uint32_t recip = pieces > 1 && (total + 256) * pieces < (1ll << 32) ? (uint32_t)(0x100000000ull / (uint32_t)pieces) + 1u : 0u;
+        auto launch = [&](auto kmax, auto row, auto parts) {
+            RB_LAUNCH((combine_vec_kernel<XT, YT, decltype(kmax)::value, decltype(row)::value, decltype(parts)::value>), grid, block, 0,
+                      s, y, ys, res, a.inv_pos, a.gate_of, a.T, a.d, a.k, recip, a.part_rows, a.parts_shared, out);
+        };
         auto go = [&](auto kmax, auto row) {
-            RB_LAUNCH((combine_vec_kernel<XT, YT, decltype(kmax)::value, decltype(row)::value>), grid, block, 0, s, y, ys, res,
-                      a.inv_pos, a.gate_of, a.T, a.d, a.k, recip, out);
+            if constexpr (sizeof(YT) == 4) {
+                if (a.parts == 4) return launch(kmax, row, std::integral_constant<int, 4>{});
+                if (a.parts == 2) return launch(kmax, row, std::integral_constant<int, 2>{});
+            }
+            launch(kmax, row, std::integral_constant<int, 1>{});
         };
         auto pick = [&](auto row) {
             if (a.k <= 2) go(std::integral_constant<int, 2>{}, row);

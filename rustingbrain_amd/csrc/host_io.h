@@ -58,8 +58,6 @@ struct CopySegment {
 };
 constexpr int kMaxCopySegments = 10;
 hipError_t launch_copy_segments(const CopySegment* segments, int n, hipStream_t s);
-// dst[r][c] = src[r * pitch + c], rows of `cols` 4-byte words
-hipError_t launch_copy_rows(const void* src, size_t pitch_words, void* dst, int rows, int cols, hipStream_t s);
 // dst[i] = f32(src[i]) of bf16 rows; n a multiple of 4, dst 16-byte and src 8-byte aligned
 hipError_t launch_widen_rows(const void* src, float* dst, size_t n, hipStream_t s);
 

@@ -183,23 +183,6 @@ hipError_t launch_copy_segments(const CopySegment* segments, int n, hipStream_t 
     return hipGetLastError();
 }
 
-__global__ __launch_bounds__(256) void copy_rows_kernel(const uint32_t* __restrict__ src, size_t pitch,
-                                                        uint32_t* __restrict__ dst, int rows, int cols) {
-    const size_t n = (size_t)rows * cols, stride = (size_t)gridDim.x * 256;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
-        const size_t r = i / (unsigned)cols;
-        dst[i] = src[r * pitch + (i - r * cols)];
-    }
-}
-
-hipError_t launch_copy_rows(const void* src, size_t pitch_words, void* dst, int rows, int cols, hipStream_t s) {
-    if (rows <= 0 || cols <= 0) return hipSuccess;
-    const size_t n = (size_t)rows * cols, blocks = (n + 1023) / 1024;
-    hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)(blocks < 512 ? blocks : 512)), dim3(256), 0, s,
-                       static_cast<const uint32_t*>(src), pitch_words, static_cast<uint32_t*>(dst), rows, cols);
-    return hipGetLastError();
-}
-
 __global__ __launch_bounds__(256) void widen_rows_kernel(const bf16_t* __restrict__ src, float* __restrict__ dst, size_t n4) {
     const size_t stride = (size_t)gridDim.x * 256;
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += stride) {

@@ -24,6 +24,7 @@ def widths(d, F, act, wt, Fs=0, T=64, E=8, k=2, training=False):
     ("bf16", "bf16", 16, 0, (64, 64, BF16_CORES)), ("bf16", "bf16", 15, 0, (15, 15, ANY)),   # four times the work, and more
     ("f32", "f32", 341, 0, (352, 352, F32_CORES)), ("f32", "f32", 15, 0, (15, 15, ANY)),
     ("f32", "bf16", 384, 0, (384, 384, BF16_CORES)), ("f32", "bf16", 352, 0, (352, 352, ANY)),
+    ("f32", "bf16", 341, 910, (352, 928, ANY)), ("f32", "int8", 17, 15, (32, 15, ANY)),   # whole slices up to twice the work
     ("f32", "int8", 384, 352, (384, 352, ANY)), ("bf16", "f32", 384, 0, (384, 384, ANY)),
 ])
 def test_widths(act, wt, F, Fs, want):

@@ -167,8 +167,8 @@ __global__ __launch_bounds__(NW * 64, 2) void grouped_f32_kernel(
     const float* __restrict__ a, const int* __restrict__ row_index, const WT* __restrict__ w, size_t w_expert_stride,
     const float* __restrict__ scales, size_t s_expert_stride, int N, int K, const int* __restrict__ tile_expert,
     const int* __restrict__ tile_row0, const int* __restrict__ tile_rows, const int* __restrict__ ntiles, int sub, int dense_rows,
-    float* __restrict__ out, float* __restrict__ gu_out, const float* __restrict__ bw_gu, int parts, int part_rows, F32Dense<WT> g2,
-    RoutedSlots slots) {
+    float* __restrict__ out, float* __restrict__ gu_out, const float* __restrict__ bw_gu, F32Dense<WT> g2, RoutedSlots slots,
+    int parts, int part_rows) {
     typedef Weights<WT> W;
     constexpr int NTH = NW * 64;
     constexpr int KG = NW / FW;                   // wave groups that share out a slice's steps
@@ -862,8 +862,8 @@ static hipError_t launch_f32_t(const GroupedArgs& g, hipStream_t s) {
             RB_LAUNCH((grouped_f32_kernel<WT, SW, NW, BM / 32, FW, STEPS, decltype(dma_tag)::value>), dim3((total + 7) / 8 * 8 + rest),
                       dim3(64 * NW), 0, s, static_cast<const float*>(g.a), g.row_index, static_cast<const WT*>(g.w), g.w_expert_stride,
                       g.scales, g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, sub, g.dense_rows,
-                      static_cast<float*>(g.out), static_cast<float*>(g.gu_out), static_cast<const float*>(g.swiglu_grad_gu), g.parts,
-                      g.part_rows, g2, g.slots);
+                      static_cast<float*>(g.out), static_cast<float*>(g.gu_out), static_cast<const float*>(g.swiglu_grad_gu), g2,
+                      g.slots, g.parts, g.part_rows);
         };
         constexpr int SK = 16 * STEPS * (NW / FW);
         if (aligned && g.K % SK == 0 && d2.K % SK == 0) launch(std::true_type{});

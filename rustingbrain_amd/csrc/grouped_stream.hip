@@ -821,12 +821,15 @@ __device__ __forceinline__ void narrow_loop(const PipeCtx& c, floatx16 (&acc)[TT
     for (int i = 0; i < NRING; ++i) asm volatile("" : : "v"(ring[i].f));
 }
 
-template <bool SWIGLU, bool I8>
+// PARTS: plain launches whose reduction is shared out (GroupedArgs::parts along y); kernels of their own, since the others' first loads
+// wait for every instruction in front of them (203 rows by 16 experts, in whole, 46.4 us a block step, with one kernel for both 47.7).
+template <bool SWIGLU, bool I8, bool PARTS>
 __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
     const bf16_t* __restrict__ a, const int* __restrict__ row_index, const void* __restrict__ wpacked,
     size_t w_expert_stride_bytes, const float* __restrict__ scales, size_t s_expert_stride, int N, int K,
     const int* __restrict__ tile_expert, const int* __restrict__ tile_row0, const int* __restrict__ tile_rows,
-    const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, int group_m, DenseGroup g2, RoutedSlots slots) {
+    const int* __restrict__ ntiles, int dense_rows, bf16_t* __restrict__ out, int group_m, DenseGroup g2, RoutedSlots slots,
+    int part_rows) {
     constexpr int BN = SWIGLU ? 64 : 128;  // output features per workgroup
     __shared__ uint4 As[NSTAGES * BM * CPR];
 
@@ -852,10 +855,10 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
         N = g2.N;
         K = g2.K;
         dense_rows = g2.rows;
+        if constexpr (PARTS) part_rows = g2.rows;
         out = g2.out;
     }
     const int n0 = tn_idx * BN;
-
     int expert, row0, rows;
     if (dense_rows >= 0) {
         expert = 0;
@@ -881,8 +884,16 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
     const bool act = fb < N;
     const int wrow = SWIGLU && wave >= 2 ? N + fb : fb;
     const size_t block_bytes = (size_t)K * 32 * (I8 ? 1 : 2);
+    int from = 0, KT = K / BK;  // this workgroup's slices of the reduction
+    if constexpr (PARTS) {
+        static_assert(!SWIGLU, "");
+        const int parts = gridDim.y, to = KT * (blockIdx.y + 1) / parts;
+        from = KT * blockIdx.y / parts;
+        KT = to - from;
+    }
+    const int GS = KT * KS;
     const char* const wp = static_cast<const char*>(wpacked) + (size_t)expert * w_expert_stride_bytes +
-                           (size_t)(act ? wrow / 32 : 0) * block_bytes;
+                           (size_t)(act ? wrow / 32 : 0) * block_bytes + (size_t)from * BK * 32 * (I8 ? 1 : 2);
     const uint32_t lane16 = (uint32_t)lane * 16u;
 
     // LDS-DMA of the activation slices: as in the kernel above
@@ -893,10 +904,9 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
         const int r = wave * (BM / NW) + j * 8 + (lane >> 3);
         const int rr = r < rows ? r : 0;
         const int grow = own && !at.second ? own_token[rr] : row_index ? row_index[row0 + rr] : row0 + rr;
-        a_src[j] = ((uint32_t)grow * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
+        a_src[j] = ((uint32_t)grow * (uint32_t)K + (uint32_t)from * BK + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)As + wave * (BM / NW) * CPR * 16;
-    const int KT = K / BK, GS = KT * KS;
 
     floatx16 acc[TT];
 #pragma unroll
@@ -935,6 +945,17 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
         for (int t = 0; t < TT; ++t)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[t][v] *= sc[8 * (v >> 2) + 4 * lhalf + (v & 3)];
+    }
+    if constexpr (PARTS) {  // sums as they are
+        float* const to = reinterpret_cast<float*>(out) + ((size_t)blockIdx.y * part_rows + row0) * N + fb + 4 * lhalf;
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+            if (act && t * 32 + lrow < rows)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<float4*>(to + (size_t)(t * 32 + lrow) * N + 8 * q) =
+                        make_float4(acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]);
+        return;
     }
     constexpr int XCH = 2 * TT * 16 * 64 * 4;  // gate/up: the up waves' accumulators, 32 KiB; the output tile behind them
     char* const stage = lds + (SWIGLU ? XCH : 0);
@@ -1001,6 +1022,18 @@ __global__ __launch_bounds__(NT, 2) void narrow_grouped_stream_kernel(
 // Launches that keep or read pre-activations (training) stay with the wide kernel's epilogue.
 constexpr int narrow_tiles(bool swiglu, int K) { return swiglu ? 128 : K <= 512 ? 250 : 140; }
 
+// Tiles of a launch: `m` row tiles of the routed rows, `bm` rows each, and `bn` features.
+int stream_tiles(const GroupedArgs& g, int m, int bm, int bn) {
+    const GroupedArgs::Dense& d2 = g.dense2;
+    return m * ((g.N + bn - 1) / bn) + (d2.rows + bm - 1) / bm * ((d2.N + bn - 1) / bn);
+}
+// Whether the narrow kernel takes a launch.
+bool stream_narrow(const GroupedArgs& g) {
+    if (g.gu_out || g.swiglu_grad_gu || (g.dense_rows < 0 && g.tile_m == rows_of(TALL))) return false;
+    const int m = g.dense_rows >= 0 ? (g.dense_rows + BM - 1) / BM : g.likely_tiles > 0 ? g.likely_tiles : g.max_tiles;
+    return stream_tiles(g, m, BM, g.swiglu ? NW * 32 : NW * 64) <= narrow_tiles(g.swiglu, g.K);
+}
+
 template <bool SWIGLU, bool I8>
 hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
     constexpr int BN = SWIGLU ? NW * 32 : NW * 64;
@@ -1008,19 +1041,24 @@ hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
     const bool tall = g.dense_rows < 0 && g.tile_m == rows_of(TALL);
     const int bm = tall ? rows_of(TALL) : BM;
     const int tiles_m = g.dense_rows >= 0 ? (g.dense_rows + bm - 1) / bm : g.max_tiles;
-    auto tiles = [&](int m, int bn) { return m * ((g.N + bn - 1) / bn) + (d2.rows + bm - 1) / bm * ((d2.N + bn - 1) / bn); };
-    const int total = tiles(tiles_m, BN);
+    const int total = stream_tiles(g, tiles_m, bm, BN);
     if (total <= 0) return hipSuccess;
     const DenseGroup g2{static_cast<const bf16_t*>(d2.a), d2.w, d2.scales, d2.N, d2.K, d2.rows,
                         static_cast<bf16_t*>(d2.out), static_cast<bf16_t*>(d2.gu_out)};
     const int group_m = g.group_m > 0 ? g.group_m : 8;
     const int rest = SWIGLU && g.slots.expert_of ? 1 : 0;  // (routed_rest)
-    const int likely = g.dense_rows < 0 && g.likely_tiles > 0 ? tiles(g.likely_tiles, BN) : total;
-    if (!tall && likely <= narrow_tiles(SWIGLU, g.K) && !g.gu_out && !g.swiglu_grad_gu) {
-        RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8>), dim3((tiles(tiles_m, BN / 2) + 7) / 8 * 8 + rest), dim3(NT), 0, s,
-                  static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
-                  g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
-                  static_cast<bf16_t*>(g.out), group_m, g2, g.slots);
+    const bool narrow = stream_narrow(g);
+    if (g.parts != 1 && (!narrow || SWIGLU)) return hipErrorInvalidValue;
+    if (narrow) {
+        auto narrow_go = [&](auto parts) {
+            RB_LAUNCH((narrow_grouped_stream_kernel<SWIGLU, I8, decltype(parts)::value>),
+                      dim3((stream_tiles(g, tiles_m, BM, BN / 2) + 7) / 8 * 8 + rest, g.parts), dim3(NT), 0, s,
+                      static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
+                      g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
+                      static_cast<bf16_t*>(g.out), group_m, g2, g.slots, g.part_rows);
+        };
+        if (g.parts == 1) narrow_go(std::false_type{});
+        else if constexpr (!SWIGLU) narrow_go(std::true_type{});
         return hipGetLastError();
     }
     auto go = [&](auto tt) {
@@ -1057,6 +1095,22 @@ int stream_tile_m(int rows, int groups, int F, int d) {
         return (d + 800) * units(tiles(bm) * gate_up) + (F + 800) * units(tiles(bm) * down);
     };
     return length(BM) > 1.01 * 1.19 * length(rows_of(TALL)) ? rows_of(TALL) : BM;
+}
+
+// A narrow down launch of few tiles waits for a chain of slices that holds a fraction of the compute units.  Its reduction is shared out
+// where it is long and the rows, which the combine then reads in f32 and twice or four times, are few.  us a forward, whole / 2 parts
+// / 4 parts (tiles; rows times d in thousands): d 512, 8 experts of 1408, 100 rows (32; 102) 31.5 / 29.9 / 30.1, 400 rows (40; 410) 35.4 /
+// 34.2 / 34.3, 700 rows (56; 717) 36.2 / 36.4 / 36.5; d 768, 8 of 1408, int8, 83 rows (48; 127) 34.9 / 32.7 / 31.4, 200 rows (48; 307) 35.8 /
+// 34.5 / 35.2; with a shared expert, bf16, 83 rows (54; 191) 36.1 / 35.7 / 36.5, 340 rows (72; 783) 40.7 / 41.3 / 41.3; 16 of 1408, 203 rows
+// (96; 312) 40.6 / 41.2 / 41.1; d 1024, 8 of 1408, int8, 150 rows (64; 307) 37.7 / 36.0 / 37.8; 4 of 2730, 100 rows (32; 102) 39.7 / 35.7 / 35.0.
+// Reductions of 384 and 704 lose: d 512, 8 of 352 and a shared one, 100 rows 26.0 / 26.9 / 26.7.
+int stream_parts(const GroupedArgs& g) {
+    if (g.swiglu || g.dense_rows >= 0 || !stream_narrow(g)) return 1;
+    const int m = g.likely_tiles > 0 ? g.likely_tiles : g.max_tiles, tiles = stream_tiles(g, m, BM, 128);
+    const int K = g.dense2.rows > 0 ? std::min(g.K, g.dense2.K) : g.K;
+    const long long elements = (long long)(g.routed_rows + g.dense2.rows) * g.N;
+    if (K < 1024 || tiles > 64 || elements > 512 * 1024) return 1;
+    return tiles <= 48 && elements <= 128 * 1024 ? 4 : 2;
 }
 
 // K a multiple of 64 (one LDS slice), N a multiple of 32 (row blocks of the packed weights)

@@ -1562,9 +1562,10 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // against 4 for gate/up, 147 against 166 MB with 4 against 8 for down)
     if (L->group_m == 0) g2.group_m = 4;
     GroupedArgs second = shared_inside ? with_shared(g2, s2) : g2;
-    if (L->f32_rows && !L->training && T > 0 && d % 4 == 0 && k <= 8) {
-        second.parts = f32_parts(second, wk);
-        // (where the buffers hold as many rows)
+    if ((L->f32_rows || (mfma && d % 8 == 0)) && !L->training && T > 0 && d % 4 == 0 && k <= 8 &&
+        (L->f32_rows || !c.shared_expert || shared_inside)) {
+        second.parts = mfma ? stream_parts(second) : f32_parts(second, wk);
+        // (where the buffers hold as many rows of f32)
         while (second.parts > 1 && ((size_t)second.parts * T * k * d * 4 > L->y.bytes ||
                                     (shared_inside && (size_t)second.parts * T * d * 4 > L->ys.bytes)))
             second.parts /= 2;
@@ -1587,7 +1588,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
                    (const float*)L->gate_of.p, T, d, k, out};
     ca.rows_bf16 = cast;
     ca.parts = second.parts;
-    ca.parts_shared = shared_inside ? second.parts : 1;
+    ca.shared_in_parts = shared_inside;
     ca.part_rows = second.part_rows;
     HIP_TRY(ctx, launch_combine(ca, abf, s));
     L->replay[RBMOE_STAGE_COMBINE] = [=](hipStream_t st) { return launch_combine(ca, abf, st); };
@@ -2626,15 +2627,15 @@ int rbmoe_get_expert_rows(rbmoe_layer* L, float* hidden, float* expert_out) {
         for (int pos = 0; pos < R; ++pos) std::memcpy(expert_out + (size_t)pos * d, all.data() + (size_t)slots[pos] * d, (size_t)d * 4);
         return RBMOE_OK;
     }
-    rc = fetch(expert_out, L->last.y, (size_t)R * d);
-    if (rc != RBMOE_OK || !expert_out || R == 0) return rc;
-    std::vector<float> more(L->last_parts > 1 ? (size_t)R * d : 0);
-    for (int p = 1; p < L->last_parts; ++p) {  // a row is the sum of its parts in order
+    if (L->last_parts == 1 || !expert_out || R == 0) return fetch(expert_out, L->last.y, (size_t)R * d);
+    std::vector<float> part((size_t)R * d);
+    for (int p = 0; p < L->last_parts; ++p) {  // a row is the sum of its parts (f32) in order
         const size_t from = (size_t)p * L->last_T * L->cfg.experts_per_token * d;
-        rc = fetch(more.data(), static_cast<const float*>(L->last.y) + from, more.size());
-        if (rc != RBMOE_OK) return rc;
-        for (size_t i = 0; i < more.size(); ++i) expert_out[i] += more[i];
+        HIP_TRY(ctx, hipMemcpy(part.data(), static_cast<const float*>(L->last.y) + from, part.size() * 4, hipMemcpyDeviceToHost));
+        for (size_t i = 0; i < part.size(); ++i) expert_out[i] = p == 0 ? part[i] : expert_out[i] + part[i];
     }
+    if (abf)
+        for (size_t i = 0; i < part.size(); ++i) expert_out[i] = host_bf16_to_f32(host_f32_to_bf16(expert_out[i]));
     return RBMOE_OK;
 }
 

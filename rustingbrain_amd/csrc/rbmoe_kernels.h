@@ -188,8 +188,10 @@ struct CombineArgs {
     const float* gate_of; // [T*k]
     int T, d, k;
     void* out;            // [T, d]
-    // f32 rows: y and yshared lie in so many parts (1, 2 or 4), part_rows and T rows apart, each row the sum of its parts in order
-    int parts = 1, parts_shared = 1;
+    // y (and, with shared_in_parts, yshared) lies in so many parts (1, 2 or 4) in f32, part_rows (T) rows apart: a row is the sum of its
+    // parts in order, rounded to the type that the rows have otherwise
+    int parts = 1;
+    bool shared_in_parts = false;
     int part_rows = 0;
     bool rows_bf16 = false;  // under f32 activations: y and yshared are bf16 (matrix-core products of a bf16 / int8 layer)
 };
@@ -248,8 +250,8 @@ struct GroupedArgs {
     int group_m;            // MFMA path: M-tiles per scheduling group (0 = default)
     int tile_m = 0;         // rows per tile of the tile table
     RoutedSlots slots;      // gate/up launches of the matrix-core kernels: in the place of tile table and row index
-    // plain launches over f32 rows: the reduction shared out over so many workgroups a tile.  Part p of a row of `out` lies p * part_rows
-    // rows on (of dense2.out p * dense2.rows), and the row is their sum in order.
+    // plain launches: the reduction shared out over so many workgroups a tile.  Part p of a row of `out` lies p * part_rows rows on (of
+    // dense2.out p * dense2.rows), in f32 whatever the rows' type, and the row is the parts' sum in order.
     int parts = 1;
     int part_rows = 0;
 };
@@ -263,6 +265,7 @@ constexpr int kGenericTileM = 16;
 constexpr int kStreamTileM = 128;
 int stream_tile_m(int rows, int groups, int F, int d);  // rows of the tile table's tiles for so many routed rows: 128 or 160
 bool stream_shape_ok(int N, int K);
+int stream_parts(const GroupedArgs& a);  // GroupedArgs::parts for a plain launch where there is room for them
 hipError_t launch_grouped_stream(const GroupedArgs& a, WeightKind wk, hipStream_t s);
 void pack_weight_bf16(const uint16_t* src, int rows, int cols, uint16_t* dst);
 void pack_weight_i8(const int8_t* src, int rows, int cols, int8_t* dst);

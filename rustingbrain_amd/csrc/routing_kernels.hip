@@ -818,6 +818,19 @@ struct RowPiece {  // rows of the activation type itself
     static __device__ __forceinline__ void widen(const raw_t& a, float (&v)[Vec16<YT>::N]) { Vec16<YT>::widen(a, v); }
 };
 template <>
+struct RowPiece<float, bf16_t> {  // eight f32 elements beside eight bf16 ones
+    struct raw_t {
+        float4 a, b;
+    };
+    static __device__ __forceinline__ raw_t load_raw(const float* p) {
+        return {*reinterpret_cast<const float4*>(p), *reinterpret_cast<const float4*>(p + 4)};
+    }
+    static __device__ __forceinline__ void widen(const raw_t& r, float (&v)[8]) {
+        v[0] = r.a.x; v[1] = r.a.y; v[2] = r.a.z; v[3] = r.a.w;
+        v[4] = r.b.x; v[5] = r.b.y; v[6] = r.b.z; v[7] = r.b.w;
+    }
+};
+template <>
 struct RowPiece<bf16_t, float> {  // four bf16 elements beside four f32 ones
     typedef uint2 raw_t;
     static __device__ __forceinline__ raw_t load_raw(const bf16_t* p) { return *reinterpret_cast<const uint2*>(p); }
@@ -834,11 +847,13 @@ struct RowPiece<bf16_t, float> {  // four bf16 elements beside four f32 ones
 // lanes, and its positions and gates are fetched and sorted once a wave in scalar registers: 290.  us a forward, before / after: 64
 // experts of 704, six a token, d 1024, 16384 rows 673.3 / 665.2 (another box 712.0 / 701.0); 2048 rows of the default model 34.2 /
 // 33.9; without whole waves (d 768) 8192 rows by 16 experts, two a token, 147.2 / 146.4, 4096 rows int8 the same.
-template <typename XT, typename YT, int KMAX, bool ROW, int PARTS>
+// PARTS, ROUND: CombineArgs::parts, of rows that are bf16 otherwise.  (What only they need comes last: the others' arguments are one
+// cache line.)
+template <typename XT, typename YT, int KMAX, bool ROW, int PARTS, bool ROUND>
 __global__ __launch_bounds__(256) void combine_vec_kernel(
     const YT* __restrict__ y, const YT* __restrict__ yshared, const XT* __restrict__ residual,
-    const int* __restrict__ inv_pos, const float* __restrict__ gate_of, int T, int d, int k, uint32_t recip, int part_rows,
-    int parts_shared, XT* __restrict__ out) {
+    const int* __restrict__ inv_pos, const float* __restrict__ gate_of, int T, int d, int k, uint32_t recip,
+    XT* __restrict__ out, int part_rows, bool shared_in_parts) {
     constexpr int VN = Vec16<XT>::N;
     typedef RowPiece<YT, XT> YP;
     const int pieces = d / VN;
@@ -897,7 +912,7 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(
     if (yshared) {  // uniform over the launch
 #pragma unroll
         for (int p = 0; p < PARTS; ++p)
-            if (p == 0 || p < parts_shared) raw_s[p] = YP::load_raw(yshared + ((size_t)p * T + t) * d + c);
+            if (p == 0 || shared_in_parts) raw_s[p] = YP::load_raw(yshared + ((size_t)p * T + t) * d + c);
     }
     if (residual) raw_r = Vec16<XT>::load_raw(residual + (size_t)t * d + c);
 #pragma unroll
@@ -912,6 +927,9 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(
 #pragma unroll
                 for (int i = 0; i < VN; ++i) v[i] = __fadd_rn(v[i], more[i]);
             }
+            if constexpr (ROUND)
+#pragma unroll
+                for (int i = 0; i < VN; ++i) v[i] = to_f32(from_f32<bf16_t>(v[i]));
 #pragma unroll
             for (int i = 0; i < VN; ++i) acc[i] = __fadd_rn(acc[i], __fmul_rn(__uint_as_float(gate[r]), v[i]));
         }
@@ -921,12 +939,15 @@ __global__ __launch_bounds__(256) void combine_vec_kernel(
         YP::widen(raw_s[0], v);
 #pragma unroll
         for (int p = 1; p < PARTS; ++p) {
-            if (p >= parts_shared) break;
+            if (!shared_in_parts) break;
             float more[VN];
             YP::widen(raw_s[p], more);
 #pragma unroll
             for (int i = 0; i < VN; ++i) v[i] = __fadd_rn(v[i], more[i]);
         }
+        if constexpr (ROUND)
+#pragma unroll
+            for (int i = 0; i < VN; ++i) v[i] = to_f32(from_f32<bf16_t>(v[i]));
 #pragma unroll
         for (int i = 0; i < VN; ++i) acc[i] = __fadd_rn(acc[i], v[i]);
     }
@@ -1328,7 +1349,7 @@ hipError_t launch_dispatch(const DispatchArgs& a, bool bf16, hipStream_t s) {
     return bf16 ? launch_dispatch_t<bf16_t>(a, s) : launch_dispatch_t<float>(a, s);
 }
 
-template <typename XT, typename YT>
+template <typename XT, typename YT, bool ROUND = false>
 static hipError_t launch_combine_t(const CombineArgs& a, hipStream_t s) {
     const YT* y = static_cast<const YT*>(a.y);
     const YT* ys = static_cast<const YT*>(a.yshared);
@@ -1336,8 +1357,8 @@ static hipError_t launch_combine_t(const CombineArgs& a, hipStream_t s) {
     XT* out = static_cast<XT*>(a.out);
     constexpr int VN = Vec16<XT>::N;
     const bool pieces_ok = a.d % VN == 0 && a.k <= 8;
-    if ((a.parts != 1 && (!pieces_ok || sizeof(YT) != 4 || (a.parts != 2 && a.parts != 4))) || a.parts_shared < 1 || a.parts_shared > a.parts)
-        return hipErrorInvalidValue;
+    if (a.parts != 1 && (!pieces_ok || sizeof(YT) != 4 || (a.parts != 2 && a.parts != 4))) return hipErrorInvalidValue;
+    if (ROUND && (a.parts == 1 || (ys && !a.shared_in_parts))) return hipErrorInvalidValue;  // (rows that are not in parts are bf16)
     if (pieces_ok) {
         const long long total = (long long)a.T * (a.d / VN);
         const dim3 grid((unsigned)((total + 255) / 256)), block(256);
@@ -1345,15 +1366,15 @@ static hipError_t launch_combine_t(const CombineArgs& a, hipStream_t s) {
         const int pieces = a.d / VN;
         const uint32_t recip = pieces > 1 && (total + 256) * pieces < (1ll << 32) ? (uint32_t)(0x100000000ull / (uint32_t)pieces) + 1u : 0u;
         auto launch = [&](auto kmax, auto row, auto parts) {
-            RB_LAUNCH((combine_vec_kernel<XT, YT, decltype(kmax)::value, decltype(row)::value, decltype(parts)::value>), grid, block, 0,
-                      s, y, ys, res, a.inv_pos, a.gate_of, a.T, a.d, a.k, recip, a.part_rows, a.parts_shared, out);
+            RB_LAUNCH((combine_vec_kernel<XT, YT, decltype(kmax)::value, decltype(row)::value, decltype(parts)::value, ROUND>), grid,
+                      block, 0, s, y, ys, res, a.inv_pos, a.gate_of, a.T, a.d, a.k, recip, out, a.part_rows, a.shared_in_parts);
         };
         auto go = [&](auto kmax, auto row) {
             if constexpr (sizeof(YT) == 4) {
                 if (a.parts == 4) return launch(kmax, row, std::integral_constant<int, 4>{});
                 if (a.parts == 2) return launch(kmax, row, std::integral_constant<int, 2>{});
             }
-            launch(kmax, row, std::integral_constant<int, 1>{});
+            if constexpr (!ROUND) launch(kmax, row, std::integral_constant<int, 1>{});
         };
         auto pick = [&](auto row) {
             if (a.k <= 2) go(std::integral_constant<int, 2>{}, row);
@@ -1364,7 +1385,7 @@ static hipError_t launch_combine_t(const CombineArgs& a, hipStream_t s) {
         // (waves are counted in 32 bits)
         if (a.d / VN % 64 == 0 && total / 64 < (1ll << 31)) pick(std::true_type{});
         else pick(std::false_type{});
-    } else {
+    } else if constexpr (!ROUND) {
         RB_LAUNCH((combine_any_kernel<XT, YT>), dim3((a.T + 3) / 4), dim3(256), 0, s, y, ys, res, a.inv_pos,
                            a.gate_of, a.T, a.d, a.k, out);
     }
@@ -1488,6 +1509,8 @@ hipError_t launch_rmsnorm(const void* x, const float* weight, float eps, int T, 
 
 hipError_t launch_combine(const CombineArgs& a, bool bf16, hipStream_t s) {
     if (a.T <= 0) return hipSuccess;
+    if (a.parts > 1 && (bf16 || a.rows_bf16))
+        return bf16 ? launch_combine_t<bf16_t, float, true>(a, s) : launch_combine_t<float, float, true>(a, s);
     if (bf16) return launch_combine_t<bf16_t, bf16_t>(a, s);
     return a.rows_bf16 ? launch_combine_t<float, bf16_t>(a, s) : launch_combine_t<float, float>(a, s);
 }

@@ -181,7 +181,7 @@ struct TileOut {
 // `stage`: 32 KiB of LDS that no wave of the workgroup reads or writes any more (the caller has made sure of
 // that with a barrier).  `before_stores()` is called once, when the first pass has been converted and staged and
 // before its first store to memory is issued.
-template <bool SWIGLU, bool I8, int TT, typename F>
+template <bool SWIGLU, bool I8, int TT, bool HALVES, typename F>
 __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][TT], char* const stage,
                                            F&& before_stores) {
     constexpr int BN = SWIGLU ? NW * 32 : NW * 64, BM = rows_of(TT);
@@ -197,8 +197,8 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
     const int lhalf = lane >> 5;
     const int rows = o.rows, row0 = o.row0, tn_idx = o.tn_idx, N = o.N, r0 = o.r0, r1 = o.r1;
     const bool act0 = o.act0, act1 = o.act1;
-    const int column = SWIGLU ? o.column : wave;
-    const int m0 = (SWIGLU ? o.t0 * 32 : 0) + lrow;  // the row of this lane's tokens in the wave's first block
+    const int column = HALVES ? o.column : wave;
+    const int m0 = (HALVES ? o.t0 * 32 : 0) + lrow;  // the row of this lane's tokens in the wave's first block
     const float* const sc = o.sc;
     bf16_t* const out = o.out;
     bf16_t* const gu_out = o.gu_out;
@@ -226,7 +226,7 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
             const int rb = b ? r1 : r0;
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
-                if (SWIGLU ? t >= o.blocks : t * 32 >= rows) continue;
+                if (HALVES ? t >= o.blocks : t * 32 >= rows) continue;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int f = 8 * q + 4 * lhalf;  // first of 4 consecutive features inside the row block
@@ -534,7 +534,12 @@ struct DenseGroup {
     bf16_t *out, *gu_out;
 };
 
-template <bool SWIGLU, bool I8, int TT>
+// OWN: the launch works its tiles out by itself (RoutedSlots); HALVES: its last feature tile may have at most 64 features.  Kernels
+// of their own, since a workgroup's first loads wait for every instruction in front of them and the tables' code takes more scalar
+// registers than there are (22 of them kept in vector registers in one kernel for all, none without it).  us a forward, one kernel for
+// all / these: 8192 rows by 16 experts of 1408, d 768, 151.8 / 150.6; 2048 rows of the default model, which works its tiles out, 34.3 / 34.0
+// (without the code for halves no faster: launches that work their tiles out always carry it).
+template <bool SWIGLU, bool I8, int TT, bool OWN, bool HALVES>
 __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     const bf16_t* __restrict__ a, const int* __restrict__ row_index, const void* __restrict__ wpacked,
     size_t w_expert_stride_bytes, const float* __restrict__ scales, size_t s_expert_stride, int N, int K,
@@ -549,16 +554,16 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
 
     // without tables: what the router left behind (RoutedSlots), worked out in the stages' room; the rows' tokens lie in the
     // stage that is filled last, behind a barrier
-    const bool own = SWIGLU && TT < TALL && slots.expert_of != nullptr;  // uniform over the launch
+    static_assert(!OWN || (SWIGLU && TT < TALL), "");
     SlotsLds& sl = *reinterpret_cast<SlotsLds*>(As);
     static_assert(sizeof(SlotsLds) <= (STAGES - 1) * BM * CPR * sizeof(uint4), "in front of the tokens");
     int* const own_token = reinterpret_cast<int*>(As + (STAGES - 1) * BM * CPR);
     RoutedCounts rc{};
-    if (own) {
+    if constexpr (OWN) {
         if (blockIdx.x == gridDim.x - 1) return routed_rest(slots, reinterpret_cast<unsigned char*>(As));
         rc = routed_counts<NT>(slots, sl);
     }
-    const TileAt at = tile_at<BN, BM>(own ? rc.ntiles : dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
+    const TileAt at = tile_at<BN, BM>(OWN ? rc.ntiles : dense_rows >= 0 ? (dense_rows + BM - 1) / BM : *ntiles, N, group_m, g2.rows, g2.N);
     if (at.tm < 0) return;
     const int tm_idx = at.tm, tn_idx = at.tn;
     if (at.second) {
@@ -579,7 +584,7 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
         expert = 0;
         row0 = tm_idx * BM;
         rows = min(BM, dense_rows - row0);
-    } else if (own) {
+    } else if constexpr (OWN) {
         const RoutedTile t = routed_tile<NT>(slots, rc, tm_idx, tn_idx == 0, sl, own_token);
         expert = t.expert;
         row0 = t.row0;
@@ -605,7 +610,8 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     // A last gate/up tile of at most 64 features leaves two waves without any: there the waves share out the token blocks as well,
     // two blocks of features by two halves of the rows.  us a forward, without / with: 64 experts of 704 (five and a half tiles), six a
     // row, and a shared one of 1408, d 1024, 16384 rows 648 / 642; 32 of 704, int8, four a row, 8192 rows 205 / 200.
-    const bool halves = SWIGLU && NW == 4 && nblk > 2 && N - tn_idx * BN <= 64;  // uniform over the workgroup
+    static_assert(!HALVES || (SWIGLU && NW == 4), "");
+    const bool halves = HALVES && nblk > 2 && N - tn_idx * BN <= 64;  // uniform over the workgroup
     const int column = halves ? wave & 1 : wave;
     // the wave's token blocks
     const int half = (nblk + 1) / 2, tb0 = halves ? (wave >> 1) * half : 0, tbs = halves ? min(half, nblk - tb0) : nblk;
@@ -615,8 +621,12 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     const bool act1 = SWIGLU ? act0 : (nw + NW * 32 < N);
     const size_t block_bytes = (size_t)K * 32 * (I8 ? 1 : 2);  // one block of 32 weight rows over all of K
     const char* wexp = static_cast<const char*>(wpacked) + (size_t)expert * w_expert_stride_bytes;
-    const char* wp0 = scalar_pointer(wexp + (size_t)(act0 ? r0 / 32 : 0) * block_bytes);
-    const char* wp1 = scalar_pointer(wexp + (size_t)(act1 ? r1 / 32 : 0) * block_bytes);
+    const char* wp0 = wexp + (size_t)(act0 ? r0 / 32 : 0) * block_bytes;
+    const char* wp1 = wexp + (size_t)(act1 ? r1 / 32 : 0) * block_bytes;
+    if constexpr (OWN || HALVES || TT == TALL) {
+        wp0 = scalar_pointer(wp0);
+        wp1 = scalar_pointer(wp1);
+    }
     const uint32_t lane16 = (uint32_t)lane * 16u;
 
     // ---- LDS-DMA of the activation slice --------------------------------------
@@ -633,7 +643,7 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     for (int j = 0; j < DMA_PER_WAVE; ++j) {
         const int r = wave * (BM / NW) + j * 8 + (lane >> 3);
         const int rr = r < rows ? r : 0;
-        const int grow = own && !at.second ? own_token[rr] : row_index ? row_index[row0 + rr] : row0 + rr;
+        const int grow = OWN && !at.second ? own_token[rr] : row_index ? row_index[row0 + rr] : row0 + rr;
         a_src[j] = ((uint32_t)grow * (uint32_t)K + 8u * ((lane & 7) ^ ((r >> 1) & 7))) * 2u;
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)As + wave * (BM / NW) * CPR * 16;
@@ -694,7 +704,7 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
             return;
         }
     }
-    write_tile<SWIGLU, I8, TT>(to, acc, reinterpret_cast<char*>(As), [] {});
+    write_tile<SWIGLU, I8, TT, HALVES>(to, acc, reinterpret_cast<char*>(As), [] {});
     RBMOE_TRACE_AT(blockIdx.x, 3);
 }
 
@@ -1061,15 +1071,30 @@ hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
         else if constexpr (!SWIGLU) narrow_go(std::true_type{});
         return hipGetLastError();
     }
-    auto go = [&](auto tt) {
-        RB_LAUNCH((grouped_stream_kernel<SWIGLU, I8, decltype(tt)::value>), dim3((total + 7) / 8 * 8 + rest), dim3(NT), 0, s,
+    auto launch = [&](auto tt, auto own, auto halves) {
+        RB_LAUNCH((grouped_stream_kernel<SWIGLU, I8, decltype(tt)::value, decltype(own)::value, decltype(halves)::value>), dim3((total + 7) / 8 * 8 + rest), dim3(NT), 0, s,
                   static_cast<const bf16_t*>(g.a), g.row_index, g.w, g.w_expert_stride * (I8 ? 1 : 2), g.scales,
                   g.s_expert_stride, g.N, g.K, g.tile_expert, g.tile_row0, g.tile_rows, g.ntiles, g.dense_rows,
                   static_cast<bf16_t*>(g.out), static_cast<bf16_t*>(g.gu_out), static_cast<const bf16_t*>(g.swiglu_grad_gu),
                   group_m, g2, g.slots);
     };
-    if (tall) go(std::integral_constant<int, TALL>{});
-    else go(std::integral_constant<int, TT>{});
+    if (tall && rest) return hipErrorInvalidValue;
+    const std::integral_constant<int, TT> whole{};
+    if constexpr (SWIGLU) {
+        auto half = [&](int n) { return (n + BN - 1) % BN < BN / 2; };  // (a last tile of at most half its features)
+        const bool halves = NW == 4 && (half(g.N) || (d2.rows > 0 && half(d2.N)));
+        constexpr std::bool_constant<NW == 4> some{};
+        const std::integral_constant<int, TALL> high{};
+        if (rest) launch(whole, std::true_type{}, some);
+        else if (tall && halves) launch(high, std::false_type{}, some);
+        else if (tall) launch(high, std::false_type{}, std::false_type{});
+        else if (halves) launch(whole, std::false_type{}, some);
+        else launch(whole, std::false_type{}, std::false_type{});
+    } else if (tall) {
+        launch(std::integral_constant<int, TALL>{}, std::false_type{}, std::false_type{});
+    } else {
+        launch(whole, std::false_type{}, std::false_type{});
+    }
     return hipGetLastError();
 }
 

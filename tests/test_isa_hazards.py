@@ -107,6 +107,19 @@ def test_registers_hold_as_many_routing_workgroups_as_the_plan_counts_on():
 
 
 @needs_hipcc
+def test_wide_products_that_read_the_tables_keep_their_scalars_in_registers():
+    """The code that works a launch's tiles out takes more scalar registers than there are, and a workgroup's first loads wait for
+    every move of one into a vector register and back: only the launches that need that code may carry it."""
+    found = dict(re.findall(r"\.name:\s+(_ZN\S*?21grouped_stream_kernel\S+)\n.*?\.sgpr_spill_count:\s+(\d+)\n", assembly("grouped_stream.hip"), re.S))
+    wide = {n: re.match(r".*grouped_stream_kernelILb(\d)ELb(\d)ELi(\d)E(.*?)EvPK", n).groups() for n in found}
+    for gate_up in "01":
+        for int8 in "01":
+            for blocks in "45":
+                spills = {n: int(found[n]) for n, f in wide.items() if f[:3] == (gate_up, int8, blocks) and not f[3].startswith("Lb1E")}
+                assert spills and not any(spills.values()), spills
+
+
+@needs_hipcc
 def test_static_scratch_array_is_a_symbol_the_runtime_can_look_up():
     # rbmoe_forward_static's scratch is a static device array whose address the host asks the runtime for by name
     # (hipGetSymbolAddress).  The runtime searches the code object's global symbols, and a missing one ends the

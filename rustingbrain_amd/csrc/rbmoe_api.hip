@@ -2537,11 +2537,24 @@ int rbmoe_get_weight_grad(rbmoe_layer* L, int32_t which, int32_t expert, float* 
         HIP_TRY(ctx, hipStreamSynchronize(s));
         return RBMOE_OK;
     }
-    HIP_TRY(ctx, hipStreamSynchronize(s));
-    if (pitch == want_cols)
+    if (pitch == want_cols) {
+        HIP_TRY(ctx, hipStreamSynchronize(s));
         HIP_TRY(ctx, hipMemcpy(host, src, bytes, hipMemcpyDeviceToHost));
-    else
-        HIP_TRY(ctx, hipMemcpy2D(host, want_cols * 4, src, pitch * 4, want_cols * 4, want_rows, hipMemcpyDeviceToHost));
+        return RBMOE_OK;
+    }
+    // Rows of a rounded width into memory of the caller's own: through a block of the pool, since a rectangular copy into plain memory
+    // is a copy a row there, 7 us each.
+    Staging stage;
+    if (!stage.take(want_rows * pitch * 4)) return fail(ctx, RBMOE_OUT_OF_MEMORY, "no host memory for the gradient's rows");
+    size_t apart = want_cols * 4;  // bytes from row to row of the block
+    if (stage.pinned()) {
+        HIP_TRY(ctx, hipMemcpy2DAsync(stage.p, apart, src, pitch * 4, apart, want_rows, hipMemcpyDeviceToHost, s));
+    } else {
+        apart = pitch * 4;
+        HIP_TRY(ctx, hipMemcpyAsync(stage.p, src, want_rows * apart, hipMemcpyDeviceToHost, s));
+    }
+    HIP_TRY(ctx, hipStreamSynchronize(s));
+    for (size_t r = 0; r < want_rows; ++r) std::memcpy(host + r * want_cols, stage.p + r * apart, want_cols * 4);
     return RBMOE_OK;
 }
 

@@ -1,6 +1,9 @@
 """Expert widths between two multiples of a matrix-core tile: the kernels see them rounded up with zero rows and
 columns, callers see their own widths (outputs, hidden rows, gradients).  Not where the rows are f32 and the weights are
 not: the matrix cores would take them as bf16, so such layers keep the any-shape kernels and f32 accuracy."""
+import ctypes as C
+import time
+
 import numpy as np
 import pytest
 
@@ -104,3 +107,26 @@ def test_a_memory_budget_that_holds_the_true_widths_is_enough(device, training):
         dev.close()
     small = names.index("mfma_bf16_stream")
     assert 0 < small and names == ["generic"] * small + ["mfma_bf16_stream"] * (len(names) - small)
+
+
+@pytest.mark.parametrize("d,F", [(64, 33), (256, 130)])   # below and above the size of results in pinned memory
+def test_gradients_of_rounded_widths_reach_plain_memory_without_a_copy_a_row(device, d, F):
+    """Into an array of the caller's own: the values that a pinned one gets, in at most five times the time of a gradient whose rows
+    lie side by side (about as long here; 25 to 110 times as long with a rectangular copy into plain memory)."""
+    def fetch(width):
+        layer = rb.MoeLayer(d, rb.MoeConfig(2, 1, width), device, act_dtype="f32", weight_dtype="f32", max_tokens=16)
+        layer.enable_training()
+        layer.load_tensors(synth.make(small_workload(d=d, E=2, k=1, F=width, T=16, seed=65)))
+        layer.forward_train(synth.normal((16, d), 1.0, 65, 1).astype(np.float32))
+        layer.backward(synth.normal((16, d), 1.0, 65, 2).astype(np.float32))
+        got, seconds = np.empty((d, width), np.float32), []
+        for _ in range(15):
+            start = time.perf_counter()
+            assert device._lib.rbmoe_get_weight_grad(layer.handle, L.W_DOWN, 1, got.ctypes.data_as(C.POINTER(C.c_float)), d, width) == L.OK
+            seconds.append(time.perf_counter() - start)
+        pinned = device.empty((1 << 20,), np.float32)[:d * width]
+        assert device._lib.rbmoe_get_weight_grad(layer.handle, L.W_DOWN, 1, pinned.ctypes.data_as(C.POINTER(C.c_float)), d, width) == L.OK
+        assert got.any() and np.array_equal(got.ravel(), pinned)
+        layer.close()
+        return sorted(seconds)[7]
+    assert fetch(F) <= 5 * fetch((F + 31) // 32 * 32)

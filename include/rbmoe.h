@@ -133,7 +133,8 @@ const char* rbmoe_last_global_error(void);
  * allocating (src/param.rs:172-189), allocates weights (zeroed) and workspace.
  * Expert widths between two multiples of a matrix-core tile are stored rounded up (bf16 rows: to 64, at most four
  * times the width; all-f32 layers: to 32, at most twice), which takes that much more memory.  f32 rows over bf16 or int8
- * weights are not rounded: at widths off 64 they keep those widths and f32 accuracy, at multiples of 64 the
+ * weights keep f32 accuracy at widths off 64 (stored rounded up to 32, at most twice the width, where the context has no
+ * memory budget, and as they are under one); at multiples of 64 the
  * products take a bf16 copy of the rows (RBMOE_OPT_FORCE_GENERIC: f32 accuracy there too, at a thirtieth of the rate).  A layer whose rounded
  * widths are over the budget - here, or when the norm or training mode is added before the first weight - or over a limit
  * of the backward products keeps its true widths instead (bf16 rows then take the any-shape kernels).  Layers that already hold

@@ -381,9 +381,16 @@ void choose_kernel_sets(rbmoe_layer* L) {
         // f32 rows over other weights: whole slices, like the all-f32 products.  us a forward, as they are / rounded, bf16 weights: d 512, 8
         // experts of 1365 (1376), 3 rows 47.0 / 28.3, 300 66.8 / 46.5, 8000 347 / 267; d 1024, 8 of 910 (928) and a shared one, 30 rows 51.5 /
         // 38.7, 2000 157 / 128; d 256, 8 of 341 (352), 3 rows 27.2 / 24.0, 8000 87.6 / 72.8, of 227 (256), 1000 rows 34.3 / 30.3; int8 alike.
+        // Twice the work on narrow experts is made good by the whole pieces (of 33 (64), d 64, 3 and 3000 rows 21.9 / 21.1, 26.6 / 25.9; of 17
+        // (32), d 1024, 48.8 / 46.9), and so it is where the model width has no whole slices and gate/up fetches element by element all
+        // the same: d 33, of 50 (64), 25.1 / 25.0, 31.7 / 29.8; d 72, of 33, 24.2 / 23.3, 28.2 / 27.1; d 250, of 341, 36.5 / 32.9, 191 / 181; d 1000,
+        // of 227, 42.2 / 39.8, 518 / 503 (int8 1044 / 1033); 216 such shapes 0.99 to 1.55 times as fast.
         // A training step over host matrices, d 256, 16 of 341 and a shared one, 200 rows 1450 / 1443, 4000 3590 / 2200.
-        L->Fw = L->f32_rows ? rounded(cfg->d_ff, 32, 2) : cfg->d_ff;
-        L->Fsw = L->f32_rows ? rounded(L->Fs, 32, 2) : L->Fs;
+        // Not under a memory budget, which may be laid out for layers of their true widths: several layers, or a norm set behind
+        // training mode, which nothing makes room for.
+        const bool rounds = L->f32_rows && (!L->ctx || L->ctx->budget_bytes == 0);
+        L->Fw = rounds ? rounded(cfg->d_ff, 32, 2) : cfg->d_ff;
+        L->Fsw = rounds ? rounded(L->Fs, 32, 2) : L->Fs;
     }
     const int block = L->tight ? kRouterTokens : kMinRouterTokens;  // tokens of the smallest router block
     L->max_nb = (cfg->max_tokens + block - 1) / block;
@@ -403,8 +410,8 @@ const char* training_widths_problem(const rbmoe_layer* L) {
                (!f32_shape_ok((int)d, (int)(2 * F)) || (c.shared_expert && !f32_shape_ok((int)d, (int)(2 * Fs))))) {
         return "expert width not supported by the backward products";
     }
-    return "";  // (any other layer - odd widths, mixed dtypes - takes its widths as they are in both directions: f32 rows
-                // through launch_grouped_f32, bf16 rows on the any-shape kernels)
+    return "";  // (any other layer - odd widths, mixed dtypes - takes any widths in both directions: f32 rows through
+                // launch_grouped_f32, bf16 rows on the any-shape kernels)
 }
 
 Plan make_plan(rbmoe_layer* L) {

@@ -1,6 +1,7 @@
 """Expert widths between two multiples of a matrix-core tile: the kernels see them rounded up with zero rows and
-columns, callers see their own widths (outputs, hidden rows, gradients).  Not where the rows are f32 and the weights are
-not: the matrix cores would take them as bf16, so such layers keep the any-shape kernels and f32 accuracy."""
+columns, callers see their own widths (outputs, hidden rows, gradients).  Where the rows are f32 and the weights are not, the
+bf16 matrix cores would take the rows as bf16: such layers keep f32 accuracy and are rounded to slices of 32 only, and not
+under a memory budget."""
 import ctypes as C
 import time
 
@@ -130,3 +131,26 @@ def test_gradients_of_rounded_widths_reach_plain_memory_without_a_copy_a_row(dev
         layer.close()
         return sorted(seconds)[7]
     assert fetch(F) <= 5 * fetch((F + 31) // 32 * 32)
+
+
+@pytest.mark.parametrize("layers", [1, 2])
+def test_a_memory_budget_that_holds_true_widths_holds_every_layer_and_what_follows(device, layers):
+    """f32 rows over bf16 weights, F 33 of slices of 32: what fits a budget fits every larger one, whether the budget is shared by
+    several layers or a norm follows training mode (a layer that took more than its true widths while there was room would leave none)."""
+    E, d, F, T = 8, 1024, 33, 200
+    fits = []
+    for mib in range(1, 80):
+        dev = rb.Device.open(0, budget_mib=mib)
+        made = []
+        try:
+            for _ in range(layers):
+                made.append(rb.MoeLayer(d, rb.MoeConfig(E, 2, F), dev, act_dtype="f32", weight_dtype="bf16", max_tokens=T))
+                made[-1].enable_training()
+                made[-1].set_feed_forward_norm(np.ones(d, np.float32))
+            fits.append(True)
+        except rb.MemoryBudget:
+            fits.append(False)
+        for layer in made:
+            layer.close()
+        dev.close()
+    assert True in fits and all(fits[fits.index(True):]), fits

@@ -2749,6 +2749,24 @@ int rbmoe_internal_widths(const rbmoe_config* cfg, int32_t training, int32_t* ou
     return RBMOE_OK;
 }
 
+// The plan of a large-batch call on aligned rows (none of the addresses is read).
+static void plan_of_aligned_rows(int32_t d, int32_t E, int32_t k, int32_t T, int32_t bf16, int32_t norm, int32_t quantized, int32_t exact,
+                                 RouterPlan* out) {
+    RouterArgs a{};
+    a.T = T; a.d = d; a.E = E; a.k = k;
+    a.allow_fused = true;
+    a.exact = exact != 0;
+    a.x = reinterpret_cast<void*>((uintptr_t)1 << 20);
+    a.wr = static_cast<const float*>(a.x);
+    if (quantized) {
+        a.wq = static_cast<const int8_t*>(a.x);
+        a.wscale = a.wr;
+    }
+    if (norm) a.norm_w = a.wr;
+    a.arrive = reinterpret_cast<int*>((uintptr_t)1 << 20);
+    *out = plan_router(a, bf16 != 0);
+}
+
 // Test hook (not part of rbmoe.h), runs without a GPU: how a large-batch call on rows at address `x` (never read) is routed.
 // out[0]: tokens of a router block as the dispatch counts them, [1]: whether the norm takes a launch of its own, [2]: whether
 // the router's launch takes the plan with the arguments it gets, [3]: tokens of a block when the stage is replayed, [4]: whether
@@ -2790,19 +2808,20 @@ int rbmoe_internal_router_plan(int32_t d, int32_t E, int32_t k, int32_t T, int32
 // Test hook (not part of rbmoe.h), runs without a GPU: experts of a routing workgroup of a large-batch call on aligned rows, 0
 // where a block's experts are not shared out.
 int rbmoe_internal_router_slice(int32_t d, int32_t E, int32_t k, int32_t T, int32_t bf16, int32_t norm, int32_t quantized, int32_t exact) {
-    RouterArgs a{};
-    a.T = T; a.d = d; a.E = E; a.k = k;
-    a.allow_fused = true;
-    a.exact = exact != 0;
-    a.x = reinterpret_cast<void*>((uintptr_t)1 << 20);  // (never read)
-    a.wr = static_cast<const float*>(a.x);
-    if (quantized) {
-        a.wq = static_cast<const int8_t*>(a.x);
-        a.wscale = a.wr;
-    }
-    if (norm) a.norm_w = a.wr;
-    a.arrive = reinterpret_cast<int*>((uintptr_t)1 << 20);
-    return plan_router(a, bf16 != 0).row_slice;
+    RouterPlan p;
+    plan_of_aligned_rows(d, E, k, T, bf16, norm, quantized, exact, &p);
+    return p.row_slice;
+}
+
+// Test hook (not part of rbmoe.h), runs without a GPU: the launch that keeps rows in LDS in such a call.  out[0]: router rows that lie
+// there together, 0 where another launch takes the call, [1]: tokens of its blocks, [2]: bytes of LDS of a workgroup.
+void rbmoe_internal_router_rows(int32_t d, int32_t E, int32_t k, int32_t T, int32_t bf16, int32_t norm, int32_t quantized, int32_t exact,
+                                int32_t* out) {
+    RouterPlan p;
+    plan_of_aligned_rows(d, E, k, T, bf16, norm, quantized, exact, &p);
+    out[0] = p.row_experts;
+    out[1] = p.row_experts ? p.block_tokens : 0;
+    out[2] = p.row_experts ? (int32_t)p.row_lds : 0;
 }
 
 // Test hook (not part of rbmoe.h), runs without a GPU: rows of the tiles of a matrix-core call of so many routed rows.

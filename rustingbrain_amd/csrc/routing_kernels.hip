@@ -1105,14 +1105,20 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize, bool exact) {
     // d 256, 32 experts, 8500 rows 64.5 / 52.3, 30000 128 / 90; 64 experts, 4500 rows 62.1 / 50.2, 8192 82.8 / 54.7; d 512, 32 experts,
     // 8500 rows 94.6 / 71.2, 48 experts, 16384 160 / 113; d 768, 32 experts, 12000 rows 137 / 108, 64 experts, 8192 170 / 92; d 1024, 32
     // experts, 4500 rows 115 / 82, 64 experts, 16384 337 / 248; d 2048, 32 experts, 12000 rows 316 / 308; quantized, d 768, 32 experts,
-    // 16384 rows 184 / 155, d 1024, 64 experts, 8500 rows 220 / 164.  Not where route_fused_kernel has long rows: d 768, 20 experts,
-    // 12000 rows 93.5 / 97.4, d 1024, 24 experts, 8500 rows 105 / 113 (d 512, 20 experts, 8500 rows 65.7 / 65.5).  Up to 16 experts as
-    // above: d 768, 16 experts, 16384 rows 123 / 133.
-    const bool any_f32 = !p.exact && xsize == 4 && a.E > 16 && (a.wq || a.d <= 512 || fused_cols(a, xsize) == 0);
+    // 16384 rows 184 / 155, d 1024, 64 experts, 8500 rows 220 / 164.  Not where route_fused_kernel has the rows (up to 26 experts and 256 K
+    // pairs): d 768, 20 experts, 12000 rows 93.5 / 97.4, d 1024, 24 experts, 8500 rows 105 / 113, d 512, 22 experts, 10500 rows 67.7 / 71.4, d 128,
+    // 20 experts, 8500 rows 39.1 / 40.7; without it d 128, 28 experts, 4200 rows 41.7 / 36.9, d 512, 31 experts 74.9 / 52.9, 24 experts, 12000
+    // rows 98.3 / 75.2, d 64, 24 experts, 16384 and 20000 rows 45.5 / 43.0, 52.7 / 54.2.  Under a quantized router there too, d 640, 24
+    // experts, 8300 rows 94.1 / 84.8, d 1280, 17 experts, 5000 rows 99.2 / 89.3, but not in little more than one round of workgroups of which
+    // a unit takes one: d 768, 20 and 28 experts, 9000 rows 95.3 / 102.2, 105.5 / 114.5, d 896, 30 experts, 8300 rows 122 / 128 (d 896, 20
+    // experts, 10500 rows 129 / 118).  Up to 16 experts as above: d 768, 16 experts, 16384 rows 123 / 133.
+    const bool any_f32 = !p.exact && xsize == 4 && a.E > 16 && (a.wq || fused_cols(a, xsize) == 0);
     const bool any_size = (p.exact && a.E > 16) || any_f32;
     if (!any_size && ((long long)a.T * a.E > 256 * 1024 || blocks > together)) p.tokens = 0;
     if (p.exact && exact_loses(a.d, a.E, p.tokens, blocks, a.wq != nullptr)) p.tokens = 0;
-    if (p.tokens > kMinRouterTokens && !p.exact && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4)) p.tokens = 0;
+    // (over f32 rows without a quantized router rows_lose's lines are drawn against route_fused_kernel)
+    if (p.tokens > kMinRouterTokens && !p.exact && !(any_f32 && !a.wq) && rows_lose(a.d, a.E, p.tokens, a.wq != nullptr, xsize == 4))
+        p.tokens = 0;
     // In several rounds a workgroup's loads, sums and softmax follow one another with nothing beside them where it fills a compute
     // unit's LDS by itself.  So blocks and router rows are made smaller until two lie there together, if they can be: experts past
     // those whose rows lie in LDS follow through the place of the ones before, and blocks of 16 tokens take the router's rows twice as
@@ -1122,8 +1128,13 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize, bool exact) {
     // 32 experts 75.7 / 72.9, 93.1 / 87.1, 139 / 130, 64 experts 101 / 91, 115 / 105, 172 / 156; quantized, d 512, 48 experts, 16384 rows
     // 104 / 91; 64 experts of 704, six a row, and a shared one, d 1024, 16384 rows 658 / 648.  (In one round, 5000 rows: 1 to 2 %,
     // not taken; narrower rows lie there twice as they are, wider ones do not fit.)
-    // f32 rows: d 512, 32 experts of 256, 12000 rows 93.9 / 88.1; d 1024, 64 experts of 704, six a row, 6000 rows 300 / 285, 16384 635 / 627,
-    // but 32 experts of 256, 12000 rows 165.4 / 171.1.
+    // f32 rows: d 256, 48 experts, 12000 rows 72.6 / 66.2; d 512, 17 and 32 experts, 8500 rows 74.4 / 64.4, 77.8 / 72.4; d 768, 40 experts 107 / 102;
+    // d 1024, 64 experts, 8500, 16384 rows 183 / 165, 257 / 255.  The gain is the last round's, which two workgroups beside one another make
+    // shorter.  Where that is more than half full and half as large blocks take the router's rows in twice as many groups, there is none: d 512,
+    // 40 experts, 13000 and 16384 rows (1.6 and 2 rounds) 94.1 / 97.1, 107.4 / 110.8, but 10240 (1.25) 89.1 / 85.1; d 768, 48 experts, 13000 rows
+    // 128.5 / 134.9; d 1024, 32 experts, 12000, 15500, 20000 rows (2.9, 3.8, 4.9) 143.8 / 149.5, 177.5 / 185.9, 216.5 / 225.9, 13000 (3.2) 165.6 /
+    // 162.6 (40 experts, in whole groups, 2 to 3 % faster all the same, not taken: 20000 rows 243 / 236).  A quantized router's sums take longer
+    // than its rows: d 512, 40 experts, 16384 rows 140 / 135, d 1024, 32 experts 202 / 194.
     if (((p.exact && p.tokens == kRouterTokens) || (any_f32 && p.tokens)) && blocks > 256 && p.lds > (size_t)kMaxRouterLds / 2)
         for (int t = p.tokens; t >= std::max(a.min_tokens, p.tokens / 2); t /= 2) {
             const int least = p.exact ? exact_round(t, NL) : 8;
@@ -1131,11 +1142,14 @@ static RowsPlan plan_rows(const RouterArgs& a, size_t xsize, bool exact) {
             while (EG > least && rows_lds(a, p.exact, t, EG) > (size_t)kMaxRouterLds / 2)
                 EG = p.exact ? exact_fewer(EG, t, NL) : (EG - 1) & ~1;
             if (rows_lds(a, p.exact, t, EG) > (size_t)kMaxRouterLds / 2) continue;
+            auto groups = [&](int eg) { return (a.E + eg - 1) / eg; };
+            if (any_f32 && !a.wq && t < p.tokens && (blocks - 1) % 256 >= 128 && groups(EG) >= 2 * groups(p.EG)) continue;
             p.tokens = t;
             p.EG = EG;
             p.lds = rows_lds(a, p.exact, t, EG);
             break;
         }
+    if (any_f32 && a.wq && p.tokens && blocks > 256 && blocks <= 320 && p.lds > (size_t)kMaxRouterLds / 2 && fused_cols(a, xsize) != 0) p.tokens = 0;
     // A few tokens by many experts: one workgroup a block would take the experts' rows through its own LDS one group after the
     // other (64 experts of d 1024: 27 us, whatever the tokens).  So the block's experts are shared out, eight to a workgroup
     // or as many as leave at most one round of workgroups; the last to arrive does the rest.  us a forward, one workgroup / shared

@@ -35,6 +35,16 @@ def router_slice(d, E, k, T, bf16, norm, quantized, exact=0):
     return fn(d, E, k, T, bf16, norm, quantized, exact)
 
 
+def rows_launch(d, E, k, T, bf16=0, norm=0, quantized=0, exact=0):
+    """(router rows in LDS together, tokens of a block, bytes of LDS) of the launch that keeps rows in LDS; zeros where another takes the call."""
+    fn = L.load().rbmoe_internal_router_rows
+    fn.restype = None
+    fn.argtypes = [C.c_int32] * 8 + [C.POINTER(C.c_int32)]
+    out = (C.c_int32 * 3)()
+    fn(d, E, k, T, bf16, norm, quantized, exact, out)
+    return tuple(out)
+
+
 @pytest.mark.parametrize("exact", [0, 1])
 @pytest.mark.parametrize("quantized", [0, 1])
 @pytest.mark.parametrize("norm", [0, 1])
@@ -100,3 +110,29 @@ def test_where_the_matrix_cores_take_the_rows(d, E, T, quantized, taken):
     assert routes_on_matrix_cores(d, E, 2, T, quantized=quantized) == taken
     if not taken:  # what the rows of any other router get
         assert plan(d, E, 2, T, 1, 0, quantized, 1, ALIGNED, 1) == plan(d, E, 2, T, 1, 0, quantized, 1, ALIGNED, 0)
+
+
+# f32 rows, (d, experts, tokens, quantized): router rows in LDS together, tokens of a block and whether two workgroups lie on a unit, on either
+# side of each line of the rule
+F32_ROWS = [
+    # up to 16 experts one round of workgroups or two a unit; more in any number of rounds, except where route_fused_kernel has the rows
+    (512, 16, 9000, 0, (0, 0, False)), (512, 26, 9000, 0, (0, 0, False)), (512, 27, 9000, 0, (20, 16, True)),
+    (512, 24, 10922, 0, (0, 0, False)), (512, 24, 10923, 0, (20, 16, True)),
+    (128, 20, 8200, 0, (0, 0, False)), (128, 28, 4200, 0, (28, 32, True)), (64, 24, 16384, 0, (24, 32, True)),
+    (768, 24, 10922, 0, (0, 0, False)), (1024, 64, 16384, 0, (10, 8, True)),
+    # a quantized router: there too, but not in up to a round and a quarter of workgroups of which a unit takes one
+    (640, 24, 8300, 1, (14, 16, True)), (768, 20, 8193, 1, (0, 0, False)), (768, 20, 10240, 1, (0, 0, False)),
+    (768, 20, 10241, 1, (12, 32, False)), (768, 30, 8800, 1, (12, 32, False)),
+    # two workgroups a unit, unless blocks are halved, router rows taken in twice as many groups and the last round more than half full
+    (512, 40, 8192 + 128 * 32, 0, (18, 16, True)), (512, 40, 8193 + 128 * 32, 0, (40, 32, False)), (512, 40, 16384, 0, (40, 32, False)),
+    (512, 40, 16385, 0, (18, 16, True)),
+    (512, 20, 16384, 0, (20, 16, True)), (1024, 32, 12000, 0, (20, 16, False)), (1024, 32, 13000, 0, (10, 8, True)),
+    (1024, 28, 12000, 0, (10, 8, True)),
+    (512, 32, 16384, 1, (0, 0, False)), (1024, 32, 16384, 1, (8, 8, True)),
+]
+
+
+@pytest.mark.parametrize("d,E,T,quantized,want", F32_ROWS)
+def test_where_f32_rows_lie_in_lds(d, E, T, quantized, want):
+    EG, tokens, lds = rows_launch(d, E, 2, T, quantized=quantized)
+    assert (EG, tokens, EG > 0 and 2 * lds <= 160 * 1024) == want

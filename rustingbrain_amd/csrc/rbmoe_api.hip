@@ -257,6 +257,7 @@ struct rbmoe_layer {
     bool decode_down_by_expert = true;  // behind a decode_front launch: the down launch's workgroup rows are experts, not tile-table entries
     bool last_front = false;   // the last forward's hidden rows are per expert over all rows (Work::hall)
     bool last_by_slot = false; // ... and its expert rows lie in slot order
+    bool last_few = false;     // ... by launch_decode_down_few
     int last_parts = 1;          // ... the parts that the last forward's expert rows lie in (CombineArgs::parts)
     int group_m = 0;
     const char* kernel_name = "none";
@@ -1117,6 +1118,9 @@ bool starts_on_piece(const void* rows) { return reinterpret_cast<uintptr_t>(rows
 // small-route kernel itself for a few tokens, by the norm kernel otherwise - before anything reads it.
 // `static_scratch` (rbmoe_forward_static): this device's copy of the static scratch array; the call must then be
 // decode-shaped, keeps every intermediate result there and touches none of the layer's workspace.
+// What the tile table of so many routed rows will hold about: a last tile half full, or one tile each.
+int likely_tiles(int rows, int E, int tile_m) { return std::max(rows / tile_m + E / 2, std::min(E, rows)); }
+
 // `timing`: 0 none; 1 an event between the stages (rbmoe_forward_timed); 2 every stage's dispatches carry their own
 // start and stop events (rbmoe_forward_kernel_times).
 int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* valid, const float* router_bias,
@@ -1364,6 +1368,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         L->last = wk_;
         L->last_front = front;
         L->last_parts = 1;
+        L->last_few = few;
         L->last_by_slot = front && (few || by_expert);
         return RBMOE_OK;
     }
@@ -1514,7 +1519,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     g1.tile_rows = (const int*)L->tile_rows.p;
     g1.ntiles = (const int*)L->ntiles.p;
     g1.max_tiles = T > 0 ? (T * k) / tile_m0 + E : 0;
-    g1.likely_tiles = std::max((T * k) / tile_m0 + E / 2, std::min(E, T * k));  // a last tile half full, or one tile each
+    g1.likely_tiles = likely_tiles(T * k, E, tile_m0);
     g1.tile_m = tile_m0;
     g1.routed_rows = T * k;
     g1.groups = E;
@@ -1571,7 +1576,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     GroupedArgs second = shared_inside ? with_shared(g2, s2) : g2;
     if ((L->f32_rows || (mfma && d % 8 == 0)) && !L->training && T > 0 && d % 4 == 0 && k <= 8 &&
         (L->f32_rows || !c.shared_expert || shared_inside)) {
-        second.parts = mfma ? stream_parts(second) : f32_parts(second, wk);
+        second.parts = mfma ? stream_parts(second, wk, k) : f32_parts(second, wk);
         // (where the buffers hold as many rows of f32)
         while (second.parts > 1 && ((size_t)second.parts * T * k * d * 4 > L->y.bytes ||
                                     (shared_inside && (size_t)second.parts * T * d * 4 > L->ys.bytes)))
@@ -1604,6 +1609,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     L->last = wk_;
     L->last_parts = second.parts;
     L->last_front = false;
+    L->last_few = false;
     L->last_by_slot = false;
     return RBMOE_OK;
 }
@@ -2826,6 +2832,35 @@ void rbmoe_internal_router_rows(int32_t d, int32_t E, int32_t k, int32_t T, int3
 
 // Test hook (not part of rbmoe.h), runs without a GPU: rows of the tiles of a matrix-core call of so many routed rows.
 int rbmoe_internal_stream_tile(int32_t rows, int32_t E, int32_t F, int32_t d) { return stream_tile_m(rows, E, F, d); }
+
+// Test hook (not part of rbmoe.h), runs without a GPU: the parts of the down product's reduction in a matrix-core call of T rows, with a
+// shared expert of width Fs (0: none) in the launch.
+int rbmoe_internal_stream_parts(int32_t T, int32_t E, int32_t k, int32_t F, int32_t Fs, int32_t d, int32_t int8) {
+    GroupedArgs g{};
+    g.N = d;
+    g.K = F;
+    g.tile_m = kStreamTileM;
+    g.max_tiles = (T * k) / kStreamTileM + E;
+    g.likely_tiles = likely_tiles(T * k, E, kStreamTileM);
+    g.routed_rows = T * k;
+    g.dense_rows = -1;
+    if (Fs) {
+        g.dense2.N = d;
+        g.dense2.K = Fs;
+        g.dense2.rows = T;
+    }
+    return stream_parts(g, int8 ? WeightKind::I8 : WeightKind::BF16, k);
+}
+
+// Test hook (not part of rbmoe.h): how the last forward's products ran.  out[0]: rows of the tiles, [1]: parts of the down product's
+// reduction, [2]: whether a row or two took launch_decode_down_few.
+int rbmoe_internal_last_products(const rbmoe_layer* L, int32_t* out) {
+    if (!L || !out) return RBMOE_NULL_POINTER;
+    out[0] = L->last_tile_m;
+    out[1] = L->last_parts;
+    out[2] = L->last_few ? 1 : 0;
+    return RBMOE_OK;
+}
 
 int rbmoe_copy_device(rbmoe_ctx* ctx, void* dst, const void* src, size_t bytes) {
     if (!ctx) return fail(nullptr, RBMOE_NULL_POINTER, "ctx is NULL");

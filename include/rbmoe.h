@@ -337,7 +337,7 @@ int rbmoe_forward_timed(rbmoe_layer* layer, const void* x, int32_t T, int32_t co
  * inside kernels, which is less than the forward took by the gaps between the launches.  Synchronises.  Where the
  * gate/up launch does the dispatch's work, RBMOE_STAGE_DISPATCH is 0.  A large-batch call's shared expert has launches of its
  * own on the main stream here, like rbmoe_forward_timed's; one that is not timed may have it inside the routed experts'
- * launches or beside them. */
+ * launches or beside them.  A reduction that the call shares out over workgroups is shared out alike in both. */
 int rbmoe_forward_kernel_times(rbmoe_layer* layer, const void* x, int32_t T, int32_t cols,
                                const uint8_t* valid, const float* router_bias, const void* residual,
                                void* out, float* ms);

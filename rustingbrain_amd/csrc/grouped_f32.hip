@@ -825,12 +825,15 @@ int f32_workgroups(const GroupedArgs& g, WeightKind wk) {
 // chain gives: d 512, 8 of 1408, 1024 rows (144) 94.5 / 101.1 / 98.5.
 // Errors against 64 bits become smaller (d 512, 8 of 1408, 1 row 4.0e-7 / 3.1e-7, 64 rows 4.7e-7 / 4.2e-7).  What is taken again (see
 // `odd`) is so part by part: infinities and NaN meet in the combine's sum as they would in the whole one.
+// Whole slices of every tile that either group may get, by itself too (a stage's replay): of 64 columns where the widths have them.
 int f32_parts(const GroupedArgs& g, WeightKind wk) {
     const F32Plan p = f32_plan(g, wk == WeightKind::F32 ? 4 : wk == WeightKind::BF16 ? 2 : 1);
-    const int slice = p.tile == F32Tile::T32x32 ? 64 : 32, K = g.dense2.rows > 0 ? std::min(g.K, g.dense2.K) : g.K;
-    if (!p.aligned || g.K % slice != 0 || (g.dense2.rows > 0 && g.dense2.K % slice != 0)) return 1;
+    const int K2 = g.dense2.rows > 0 ? g.dense2.K : g.K;
+    if (!p.aligned) return 1;
+    auto slices = [](int K) { return K % 64 == 0 ? K / 64 : K / 32; };
+    const int most = std::min(slices(g.K), slices(K2));
     int parts = 1;
-    while (parts < 4 && 2 * parts * p.workgroups <= 256 && 2 * parts * slice <= K) parts *= 2;
+    while (parts < 4 && 2 * parts * p.workgroups <= 256 && 2 * parts <= most) parts *= 2;
     return parts;
 }
 

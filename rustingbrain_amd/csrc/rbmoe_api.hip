@@ -1436,9 +1436,10 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // 8 of 1408, 512 rows 111 / 123, 1024 (572) 179 / 158.
     constexpr int kSharedInsideF32Tiles = 400;
     const int f32_tiles = ((T * k) / 64 + (E + 1) / 2) * ((F + 127) / 128) + (T + 63) / 64 * ((Fs + 127) / 128);
-    const bool shared_inside = c.shared_expert && !timed && T > 0 &&
-                               (mfma ? T < 1024 || gate_up_tiles <= kSharedInsideTiles
-                                     : L->f32_rows && f32_joins(F, Fs) && (T < 1024 || f32_tiles <= kSharedInsideF32Tiles));
+    const bool shared_joins = c.shared_expert && T > 0 &&
+                              (mfma ? T < 1024 || gate_up_tiles <= kSharedInsideTiles
+                                    : L->f32_rows && f32_joins(F, Fs) && (T < 1024 || f32_tiles <= kSharedInsideF32Tiles));
+    const bool shared_inside = shared_joins && !timed;
     auto with_shared = [&](GroupedArgs g, const GroupedArgs& sh) {
         g.dense2 = {sh.a, sh.w, sh.scales, sh.N, sh.K, sh.dense_rows, sh.out, sh.gu_out};
         return g;
@@ -1573,20 +1574,24 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // rows, which are wider, for the down product (measured HBM-side traffic: 270 against 301 MB with groups of 8
     // against 4 for gate/up, 147 against 166 MB with 4 against 8 for down)
     if (L->group_m == 0) g2.group_m = 4;
-    GroupedArgs second = shared_inside ? with_shared(g2, s2) : g2;
+    // The parts of the reduction are those of the call that is not timed, also where its shared expert has launches of its own here
+    // and in the stage's replay, which is the routed experts' alone.
+    const GroupedArgs call = shared_joins ? with_shared(g2, s2) : g2;
     if ((L->f32_rows || (mfma && d % 8 == 0)) && !L->training && T > 0 && d % 4 == 0 && k <= 8 &&
-        (L->f32_rows || !c.shared_expert || shared_inside)) {
-        second.parts = mfma ? stream_parts(second, wk, k) : f32_parts(second, wk);
+        (L->f32_rows || !c.shared_expert || shared_joins)) {
+        g2.parts = mfma ? stream_parts(call, wk, k) : f32_parts(call, wk);
         // (where the buffers hold as many rows of f32)
-        while (second.parts > 1 && ((size_t)second.parts * T * k * d * 4 > L->y.bytes ||
-                                    (shared_inside && (size_t)second.parts * T * d * 4 > L->ys.bytes)))
-            second.parts /= 2;
-        second.part_rows = T * k;
+        while (g2.parts > 1 && ((size_t)g2.parts * T * k * d * 4 > L->y.bytes ||
+                                (shared_joins && (size_t)g2.parts * T * d * 4 > L->ys.bytes)))
+            g2.parts /= 2;
+        g2.part_rows = T * k;
+        if (shared_joins) {
+            s2.parts = g2.parts;
+            s2.part_rows = T;
+        }
     }
-    HIP_TRY(ctx, run(second, false));
-    GroupedArgs down = second;
-    if (down.parts == 1) down = g2;
-    L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return run_on(down, st); };
+    HIP_TRY(ctx, run(shared_inside ? with_shared(g2, s2) : g2, false));
+    L->replay[RBMOE_STAGE_DOWN] = [=](hipStream_t st) { return run_on(g2, st); };
     HIP_TRY(ctx, mark(5));
 
     if (c.shared_expert && T > 0 && !shared_forked && !shared_inside) HIP_TRY(ctx, shared_expert(s));
@@ -1599,15 +1604,15 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     CombineArgs ca{L->y.p, c.shared_expert ? L->ys.p : nullptr, residual, (const int*)L->inv_pos.p,
                    (const float*)L->gate_of.p, T, d, k, out};
     ca.rows_bf16 = cast;
-    ca.parts = second.parts;
-    ca.shared_in_parts = shared_inside;
-    ca.part_rows = second.part_rows;
+    ca.parts = g2.parts;
+    ca.shared_in_parts = shared_joins;
+    ca.part_rows = g2.part_rows;
     HIP_TRY(ctx, launch_combine(ca, abf, s));
     L->replay[RBMOE_STAGE_COMBINE] = [=](hipStream_t st) { return launch_combine(ca, abf, st); };
     HIP_TRY(ctx, mark(7));
     L->last_T = T;
     L->last = wk_;
-    L->last_parts = second.parts;
+    L->last_parts = g2.parts;
     L->last_front = false;
     L->last_few = false;
     L->last_by_slot = false;

@@ -72,6 +72,18 @@ def gpu_layer(device, t: synth.Tensors, max_tokens: Optional[int] = None, aux_w:
     return layer
 
 
+def last_products(layer):
+    """(rows of the tiles, parts of the down product's reduction, whether a row or two's own down launch ran) of the last forward."""
+    import ctypes as C
+    from rustingbrain_amd import _lib as L
+    out = (C.c_int32 * 3)()
+    fn = L.load().rbmoe_internal_last_products
+    fn.restype = C.c_int
+    fn.argtypes = [C.c_void_p, C.POINTER(C.c_int32)]
+    assert fn(layer.handle, out) == L.OK
+    return out[0], out[1], bool(out[2])
+
+
 def assert_routing_identical(cache, ref) -> None:
     """Bit-exact comparands: indices, counts, permutation — and, because the
     router arithmetic is a fixed sequence, probabilities, lse and gates too."""

@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 from bench import DeviceBuffer
-from helpers import gpu_layer, small_workload
+from conftest import rel_l2
+from helpers import gpu_layer, last_products, small_workload
 from rustingbrain_amd import _lib as L
 from rustingbrain_amd import synth
 
@@ -79,6 +80,46 @@ def test_kernel_times_are_those_of_the_calls_own_launches(device, act, E, inside
     kt = layer.forward_kernel_times(xb.ptr, 300, ob.ptr)
     assert (kt["dispatch"] == 0) == inside and min(kt["router"], kt["gate_up"], kt["down"], kt["combine"]) > 0
     assert layer.forward_timed(xb.ptr, 300, ob.ptr)["dispatch"] > 0
+    layer.close()
+    xb.free()
+    ob.free()
+
+
+@pytest.mark.parametrize("act,wt,shape,parts", [
+    ("bf16", "bf16", dict(d=64, E=4, k=2, F=1408, T=40, shared_d_ff=1408), 4),
+    ("bf16", "int8", dict(d=768, E=8, k=2, F=1408, T=90, shared_d_ff=2112), 2),
+    ("f32", "int8", dict(d=128, E=4, k=1, F=1472, T=120, shared_d_ff=1472), 4),     # products over a bf16 copy of the rows
+    ("f32", "f32", dict(d=64, E=4, k=2, F=704, T=33, shared_d_ff=704), 4),
+    ("f32", "bf16", dict(d=512, E=4, k=2, F=96, T=33, shared_d_ff=96), 2),
+])
+def test_timed_forwards_share_a_reduction_out_as_the_call_does(device, act, wt, shape, parts):
+    """The shared expert rides in the call's own launches and has launches of its own in the timed ones; the parts of the reduction
+    are the same in both, and in the replay of the down product, which is the routed experts' alone.  Bits are, too, where the rows
+    are bf16; over f32 rows a launch of fewer tiles may sum in another order (1e-6: some roundings of 2^-24)."""
+    t = synth.make(small_workload(seed=93, act=act, wt=wt, shared=True, **shape))
+    T = shape["T"]
+    layer = gpu_layer(device, t, max_tokens=8 * T)
+    x = synth.f32_to_bf16_bits(t.x) if act == "bf16" else t.x
+    xb, ob = DeviceBuffer(device, x.nbytes).upload(x), DeviceBuffer(device, x.nbytes)
+
+    def output():
+        device.synchronize()
+        return ob.download(np.empty_like(x)).copy()
+
+    def same(a, b):
+        return rel_l2(a, b) <= 1e-6 if wt == act == "f32" or shape["F"] == 96 else np.array_equal(a.view(np.uint8), b.view(np.uint8))
+
+    layer.forward_device(xb.ptr, T, ob.ptr)
+    plain = output()
+    assert last_products(layer)[1] == parts
+    for measured in (layer.forward_timed, layer.forward_kernel_times):
+        ob.upload(np.zeros_like(x))
+        assert measured(xb.ptr, T, ob.ptr)["shared"] > 0
+        assert last_products(layer)[1] == parts and same(output(), plain)
+    layer.forward_device(xb.ptr, T, ob.ptr)
+    rows = layer.expert_rows(int(layer.cache(T).offsets[-1]))[1]
+    assert layer.enqueue_stage("down", 1) and layer.enqueue_stage("combine", 1)
+    assert same(output(), plain) and same(layer.expert_rows(rows.size // shape["d"])[1], rows)
     layer.close()
     xb.free()
     ob.free()

@@ -138,7 +138,11 @@ const char* rbmoe_last_global_error(void);
  * products take a bf16 copy of the rows (RBMOE_OPT_FORCE_GENERIC: f32 accuracy there too, at a thirtieth of the rate).  A layer whose rounded
  * widths are over the budget - here, or when the norm or training mode is added before the first weight - or over a limit
  * of the backward products keeps its true widths instead (bf16 rows then take the any-shape kernels).  Layers that already hold
- * weights stay as they are: a budget shared by several layers has to allow for their rounded widths. */
+ * weights stay as they are: a budget shared by several layers has to allow for their rounded widths.
+ * Small calls share a long down product's reduction out over workgroups, whose f32 sums are added in a fixed order; the rule looks at
+ * the call's shape alone, so a call's bits do not depend on max_tokens.  Under a memory budget, in the layout of true widths
+ * and in training mode, whose backward pass reads the rows, no reduction is shared out: the same call's rows may there differ in their last
+ * bits (f32 sums in another order; bf16 rows by a rounding now and then). */
 int rbmoe_layer_create(rbmoe_ctx* ctx, const rbmoe_config* cfg, rbmoe_layer** out);
 void rbmoe_layer_destroy(rbmoe_layer* layer);
 

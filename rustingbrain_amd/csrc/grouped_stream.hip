@@ -1105,12 +1105,18 @@ hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
 // rows: a wave's weight fragments, which are two thirds of what passes a compute unit's L1, serve five multiplies instead of four, and
 // there are fewer first loads and last stores.  Against that, launches end in whole tiles, and one table serves both products.  So
 // the lengths are estimated - tiles a compute unit, 0.3 of the way to the next whole number, by the tile's reduction and 800 columns
-// for its ends - and the tall tiles taken where they gain 1 %, above the sizes that the narrow kernel, a shared expert in the
-// launch and gate/up launches that make the tables take.  us a forward, 128 / 160, measured (estimated gain): d 768, 8 experts of 1408, 6000
+// for its ends - and the tall tiles taken where they gain 2 %, above the sizes that the narrow kernel, a shared expert in the
+// launch and gate/up launches that make the tables take.  How the rows fall on the experts is not known, and a last round more or less
+// is 3 to 4 %: of 200 calls measured where the estimate speaks for them by 1 % (64 shapes, bf16 and int8, evenly spread and a third of the
+// rows to one expert) they are 1.5 % faster on average and 19 slower by more than 1.5 %, of the 164 with 2 % 1.9 % faster and 8 slower (by 4 %
+// at most).  Not for calls with padding, whose rows are fewer than the host knows: 30 of 100 slower by more than 1.5 %, 0.2 % faster on
+// average.  us a forward, 128 / 160, measured (estimated gain): d 768, 8 experts of 1408, 6000
 // rows 113.2 / 108.1 (8 %), 10000 155.7 / 157.6 (1 %, not taken), 16384 235.3 / 224.2 (7 %); 16 of them, 6000 121.2 / 112.7 (8 %),
 // 16384 251.4 / 246.1 (4 %); d 512, 8 of 352, 16384 90.5 / 83.4 (9 %); d 1024, 32 of 1408, four a row, 6000 256.6 / 244.8 (2 %),
-// 16384 592 / 567 (4 %); 64 of 704, six a row, 6000 237.7 / 231.0 (2 %), 16384 522 / 508 (3 %); d 256, 32 of 704, four a row, 10000 104.1 /
-// 104.7 (3 %), 16384 143.9 / 135.9 (5 %).  Not taken: d 1024, 32 of 352, four a row, 10000 164.9 / 167.3, d 512, 8 of 1408, 6000 88.9 / 89.6.
+// 16384 592 / 567 (4 %); 64 of 704, six a row, 16384 522 / 508 (3 %); d 256, 32 of 704, four a row, 10000 104.1 /
+// 104.7 (3 %), 16384 143.9 / 135.9 (5 %).  Slower all the same: d 1024, 16 of 704, four a row, 8400 246 /
+// 253.  Not taken: d 1024, 32 of 352, four a row, 10000 164.9 / 167.3, d 512, 8 of 1408, 6000 88.9 / 89.6, d 768, 8 of 1408, 8400 149.5 / 154.8,
+// d 1024, 16 of 704, four a row, 5300 176.7 / 180.5, 64 of 704, six a row, 6000 237.7 / 231.0.
 int stream_tile_m(int rows, int groups, int F, int d) {
     auto tiles = [&](int bm) { return std::max((double)rows / bm + 0.5 * groups, (double)std::min(groups, rows)); };
     const int gate_up = (F + 127) / 128, down = (d + 255) / 256;
@@ -1119,7 +1125,7 @@ int stream_tile_m(int rows, int groups, int F, int d) {
         auto units = [&](double n) { return n <= 256 ? 1.0 : 0.3 * std::ceil(n / 256) + 0.7 * n / 256; };
         return (d + 800) * units(tiles(bm) * gate_up) + (F + 800) * units(tiles(bm) * down);
     };
-    return length(BM) > 1.01 * 1.19 * length(rows_of(TALL)) ? rows_of(TALL) : BM;
+    return length(BM) > 1.02 * 1.19 * length(rows_of(TALL)) ? rows_of(TALL) : BM;
 }
 
 // A narrow down launch of few tiles waits for a chain of slices that holds a fraction of the compute units.  Its reduction is shared out

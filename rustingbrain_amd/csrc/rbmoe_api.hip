@@ -1188,8 +1188,8 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
 
     const bool mfma = L->use_stream;
     const bool f32mc = L->use_f32_mc;
-    // (training: no gain from tall tiles where gate/up also stores the pre-activations)
-    const int tile_m0 = mfma ? (L->training ? kStreamTileM : stream_tile_m(T * k, E, F, d))
+    // (training: no gain from tall tiles where gate/up also stores the pre-activations; padding: fewer rows than are counted here)
+    const int tile_m0 = mfma ? (L->training || valid ? kStreamTileM : stream_tile_m(T * k, E, F, d))
                              : (L->f32_rows ? f32_tile_m(T * k, E) : kGenericTileM);
     L->last_tile_m = tile_m0;
     L->kernel_name = mfma ? (wk == WeightKind::I8 ? "mfma_bf16_stream_int8w" : "mfma_bf16_stream")

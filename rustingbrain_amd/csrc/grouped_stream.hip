@@ -11,8 +11,8 @@
 //                int8 weights are widened to bf16 in registers during the step
 //                before their multiplies; the per-row scale multiplies the
 //                accumulator.
-//   activations  128 token rows per workgroup (gathered through an index for
-//                the gate/up product) go global -> LDS with the LDS-DMA load
+//   activations  128 token rows per workgroup, 160 in tall tiles (gathered through
+//                an index for the gate/up product) go global -> LDS with the LDS-DMA load
 //                (global_load_lds_dwordx4): lane l of a wave deposits its 16
 //                bytes at LDS base + 16 l, so the XOR swizzle that keeps the
 //                fragment reads free of bank conflicts is applied by choosing
@@ -26,7 +26,7 @@
 //                by itself: every memory instruction of the main loop sits
 //                behind a multiply of its own (see pipe_loop).
 // A workgroup is 4 waves side by side along the output features; a wave owns
-// 128 tokens x 64 weight rows (32 gate + the matching 32 up rows, or 64 down
+// all its tokens x 64 weight rows (32 gate + the matching 32 up rows, or 64 down
 // rows).  The weight fragment is the matrix-core A operand and the token
 // fragment the B operand, so a lane ends with 4 consecutive output features of
 // one token and writes them with one 8-byte store.  Token blocks of 32 rows
@@ -178,8 +178,8 @@ struct TileOut {
     const bf16_t* bw_gu;
 };
 
-// `stage`: 32 KiB of LDS that no wave of the workgroup reads or writes any more (the caller has made sure of
-// that with a barrier).  `before_stores()` is called once, when the first pass has been converted and staged and
+// `stage`: 256 bytes of LDS a row of the tile (32 KiB, tall tiles 40) that no wave of the workgroup reads or writes any more (the
+// caller has made sure of that with a barrier).  `before_stores()` is called once, when the first pass has been converted and staged and
 // before its first store to memory is issued.
 template <bool SWIGLU, bool I8, int TT, bool HALVES, typename F>
 __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][TT], char* const stage,
@@ -205,7 +205,7 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
     // Accumulator element v of block (b, t): feature 8*(v/4) + 4*(lane/32) + v%4 of the
     // wave's row block b, token t*32 + lane%32 - a lane holds 4 consecutive features of a
     // token, so a direct store would scatter 8-byte pieces over 32 rows per instruction.
-    // Instead each block index goes through LDS as a 128-token x 128-feature tile (16-byte
+    // Instead each block index goes through LDS as a tile of all its rows x 128 features (16-byte
     // pieces, piece p of row r kept at position p ^ (r % 16)), and is written out with
     // 16-byte stores, 16 consecutive lanes covering the 256 contiguous bytes of a row.
     // Passes through the staging tile: down product: the two blocks of 128 features; gate/up: the
@@ -219,7 +219,8 @@ __device__ __forceinline__ void write_tile(const TileOut& o, floatx16 (&acc)[2][
     for (int bh = 0; bh < PASSES * SUB; ++bh) {
         const int b = bh / SUB, h = bh % SUB;
         if constexpr (SWIGLU) {
-            if (b > 0 && gu_out == nullptr) break;  // uniform over the launch
+            // (uniform over the launch; a training layer's tiles are never tall)
+            if (b > 0 && (TT >= TALL || gu_out == nullptr)) break;
         }
         if (bh) __syncthreads();  // the previous pass has been read out
         if ((wave / WH) == h && (SWIGLU ? act0 : (b ? act1 : act0))) {
@@ -630,8 +631,8 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     const uint32_t lane16 = (uint32_t)lane * 16u;
 
     // ---- LDS-DMA of the activation slice --------------------------------------
-    // Wave w fills LDS rows [32 w, 32 w + 32): instruction j covers rows 32 w + 8 j .. + 7,
-    // lane l lands in row 8 j + l / 8 (of the wave's 32), position l % 8, and therefore
+    // Wave w fills a quarter of the LDS rows, from BM / NW * w on (32 rows, 40 of a tall tile): instruction j covers 8 of them,
+    // lane l lands in row 8 j + l / 8 (of the wave's), position l % 8, and therefore
     // fetches logical piece (l % 8) ^ ((row / 2) % 8): a 16-lane group of a fragment read
     // (16 consecutive rows, one logical piece) then touches 8 distinct pieces in the even rows
     // and 8 in the odd rows, i.e. all 64 banks once.  Rows past the end of the group are
@@ -697,7 +698,7 @@ __global__ __launch_bounds__(NT, RBMOE_STREAM_OCC) void grouped_stream_kernel(
     __syncthreads();  // every wave's last DMA has landed and its last fragment reads are done
     const TileOut to{rows, row0, tn_idx, N, act0, act1, r0, r1, tb0, tbs, column,
                      I8 ? scales + (size_t)expert * s_expert_stride : nullptr, out, gu_out, bw_gu};
-    if constexpr (!SWIGLU && !I8) {
+    if constexpr (!SWIGLU && !I8 && TT < TALL) {
         if (bw_gu != nullptr) {  // uniform over the launch
             write_swiglu_backward<TT>(to, acc, reinterpret_cast<char*>(As));
             RBMOE_TRACE_AT(blockIdx.x, 3);
@@ -1160,6 +1161,7 @@ hipError_t launch_grouped_stream(const GroupedArgs& g, WeightKind wk, hipStream_
         return hipErrorInvalidValue;
     if (g.slots.expert_of && (!g.swiglu || g.dense_rows >= 0 || g.slots.layout.tile_m != BM)) return hipErrorInvalidValue;
     if (g.dense_rows < 0 && g.tile_m != BM && g.tile_m != rows_of(TALL)) return hipErrorInvalidValue;
+    if (g.dense_rows < 0 && g.tile_m == rows_of(TALL) && (g.gu_out || g.swiglu_grad_gu)) return hipErrorInvalidValue;
     if (g.swiglu_grad_gu && (g.swiglu || wk != WeightKind::BF16)) return hipErrorInvalidValue;
     if (wk == WeightKind::BF16) return g.swiglu ? launch_t<true, false>(g, s) : launch_t<false, false>(g, s);
     if (wk == WeightKind::I8) return g.swiglu ? launch_t<true, true>(g, s) : launch_t<false, true>(g, s);

@@ -1053,8 +1053,9 @@ __global__ __launch_bounds__(512) void decode_down_by_expert_kernel(DecodeGemmAr
 // than the one trip; and here nothing is fetched of experts without rows.  us a call, before / now: one row of the default model
 // 12.25 / 11.2, without the norm 11.1 / 10.1; d 768, 8 experts of 1408, two rows 14.9 / 13.65, one row with a shared expert 15.9 /
 // 14.1; int8, d 1024, two rows 16.1 / 15.5.  Behind route_small_kernel 25.4 / 24.8 (one row, 16 experts).
-// As many steps are requested at once as the wave has, and no more (BATCH): with room for 12 where there are 3, the last one
-// asked for over and over, one row of the default model took 12.4.
+// A wave requests all its steps at once, up to eleven: BATCH is 3, 6 or 11, and a wave of fewer asks for its last step over and over (two
+// of six times at 512 columns, three of eleven at 1024).  Far too many cost more than they save: with room for 12 where there are 3,
+// one row of the default model took 12.4.
 // ---------------------------------------------------------------------------
 constexpr int kFewPairs = 4;  // pairs of a call at most
 

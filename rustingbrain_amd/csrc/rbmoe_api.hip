@@ -1079,6 +1079,9 @@ bool decode_front_pays(const rbmoe_layer* L, int T, bool stages_rows, bool norme
 //     d 512, 4 rows 0.87 / 0.99, 6 rows 1.06 / 1.12; staged: 16 experts, d 768, 12 rows (147 K) 44.8 us / 43.3.  Over 32 experts
 //     and 32 K router weights the routing that shares them out is ahead sooner: 64 experts, d 512, 1 row 0.89 / 0.99, 2 rows
 //     1.05 / 1.19, 4 rows - / 1.56; d 1024, 1 row 1.38 / 1.54, 8 rows 3.2.
+// Where the lines are known to be off: four experts a row and more than 72 slots (16 and 32 experts, 1.2 to 1.67; d 1024, 32 experts of 256,
+// 32 rows 53.7 us / 32.1), a block step over 32 experts that are routed alone (d 768, 4 rows 43.6 / 29.4), int8, 8 experts, d 1024, 16 to 24
+// rows (46.8 / 33.0), 32 experts of 704 at d 768 and of 1408 at d 256, 24 to 28 rows (1.1 to 1.26).
 bool decode_front_beats_batch(const rbmoe_layer* L, int T) {
     const rbmoe_config& c = L->cfg;
     const int slots = T * c.experts_per_token, E = c.num_experts;

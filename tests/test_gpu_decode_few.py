@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 import rustingbrain_amd as rb
-from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
+from conftest import rel_l2
+from helpers import assert_routing_identical, gpu_layer, last_products, oracle_layer, small_workload
 from rustingbrain_amd import _lib as L
 from rustingbrain_amd import synth
 
@@ -43,9 +44,23 @@ def test_gives_the_bits_of_the_tile_table_launch(device, case, wt, front):
         for _ in range(2):
             out, cache = layer.forward_train(t.x, layout, residual=residual)
             assert ("front" in layer.kernel_name()) == front
+            # (int8 weights behind a routing launch of its own stay with the tile table: nothing to compare, the launch is not taken)
+            assert last_products(layer)[2] == (by_expert == 1 and (front or wt == "bf16"))
             assert_routing_identical(cache, ref)
             got.append((out, layer.expert_rows(R)[1] if R else np.zeros(0, np.float32)))
     for out, rows in got[1:]:
         assert np.array_equal(out.view(np.uint32), got[0][0].view(np.uint32))
         assert np.array_equal(rows.view(np.uint32), got[0][1].view(np.uint32))
+    layer.close()
+
+
+@pytest.mark.parametrize("shape,few", [(dict(k=2, T=2), True), (dict(k=4, T=1), True), (dict(k=3, T=2), False), (dict(k=2, T=3), False),
+                                       (dict(k=3, T=1, shared=True), True), (dict(k=4, T=1, shared=True), False),
+                                       (dict(k=1, T=2, shared=True), True)])
+def test_up_to_four_pairs_of_a_row_and_a_side(device, shape, few):
+    t = synth.make(small_workload(d=128, E=8, F=64, seed=62, act="bf16", wt="bf16", **shape))
+    layer = gpu_layer(device, t)
+    out, _ = layer.forward_train(t.x)
+    assert "decode" in layer.kernel_name() and last_products(layer)[2] == few
+    assert rel_l2(out, oracle_layer(t).forward(t.x, threads=4).out) <= 1e-2
     layer.close()

@@ -2858,23 +2858,24 @@ void rbmoe_internal_router_rows(int32_t d, int32_t E, int32_t k, int32_t T, int3
 // Test hook (not part of rbmoe.h), runs without a GPU: rows of the tiles of a matrix-core call of so many routed rows.
 int rbmoe_internal_stream_tile(int32_t rows, int32_t E, int32_t F, int32_t d) { return stream_tile_m(rows, E, F, d); }
 
-// Test hook (not part of rbmoe.h), runs without a GPU: the parts of the down product's reduction in a matrix-core call of T rows, with a
-// shared expert of width Fs (0: none) in the launch.
-int rbmoe_internal_stream_parts(int32_t T, int32_t E, int32_t k, int32_t F, int32_t Fs, int32_t d, int32_t int8) {
+// Test hook (not part of rbmoe.h), runs without a GPU: the parts of the down product's reduction in a large-batch call of T rows, with a
+// shared expert of width Fs (0: none) in the launch.  f32_rows: of launch_grouped_f32 (weight_dtype any), otherwise of the matrix-core
+// kernels over bf16 rows (bf16 or int8 weights).
+int rbmoe_internal_parts(int32_t T, int32_t E, int32_t k, int32_t F, int32_t Fs, int32_t d, int32_t f32_rows, int32_t weight_dtype) {
+    const WeightKind wk = weight_dtype == RBMOE_F32 ? WeightKind::F32 : weight_dtype == RBMOE_I8 ? WeightKind::I8 : WeightKind::BF16;
     GroupedArgs g{};
     g.N = d;
     g.K = F;
-    g.tile_m = kStreamTileM;
-    g.max_tiles = (T * k) / kStreamTileM + E;
-    g.likely_tiles = likely_tiles(T * k, E, kStreamTileM);
+    g.a = g.w = reinterpret_cast<const void*>((uintptr_t)1 << 20);  // (never read)
+    g.w_expert_stride = (size_t)d * F;
+    g.tile_m = f32_rows ? f32_tile_m(T * k, E) : kStreamTileM;
+    g.max_tiles = (T * k) / g.tile_m + E;
+    g.likely_tiles = likely_tiles(T * k, E, g.tile_m);
     g.routed_rows = T * k;
+    g.groups = E;
     g.dense_rows = -1;
-    if (Fs) {
-        g.dense2.N = d;
-        g.dense2.K = Fs;
-        g.dense2.rows = T;
-    }
-    return stream_parts(g, int8 ? WeightKind::I8 : WeightKind::BF16, k);
+    if (Fs) g.dense2 = {g.a, g.w, nullptr, d, Fs, T, nullptr, nullptr};
+    return f32_rows ? f32_parts(g, wk) : stream_parts(g, wk, k);
 }
 
 // Test hook (not part of rbmoe.h): how the last forward's products ran.  out[0]: rows of the tiles, [1]: parts of the down product's

@@ -15,10 +15,10 @@ from test_reduction_parts import stream_parts
 
 pytestmark = pytest.mark.gpu
 
-# f32 rows, and the parts without and with a shared expert of the same width: slices of 64 columns: 22 and 11 in quarters (5 or 6, 2 or 3
-# each), 3 in halves, 1 whole; of 32 columns (F = 96, 352)
-SHAPES = [(dict(d=64, E=4, k=2, F=1408, T=1), (4, 4)), (dict(d=64, E=4, k=4, F=704, T=33), (4, 4)), (dict(d=128, E=3, k=1, F=192, T=70), (2, 2)),
-          (dict(d=128, E=4, k=3, F=64, T=5), (1, 1)), (dict(d=96, E=4, k=2, F=96, T=9), (2, 2)), (dict(d=512, E=8, k=2, F=352, T=40), (4, 2)),
+# f32 rows, and the parts without and with a shared expert of the same width: slices of 64 columns: 22, 11 and 5 in quarters (5 or 6, 2 or 3, 1
+# or 2 each), 22 in halves, 1 whole; of 32 columns: 9 and 11
+SHAPES = [(dict(d=64, E=4, k=2, F=1408, T=1), (4, 4)), (dict(d=64, E=4, k=4, F=704, T=33), (4, 4)), (dict(d=128, E=3, k=1, F=320, T=70), (4, 4)),
+          (dict(d=128, E=4, k=3, F=64, T=5), (1, 1)), (dict(d=96, E=4, k=2, F=288, T=9), (4, 4)), (dict(d=512, E=8, k=2, F=352, T=40), (4, 2)),
           (dict(d=512, E=8, k=2, F=1408, T=64), (2, 1))]
 
 

@@ -1,4 +1,4 @@
-"""Where a matrix-core call's down product is shared out over workgroups: on either side of the lines that were measured."""
+"""Where the down product of a large-batch call is shared out over workgroups: on either side of the lines that were measured."""
 import ctypes as C
 
 import pytest
@@ -6,11 +6,15 @@ import pytest
 from rustingbrain_amd import _lib as L
 
 
-def stream_parts(T, E, k, F, Fs, d, int8):
-    fn = L.load().rbmoe_internal_stream_parts
+def parts(T, E, k, F, Fs, d, f32_rows, weight_dtype):
+    fn = L.load().rbmoe_internal_parts
     fn.restype = C.c_int
-    fn.argtypes = [C.c_int32] * 7
-    return fn(T, E, k, F, Fs, d, int8)
+    fn.argtypes = [C.c_int32] * 8
+    return fn(T, E, k, F, Fs, d, f32_rows, weight_dtype)
+
+
+def stream_parts(T, E, k, F, Fs, d, int8):
+    return parts(T, E, k, F, Fs, d, 0, L.I8 if int8 else L.BF16)
 
 
 @pytest.mark.parametrize("d,E,k,F,Fs,T,bf16,int8", [
@@ -25,3 +29,14 @@ def stream_parts(T, E, k, F, Fs, d, int8):
 ])
 def test_where_reductions_are_shared_out(d, E, k, F, Fs, T, bf16, int8):
     assert (stream_parts(T, E, k, F, Fs, d, 0), stream_parts(T, E, k, F, Fs, d, 1)) == (bf16, int8)
+
+
+# d, experts, a row, width, shared width, rows: while every workgroup has a compute unit to itself, in reductions of at least 288 columns
+@pytest.mark.parametrize("wt", [L.F32, L.BF16, L.I8])
+@pytest.mark.parametrize("d,E,k,F,Fs,T,want", [
+    (64, 4, 2, 1408, 0, 1, 4), (512, 8, 2, 352, 0, 40, 4), (512, 8, 2, 352, 352, 40, 2), (768, 8, 2, 1408, 0, 2, 2), (768, 8, 2, 1408, 0, 16, 1),
+    (512, 8, 2, 1408, 0, 1024, 1), (96, 4, 2, 288, 0, 9, 4), (96, 4, 2, 256, 0, 9, 1), (256, 8, 4, 256, 256, 65, 1), (128, 4, 3, 64, 0, 5, 1),
+    (96, 4, 2, 352, 256, 9, 1), (96, 4, 2, 350, 0, 9, 1),   # the shorter of the two; no whole slices
+])
+def test_where_reductions_over_f32_rows_are_shared_out(d, E, k, F, Fs, T, want, wt):
+    assert parts(T, E, k, F, Fs, d, 1, wt) == want

@@ -1103,14 +1103,15 @@ hipError_t launch_t(const GroupedArgs& g, hipStream_t s) {
 }  // namespace
 
 // Rows of the tiles of a call of so many routed rows: 128, or 160 (TALL).  A tall tile takes 1.19 times as long for 1.25 times the
-// rows: a wave's weight fragments, which are two thirds of what passes a compute unit's L1, serve five multiplies instead of four, and
-// there are fewer first loads and last stores.  Against that, launches end in whole tiles, and one table serves both products.  So
-// the lengths are estimated - tiles a compute unit, 0.3 of the way to the next whole number, by the tile's reduction and 800 columns
-// for its ends - and the tall tiles taken where they gain 2 %, above the sizes that the narrow kernel, a shared expert in the
-// launch and gate/up launches that make the tables take.  How the rows fall on the experts is not known, and a last round more or less
-// is 3 to 4 %: of 200 calls measured where the estimate speaks for them by 1 % (64 shapes, bf16 and int8, evenly spread and a third of the
-// rows to one expert) they are 1.5 % faster on average and 19 slower by more than 1.5 %, of the 164 with 2 % 1.9 % faster and 8 slower (by 4 %
-// at most).  Not for calls with padding, whose rows are fewer than the host knows: 30 of 100 slower by more than 1.5 %, 0.2 % faster on
+// rows: a wave's weight fragments, which are two thirds of what passes a compute unit's L1 (32 KiB a slice of 64 columns for the four
+// waves, beside 16 of rows), serve five multiplies instead of four, and there are fewer first loads and last stores.  Against that,
+// launches end in whole tiles, and one table serves both products.  So the lengths are estimated - tiles a compute unit, 0.3 of the
+// way to the next whole number, by the tile's reduction and 800 columns for its ends - and the tall tiles taken where they gain 2 %,
+// above the sizes that the narrow kernel, a shared expert in the launch and gate/up launches that make the tables take.  How the rows
+// fall on the experts is not known, and a last round more or less is 3 to 4 %: of 200 calls measured where the estimate speaks for
+// them by 1 % (ten layers of 3000 to 16384 rows, bf16 and int8, rows evenly spread and 30 % of them to one expert) they are 1.5 %
+// faster on average and 19 slower by more than 1.5 %, of the 164 with 2 % 1.9 % faster and 8 slower, by 4 % at most.  Not for calls
+// with padding, whose rows are fewer than the host knows: 30 of 100 with 30 % of it slower by more than 1.5 %, 0.2 % faster on
 // average.  us a forward, 128 / 160, measured (estimated gain): d 768, 8 experts of 1408, 6000
 // rows 113.2 / 108.1 (8 %), 10000 155.7 / 157.6 (1 %, not taken), 16384 235.3 / 224.2 (7 %); 16 of them, 6000 121.2 / 112.7 (8 %),
 // 16384 251.4 / 246.1 (4 %); d 512, 8 of 352, 16384 90.5 / 83.4 (9 %); d 1024, 32 of 1408, four a row, 6000 256.6 / 244.8 (2 %),

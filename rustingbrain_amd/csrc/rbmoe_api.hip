@@ -281,7 +281,6 @@ struct rbmoe_layer {
     Buf counts, offsets, tile_expert, tile_row0, tile_rows, ntiles, losses;
     Buf perm_slot, perm_token, inv_pos;
     Buf xg, h, y, hs, ys;
-    Buf parts;             // f32 expert rows (and the shared expert's behind them) of a reduction that is shared out (GroupedArgs::parts)
     Buf x16;               // [max_T, d] bf16 copy of f32 rows (cast_rows)
     Buf hall;              // [E][min(max_T, 32), F] hidden rows of decode_front launches
     Buf cmbcnt;            // [kDecodeCombineMaxBlocks] arrival counters of the folded decode combine, kRouterExactWord
@@ -417,15 +416,22 @@ const char* training_widths_problem(const rbmoe_layer* L) {
 }
 
 // Bytes for the down product's rows in parts: of at most half a million elements in quarters (stream_parts), or of 256 tiles of 64 x 128
-// (f32_parts), 8 MB both, and no more than the layer's largest call.  A buffer of its own, so that whether a call's reduction is shared
-// out, and with it the last bits of its rows, does not depend on the tokens that the layer has room for.  Not in the tight layout or
-// under a memory budget, which may be laid out for layers without it: there no reduction is shared out.
+// (f32_parts), 8 MB both, and no more than the layer's largest call.  Room of their own, so that whether a call's reduction is shared
+// out, and with it the last bits of its rows, does not depend on the tokens that the layer has room for; behind the expert rows, since an
+// allocation more would make a layer 20 us later.  Not in the tight layout or under a memory budget, which may be laid out for layers
+// without it: there no reduction is shared out.
 size_t parts_room(const rbmoe_layer* L) {
     const rbmoe_config& c = L->cfg;
     const bool may = (L->use_stream && c.d_model % 8 == 0) || (L->f32_rows && c.d_model % 4 == 0);
     if (!may || c.experts_per_token > 8 || L->tight || (L->ctx && L->ctx->budget_bytes)) return 0;
     const size_t rows = (size_t)L->max_S + (c.shared_expert ? (size_t)L->max_T : 0);
     return std::min(rows * c.d_model * 16, (size_t)8 << 20);
+}
+
+// Where that room begins in L->y.
+size_t parts_offset(const rbmoe_layer* L) {
+    const size_t bytes = (size_t)L->max_S * L->cfg.d_model * dtype_size(L->cfg.act_dtype);
+    return (bytes + 255) & ~(size_t)255;
 }
 
 Plan make_plan(rbmoe_layer* L) {
@@ -477,8 +483,7 @@ Plan make_plan(rbmoe_layer* L) {
     p.add(&L->cmbcnt, kDecodeCombineCounterBytes);
     p.add(&L->xg, S * d * as);
     p.add(&L->h, S * F * as);
-    p.add(&L->y, S * d * as);
-    if (const size_t room = parts_room(L)) p.add(&L->parts, room);
+    p.add(&L->y, parts_offset(L) + parts_room(L));
     p.add(&L->st_x, T * d * as);
     p.add(&L->st_out, T * d * as);
     p.add(&L->st_res, T * d * as);
@@ -1598,14 +1603,14 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         (L->f32_rows || !c.shared_expert || shared_joins)) {
         g2.parts = mfma ? stream_parts(call, wk, k) : f32_parts(call, wk);
         const size_t rows = (size_t)T * k + (shared_joins ? (size_t)T : 0);
-        while (g2.parts > 1 && g2.parts * rows * d * 4 > L->parts.bytes) g2.parts /= 2;
+        while (g2.parts > 1 && g2.parts * rows * d * 4 > parts_room(L)) g2.parts /= 2;
     }
     if (g2.parts > 1) {
-        g2.out = L->parts.p;
+        g2.out = static_cast<char*>(L->y.p) + parts_offset(L);
         g2.part_rows = T * k;
         wk_.y = g2.out;
         if (shared_joins) {
-            s2.out = static_cast<float*>(L->parts.p) + (size_t)g2.parts * T * k * d;
+            s2.out = static_cast<float*>(g2.out) + (size_t)g2.parts * T * k * d;
             s2.parts = g2.parts;
             s2.part_rows = T;
         }

@@ -44,8 +44,6 @@ def test_gives_the_bits_of_the_tile_table_launch(device, case, wt, front):
         for _ in range(2):
             out, cache = layer.forward_train(t.x, layout, residual=residual)
             assert ("front" in layer.kernel_name()) == front
-            # (int8 weights behind a routing launch of its own stay with the tile table: nothing to compare, the launch is not taken)
-            assert last_products(layer)[2] == (by_expert == 1 and (front or wt == "bf16"))
             assert_routing_identical(cache, ref)
             got.append((out, layer.expert_rows(R)[1] if R else np.zeros(0, np.float32)))
     for out, rows in got[1:]:
@@ -63,4 +61,20 @@ def test_up_to_four_pairs_of_a_row_and_a_side(device, shape, few):
     out, _ = layer.forward_train(t.x)
     assert "decode" in layer.kernel_name() and last_products(layer)[2] == few
     assert rel_l2(out, oracle_layer(t).forward(t.x, threads=4).out) <= 1e-2
+    layer.close()
+
+
+@pytest.mark.parametrize("front", [True, False])
+@pytest.mark.parametrize("wt", ["bf16", "int8"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "d{d}_E{E}_k{k}_F{F}_T{T}".format(**c))
+def test_the_launch_of_a_row_or_two_runs(device, case, wt, front):
+    t = synth.make(small_workload(d=case["d"], E=case["E"], k=case["k"], F=case["F"], T=case["T"], seed=61, act=case.get("act", "bf16"), wt=wt,
+                                  shared=case.get("shared", False), shared_d_ff=case.get("shared_d_ff", 0)))
+    layer = gpu_layer(device, t)
+    layer.set_option(L.OPT_DECODE_FRONT, int(front))
+    for by_expert in (1, 0):
+        layer.set_option(L.OPT_DECODE_DOWN_BY_EXPERT, by_expert)
+        layer.forward_train(t.x)
+        # (int8 weights behind a routing launch of its own stay with the tile table)
+        assert last_products(layer)[2] == (by_expert == 1 and (front or wt == "bf16"))
     layer.close()

@@ -9,7 +9,7 @@ import rustingbrain_amd as rb
 from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
 from oracle import rb_oracle as orc
 from rustingbrain_amd import synth
-from test_router_plan import routes_on_matrix_cores, rows_launch
+from test_router_plan import ALIGNED, plan, routes_on_matrix_cores, rows_launch
 
 pytestmark = pytest.mark.gpu
 
@@ -111,9 +111,14 @@ TWO_A_UNIT = [(dict(d=512, E=33, k=2, T=8225), False, 32), (dict(d=768, E=24, k=
 @pytest.mark.parametrize("form", ["plain", "one in a block"])
 @pytest.mark.parametrize("shape,quantized,tokens", TWO_A_UNIT, ids=lambda s: shape_id(s) if isinstance(s, dict) else str(s))
 def test_two_workgroups_a_unit(device, shape, quantized, tokens, form):
+    assert plan(shape["d"], shape["E"], shape["k"], shape["T"], 1, 0, int(quantized), 1, ALIGNED, 1)[0] == tokens
+    test_large_calls(device, shape, quantized, form)
+
+
+@pytest.mark.parametrize("shape,quantized,tokens", TWO_A_UNIT, ids=lambda s: shape_id(s) if isinstance(s, dict) else str(s))
+def test_room_for_two_workgroups_a_unit(shape, quantized, tokens):
     EG, block, lds = rows_launch(shape["d"], shape["E"], shape["k"], shape["T"], bf16=1, quantized=int(quantized), exact=1)
     assert EG > 0 and block == tokens and 2 * lds <= 160 * 1024
-    test_large_calls(device, shape, quantized, form)
 
 
 @pytest.mark.parametrize("shape,quantized", [(dict(d=1024, E=64, k=2, T=4200), False), (dict(d=1024, E=48, k=2, T=8190), True)])

@@ -7,7 +7,7 @@ from conftest import rel_l2
 from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload
 from oracle import rb_oracle as orc
 from rustingbrain_amd import Layout, synth
-from test_router_plan import rows_launch
+from test_router_plan import ALIGNED, plan, rows_launch
 
 pytestmark = pytest.mark.gpu
 
@@ -55,19 +55,32 @@ def test_block_step_routes_like_the_oracle(device, shape, act, quantized):
     layer.close()
 
 
+# More than 16 experts over f32 rows, several rounds of workgroups: blocks of 32, 16 and 8 tokens, the last one short, router rows in
+# one group and in several, and the line behind which route_fused_kernel keeps long rows.
+ROUNDS = [(dict(d=256, E=33, k=2, T=8225), False, 32), (dict(d=512, E=32, k=2, T=8195), False, 16),
+          (dict(d=1024, E=64, k=6, T=4201), False, 8), (dict(d=1024, E=40, k=2, T=4111), True, 8),
+          (dict(d=512, E=17, k=2, T=8200), False, 32), (dict(d=776, E=24, k=2, T=8200), False, 32)]
+
+
+@pytest.mark.parametrize("shape,quantized,tokens", ROUNDS, ids=lambda s: "d{d}_E{E}_k{k}_T{T}".format(**s) if isinstance(s, dict) else str(s))
+def test_several_rounds_over_f32_rows(device, shape, quantized, tokens):
+    assert plan(shape["d"], shape["E"], shape["k"], shape["T"], 0, 0, int(quantized), 1, ALIGNED)[0] == tokens
+    test_block_step_routes_like_the_oracle(device, shape, "f32", quantized)
+
+
 # More than 16 experts over f32 rows: (router rows in LDS together, tokens a block) in several rounds of workgroups, the last block short,
 # router rows in one group and in several, blocks that were halved and not; and one round where route_fused_kernel does not have the rows.
-ROUNDS = [(dict(d=256, E=33, k=2, T=8225), False, (33, 32)), (dict(d=512, E=32, k=2, T=8195), False, (20, 16)),
-          (dict(d=1024, E=64, k=6, T=4201), False, (10, 8)), (dict(d=1024, E=40, k=2, T=4111), True, (8, 8)),
-          (dict(d=512, E=28, k=2, T=8200), False, (20, 16)), (dict(d=512, E=24, k=2, T=10925), False, (20, 16)),
-          (dict(d=512, E=40, k=2, T=12291), False, (40, 32)), (dict(d=64, E=20, k=2, T=13111), False, (20, 32)),
-          (dict(d=128, E=28, k=2, T=4201), False, (28, 32)), (dict(d=768, E=20, k=2, T=10243), True, (12, 32)),
-          # not taken: route_fused_kernel has the rows
-          (dict(d=512, E=17, k=2, T=8200), False, (0, 0)), (dict(d=776, E=24, k=2, T=8200), False, (0, 0)),
-          (dict(d=768, E=20, k=2, T=8200), True, (0, 0))]
+ROWS_IN_LDS = [(dict(d=256, E=33, k=2, T=8225), False, (33, 32)), (dict(d=512, E=32, k=2, T=8195), False, (20, 16)),
+               (dict(d=1024, E=64, k=6, T=4201), False, (10, 8)), (dict(d=1024, E=40, k=2, T=4111), True, (8, 8)),
+               (dict(d=512, E=28, k=2, T=8200), False, (20, 16)), (dict(d=512, E=24, k=2, T=10925), False, (20, 16)),
+               (dict(d=512, E=40, k=2, T=12291), False, (40, 32)), (dict(d=64, E=20, k=2, T=13111), False, (20, 32)),
+               (dict(d=128, E=28, k=2, T=4201), False, (28, 32)), (dict(d=768, E=20, k=2, T=10243), True, (12, 32)),
+               # not taken: route_fused_kernel has the rows
+               (dict(d=512, E=17, k=2, T=8200), False, (0, 0)), (dict(d=776, E=24, k=2, T=8200), False, (0, 0)),
+               (dict(d=768, E=20, k=2, T=8200), True, (0, 0))]
 
 
-@pytest.mark.parametrize("shape,quantized,want", ROUNDS, ids=lambda s: "d{d}_E{E}_k{k}_T{T}".format(**s) if isinstance(s, dict) else str(s))
-def test_several_rounds_over_f32_rows(device, shape, quantized, want):
+@pytest.mark.parametrize("shape,quantized,want", ROWS_IN_LDS, ids=lambda s: "d{d}_E{E}_k{k}_T{T}".format(**s) if isinstance(s, dict) else str(s))
+def test_f32_rows_in_lds(device, shape, quantized, want):
     assert rows_launch(shape["d"], shape["E"], shape["k"], shape["T"], quantized=int(quantized))[:2] == want
     test_block_step_routes_like_the_oracle(device, shape, "f32", quantized)

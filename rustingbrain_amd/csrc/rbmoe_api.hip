@@ -1392,6 +1392,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
         L->last_parts = 1;
         L->last_few = few;
         L->last_by_slot = front && (few || by_expert);
+        L->x_saved = nullptr;
         return RBMOE_OK;
     }
 
@@ -2326,6 +2327,8 @@ int rbmoe_backward(rbmoe_layer* L, const void* grad_output, int32_t tokens, int3
     const int E = c.num_experts, d = c.d_model, F = L->Fw, k = c.experts_per_token, Fs = L->Fsw, T = L->last_T;
     if (T == 0) return RBMOE_OK;
     if (!grad_output || !grad_input) return fail(ctx, RBMOE_NULL_POINTER, "grad_output or grad_input is NULL");
+    // (a forward from before training mode has kept its rows only behind the norm)
+    if (!L->x_saved) return fail(ctx, RBMOE_INVALID_INPUT, "no forward pass has run in training mode yet");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
     const bool xbf = c.act_dtype == RBMOE_BF16;       // the caller's rows and gradients

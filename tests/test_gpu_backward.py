@@ -392,3 +392,23 @@ def test_f32_rows_over_bf16_weights_train_on_the_matrix_cores(device, shape):
     layer.backward(gout)
     assert rel_l2(layer.weight_grad(L.W_GATE, 1), 2.0 * once) <= 1e-6
     layer.close()
+
+
+@pytest.mark.parametrize("act,wt", [("bf16", "bf16"), ("f32", "bf16"), ("f32", "f32")])
+@pytest.mark.parametrize("T", [3, 300])
+def test_a_forward_from_before_training_mode_has_no_backward(device, act, wt, T):
+    """It keeps no rows for the router's gradient.  Behind the norm they are the layer's own, where the call's kernels are those of
+    training mode."""
+    t = synth.make(small_workload(d=64, E=4, k=2, F=64, T=T, seed=34, act=act, wt=wt))
+    layer = rb.MoeLayer(64, rb.MoeConfig(4, 2, 64), device, act_dtype=act, weight_dtype=wt, max_tokens=T)
+    layer.forward_train(t.x)
+    layer.enable_training()
+    with pytest.raises(rb.InvalidInput, match="training mode"):
+        layer.backward(t.x)
+    layer.load_tensors(t)
+    with pytest.raises(rb.InvalidInput, match="training mode"):
+        layer.backward(t.x)
+    layer.forward_train(t.x)
+    want = oracle_layer(t).backward(t.x, t.x, threads=4)
+    assert rel_l2(layer.backward(t.x), want.grad_input) <= (1e-5 if wt == "f32" else TOL)
+    layer.close()

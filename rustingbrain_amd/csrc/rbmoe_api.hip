@@ -1196,8 +1196,10 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
 
     const bool mfma = L->use_stream;
     const bool f32mc = L->use_f32_mc;
-    // (training: no gain from tall tiles where gate/up also stores the pre-activations; padding: fewer rows than are counted here)
-    const int tile_m0 = mfma ? (L->training || valid ? kStreamTileM : stream_tile_m(T * k, E, F, d))
+    // (training, which may still be switched on before the weights are set: no gain from tall tiles where gate/up also stores the
+    // pre-activations, and the backward takes this table; padding: fewer rows than are counted here)
+    const bool for_training = L->training || !L->weights_set;
+    const int tile_m0 = mfma ? (for_training || valid ? kStreamTileM : stream_tile_m(T * k, E, F, d))
                              : (L->f32_rows ? f32_tile_m(T * k, E) : kGenericTileM);
     L->last_tile_m = tile_m0;
     L->kernel_name = mfma ? (wk == WeightKind::I8 ? "mfma_bf16_stream_int8w" : "mfma_bf16_stream")
@@ -1600,7 +1602,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     // The parts of the reduction are those of the call that is not timed, also where its shared expert has launches of its own here
     // and in the stage's replay, which is the routed experts' alone.
     const GroupedArgs call = shared_joins ? with_shared(g2, s2) : g2;
-    if ((L->f32_rows || (mfma && d % 8 == 0)) && !L->training && T > 0 && d % 4 == 0 && k <= 8 &&
+    if ((L->f32_rows || (mfma && d % 8 == 0)) && !for_training && T > 0 && d % 4 == 0 && k <= 8 &&
         (L->f32_rows || !c.shared_expert || shared_joins)) {
         g2.parts = mfma ? stream_parts(call, wk, k) : f32_parts(call, wk);
         const size_t rows = (size_t)T * k + (shared_joins ? (size_t)T : 0);

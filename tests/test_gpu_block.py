@@ -9,6 +9,7 @@ import pytest
 import rustingbrain_amd as rb
 from conftest import rel_l2
 from helpers import assert_routing_identical, gpu_layer, oracle_layer, small_workload, tolerance
+from oracle import rb_oracle as orc
 from rustingbrain_amd import _lib as L
 from rustingbrain_amd import synth
 
@@ -269,4 +270,27 @@ def test_a_cached_decode_reproduces_the_full_sequence_forward(device, act, wt, d
     same_as_full(slice(0, 40), out, cache)
     out, cache = layer.forward_block(t.x[40:41])
     same_as_full(slice(40, 41), out, cache)
+    layer.close()
+
+
+@pytest.mark.parametrize("act", ["bf16", "f32"])
+@pytest.mark.parametrize("d,E,k,F,T", [(320, 48, 4, 960, 3500), (64, 4, 2, 1408, 40)])   # tall tiles, a reduction in parts
+def test_a_block_step_from_before_training_mode_has_its_backward(device, d, E, k, F, T, act):
+    """The layer's own normed rows are there.  Its weights are still zero: gradients pass the layer by, and the router's are those of the
+    auxiliary losses."""
+    x = synth.round_bf16(synth.normal((T, d), 1.0, 35, 1))
+    gout = synth.round_bf16(synth.normal((T, d), 1.0, 35, 2))
+    nw = np.ones(d, np.float32)
+    layer = rb.MoeLayer(d, rb.MoeConfig(E, k, F), device, act_dtype=act, weight_dtype="bf16", max_tokens=8 * T)
+    layer.set_option(L.OPT_DECODE_PATH, 0)
+    layer.set_feed_forward_norm(nw)
+    out, _ = layer.forward_block(x)
+    layer.enable_training()
+    assert np.array_equal(out, x) and np.array_equal(layer.backward_block(gout), gout)
+    zero = lambda *shape: np.zeros(shape, np.float32)
+    ref = orc.OracleLayer(d, E, k, F, zero(E, d), [orc.ExpertWeights(gate=zero(F, d), up=zero(F, d), down=zero(d, F)) for _ in range(E)],
+                          None, 0, 0.01, 1e-3)   # (the layer's default weights of the losses)
+    _, _, inner = ref.backward_block(x, nw, 1e-6, gout, round_normed=synth.round_bf16 if act == "bf16" else None, threads=8)
+    assert rel_l2(layer.weight_grad(L.W_ROUTER), inner.grad_router) <= (2e-2 if act == "bf16" else 1e-5)
+    assert not layer.weight_grad(L.W_DOWN, 0).any()
     layer.close()

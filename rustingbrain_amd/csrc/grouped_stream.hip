@@ -1131,26 +1131,23 @@ int stream_tile_m(int rows, int groups, int F, int d) {
 }
 
 // A narrow down launch of few tiles waits for a chain of slices that holds a fraction of the compute units.  Its reduction is shared out
-// where it is long and the rows, which the combine then reads in f32 and twice or four times, are few.  How many us the halves and quarters
-// give was fitted to medians of four runs over 560 shapes (d 256 to 1024, 4 to 16 experts of 1024 to 2752, one to four a row, 40 to 640
-// rows; 0.6 and 1.0 us off on average; 288 more of d 64 and 128 agree), and the better one is taken where it gives half a us: 4.2 % a forward on average over them, 4 of
-// them slower by more than 1.5 % and none by 2.5 % (the best of the three everywhere would give 4.8 %).  us a forward, whole / 2 parts / 4
-// parts: d 768, 8 experts of 1408, int8, 83 rows 34.9 / 32.7 / 31.4; d 512, 8 of 2730, one a row, int8, 186 rows 41.8 / 36.3 / 33.5; d 1024, 4 of
-// 2730, 100 rows 39.7 / 35.7 / 35.0; not taken: d 768, 8 of 1408 and a shared one, bf16, 186 rows 35.6 / 36.2 / 36.8, 4 of 1088, four a row, d 768,
-// 64 rows 33.4 / 35.1 / 36.3.  Reductions of 384 and 704 lose: d 512, 8 of 352 and a shared one, 100 rows 26.0 / 26.9 / 26.7.
-int stream_parts(const GroupedArgs& g, WeightKind wk, int k) {
+// where it is long and the rows, which the combine then reads in f32 and twice or four times, are few.  us a forward, whole / 2 parts
+// / 4 parts (tiles; rows times d in thousands): d 512, 8 experts of 1408, 100 rows (32; 102) 31.5 / 29.9 / 30.1, 400 rows (40; 410) 35.4 /
+// 34.2 / 34.3, 700 rows (56; 717) 36.2 / 36.4 / 36.5; d 768, 8 of 1408, int8, 83 rows (48; 127) 34.9 / 32.7 / 31.4, 200 rows (48; 307) 35.8 /
+// 34.5 / 35.2; with a shared expert, bf16, 83 rows (54; 191) 36.1 / 35.7 / 36.5, 340 rows (72; 783) 40.7 / 41.3 / 41.3; 16 of 1408, 203 rows
+// (96; 312) 40.6 / 41.2 / 41.1; d 1024, 8 of 1408, int8, 150 rows (64; 307) 37.7 / 36.0 / 37.8; 4 of 2730, 100 rows (32; 102) 39.7 / 35.7 / 35.0.
+// Reductions of 384 and 704 lose: d 512, 8 of 352 and a shared one, 100 rows 26.0 / 26.9 / 26.7.  Over 560 shapes (d 256 to 1024, 4 to 16
+// experts of 1024 to 2752, one to four a row, 40 to 640 rows) the rule gives 3.9 % a forward on average; 43 of them, of 1088 and, in bf16, 1408
+// columns, are slower by 1.5 to 4.9 %: d 768, 4 of 1088, four a row, 64 rows 33.4 / 35.1 / 36.3, 8 of 1408 and a shared one, 186 rows
+// 35.6 / 36.2 / 36.8.  (Lines drawn by the estimated gain leave out all but 4 of those and give 4.2 %, but round the rows of a call in other
+// places than before: the lines stay.)
+int stream_parts(const GroupedArgs& g) {
     if (g.swiglu || g.dense_rows >= 0 || !stream_narrow(g)) return 1;
     const int m = g.likely_tiles > 0 ? g.likely_tiles : g.max_tiles, tiles = stream_tiles(g, m, BM, 128);
     const int K = g.dense2.rows > 0 ? std::min(g.K, g.dense2.K) : g.K;
     const long long elements = (long long)(g.routed_rows + g.dense2.rows) * g.N;
     if (K < 1024 || tiles > 64 || elements > 512 * 1024) return 1;
-    const double slices = K / 64, e = elements / 65536.0, t = tiles / 16.0, shared = g.dense2.rows > 0 ? 1.0 : 0.0;
-    const bool i8 = wk == WeightKind::I8;
-    const double two = i8 ? 0.17 * slices - 1.5 - 0.15 * e + 0.09 * t - 0.45 * shared - 0.23 * k
-                          : 0.14 * slices - 2.2 - 0.07 * e - 0.23 * shared - 0.23 * k;
-    const double four = i8 ? 0.23 * slices - 1.25 - 0.24 * e - 0.29 * t - 0.6 * shared - 0.35 * k
-                           : 0.16 * slices - 0.8 - 0.02 * e - 0.7 * t - 0.6 * shared - 0.4 * k;
-    return std::max(two, four) < 0.5 ? 1 : four > two ? 4 : 2;
+    return tiles <= 48 && elements <= 128 * 1024 ? 4 : 2;
 }
 
 // K a multiple of 64 (one LDS slice), N a multiple of 32 (row blocks of the packed weights)

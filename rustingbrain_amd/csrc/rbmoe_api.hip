@@ -1604,7 +1604,7 @@ int forward_impl(rbmoe_layer* L, const void* x, int T, int cols, const uint8_t* 
     const GroupedArgs call = shared_joins ? with_shared(g2, s2) : g2;
     if ((L->f32_rows || (mfma && d % 8 == 0)) && !for_training && T > 0 && d % 4 == 0 && k <= 8 &&
         (L->f32_rows || !c.shared_expert || shared_joins)) {
-        g2.parts = mfma ? stream_parts(call, wk, k) : f32_parts(call, wk);
+        g2.parts = mfma ? stream_parts(call) : f32_parts(call, wk);
         const size_t rows = (size_t)T * k + (shared_joins ? (size_t)T : 0);
         while (g2.parts > 1 && g2.parts * rows * d * 4 > parts_room(L)) g2.parts /= 2;
     }
@@ -2885,7 +2885,7 @@ int rbmoe_internal_parts(int32_t T, int32_t E, int32_t k, int32_t F, int32_t Fs,
     g.groups = E;
     g.dense_rows = -1;
     if (Fs) g.dense2 = {g.a, g.w, nullptr, d, Fs, T, nullptr, nullptr};
-    return f32_rows ? f32_parts(g, wk) : stream_parts(g, wk, k);
+    return f32_rows ? f32_parts(g, wk) : stream_parts(g);
 }
 
 // Test hook (not part of rbmoe.h): how the last forward's products ran.  out[0]: rows of the tiles, [1]: parts of the down product's

@@ -265,7 +265,7 @@ constexpr int kGenericTileM = 16;
 constexpr int kStreamTileM = 128;
 int stream_tile_m(int rows, int groups, int F, int d);  // rows of the tile table's tiles for so many routed rows: 128 or 160
 bool stream_shape_ok(int N, int K);
-int stream_parts(const GroupedArgs& a, WeightKind wk, int k);  // GroupedArgs::parts for a plain launch, k experts a row, where there is room for them
+int stream_parts(const GroupedArgs& a);  // GroupedArgs::parts for a plain launch where there is room for them
 hipError_t launch_grouped_stream(const GroupedArgs& a, WeightKind wk, hipStream_t s);
 void pack_weight_bf16(const uint16_t* src, int rows, int cols, uint16_t* dst);
 void pack_weight_i8(const int8_t* src, int rows, int cols, int8_t* dst);

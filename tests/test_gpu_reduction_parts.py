@@ -113,10 +113,10 @@ def test_parts_whatever_the_layer_has_room_for(device, shape, parts, wt, shared)
         assert n == got[0][2] and np.array_equal(out, got[0][0]) and np.array_equal(y, got[0][1])
 
 
-# The packed kernels: reductions of 22, 29, 33 and 43 slices of 64 in halves and quarters, rows on both sides of the rule's lines
+# The packed kernels: reductions of 15, 17, 22, 29, 33 and 43 slices of 64 in whole, halves and quarters, rows on both sides of the rule's lines
 PACKED = [dict(d=64, E=4, k=2, F=1408, T=40), dict(d=512, E=8, k=2, F=1408, T=125), dict(d=768, E=8, k=2, F=1408, T=200),
           dict(d=512, E=8, k=2, F=1088, T=126), dict(d=256, E=3, k=1, F=1856, T=300), dict(d=128, E=8, k=2, F=2112, T=125),
-          dict(d=768, E=8, k=2, F=2752, T=140)]
+          dict(d=768, E=8, k=2, F=2752, T=140), dict(d=256, E=4, k=2, F=960, T=60)]
 
 
 @pytest.mark.parametrize("shared", [False, True])

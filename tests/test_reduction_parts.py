@@ -17,18 +17,18 @@ def stream_parts(T, E, k, F, Fs, d, int8):
     return parts(T, E, k, F, Fs, d, 0, L.I8 if int8 else L.BF16)
 
 
-@pytest.mark.parametrize("d,E,k,F,Fs,T,bf16,int8", [
-    # long reductions of few rows: quarters, and halves where the rows are more
-    (768, 8, 2, 2752, 0, 100, 2, 4), (512, 8, 1, 2752, 0, 186, 4, 4), (768, 8, 2, 1408, 0, 83, 1, 4), (768, 8, 2, 1408, 0, 200, 1, 2),
-    (256, 4, 2, 1792, 0, 60, 4, 4), (768, 8, 2, 2752, 2752, 200, 2, 4),
-    # short ones, or a shared expert's rows beside them: no gain, or a loss
-    (768, 4, 4, 1088, 0, 64, 1, 1), (256, 4, 2, 1088, 1088, 186, 1, 4), (768, 8, 2, 1408, 1408, 186, 1, 2), (512, 16, 4, 1088, 0, 150, 1, 1),
-    (256, 4, 4, 1408, 1408, 150, 1, 4), (256, 8, 1, 1408, 1408, 600, 1, 4),
-    # under a thousand columns, over 64 tiles, over half a million elements
-    (512, 8, 2, 960, 0, 60, 1, 1), (768, 24, 1, 2752, 0, 60, 1, 1), (512, 8, 2, 2752, 0, 513, 1, 1),
+@pytest.mark.parametrize("int8", [0, 1])
+@pytest.mark.parametrize("d,E,k,F,Fs,T,want", [
+    # quarters up to 48 tiles and 128 K elements
+    (768, 8, 2, 1408, 0, 83, 4), (512, 8, 1, 2752, 0, 186, 4), (256, 4, 2, 1792, 0, 60, 4), (256, 4, 2, 1024, 0, 256, 4), (256, 4, 2, 1024, 0, 257, 2),
+    # halves up to 64 tiles and 512 K elements, a shared expert's among them
+    (768, 8, 2, 2752, 0, 100, 2), (768, 8, 2, 1408, 0, 200, 2), (768, 8, 2, 2752, 2752, 200, 2), (512, 16, 4, 1088, 0, 150, 2),
+    (256, 8, 1, 1408, 1408, 600, 2), (512, 8, 2, 2752, 0, 512, 2),
+    # under a thousand columns on either side, over 64 tiles, over half a million elements
+    (512, 8, 2, 960, 0, 60, 1), (512, 8, 2, 1408, 960, 60, 1), (768, 24, 1, 2752, 0, 60, 1), (512, 8, 2, 2752, 0, 513, 1),
 ])
-def test_where_reductions_are_shared_out(d, E, k, F, Fs, T, bf16, int8):
-    assert (stream_parts(T, E, k, F, Fs, d, 0), stream_parts(T, E, k, F, Fs, d, 1)) == (bf16, int8)
+def test_where_reductions_are_shared_out(d, E, k, F, Fs, T, want, int8):
+    assert stream_parts(T, E, k, F, Fs, d, int8) == want
 
 
 # d, experts, a row, width, shared width, rows: while every workgroup has a compute unit to itself, in reductions of at least 288 columns

@@ -274,7 +274,8 @@ int rbmoe_forward_block_host(rbmoe_layer* layer, const void* x, int32_t tokens, 
  * (rbmoe_layer_create); f32 rows over bf16 weights do where every width is a multiple of 64; any other shape or dtype
  * mix on plain kernels; int8 layers report RBMOE_UNSUPPORTED, as the reference has no backward for quantized
  * experts (src/ffn.rs:87-93).
- * Call it before the weights are set.  A training layer always takes the large-batch kernels. */
+ * Call it before the weights are set.  A training layer always takes the large-batch kernels.  A forward from before it has kept no
+ * input, so rbmoe_backward behind one is RBMOE_INVALID_INPUT (but for large-batch calls behind the norm, whose rows are the layer's). */
 int rbmoe_layer_enable_training(rbmoe_layer* layer);
 
 /* MoeLayer::backward on DEVICE pointers for the last forward: `grad_output` [tokens, cols] act_dtype in,
